@@ -124,255 +124,266 @@ extern "C" int ninfer_lightning_attention(const void* qkv, int stride, int q_off
 //
 // which is the recurrence written out; all powers of the decay have exponents >= 0, so nothing
 // grows. Every product runs on v_mfma_f32_32x32x2_f32: q, k, v (silu of the projections), the
-// decays and the state enter in 32-bit and are never rounded to a shorter type. A block owns
-// one (request, head, 32 value columns): the chunks of a request follow each other in it, and
-// the value columns of a head are independent, which gives the launch heads x vdim / 32 blocks
-// per request. Waves 0 and 1 form the chunk's outputs, waves 2 and 3 carry the state in their
-// accumulators and hand a copy to the others through LDS.
+// decays and the state enter in 32-bit and are never rounded to a shorter type.
+//
+// The chunks of a step lie side by side: a block per (chunk, head, 128 value columns) forms the sum
+// of S' (lightning_chunk_sums), a thread per number of the state walks a request's chunks and leaves
+// the state before each in the sum's place (lightning_chunk_carry), and a block per (chunk, head,
+// 128 value columns) forms the outputs (lightning_chunk_outputs). That is 3 passes over 64 KB of
+// state per chunk and head of 128 x 128 where one block that walks the chunks of a request keeps it
+// in registers, but 512 blocks instead of 64 for a prompt of 2,048 tokens with 16 heads, and no
+// chain of 32 chunks with three barriers each: 25 + 15 + 51 us against 903 for that prompt. (Three
+// GFLOP are 20 us at the rate of the 32-bit matrix instruction; the sums and the outputs are bound
+// by silu of the rows and LDS before it, one and two blocks a CU.)
 namespace ninfer {
 
 typedef float lt_f32x16 __attribute__((ext_vector_type(16)));
 typedef __bf16 lt_bf16x8 __attribute__((ext_vector_type(8)));
 constexpr int kLtChunk = 64;
-constexpr int kLtStateTiles = 4;   // 32-row tiles of the state per carrying wave: dim up to 256
+constexpr int kLtCols = 128;       // value columns of a block
+constexpr int kLtThreads = 512;
+constexpr int kLtMaxDim = 256;
+constexpr int kLtTile = 32 * 33;   // a 32 x 32 tile of decayed scores in LDS
+
+struct LightningChunks {
+  const bf16* qkv;
+  const float* decay;
+  float* state;
+  float* out;
+  float* sums;   // [chunks, H, dim, vdim]: a chunk's sum, then the state before it
+  const int* seq_row_start;
+  const int* seq_slots;
+  int64_t state_stride;
+  int stride, q_off, k_off, v_off, S, H, dim, vdim;
+};
 
 __device__ __forceinline__ float decay_pow(float log2d, int n) {
   return n == 0 ? 1.f : exp2f((float)n * log2d);   // (a decay of 0 has log2 -inf: 0 * -inf is no number)
 }
 
-template <typename T>
-__global__ __launch_bounds__(256) void lightning_chunk_kernel(
-    const T* __restrict__ qkv, int stride, int q_off, int k_off, int v_off,
-    const float* __restrict__ decay, float* __restrict__ state, int64_t state_stride,
-    float* __restrict__ out, const int* __restrict__ seq_row_start,
-    const int* __restrict__ seq_slots, int H, int dim, int vdim) {
-  extern __shared__ float smem[];
-  const int qs = dim + 1;                 // row length of q and k in LDS (odd: column reads spread)
-  float* Qs = smem;                       // [64][dim + 1]
-  float* Ks = Qs + kLtChunk * qs;         // [64][dim + 1]
-  float* Vs = Ks + kLtChunk * qs;         // [64][33]
-  float* As = Vs + kLtChunk * 33;         // [64][65]
-  float* Ss = As + kLtChunk * 65;         // [dim32][33]
-  float* Ws = Ss + ((dim + 31) / 32 * 32) * 33;   // [64] d^(L - 1 - j) of the chunk's rows
-  const int s = blockIdx.x, h = blockIdx.y, c0 = 32 * blockIdx.z;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, lr = lane & 31, lk = lane >> 5;
-  const int r0 = seq_row_start[s], n = seq_row_start[s + 1] - r0;
-  const int dim32 = (dim + 31) / 32 * 32;
-  const int d_tiles = dim32 / 32;
-  float* st = state + (int64_t)seq_slots[s] * state_stride + (int64_t)h * dim * vdim;
-  const float dec = decay[h];
-  const float log2d = log2f(dec);
-  const bool col_ok = c0 + lr < vdim;
-  // rows of bfloat16 whose q and k parts start at multiples of 16 bytes
-  const bool wide = sizeof(T) == 2 && dim % 8 == 0 && stride % 8 == 0 && q_off % 8 == 0 &&
-                    k_off % 8 == 0 && ((uintptr_t)qkv % 16 == 0);
+// Chunk `at` of the step, chunks counted request after request.
+__device__ __forceinline__ bool lightning_find_chunk(const LightningChunks& a, int at, int* row0, int* rows) {
+  for (int s = 0; s < a.S; ++s) {
+    const int r = a.seq_row_start[s], n = a.seq_row_start[s + 1] - r;
+    const int chunks = (n + kLtChunk - 1) / kLtChunk;
+    if (at < chunks) {
+      *row0 = r + at * kLtChunk;
+      *rows = min(kLtChunk, n - at * kLtChunk);
+      return true;
+    }
+    at -= chunks;
+  }
+  return false;
+}
 
-  // the state: in the accumulators of waves 2 and 3 (tiles w - 2, w, ...), a copy in LDS
-  lt_f32x16 sacc[kLtStateTiles];
+// Columns col .. col + width - 1 of the chunk's rows, silu applied, times `scale` per row where
+// given, into LDS rows of `row` floats, zeros beyond the last row and from `width` to `padded`
+// (a multiple of 8). WIDE: the columns start and end at multiples of 16 bytes.
+template <bool WIDE>
+__device__ __forceinline__ void lightning_rows(const LightningChunks& a, int row0, int L, int col, int width,
+                                               int padded, float* lds, int row, const float* scale) {
+  const bf16* rows = a.qkv + (int64_t)row0 * a.stride + col;
+  const int per_row = padded / 8;
+  for (int e = threadIdx.x; e < kLtChunk * per_row; e += kLtThreads) {
+    const int i = e / per_row, d = 8 * (e % per_row);
+    float z[8];
+    if (WIDE) {
+      const lt_bf16x8 x = *(const lt_bf16x8*)(rows + (int64_t)min(i, L - 1) * a.stride + min(d, width - 8));
 #pragma unroll
-  for (int x = 0; x < kLtStateTiles; ++x)
-#pragma unroll
-    for (int i = 0; i < 16; ++i) sacc[x][i] = 0.f;
-  for (int e = tid; e < dim32 * 33; e += 256) {
-    const int d = e / 33, c = e % 33;
-    Ss[e] = (d < dim && c < 32 && c0 + c < vdim) ? st[(int64_t)d * vdim + c0 + c] : 0.f;
-  }
-  __syncthreads();
-  if (w >= 2) {
-#pragma unroll
-    for (int x = 0; x < kLtStateTiles; ++x) {
-      const int dt = (w - 2) + 2 * x;
-      if (dt < d_tiles) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) sacc[x][4 * q + r] = Ss[(32 * dt + 8 * q + 4 * lk + r) * 33 + lr];
-      }
-    }
-  }
-
-  for (int i0 = 0; i0 < n; i0 += kLtChunk) {
-    const int L = min(kLtChunk, n - i0);
-    // 1. the chunk's q, k (all of the head's numbers) and this block's value columns
-    if (wide) {   // eight neighbouring numbers per load
-      const int per_row = dim / 8;
-      for (int e = tid; e < kLtChunk * per_row; e += 256) {
-        const int i = e / per_row, d = 8 * (e % per_row);
-        float qv[8], kv[8];
-#pragma unroll
-        for (int x = 0; x < 8; ++x) qv[x] = kv[x] = 0.f;
-        if (i < L) {
-          const T* row = qkv + (int64_t)(r0 + i0 + i) * stride;
-          const lt_bf16x8 a = *(const lt_bf16x8*)(row + q_off + h * dim + d);
-          const lt_bf16x8 b = *(const lt_bf16x8*)(row + k_off + h * dim + d);
-#pragma unroll
-          for (int x = 0; x < 8; ++x) {
-            qv[x] = silu_f((float)a[x]);
-            kv[x] = silu_f((float)b[x]);
-          }
-        }
-#pragma unroll
-        for (int x = 0; x < 8; ++x) {
-          Qs[i * qs + d + x] = qv[x];
-          Ks[i * qs + d + x] = kv[x];
-        }
-      }
+      for (int n = 0; n < 8; ++n) z[n] = (float)x[n];
     } else {
-      for (int e = tid; e < kLtChunk * dim; e += 256) {
-        const int i = e / dim, d = e % dim;
-        float qv = 0.f, kv = 0.f;
-        if (i < L) {
-          const T* row = qkv + (int64_t)(r0 + i0 + i) * stride;
-          qv = silu_f(to_f32(row[q_off + h * dim + d]));
-          kv = silu_f(to_f32(row[k_off + h * dim + d]));
-        }
-        Qs[i * qs + d] = qv;
-        Ks[i * qs + d] = kv;
-      }
+#pragma unroll
+      for (int n = 0; n < 8; ++n) z[n] = to_f32(rows[(int64_t)min(i, L - 1) * a.stride + min(d + n, width - 1)]);
     }
-    for (int e = tid; e < kLtChunk * 32; e += 256) {
-      const int i = e >> 5, c = e & 31;
-      float vv = 0.f;
-      if (i < L && c0 + c < vdim)
-        vv = silu_f(to_f32(qkv[(int64_t)(r0 + i0 + i) * stride + v_off + h * vdim + c0 + c]));
-      Vs[i * 33 + c] = vv;
-    }
-    if (tid < kLtChunk) Ws[tid] = tid < L ? decay_pow(log2d, L - 1 - tid) : 0.f;
-    __syncthreads();   // (also: the state's copy in LDS is the one before this chunk)
-    // 2. A[i][j] = d^(i - j) q_i . k_j for j <= i: wave w has rows 32 (w / 2).., keys 32 (w % 2)..
-    {
-      const int mi = w >> 1, nj = w & 1;
-      lt_f32x16 a;
+    const float f = scale ? scale[i] : 1.f;
 #pragma unroll
-      for (int i = 0; i < 16; ++i) a[i] = 0.f;
-      if (nj <= mi) {
-        const float* qrow = Qs + (32 * mi + lr) * qs + lk;
-        const float* krow = Ks + (32 * nj + lr) * qs + lk;
-#pragma unroll 8
-        for (int d = 0; d < dim; d += 2) {
-          const float qa = (d + lk < dim) ? qrow[d] : 0.f;
-          const float kb = (d + lk < dim) ? krow[d] : 0.f;
-          a = __builtin_amdgcn_mfma_f32_32x32x2f32(qa, kb, a, 0, 0, 0);
-        }
-      }
-      const int j = 32 * nj + lr;
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int i = 32 * mi + 8 * q + 4 * lk + r;
-          As[i * 65 + j] = j <= i ? a[4 * q + r] * decay_pow(log2d, i - j) : 0.f;
-        }
-    }
-    __syncthreads();
-    // 3. waves 0, 1: the outputs of rows 32 w ..; waves 2, 3: the state after the chunk
-    if (w < 2) {
-      lt_f32x16 o;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) o[i] = 0.f;
-      const int row = 32 * w + lr;
-      const float* arow = As + row * 65 + lk;
-#pragma unroll 8
-      for (int j = 0; j < 32 * (w + 1); j += 2)
-        o = __builtin_amdgcn_mfma_f32_32x32x2f32(arow[j], Vs[(j + lk) * 33 + lr], o, 0, 0, 0);
-      const float carry = decay_pow(log2d, row + 1);
-      const float* qrow = Qs + row * qs + lk;
-#pragma unroll 8
-      for (int d = 0; d < dim; d += 2) {
-        const float qa = (d + lk < dim) ? qrow[d] * carry : 0.f;
-        o = __builtin_amdgcn_mfma_f32_32x32x2f32(qa, Ss[(d + lk) * 33 + lr], o, 0, 0, 0);
-      }
-      if (col_ok) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int i = 32 * w + 8 * q + 4 * lk + r;
-            if (i < L) out[((int64_t)(r0 + i0 + i) * H + h) * vdim + c0 + lr] = o[4 * q + r];
-          }
-      }
-    } else {
-      const float whole = decay_pow(log2d, L);
-#pragma unroll
-      for (int x = 0; x < kLtStateTiles; ++x) {
-        const int dt = (w - 2) + 2 * x;
-        if (dt < d_tiles) {
-#pragma unroll
-          for (int i = 0; i < 16; ++i) sacc[x][i] *= whole;
-          const int d = 32 * dt + lr;
-#pragma unroll 8
-          for (int j = 0; j < kLtChunk; j += 2) {
-            const int jj = j + lk;
-            const float ka = (jj < L && d < dim) ? Ks[jj * qs + d] * Ws[jj] : 0.f;
-            sacc[x] = __builtin_amdgcn_mfma_f32_32x32x2f32(ka, Vs[jj * 33 + lr], sacc[x], 0, 0, 0);
-          }
-        }
-      }
-    }
-    __syncthreads();   // everyone has read the old copy of the state
-    if (w >= 2) {
-#pragma unroll
-      for (int x = 0; x < kLtStateTiles; ++x) {
-        const int dt = (w - 2) + 2 * x;
-        if (dt < d_tiles) {
-#pragma unroll
-          for (int q = 0; q < 4; ++q)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) Ss[(32 * dt + 8 * q + 4 * lk + r) * 33 + lr] = sacc[x][4 * q + r];
-        }
-      }
-    }
-    // (the barrier after the next chunk's loads publishes the copy; nothing reads it before)
-  }
-  if (w >= 2 && col_ok) {
-#pragma unroll
-    for (int x = 0; x < kLtStateTiles; ++x) {
-      const int dt = (w - 2) + 2 * x;
-      if (dt < d_tiles) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int d = 32 * dt + 8 * q + 4 * lk + r;
-            if (d < dim) st[(int64_t)d * vdim + c0 + lr] = sacc[x][4 * q + r];
-          }
-      }
-    }
+    for (int n = 0; n < 8; ++n) lds[i * row + d + n] = i < L && d + n < width ? silu_f(z[n]) * f : 0.f;
   }
 }
 
-static size_t lightning_chunk_lds(int dim) {
-  const int dim32 = (dim + 31) / 32 * 32;
-  return ((size_t)2 * kLtChunk * (dim + 1) + kLtChunk * 33 + kLtChunk * 65 + (size_t)dim32 * 33 + kLtChunk) * sizeof(float);
+// sum_j d^(L - 1 - j) k_j v_j^T of a chunk. The 32 x 32 tiles of [dim, 128 columns] go round the waves.
+template <bool WIDE>
+__global__ __launch_bounds__(kLtThreads) void lightning_chunk_sums_kernel(LightningChunks a) {
+  extern __shared__ float smem[];
+  __shared__ float w_s[kLtChunk];
+  int row0, L;
+  if (!lightning_find_chunk(a, blockIdx.x, &row0, &L)) return;
+  const int h = blockIdx.y, c0 = kLtCols * blockIdx.z, tid = threadIdx.x;
+  const int lane = tid & 63, w = tid >> 6, lr = lane & 31, lk = lane >> 5;
+  const int dim32 = (a.dim + 31) / 32 * 32, ks = dim32 + 1, vs = kLtCols + 1;
+  float* Ks = smem;                       // [64][dim32 + 1], times the decay to the chunk's end
+  float* Vs = Ks + kLtChunk * ks;         // [64][129]
+  if (tid < kLtChunk) w_s[tid] = tid < L ? decay_pow(log2f(a.decay[h]), L - 1 - tid) : 0.f;
+  __syncthreads();
+  lightning_rows<WIDE>(a, row0, L, a.k_off + h * a.dim, a.dim, dim32, Ks, ks, w_s);
+  lightning_rows<WIDE>(a, row0, L, a.v_off + h * a.vdim + c0, min(kLtCols, a.vdim - c0), kLtCols, Vs, vs, nullptr);
+  __syncthreads();
+  float* sum = a.sums + ((int64_t)blockIdx.x * a.H + h) * a.dim * a.vdim;
+  for (int t = w; t < dim32 / 32 * (kLtCols / 32); t += kLtThreads / 64) {
+    const int dt = t / (kLtCols / 32), ct = t % (kLtCols / 32);
+    if (c0 + 32 * ct >= a.vdim) continue;
+    lt_f32x16 acc = {};
+    const float* kc = Ks + lk * ks + 32 * dt + lr;
+    const float* vc = Vs + lk * vs + 32 * ct + lr;
+#pragma unroll 8
+    for (int j = 0; j < kLtChunk; j += 2)
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(kc[j * ks], vc[j * vs], acc, 0, 0, 0);
+    const int c = c0 + 32 * ct + lr;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int d = 32 * dt + 8 * q + 4 * lk + r;
+        if (d < a.dim && c < a.vdim) sum[(int64_t)d * a.vdim + c] = acc[4 * q + r];
+      }
+  }
+}
+
+// S before every chunk in place of the chunk's sum, and the state after the last.
+__global__ __launch_bounds__(256) void lightning_chunk_carry_kernel(LightningChunks a) {
+  const int64_t numbers = (int64_t)a.H * a.dim * a.vdim, e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (e >= numbers) return;
+  const int s = blockIdx.y;
+  int first = 0;
+  for (int i = 0; i < s; ++i) first += (a.seq_row_start[i + 1] - a.seq_row_start[i] + kLtChunk - 1) / kLtChunk;
+  const int n = a.seq_row_start[s + 1] - a.seq_row_start[s], count = (n + kLtChunk - 1) / kLtChunk;
+  const float log2d = log2f(a.decay[e / ((int64_t)a.dim * a.vdim)]);
+  const float whole = decay_pow(log2d, kLtChunk);
+  float* slot = a.state + (int64_t)a.seq_slots[s] * a.state_stride + e;
+  float* at = a.sums + first * numbers + e;
+  float S = *slot;
+  for (int i0 = 0; i0 < count; i0 += 8) {
+    float sum[8];   // eight loads on their way before the first is used
+#pragma unroll
+    for (int i = 0; i < 8; ++i) sum[i] = at[min(i0 + i, count - 1) * numbers];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (i0 + i < count) {
+        at[(i0 + i) * numbers] = S;
+        S = S * (i0 + i + 1 < count ? whole : decay_pow(log2d, n - (count - 1) * kLtChunk)) + sum[i];
+      }
+  }
+  *slot = S;
+}
+
+// The outputs of a chunk: wave w has rows 32 (w / 4) .. and value columns 32 (w % 4) .. of the
+// block's 128. The decayed scores are formed once, by three waves; values take the keys' place.
+template <bool WIDE>
+__global__ __launch_bounds__(kLtThreads) void lightning_chunk_outputs_kernel(LightningChunks a) {
+  extern __shared__ float smem[];
+  int row0, L;
+  if (!lightning_find_chunk(a, blockIdx.x, &row0, &L)) return;
+  const int h = blockIdx.y, c0 = kLtCols * blockIdx.z, tid = threadIdx.x;
+  const int lane = tid & 63, w = tid >> 6, lr = lane & 31, lk = lane >> 5;
+  const int dim32 = (a.dim + 31) / 32 * 32, qs = dim32 + 1, vs = kLtCols + 1;
+  const float log2d = log2f(a.decay[h]);
+  float* Qs = smem;                        // [64][dim32 + 1]
+  float* As = Qs + kLtChunk * qs;          // scores of tiles (0, 0), (1, 0), (1, 1)
+  float* Ks = As + 3 * kLtTile;            // [64][dim32 + 1], then the values [64][129]
+  lightning_rows<WIDE>(a, row0, L, a.q_off + h * a.dim, a.dim, dim32, Qs, qs, nullptr);
+  lightning_rows<WIDE>(a, row0, L, a.k_off + h * a.dim, a.dim, dim32, Ks, qs, nullptr);
+  __syncthreads();
+  if (w < 3) {
+    const int mi = w > 0, nj = w > 1;
+    lt_f32x16 s = {};
+    const float* qrow = Qs + (32 * mi + lr) * qs + lk;
+    const float* krow = Ks + (32 * nj + lr) * qs + lk;
+#pragma unroll 8
+    for (int d = 0; d < dim32; d += 2) s = __builtin_amdgcn_mfma_f32_32x32x2f32(qrow[d], krow[d], s, 0, 0, 0);
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int i = 8 * q + 4 * lk + r, back = 32 * (mi - nj) + i - lr;
+        As[w * kLtTile + i * 33 + lr] = back >= 0 ? s[4 * q + r] * decay_pow(log2d, back) : 0.f;
+      }
+  }
+  __syncthreads();
+  float* Vs = Ks;
+  lightning_rows<WIDE>(a, row0, L, a.v_off + h * a.vdim + c0, min(kLtCols, a.vdim - c0), kLtCols, Vs, vs, nullptr);
+  __syncthreads();
+  const int mi = w >> 2, col = 32 * (w & 3);
+  if (c0 + col >= a.vdim || 32 * mi >= L) return;
+  const int c = min(c0 + col + lr, a.vdim - 1);
+  lt_f32x16 o = {};
+  for (int nj = 0; nj <= mi; ++nj) {
+    const float* arow = As + (mi + nj) * kLtTile + lr * 33 + lk;
+#pragma unroll 8
+    for (int j = 0; j < 32; j += 2)
+      o = __builtin_amdgcn_mfma_f32_32x32x2f32(arow[j], Vs[(32 * nj + j + lk) * vs + col + lr], o, 0, 0, 0);
+  }
+  const float carry = decay_pow(log2d, 32 * mi + lr + 1);
+  const float* qrow = Qs + (32 * mi + lr) * qs + lk;
+  const float* S = a.sums + ((int64_t)blockIdx.x * a.H + h) * a.dim * a.vdim + c;
+#pragma unroll 16
+  for (int d = 0; d < dim32; d += 2)   // (queries beyond dim are zeros)
+    o = __builtin_amdgcn_mfma_f32_32x32x2f32(qrow[d] * carry, S[(int64_t)min(d + lk, a.dim - 1) * a.vdim], o, 0, 0, 0);
+  if (c0 + col + lr >= a.vdim) return;
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int i = 32 * mi + 8 * q + 4 * lk + r;
+      if (i < L) a.out[((int64_t)(row0 + i) * a.H + h) * a.vdim + c] = o[4 * q + r];
+    }
+}
+
+static int64_t lightning_most_chunks(int T, int S) { return T / kLtChunk + S; }   // no step has more
+
+static int lightning_lds(const void* kern, size_t lds) {
+  if (lds <= 48 * 1024) return 0;
+  hipError_t e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  if (e != hipSuccess) return set_error(-2, "lightning_attention: cannot get %zu bytes of LDS", lds);
+  return 0;
+}
+
+template <bool WIDE>
+static int lightning_chunks(const LightningChunks& a, int T, hipStream_t stream) {
+  const int qs = (a.dim + 31) / 32 * 32 + 1, vs = kLtCols + 1;
+  const size_t rows = (size_t)kLtChunk * sizeof(float);
+  const size_t lds_sums = rows * (qs + vs), lds_out = rows * (qs + (qs > vs ? qs : vs)) + 3 * kLtTile * sizeof(float);
+  if (int rc = lightning_lds((const void*)lightning_chunk_sums_kernel<WIDE>, lds_sums)) return rc;
+  if (int rc = lightning_lds((const void*)lightning_chunk_outputs_kernel<WIDE>, lds_out)) return rc;
+  const dim3 grid(lightning_most_chunks(T, a.S), a.H, (a.vdim + kLtCols - 1) / kLtCols);
+  const int64_t numbers = (int64_t)a.H * a.dim * a.vdim;
+  lightning_chunk_sums_kernel<WIDE><<<grid, kLtThreads, lds_sums, stream>>>(a);
+  NINFER_LAUNCH_CHECK();
+  lightning_chunk_carry_kernel<<<dim3((numbers + 255) / 256, a.S), 256, 0, stream>>>(a);
+  NINFER_LAUNCH_CHECK();
+  lightning_chunk_outputs_kernel<WIDE><<<grid, kLtThreads, lds_out, stream>>>(a);
+  NINFER_LAUNCH_CHECK();
+  return 0;
 }
 
 }  // namespace ninfer
 
+// Floats of workspace with which a step runs in chunks; 0 when the sizes do not fit (the
+// token-by-token kernel takes them).
+extern "C" long long ninfer_lightning_chunk_floats(int T, int S, int H, int dim, int vdim, int dtype) {
+  if (dtype != kBF16 || dim > kLtMaxDim) return 0;
+  return lightning_most_chunks(T, S) * H * dim * vdim;
+}
+
 // The same as ninfer_lightning_attention for bfloat16 rows, chunk by chunk on the matrix cores:
-// for steps that bring prompt portions. Returns 1 (nothing launched) when the sizes do not fit.
+// for steps that bring prompt portions. `work`: ninfer_lightning_chunk_floats floats.
 extern "C" int ninfer_lightning_attention_chunks(const void* qkv, int stride, int q_off, int k_off,
                                                  int v_off, const float* decay, float* state,
                                                  long long state_stride, float* out,
                                                  const int* seq_row_start, const int* seq_slots,
                                                  int T, int S, int H, int dim, int vdim, int dtype,
-                                                 hipStream_t stream) {
+                                                 float* work, hipStream_t stream) {
   NINFER_REQUIRE(T > 0 && S > 0 && H > 0 && dim > 0 && vdim > 0,
                  "lightning_attention: T=%d S=%d heads=%d dim=%d vdim=%d must be positive", T, S,
                  H, dim, vdim);
   NINFER_REQUIRE(state_stride >= (long long)H * dim * vdim,
                  "lightning_attention: a request's state of %lld floats holds no %d x %d x %d",
                  state_stride, H, dim, vdim);
-  const size_t lds = lightning_chunk_lds(dim);
-  if (dtype != kBF16 || dim > 64 * kLtStateTiles || lds > 160 * 1024) return 1;
-  auto kern = lightning_chunk_kernel<bf16>;
-  if (lds > 48 * 1024) {
-    hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       (int)lds);
-    if (e != hipSuccess) return set_error(-2, "lightning_attention: cannot get %zu bytes of LDS", lds);
-  }
-  kern<<<dim3(S, H, (vdim + 31) / 32), 256, lds, stream>>>(
-      (const bf16*)qkv, stride, q_off, k_off, v_off, decay, state, state_stride, out,
-      seq_row_start, seq_slots, H, dim, vdim);
-  NINFER_LAUNCH_CHECK();
-  return 0;
+  NINFER_REQUIRE(ninfer_lightning_chunk_floats(T, S, H, dim, vdim, dtype) > 0 && work,
+                 "lightning_attention: dtype %d, key size %d do not run in chunks, or no workspace", dtype, dim);
+  LightningChunks a = {(const bf16*)qkv, decay, state, out, work, seq_row_start, seq_slots, state_stride,
+                       stride, q_off, k_off, v_off, S, H, dim, vdim};
+  // rows whose q, k and v parts start and end at multiples of 16 bytes
+  const bool wide = dim % 8 == 0 && vdim % 8 == 0 && stride % 8 == 0 && q_off % 8 == 0 && k_off % 8 == 0 &&
+                    v_off % 8 == 0 && (uintptr_t)qkv % 16 == 0;
+  return wide ? lightning_chunks<true>(a, T, stream) : lightning_chunks<false>(a, T, stream);
 }

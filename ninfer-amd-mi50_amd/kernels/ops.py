@@ -343,6 +343,7 @@ class HipOps:
         self.lib.ninfer_sample_few_places.restype = ctypes.c_longlong
         self.lib.ninfer_latent_attention_workspace_floats.restype = ctypes.c_longlong
         self.lib.ninfer_gla_segment_floats.restype = ctypes.c_longlong
+        self.lib.ninfer_lightning_chunk_floats.restype = ctypes.c_longlong
         self.lib.ninfer_decay_scan_chunk_floats.restype = ctypes.c_longlong
         self.lib.ninfer_diff_attention_workspace_floats.restype = ctypes.c_longlong
         self.lib.ninfer_sigmoid_attention_workspace_floats.restype = ctypes.c_longlong
@@ -1507,18 +1508,19 @@ class HipOps:
                 ctypes.c_void_p(decay.data_ptr()), ctypes.c_void_p(state.data_ptr()),
                 ctypes.c_longlong(state.stride(0)), ctypes.c_void_p(out.data_ptr()),
                 ctypes.c_void_p(ctx.seq_row_start.data_ptr()), ctypes.c_void_p(ctx.seq_slots.data_ptr()),
-                t, ctx.S, heads, dim, vdim, _DT[qkv.dtype], self._stream())
-        # bfloat16 steps that bring prompt portions: chunks of 64 rows on the matrix cores (the
+                t, ctx.S, heads, dim, vdim, _DT[qkv.dtype])
+        # bfloat16 steps that bring prompt portions: chunks of 64 rows on the matrix cores, side by side (the
         # sums of a chunk are ordered otherwise than token by token, so the 32-bit path, whose
         # logits do not depend on the cut to the bit, stays on the token-by-token kernel)
         if qkv.dtype == torch.bfloat16 and ctx.max_qlen >= self.lightning_chunk_min_rows \
                 and not self.force_generic:
-            rc = self.lib.ninfer_lightning_attention_chunks(*args)
-            if rc == 0:
+            floats = self.lib.ninfer_lightning_chunk_floats(t, ctx.S, heads, dim, vdim, _DT[qkv.dtype])
+            if floats > 0:
+                work = torch.empty(floats, dtype=torch.float32, device=qkv.device)
+                self._ok(self.lib.ninfer_lightning_attention_chunks(
+                    *args, ctypes.c_void_p(work.data_ptr()), self._stream()))
                 return
-            if rc < 0:
-                self._ok(rc)
-        self._ok(self.lib.ninfer_lightning_attention(*args))
+        self._ok(self.lib.ninfer_lightning_attention(*args, self._stream()))
 
     def _latent_args(self, ctx, pool, block_table, heads, dim, rank, rot_dim, rot_n, page_size,
                      dtype):

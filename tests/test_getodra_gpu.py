@@ -163,6 +163,38 @@ def test_lightning_in_portions(ops, dtype, heads, dim, vdim):
     assert state_all[0].abs().max() == 0 and state_all[2].abs().max() == 0
 
 
+@pytest.mark.parametrize("heads,dim,vdim", [(2, 128, 136), (1, 256, 64), (3, 8, 8), (2, 72, 260)])
+@pytest.mark.parametrize("lens", [[64], [65, 1, 63], [200, 8], [129, 64, 128]])
+def test_lightning_chunks_of_aligned_rows(ops, heads, dim, vdim, lens):
+    """Rows in whole 16-byte pieces: chunks of 64 rows and one row more or less, requests that
+    bring one row beside them, value columns beyond a block's 128, on a state that is there."""
+    torch.manual_seed(dim + sum(lens))
+    decay = [0.97, 0.0, 1.0][:heads]
+    qk, vw = heads * dim, heads * vdim
+    x = torch.randn(sum(lens), 2 * qk + vw).to(torch.bfloat16)
+    state = torch.randn(len(lens) + 1, heads * dim * vdim)
+    ctx = util.make_context(ops, torch.bfloat16, [(0, n) for n in lens])
+    got_state, out = state.to(DEV), torch.empty(sum(lens), vw, device=DEV)
+    ops.lightning_attention(x.to(DEV), 0, qk, 2 * qk, heads, dim, vdim, torch.tensor(decay, device=DEV),
+                            got_state, ctx, out)
+    slots = ctx.seq_slots.cpu().tolist()
+    f = plain_getodra.silu(x.double())
+    at = 0
+    for slot, n in zip(slots, lens):
+        q, k, v = f[at:at + n, :qk], f[at:at + n, qk:2 * qk], f[at:at + n, 2 * qk:]
+        S = state[slot].double().reshape(heads, dim, vdim).clone()
+        want = torch.zeros(n, heads, vdim, dtype=torch.float64)
+        for t in range(n):
+            S = torch.tensor(decay).double()[:, None, None] * S + \
+                k[t].reshape(heads, dim, 1) * v[t].reshape(heads, 1, vdim)
+            want[t] = (q[t].reshape(heads, dim, 1) * S).sum(1)
+        assert rel_err(out[at:at + n].double().cpu().reshape(n, heads, vdim), want) < 2e-5
+        assert rel_err(got_state[slot].double().cpu().reshape(S.shape), S) < 2e-5
+        at += n
+    untouched = [i for i in range(len(lens) + 1) if i not in slots]
+    assert torch.equal(got_state[untouched].cpu(), state[untouched])
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("heads,k,n", [(3, 24, 40), (4, 64, 160), (1, 16, 32), (5, 40, 20), (2, 12, 10)])
 @pytest.mark.parametrize("rows", [1, 7, 70])
