@@ -16,15 +16,22 @@
 //                    row's position alone. The head's output may be multiplied by
 //                    sigmoid(gate[row, head]).
 //
-//   latent_attention_tile (bfloat16, matrix cores): a block of four waves owns 32 rows of
-//                    (token, head) pairs of one request, all of which read the same cached
-//                    rows. Keys come in tiles of 64 through LDS as they lie in the cache
-//                    ([key][numbers]); S = Q' K^T and O += P V run on v_mfma_f32_32x32x16_bf16,
-//                    the softmax between them in 32-bit on eight lanes per row. The value
-//                    operand needs eight keys of one column per lane and takes them from
-//                    the tile by eight two-byte LDS reads. The keys of long contexts are cut
-//                    into chunks over several blocks whose partial sums a second kernel
-//                    merges (steps of few rows would otherwise leave most of the GPU idle).
+//   latent_attention_tile (bfloat16, matrix cores): a block of eight waves owns 64 rows (16 in
+//                    decode-only steps) of (token, head) pairs of one request, all of which read
+//                    the same cached rows. Keys come in tiles of 64 through LDS as they lie in
+//                    the cache ([key][numbers]), the next tile on its way in registers; the
+//                    queries stay in registers, each wave with half of the numbers, so a key is
+//                    read from LDS twice for 64 rows. The values' operand comes from the same
+//                    tile through the transposing LDS read. S and O += P V run on the matrix
+//                    cores, the softmax between them in 32-bit. The keys of long contexts are cut
+//                    into chunks over several blocks whose partial sums a second kernel merges
+//                    (steps of few rows would otherwise leave most of the GPU idle); a request's
+//                    tiles are shared out evenly over its chunks.
+//
+// Latent 512 + 64, 16 heads, against blocks of four waves and 32 rows with the queries in LDS and the
+// values gathered by two-byte reads: a 2,048-token prompt 688 -> 209 us (73 GFLOP, 350 TFLOP/s; the
+// LDS traffic alone, 3,000 cycles a tile of 64 keys, is 42 us), 64 requests at 1,950 to 2,600 keys
+// 188 -> 59 us (168 MB, 2.8 TB/s: a tile's way into the CU and four barriers, 6.5 us a tile).
 //
 // The rotation turns pair (i, i + n/2), or with `interleaved` pair (2i, 2i + 1), of the first
 // n = rot_n numbers of the rotated part by pos * freq[i]; cosine and sine are multiplied by `magnitude` (1 without a scaled table).
@@ -262,25 +269,29 @@ namespace ninfer {
 typedef __bf16 lat_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float lat_f32x16 __attribute__((ext_vector_type(16)));
 
-constexpr int kLatRows = 32;      // (token, head) rows per block
+typedef float lat_f32x4 __attribute__((ext_vector_type(4)));
+typedef short lat_short4 __attribute__((ext_vector_type(4)));
+typedef short lat_short8 __attribute__((ext_vector_type(8)));
+typedef __attribute__((address_space(3))) lat_short4 lat_lds_short4;
+
 constexpr int kLatKeys = 64;      // keys per tile
-constexpr int kLatColTiles = 4;   // 32-column tiles of the output per wave: latent sizes up to 512
-constexpr int kLatPieces = 20;    // 16-byte pieces of a tile per thread: cached rows of up to 640 numbers
+constexpr int kLatThreads = 512;
+constexpr int kLatPRow = kLatKeys + 8;   // row length of the probabilities in LDS
+constexpr int kLatMaxHalf = 20;   // steps of 16 numbers of half a cached row: rows of up to 640
+constexpr float kLatLog2e = 1.44269504088896f;
 
 struct LatentTilePlan {
+  int rows;         // (token, head) rows of a block
   int tiles;        // upper bound of row tiles over all requests
   int n_chunks;     // key chunks per row tile
-  int chunk;        // keys per chunk (a multiple of 64)
-  int dkp;          // row length of Q in LDS (numbers)
-  int kstr;         // row length of a key in LDS (numbers)
+  int half;         // steps of 16 numbers in half a cached row (the kernel's own: 9, 18 or 20)
   int page_shift;
   size_t lds;
 };
 
 static bool latent_tile_takes(const LatentArgs& a) {
   const int Dk = a.R + a.rd;
-  return a.dtype == kBF16 && !a.force_plain && Dk % 8 == 0 && a.R <= 32 * 4 * kLatColTiles &&
-         kLatKeys * (Dk / 8) <= 256 * kLatPieces &&
+  return a.dtype == kBF16 && !a.force_plain && Dk % 8 == 0 && a.R <= 512 && Dk <= 32 * kLatMaxHalf &&
          (a.page_size & (a.page_size - 1)) == 0 && a.seq_row_start && a.seq_pos0 && a.S > 0 &&
          ((uintptr_t)a.pool % 16 == 0) && ((uintptr_t)a.q_abs % 16 == 0);
 }
@@ -288,27 +299,23 @@ static bool latent_tile_takes(const LatentArgs& a) {
 static LatentTilePlan latent_tile_plan(const LatentArgs& a) {
   LatentTilePlan p;
   const int Dk = a.R + a.rd;
-  const int dk16 = (Dk + 15) / 16 * 16;
-  const int cols = (a.R + 31) / 32 * 32;
-  p.dkp = dk16 + 8;
-  p.kstr = (dk16 > cols ? dk16 : cols) + 8;
+  p.half = Dk <= 32 * 9 ? 9 : Dk <= 32 * 18 ? 18 : kLatMaxHalf;
+  // A decode-only step's request has as many rows as heads: up to 16 of them take a block whose
+  // products are 16 rows high and which is bound by the cached rows' way into the CU.
+  p.rows = a.max_qlen == 1 && a.Hq <= 16 ? 16 : 64;
   // row tiles: in a decode-only step every request has the same number; otherwise a bound
   // (a request's last tile may be partial; tiles that do not exist exit at once)
-  p.tiles = a.max_qlen == 1 ? a.S * ((a.Hq + kLatRows - 1) / kLatRows)
-                            : (int)(((int64_t)a.T * a.Hq + kLatRows - 1) / kLatRows) + a.S;
+  p.tiles = a.max_qlen == 1 ? a.S * ((a.Hq + p.rows - 1) / p.rows)
+                            : (int)(((int64_t)a.T * a.Hq + p.rows - 1) / p.rows) + a.S;
   const int key_tiles = (a.max_kv_len + kLatKeys - 1) / kLatKeys;
-  // a block fills a CU (its LDS and registers): one block per CU, each with as long a walk as
-  // that allows, since a block's start (Q', its first tile) costs as much as two tiles
+  // a block fills a CU (its LDS): one block per CU, each with as long a walk as that allows
   int want = device_cu_count() / p.tiles;
   if (want > key_tiles) want = key_tiles;
-  if (want < 1) want = 1;
-  const int tiles_per_chunk = (key_tiles + want - 1) / want;
-  p.chunk = tiles_per_chunk * kLatKeys;
-  p.n_chunks = (key_tiles + tiles_per_chunk - 1) / tiles_per_chunk;
+  p.n_chunks = want < 1 ? 1 : want;
   p.page_shift = 0;
   while ((1 << p.page_shift) < a.page_size) ++p.page_shift;
-  p.lds = (size_t)kLatRows * p.dkp * 2 + (size_t)kLatKeys * p.kstr * 2 +
-          2 * kLatRows * kLatKeys * 4 + kLatRows * (kLatKeys + 8) * 2 + 3 * kLatRows * 4;
+  p.lds = (size_t)kLatKeys * (32 * p.half + 8) * 2 + (size_t)2 * p.rows * kLatKeys * 4 +
+          (size_t)p.rows * kLatPRow * 2 + 3 * p.rows * 4;
   return p;
 }
 
@@ -316,18 +323,26 @@ static int64_t latent_tile_workspace_floats(const LatentArgs& a, const LatentTil
   return p.n_chunks > 1 ? (int64_t)a.T * a.Hq * p.n_chunks * (a.R + 2) : 0;
 }
 
-__global__ __launch_bounds__(256) void latent_attention_tile_kernel(LatentArgs a, LatentTilePlan pl) {
+// Eight waves. HALF: steps of 16 numbers of half a cached row. CT: tiles of 16 output columns of a
+// wave, whose columns are 16 CT w ... In LDS lie one tile of 64 keys, the scores (two halves of
+// the sum) and the probabilities; the queries stay in registers.
+template <int ROWS, int HALF, int CT>
+__global__ __launch_bounds__(kLatThreads, 2) void latent_attention_tile_kernel(LatentArgs a, LatentTilePlan pl) {
   extern __shared__ float smem[];
+  constexpr int KROW = 32 * HALF + 8;                 // row length of a key in LDS (numbers)
+  constexpr int RT = ROWS / 16;
+  constexpr int PIECES = (kLatKeys * 4 * HALF + kLatThreads - 1) / kLatThreads;   // 16-byte pieces a thread fetches
+  constexpr int PARTS = kLatThreads / ROWS, KEYS = kLatKeys / PARTS;   // threads of a row in the softmax, keys of each
+  constexpr bool WIDE = ROWS == 64;   // scores in tiles of 32 rows x 32 keys, else 16 x 16
+  constexpr int QF = WIDE ? HALF : (HALF + 1) / 2;
   const int Dk = a.R + a.rd, R = a.R, H = a.Hq;
-  __bf16* Qs = (__bf16*)smem;                                   // [32][dkp]
-  __bf16* Ks = Qs + kLatRows * pl.dkp;                          // [64][kstr]
-  float* Sp = (float*)(Ks + kLatKeys * pl.kstr);                // [2][32][64]
-  __bf16* Ps = (__bf16*)(Sp + 2 * kLatRows * kLatKeys);         // [32][72]
-  float* alpha_s = (float*)(Ps + kLatRows * (kLatKeys + 8));    // [32], then m [32], l [32]
-  float* m_s = alpha_s + kLatRows;
-  float* l_s = m_s + kLatRows;
+  __bf16* Ks = (__bf16*)smem;                                   // [64][KROW]
+  float* Sp = (float*)(Ks + kLatKeys * KROW);                   // [2][ROWS][64]
+  __bf16* Ps = (__bf16*)(Sp + 2 * ROWS * kLatKeys);             // [ROWS][72]
+  float* alpha_s = (float*)(Ps + ROWS * kLatPRow);              // [ROWS], then m and l
+  float* m_s = alpha_s + ROWS;
+  float* l_s = m_s + ROWS;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int lr = lane & 31, lk = lane >> 5;
 
   // Which request and which of its row tiles is this block's? The tiles are dealt out from
   // the last one backwards: within a request the later tiles see more keys and run longer,
@@ -336,11 +351,11 @@ __global__ __launch_bounds__(256) void latent_attention_tile_kernel(LatentArgs a
   {
     int total = 0;
     for (int i = 0; i < a.S; ++i)
-      total += ((a.seq_row_start[i + 1] - a.seq_row_start[i]) * H + kLatRows - 1) / kLatRows;
+      total += ((a.seq_row_start[i + 1] - a.seq_row_start[i]) * H + ROWS - 1) / ROWS;
     int left = total - 1 - (int)blockIdx.x;
     for (int i = 0; i < a.S && left >= 0; ++i) {
       const int n = (a.seq_row_start[i + 1] - a.seq_row_start[i]) * H;
-      const int nt = (n + kLatRows - 1) / kLatRows;
+      const int nt = (n + ROWS - 1) / ROWS;
       if (left < nt) {
         s = i;
         lt = left;
@@ -354,253 +369,227 @@ __global__ __launch_bounds__(256) void latent_attention_tile_kernel(LatentArgs a
   const int row0 = a.seq_row_start[s];
   const int n_flat = (a.seq_row_start[s + 1] - row0) * H;
   const int pos0 = a.seq_pos0[s];
-  const int f0 = lt * kLatRows;                          // first flattened row of the tile
-  const int rows_here = min(kLatRows, n_flat - f0);
+  const int f0 = lt * ROWS;                          // first flattened row of the tile
+  const int rows_here = min(ROWS, n_flat - f0);
   const int tok_first = f0 / H, tok_last = (f0 + rows_here - 1) / H;
   const int pos_last = pos0 + tok_last;
   const int lo_first = a.window > 0 ? max(0, pos0 + tok_first - a.window + 1) : 0;
-  // this block's keys: its chunk of the context, cut to what its rows can see
-  const int k_begin = max(chunk_id * pl.chunk, lo_first / kLatKeys * kLatKeys);
-  const int k_end = min((chunk_id + 1) * pl.chunk, pos_last + 1);
+  // this block's keys: its part of the tiles that its rows can see (so that the chunks of a
+  // request are even, however much shorter it is than the longest)
+  const int first_tile = lo_first / kLatKeys, n_tiles = pos_last / kLatKeys + 1 - first_tile;
+  const int per_chunk = (n_tiles + pl.n_chunks - 1) / pl.n_chunks;
+  const int k_begin = (first_tile + min(chunk_id * per_chunk, n_tiles)) * kLatKeys;
+  const int k_end = min((first_tile + min((chunk_id + 1) * per_chunk, n_tiles)) * kLatKeys, pos_last + 1);
   const int* bt = a.block_table + (int64_t)s * a.bt_stride;
   const __bf16* pool = (const __bf16*)a.pool;
 
-  // Q' of the tile's rows as bfloat16, zeros in rows and columns that are not there: eight
-  // threads per row
-  {
-    const int i = tid >> 3;
-    const float* src = nullptr;
-    if (i < rows_here) {
-      const int f = f0 + i;
-      src = a.q_abs + ((int64_t)(row0 + f / H) * H + f % H) * Dk;
+  // A tile's keys travel page -> registers -> LDS; the loads of the next tile are issued before
+  // the products of this one. Keys outside what the rows see are fetched from the nearest that
+  // they do (their probabilities are 0), so that no load waits for a condition.
+  const int cpr = Dk / 8;   // 16-byte pieces of a cached row
+  lat_bf16x8 next[PIECES];
+  int piece[PIECES];        // key of the tile << 16 | first number of the piece
+#pragma unroll
+  for (int i = 0; i < PIECES; ++i) {
+    const int e = min(tid + kLatThreads * i, kLatKeys * cpr - 1);
+    piece[i] = ((e / cpr) << 16) | (8 * (e % cpr));
+  }
+  auto fetch = [&](int kt) {
+    int page[PIECES];
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i)
+      page[i] = bt[min(max(kt + (piece[i] >> 16), lo_first), pos_last) >> pl.page_shift];
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) {
+      const int kp = min(max(kt + (piece[i] >> 16), lo_first), pos_last);
+      next[i] = *(const lat_bf16x8*)(pool + ((int64_t)page[i] * a.page_size + (kp & (a.page_size - 1))) * Dk +
+                                     (piece[i] & 0xffff));
     }
-    // (the row has a multiple of 8 numbers and so has its place in LDS: four at a time, and
-    // several loads under way)
-#pragma unroll 5
-    for (int d = 4 * (tid & 7); d < pl.dkp; d += 32) {
-      float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (src && d < Dk) v = *(const float4*)(src + d);
-      __bf16* dst = Qs + i * pl.dkp + d;
-      dst[0] = (__bf16)v.x;
-      dst[1] = (__bf16)v.y;
-      dst[2] = (__bf16)v.z;
-      dst[3] = (__bf16)v.w;
+  };
+  if (k_begin < k_end) fetch(k_begin);
+
+  // Q' as the products' operand, rounded to bfloat16 once; zeros beyond the row's numbers. In the
+  // wide form wave w has rows 32 (w / 4) .., keys 32 (w / 2 % 2) .. and one half of the numbers;
+  // in the other all 16 rows, keys 16 (w / 2) .. and one half of the numbers.
+  const int kh = w & 1, kn = WIDE ? (w >> 1) & 1 : w >> 1;
+  const int q_lane = WIDE ? lane & 31 : lane & 15, q_k = 8 * (WIDE ? lane >> 5 : lane >> 4);
+  constexpr int STEP = WIDE ? 16 : 32;
+  lat_bf16x8 qf[QF];
+  {
+    const int f = f0 + min((WIDE ? 32 * (w >> 2) : 0) + q_lane, rows_here - 1);
+    const float* src = a.q_abs + ((int64_t)(row0 + f / H) * H + f % H) * Dk;
+#pragma unroll
+    for (int st = 0; st < QF; ++st) {
+      const int in_half = STEP * st + q_k, d = 16 * HALF * kh + in_half;
+      const bool in = d < Dk && in_half < 16 * HALF;
+      const lat_f32x4 lo = *(const lat_f32x4*)(src + (in ? d : 0)), up = *(const lat_f32x4*)(src + (in ? d + 4 : 0));
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        qf[st][x] = in ? (__bf16)lo[x] : (__bf16)0.f;
+        qf[st][4 + x] = in ? (__bf16)up[x] : (__bf16)0.f;
+      }
     }
   }
   {   // the columns of a key's row beyond its numbers are read as zeros and never written again
-    const int pad = pl.kstr - Dk;
-    for (int e = tid; e < kLatKeys * pad; e += 256) Ks[(e / pad) * pl.kstr + Dk + e % pad] = (__bf16)0.f;
+    const int pad = KROW - Dk;
+    for (int e = tid; e < kLatKeys * pad; e += kLatThreads) Ks[(e / pad) * KROW + Dk + e % pad] = (__bf16)0.f;
   }
-  __syncthreads();
 
-  // softmax threads: row tid / 8, keys 8 (tid % 8) .. + 7 of a tile
-  const int sm_row = tid >> 3, sm_part = tid & 7;
+  // softmax threads: row tid / PARTS, keys KEYS (tid % PARTS) .. of a tile
+  const int sm_row = tid / PARTS, sm_part = tid % PARTS;
   int sm_pos = -1, sm_lo = 0;
   if (sm_row < rows_here) {
     sm_pos = pos0 + (f0 + sm_row) / H;
     sm_lo = a.window > 0 ? max(0, sm_pos - a.window + 1) : 0;
   }
-  float m_run = -INFINITY, l_run = 0.f;
+  const float scale2 = a.scale * kLatLog2e;
+  float m_run = -INFINITY, l_run = 0.f;   // (of the scores times log2 e)
 
-  lat_f32x16 acc[kLatColTiles];
+  lat_f32x4 acc[CT][RT];
 #pragma unroll
-  for (int c = 0; c < kLatColTiles; ++c)
+  for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) acc[c][i] = 0.f;
-  const int n_ct = (R + 31) / 32;
-  const int ct_per_wave = (n_ct + 3) / 4;
-  const int ksteps = (Dk + 15) / 16;
-  const int ks_half = (ksteps + 1) / 2;
-  const int cpr = Dk / 8;   // 16-byte pieces of a cached row
+    for (int rt = 0; rt < RT; ++rt) acc[ct][rt] = lat_f32x4{0.f, 0.f, 0.f, 0.f};
+  const int c = lane & 15, g = lane >> 4;
 
-  // A tile's keys travel page -> registers -> LDS; the loads of the next tile are issued before
-  // the products of this one, so that their way from memory is hidden behind them.
-  lat_bf16x8 next[kLatPieces];
-  int piece[kLatPieces];   // key of the tile << 16 | first number of the piece; -1: none
-#pragma unroll
-  for (int i = 0; i < kLatPieces; ++i) {
-    const int e = tid + 256 * i;
-    piece[i] = e < kLatKeys * cpr ? ((e / cpr) << 16) | (8 * (e % cpr)) : -1;
-  }
-  auto fetch = [&](int kt) {
-#pragma unroll
-    for (int i = 0; i < kLatPieces; ++i) {
-      lat_bf16x8 v;
-#pragma unroll
-      for (int x = 0; x < 8; ++x) v[x] = (__bf16)0.f;
-      if (piece[i] >= 0) {
-        const int kp = kt + (piece[i] >> 16);
-        if (kp <= pos_last) {
-          const int page = bt[kp >> pl.page_shift];
-          if (page >= 0)
-            v = *(const lat_bf16x8*)(pool + ((int64_t)page * a.page_size + (kp & (a.page_size - 1))) * Dk +
-                                     (piece[i] & 0xffff));
-        }
-      }
-      next[i] = v;
-    }
-  };
-  if (k_begin < k_end) fetch(k_begin);
   for (int kt = k_begin; kt < k_end; kt += kLatKeys) {
     // 1. the tile's keys into LDS as they lie in their pages
 #pragma unroll
-    for (int i = 0; i < kLatPieces; ++i)
-      if (piece[i] >= 0)
-        *(lat_bf16x8*)(Ks + (piece[i] >> 16) * pl.kstr + (piece[i] & 0xffff)) = next[i];
+    for (int i = 0; i < PIECES; ++i)
+      *(lat_bf16x8*)(Ks + (piece[i] >> 16) * KROW + (piece[i] & 0xffff)) = next[i];
     if (kt + kLatKeys < k_end) fetch(kt + kLatKeys);
     lds_barrier();   // (orders LDS traffic only: the next tile's loads stay under way)
-    // 2. S = Q' K^T: wave w meets keys 32 (w & 1) .. + 31 over one half of the numbers
-    {
-      const int n = w & 1, kh = w >> 1;
-      lat_f32x16 sacc;
+    // 2. scores over one half of the numbers
+    float* sp = Sp + kh * ROWS * kLatKeys;
+    if constexpr (WIDE) {
+      lat_f32x16 sacc = {};
+      const __bf16* krow = Ks + (32 * kn + q_lane) * KROW + 16 * HALF * kh + q_k;
 #pragma unroll
-      for (int i = 0; i < 16; ++i) sacc[i] = 0.f;
-      const int s_lo = kh ? ks_half : 0, s_hi = kh ? ksteps : ks_half;
-      const __bf16* qrow = Qs + lr * pl.dkp + 8 * lk;
-      const __bf16* krow = Ks + (32 * n + lr) * pl.kstr + 8 * lk;
-      int st = s_lo;
-      for (; st + 6 <= s_hi; st += 6) {   // six steps' operands are read before the first product
-        lat_bf16x8 qf[6], kf[6];
-#pragma unroll
-        for (int u = 0; u < 6; ++u) {
-          qf[u] = *(const lat_bf16x8*)(qrow + 16 * (st + u));
-          kf[u] = *(const lat_bf16x8*)(krow + 16 * (st + u));
-        }
-#pragma unroll
-        for (int u = 0; u < 6; ++u) sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qf[u], kf[u], sacc, 0, 0, 0);
-      }
-      for (; st < s_hi; ++st) {
-        const lat_bf16x8 qf = *(const lat_bf16x8*)(qrow + 16 * st);
-        const lat_bf16x8 kf = *(const lat_bf16x8*)(krow + 16 * st);
-        sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qf, kf, sacc, 0, 0, 0);
-      }
-      // the lane holds key 32 n + lr for rows 8 q + 4 lk + r in register 4 q + r
-      float* sp = Sp + kh * kLatRows * kLatKeys + 32 * n + lr;
+      for (int st = 0; st < QF; ++st)
+        sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qf[st], *(const lat_bf16x8*)(krow + 16 * st), sacc, 0, 0, 0);
+      // the lane holds key 32 kn + q_lane for rows 8 q + 4 (lane / 32) + r in register 4 q + r
 #pragma unroll
       for (int q = 0; q < 4; ++q)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) sp[(8 * q + 4 * lk + r) * kLatKeys] = sacc[4 * q + r];
+        for (int r = 0; r < 4; ++r)
+          sp[(32 * (w >> 2) + 8 * q + 4 * (lane >> 5) + r) * kLatKeys + 32 * kn + q_lane] = sacc[4 * q + r];
+    } else {
+      lat_f32x4 sacc = {};
+      // (the last step of an odd HALF has 16 numbers of the half: the lanes beyond have zeros in
+      // the queries, and read any number)
+      const __bf16* krow = Ks + (16 * kn + c) * KROW + 16 * HALF * kh + q_k;
+#pragma unroll
+      for (int st = 0; st < QF; ++st) {
+        const bool past = HALF % 2 && st == QF - 1 && g >= 2;
+        const lat_bf16x8 kf = *(const lat_bf16x8*)(krow + (past ? 0 : 32 * st));
+        sacc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qf[st], kf, sacc, 0, 0, 0);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) sp[(4 * g + r) * kLatKeys + 16 * kn + c] = sacc[r];
     }
-    lds_barrier();   // (orders LDS traffic only: the next tile's loads stay under way)
-    // 3. softmax of the tile, 32-bit: eight lanes per row
+    lds_barrier();
+    // 3. softmax of the tile, 32-bit
     {
-      float sv[8];
+      float sv[KEYS];
       float mx = -INFINITY;
 #pragma unroll
-      for (int x = 0; x < 8; ++x) {
-        const int j = 8 * sm_part + x;
-        const int kp = kt + j;
-        const float v = (Sp[sm_row * kLatKeys + j] + Sp[kLatRows * kLatKeys + sm_row * kLatKeys + j]) * a.scale;
-        const bool see = kp <= sm_pos && kp >= sm_lo;
-        sv[x] = see ? v : -INFINITY;
+      for (int x = 0; x < KEYS; ++x) {
+        const int j = KEYS * sm_part + x, kp = kt + j;
+        const float v = (Sp[sm_row * kLatKeys + j] + Sp[(ROWS + sm_row) * kLatKeys + j]) * scale2;
+        sv[x] = kp <= sm_pos && kp >= sm_lo ? v : -INFINITY;
         mx = fmaxf(mx, sv[x]);
       }
-      mx = fmaxf(mx, __shfl_xor(mx, 1, 64));
-      mx = fmaxf(mx, __shfl_xor(mx, 2, 64));
-      mx = fmaxf(mx, __shfl_xor(mx, 4, 64));
+#pragma unroll
+      for (int off = 1; off < PARTS; off *= 2) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
       const float m_new = fmaxf(m_run, mx);
-      float al = 1.f, sum = 0.f;
-      lat_bf16x8 pv;
-      if (m_new == -INFINITY) {   // nothing seen so far
+      const float ref = m_new == -INFINITY ? 0.f : m_new;   // nothing seen so far: all terms are 0
+      const float al = __builtin_amdgcn_exp2f(m_run - ref);   // 0 while m_run is minus infinity
+      float sum = 0.f;
+      __bf16* prow = Ps + sm_row * kLatPRow + KEYS * sm_part;
 #pragma unroll
-        for (int x = 0; x < 8; ++x) pv[x] = (__bf16)0.f;
-      } else {
-        al = expf(m_run - m_new);   // 0 while m_run is minus infinity
-#pragma unroll
-        for (int x = 0; x < 8; ++x) {
-          const float p = expf(sv[x] - m_new);
-          pv[x] = (__bf16)p;
-          sum += p;
-        }
+      for (int x = 0; x < KEYS; ++x) {
+        const float p = __builtin_amdgcn_exp2f(sv[x] - ref);
+        prow[x] = (__bf16)p;
+        sum += p;
       }
-      sum += __shfl_xor(sum, 1, 64);
-      sum += __shfl_xor(sum, 2, 64);
-      sum += __shfl_xor(sum, 4, 64);
+#pragma unroll
+      for (int off = 1; off < PARTS; off *= 2) sum += __shfl_xor(sum, off, 64);
       l_run = l_run * al + sum;
       m_run = m_new;
-      *(lat_bf16x8*)(Ps + sm_row * (kLatKeys + 8) + 8 * sm_part) = pv;
       if (sm_part == 0) alpha_s[sm_row] = al;
     }
-    lds_barrier();   // (orders LDS traffic only: the next tile's loads stay under way)
-    // 4. O = O alpha + P V on this wave's column tiles
+    lds_barrier();
+    // 4. O = O alpha + P V on this wave's columns: V^T comes through the transposing read, a lane
+    // (c, g) holds column c of a tile for keys 8 g .. + 7; P^T row c of a tile for the same keys
     {
-      const float al = alpha_s[lr];   // every register of the lane belongs to row lr
-      lat_bf16x8 pf[4];
+      float al[RT];
 #pragma unroll
-      for (int st = 0; st < 4; ++st)
-        pf[st] = *(const lat_bf16x8*)(Ps + lr * (kLatKeys + 8) + 16 * st + 8 * lk);
+      for (int rt = 0; rt < RT; ++rt) al[rt] = alpha_s[16 * rt + c];
 #pragma unroll
-      for (int c = 0; c < kLatColTiles; ++c) {
-        const int ct = w * ct_per_wave + c;
-        if (c < ct_per_wave && ct < n_ct) {
+      for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
-          for (int i = 0; i < 16; ++i) acc[c][i] *= al;
-          const __bf16* vcol = Ks + 32 * ct + lr;
+        for (int rt = 0; rt < RT; ++rt) acc[ct][rt] *= al[rt];
 #pragma unroll
-          for (int st = 0; st < 4; ++st) {
-            lat_bf16x8 vf;
+      for (int k0 = 0; k0 < kLatKeys; k0 += 32) {
+        lat_bf16x8 pf[RT];
 #pragma unroll
-            for (int x = 0; x < 8; ++x) vf[x] = vcol[(16 * st + 8 * lk + x) * pl.kstr];
-            // A = V^T: lane holds column 32 ct + lr for 8 keys; B = P^T: row lr for the same keys
-            acc[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf[st], acc[c], 0, 0, 0);
+        for (int rt = 0; rt < RT; ++rt) pf[rt] = *(const lat_bf16x8*)(Ps + (16 * rt + c) * kLatPRow + k0 + 8 * g);
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) {
+          const int col = 16 * (CT * w + ct);
+          if (col < R) {
+            const __bf16* v = Ks + (k0 + 8 * g + (c >> 2)) * KROW + col + 4 * (c & 3);
+            const lat_short4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lat_lds_short4*)v);
+            const lat_short4 up = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lat_lds_short4*)(v + 4 * KROW));
+            const lat_short8 both = {lo.x, lo.y, lo.z, lo.w, up.x, up.y, up.z, up.w};
+            const lat_bf16x8 vf = __builtin_bit_cast(lat_bf16x8, both);
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt)
+              acc[ct][rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf[rt], acc[ct][rt], 0, 0, 0);
           }
         }
       }
     }
-    lds_barrier();   // (orders LDS traffic only: the next tile's loads stay under way)
+    lds_barrier();
   }
 
   if (sm_part == 0) {
-    m_s[sm_row] = m_run;
+    m_s[sm_row] = m_run * (1.f / kLatLog2e);   // (of the scores themselves: what the merge expects)
     l_s[sm_row] = l_run;
   }
   __syncthreads();
-  // With A = V^T and B = P^T the lane holds row lr of the tile (a (token, head) pair) and the
-  // columns 32 ct + 8 q + 4 lk + r in register 4 q + r.
-  if (lr < rows_here) {
-    const int f = f0 + lr;
-    const int t = row0 + f / H, h = f % H;
-    const float l = l_s[lr], m = m_s[lr];
+  // The lane holds row c of every row tile (a (token, head) pair) and columns 4 g .. of every column tile.
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) {
+    const int i = 16 * rt + c;
+    if (i >= rows_here) continue;
+    const int f = f0 + i, t = row0 + f / H, h = f % H;
+    const float l = l_s[i];
+    float factor = 1.f;
+    float* part = nullptr;
     if (pl.n_chunks == 1) {
-      float inv = l > 0.f ? 1.f / l : 0.f;
+      factor = l > 0.f ? 1.f / l : 0.f;
       if (a.gate) {
-        const float g = __bfloat162float(((const bf16*)a.gate)[(int64_t)t * a.gate_stride + h]);
-        inv *= 1.f / (1.f + expf(-g));
-      }
-      __bf16* orow = (__bf16*)a.out + ((int64_t)t * H + h) * R;
-#pragma unroll
-      for (int c = 0; c < kLatColTiles; ++c) {
-        const int ct = w * ct_per_wave + c;
-        if (c < ct_per_wave && ct < n_ct) {
-#pragma unroll
-          for (int q = 0; q < 4; ++q)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              const int d = 32 * ct + 8 * q + 4 * lk + r;
-              if (d < R) orow[d] = (__bf16)(acc[c][4 * q + r] * inv);
-            }
-        }
+        const float z = __bfloat162float(((const bf16*)a.gate)[(int64_t)t * a.gate_stride + h]);
+        factor *= 1.f / (1.f + expf(-z));
       }
     } else {
-      float* part = a.workspace + (((int64_t)t * H + h) * pl.n_chunks + chunk_id) * (R + 2);
-      if (w == 0 && lk == 0) {
-        part[R] = m;
+      part = a.workspace + (((int64_t)t * H + h) * pl.n_chunks + chunk_id) * (R + 2);
+      if (w == 0 && g == 0) {
+        part[R] = m_s[i];
         part[R + 1] = l;
       }
-#pragma unroll
-      for (int c = 0; c < kLatColTiles; ++c) {
-        const int ct = w * ct_per_wave + c;
-        if (c < ct_per_wave && ct < n_ct) {
-#pragma unroll
-          for (int q = 0; q < 4; ++q)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              const int d = 32 * ct + 8 * q + 4 * lk + r;
-              if (d < R) part[d] = acc[c][4 * q + r];
-            }
-        }
-      }
     }
+    __bf16* orow = (__bf16*)a.out + ((int64_t)t * H + h) * R;
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int d = 16 * (CT * w + ct) + 4 * g + r;
+        if (d >= R) continue;
+        if (part) part[d] = acc[ct][rt][r];
+        else orow[d] = (__bf16)(acc[ct][rt][r] * factor);
+      }
   }
 }
 
@@ -639,22 +628,32 @@ __global__ void latent_attention_merge_kernel(LatentArgs a, int n_chunks) {
   }
 }
 
+template <int ROWS, int HALF, int CT>
+static int launch_latent_tile(const LatentArgs& a, const LatentTilePlan& p, hipStream_t stream) {
+  auto kern = latent_attention_tile_kernel<ROWS, HALF, CT>;
+  hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)p.lds);
+  if (e != hipSuccess) return set_error(-2, "latent_attention: cannot get %zu bytes of LDS", p.lds);
+  kern<<<dim3(p.tiles, p.n_chunks), kLatThreads, p.lds, stream>>>(a, p);
+  NINFER_LAUNCH_CHECK();
+  return 0;
+}
+
+template <int ROWS>
+static int launch_latent_rows(const LatentArgs& a, const LatentTilePlan& p, hipStream_t stream) {
+  const bool few = a.R <= 256;   // output columns: 8 waves of 2 or 4 tiles of 16
+  if (p.half == 9) return few ? launch_latent_tile<ROWS, 9, 2>(a, p, stream) : launch_latent_tile<ROWS, 9, 4>(a, p, stream);
+  if (p.half == 18) return few ? launch_latent_tile<ROWS, 18, 2>(a, p, stream) : launch_latent_tile<ROWS, 18, 4>(a, p, stream);
+  return few ? launch_latent_tile<ROWS, kLatMaxHalf, 2>(a, p, stream) : launch_latent_tile<ROWS, kLatMaxHalf, 4>(a, p, stream);
+}
+
 static int latent_attention_tile(const LatentArgs& a, hipStream_t stream) {
   const LatentTilePlan p = latent_tile_plan(a);
-  NINFER_REQUIRE(p.lds <= 160 * 1024, "latent_attention: rows of %d numbers do not fit the LDS",
-                 a.R + a.rd);
   const int64_t need = latent_tile_workspace_floats(a, p);
   NINFER_REQUIRE(need == 0 || (a.workspace && a.workspace_floats >= need),
                  "latent_attention: the workspace holds %lld floats, %lld are needed",
                  (long long)a.workspace_floats, (long long)need);
-  auto kern = latent_attention_tile_kernel;
-  if (p.lds > 48 * 1024) {
-    hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       (int)p.lds);
-    if (e != hipSuccess) return set_error(-2, "latent_attention: cannot get %zu bytes of LDS", p.lds);
-  }
-  kern<<<dim3(p.tiles, p.n_chunks), 256, p.lds, stream>>>(a, p);
-  NINFER_LAUNCH_CHECK();
+  int rc = p.rows == 16 ? launch_latent_rows<16>(a, p, stream) : launch_latent_rows<64>(a, p, stream);
+  if (rc) return rc;
   if (p.n_chunks > 1) {
     const int block = a.R >= 256 ? 256 : (a.R + 63) / 64 * 64;
     latent_attention_merge_kernel<<<(unsigned)((int64_t)a.T * a.Hq), block, p.n_chunks * sizeof(float), stream>>>(a, p.n_chunks);
