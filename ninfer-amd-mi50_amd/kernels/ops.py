@@ -1974,11 +1974,10 @@ class HipOps:
             places = int(self.lib.ninfer_sample_few_places(v))
             cand_val = torch.empty((r, places), dtype=torch.float32, device=logits.device)
             cand_idx = torch.empty((r, places), dtype=torch.int32, device=logits.device)
-            work = torch.empty((r, places), dtype=torch.float32, device=logits.device)
             self._ok(self.lib.ninfer_sample_few(
                 ctypes.c_void_p(logits.data_ptr()), logits.stride(0), v, r,
                 ctypes.c_void_p(cand_val.data_ptr()), ctypes.c_void_p(cand_idx.data_ptr()),
-                ctypes.c_void_p(work.data_ptr()), ctypes.c_void_p(temperature.data_ptr()),
+                ctypes.c_void_p(temperature.data_ptr()),
                 ctypes.c_void_p(top_k.data_ptr()), ctypes.c_void_p(_ptr(top_p)),
                 ctypes.c_void_p(_ptr(rep_penalty)), ctypes.c_void_p(_ptr(pen_tokens)),
                 ctypes.c_void_p(_ptr(pen_counts)), ctypes.c_void_p(_ptr(pen_offsets)),
