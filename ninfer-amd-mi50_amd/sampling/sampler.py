@@ -34,6 +34,21 @@ def uniform(seed: int, key: int, draw: int) -> float:
     return (h >> 40) / float(1 << 24)
 
 
+def uniforms(rows: Sequence["SampleRow"]) -> np.ndarray:
+    """`uniform` of every row's (seed, key, draw) at once, in 32-bit floats (24 bits each: exact)."""
+    u64 = np.uint64
+
+    def mix(x):
+        x = x + u64(0x9E3779B97F4A7C15)
+        x = (x ^ (x >> u64(30))) * u64(0xBF58476D1CE4E5B9)
+        x = (x ^ (x >> u64(27))) * u64(0x94D049BB133111EB)
+        return x ^ (x >> u64(31))
+
+    seed, key, draw = (np.array([v & _MASK for v in vs], dtype=u64)
+                       for vs in zip(*((row.seed, row.key, row.draw) for row in rows)))
+    return (mix(mix(mix(seed) ^ key) ^ draw) >> u64(40)).astype(np.float32) / np.float32(1 << 24)
+
+
 def fresh_seed() -> int:
     return int.from_bytes(os.urandom(8), "little") | 1
 
@@ -102,30 +117,24 @@ class Sampler:
         self._staging: List[list] = []   # pinned buffers (and the event after each one's copy)
         self._staging_next = 0
 
-    def _to_device(self, packed: np.ndarray) -> torch.Tensor:
-        """The rows' packed parameters on the device, through one of a few pinned buffers used in
-        turn: the copy is queued behind the step that makes the logits and the host goes on (a
-        copy out of pageable memory makes the host wait until the device has reached it, and the
-        sampling kernel would then be launched only after the step has ended)."""
-        host = torch.from_numpy(packed)
-        if self.device.type != "cuda":
-            return host.to(self.device)
-        n = host.numel()
+    def _staged(self, n: int) -> list:
+        """[a buffer of at least n ints, the event after its last copy, the same memory as an array]:
+        one of a few pinned buffers used in turn, its last copy done. The rows' parameters are
+        written into it and copied from it, so that the copy is queued behind the step that makes
+        the logits and the host goes on (a copy out of pageable memory makes the host wait until
+        the device has reached it, and the sampling kernel would then be launched only after the
+        step has ended)."""
         if len(self._staging) < 4:
-            self._staging.append([torch.empty(max(n, 1024), dtype=torch.int32).pin_memory(),
-                                  torch.cuda.Event()])
-            slot = self._staging[-1]
+            slot = [None, torch.cuda.Event(), None]
+            self._staging.append(slot)
         else:
             slot = self._staging[self._staging_next]
             self._staging_next = (self._staging_next + 1) % len(self._staging)
             slot[1].synchronize()
-            if slot[0].numel() < n:
-                slot[0] = torch.empty(2 * n, dtype=torch.int32).pin_memory()
-        slot[0][:n].copy_(host)
-        dev = torch.empty(n, dtype=torch.int32, device=self.device)
-        dev.copy_(slot[0][:n], non_blocking=True)
-        slot[1].record()
-        return dev
+        if slot[0] is None or slot[0].numel() < n:
+            slot[0] = torch.empty(max(n if slot[0] is None else 2 * n, 1024), dtype=torch.int32).pin_memory()
+            slot[2] = slot[0].numpy()
+        return slot
 
     def sample(self, logits: torch.Tensor, rows: Sequence[SampleRow]) -> List[int]:
         """One token per row of `logits` [R, vocab]."""
@@ -135,33 +144,50 @@ class Sampler:
         # 32-bit floats and one int per row, the offsets of the penalties, then their tokens
         # and counts. (Copies queue behind the step that makes the logits, one after the other:
         # every further one would add its latency to the step.)
-        pen_t: List[np.ndarray] = []
-        pen_c: List[np.ndarray] = []
-        pen_o = np.zeros(r + 1, np.int32)
-        for i, row in enumerate(rows):
-            n = 0
+        pens = []
+        offsets = [0]
+        for row in rows:
+            n = offsets[-1]
             if row.params.repetition_penalty != 1.0:
-                toks, cnts = row.history.arrays()
-                pen_t.append(toks)
-                pen_c.append(cnts)
-                n = toks.shape[0]
-            pen_o[i + 1] = pen_o[i] + n
-        floats = np.empty((4, r), np.float32)
+                pens.append(row.history.arrays())
+                n += pens[-1][0].shape[0]
+            offsets.append(n)
+        n_pen = offsets[-1]
+        o = 5 * r
+        n = o + (r + 1 + 2 * n_pen if n_pen > 0 else 0)
+        cuda = self.device.type == "cuda"
+        if cuda:
+            pinned, copied, packed = self._staged(n)
+        else:
+            packed = np.empty(n, np.int32)
+        floats = packed[:4 * r].view(np.float32).reshape(4, r)
         floats[0] = [row.params.temperature for row in rows]
         floats[1] = [row.params.top_p for row in rows]
         floats[2] = [row.params.repetition_penalty for row in rows]
-        floats[3] = [uniform(row.seed, row.key, row.draw) for row in rows]
-        top_k = np.asarray([row.params.top_k for row in rows], np.int32)
-        n_pen = int(pen_o[-1])
-        packed = np.concatenate([floats.reshape(-1).view(np.int32), top_k, pen_o] + pen_t + pen_c)
-        dev = self._to_device(packed)
+        drawn = [i for i, row in enumerate(rows) if row.params.temperature > 0]   # (greedy rows draw nothing)
+        floats[3] = 0.0
+        if len(drawn) > 8:   # from there on whole arrays are the shorter way
+            floats[3, drawn] = uniforms([rows[i] for i in drawn])
+        else:
+            for i in drawn:
+                floats[3, i] = uniform(rows[i].seed, rows[i].key, rows[i].draw)
+        packed[4 * r:o] = [row.params.top_k for row in rows]
+        if n_pen > 0:
+            packed[o:o + r + 1] = offsets
+            o += r + 1
+            np.concatenate([p[0] for p in pens], out=packed[o:o + n_pen])
+            np.concatenate([p[1] for p in pens], out=packed[o + n_pen:n])
+        if cuda:
+            dev = torch.empty(n, dtype=torch.int32, device=self.device)
+            dev.copy_(pinned[:n], non_blocking=True)
+            copied.record()
+        else:
+            dev = torch.from_numpy(packed)
         f = dev[:4 * r].view(torch.float32)
-        o = 4 * r
         pen = {}
         if n_pen > 0:
-            pen = dict(pen_offsets=dev[o + r:o + 2 * r + 1],
-                       pen_tokens=dev[o + 2 * r + 1:o + 2 * r + 1 + n_pen],
-                       pen_counts=dev[o + 2 * r + 1 + n_pen:o + 2 * r + 1 + 2 * n_pen])
+            pen = dict(pen_offsets=dev[o - r - 1:o], pen_tokens=dev[o:o + n_pen],
+                       pen_counts=dev[o + n_pen:n])
         out = torch.empty(r, dtype=torch.int32, device=self.device)
         # rows that are greedy or keep at most a few dozen tokens (the reference's default is
         # top_k = 50) take the path that reads the logits with the whole GPU
@@ -170,6 +196,6 @@ class Sampler:
         if most and any(row.params.temperature > 0 for row in rows) and all(
                 row.params.temperature <= 0 or 1 <= row.params.top_k <= most for row in rows):
             pen["few"] = True
-        self.ops.sample(logits, f[:r], f[3 * r:4 * r], out, top_k=dev[o:o + r], top_p=f[r:2 * r],
+        self.ops.sample(logits, f[:r], f[3 * r:4 * r], out, top_k=dev[4 * r:5 * r], top_p=f[r:2 * r],
                         rep_penalty=f[2 * r:3 * r], **pen)
         return out.tolist()
