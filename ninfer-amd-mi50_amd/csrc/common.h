@@ -80,6 +80,45 @@ template <typename V> __device__ __forceinline__ V stream_load(const V* p) {
   return __builtin_nontemporal_load(p);
 }
 
+// VEC (1 or 4) neighbouring numbers of a row in 32-bit; 4: one aligned load or store of 8 or 16 bytes.
+template <int VEC>
+__device__ __forceinline__ void load_row(const float* p, float* f) {
+  if constexpr (VEC == 4) {
+    const float4 v = *(const float4*)p;
+    f[0] = v.x; f[1] = v.y; f[2] = v.z; f[3] = v.w;
+  } else {
+    f[0] = p[0];
+  }
+}
+template <int VEC>
+__device__ __forceinline__ void load_row(const bf16* p, float* f) {
+  if constexpr (VEC == 4) {
+    const uint2 v = *(const uint2*)p;   // four bf16: the upper halves of four floats
+    f[0] = __uint_as_float(v.x << 16); f[1] = __uint_as_float(v.x & 0xffff0000u);
+    f[2] = __uint_as_float(v.y << 16); f[3] = __uint_as_float(v.y & 0xffff0000u);
+  } else {
+    f[0] = to_f32(p[0]);
+  }
+}
+template <int VEC>
+__device__ __forceinline__ void store_row(float* p, const float* f) {
+  if constexpr (VEC == 4) *(float4*)p = make_float4(f[0], f[1], f[2], f[3]);
+  else p[0] = f[0];
+}
+template <int VEC>
+__device__ __forceinline__ void store_row(bf16* p, const float* f) {
+  if constexpr (VEC == 4) {
+    union { bf16 b[4]; uint2 u; } o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o.b[e] = from_f32<bf16>(f[e]);
+    *(uint2*)p = o.u;
+  } else {
+    p[0] = from_f32<bf16>(f[0]);
+  }
+}
+// Whether a pointer (null too) lets rows of a width that is a multiple of 4 be read that way.
+inline bool row_aligned(const void* p) { return ((uintptr_t)p & 15) == 0; }
+
 int set_error(int code, const char* fmt, ...);
 
 // Compute units of the current device (asked once per device; 256 if the runtime cannot

@@ -66,31 +66,53 @@ __global__ void concat_rows_kernel(const float* __restrict__ a, const float* __r
 // (`dense`), or the weighted sum of a sparse feed-forward's rows
 // sum_j w[t,j] * y[t*k + j, c] + sigmoid(gate[t * gate_stride]) * shared[t,c], or nothing.
 // s1 / s2 null: factor 1.
-template <typename T>
+// A thread has VEC neighbouring columns (4 where the rows are whole 16-byte pieces: the sums' terms are
+// the same, the loads a quarter as many; 1,531 rows of 2,048 with four experts and a shared one, 60
+// MB: 25 -> 12 us, 4.9 TB/s; the gated sum of 2,048 rows 39 -> 18).
+template <typename T, int VEC>
 __global__ void scaled_sum_add_kernel(float* __restrict__ residual, const T* __restrict__ a,
                                       const float* __restrict__ s1, const T* __restrict__ dense,
                                       const T* __restrict__ y, const float* __restrict__ w, int k,
                                       const T* __restrict__ shared, const float* __restrict__ gate,
                                       int gate_stride, const float* __restrict__ s2, int H) {
   const int64_t t = blockIdx.x;
-  const int i = blockIdx.y * blockDim.x + threadIdx.x;
+  const int i = VEC * (blockIdx.y * blockDim.x + threadIdx.x);
   if (i >= H) return;
-  float m = a ? to_f32(a[t * H + i]) * (s1 ? s1[i] : 1.f) : 0.f;
-  float f = 0.f;
+  float res[VEC], m[VEC] = {}, f[VEC] = {}, x[VEC], sc[VEC];
+  load_row<VEC>(residual + t * H + i, res);
+  if (a) {
+    load_row<VEC>(a + t * H + i, x);
+    if (s1) load_row<VEC>(s1 + i, sc);
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) m[e] = x[e] * (s1 ? sc[e] : 1.f);
+  }
   bool has_f = false;
   if (dense) {
-    f = to_f32(dense[t * H + i]);
+    load_row<VEC>(dense + t * H + i, f);
     has_f = true;
   } else if (y) {
-    for (int j = 0; j < k; ++j) f += w[t * k + j] * to_f32(y[(t * k + j) * H + i]);
+#pragma unroll 4
+    for (int j = 0; j < k; ++j) {
+      load_row<VEC>(y + (t * k + j) * H + i, x);
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) f[e] += w[t * k + j] * x[e];
+    }
     if (shared) {
       const float g = gate ? 1.f / (1.f + expf(-gate[t * gate_stride])) : 1.f;
-      f += g * to_f32(shared[t * H + i]);
+      load_row<VEC>(shared + t * H + i, x);
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) f[e] += g * x[e];
     }
     has_f = true;
   }
-  if (has_f) m += f * (s2 ? s2[i] : 1.f);
-  residual[t * H + i] += m;
+  if (has_f) {
+    if (s2) load_row<VEC>(s2 + i, sc);
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) m[e] += f[e] * (s2 ? sc[e] : 1.f);
+  }
+#pragma unroll
+  for (int e = 0; e < VEC; ++e) res[e] += m[e];
+  store_row<VEC>(residual + t * H + i, res);
 }
 
 // What the gated sum adds: residual[t,c] += mult (c1(t,c) a[t,c] + c2(t,c) f(t,c)) in 32-bit,
@@ -114,36 +136,46 @@ struct GatedSumArgs {
   float mult;
 };
 
-template <typename T>
+template <typename T, int VEC>
 __global__ void gated_sum_add_kernel(GatedSumArgs p) {
   const int64_t t = blockIdx.x;
-  const int i = blockIdx.y * blockDim.x + threadIdx.x;
+  const int i = VEC * (blockIdx.y * blockDim.x + threadIdx.x);
   const int H = p.H;
   if (i >= H) return;
-  float m = 0.f;
+  float res[VEC], m[VEC] = {}, f[VEC] = {}, x[VEC], g[VEC], b[VEC];
+  load_row<VEC>(p.residual + t * H + i, res);
+  auto gated = [&](float (&v)[VEC], const void* logits, const float* bias) {
+    load_row<VEC>((const T*)logits + t * H + i, g);
+    if (bias) load_row<VEC>(bias + i, b);
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) v[e] *= 1.f / (1.f + expf(-(g[e] + (bias ? b[e] : 0.f))));
+  };
   if (p.a) {
-    m = to_f32(((const T*)p.a)[t * H + i]);
-    if (p.g1) m *= 1.f / (1.f + expf(-(to_f32(((const T*)p.g1)[t * H + i]) + (p.b1 ? p.b1[i] : 0.f))));
+    load_row<VEC>((const T*)p.a + t * H + i, m);
+    if (p.g1) gated(m, p.g1, p.b1);
   }
-  float f = 0.f;
   bool has_f = false;
   if (p.dense) {
-    f = to_f32(((const T*)p.dense)[t * H + i]);
+    load_row<VEC>((const T*)p.dense + t * H + i, f);
     has_f = true;
   } else if (p.y) {
-    const T* y = (const T*)p.y;
+#pragma unroll 4
     for (int j = 0; j < p.k; ++j) {
       const bool back = p.ids && p.ids[t * p.k + j] >= p.real;
-      const float v = back ? to_f32(((const T*)p.xin)[t * H + i]) : to_f32(y[(t * p.k + j) * H + i]);
-      f = fmaf(p.w[t * p.k + j], v, f);
+      load_row<VEC>(back ? (const T*)p.xin + t * H + i : (const T*)p.y + (t * p.k + j) * H + i, x);
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) f[e] = fmaf(p.w[t * p.k + j], x[e], f[e]);
     }
     has_f = true;
   }
   if (has_f) {
-    if (p.g2) f *= 1.f / (1.f + expf(-(to_f32(((const T*)p.g2)[t * H + i]) + (p.b2 ? p.b2[i] : 0.f))));
-    m += f;
+    if (p.g2) gated(f, p.g2, p.b2);
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) m[e] += f[e];
   }
-  p.residual[t * H + i] += p.mult * m;
+#pragma unroll
+  for (int e = 0; e < VEC; ++e) res[e] += p.mult * m[e];
+  store_row<VEC>(p.residual + t * H + i, res);
 }
 
 // x <- cap * tanh(x / cap), in place (32-bit numbers).
@@ -214,15 +246,21 @@ extern "C" int ninfer_scaled_sum_add(float* residual, const void* a, const float
   NINFER_REQUIRE(dtype == kF32 || dtype == kBF16, "scaled_sum_add: unknown dtype %d", dtype);
   NINFER_REQUIRE(!(dense && y), "scaled_sum_add: dense rows or a weighted sum, not both");
   NINFER_REQUIRE(!y || (w && k > 0), "scaled_sum_add: a weighted sum needs weights and k=%d > 0", k);
-  dim3 grid(T, (H + 255) / 256);
-  if (dtype == kF32)
-    scaled_sum_add_kernel<float><<<grid, 256, 0, stream>>>(
-        residual, (const float*)a, s1, (const float*)dense, (const float*)y, w, k,
-        (const float*)shared, gate, gate_stride, s2, H);
-  else
-    scaled_sum_add_kernel<bf16><<<grid, 256, 0, stream>>>(
-        residual, (const bf16*)a, s1, (const bf16*)dense, (const bf16*)y, w, k,
-        (const bf16*)shared, gate, gate_stride, s2, H);
+  bool wide = H % 4 == 0;
+  for (const void* p : {(const void*)residual, a, (const void*)s1, dense, y, shared, (const void*)s2})
+    wide = wide && row_aligned(p);
+  const int per = wide ? 4 : 1;
+  const dim3 grid(T, (H / per + 255) / 256);
+#define NINFER_SCALED_SUM(TYPE, VEC)                                                                  \
+  scaled_sum_add_kernel<TYPE, VEC><<<grid, 256, 0, stream>>>(                                         \
+      residual, (const TYPE*)a, s1, (const TYPE*)dense, (const TYPE*)y, w, k, (const TYPE*)shared,    \
+      gate, gate_stride, s2, H)
+  if (dtype == kF32) {
+    if (wide) NINFER_SCALED_SUM(float, 4); else NINFER_SCALED_SUM(float, 1);
+  } else {
+    if (wide) NINFER_SCALED_SUM(bf16, 4); else NINFER_SCALED_SUM(bf16, 1);
+  }
+#undef NINFER_SCALED_SUM
   NINFER_LAUNCH_CHECK();
   return 0;
 }
@@ -235,9 +273,19 @@ extern "C" int ninfer_gated_sum_add(const GatedSumArgs* p, hipStream_t stream) {
   NINFER_REQUIRE(!p->ids || (p->xin && p->real >= 0), "gated_sum_add: experts that hand their input "
                  "back need that input");
   NINFER_REQUIRE(p->mult == p->mult, "gated_sum_add: the multiplier is no number");
-  dim3 grid(p->T, (p->H + 255) / 256);
-  if (p->dtype == kF32) gated_sum_add_kernel<float><<<grid, 256, 0, stream>>>(*p);
-  else gated_sum_add_kernel<bf16><<<grid, 256, 0, stream>>>(*p);
+  bool wide = p->H % 4 == 0;
+  for (const void* q : {(const void*)p->residual, p->a, p->g1, (const void*)p->b1, p->dense, p->y, p->xin, p->g2,
+                        (const void*)p->b2})
+    wide = wide && row_aligned(q);
+  const int per = wide ? 4 : 1;
+  const dim3 grid(p->T, (p->H / per + 255) / 256);
+  if (p->dtype == kF32) {
+    if (wide) gated_sum_add_kernel<float, 4><<<grid, 256, 0, stream>>>(*p);
+    else gated_sum_add_kernel<float, 1><<<grid, 256, 0, stream>>>(*p);
+  } else {
+    if (wide) gated_sum_add_kernel<bf16, 4><<<grid, 256, 0, stream>>>(*p);
+    else gated_sum_add_kernel<bf16, 1><<<grid, 256, 0, stream>>>(*p);
+  }
   NINFER_LAUNCH_CHECK();
   return 0;
 }

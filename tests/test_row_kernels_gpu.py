@@ -1,0 +1,65 @@
+"""Row kernels in whole 16-byte pieces against the same kernels number by number (operands that do
+not lie at multiples of 16 bytes): the same sums in the same order, so the same bits."""
+import pytest
+import torch
+
+import util
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from ninfer_amd.kernels import load_ops
+    return load_ops()
+
+
+def shifted(x):
+    """The same numbers one element behind a multiple of 16 bytes."""
+    buf = torch.empty(x.numel() + 1, dtype=x.dtype, device=x.device)
+    y = buf[1:].view(x.shape)
+    y.copy_(x)
+    return y
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("taps", [2, 3, 4])
+@pytest.mark.parametrize("width", [4, 1028])
+@pytest.mark.parametrize("seqs", [[(0, 1)], [(0, 1), (7, 1), (2, 1)], [(0, 2), (3, 1), (0, 5)], [(5, 255), (0, 2)],
+                                  [(0, 254), (9, 1), (0, 6)]])
+def test_short_conv(ops, dtype, taps, width, seqs):
+    g = torch.Generator(DEV).manual_seed(taps * width + len(seqs))
+    ctx = util.make_context(ops, dtype, seqs)
+    x = torch.randn(ctx.T, width, generator=g, device=DEV)
+    w = torch.randn(width, taps, generator=g, device=DEV)
+    first = torch.randn(len(seqs) + 1, (taps - 1) * width, generator=g, device=DEV)
+    states, outs = [first.clone(), shifted(first)], []
+    for state, xs in zip(states, (x, shifted(x))):
+        outs.append(torch.empty(ctx.T, width, dtype=dtype, device=DEV))
+        ops.short_conv(xs, w, state, ctx, outs[-1])
+    assert torch.equal(outs[0], outs[1])
+    assert torch.equal(states[0], states[1]) and torch.equal(states[0][-1], first[-1])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("width", [4, 1028])
+@pytest.mark.parametrize("k", [0, 1, 5])
+def test_sums(ops, dtype, width, k):
+    from ninfer_amd.parts import PendingRows
+    g = torch.Generator(DEV).manual_seed(width + k)
+    t = 9
+    rnd = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    x, s1, s2, wts, gate = rnd(t, width), rnd(width), rnd(width), rnd(t, max(k, 1)), rnd(t)
+    a, sh, dense, g1, g2 = (rnd(t, width).to(dtype) for _ in range(5))
+    y = rnd(t * max(k, 1), width).to(dtype)
+    got = []
+    for at in (lambda v: v, shifted):
+        f = PendingRows(at(y), wts, at(sh), gate) if k else at(dense)
+        res = at(x.clone())
+        ops.scaled_sum_add(res, at(a), at(s1), f, at(s2))
+        gated = at(x.clone())
+        ops.gated_sum_add(gated, at(a), at(g1), at(s1), PendingRows(at(y), wts) if k else at(dense), at(g2), at(s2), 0.7)
+        got.append((res, gated))
+    for u, v in zip(*got):
+        assert torch.equal(u, v) and not torch.equal(u, x)
