@@ -83,6 +83,8 @@ struct GemmArgs {
                          // the shape allows, -1 = never
   float act_limit;       // kEpilogueClampedSwish: the range both halves are cut to (> 0)
   float act_alpha;       // kEpilogueClampedSwish: the factor on the gate inside the sigmoid
+  int beside;            // other products run at the same time on another stream (they fill the
+                         // units that a last round leaves idle)
 };
 
 // Which rows does tile `ti` of the grouped enumeration cover? Tiles of

@@ -21,20 +21,12 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 // the other feature tiles; every (expert, feature tile) panel of W is read by
 // one block and streams from HBM whatever the order. The launcher rounds the
 // row tiles up to a multiple of 8, which makes this a bijection.
-__device__ inline void block_to_tile(bool grouped, int& bx, int& by) {
-  if (grouped) {
-    const int id = blockIdx.x + gridDim.x * blockIdx.y;
-    const int x = id % kXcds, slot = id / kXcds;
-    bx = x + kXcds * (slot / (int)gridDim.y);
-    by = slot % (int)gridDim.y;
-    return;
-  }
-  const int total = gridDim.x * gridDim.y;
-  const int id = blockIdx.x + gridDim.x * blockIdx.y;
+__device__ inline int spread_over_xcds(int id, int total) {
   // ids congruent to x mod 8 number total / 8 (one more for x < total % 8): a bijection
-  const int x = id % kXcds, q = total / kXcds, rem8 = total % kXcds;
-  const int w = x * q + min(x, rem8) + id / kXcds;
-  const int nt = gridDim.y, mt = gridDim.x;
+  const int x = id % kXcds;
+  return x * (total / kXcds) + min(x, total % kXcds) + id / kXcds;
+}
+__device__ inline void dense_tile(int w, int mt, int nt, int& bx, int& by) {   // w-th of mt x nt
   const int chunk = w / (4 * nt), rem = w % (4 * nt);
   const int full = mt / 4;   // chunks of four row tiles; the rest is walked one by one
   if (chunk < full) {
@@ -45,6 +37,16 @@ __device__ inline void block_to_tile(bool grouped, int& bx, int& by) {
     by = w2 / left;
     bx = full * 4 + w2 % left;
   }
+}
+__device__ inline void block_to_tile(bool grouped, int& bx, int& by) {
+  const int id = blockIdx.x + gridDim.x * blockIdx.y;
+  if (grouped) {
+    const int x = id % kXcds, slot = id / kXcds;
+    bx = x + kXcds * (slot / (int)gridDim.y);
+    by = slot % (int)gridDim.y;
+    return;
+  }
+  dense_tile(spread_over_xcds(id, gridDim.x * gridDim.y), gridDim.x, gridDim.y, bx, by);
 }
 
 // The rows of A of tile bx: {first row, end of the rows it may take}, and the

@@ -254,12 +254,31 @@ static int launch_tile(const GemmArgs& a, hipStream_t stream) {
   return 0;
 }
 
+// What a dense product takes in tiles of 128 x 128 (two blocks a CU side by side) and of 256 x 256
+// (one a CU, the last round cut into lower blocks: gemm_tile_direct), in us on this part. Measured
+// on gated products of 300 to 2,048 rows with 2 x 2,816 and 2 x 5,632 features and K 1,024 and
+// 2,048; at K 2,048, 128 rows against 256: 640 rows of 2 x 5,632 48 and 51, 768 69 and 52, 1,024 73
+// and 54, 1,116 87 and 71, 2,048 137 and 119; 1,280 of 2 x 2,816 49 and 49, 1,531 72 and 51. (256-row
+// tiles used to be taken from as many tiles as CUs on.)
+static float dense_us_128(int blocks, int cus, int K) {
+  float rounds = blocks / (2.f * cus);
+  const float last = rounds - floorf(rounds);
+  if (rounds > 1.f && last > 0.f && last < 0.3f) rounds += 0.3f - last;   // a short last round is not cheap
+  return 2.f + K * (0.0049f + 0.022f * rounds);
+}
+static float dense_us_256(int tiles, int cus, int K) {
+  const float round = 8.f + 0.0215f * K;                 // of up to three quarters of the CUs
+  if (4 * tiles <= 3 * cus) return round;
+  const int whole = tiles / cus, last = tiles % cus;
+  return round * (1.37f * whole + (last == 0 ? 0.f : 4 * last <= cus ? 0.65f : 2 * last <= cus ? 0.95f : 1.37f));
+}
+
 int gemm_tile(const GemmArgs& a, hipStream_t stream) {
   // Tile height. Grouped: the tall tile (it loads and multiplies only the 32-row blocks that
   // hold rows, so it beats the lower ones from 17 rows per expert on, the fewest that come
-  // here). Dense: the tallest tile that still gives every CU a block (taller tiles read less
-  // per product, but fewer of them fill the chip). force_kernel (tests) forces 64, 128 or
-  // 256 rows.
+  // here). Dense: 64 rows while taller tiles would leave CUs without a block, else 128 or 256 by
+  // an estimate of both times (dense_us_128, dense_us_256). force_kernel (tests) forces 64, 128
+  // or 256 rows.
   int rows;
   if (a.force_kernel >= 1 && a.force_kernel <= 3) {
     rows = 32 << a.force_kernel;
@@ -269,9 +288,11 @@ int gemm_tile(const GemmArgs& a, hipStream_t stream) {
     const int n_units = epilogue_gated(a.epilogue) ? 2 * a.N : a.N;   // W rows
     auto blocks = [&](int tm, int tn) { return ((a.M + tm - 1) / tm) * ((n_units + tn - 1) / tn); };
     const int cus = device_cu_count();
-    rows = blocks(256, 256) >= cus ? 256 : blocks(128, 128) >= cus ? 128 : 64;
+    rows = blocks(128, 128) >= cus ? 128 : 64;
     if (a.M <= 64) rows = 64;           // and no taller than the rows there are
-    else if (a.M <= 128 && rows > 128) rows = 128;
+    else if (a.M > 128 && rows == 128 &&
+             dense_us_256(blocks(256, 256), cus, a.K) < dense_us_128(blocks(128, 128), cus, a.K))
+      rows = 256;
   }
   if (rows == 256) return gemm_tile_direct(a, stream);
   if (rows == 128) return launch_tile<128, 128, 64, 4, 2, 2>(a, stream);

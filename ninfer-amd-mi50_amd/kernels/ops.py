@@ -39,7 +39,8 @@ class _GemmArgs(ctypes.Structure):
                 ("k_parts", ctypes.c_int), ("workspace", ctypes.c_void_p),
                 ("workspace_floats", ctypes.c_int64), ("split_min_bytes", ctypes.c_int64),
                 ("force_kernel", ctypes.c_int), ("skinny_two", ctypes.c_int),
-                ("act_limit", ctypes.c_float), ("act_alpha", ctypes.c_float)]
+                ("act_limit", ctypes.c_float), ("act_alpha", ctypes.c_float),
+                ("beside", ctypes.c_int)]
 
 
 class _RouteArgs(ctypes.Structure):
@@ -308,12 +309,14 @@ class _Beside:
             ops.join()
         ops._ok(ops.lib.ninfer_stream_after(ops._side.cuda_stream, raw, ops._side_events[0]))
         torch.cuda.set_stream(ops._side)
+        ops._side_inside = True
         return self
 
     def __exit__(self, exc_type, exc, tb):
         # nothing is given to the second stream outside such blocks: the event that marks the
         # block's end is recorded by `join()`, together with the wait for it
         torch.cuda.set_stream(self.ops._main)
+        self.ops._side_inside = False
         self.ops._side_open = True
         return False
 
@@ -353,6 +356,7 @@ class HipOps:
         self._held_route = None     # ... and a routing by the logits one of them writes
         self._side = None           # the second stream of `beside()`, made at first use
         self._side_events = None    # (start, end) of the `beside()` block
+        self._side_inside = False   # inside a `beside()` block
         self._side_open = False     # a `beside()` block that `join()` has not waited for
         self._main = None           # the stream that the last `beside()` block left and returns to
         # rows from which independent work is worth a second stream (with fewer rows the
@@ -667,6 +671,7 @@ class HipOps:
         args.split_min_bytes = self._tune["split_min_bytes"]
         args.skinny_two = self._tune["skinny_two"]
         args.act_limit, args.act_alpha = float(act_limit), float(act_alpha)
+        args.beside = 1 if self._side_inside or self._side_open else 0
         if only_if_split:
             # a dense product of few dozen rows: the library's unless the kernels here cut it
             # along K (its output tiles alone would not fill the GPU). The one workspace of
