@@ -29,9 +29,9 @@
 //                    tiles are shared out evenly over its chunks.
 //
 // Latent 512 + 64, 16 heads, against blocks of four waves and 32 rows with the queries in LDS and the
-// values gathered by two-byte reads: a 2,048-token prompt 688 -> 209 us (73 GFLOP, 350 TFLOP/s; the
+// values gathered by two-byte reads: a 2,048-token prompt 688 -> 203 us (73 GFLOP, 360 TFLOP/s; the
 // LDS traffic alone, 3,000 cycles a tile of 64 keys, is 42 us), 64 requests at 1,950 to 2,600 keys
-// 188 -> 59 us (168 MB, 2.8 TB/s: a tile's way into the CU and four barriers, 6.5 us a tile).
+// 188 -> 48 us (168 MB, 3.5 TB/s: a tile's way through LDS and four barriers, about 5 us a tile).
 //
 // The rotation turns pair (i, i + n/2), or with `interleaved` pair (2i, 2i + 1), of the first
 // n = rot_n numbers of the rotated part by pos * freq[i]; cosine and sine are multiplied by `magnitude` (1 without a scaled table).
@@ -342,13 +342,20 @@ __global__ __launch_bounds__(kLatThreads, 2) void latent_attention_tile_kernel(L
   float* alpha_s = (float*)(Ps + ROWS * kLatPRow);              // [ROWS], then m and l
   float* m_s = alpha_s + ROWS;
   float* l_s = m_s + ROWS;
+  __shared__ int page_s[2][kLatKeys];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
 
   // Which request and which of its row tiles is this block's? The tiles are dealt out from
   // the last one backwards: within a request the later tiles see more keys and run longer,
   // and the long ones should start first.
   int s = -1, lt = 0;
-  {
+  if (a.max_qlen == 1) {   // every request has one row's tiles: no walk over the requests
+    const int nt = (H + ROWS - 1) / ROWS, from_last = (int)blockIdx.x;
+    if (from_last < a.S * nt) {
+      s = a.S - 1 - from_last / nt;
+      lt = nt - 1 - from_last % nt;
+    }
+  } else {
     int total = 0;
     for (int i = 0; i < a.S; ++i)
       total += ((a.seq_row_start[i + 1] - a.seq_row_start[i]) * H + ROWS - 1) / ROWS;
@@ -394,11 +401,13 @@ __global__ __launch_bounds__(kLatThreads, 2) void latent_attention_tile_kernel(L
     const int e = min(tid + kLatThreads * i, kLatKeys * cpr - 1);
     piece[i] = ((e / cpr) << 16) | (8 * (e % cpr));
   }
-  auto fetch = [&](int kt) {
+  // The pages of a tile's keys come through LDS, looked up two tiles ahead by one wave: a wave's loads
+  // return in order, and an address that waits for the block table would wait for the tile before.
+  auto page_of = [&](int kt) { return bt[min(max(kt + lane, lo_first), pos_last) >> pl.page_shift]; };
+  auto fetch = [&](int kt, const int* pages) {
     int page[PIECES];
 #pragma unroll
-    for (int i = 0; i < PIECES; ++i)
-      page[i] = bt[min(max(kt + (piece[i] >> 16), lo_first), pos_last) >> pl.page_shift];
+    for (int i = 0; i < PIECES; ++i) page[i] = pages[piece[i] >> 16];
 #pragma unroll
     for (int i = 0; i < PIECES; ++i) {
       const int kp = min(max(kt + (piece[i] >> 16), lo_first), pos_last);
@@ -406,7 +415,14 @@ __global__ __launch_bounds__(kLatThreads, 2) void latent_attention_tile_kernel(L
                                      (piece[i] & 0xffff));
     }
   };
-  if (k_begin < k_end) fetch(k_begin);
+  int page_next = 0;   // wave 0: the page of key `lane`, two tiles ahead
+  if (w == 0 && k_begin < k_end) {
+    page_s[0][lane] = page_of(k_begin);
+    page_s[1][lane] = page_of(k_begin + kLatKeys);
+    page_next = page_of(k_begin + 2 * kLatKeys);
+  }
+  __syncthreads();
+  if (k_begin < k_end) fetch(k_begin, page_s[0]);
 
   // Q' as the products' operand, rounded to bfloat16 once; zeros beyond the row's numbers. In the
   // wide form wave w has rows 32 (w / 4) .., keys 32 (w / 2 % 2) .. and one half of the numbers;
@@ -452,12 +468,15 @@ __global__ __launch_bounds__(kLatThreads, 2) void latent_attention_tile_kernel(L
     for (int rt = 0; rt < RT; ++rt) acc[ct][rt] = lat_f32x4{0.f, 0.f, 0.f, 0.f};
   const int c = lane & 15, g = lane >> 4;
 
-  for (int kt = k_begin; kt < k_end; kt += kLatKeys) {
+  int turn = 0;   // of the two places for pages: this tile's, where those two tiles ahead go
+  for (int kt = k_begin; kt < k_end; kt += kLatKeys, turn ^= 1) {
     // 1. the tile's keys into LDS as they lie in their pages
 #pragma unroll
     for (int i = 0; i < PIECES; ++i)
       *(lat_bf16x8*)(Ks + (piece[i] >> 16) * KROW + (piece[i] & 0xffff)) = next[i];
-    if (kt + kLatKeys < k_end) fetch(kt + kLatKeys);
+    if (w == 0) page_s[turn][lane] = page_next;
+    if (kt + kLatKeys < k_end) fetch(kt + kLatKeys, page_s[turn ^ 1]);
+    if (w == 0) page_next = page_of(kt + 3 * kLatKeys);
     lds_barrier();   // (orders LDS traffic only: the next tile's loads stay under way)
     // 2. scores over one half of the numbers
     float* sp = Sp + kh * ROWS * kLatKeys;

@@ -329,12 +329,14 @@ __global__ __launch_bounds__(kSgThreads) void sigmoid_attention_tiles_kernel(Sig
   }
 }
 
-// out[t, e] = sum over the splits, in their order.
+// out[t, e] = sum over the splits, in their order; several splits' loads under way together (34
+// splits of 8 rows with 16 heads of 128: 11.0 -> 4.7 us).
 __global__ void sigmoid_attention_sum_kernel(const float* __restrict__ part, __hip_bfloat16* __restrict__ out,
                                              int64_t n, int n_splits) {
   const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
   if (i >= n) return;
   float4 s = *(const float4*)(part + i);
+#pragma unroll 8
   for (int k = 1; k < n_splits; ++k) {
     const float4 x = *(const float4*)(part + k * n + i);
     s.x += x.x, s.y += x.y, s.z += x.z, s.w += x.w;
@@ -391,7 +393,8 @@ static int launch_sig_tiles(const SigAttnArgs& a, float* part, int n_splits, hip
   NINFER_LAUNCH_CHECK();
   if (part) {
     const int64_t n = (int64_t)a.T * a.Hq * a.vdim;
-    sigmoid_attention_sum_kernel<<<(unsigned)((n / 4 + 255) / 256), 256, 0, stream>>>(
+    const int block = n / 4 < 256 * (int64_t)device_cu_count() ? 64 : 256;   // few rows: more blocks than CUs sooner
+    sigmoid_attention_sum_kernel<<<(unsigned)((n / 4 + block - 1) / block), block, 0, stream>>>(
         part, (__hip_bfloat16*)a.out, n, n_splits);
     NINFER_LAUNCH_CHECK();
   }
