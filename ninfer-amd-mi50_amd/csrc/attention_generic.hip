@@ -20,7 +20,10 @@ namespace ninfer {
 
 constexpr int kMaxDPerLane = 8;  // head sizes up to 512
 
-template <typename T>
+// PIECES: a key's row is whole pieces of 16 bytes, which a lane loads one by one (its key lies in a
+// line of its own: four numbers of 32-bit a load instead of one. 173 rows of 16 heads of 128 in
+// 32-bit, a prompt of its own: 109 -> 41 us).
+template <typename T, bool PIECES>
 __global__ __launch_bounds__(64) void paged_attention_generic_kernel(AttnArgs a) {
   extern __shared__ float smem[];
   const int D = a.D, Dv = a.Dv, Hkv = a.Hkv;
@@ -54,8 +57,19 @@ __global__ __launch_bounds__(64) void paged_attention_generic_kernel(AttnArgs a)
         int page = bt[j / page_size];
         off = ((int64_t)page * Hkv + g) * page_size + (j % page_size);
         const T* kr = kpool + off * D;
-        float dot = 0.f;
-        for (int d = 0; d < D; ++d) dot = fmaf(q_s[d], to_f32(kr[d]), dot);
+        float dot = 0.f;   // (d ascending in both forms: the same bits)
+        if (PIECES) {
+          constexpr int N = 16 / sizeof(T);
+#pragma unroll 4
+          for (int d = 0; d < D; d += N) {
+            union { uint4 u; T x[N]; } k;
+            k.u = *(const uint4*)(kr + d);
+#pragma unroll
+            for (int e = 0; e < N; ++e) dot = fmaf(q_s[d + e], to_f32(k.x[e]), dot);
+          }
+        } else {
+          for (int d = 0; d < D; ++d) dot = fmaf(q_s[d], to_f32(kr[d]), dot);
+        }
         s = fmaf(slope, (float)(j - pos), dot * a.scale);
       }
       float m_new = fmaxf(m, wave_max(s));
@@ -73,6 +87,7 @@ __global__ __launch_bounds__(64) void paged_attention_generic_kernel(AttnArgs a)
         int d = lane + i * 64;
         if (d < Dv) {
           float x = acc[i] * alpha;
+#pragma unroll 8
           for (int jj = first; jj < n_keys; ++jj) x = fmaf(p_s[jj], to_f32(vpool[off_s[jj] * Dv + d]), x);
           acc[i] = x;
         }
@@ -107,8 +122,15 @@ int attention_generic(const AttnArgs& args, hipStream_t stream) {
                  "paged_attention: head sizes %d, %d exceed %d", a.D, a.Dv, 64 * kMaxDPerLane);
   dim3 grid(a.T, a.Hq);
   size_t lds = (a.D + 64) * sizeof(float) + 64 * sizeof(int64_t);
-  if (a.dtype == kF32) paged_attention_generic_kernel<float><<<grid, 64, lds, stream>>>(a);
-  else paged_attention_generic_kernel<bf16><<<grid, 64, lds, stream>>>(a);
+  const bool pieces = a.D % (a.dtype == kF32 ? 4 : 8) == 0 &&
+                      ((uintptr_t)a.kpool | (a.kblk ? (uintptr_t)a.kblk : 0)) % 16 == 0;
+  if (a.dtype == kF32) {
+    if (pieces) paged_attention_generic_kernel<float, true><<<grid, 64, lds, stream>>>(a);
+    else paged_attention_generic_kernel<float, false><<<grid, 64, lds, stream>>>(a);
+  } else {
+    if (pieces) paged_attention_generic_kernel<bf16, true><<<grid, 64, lds, stream>>>(a);
+    else paged_attention_generic_kernel<bf16, false><<<grid, 64, lds, stream>>>(a);
+  }
   NINFER_LAUNCH_CHECK();
   return 0;
 }
