@@ -66,6 +66,77 @@ __global__ void lightning_seq_kernel(const T* __restrict__ qkv, int stride, int 
   for (int e = tid; e < dim * vdim; e += blockDim.x) st[e] = S[e];
 }
 
+// Steps whose requests bring a row each. What a row costs there is the state's way from memory and
+// back, which the kernel above takes through the LDS: 69 KB for a head of 128 x 128, two blocks a CU.
+// Here the state goes memory -> registers -> memory: a block owns up to 64 value columns of a head,
+// thread (part, v) the same numbers S[d][v] as above with the sums in the same order (the same
+// bits), 16 of them loaded together. A thread reads back only what it wrote, so requests of more
+// rows are right too, one trip per row. 64 requests of 16 heads of 128 x 128 (134 MB there and
+// back): 80 -> 35 us, 3.8 TB/s, bound by memory. (64 numbers loaded together: 76 us; blocks of 32
+// columns 35, of 128 41. 8 requests 12 us, one 10: four trips to memory one after the other.)
+template <typename T>
+__global__ void lightning_step_kernel(const T* __restrict__ qkv, int stride, int q_off, int k_off,
+                                      int v_off, const float* __restrict__ decay,
+                                      float* __restrict__ state, int64_t state_stride,
+                                      float* __restrict__ out, const int* __restrict__ seq_row_start,
+                                      const int* __restrict__ seq_slots, int H, int dim, int vdim,
+                                      int parts, int cols) {
+  constexpr int B = 16;
+  extern __shared__ float smem[];
+  float* q_s = smem;               // [dim]
+  float* k_s = q_s + dim;          // [dim]
+  float* part_s = k_s + dim;       // [parts * cols]
+  const int s = blockIdx.x, h = blockIdx.y;
+  const int r0 = seq_row_start[s], n = seq_row_start[s + 1] - r0;
+  const int tid = threadIdx.x;     // blockDim.x == parts * cols
+  const int part = tid / cols, vv = (int)blockIdx.z * cols + tid % cols;
+  const bool mine = vv < vdim;
+  const int col = mine ? vv : vdim - 1;   // (threads beyond the last column load, and write nothing)
+  float* st = state + (int64_t)seq_slots[s] * state_stride + (int64_t)h * dim * vdim + col;
+  const float dec = decay[h];
+  for (int i = 0; i < n; ++i) {
+    const T* row = qkv + (int64_t)(r0 + i) * stride;
+    float S[B];
+#pragma unroll
+    for (int u = 0; u < B; ++u) {   // (on their way while q and k are prepared)
+      const int d = part + u * parts;
+      S[u] = st[(int64_t)(d < dim ? d : dim - 1) * vdim];
+    }
+    const float v_t = silu_f(to_f32(row[v_off + h * vdim + col]));
+#pragma unroll 4
+    for (int e = tid; e < 2 * dim; e += blockDim.x)
+      q_s[e] = silu_f(to_f32(row[e < dim ? q_off + h * dim + e : k_off + h * dim + (e - dim)]));
+    __syncthreads();   // q and k are in LDS; the sums of the previous row have been added
+    float acc = 0.f;
+    for (int d0 = part; d0 < dim; d0 += B * parts) {
+      if (d0 != part) {
+#pragma unroll
+        for (int u = 0; u < B; ++u) {
+          const int d = d0 + u * parts;
+          S[u] = st[(int64_t)(d < dim ? d : dim - 1) * vdim];
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < B; ++u) {
+        const int d = d0 + u * parts;
+        if (d < dim) {
+          const float sn = fmaf(dec, S[u], k_s[d] * v_t);
+          if (mine) st[(int64_t)d * vdim] = sn;
+          acc = fmaf(sn, q_s[d], acc);
+        }
+      }
+    }
+    part_s[tid] = acc;
+    __syncthreads();
+    if (part == 0 && mine) {
+      float o = 0.f;
+      for (int p = 0; p < parts; ++p) o += part_s[p * cols + tid];
+      out[((int64_t)(r0 + i) * H + h) * vdim + vv] = o;
+    }
+    // (part_s is written again only after the next row's first barrier)
+  }
+}
+
 }  // namespace ninfer
 
 using namespace ninfer;
@@ -94,6 +165,20 @@ extern "C" int ninfer_lightning_attention(const void* qkv, int stride, int q_off
   NINFER_REQUIRE(lds <= 160 * 1024, "lightning_attention: a head's state of %d x %d does not fit "
                  "the LDS", dim, vdim);
   const dim3 grid(S, H);
+  // (a row per request as a rule; more rows than requests go through the LDS: one trip for all rows)
+  if (T <= S) {
+    const int cols = vdim < 64 ? vdim : 64;
+    const dim3 grid(S, H, (vdim + cols - 1) / cols);
+    const size_t bytes = (2 * (size_t)dim + (size_t)parts * cols) * sizeof(float);
+#define NINFER_LIGHTNING_STEP(TYPE)                                                             \
+  lightning_step_kernel<TYPE><<<grid, parts * cols, bytes, stream>>>(                           \
+      (const TYPE*)qkv, stride, q_off, k_off, v_off, decay, state, state_stride, out,           \
+      seq_row_start, seq_slots, H, dim, vdim, parts, cols)
+    if (dtype == kF32) NINFER_LIGHTNING_STEP(float); else NINFER_LIGHTNING_STEP(bf16);
+#undef NINFER_LIGHTNING_STEP
+    NINFER_LAUNCH_CHECK();
+    return 0;
+  }
 #define NINFER_LIGHTNING_LAUNCH(TYPE)                                                          \
   do {                                                                                         \
     auto kern = lightning_seq_kernel<TYPE>;                                                    \

@@ -196,6 +196,39 @@ def test_lightning_chunks_of_aligned_rows(ops, heads, dim, vdim, lens):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("heads,dim,vdim", [(2, 128, 128), (1, 64, 64), (3, 16, 24), (2, 33, 40), (1, 5, 300),
+                                            (1, 130, 256), (2, 1, 1)])
+def test_lightning_a_row_per_request(ops, dtype, heads, dim, vdim):
+    """Steps of no more rows than requests keep the state in registers: the same bits, row by row, as
+    the walk that holds it in LDS (which steps of more rows than requests take)."""
+    torch.manual_seed(dim + vdim)
+    qk, vw = heads * dim, heads * vdim
+    x = torch.randn(12, 2 * qk + vw + 3).to(dtype).to(DEV)
+    state = torch.randn(8, heads * dim * vdim + 5).to(DEV)
+    dec = torch.tensor([0.97, 0.0, 1.0][:heads], device=DEV)
+
+    def run(rows, counts, st):
+        ctx = util.make_context(ops, dtype, [(0, n) for n in counts])
+        out = torch.full((len(rows), vw), 7.0, device=DEV)
+        ops.lightning_attention(x[rows].contiguous(), 3, 3 + qk, 3 + 2 * qk, heads, dim, vdim, dec, st, ctx, out)
+        return out, ctx.seq_slots.cpu().tolist()
+
+    whole, parts = state.clone(), state.clone()
+    want, slots = run([0, 1, 2, 3, 4, 5, 6, 7, 8], [3, 3, 3], whole)
+    for i in range(3):
+        got, at = run([i, 3 + i, 6 + i], [1, 1, 1], parts)
+        assert at == slots and torch.equal(got, want[i::3])
+    assert torch.equal(whole, parts) and not torch.equal(whole, state)
+    # as many rows as requests, unevenly: two rows of one, none of another
+    whole, parts = state.clone(), state.clone()
+    want, _ = run([0, 1, 2, 9, 10, 11], [3, 0, 3], whole)
+    got, _ = run([0, 1, 9], [2, 0, 1], parts)
+    assert torch.equal(got, want[[0, 1, 3]])
+    got, _ = run([2, 10, 11], [1, 0, 2], parts)
+    assert torch.equal(got, want[[2, 4, 5]]) and torch.equal(whole, parts)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("heads,k,n", [(3, 24, 40), (4, 64, 160), (1, 16, 32), (5, 40, 20), (2, 12, 10)])
 @pytest.mark.parametrize("rows", [1, 7, 70])
 def test_per_head_linear(ops, dtype, heads, k, n, rows):
