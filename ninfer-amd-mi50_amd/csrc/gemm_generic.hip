@@ -2,8 +2,8 @@
 // the plain tiled kernel of the product family. 32-bit accumulation by FMA in
 // a fixed order (k ascending) for every output element, whatever M is and
 // wherever the row sits in its tile, so a row's result does not depend on the
-// batch it came in. This is the kernel of the true 32-bit path and the
-// fallback of the bf16 path for shapes its MFMA kernels refuse.
+// batch it came in. This is the fallback for operands that the matrix-core
+// kernels refuse (32-bit: rows that are no whole 16-byte pieces).
 //
 // Linear weights are [out, in] row-major, y = x W^T, as in the reference
 // (src/ops/ops.h:16-18). Grouped form: sorted row r belongs to the expert g
