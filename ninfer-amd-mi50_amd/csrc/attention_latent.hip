@@ -468,6 +468,9 @@ __global__ __launch_bounds__(kLatThreads, 2) void latent_attention_tile_kernel(L
     for (int rt = 0; rt < RT; ++rt) acc[ct][rt] = lat_f32x4{0.f, 0.f, 0.f, 0.f};
   const int c = lane & 15, g = lane >> 4;
 
+  // The loop writes a place of page_s that the fetch one tile before has read, always with a barrier
+  // of that tile between the two; before the first tile this is that barrier.
+  lds_barrier();
   int turn = 0;   // of the two places for pages: this tile's, where those two tiles ahead go
   for (int kt = k_begin; kt < k_end; kt += kLatKeys, turn ^= 1) {
     // 1. the tile's keys into LDS as they lie in their pages

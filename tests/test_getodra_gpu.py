@@ -328,6 +328,58 @@ def test_latent_attention_whole_prompt_on_matrix_cores(ops, heads, rank, rd):
     assert rel_err(outs[0][:3], want[:3]) < 8e-3 and rel_err(outs[0][-1], want[-1]) < 8e-3
 
 
+# rows of a cached latent at the edges of the bfloat16 kernel's forms: up to 288, 576 and 640 numbers,
+# latents of up to 256 and 512
+# (Bounds: the queries, the probabilities and the output each round to bfloat16 once, 2^-9 at most; the
+# queries' rounding counts times the scores' size, about 2 here: 4 * 2^-9 = 8e-3.)
+LATENT_FORMS = [(256, 32), (264, 24), (288, 0), (64, 16), (256, 64), (200, 376), (512, 64), (512, 128),
+                (256, 328), (504, 80)]
+
+
+@pytest.mark.parametrize("rank,rd", LATENT_FORMS)
+@pytest.mark.parametrize("heads,window", [(16, 0), (17, 150), (1, 0)])
+def test_latent_decode_of_many_requests(ops, rank, rd, heads, window):
+    """A decode step of so many requests that a block walks all of a request's keys, six tiles and
+    more of the long ones, each of whose keys lie in pages of their own; up to 16 heads take blocks
+    of 16 rows, more of them blocks of 64. Twice: the same bits."""
+    ps = 8
+    lengths = [[1, 64, 65, 130, 191, 257, 400, 449][i % 8] for i in range(260)]
+    few = [i for i in range(260) if i < 16 or i % 37 == 0]   # (those compared with the softmax in 64 bits)
+    new_rows = [1] * len(lengths)
+    ctx, pool, table, q, cached = _latent_case(ops, torch.bfloat16, heads, rank, rd, ps, lengths, new_rows,
+                                               seed=rank + heads)
+    pool_dev, table_dev, q_dev = pool.to(torch.bfloat16).to(DEV), table.to(DEV), q.to(DEV)
+    outs = []
+    for _ in range(2):
+        out = torch.full((ctx.T, heads * rank), 7.0, dtype=torch.bfloat16, device=DEV)
+        ops.latent_attention(q_dev, pool_dev, table_dev, ctx, heads, rank, rd, ps, 0.1, out, window=window)
+        outs.append(out)
+    assert torch.equal(outs[0], outs[1])
+    got = outs[0].float().cpu().reshape(ctx.T, heads, rank)
+    want = _plain_latent_rows(q[few], [cached[i] for i in few], [lengths[i] for i in few], [1] * len(few), rank,
+                              0.1, window)
+    for i, w in zip(few, want):
+        assert rel_err(got[i], w) < 8e-3, (i, lengths[i])
+
+
+@pytest.mark.parametrize("rank,rd", LATENT_FORMS)
+@pytest.mark.parametrize("heads,new_rows", [(16, [260, 130, 64]), (40, [1, 1, 1]), (70, [1, 1, 1]), (3, [1, 90, 40])])
+def test_latent_forms(ops, rank, rd, heads, new_rows):
+    """Prompts, decode steps of more heads than a block has rows, and both in one step, with a gate:
+    every form of the bfloat16 kernel, each request's keys cut into chunks."""
+    ps, lengths = 16, [260, 131, 300]
+    ctx, pool, table, q, cached = _latent_case(ops, torch.bfloat16, heads, rank, rd, ps, lengths, new_rows,
+                                               seed=rank + heads)
+    gate = torch.randn(ctx.T, heads + 3).bfloat16()
+    out = torch.empty(ctx.T, heads * rank, dtype=torch.bfloat16, device=DEV)
+    ops.latent_attention(q.to(DEV), pool.bfloat16().to(DEV), table.to(DEV), ctx, heads, rank, rd, ps, 0.1, out,
+                         gate=gate.to(DEV)[:, 3:])
+    want = _plain_latent_rows(q, cached, lengths, new_rows, rank, 0.1, 0, gate[:, 3:].float())
+    got = out.float().cpu().reshape(ctx.T, heads, rank)
+    worst = max(rel_err(g, w) for g, w in zip(got, want))
+    assert worst < 8e-3
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("where", [0, 1, 15, 16, 63, 64, 300, 498])
 def test_latent_attention_finds_one_key(ops, dtype, where):
