@@ -378,6 +378,7 @@ __global__ __launch_bounds__(kLatThreads, 2) void latent_attention_tile_kernel(L
   const int pos0 = a.seq_pos0[s];
   const int f0 = lt * ROWS;                          // first flattened row of the tile
   const int rows_here = min(ROWS, n_flat - f0);
+  if (rows_here <= 0) return;   // (a request without rows in a decode-only step)
   const int tok_first = f0 / H, tok_last = (f0 + rows_here - 1) / H;
   const int pos_last = pos0 + tok_last;
   const int lo_first = a.window > 0 ? max(0, pos0 + tok_first - a.window + 1) : 0;

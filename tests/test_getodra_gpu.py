@@ -362,6 +362,21 @@ def test_latent_decode_of_many_requests(ops, rank, rd, heads, window):
         assert rel_err(got[i], w) < 8e-3, (i, lengths[i])
 
 
+@pytest.mark.parametrize("heads", [1, 2, 16, 17, 70])
+@pytest.mark.parametrize("new_rows", [[0, 1, 0, 1, 0], [1, 0, 0, 0, 0], [0, 0, 0, 0, 1]])
+def test_latent_decode_with_requests_without_rows(ops, heads, new_rows):
+    """Requests that bring no row to a decode-only step are passed over, the first and the last too."""
+    rank, rd, ps = 64, 16, 16
+    lengths = [70, 200, 1, 64, 130]
+    ctx, pool, table, q, cached = _latent_case(ops, torch.bfloat16, heads, rank, rd, ps, lengths, new_rows, seed=heads)
+    assert ctx.max_qlen == 1 and ctx.T == sum(new_rows)
+    out = torch.full((ctx.T + 1, heads * rank), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops.latent_attention(q.to(DEV), pool.bfloat16().to(DEV), table.to(DEV), ctx, heads, rank, rd, ps, 0.2, out[:-1])
+    want = _plain_latent_rows(q, cached, lengths, new_rows, rank, 0.2, 0)
+    assert rel_err(out[:-1].float().cpu().reshape(ctx.T, heads, rank), want) < 8e-3
+    assert (out[-1] == 7.0).all()
+
+
 @pytest.mark.parametrize("rank,rd", LATENT_FORMS)
 @pytest.mark.parametrize("heads,new_rows", [(16, [260, 130, 64]), (40, [1, 1, 1]), (70, [1, 1, 1]), (3, [1, 90, 40])])
 def test_latent_forms(ops, rank, rd, heads, new_rows):
