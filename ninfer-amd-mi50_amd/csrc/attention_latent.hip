@@ -393,7 +393,7 @@ __global__ __launch_bounds__(kLatThreads, 2) void latent_attention_tile_kernel(L
 
   // A tile's keys travel page -> registers -> LDS; the loads of the next tile are issued before
   // the products of this one. Keys outside what the rows see are fetched from the nearest that
-  // they do (their probabilities are 0), so that no load waits for a condition.
+  // they do (their probabilities are 0); keys whose page the table does not hold (-1) are zeros.
   const int cpr = Dk / 8;   // 16-byte pieces of a cached row
   lat_bf16x8 next[PIECES];
   int piece[PIECES];        // key of the tile << 16 | first number of the piece
@@ -412,8 +412,10 @@ __global__ __launch_bounds__(kLatThreads, 2) void latent_attention_tile_kernel(L
 #pragma unroll
     for (int i = 0; i < PIECES; ++i) {
       const int kp = min(max(kt + (piece[i] >> 16), lo_first), pos_last);
-      next[i] = *(const lat_bf16x8*)(pool + ((int64_t)page[i] * a.page_size + (kp & (a.page_size - 1))) * Dk +
-                                     (piece[i] & 0xffff));
+      next[i] = lat_bf16x8{};
+      if (page[i] >= 0)
+        next[i] = *(const lat_bf16x8*)(pool + ((int64_t)page[i] * a.page_size + (kp & (a.page_size - 1))) * Dk +
+                                       (piece[i] & 0xffff));
     }
   };
   int page_next = 0;   // wave 0: the page of key `lane`, two tiles ahead

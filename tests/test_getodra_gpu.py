@@ -377,6 +377,21 @@ def test_latent_decode_with_requests_without_rows(ops, heads, new_rows):
     assert (out[-1] == 7.0).all()
 
 
+@pytest.mark.parametrize("rank,rd", [(64, 16), (512, 64), (512, 128)])
+@pytest.mark.parametrize("heads,new_rows", [(16, [1, 1]), (16, [90, 1]), (40, [1, 1])])
+def test_latent_pages_that_the_table_does_not_hold(ops, rank, rd, heads, new_rows):
+    """A visible key whose page is -1 in the table counts as a row of zeros (the bfloat16 kernel)."""
+    ps, lengths = 16, [300, 150]
+    ctx, pool, table, q, cached = _latent_case(ops, torch.bfloat16, heads, rank, rd, ps, lengths, new_rows, seed=heads)
+    for i, p in ((0, 0), (0, 5), (0, 18), (1, 3)):
+        table[i, p] = -1
+        cached[i][p * ps:(p + 1) * ps] = 0
+    out = torch.empty(ctx.T, heads * rank, dtype=torch.bfloat16, device=DEV)
+    ops.latent_attention(q.to(DEV), pool.bfloat16().to(DEV), table.to(DEV), ctx, heads, rank, rd, ps, 0.1, out)
+    want = _plain_latent_rows(q, cached, lengths, new_rows, rank, 0.1, 0)
+    assert rel_err(out.float().cpu().reshape(ctx.T, heads, rank), want) < 8e-3
+
+
 @pytest.mark.parametrize("rank,rd", LATENT_FORMS)
 @pytest.mark.parametrize("heads,new_rows", [(16, [260, 130, 64]), (40, [1, 1, 1]), (70, [1, 1, 1]), (3, [1, 90, 40])])
 def test_latent_forms(ops, rank, rd, heads, new_rows):
