@@ -16,8 +16,8 @@
 //                    row's position alone. The head's output may be multiplied by
 //                    sigmoid(gate[row, head]).
 //
-//   latent_attention_tile (bfloat16, matrix cores): a block of eight waves owns 64 rows (16 in
-//                    decode-only steps) of (token, head) pairs of one request, all of which read
+//   latent_attention_tile (bfloat16, matrix cores): a block of eight waves owns 64 rows (or 16, in
+//                    steps of few rows) of (token, head) pairs of one request, all of which read
 //                    the same cached rows. Keys come in tiles of 64 through LDS as they lie in
 //                    the cache ([key][numbers]), the next tile on its way in registers; the
 //                    queries stay in registers, each wave with half of the numbers, so a key is
@@ -300,22 +300,43 @@ static bool latent_tile_takes(const LatentArgs& a) {
          ((uintptr_t)a.pool % 16 == 0) && ((uintptr_t)a.q_abs % 16 == 0);
 }
 
+// Row tiles and key chunks of a step in blocks of `rows` rows. Row tiles: in a decode-only step
+// every request has the same number; otherwise a bound (a request's last tile may be partial; tiles
+// that do not exist exit at once). A block counts on a CU of its own, with as long a walk over the
+// keys as that allows.
+static void latent_tile_split(const LatentArgs& a, int rows, int* tiles, int* n_chunks) {
+  *tiles = a.max_qlen == 1 ? a.S * ((a.Hq + rows - 1) / rows)
+                           : (int)(((int64_t)a.T * a.Hq + rows - 1) / rows) + a.S;
+  const int key_tiles = (a.max_kv_len + kLatKeys - 1) / kLatKeys;
+  int want = device_cu_count() / *tiles;
+  if (want > key_tiles) want = key_tiles;
+  *n_chunks = want < 1 ? 1 : want;
+}
+
+// What a step takes in blocks of 16 or 64 rows, in us on this part: rounds of blocks, each a start and
+// a walk over its keys, and the merge of chunks. Low blocks start sooner (queries, first tile, output:
+// 10 against 24 us at 576 numbers a row) and meet a tile of 64 keys in 0.9 us while few of them run and
+// in 2.1 when they fill the GPU (every block brings the same bytes from L2), high ones in 3.6 and for
+// four times the rows. 512 + 64 numbers, 16 heads, us in low and in high blocks: a prompt of 64 tokens 14
+// and 32 (blocks of 32 rows of four waves, the kernel before: 23), of 300 30 and 54, of 2,048 389 and
+// 188; 40 heads, 64 requests at 2,500 keys 118 and 84, at 300 26 and 44.
+static float latent_tile_us(const LatentArgs& a, int rows, int half) {
+  int tiles, n_chunks;
+  latent_tile_split(a, rows, &tiles, &n_chunks);
+  const int key_tiles = (a.max_kv_len + kLatKeys - 1) / kLatKeys, steps = (key_tiles + n_chunks - 1) / n_chunks;
+  const float filled = (float)tiles * n_chunks / device_cu_count(), numbers = half / 18.f;
+  const float start = rows == 16 ? 10.f : 24.f;
+  const float step = rows == 16 ? 0.9f + 1.2f * (filled < 1.f ? filled : 1.f) : 3.6f;
+  const float round = start * (0.4f + 0.6f * numbers) + steps * step * numbers;
+  return round * (filled > 1.f ? filled : 1.f) + (n_chunks > 1 ? 6.f : 0.f);
+}
+
 static LatentTilePlan latent_tile_plan(const LatentArgs& a) {
   LatentTilePlan p;
   const int Dk = a.R + a.rd;
   p.half = Dk <= 32 * 9 ? 9 : Dk <= 32 * 18 ? 18 : kLatMaxHalf;
-  // A decode-only step's request has as many rows as heads: up to 16 of them take a block whose
-  // products are 16 rows high and which is bound by the cached rows' way into the CU.
-  p.rows = a.max_qlen == 1 && a.Hq <= 16 ? 16 : 64;
-  // row tiles: in a decode-only step every request has the same number; otherwise a bound
-  // (a request's last tile may be partial; tiles that do not exist exit at once)
-  p.tiles = a.max_qlen == 1 ? a.S * ((a.Hq + p.rows - 1) / p.rows)
-                            : (int)(((int64_t)a.T * a.Hq + p.rows - 1) / p.rows) + a.S;
-  const int key_tiles = (a.max_kv_len + kLatKeys - 1) / kLatKeys;
-  // a block fills a CU (its LDS): one block per CU, each with as long a walk as that allows
-  int want = device_cu_count() / p.tiles;
-  if (want > key_tiles) want = key_tiles;
-  p.n_chunks = want < 1 ? 1 : want;
+  p.rows = latent_tile_us(a, 16, p.half) <= latent_tile_us(a, 64, p.half) ? 16 : 64;
+  latent_tile_split(a, p.rows, &p.tiles, &p.n_chunks);
   p.page_shift = 0;
   while ((1 << p.page_shift) < a.page_size) ++p.page_shift;
   p.lds = (size_t)kLatKeys * (32 * p.half + 8) * 2 + (size_t)2 * p.rows * kLatKeys * 4 +

@@ -340,8 +340,8 @@ LATENT_FORMS = [(256, 32), (264, 24), (288, 0), (64, 16), (256, 64), (200, 376),
 @pytest.mark.parametrize("heads,window", [(16, 0), (17, 150), (1, 0)])
 def test_latent_decode_of_many_requests(ops, rank, rd, heads, window):
     """A decode step of so many requests that a block walks all of a request's keys, six tiles and
-    more of the long ones, each of whose keys lie in pages of their own; up to 16 heads take blocks
-    of 16 rows, more of them blocks of 64. Twice: the same bits."""
+    more of the long ones, in pages of eight keys, mostly in blocks of 16 rows. Twice:
+    the same bits."""
     ps = 8
     lengths = [[1, 64, 65, 130, 191, 257, 400, 449][i % 8] for i in range(260)]
     few = [i for i in range(260) if i < 16 or i % 37 == 0]   # (those compared with the softmax in 64 bits)
@@ -356,6 +356,25 @@ def test_latent_decode_of_many_requests(ops, rank, rd, heads, window):
         outs.append(out)
     assert torch.equal(outs[0], outs[1])
     got = outs[0].float().cpu().reshape(ctx.T, heads, rank)
+    want = _plain_latent_rows(q[few], [cached[i] for i in few], [lengths[i] for i in few], [1] * len(few), rank,
+                              0.1, window)
+    for i, w in zip(few, want):
+        assert rel_err(got[i], w) < 8e-3, (i, lengths[i])
+
+
+@pytest.mark.parametrize("rank,rd", LATENT_FORMS)
+@pytest.mark.parametrize("window", [0, 150])
+def test_latent_decode_in_high_blocks(ops, rank, rd, window):
+    """A decode step of more heads and keys than low blocks are worth: blocks of 64 rows, two of a
+    request's 70, whose keys are cut into chunks of several tiles; and requests of a few keys."""
+    ps, heads = 64, 70
+    lengths = [2600 if i % 19 == 0 else [1, 64, 65, 300, 700][i % 5] for i in range(100)]
+    few = [0, 1, 2, 3, 4, 7, 19]
+    ctx, pool, table, q, cached = _latent_case(ops, torch.bfloat16, heads, rank, rd, ps, lengths, [1] * 100, seed=rank)
+    out = torch.full((ctx.T, heads * rank), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops.latent_attention(q.to(DEV), pool.bfloat16().to(DEV), table.to(DEV), ctx, heads, rank, rd, ps, 0.1, out,
+                         window=window)
+    got = out.float().cpu().reshape(ctx.T, heads, rank)
     want = _plain_latent_rows(q[few], [cached[i] for i in few], [lengths[i] for i in few], [1] * len(few), rank,
                               0.1, window)
     for i, w in zip(few, want):
@@ -393,7 +412,8 @@ def test_latent_pages_that_the_table_does_not_hold(ops, rank, rd, heads, new_row
 
 
 @pytest.mark.parametrize("rank,rd", LATENT_FORMS)
-@pytest.mark.parametrize("heads,new_rows", [(16, [260, 130, 64]), (40, [1, 1, 1]), (70, [1, 1, 1]), (3, [1, 90, 40])])
+@pytest.mark.parametrize("heads,new_rows", [(16, [260, 130, 64]), (40, [1, 1, 1]), (70, [1, 1, 1]), (3, [1, 90, 40]),
+                                            (40, [260, 1, 200])])
 def test_latent_forms(ops, rank, rd, heads, new_rows):
     """Prompts, decode steps of more heads than a block has rows, and both in one step, with a gate:
     every form of the bfloat16 kernel, each request's keys cut into chunks."""
