@@ -277,7 +277,13 @@ typedef __attribute__((address_space(3))) lat_short4 lat_lds_short4;
 constexpr int kLatKeys = 64;      // keys per tile
 constexpr int kLatThreads = 512;
 constexpr int kLatPRow = kLatKeys + 8;   // row length of the probabilities in LDS
-constexpr int kLatMaxHalf = 20;   // steps of 16 numbers of half a cached row: rows of up to 640
+// Steps of 16 numbers of half a cached row that the kernel is built for: rows of up to 160, 288, 416, 576
+// and 640 numbers (what fits the registers). A row between two of them is padded up to the longer one
+// with zeros, up to half as many numbers again, or as many as 80 of 160. Rows of 80 in the form of
+// 288: a request of 200 keys 13.7 us, in their own 11.6; of 384 in that of 576: a 2,048-token prompt of 16 heads
+// 172 us, in that of 416 160.
+constexpr int kLatHalves[] = {5, 9, 13, 18, 20};
+constexpr int kLatMaxHalf = 20;
 constexpr float kLatLog2e = 1.44269504088896f;
 // What keys whose page the table does not hold (-1) are read from. (A prompt of 2,048 tokens of 16 heads
 // with 512 + 64 numbers: 188 us without the check, 192 so, 206 with such loads switched off, 228 with
@@ -288,7 +294,7 @@ struct LatentTilePlan {
   int rows;         // (token, head) rows of a block
   int tiles;        // upper bound of row tiles over all requests
   int n_chunks;     // key chunks per row tile
-  int half;         // steps of 16 numbers in half a cached row (the kernel's own: 9, 18 or 20)
+  int half;         // steps of 16 numbers in half a cached row (of kLatHalves)
   int page_shift;
   size_t lds;
 };
@@ -334,7 +340,8 @@ static float latent_tile_us(const LatentArgs& a, int rows, int half) {
 static LatentTilePlan latent_tile_plan(const LatentArgs& a) {
   LatentTilePlan p;
   const int Dk = a.R + a.rd;
-  p.half = Dk <= 32 * 9 ? 9 : Dk <= 32 * 18 ? 18 : kLatMaxHalf;
+  for (const int half : kLatHalves)
+    if (Dk <= 32 * (p.half = half)) break;
   p.rows = latent_tile_us(a, 16, p.half) <= latent_tile_us(a, 64, p.half) ? 16 : 64;
   latent_tile_split(a, p.rows, &p.tiles, &p.n_chunks);
   p.page_shift = 0;
@@ -689,9 +696,14 @@ static int launch_latent_tile(const LatentArgs& a, const LatentTilePlan& p, hipS
 template <int ROWS>
 static int launch_latent_rows(const LatentArgs& a, const LatentTilePlan& p, hipStream_t stream) {
   const bool few = a.R <= 256;   // output columns: 8 waves of 2 or 4 tiles of 16
-  if (p.half == 9) return few ? launch_latent_tile<ROWS, 9, 2>(a, p, stream) : launch_latent_tile<ROWS, 9, 4>(a, p, stream);
-  if (p.half == 18) return few ? launch_latent_tile<ROWS, 18, 2>(a, p, stream) : launch_latent_tile<ROWS, 18, 4>(a, p, stream);
-  return few ? launch_latent_tile<ROWS, kLatMaxHalf, 2>(a, p, stream) : launch_latent_tile<ROWS, kLatMaxHalf, 4>(a, p, stream);
+#define NINFER_LATENT_HALF(H) \
+  if (p.half == H) return few ? launch_latent_tile<ROWS, H, 2>(a, p, stream) : launch_latent_tile<ROWS, H, 4>(a, p, stream)
+  NINFER_LATENT_HALF(5);
+  NINFER_LATENT_HALF(9);
+  NINFER_LATENT_HALF(13);
+  NINFER_LATENT_HALF(18);
+#undef NINFER_LATENT_HALF
+  return few ? launch_latent_tile<ROWS, 20, 2>(a, p, stream) : launch_latent_tile<ROWS, 20, 4>(a, p, stream);
 }
 
 static int latent_attention_tile(const LatentArgs& a, hipStream_t stream) {

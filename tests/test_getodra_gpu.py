@@ -328,12 +328,13 @@ def test_latent_attention_whole_prompt_on_matrix_cores(ops, heads, rank, rd):
     assert rel_err(outs[0][:3], want[:3]) < 8e-3 and rel_err(outs[0][-1], want[-1]) < 8e-3
 
 
-# rows of a cached latent at the edges of the bfloat16 kernel's forms: up to 288, 576 and 640 numbers,
+# rows of a cached latent at the edges of the bfloat16 kernel's forms: up to 160, 288, 416, 576 and 640 numbers,
 # latents of up to 256 and 512
 # (Bounds: the queries, the probabilities and the output each round to bfloat16 once, 2^-9 at most; the
 # queries' rounding counts times the scores' size, about 2 here: 4 * 2^-9 = 8e-3.)
 LATENT_FORMS = [(256, 32), (264, 24), (288, 0), (64, 16), (256, 64), (200, 376), (512, 64), (512, 128),
-                (256, 328), (504, 80)]
+                (256, 328), (504, 80),
+                (160, 0), (128, 40), (256, 160), (257, 167)]
 
 
 @pytest.mark.parametrize("rank,rd", LATENT_FORMS)
