@@ -137,6 +137,16 @@ __global__ void lightning_step_kernel(const T* __restrict__ qkv, int stride, int
   }
 }
 
+// Threads that share a value column.
+static int lightning_parts(int dim, int vdim) {
+  const int parts = vdim < 256 ? 256 / vdim : 1;
+  return parts < dim ? parts : dim;
+}
+
+static size_t lightning_seq_lds(int dim, int vdim) {
+  return ((size_t)dim * vdim + 2 * (2 * dim + vdim) + (size_t)lightning_parts(dim, vdim) * vdim) * sizeof(float);
+}
+
 }  // namespace ninfer
 
 using namespace ninfer;
@@ -157,19 +167,17 @@ extern "C" int ninfer_lightning_attention(const void* qkv, int stride, int q_off
                  "lightning_attention: a request's state of %lld floats holds no %d x %d x %d",
                  state_stride, H, dim, vdim);
   NINFER_REQUIRE(dtype == kF32 || dtype == kBF16, "lightning_attention: unknown dtype %d", dtype);
-  int parts = 256 / vdim;
-  if (parts < 1) parts = 1;
-  if (parts > dim) parts = dim;
+  const int parts = lightning_parts(dim, vdim);
   const int block = parts * vdim;
-  const size_t lds = ((size_t)dim * vdim + 2 * (2 * dim + vdim) + (size_t)parts * vdim) * sizeof(float);
+  const size_t lds = lightning_seq_lds(dim, vdim);
   NINFER_REQUIRE(lds <= 160 * 1024, "lightning_attention: a head's state of %d x %d does not fit "
                  "the LDS", dim, vdim);
   const dim3 grid(S, H);
   // (a row per request as a rule; more rows than requests go through the LDS: one trip for all rows)
-  if (T <= S) {
-    const int cols = vdim < 64 ? vdim : 64;
+  const int cols = vdim < 64 ? vdim : 64;
+  const size_t bytes = (2 * (size_t)dim + (size_t)parts * cols) * sizeof(float);
+  if (T <= S && bytes <= 48 * 1024) {
     const dim3 grid(S, H, (vdim + cols - 1) / cols);
-    const size_t bytes = (2 * (size_t)dim + (size_t)parts * cols) * sizeof(float);
 #define NINFER_LIGHTNING_STEP(TYPE)                                                             \
   lightning_step_kernel<TYPE><<<grid, parts * cols, bytes, stream>>>(                           \
       (const TYPE*)qkv, stride, q_off, k_off, v_off, decay, state, state_stride, out,           \
@@ -211,15 +219,24 @@ extern "C" int ninfer_lightning_attention(const void* qkv, int stride, int q_off
 // grows. Every product runs on v_mfma_f32_32x32x2_f32: q, k, v (silu of the projections), the
 // decays and the state enter in 32-bit and are never rounded to a shorter type.
 //
-// The chunks of a step lie side by side: a block per (chunk, head, 128 value columns) forms the sum
-// of S' (lightning_chunk_sums), a thread per number of the state walks a request's chunks and leaves
-// the state before each in the sum's place (lightning_chunk_carry), and a block per (chunk, head,
-// 128 value columns) forms the outputs (lightning_chunk_outputs). That is 3 passes over 64 KB of
-// state per chunk and head of 128 x 128 where one block that walks the chunks of a request keeps it
-// in registers, but 512 blocks instead of 64 for a prompt of 2,048 tokens with 16 heads, and no
-// chain of 32 chunks with three barriers each: 25 + 15 + 51 us against 903 for that prompt. (Three
-// GFLOP are 20 us at the rate of the 32-bit matrix instruction; the sums and the outputs are bound
-// by silu of the rows and LDS before it, one and two blocks a CU.)
+// Two forms, and single rows apart from both:
+//
+//   side by side  a block per (chunk, head, 128 value columns) forms the sum of S' (lightning_chunk_sums),
+//                 a thread per number of the state walks a request's chunks and leaves the state before
+//                 each in the sum's place (lightning_chunk_carry), and a block per (chunk, head, 128 value
+//                 columns) forms the outputs (lightning_chunk_outputs). That is 3 passes over 64 KB of state
+//                 per chunk and head of 128 x 128, but 512 blocks for a prompt of 2,048 tokens with 16
+//                 heads, and no chain of 32 chunks: 25 + 15 + 51 us against 903 of the walk. (Three GFLOP
+//                 are 20 us at the rate of the 32-bit matrix instruction; the sums and the outputs are
+//                 bound by silu of the rows and LDS before it, one and two blocks a CU.)
+//   the walk      a block per (request, head, 32 value columns) takes the request's chunks one after the
+//                 other with the state in registers: one launch, and the state goes to memory and back
+//                 once. Better for short portions: one of 8 to 64 rows 26 to 31 us against 40 to 47.
+//   single rows   requests of one row, the step's first, may go through lightning_step_kernel beside either
+//                 form, which would take each for a chunk: 64 of them and a portion of 448 rows 508 us as
+//                 chunks side by side, 83 apart.
+//
+// lightning_form chooses by an estimate of all four.
 namespace ninfer {
 
 typedef float lt_f32x16 __attribute__((ext_vector_type(16)));
@@ -228,6 +245,7 @@ constexpr int kLtChunk = 64;
 constexpr int kLtCols = 128;       // value columns of a block
 constexpr int kLtThreads = 512;
 constexpr int kLtMaxDim = 256;
+constexpr int kLtStateTiles = 4;   // 32-row tiles of the state of a carrying wave (the walk): dim up to 256
 constexpr int kLtTile = 32 * 33;   // a 32 x 32 tile of decayed scores in LDS
 
 struct LightningChunks {
@@ -259,6 +277,195 @@ __device__ __forceinline__ bool lightning_find_chunk(const LightningChunks& a, i
     at -= chunks;
   }
   return false;
+}
+
+// A block walks one request's chunks, 32 value columns of a head: waves 0 and 1 form a chunk's
+// outputs, waves 2 and 3 carry the state in their accumulators and hand a copy to the others through LDS.
+template <bool WIDE>
+__global__ __launch_bounds__(256) void lightning_walk_kernel(LightningChunks a) {
+  extern __shared__ float smem[];
+  const int dim = a.dim, vdim = a.vdim, H = a.H;
+  const bf16* qkv = a.qkv;
+  const int stride = a.stride, q_off = a.q_off, k_off = a.k_off, v_off = a.v_off;
+  const int qs = dim + 1;                 // row length of q and k in LDS (odd: column reads spread)
+  float* Qs = smem;                       // [64][dim + 1]
+  float* Ks = Qs + kLtChunk * qs;         // [64][dim + 1]
+  float* Vs = Ks + kLtChunk * qs;         // [64][33]
+  float* As = Vs + kLtChunk * 33;         // [64][65]
+  float* Ss = As + kLtChunk * 65;         // [dim32][33]
+  float* Ws = Ss + ((dim + 31) / 32 * 32) * 33;   // [64] d^(L - 1 - j) of the chunk's rows
+  const int s = blockIdx.x, h = blockIdx.y, c0 = 32 * blockIdx.z;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, lr = lane & 31, lk = lane >> 5;
+  const int r0 = a.seq_row_start[s], n = a.seq_row_start[s + 1] - r0;
+  const int dim32 = (dim + 31) / 32 * 32;
+  const int d_tiles = dim32 / 32;
+  float* st = a.state + (int64_t)a.seq_slots[s] * a.state_stride + (int64_t)h * dim * vdim;
+  const float log2d = log2f(a.decay[h]);
+  const bool col_ok = c0 + lr < vdim;
+  // the state: in the accumulators of waves 2 and 3 (tiles w - 2, w, ...), a copy in LDS
+  lt_f32x16 sacc[kLtStateTiles] = {};
+  for (int e = tid; e < dim32 * 33; e += 256) {
+    const int d = e / 33, c = e % 33;
+    Ss[e] = (d < dim && c < 32 && c0 + c < vdim) ? st[(int64_t)d * vdim + c0 + c] : 0.f;
+  }
+  __syncthreads();
+  if (w >= 2) {
+#pragma unroll
+    for (int x = 0; x < kLtStateTiles; ++x) {
+      const int dt = (w - 2) + 2 * x;
+      if (dt < d_tiles) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) sacc[x][4 * q + r] = Ss[(32 * dt + 8 * q + 4 * lk + r) * 33 + lr];
+      }
+    }
+  }
+
+  for (int i0 = 0; i0 < n; i0 += kLtChunk) {
+    const int L = min(kLtChunk, n - i0);
+    // 1. the chunk's q, k (all of the head's numbers) and this block's value columns
+    if (WIDE) {   // eight neighbouring numbers per load
+      const int per_row = dim / 8;
+      for (int e = tid; e < kLtChunk * per_row; e += 256) {
+        const int i = e / per_row, d = 8 * (e % per_row);
+        float qv[8], kv[8];
+#pragma unroll
+        for (int x = 0; x < 8; ++x) qv[x] = kv[x] = 0.f;
+        if (i < L) {
+          const bf16* row = qkv + (int64_t)(r0 + i0 + i) * stride;
+          const lt_bf16x8 qx = *(const lt_bf16x8*)(row + q_off + h * dim + d);
+          const lt_bf16x8 kx = *(const lt_bf16x8*)(row + k_off + h * dim + d);
+#pragma unroll
+          for (int x = 0; x < 8; ++x) {
+            qv[x] = silu_f((float)qx[x]);
+            kv[x] = silu_f((float)kx[x]);
+          }
+        }
+#pragma unroll
+        for (int x = 0; x < 8; ++x) {
+          Qs[i * qs + d + x] = qv[x];
+          Ks[i * qs + d + x] = kv[x];
+        }
+      }
+    } else {
+      for (int e = tid; e < kLtChunk * dim; e += 256) {
+        const int i = e / dim, d = e % dim;
+        float qv = 0.f, kv = 0.f;
+        if (i < L) {
+          const bf16* row = qkv + (int64_t)(r0 + i0 + i) * stride;
+          qv = silu_f(to_f32(row[q_off + h * dim + d]));
+          kv = silu_f(to_f32(row[k_off + h * dim + d]));
+        }
+        Qs[i * qs + d] = qv;
+        Ks[i * qs + d] = kv;
+      }
+    }
+    for (int e = tid; e < kLtChunk * 32; e += 256) {
+      const int i = e >> 5, c = e & 31;
+      float vv = 0.f;
+      if (i < L && c0 + c < vdim)
+        vv = silu_f(to_f32(qkv[(int64_t)(r0 + i0 + i) * stride + v_off + h * vdim + c0 + c]));
+      Vs[i * 33 + c] = vv;
+    }
+    if (tid < kLtChunk) Ws[tid] = tid < L ? decay_pow(log2d, L - 1 - tid) : 0.f;
+    __syncthreads();   // (also: the state's copy in LDS is the one before this chunk)
+    // 2. A[i][j] = d^(i - j) q_i . k_j for j <= i: wave w has rows 32 (w / 2).., keys 32 (w % 2)..
+    {
+      const int mi = w >> 1, nj = w & 1;
+      lt_f32x16 sc = {};
+      if (nj <= mi) {
+        const float* qrow = Qs + (32 * mi + lr) * qs + lk;
+        const float* krow = Ks + (32 * nj + lr) * qs + lk;
+#pragma unroll 8
+        for (int d = 0; d < dim; d += 2) {
+          const float qa = (d + lk < dim) ? qrow[d] : 0.f;
+          const float kb = (d + lk < dim) ? krow[d] : 0.f;
+          sc = __builtin_amdgcn_mfma_f32_32x32x2f32(qa, kb, sc, 0, 0, 0);
+        }
+      }
+      const int j = 32 * nj + lr;
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int i = 32 * mi + 8 * q + 4 * lk + r;
+          As[i * 65 + j] = j <= i ? sc[4 * q + r] * decay_pow(log2d, i - j) : 0.f;
+        }
+    }
+    __syncthreads();
+    // 3. waves 0, 1: the outputs of rows 32 w ..; waves 2, 3: the state after the chunk
+    if (w < 2) {
+      lt_f32x16 o = {};
+      const int row = 32 * w + lr;
+      const float* arow = As + row * 65 + lk;
+#pragma unroll 8
+      for (int j = 0; j < 32 * (w + 1); j += 2)
+        o = __builtin_amdgcn_mfma_f32_32x32x2f32(arow[j], Vs[(j + lk) * 33 + lr], o, 0, 0, 0);
+      const float carry = decay_pow(log2d, row + 1);
+      const float* qrow = Qs + row * qs + lk;
+#pragma unroll 8
+      for (int d = 0; d < dim; d += 2) {
+        const float qa = (d + lk < dim) ? qrow[d] * carry : 0.f;
+        o = __builtin_amdgcn_mfma_f32_32x32x2f32(qa, Ss[(d + lk) * 33 + lr], o, 0, 0, 0);
+      }
+      if (col_ok) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int i = 32 * w + 8 * q + 4 * lk + r;
+            if (i < L) a.out[((int64_t)(r0 + i0 + i) * H + h) * vdim + c0 + lr] = o[4 * q + r];
+          }
+      }
+    } else {
+      const float whole = decay_pow(log2d, L);
+#pragma unroll
+      for (int x = 0; x < kLtStateTiles; ++x) {
+        const int dt = (w - 2) + 2 * x;
+        if (dt < d_tiles) {
+#pragma unroll
+          for (int i = 0; i < 16; ++i) sacc[x][i] *= whole;
+          const int d = 32 * dt + lr;
+#pragma unroll 8
+          for (int j = 0; j < kLtChunk; j += 2) {
+            const int jj = j + lk;
+            const float ka = (jj < L && d < dim) ? Ks[jj * qs + d] * Ws[jj] : 0.f;
+            sacc[x] = __builtin_amdgcn_mfma_f32_32x32x2f32(ka, Vs[jj * 33 + lr], sacc[x], 0, 0, 0);
+          }
+        }
+      }
+    }
+    __syncthreads();   // everyone has read the old copy of the state
+    if (w >= 2) {
+#pragma unroll
+      for (int x = 0; x < kLtStateTiles; ++x) {
+        const int dt = (w - 2) + 2 * x;
+        if (dt < d_tiles) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) Ss[(32 * dt + 8 * q + 4 * lk + r) * 33 + lr] = sacc[x][4 * q + r];
+        }
+      }
+    }
+    // (the barrier after the next chunk's loads publishes the copy; nothing reads it before)
+  }
+  if (w >= 2 && col_ok) {
+#pragma unroll
+    for (int x = 0; x < kLtStateTiles; ++x) {
+      const int dt = (w - 2) + 2 * x;
+      if (dt < d_tiles) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int d = 32 * dt + 8 * q + 4 * lk + r;
+            if (d < dim) st[(int64_t)d * vdim + c0 + lr] = sacc[x][4 * q + r];
+          }
+      }
+    }
+  }
 }
 
 // Columns col .. col + width - 1 of the chunk's rows, silu applied, times `scale` per row where
@@ -415,10 +622,57 @@ __global__ __launch_bounds__(kLtThreads) void lightning_chunk_outputs_kernel(Lig
 
 static int64_t lightning_most_chunks(int T, int S) { return T / kLtChunk + S; }   // no step has more
 
+static size_t lightning_walk_lds(int dim) {
+  const int dim32 = (dim + 31) / 32 * 32;
+  return ((size_t)2 * kLtChunk * (dim + 1) + kLtChunk * 33 + kLtChunk * 65 + (size_t)dim32 * 33 + kLtChunk) * sizeof(float);
+}
+
+struct LightningForm {
+  int apart;   // requests of one row that lightning_step_kernel takes
+  bool side;   // the others' chunks side by side, not by the walk
+};
+
+// What a step of T rows in S requests takes each way, in us on this part (1 us more or less where one
+// launch is enough; 16 heads of 128 x 128: the walk 26 for up to 8 rows, 31 for 64, 49 for two chunks and
+// 23 for each more, times the rounds of its blocks, one to a CU; side by side 43 and 1.2 for every chunk, 3.2
+// for every request; single rows 9 and 0.4 each). `single` of the requests, the first, bring one row each.
+static LightningForm lightning_form(int T, int S, int single, int max_qlen, int H, int dim, int vdim) {
+  const float numbers = (float)H * dim * vdim / (16 * 128 * 128), longest = (max_qlen + kLtChunk - 1) / kLtChunk;
+  const bool walks = lightning_walk_lds(dim) <= 160 * 1024;
+  auto walk = [&](int requests) {
+    const float rounds = (float)requests * H * ((vdim + 31) / 32) / device_cu_count();
+    return (rounds > 1.f ? rounds : 1.f) * (6.f + longest * (5.f + 18.f * dim / 128));
+  };
+  auto side = [&](int rows, int requests) {
+    return 43.f + numbers * (1.2f * (rows / kLtChunk + requests) + 3.2f * requests);
+  };
+  const float apart = single > 0 ? 9.f + 0.4f * single * numbers : 0.f;
+  LightningForm best = {0, true};
+  float least = side(T, S);
+  auto look = [&](float us, int a, bool s) {
+    if (us < least) least = us, best = {a, s};
+  };
+  if (walks) look(walk(S), 0, false);
+  if (single > 0 && single < S && lightning_seq_lds(dim, vdim) <= 160 * 1024) {
+    look(apart + side(T - single, S - single), single, true);
+    if (walks) look(apart + walk(S - single), single, false);
+  }
+  return best;
+}
+
 static int lightning_lds(const void* kern, size_t lds) {
   if (lds <= 48 * 1024) return 0;
   hipError_t e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e != hipSuccess) return set_error(-2, "lightning_attention: cannot get %zu bytes of LDS", lds);
+  return 0;
+}
+
+template <bool WIDE>
+static int lightning_walk(const LightningChunks& a, hipStream_t stream) {
+  const size_t lds = lightning_walk_lds(a.dim);
+  if (int rc = lightning_lds((const void*)lightning_walk_kernel<WIDE>, lds)) return rc;
+  lightning_walk_kernel<WIDE><<<dim3(a.S, a.H, (a.vdim + 31) / 32), 256, lds, stream>>>(a);
+  NINFER_LAUNCH_CHECK();
   return 0;
 }
 
@@ -442,33 +696,55 @@ static int lightning_chunks(const LightningChunks& a, int T, hipStream_t stream)
 
 }  // namespace ninfer
 
-// Floats of workspace with which a step runs in chunks; 0 when the sizes do not fit (the
-// token-by-token kernel takes them).
-extern "C" long long ninfer_lightning_chunk_floats(int T, int S, int H, int dim, int vdim, int dtype) {
-  if (dtype != kBF16 || dim > kLtMaxDim) return 0;
-  return lightning_most_chunks(T, S) * H * dim * vdim;
+// Can a step of these sizes run in chunks? (If not, the token-by-token kernel takes it. Keys too long for
+// the walk come here if the kernel for single rows takes their state: a prompt that could not go on
+// token by token is refused there.)
+static bool lightning_chunks_take(int dim, int vdim, int dtype) {
+  return dtype == kBF16 && dim <= kLtMaxDim &&
+         (lightning_walk_lds(dim) <= 160 * 1024 || lightning_seq_lds(dim, vdim) <= 160 * 1024);
 }
 
-// The same as ninfer_lightning_attention for bfloat16 rows, chunk by chunk on the matrix cores:
-// for steps that bring prompt portions. `work`: ninfer_lightning_chunk_floats floats.
+// Floats of workspace that ninfer_lightning_attention_chunks needs for a step, 0 for none; -1 when the sizes
+// do not fit (the token-by-token kernel takes them).
+extern "C" long long ninfer_lightning_chunk_floats(int T, int S, int single, int max_qlen, int H, int dim, int vdim,
+                                                   int dtype) {
+  if (!lightning_chunks_take(dim, vdim, dtype)) return -1;
+  const LightningForm f = lightning_form(T, S, single, max_qlen, H, dim, vdim);
+  return f.side ? lightning_most_chunks(T - f.apart, S - f.apart) * H * dim * vdim : 0;
+}
+
+// The same as ninfer_lightning_attention for bfloat16 rows, chunk by chunk on the matrix cores: for steps that
+// bring prompt portions. The first `single` requests bring one row each, the longest brings max_qlen rows.
+// `work`: ninfer_lightning_chunk_floats floats.
 extern "C" int ninfer_lightning_attention_chunks(const void* qkv, int stride, int q_off, int k_off,
                                                  int v_off, const float* decay, float* state,
                                                  long long state_stride, float* out,
                                                  const int* seq_row_start, const int* seq_slots,
                                                  int T, int S, int H, int dim, int vdim, int dtype,
-                                                 float* work, hipStream_t stream) {
+                                                 int single, int max_qlen, float* work, hipStream_t stream) {
   NINFER_REQUIRE(T > 0 && S > 0 && H > 0 && dim > 0 && vdim > 0,
                  "lightning_attention: T=%d S=%d heads=%d dim=%d vdim=%d must be positive", T, S,
                  H, dim, vdim);
+  NINFER_REQUIRE(single >= 0 && single <= S && single <= T && max_qlen > 0,
+                 "lightning_attention: %d single rows of %d requests, %d rows the longest", single, S, max_qlen);
   NINFER_REQUIRE(state_stride >= (long long)H * dim * vdim,
                  "lightning_attention: a request's state of %lld floats holds no %d x %d x %d",
                  state_stride, H, dim, vdim);
-  NINFER_REQUIRE(ninfer_lightning_chunk_floats(T, S, H, dim, vdim, dtype) > 0 && work,
-                 "lightning_attention: dtype %d, key size %d do not run in chunks, or no workspace", dtype, dim);
-  LightningChunks a = {(const bf16*)qkv, decay, state, out, work, seq_row_start, seq_slots, state_stride,
-                       stride, q_off, k_off, v_off, S, H, dim, vdim};
-  // rows whose q, k and v parts start and end at multiples of 16 bytes
-  const bool wide = dim % 8 == 0 && vdim % 8 == 0 && stride % 8 == 0 && q_off % 8 == 0 && k_off % 8 == 0 &&
-                    v_off % 8 == 0 && (uintptr_t)qkv % 16 == 0;
-  return wide ? lightning_chunks<true>(a, T, stream) : lightning_chunks<false>(a, T, stream);
+  NINFER_REQUIRE(lightning_chunks_take(dim, vdim, dtype),
+                 "lightning_attention: dtype %d, key size %d do not run in chunks", dtype, dim);
+  const LightningForm f = lightning_form(T, S, single, max_qlen, H, dim, vdim);
+  NINFER_REQUIRE(!f.side || work, "lightning_attention: no workspace");
+  if (f.apart) {
+    if (int rc = ninfer_lightning_attention(qkv, stride, q_off, k_off, v_off, decay, state, state_stride, out,
+                                            seq_row_start, seq_slots, f.apart, f.apart, H, dim, vdim, dtype, stream))
+      return rc;
+  }
+  // (rows are counted from the step's first whatever the first request)
+  LightningChunks a = {(const bf16*)qkv, decay, state, out, work, seq_row_start + f.apart, seq_slots + f.apart,
+                       state_stride, stride, q_off, k_off, v_off, S - f.apart, H, dim, vdim};
+  // rows whose q and k parts, and v parts, start and end at multiples of 16 bytes
+  const bool wide_qk = dim % 8 == 0 && stride % 8 == 0 && q_off % 8 == 0 && k_off % 8 == 0 && (uintptr_t)qkv % 16 == 0;
+  const bool wide = wide_qk && vdim % 8 == 0 && v_off % 8 == 0;
+  if (!f.side) return wide_qk ? lightning_walk<true>(a, stream) : lightning_walk<false>(a, stream);
+  return wide ? lightning_chunks<true>(a, T - f.apart, stream) : lightning_chunks<false>(a, T - f.apart, stream);
 }

@@ -1514,16 +1514,18 @@ class HipOps:
                 ctypes.c_longlong(state.stride(0)), ctypes.c_void_p(out.data_ptr()),
                 ctypes.c_void_p(ctx.seq_row_start.data_ptr()), ctypes.c_void_p(ctx.seq_slots.data_ptr()),
                 t, ctx.S, heads, dim, vdim, _DT[qkv.dtype])
-        # bfloat16 steps that bring prompt portions: chunks of 64 rows on the matrix cores, side by side (the
+        # bfloat16 steps that bring prompt portions: chunks of 64 rows on the matrix cores (the
         # sums of a chunk are ordered otherwise than token by token, so the 32-bit path, whose
         # logits do not depend on the cut to the bit, stays on the token-by-token kernel)
         if qkv.dtype == torch.bfloat16 and ctx.max_qlen >= self.lightning_chunk_min_rows \
                 and not self.force_generic:
-            floats = self.lib.ninfer_lightning_chunk_floats(t, ctx.S, heads, dim, vdim, _DT[qkv.dtype])
-            if floats > 0:
-                work = torch.empty(floats, dtype=torch.float32, device=qkv.device)
+            single = int(getattr(ctx, "single_rows", 0))
+            floats = self.lib.ninfer_lightning_chunk_floats(t, ctx.S, single, ctx.max_qlen, heads, dim, vdim,
+                                                            _DT[qkv.dtype])
+            if floats >= 0:
+                work = torch.empty(floats, dtype=torch.float32, device=qkv.device) if floats else None
                 self._ok(self.lib.ninfer_lightning_attention_chunks(
-                    *args, ctypes.c_void_p(work.data_ptr()), self._stream()))
+                    *args, single, ctx.max_qlen, ctypes.c_void_p(_ptr(work)), self._stream()))
                 return
         self._ok(self.lib.ninfer_lightning_attention(*args, self._stream()))
 

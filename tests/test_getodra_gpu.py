@@ -195,6 +195,37 @@ def test_lightning_chunks_of_aligned_rows(ops, heads, dim, vdim, lens):
     assert torch.equal(got_state[untouched].cpu(), state[untouched])
 
 
+@pytest.mark.parametrize("heads,dim,vdim", [(16, 128, 128), (3, 60, 36), (2, 72, 260), (1, 256, 64), (1, 8, 8)])
+@pytest.mark.parametrize("lens", [[8], [33, 64], [1] * 3 + [9], [1] * 60 + [20], [1] * 60 + [2, 150], [1, 1, 140, 64]])
+def test_lightning_single_rows_beside_portions(ops, heads, dim, vdim, lens):
+    """Steps whose first requests bring one row each, beside portions short and long: single rows apart or
+    not, the rest walked or with its chunks side by side, as the sizes have it."""
+    torch.manual_seed(dim + sum(lens))
+    decay = torch.linspace(0.3, 1.0, heads)
+    qk, vw = heads * dim, heads * vdim
+    x = torch.randn(sum(lens), 2 * qk + vw).to(torch.bfloat16)
+    state = torch.randn(len(lens) + 1, heads * dim * vdim + 4)
+    ctx = util.make_context(ops, torch.bfloat16, [(0, n) for n in lens])
+    ctx.single_rows = lens.count(1)
+    slots = [len(lens) - i for i in range(len(lens))]
+    ctx.seq_slots = torch.tensor(slots, dtype=torch.int32, device=DEV)
+    got_state, out = state.to(DEV), torch.full((sum(lens) + 1, vw), 7.0, device=DEV)
+    ops.lightning_attention(x.to(DEV), 0, qk, 2 * qk, heads, dim, vdim, decay.to(DEV), got_state, ctx, out[:-1])
+    f = plain_getodra.silu(x.double())
+    S_all = state[:, :heads * dim * vdim].double().reshape(-1, heads, dim, vdim)
+    at = 0
+    for slot, n in zip(slots, lens):
+        S = S_all[slot].clone()
+        for t in range(at, at + n):
+            S = decay.double()[:, None, None] * S + f[t, qk:2 * qk].reshape(heads, dim, 1) * f[t, 2 * qk:].reshape(heads, 1, vdim)
+            want = (f[t, :qk].reshape(heads, dim, 1) * S).sum(1)
+            assert rel_err(out[t].double().cpu().reshape(heads, vdim), want) < 2e-5, (slot, t - at)
+        assert rel_err(got_state[slot, :heads * dim * vdim].double().cpu().reshape(S.shape), S) < 2e-5
+        at += n
+    assert (out[-1] == 7.0).all() and torch.equal(got_state[0].cpu(), state[0])
+    assert torch.equal(got_state[:, heads * dim * vdim:].cpu(), state[:, heads * dim * vdim:])
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("heads,dim,vdim", [(2, 128, 128), (1, 64, 64), (3, 16, 24), (2, 33, 40), (1, 5, 300),
                                             (1, 130, 256), (2, 1, 1)])

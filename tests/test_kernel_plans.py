@@ -1,0 +1,36 @@
+"""What the kernel library decides on the host, without a GPU: which form a step takes and how much scratch
+that needs."""
+import ctypes
+
+import pytest
+
+BF16 = 1
+
+
+@pytest.fixture(scope="module")
+def lib():
+    from ninfer_amd.kernels.build import ensure_built
+    lib = ctypes.CDLL(ensure_built())
+    lib.ninfer_lightning_chunk_floats.restype = ctypes.c_longlong
+    return lib
+
+
+def test_lightning_scratch_does_not_grow_with_decoding_requests(lib):
+    """Single rows beside a portion take no chunk of their own once they are many: the scratch is that
+    of the portion's chunks."""
+    heads, dim, vdim = 16, 128, 128
+    state = heads * dim * vdim
+    for singles in (0, 16, 64, 256):
+        for rows in (8, 64, 448, 2048):
+            floats = lib.ninfer_lightning_chunk_floats(singles + rows, singles + 1, singles, rows, heads, dim, vdim, BF16)
+            assert floats in (0, (rows // 64 + 1) * state), (singles, rows)
+            assert floats or rows <= 64
+
+
+def test_lightning_sizes_that_do_not_run_in_chunks(lib):
+    floats = lambda dim, vdim, dtype=BF16: lib.ninfer_lightning_chunk_floats(512, 1, 0, 512, 2, dim, vdim, dtype)
+    assert floats(128, 128) > 0 and floats(256, 64) > 0
+    assert floats(128, 1024) > 0            # (single rows of it are refused, as ever)
+    assert floats(257, 16) == -1            # keys too long
+    assert floats(256, 256) == -1           # ... and for the walk, with a state too large for single rows
+    assert floats(128, 128, 0) == -1        # 32-bit goes token by token
