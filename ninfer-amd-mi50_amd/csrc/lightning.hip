@@ -173,10 +173,13 @@ extern "C" int ninfer_lightning_attention(const void* qkv, int stride, int q_off
   NINFER_REQUIRE(lds <= 160 * 1024, "lightning_attention: a head's state of %d x %d does not fit "
                  "the LDS", dim, vdim);
   const dim3 grid(S, H);
-  // (a row per request as a rule; more rows than requests go through the LDS: one trip for all rows)
+  // (a row per request as a rule; more rows than requests go through the LDS: one trip for all rows; so
+  // do small states, many of which fit a CU's LDS: us there and in registers, heads of 16 x 16 of 256
+  // requests 6.7 and 11.9, of 64 x 16 of 64 4.6 and 5.7, of 48 x 48 of 256 8.8 and 10.4, but of 100 x 40
+  // of 64 7.6 and 7.0, of 64 x 64 and more less still)
   const int cols = vdim < 64 ? vdim : 64;
   const size_t bytes = (2 * (size_t)dim + (size_t)parts * cols) * sizeof(float);
-  if (T <= S && bytes <= 48 * 1024) {
+  if (T <= S && dim * vdim >= 3000 && bytes <= 48 * 1024) {
     const dim3 grid(S, H, (vdim + cols - 1) / cols);
 #define NINFER_LIGHTNING_STEP(TYPE)                                                             \
   lightning_step_kernel<TYPE><<<grid, parts * cols, bytes, stream>>>(                           \

@@ -228,7 +228,7 @@ def test_lightning_single_rows_beside_portions(ops, heads, dim, vdim, lens):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("heads,dim,vdim", [(2, 128, 128), (1, 64, 64), (3, 16, 24), (2, 33, 40), (1, 5, 300),
-                                            (1, 130, 256), (2, 1, 1)])
+                                            (1, 130, 256), (2, 1, 1), (2, 77, 41), (1, 11, 300), (1, 3, 1024)])
 def test_lightning_a_row_per_request(ops, dtype, heads, dim, vdim):
     """Steps of no more rows than requests keep the state in registers: the same bits, row by row, as
     the walk that holds it in LDS (which steps of more rows than requests take)."""
