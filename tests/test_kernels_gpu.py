@@ -1050,6 +1050,24 @@ def test_qkv_rope(ops_mode, gen, dtype, n_q, n_kv, d, rot, hidden, seqs):
                 assert torch.equal(k1, k_pool) and torch.equal(v1, v_pool)
 
 
+@pytest.mark.parametrize("v", [1, 63, 1024, 1025, 16383, 16384, 16385, 17409, 32768, 40000])
+def test_sample_greedy_finds_the_first_best(ops, gen, v):
+    """Vocabularies at the edges of the batches that a thread loads: the best token first, last, at a
+    batch's border and everywhere (ties: the lowest); nothing behind the row is read as its token."""
+    spots = sorted({0, v - 1, v // 2, min(v - 1, 16383), min(v - 1, 16384)})
+    n = len(spots) + 1
+    flat = torch.full((n * v + 20000,), 90.0, device="cuda")
+    logits = flat[:n * v].view(n, v)
+    logits.copy_(torch.randn(n, v, generator=gen, device="cuda"))
+    for r, at in enumerate(spots):
+        logits[r, at] = logits[r, v - 1] = 50.0
+    logits[-1] = -2.5
+    out = torch.full((n,), -1, device="cuda", dtype=torch.int32)
+    zero = torch.zeros(n, device="cuda")
+    ops.sample(logits, zero, zero, out)
+    assert out.tolist() == spots + [0]
+
+
 def test_sample_greedy_and_distribution(ops, gen):
     import plain_model
     v = 1000
