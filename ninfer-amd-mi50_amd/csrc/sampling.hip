@@ -632,6 +632,8 @@ __global__ __launch_bounds__(kCandThreads) void sample_few_kernel(
   const u64 mass = have ? (u64)(expf(val_s[lane] * inv_t - m) * 4294967296.f) : 0;
   mass_s[lane] = mass;
   key_s[lane] = kk;
+  // (one wave: its LDS accesses run in order, and the fence keeps the compiler from changing that)
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
   u64 total = 0, ahead = 0;
 #pragma unroll 8
