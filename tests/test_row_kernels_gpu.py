@@ -45,10 +45,10 @@ def test_short_conv(ops, dtype, taps, width, seqs):
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("width", [4, 1028])
 @pytest.mark.parametrize("k", [0, 1, 5])
-def test_sums(ops, dtype, width, k):
+@pytest.mark.parametrize("t", [9, 300])   # (from 2^18 numbers on the gated sum goes in pieces)
+def test_sums(ops, dtype, width, k, t):
     from ninfer_amd.parts import PendingRows
     g = torch.Generator(DEV).manual_seed(width + k)
-    t = 9
     rnd = lambda *s: torch.randn(*s, generator=g, device=DEV)
     x, s1, s2, wts, gate = rnd(t, width), rnd(width), rnd(width), rnd(t, max(k, 1)), rnd(t)
     a, sh, dense, g1, g2 = (rnd(t, width).to(dtype) for _ in range(5))
