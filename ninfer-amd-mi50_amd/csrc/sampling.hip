@@ -29,6 +29,13 @@ __device__ __forceinline__ uint32_t ordered_key(float v) {
   return (b & 0x80000000u) ? ~b : (b | 0x80000000u);  // ascending with the float order
 }
 
+// Probability of a token as 32.32 fixed point, from its scaled logit as the key has it, rounded (tokens of equal
+// key have equal mass, the same in every pass and kernel); m: the largest of the row.
+__device__ __forceinline__ unsigned long long token_mass(float scaled, float m) {
+#pragma clang fp contract(off)   // both are products, which must not go unrounded into the difference
+  return (unsigned long long)(expf(scaled - m) * 4294967296.f);
+}
+
 // Copies of the histogram that a radix pass adds into, lane by lane: the keys of logits share few
 // upper bytes, and atomics of a wave's lanes on one address follow each other.
 template <int COPIES>
@@ -200,11 +207,10 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
   typedef unsigned long long u64;
   auto key_of = [&](float x) { return ordered_key(x * inv_t); };
   auto key = [&](int i) { return key_of(w[i]); };
-  // probability of a token as 32.32 fixed point; tokens of equal key have equal mass
-  auto mass_of = [&](float x) -> u64 { return (u64)(expf(x * inv_t - m) * 4294967296.f); };
+  auto mass_of = [&](float x) -> u64 { return token_mass(x * inv_t, m); };
   auto mass_at = [&](uint32_t kk) -> u64 {
     const uint32_t bits = (kk & 0x80000000u) ? (kk & 0x7fffffffu) : ~kk;   // ordered_key's inverse
-    return (u64)(expf(__uint_as_float(bits) - m) * 4294967296.f);
+    return token_mass(__uint_as_float(bits), m);
   };
   auto block_sum = [&](u64 v) -> u64 {
 #pragma unroll
@@ -629,7 +635,7 @@ __global__ __launch_bounds__(kCandThreads) void sample_few_kernel(
   // it in the order (logit descending, index ascending): top-p keeps those before the target.
   const bool have = lane < k;
   const uint32_t kk = have ? ordered_key(val_s[lane] * inv_t) : 0;
-  const u64 mass = have ? (u64)(expf(val_s[lane] * inv_t - m) * 4294967296.f) : 0;
+  const u64 mass = have ? token_mass(val_s[lane] * inv_t, m) : 0;
   mass_s[lane] = mass;
   key_s[lane] = kk;
   // (one wave: its LDS accesses run in order, and the fence keeps the compiler from changing that)

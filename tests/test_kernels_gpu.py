@@ -1174,6 +1174,29 @@ def test_sample_rows_that_keep_few_tokens(ops, gen, v):
     assert int(a[2]) == v - 1 or float(temp[2]) > 0
 
 
+@pytest.mark.parametrize("top_p", [1.0, 0.999])
+def test_few_tokens_path_has_the_masses_of_the_whole_row(ops, gen, top_p):
+    """Numbers drawn right at the border between two kept tokens, one of them at the threshold: both paths
+    give the same token, so the masses are the same to the last few of their 32 bits."""
+    n, v = 4096, 5000
+    low, high = (30 + torch.rand(n, generator=gen, device="cuda") + i for i in (0, 0.5))
+    logits = torch.full((n, v), -50.0, device="cuda")
+    logits[:, 7], logits[:, 4500] = low, high
+    full = lambda x, dtype=torch.float32: torch.full((n,), x, device="cuda", dtype=dtype)
+    args = dict(top_k=full(2, torch.int32), top_p=full(top_p))
+    scaled = torch.stack([low, high]).double() / 0.7
+    border = torch.softmax(scaled, 0)[0]
+    a, b = full(0, torch.int32), full(0, torch.int32)
+    taken = set()
+    for step in range(-60, 61, 5):
+        uniform = (border + step * 2.0 ** -24).float()
+        ops.sample(logits, full(0.7), uniform, a, **args)
+        ops.sample(logits, full(0.7), uniform, b, few=True, **args)
+        assert torch.equal(a, b), int((a != b).sum())
+        taken |= set(a.tolist())
+    assert taken == {7, 4500}
+
+
 @pytest.mark.parametrize("t,e,k,h,inner", [(8, 60, 4, 256, 160), (64, 8, 3, 96, 64), (40, 6, 2, 160, 96),
                                            (3, 130, 6, 64, 32), (17, 5, 2, 320, 1408)])
 def test_grouped_down_with_two_feature_sets_per_block(ops, gen, t, e, k, h, inner):
