@@ -266,34 +266,38 @@ static float dense_us_128(int blocks, int cus, int K) {
   if (rounds > 1.f && last > 0.f && last < 0.3f) rounds += 0.3f - last;   // a short last round is not cheap
   return 2.f + K * (0.0049f + 0.022f * rounds);
 }
-static float dense_us_256(int tiles, int cus, int K) {
+// (Beside other products, which take the CUs that a last round leaves, it is not cut, and the part of a
+// round counts as that: the headline model's prompts of 1,400 tokens, 264 tiles a time, 11.9 ms, in tiles of
+// 128 12.1; of 700 to 1,280 tokens, up to 220 tiles, 9.2 to 11.1 where tiles of 128 take 9.3 to 11.6.)
+static float dense_us_256(int tiles, int cus, int K, bool beside) {
   const float round = 8.f + 0.0215f * K;                 // of up to three quarters of the CUs
   if (4 * tiles <= 3 * cus) return round;
+  if (beside) return round * 1.37f * (tiles > cus ? (float)tiles / cus : 1.f);
   const int whole = tiles / cus, last = tiles % cus;
   return round * (1.37f * whole + (last == 0 ? 0.f : 4 * last <= cus ? 0.65f : 2 * last <= cus ? 0.95f : 1.37f));
 }
 
+// Tile height of a product. Grouped: the tall tile (it loads and multiplies only the 32-row blocks that
+// hold rows, so it beats the lower ones from 17 rows per expert on, the fewest that come
+// here). Dense: 64 rows while taller tiles would leave CUs without a block, else 128 or 256 by
+// an estimate of both times (dense_us_128, dense_us_256); where one output a feature is stored instead of
+// one of two, as many tall tiles as CUs decide for them too, whose stores cost less (32-bit outputs, K
+// 1,024: 1,531 x 12,800 56 us in tiles of 256 and 68 in those of 128, 3,000 x 6,144 53 and 66). force_kernel
+// (tests) forces 64, 128 or 256 rows.
+static int tile_rows_of(const GemmArgs& a) {
+  if (a.force_kernel >= 1 && a.force_kernel <= 3) return 32 << a.force_kernel;
+  if (a.offsets) return kGroupedTileRows;
+  const bool gated = epilogue_gated(a.epilogue);
+  const int n_units = gated ? 2 * a.N : a.N;   // W rows
+  auto blocks = [&](int tm, int tn) { return ((a.M + tm - 1) / tm) * ((n_units + tn - 1) / tn); };
+  const int cus = device_cu_count(), low = blocks(128, 128), tall = blocks(256, 256);
+  if (a.M <= 64 || low < cus) return 64;   // (no taller than the rows there are)
+  if (a.M <= 128) return 128;
+  return (!gated && tall >= cus) || dense_us_256(tall, cus, a.K, a.beside) < dense_us_128(low, cus, a.K) ? 256 : 128;
+}
+
 int gemm_tile(const GemmArgs& a, hipStream_t stream) {
-  // Tile height. Grouped: the tall tile (it loads and multiplies only the 32-row blocks that
-  // hold rows, so it beats the lower ones from 17 rows per expert on, the fewest that come
-  // here). Dense: 64 rows while taller tiles would leave CUs without a block, else 128 or 256 by
-  // an estimate of both times (dense_us_128, dense_us_256). force_kernel (tests) forces 64, 128
-  // or 256 rows.
-  int rows;
-  if (a.force_kernel >= 1 && a.force_kernel <= 3) {
-    rows = 32 << a.force_kernel;
-  } else if (a.offsets) {
-    rows = kGroupedTileRows;
-  } else {
-    const int n_units = epilogue_gated(a.epilogue) ? 2 * a.N : a.N;   // W rows
-    auto blocks = [&](int tm, int tn) { return ((a.M + tm - 1) / tm) * ((n_units + tn - 1) / tn); };
-    const int cus = device_cu_count();
-    rows = blocks(128, 128) >= cus ? 128 : 64;
-    if (a.M <= 64) rows = 64;           // and no taller than the rows there are
-    else if (a.M > 128 && rows == 128 &&
-             dense_us_256(blocks(256, 256), cus, a.K) < dense_us_128(blocks(128, 128), cus, a.K))
-      rows = 256;
-  }
+  const int rows = tile_rows_of(a);
   if (rows == 256) return gemm_tile_direct(a, stream);
   if (rows == 128) return launch_tile<128, 128, 64, 4, 2, 2>(a, stream);
   return launch_tile<64, 128, 64, 4, 2, 2>(a, stream);
@@ -368,3 +372,5 @@ int gemm_split(const GemmArgs& a, hipStream_t stream) {
 
 }  // namespace ninfer
 
+// Rows of the tiles that ninfer_gemm would run a product of many rows in.
+extern "C" int ninfer_gemm_tile_rows(const ninfer::GemmArgs* args) { return ninfer::tile_rows_of(*args); }

@@ -34,3 +34,18 @@ def test_lightning_sizes_that_do_not_run_in_chunks(lib):
     assert floats(257, 16) == -1            # keys too long
     assert floats(256, 256) == -1           # ... and for the walk, with a state too large for single rows
     assert floats(128, 128, 0) == -1        # 32-bit goes token by token
+
+
+# (an epilogue of 1 is SwiGLU: 2 N rows of weights. 256 CUs, as the library assumes without a GPU)
+@pytest.mark.parametrize("m,n,k,gated,beside,rows", [
+    (64, 5632, 2048, 1, 0, 64), (640, 5632, 2048, 1, 0, 128), (768, 5632, 2048, 1, 0, 256),
+    (1400, 5632, 2048, 1, 0, 128),    # 264 tiles of 256, the last 8 a round of their own, even cut
+    (1400, 5632, 2048, 1, 1, 256),    # ... which costs next to nothing beside other products
+    (1280, 5632, 2048, 1, 1, 256), (640, 5632, 2048, 1, 1, 128), (2048, 5632, 2048, 1, 1, 256),
+    (1531, 12800, 1024, 0, 0, 256), (3000, 6144, 768, 0, 0, 256), (2048, 12800, 512, 0, 0, 256),   # (stores)
+    (900, 12800, 512, 0, 0, 128), (1280, 6144, 768, 0, 0, 128), (1280, 8192, 2048, 0, 0, 256)])
+def test_height_of_dense_tiles(lib, m, n, k, gated, beside, rows):
+    from ninfer_amd.kernels.ops import _GemmArgs
+    args = _GemmArgs(M=m, N=n, K=k, lda=k, ldc=n, in_dtype=BF16, out_dtype=BF16 if gated else 0, epilogue=gated,
+                     beside=beside)
+    assert lib.ninfer_gemm_tile_rows(ctypes.byref(args)) == rows
