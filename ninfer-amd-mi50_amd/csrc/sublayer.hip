@@ -461,16 +461,19 @@ static void launch_short_conv(const float* x, const float* w, float* state, long
         x, w, state, state_stride, out, row_seq, seq_row_start, seq_slots, H, taps, update);
     return;
   }
-  // few rows: one to a thread, so that every CU has some
-  const int per = rows >= 256 ? 4 : 1;
-  const dim3 grid((rows + per - 1) / per, (H / 4 + 255) / 256);
+  // four rows to a thread share its weights where that leaves the CUs enough waves, from 1.5 Mi numbers on:
+  // 2,048 rows of 2,048 channels 10.1 us and 15.2 with one row to a thread, of 1,024 6.3 and 9.3; but 516 rows
+  // of 2,048 6.5 and 5.9, 300 of 1,024 5.3 and 4.7, 300 of 64 4.7 and 4.1 (four taps)
+  const int per = (int64_t)rows * H >= (3 << 19) ? 4 : 1;
+  const int block = row_block(H / 4);
+  const dim3 grid((rows + per - 1) / per, (H / 4 + block - 1) / block);
 #define NINFER_CONV(TAPS)                                                                                     \
   do {                                                                                                        \
     if (per == 4)                                                                                             \
-      short_conv_rows_kernel<T, TAPS, 4><<<grid, 256, 0, stream>>>(x, w, state, state_stride, out, row_seq,   \
+      short_conv_rows_kernel<T, TAPS, 4><<<grid, block, 0, stream>>>(x, w, state, state_stride, out, row_seq,   \
                                                                    seq_row_start, seq_slots, rows, H, update); \
     else                                                                                                      \
-      short_conv_rows_kernel<T, TAPS, 1><<<grid, 256, 0, stream>>>(x, w, state, state_stride, out, row_seq,   \
+      short_conv_rows_kernel<T, TAPS, 1><<<grid, block, 0, stream>>>(x, w, state, state_stride, out, row_seq,   \
                                                                    seq_row_start, seq_slots, rows, H, update); \
   } while (0)
   if (taps == 2) NINFER_CONV(2);

@@ -27,7 +27,9 @@ def shifted(x):
 @pytest.mark.parametrize("taps", [2, 3, 4])
 @pytest.mark.parametrize("width", [4, 1028])
 @pytest.mark.parametrize("seqs", [[(0, 1)], [(0, 1), (7, 1), (2, 1)], [(0, 2), (3, 1), (0, 5)], [(5, 255), (0, 2)],
-                                  [(0, 254), (9, 1), (0, 6)]])
+                                  [(0, 254), (9, 1), (0, 6)],
+                                  # (1,028 wide, four rows to a thread: one row per request, and a last one of three)
+                                  [(3, 1)] * 1600, [(5, 1597), (0, 2)]])
 def test_short_conv(ops, dtype, taps, width, seqs):
     g = torch.Generator(DEV).manual_seed(taps * width + len(seqs))
     ctx = util.make_context(ops, dtype, seqs)
