@@ -1050,7 +1050,7 @@ def test_qkv_rope(ops_mode, gen, dtype, n_q, n_kv, d, rot, hidden, seqs):
                 assert torch.equal(k1, k_pool) and torch.equal(v1, v_pool)
 
 
-@pytest.mark.parametrize("v", [1, 63, 1024, 1025, 16383, 16384, 16385, 17409, 32768, 40000])
+@pytest.mark.parametrize("v", [1, 63, 1024, 1025, 4096, 4097, 16383, 16384, 16385, 17409, 20480, 20481, 32768, 40000])
 def test_sample_greedy_finds_the_first_best(ops, gen, v):
     """Vocabularies at the edges of the batches that a thread loads: the best token first, last, at a
     batch's border and everywhere (ties: the lowest); nothing behind the row is read as its token."""
@@ -1141,7 +1141,7 @@ def test_sample_ties_keep_the_sorted_prefix(ops, seed):
         assert len(set(draws)) == 1
 
 
-@pytest.mark.parametrize("v", [70, 4096, 4097, 20011, 151936])
+@pytest.mark.parametrize("v", [70, 4096, 4097, 12288, 12289, 20011, 151936])
 def test_sample_rows_that_keep_few_tokens(ops, gen, v):
     """Rows that are greedy or keep at most 64 tokens have a path of two launches that reads
     the logits with the whole GPU: the same tokens as the one-block path, row by row, with
