@@ -166,7 +166,7 @@ class Sampler:
         floats[2] = [row.params.repetition_penalty for row in rows]
         drawn = [i for i, row in enumerate(rows) if row.params.temperature > 0]   # (greedy rows draw nothing)
         floats[3] = 0.0
-        if len(drawn) > 8:   # from there on whole arrays are the shorter way
+        if len(drawn) > 24:   # (whole arrays 32 us for 16 rows, 34 for 24, 47 for 64; one by one 21, 31 and 83)
             floats[3, drawn] = uniforms([rows[i] for i in drawn])
         else:
             for i in drawn:
