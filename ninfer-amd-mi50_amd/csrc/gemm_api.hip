@@ -21,6 +21,9 @@ static bool many_rows(const GemmArgs& a) {
   return (a.M > 32 || huge) && a.N > 128;
 }
 
+// Bytes of GemmArgs: a caller that lays it out for itself compares its own.
+extern "C" int ninfer_gemm_args_bytes() { return (int)sizeof(GemmArgs); }
+
 // force_generic != 0 runs the plain tiled kernel whatever the shape (tests
 // compare the fast kernels with it).
 extern "C" int ninfer_gemm(const GemmArgs* args, int force_generic, hipStream_t stream) {

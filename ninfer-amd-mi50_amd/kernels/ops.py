@@ -340,6 +340,8 @@ class HipOps:
         self.lib_path = lib_path or ensure_built()
         self.lib = ctypes.CDLL(self.lib_path)
         self.lib.ninfer_last_error.restype = ctypes.c_char_p
+        _need(self.lib.ninfer_gemm_args_bytes() == ctypes.sizeof(_GemmArgs),
+              f"{self.lib_path} and these bindings lay a product's arguments out differently")
         self.lib.ninfer_attention_workspace_floats.restype = ctypes.c_longlong
         self.lib.ninfer_event_create.restype = ctypes.c_void_p
         self.lib.ninfer_stream_after.argtypes = [ctypes.c_void_p] * 3

@@ -49,3 +49,15 @@ def test_height_of_dense_tiles(lib, m, n, k, gated, beside, rows):
     args = _GemmArgs(M=m, N=n, K=k, lda=k, ldc=n, in_dtype=BF16, out_dtype=BF16 if gated else 0, epilogue=gated,
                      beside=beside)
     assert lib.ninfer_gemm_tile_rows(ctypes.byref(args)) == rows
+
+
+def test_a_products_arguments_have_one_size(lib, monkeypatch):
+    """The bindings' layout against the library's, compared when the library is loaded."""
+    from ninfer_amd.kernels import ops
+    assert lib.ninfer_gemm_args_bytes() == ctypes.sizeof(ops._GemmArgs)
+
+    class Longer(ops._GemmArgs):
+        _fields_ = [("one_more", ctypes.c_int64)]
+    monkeypatch.setattr(ops, "_GemmArgs", Longer)
+    with pytest.raises(ops.KernelError, match="lay a product's arguments out differently"):
+        ops.HipOps()
