@@ -29,9 +29,10 @@
 //                    tiles are shared out evenly over its chunks.
 //
 // Latent 512 + 64, 16 heads, against blocks of four waves and 32 rows with the queries in LDS and the
-// values gathered by two-byte reads: a 2,048-token prompt 688 -> 203 us (73 GFLOP, 360 TFLOP/s; the
+// values gathered by two-byte reads: a 2,048-token prompt 688 -> 192 us (73 GFLOP, 380 TFLOP/s; the
 // LDS traffic alone, 3,000 cycles a tile of 64 keys, is 42 us), 64 requests at 1,950 to 2,600 keys
-// 188 -> 48 us (168 MB, 3.5 TB/s: a tile's way through LDS and four barriers, about 5 us a tile).
+// 188 -> 49 us (168 MB, 3.4 TB/s; at 4,000 keys, 295 MB, 71 us, 4.2 TB/s: a tile's way through LDS and
+// four barriers, about 5 us a tile).
 //
 // The rotation turns pair (i, i + n/2), or with `interleaved` pair (2i, 2i + 1), of the first
 // n = rot_n numbers of the rotated part by pos * freq[i]; cosine and sine are multiplied by `magnitude` (1 without a scaled table).
