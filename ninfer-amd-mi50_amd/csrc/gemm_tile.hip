@@ -258,8 +258,7 @@ static int launch_tile(const GemmArgs& a, hipStream_t stream) {
 // (one a CU, the last round cut into lower blocks: gemm_tile_direct), in us on this part. Measured
 // on gated products of 300 to 2,048 rows with 2 x 2,816 and 2 x 5,632 features and K 1,024 and
 // 2,048; at K 2,048, 128 rows against 256: 640 rows of 2 x 5,632 48 and 51, 768 69 and 52, 1,024 73
-// and 54, 1,116 87 and 71, 2,048 137 and 119; 1,280 of 2 x 2,816 49 and 49, 1,531 72 and 51. (256-row
-// tiles used to be taken from as many tiles as CUs on.)
+// and 54, 1,116 87 and 71, 2,048 137 and 119; 1,280 of 2 x 2,816 49 and 49, 1,531 72 and 51.
 static float dense_us_128(int blocks, int cus, int K) {
   float rounds = blocks / (2.f * cus);
   const float last = rounds - floorf(rounds);
