@@ -637,14 +637,15 @@ struct LightningForm {
 
 // What a step of T rows in S requests takes each way, in us on this part (1 us more or less where one
 // launch is enough; 16 heads of 128 x 128: the walk 26 for up to 8 rows, 31 for 64, 49 for two chunks and
-// 23 for each more, times the rounds of its blocks, one to a CU; side by side 43 and 1.2 for every chunk, 3.2
-// for every request; single rows 9 and 0.4 each). `single` of the requests, the first, bring one row each.
+// 23 for each more, times the rounds of its blocks, one to a CU, and part of one more; side by side 43 and
+// 1.2 for every chunk, 3.2 for every request; single rows 9 and 0.4 each). `single` of the requests, the
+// first, bring one row each.
 static LightningForm lightning_form(int T, int S, int single, int max_qlen, int H, int dim, int vdim) {
   const float numbers = (float)H * dim * vdim / (16 * 128 * 128), longest = (max_qlen + kLtChunk - 1) / kLtChunk;
   const bool walks = lightning_walk_lds(dim) <= 160 * 1024;
   auto walk = [&](int requests) {
     const float rounds = (float)requests * H * ((vdim + 31) / 32) / device_cu_count();
-    return (rounds > 1.f ? rounds : 1.f) * (6.f + longest * (5.f + 18.f * dim / 128));
+    return (rounds > 1.f ? rounds + 0.4f : 1.f) * (3.f + longest * (5.f + 18.f * dim / 128));
   };
   auto side = [&](int rows, int requests) {
     return 43.f + numbers * (1.2f * (rows / kLtChunk + requests) + 3.2f * requests);
@@ -712,6 +713,9 @@ static bool lightning_chunks_take(int dim, int vdim, int dtype) {
 extern "C" long long ninfer_lightning_chunk_floats(int T, int S, int single, int max_qlen, int H, int dim, int vdim,
                                                    int dtype) {
   if (!lightning_chunks_take(dim, vdim, dtype)) return -1;
+  // (keys too long for the walk: side by side costs 64 us and more, token by token 7 us a row: 4 heads of
+  // 256 x 64, 16 portions of 9 rows 82 and 63 us, one of 8 64 and 57, one of 30 68 and 181)
+  if (max_qlen < 10 && lightning_walk_lds(dim) > 160 * 1024 && lightning_seq_lds(dim, vdim) <= 160 * 1024) return -1;
   const LightningForm f = lightning_form(T, S, single, max_qlen, H, dim, vdim);
   return f.side ? lightning_most_chunks(T - f.apart, S - f.apart) * H * dim * vdim : 0;
 }

@@ -36,6 +36,17 @@ def test_lightning_sizes_that_do_not_run_in_chunks(lib):
     assert floats(128, 128, 0) == -1        # 32-bit goes token by token
 
 
+def test_lightning_short_portions(lib):
+    """Keys too long for the walk: portions of fewer than 10 rows go token by token. Many short portions of
+    shorter ones are walked, without scratch."""
+    floats = lambda rows, portions, heads, dim, vdim: lib.ninfer_lightning_chunk_floats(
+        rows * portions, portions, 0, rows, heads, dim, vdim, BF16)
+    assert floats(8, 1, 4, 256, 64) == -1 and floats(9, 16, 4, 256, 64) == -1
+    assert floats(10, 1, 4, 256, 64) > 0
+    assert floats(9, 16, 16, 128, 128) == 0
+    assert floats(9, 16, 32, 128, 128) > 0
+
+
 # (an epilogue of 1 is SwiGLU: 2 N rows of weights. 256 CUs, as the library assumes without a GPU)
 @pytest.mark.parametrize("m,n,k,gated,beside,rows", [
     (64, 5632, 2048, 1, 0, 64), (640, 5632, 2048, 1, 0, 128), (768, 5632, 2048, 1, 0, 256),
