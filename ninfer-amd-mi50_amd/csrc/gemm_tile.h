@@ -7,7 +7,7 @@
 namespace ninfer {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // Which tile does this block work on? bx: row tile (0 .. gridDim.x - 1), by: tile
 // of output features.
@@ -101,14 +101,14 @@ __device__ inline void store_quad(bf16* p, const float (&v)[4]) {
   *(bf16x4*)p = (bf16x4){(__bf16)v[0], (__bf16)v[1], (__bf16)v[2], (__bf16)v[3]};
 }
 
-// A wave's accumulators to C. The lane holds staged token row tok0 + 32 jj +
-// lane % 32, which is row row_of(..) of the tile, and of every 32-row block of
-// W rows the features 8 q + 4 (lane / 32) + r in register 4 q + r.
+// A wave's accumulators to C. The lane holds staged token row tok0 + 16 jj +
+// lane % 16, which is row row_of(..) of the tile, and of every 16-row block of
+// W rows the features 4 (lane / 16) + r in register r.
 // feat0: first output feature of the wave.
 template <int FI, int FJ, bool SWIGLU, typename TC, typename RowOf>
-__device__ inline void write_accumulators(const GemmArgs& a, const f32x16 (&acc)[FI][FJ], int tok0,
+__device__ inline void write_accumulators(const GemmArgs& a, const f32x4 (&acc)[FI][FJ], int tok0,
                                           int row0, int rows_here, int feat0, RowOf row_of) {
-  const int lane = threadIdx.x & 63, lr = lane & 31, lk = lane >> 5;
+  const int lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
   const int N = a.N;
   TC* C = (TC*)a.C;
   // four features side by side go out in one store when every such group is whole and aligned
@@ -116,117 +116,111 @@ __device__ inline void write_accumulators(const GemmArgs& a, const f32x16 (&acc)
   const bool relu_sq = a.epilogue == kEpilogueReluSq;
 #pragma unroll
   for (int jj = 0; jj < FJ; ++jj) {
-    const int r_tile = row_of(tok0 + 32 * jj + lr);
+    const int r_tile = row_of(tok0 + 16 * jj + lr);
     if (r_tile >= rows_here) continue;
     const int row = row0 + r_tile;
     const int64_t c_row = a.c_index ? a.c_index[row] : row;
     TC* crow = C + c_row * a.ldc;
     if (SWIGLU) {
 #pragma unroll
-      for (int i = 0; i < FI / 2; ++i)
+      for (int i = 0; i < FI / 2; ++i) {
+        const int f0 = feat0 + 16 * i + 4 * lk;
+        float v[4];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int f0 = feat0 + 32 * i + 8 * q + 4 * lk;
-          float v[4];
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            float g = acc[i][jj][4 * q + r], u = acc[i + (SWIGLU ? FI / 2 : 0)][jj][4 * q + r];
-            if (a.bias && f0 + r < N) {
-              g += a.bias[f0 + r];
-              u += a.bias[N + f0 + r];
-            }
-            v[r] = gated_times(g, u, a);
+        for (int r = 0; r < 4; ++r) {
+          float g = acc[i][jj][r], u = acc[i + (SWIGLU ? FI / 2 : 0)][jj][r];
+          if (a.bias && f0 + r < N) {
+            g += a.bias[f0 + r];
+            u += a.bias[N + f0 + r];
           }
-          if (whole_quads) {
-            if (f0 < N) store_quad(crow + f0, v);
-          } else {
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-              if (f0 + r < N) crow[f0 + r] = from_f32<TC>(v[r]);
-          }
+          v[r] = gated_times(g, u, a);
         }
+        if (whole_quads) {
+          if (f0 < N) store_quad(crow + f0, v);
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (f0 + r < N) crow[f0 + r] = from_f32<TC>(v[r]);
+        }
+      }
     } else {
 #pragma unroll
-      for (int i = 0; i < FI; ++i)
+      for (int i = 0; i < FI; ++i) {
+        const int f0 = feat0 + 16 * i + 4 * lk;
+        float v[4];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int f0 = feat0 + 32 * i + 8 * q + 4 * lk;
-          float v[4];
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            v[r] = acc[i][jj][4 * q + r];
-            if (a.bias && f0 + r < N) v[r] += a.bias[f0 + r];
-            v[r] = ungated_output(v[r], relu_sq);
-          }
-          if (whole_quads) {   // N % 4 == 0: the four features are in or out together
-            if (f0 < N) store_quad(crow + f0, v);
-          } else {
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-              if (f0 + r < N) crow[f0 + r] = from_f32<TC>(v[r]);
-          }
+        for (int r = 0; r < 4; ++r) {
+          v[r] = acc[i][jj][r];
+          if (a.bias && f0 + r < N) v[r] += a.bias[f0 + r];
+          v[r] = ungated_output(v[r], relu_sq);
         }
+        if (whole_quads) {   // N % 4 == 0: the four features are in or out together
+          if (f0 < N) store_quad(crow + f0, v);
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (f0 + r < N) crow[f0 + r] = from_f32<TC>(v[r]);
+        }
+      }
     }
   }
 }
 
 // The same for bf16 output, through LDS, so that rows of C are written in whole
 // 16-byte pieces side by side (the accumulator layout gives a lane 4 features
-// of 32 different rows). `stage` is LDS of the wave's own, FJ * 32 rows of
+// of 16 different rows). `stage` is LDS of the wave's own, FJ * 16 rows of
 // FEAT * 2 bytes; the 16-byte pieces of a row are stored in the order
 // v ^ (row % pieces), which spreads the lanes of a write over the banks.
 // Needs N % 8 == 0, ldc % 8 == 0 and C aligned to 16 bytes.
 template <int FI, int FJ, bool SWIGLU, typename RowOf>
-__device__ inline void write_accumulators_staged(const GemmArgs& a, const f32x16 (&acc)[FI][FJ],
+__device__ inline void write_accumulators_staged(const GemmArgs& a, const f32x4 (&acc)[FI][FJ],
                                                  unsigned char* stage, int tok0, int row0,
                                                  int rows_here, int feat0, RowOf row_of) {
   typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-  constexpr int FB = SWIGLU ? FI / 2 : FI;     // 32-feature blocks the wave writes
-  constexpr int RB = FB * 64;                  // bytes of a staged row
+  constexpr int FB = SWIGLU ? FI / 2 : FI;     // 16-feature blocks the wave writes
+  constexpr int RB = FB * 32;                  // bytes of a staged row
   constexpr int U = RB / 16;                   // 16-byte pieces of a row
-  constexpr int ROWS = FJ * 32;
+  constexpr int ROWS = FJ * 16;
   constexpr int RPI = 64 / U;                  // rows one store instruction covers
   static_assert(U >= 2 && U <= 64 && (U & (U - 1)) == 0, "row pieces");
-  const int lane = threadIdx.x & 63, lr = lane & 31, lk = lane >> 5;
+  const int lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
   const int N = a.N;
   const bool relu_sq = a.epilogue == kEpilogueReluSq;
 #pragma unroll
   for (int jj = 0; jj < FJ; ++jj) {
-    const int tok = 32 * jj + lr;
+    const int tok = 16 * jj + lr;
 #pragma unroll
-    for (int i = 0; i < FB; ++i)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        bf16x4 val;
-        if (SWIGLU) {
-          float bg[4] = {0.f, 0.f, 0.f, 0.f}, bu[4] = {0.f, 0.f, 0.f, 0.f};
-          const int f = feat0 + 32 * i + 8 * q + 4 * lk;
-          if (a.bias && f < N) {   // N % 4 == 0: four features are in or out together
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              bg[r] = a.bias[f + r];
-              bu[r] = a.bias[N + f + r];
-            }
-          }
+    for (int i = 0; i < FB; ++i) {
+      bf16x4 val;
+      if (SWIGLU) {
+        float bg[4] = {0.f, 0.f, 0.f, 0.f}, bu[4] = {0.f, 0.f, 0.f, 0.f};
+        const int f = feat0 + 16 * i + 4 * lk;
+        if (a.bias && f < N) {   // N % 4 == 0: four features are in or out together
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            const float g = acc[i][jj][4 * q + r] + bg[r];
-            const float u = acc[i + (SWIGLU ? FI / 2 : 0)][jj][4 * q + r] + bu[r];
-            val[r] = (__bf16)gated_times(g, u, a);
+            bg[r] = a.bias[f + r];
+            bu[r] = a.bias[N + f + r];
           }
-        } else {
-          float b[4] = {0.f, 0.f, 0.f, 0.f};
-          const int f = feat0 + 32 * i + 8 * q + 4 * lk;
-          if (a.bias && f < N) {   // N % 4 == 0: four features are in or out together
-#pragma unroll
-            for (int r = 0; r < 4; ++r) b[r] = a.bias[f + r];
-          }
-#pragma unroll
-          for (int r = 0; r < 4; ++r) val[r] = (__bf16)ungated_output(acc[i][jj][4 * q + r] + b[r], relu_sq);
         }
-        const int v = 4 * i + q;
-        *(bf16x4*)(stage + tok * RB + ((v ^ (tok & (U - 1))) << 4) + 8 * lk) = val;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float g = acc[i][jj][r] + bg[r];
+          const float u = acc[i + (SWIGLU ? FI / 2 : 0)][jj][r] + bu[r];
+          val[r] = (__bf16)gated_times(g, u, a);
+        }
+      } else {
+        float b[4] = {0.f, 0.f, 0.f, 0.f};
+        const int f = feat0 + 16 * i + 4 * lk;
+        if (a.bias && f < N) {   // N % 4 == 0: four features are in or out together
+#pragma unroll
+          for (int r = 0; r < 4; ++r) b[r] = a.bias[f + r];
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) val[r] = (__bf16)ungated_output(acc[i][jj][r] + b[r], relu_sq);
       }
+      const int v = 2 * i + lk / 2;   // the 16-byte piece, of which the lane has one half
+      *(bf16x4*)(stage + tok * RB + ((v ^ (tok & (U - 1))) << 4) + 8 * (lk & 1)) = val;
+    }
   }
   // row of C for staged rows lane and lane + 64 (-1: not a row of the tile)
   int c_row[(ROWS + 63) / 64];
@@ -257,10 +251,10 @@ __device__ inline bool c_takes_vectors(const GemmArgs& a) {
 
 // The epilogue of a wave: through LDS when C is bf16 and takes 16-byte pieces,
 // element by element otherwise. The caller has made sure (a barrier) that no
-// wave still reads the LDS that `stage` reuses; a wave needs FJ * 32 rows of
-// 64 bytes per 32 features it writes.
+// wave still reads the LDS that `stage` reuses; a wave needs FJ * 16 rows of
+// 32 bytes per 16 features it writes.
 template <int FI, int FJ, bool SWIGLU, typename TC, typename RowOf>
-__device__ inline void write_tile(const GemmArgs& a, const f32x16 (&acc)[FI][FJ], unsigned char* stage,
+__device__ inline void write_tile(const GemmArgs& a, const f32x4 (&acc)[FI][FJ], unsigned char* stage,
                                   int tok0, int row0, int rows_here, int feat0, RowOf row_of) {
   if constexpr (std::is_same<TC, bf16>::value) {
     if (c_takes_vectors(a)) {

@@ -4,10 +4,10 @@
 //
 // A block of NW waves owns TM rows of A (sorted rows of one expert in the
 // grouped form) and TN rows of W; the waves form a WGM x WGN grid, each with
-// FI x FJ tiles of v_mfma_f32_32x32x16_bf16. W rows are the A operand (lane l:
-// row l % 32, k = 8 (l / 32) .. +7), activation rows the B operand, so a lane's
-// accumulator holds, for token l % 32, four consecutive output features per
-// register quad: C^T[feature 8 (v / 4) + 4 (l / 32) + v % 4][token l % 32].
+// FI x FJ tiles of v_mfma_f32_16x16x32_bf16 (a fifth more of it than of 32x32x16 for the same
+// power: gemm_tile_direct.hip). W rows are the A operand (lane l: row l % 16, k = 8 (l / 16) .. +7),
+// activation rows the B operand, so a lane's accumulator holds, for token l % 16, four consecutive
+// output features: C^T[feature 4 (l / 16) + v][token l % 16].
 // With the SwiGLU epilogue the first half of a wave's W rows are gate rows and
 // the second half their up rows, so silu(g) * u is formed in registers and the
 // block writes TN / 2 output features.
@@ -33,8 +33,8 @@ __global__ __launch_bounds__(NW * 64, OCC) void gemm_tile_kernel(GemmArgs a) {
   constexpr int NT = NW * 64;            // threads
   constexpr int WGN = NW / WGM;
   constexpr int COL = TM / WGN;          // tile rows of one wave column
-  constexpr int FI = TN / WGM / 32;      // 32-row blocks of W per wave
-  constexpr int FJ = COL / 32;           // 32-row blocks of tokens per wave
+  constexpr int FI = TN / WGM / 16;      // 16-row blocks of W per wave
+  constexpr int FJ = COL / 16;           // 16-row blocks of tokens per wave
   constexpr int TPAD = TK + 8;           // bf16 per LDS row
   constexpr int VPR = TK / 8;            // 16-byte vectors per row and k tile
   constexpr int XV = TM * VPR / NT;     // vectors of A per thread and k tile
@@ -124,20 +124,20 @@ __global__ __launch_bounds__(NW * 64, OCC) void gemm_tile_kernel(GemmArgs a) {
     }
   };
 
-  f32x16 acc[FI][FJ];
+  f32x4 acc[FI][FJ];
 #pragma unroll
   for (int i = 0; i < FI; ++i)
 #pragma unroll
     for (int jj = 0; jj < FJ; ++jj)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][jj][v] = 0.f;
+      for (int v = 0; v < 4; ++v) acc[i][jj][v] = 0.f;
 
   // rows dealt to this wave's column, and its 32-row blocks that hold any
   const int col_rows = rows_here > wn ? (rows_here - wn + WGN - 1) / WGN : 0;
   const int n_jj = (col_rows + 31) / 32;
   const int tok0 = wn * COL;
 
-  const int lr = lane & 31, lk = lane >> 5;
+  const int lr = lane & 15, lk = lane >> 4;
   // products of one k tile from LDS buffer `buf`; NJ token blocks are live (a
   // compile-time count, so the loop body is straight-line code)
   auto multiply = [&](int buf, auto nj_tag) {
@@ -146,19 +146,19 @@ __global__ __launch_bounds__(NW * 64, OCC) void gemm_tile_kernel(GemmArgs a) {
     const bf16* xb = xs + buf * TM * TPAD;
     const bf16* wb = ws + buf * TN * TPAD;
 #pragma unroll
-    for (int kk = 0; kk < TK / 16; ++kk) {
+    for (int kk = 0; kk < TK / 32; ++kk) {
       bf16x8 wf[FI], xf[NJ > 0 ? NJ : 1];
 #pragma unroll
       for (int i = 0; i < FI; ++i)
-        wf[i] = *(const bf16x8*)(wb + (wm * (TN / WGM) + 32 * i + lr) * TPAD + 16 * kk + 8 * lk);
+        wf[i] = *(const bf16x8*)(wb + (wm * (TN / WGM) + 16 * i + lr) * TPAD + 32 * kk + 8 * lk);
 #pragma unroll
       for (int jj = 0; jj < NJ; ++jj)
-        xf[jj] = *(const bf16x8*)(xb + (tok0 + 32 * jj + lr) * TPAD + 16 * kk + 8 * lk);
+        xf[jj] = *(const bf16x8*)(xb + (tok0 + 16 * jj + lr) * TPAD + 32 * kk + 8 * lk);
 #pragma unroll
       for (int jj = 0; jj < NJ; ++jj)
 #pragma unroll
         for (int i = 0; i < FI; ++i)
-          acc[i][jj] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[i], xf[jj], acc[i][jj], 0, 0, 0);
+          acc[i][jj] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[i], xf[jj], acc[i][jj], 0, 0, 0);
     }
   };
   // The k loop, unrolled by the P register stages so that every stage index is
@@ -202,19 +202,16 @@ __global__ __launch_bounds__(NW * 64, OCC) void gemm_tile_kernel(GemmArgs a) {
   // one straight-line instance per count of live token blocks
   if (n_jj == 0) {
     run(std::integral_constant<int, 0>{});
-  } else if (FJ > 1 && n_jj == 1) {
-    run(std::integral_constant<int, 1>{});
-  } else if (FJ > 2 && n_jj == 2) {
-    run(std::integral_constant<int, (FJ > 2 ? 2 : FJ)>{});
-  } else if (FJ > 3 && n_jj == 3) {
-    run(std::integral_constant<int, (FJ > 3 ? 3 : FJ)>{});
+  } else if (FJ > 2 && n_jj == 1) {
+    run(std::integral_constant<int, 2>{});
   } else {
     run(std::integral_constant<int, FJ>{});
   }
+  static_assert(FJ == 2 || FJ == 4, "one instance per count of live 32-row token blocks");
 
-  static_assert(NW * FJ * 32 * FI * 64 <= 2 * (TM + TN) * TPAD * 2, "the epilogue's stage exceeds the tiles' LDS");
+  static_assert(NW * FJ * 16 * FI * 32 <= 2 * (TM + TN) * TPAD * 2, "the epilogue's stage exceeds the tiles' LDS");
   __syncthreads();   // every wave has read its last fragments: the buffers become the epilogue's stage
-  write_tile<FI, FJ, SWIGLU, TC>(a, acc, smem + wave * (FJ * 32 * FI * 64), tok0, row0, rows_here,
+  write_tile<FI, FJ, SWIGLU, TC>(a, acc, smem + wave * (FJ * 16 * FI * 32), tok0, row0, rows_here,
                                  out0 + OUT_PER_WAVE * wm, row_of);
 }
 
@@ -284,15 +281,16 @@ static float dense_us_256(int tiles, int cus, int K, bool beside) {
 // 1,024: 1,531 x 12,800 56 us in tiles of 256 and 68 in those of 128, 3,000 x 6,144 53 and 66). force_kernel
 // (tests) forces 64, 128 or 256 rows.
 static int tile_rows_of(const GemmArgs& a) {
-  if (a.force_kernel >= 1 && a.force_kernel <= 3) return 32 << a.force_kernel;
-  if (a.offsets) return kGroupedTileRows;
+  const bool direct = gemm_tile_direct_takes(a);   // (the others run in tiles of 128, counted from the offsets)
+  if (a.force_kernel >= 1 && a.force_kernel <= 3) return a.force_kernel == 3 && !direct ? 128 : 32 << a.force_kernel;
+  if (a.offsets) return direct ? kGroupedTileRows : 128;
   const bool gated = epilogue_gated(a.epilogue);
   const int n_units = gated ? 2 * a.N : a.N;   // W rows
   auto blocks = [&](int tm, int tn) { return ((a.M + tm - 1) / tm) * ((n_units + tn - 1) / tn); };
   const int cus = device_cu_count(), low = blocks(128, 128), tall = blocks(256, 256);
   if (a.M <= 64 || low < cus) return 64;   // (no taller than the rows there are)
   if (a.M <= 128) return 128;
-  return (!gated && tall >= cus) || dense_us_256(tall, cus, a.K, a.beside) < dense_us_128(low, cus, a.K) ? 256 : 128;
+  return direct && ((!gated && tall >= cus) || dense_us_256(tall, cus, a.K, a.beside) < dense_us_128(low, cus, a.K)) ? 256 : 128;
 }
 
 int gemm_tile(const GemmArgs& a, hipStream_t stream) {

@@ -1,25 +1,24 @@
 // C = A W^T for very many rows per weight matrix (bf16): 256 x 256 tiles, loaded
-// from global memory straight into LDS (global_load_lds_dwordx4), so that no
+// from global memory straight into LDS (buffer_load_dwordx4 ... lds), so that no
 // registers stage the tiles, in k tiles of 64 (whole 128-byte lines of every
 // row): two buffers for the rows of A, which neighbours share through L2, and
-// three for the rows of W, which come from HBM and are the bytes that have to
-// be on their way (all 160 KB of a CU's LDS). Dense or grouped by expert, bias or SwiGLU epilogue, as
-// the staged kernel beside it; the reference sends these products to rocBLAS
+// three for the rows of W (all 160 KB of a CU's LDS). Dense or grouped by expert, bias or
+// SwiGLU epilogue, as the staged kernel beside it; the reference sends these products to rocBLAS
 // (src/ops/linear.hip:21-35, src/models/model.hip:406-425).
 //
 // A block has 8 waves, two per SIMD, as a 4 x 2 grid; each wave owns 64 W rows
-// x 128 tokens = 2 x 4 tiles of v_mfma_f32_32x32x16_bf16 (128 accumulator
-// registers). Four waves of 128 x 128 read a third less from LDS per product,
-// but on this part a CU's loads into LDS and its matrix instructions do not
-// overlap (a block's time is their sum, whatever the order of issue), and what
-// is left to hide is the rest: with two waves per SIMD the epilogue and the
-// waits at the barrier of one run beside the products of the other (3 to 15%
-// on the experts' products of 1,024 to 8,192 tokens).
+// x 128 tokens = 4 x 8 tiles of v_mfma_f32_16x16x32_bf16 (128 accumulator
+// registers).
+// What bounds it on full tiles is power: the matrix cores alone reach 2.06 PFLOP/s with
+// this instruction and 1.75 with 32x32x16 on random operands (2.4 both on zeros): its
+// accumulators travel half as often per product. Products and fragment reads without the loads
+// from global memory run at 1.75 PFLOP/s (8,192 x 8,192, K 8,192), the whole at 1.47; with
+// 32x32x16, loads in one burst per k tile and k walks of their own per block it was 1.17.
+// Four waves of 128 x 128 read a third less from LDS and were slower (0.98).
 // A wave column multiplies only its 32-row blocks that hold rows (the tile's rows
 // fill the columns' blocks one after the other, the first column's first), and
-// after the first two k tiles a wave loads only the pieces of A that hold rows,
-// so a tile with few rows costs little more than its share: one tile height
-// serves every count of rows per expert.
+// a wave loads only the pieces of A that hold rows, so a tile with few rows costs little
+// more than its share: one tile height serves every count of rows per expert.
 //
 // LDS rows are 128 bytes (64 bf16) and unpadded, because a wave's load writes
 // 1 KB contiguously (lane l at 16 l); the eight 16-byte chunks of row r are
@@ -27,11 +26,16 @@
 // 16 rows which one pass of a fragment read touches fall into 16 different
 // 16-byte columns of the banks.
 //
-// One barrier per k tile, before its last quarter: when a wave passes the
-// barrier of tile t, tile t + 1 has landed for every wave and every wave holds
-// the last fragments of tile t in registers, so the loads of A's tile t + 2 and
-// of W's tile t + 3 may overwrite tile t. The fragments of every quarter are read while the products
-// of the quarter before run, across the barrier too.
+// A k tile is four phases: each half of its depth against the first and the second half of the
+// wave's token blocks, so that only one half's fragments of A are read ahead (64 registers of
+// fragments). The fragments of every phase are read while the products of the phase before run.
+// One barrier per k tile, before its last phase: when a wave passes the barrier of tile t, tile
+// t + 1 has landed for every wave and every wave holds the last fragments of tile t in registers,
+// so the loads of A's tile t + 2, in that last phase, may overwrite tile t; those of W's tile
+// t + 2 go one by one between the products of the first three phases (into the third buffer).
+// All loads in one burst behind the barrier keep the waves from issuing products while the CU
+// takes them in: 0.79 against 0.75 ms at 8,192 x 8,192, K 8,192, and 90 against 85 us at 2,048 rows of
+// 2 x 5,632, K 2,048.
 #include "gemm_tile.h"
 #include <type_traits>
 
@@ -42,7 +46,7 @@ constexpr int TM = 256, TN = 256;
 constexpr int WGM = 4, WGN = 2;
 constexpr int WAVES = WGM * WGN;
 constexpr int COL = TM / WGN;             // staged token rows per wave column
-constexpr int FI = TN / WGM / 32, FJ = TM / WGN / 32;
+constexpr int FI = TN / WGM / 16, FJ = TM / WGN / 16;
 }  // namespace direct
 
 // Wait until at most N of this wave's loads are under way (and, with LDS, until its LDS
@@ -66,11 +70,27 @@ struct DirectGrid {
   int parts;   // blocks of each tile of the last round
 };
 
-// (CUT: the launch cuts its last round; the others keep the shorter prologue, 3 us of 240.)
-template <int TK, bool SWIGLU, typename TC, bool CUT>
+// What the scheduler is asked for in a phase of M products: R fragment reads and L loads spread
+// evenly between them.
+template <int I, int M, int R, int L> __device__ __forceinline__ void spread_over_products() {
+  if constexpr (I < M) {
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // one MFMA
+    constexpr int r = (I + 1) * R / M - I * R / M, l = (I + 1) * L / M - I * L / M;
+    if constexpr (r > 0) __builtin_amdgcn_sched_group_barrier(0x100, r, 0);   // LDS reads
+    if constexpr (l > 0) __builtin_amdgcn_sched_group_barrier(0x010, l, 0);   // global memory
+    spread_over_products<I + 1, M, R, L>();
+  }
+}
+
+enum DirectMode : int { kDense, kDenseCut, kGrouped };   // (kDenseCut: the launch cuts its last round)
+
+template <int TK, bool SWIGLU, typename TC, DirectMode MODE>
 __global__ __launch_bounds__(direct::WAVES * 64, 1) void gemm_tile_direct_kernel(GemmArgs a, DirectGrid grid) {
+#if defined(__HIP_DEVICE_COMPILE__)   // (the host pass does not know buffer resources)
   using namespace direct;
-  constexpr int KK = TK / 16;                // parts of a k tile: one MFMA depth each
+  constexpr bool CUT = MODE == kDenseCut, GROUPED = MODE == kGrouped;
+  constexpr int KK = TK / 32;                // parts of a k tile: one MFMA depth each
+  static_assert(KK == 2, "the phases of a k tile are written for two depths");
   constexpr int ROW_BYTES = TK * 2;
   constexpr int CPR = ROW_BYTES / 16;        // 16-byte chunks of a staged row
   constexpr int RPP = 64 / CPR;              // rows of a 1 KB piece
@@ -91,7 +111,7 @@ __global__ __launch_bounds__(direct::WAVES * 64, 1) void gemm_tile_direct_kernel
     }
     dense_tile(w, grid.m_tiles, grid.n_tiles, bx, by);
   } else {
-    block_to_tile(a.offsets != nullptr, bx, by);
+    block_to_tile(GROUPED, bx, by);
   }
   int row0, row_end, group;
   // the search's three ints lie in the buffers: no load may land before every wave has them
@@ -126,18 +146,17 @@ __global__ __launch_bounds__(direct::WAVES * 64, 1) void gemm_tile_direct_kernel
     return rows0 + i < rows_here ? rows0 + i : TM;
   };
 
-  // Loads: instruction i of wave w fills the 1 KB piece i * 4 + w of the X (and
+  // Loads: instruction i of wave w fills the 1 KB piece i * 8 + w of the X (and
   // of the W) part of a buffer: RPP rows, lane l at row l / CPR, stored chunk
   // l % CPR, which holds the row's chunk (l % CPR) ^ swizzle(row), where
   // swizzle(row) = (row / (16 / CPR)) % CPR.
   constexpr int NL = TM * ROW_BYTES / 1024 / WAVES;   // load instructions per wave, k tile and operand
-  constexpr int NLT = 2 * NL;                     // loads per wave and k tile
-  // the row's part of the swizzle that the piece's number leaves: pieces i * 4 + w differ
-  // in multiples of 4 RPP rows between the loads of a wave, which the swizzle does not see
+  // the row's part of the swizzle that the piece's number leaves: pieces i * 8 + w differ
+  // in multiples of 8 RPP rows between the loads of a wave, which the swizzle does not see
   const int chunk = (lane % CPR) ^ (((wave * RPP + lane / CPR) / (16 / CPR)) % CPR);
   static_assert((WAVES * RPP / (16 / CPR)) % CPR == 0, "the loads of a wave must share their swizzle");
-  const bf16* xsrc[NL];
-  const bf16* wsrc[NL];
+  // byte offsets from A and from the group's W (gemm_tile_direct_takes: below 4 GB)
+  unsigned xoff[NL], woff[NL];
   int x_row[NL];
   unsigned x_live = 0;   // bit i: piece i of this wave's loads of A holds rows of the tile
 #pragma unroll
@@ -147,11 +166,11 @@ __global__ __launch_bounds__(direct::WAVES * 64, 1) void gemm_tile_direct_kernel
     // rows beyond the tile's last read its first row (one line, from L1): their results are
     // never stored
     x_row[i] = r < rows_here ? row0 + r : row0;
-    // a piece none of whose rows the tile has is loaded with the first tiles only (what the
-    // fragments read there afterwards goes into sums that are never stored); staged rows
-    // of a piece are neighbours in one column, so its first row decides
+    // a piece none of whose rows the tile has is not loaded (what the fragments read there goes
+    // into sums that are never stored); staged rows of a piece are neighbours in one column, so
+    // its first row decides
     if (row_of((i * WAVES + wave) * RPP) < rows_here) x_live |= 1u << i;
-    wsrc[i] = W + (int64_t)staged_w_row<TN, WGM, SWIGLU>(l, out0, N) * K + 8 * chunk;
+    woff[i] = (unsigned)staged_w_row<TN, WGM, SWIGLU>(l, out0, N) * (unsigned)(2 * K) + 16 * chunk;
   }
   if (a.a_index) {   // the index loads in flight together
     int idx[NL];
@@ -161,174 +180,202 @@ __global__ __launch_bounds__(direct::WAVES * 64, 1) void gemm_tile_direct_kernel
     for (int i = 0; i < NL; ++i) x_row[i] = idx[i] / a.a_div;
   }
 #pragma unroll
-  for (int i = 0; i < NL; ++i) xsrc[i] = (const bf16*)a.A + (int64_t)x_row[i] * a.lda + 8 * chunk;
-  typedef const __attribute__((address_space(1))) void* gptr;
+  for (int i = 0; i < NL; ++i) xoff[i] = (unsigned)x_row[i] * (unsigned)(2 * a.lda) + 16 * chunk;
+  const auto x_res = __builtin_amdgcn_make_buffer_rsrc((void*)a.A, 0, 0xffffffffu, 0x00020000);
+  const auto w_res = __builtin_amdgcn_make_buffer_rsrc((void*)W, 0, 0xffffffffu, 0x00020000);
   typedef __attribute__((address_space(3))) void* lptr;
   // Every lane of every load takes part: with some lanes switched off, a load into LDS did
   // not leave the other lanes' bytes where this layout expects them (products came out wrong).
-  // Every block walks the k tiles in a circle from a start of its own: blocks that start
-  // together would otherwise read the same columns of rows that lie a power of two apart at
-  // the same time, which fall on few memory channels.
-  const int nk_all = K / TK;
-  // (Grouped: the start depends on the expert, not on the row tile, so that a row's sum has the
-  // same order whichever tile of its expert the grouping put it in.)
-  const int phase = (int)(((a.offsets ? group : bx) * 5u + by * 3u) % (unsigned)nk_all);
-  // the t-th k tile of this block's walk: A rows into their buffer t % NBX, W rows into
-  // theirs at byte w_off (the caller's count of t % NBW)
-  auto issue_x = [&](int t) {
-    unsigned char* buf = smem + (t % NBX) * X_BYTES + wave * 1024;
-    int kt = t + phase;
-    kt = kt >= nk_all ? kt - nk_all : kt;
-#pragma unroll
-    for (int i = 0; i < NL; ++i)
-      if (t < NBX || (x_live & (1u << i)))
-        __builtin_amdgcn_global_load_lds((gptr)(xsrc[i] + kt * TK), (lptr)(buf + i * (WAVES * 1024)), 16, 0, 0);
-  };
-  // An expert whose rows fit one tile (or a dense product of one row tile) has its W panel read
-  // by this block alone: those loads
-  // are marked non-temporal (the last argument: 2), so that they do not push the rows of A,
-  // which the expert's other feature tiles read again, out of L2 (6 to 9% at 137 rows per
-  // expert; with two tiles per expert the second finds the panel in L2 and the mark costs 4%).
-  const bool w_once = a.offsets != nullptr ? row_end - a.offsets[group] <= TM : a.M <= TM;
-  auto issue_w = [&](int t, int w_off) {
-    unsigned char* buf = smem + W_BASE + w_off + wave * 1024;
-    int kt = t + phase;
-    kt = kt >= nk_all ? kt - nk_all : kt;
-    if (w_once) {
-#pragma unroll
-      for (int i = 0; i < NL; ++i)
-        __builtin_amdgcn_global_load_lds((gptr)(wsrc[i] + kt * TK), (lptr)(buf + i * (WAVES * 1024)), 16, 0, 2);
-    } else {
-#pragma unroll
-      for (int i = 0; i < NL; ++i)
-        __builtin_amdgcn_global_load_lds((gptr)(wsrc[i] + kt * TK), (lptr)(buf + i * (WAVES * 1024)), 16, 0, 0);
-    }
+  const int nk = K / TK;
+  // Where the walk over the k tiles starts. Dense: at the first for every block: the 32 blocks of an
+  // XCD share their rows of A and W through its L2 only while they walk in step (with starts of their own
+  // 8,192 x 8,192, K 8,192 took 0.94 instead of 0.85 ms, 2,048 rows of 2 x 5,632, K 2,048, 119 instead of
+  // 99 us). Grouped: in a circle from a start of the block's own, because every W panel has one reader, and
+  // blocks in step read the same columns of rows that lie a power of two apart, which fall on few memory
+  // channels (34 rows per expert, 60 x 2 x 1,408 x 2,048: 129 against 161 us). The start depends on the
+  // expert, not on the row tile, so that a row's sum has the same order whichever tile of its expert the
+  // grouping put it in.
+  const int phase = GROUPED ? (int)((group * 5u + by * 3u) % (unsigned)nk) : 0;
+  auto k_bytes = [&](int t) {   // of the t-th k tile of this block's walk
+    const int kt = t + phase;
+    return (GROUPED && kt >= nk ? kt - nk : kt) * (2 * TK);
   };
   auto next_w = [](int w_off) { return w_off == (NBW - 1) * W_BYTES ? 0 : w_off + W_BYTES; };
 
-  f32x16 acc[FI][FJ];
+  f32x4 acc[FI][FJ];
 #pragma unroll
   for (int i = 0; i < FI; ++i)
 #pragma unroll
     for (int jj = 0; jj < FJ; ++jj)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][jj][v] = 0.f;
+      for (int v = 0; v < 4; ++v) acc[i][jj][v] = 0.f;
 
   // rows dealt to this wave's column, and its 32-row blocks that hold any
   const int col_rows = wn == 0 ? rows0 : rows_here - rows0;
   const int n_jj = (col_rows + 31) / 32;
   const int tok0 = wn * COL;
 
-  // fragment addresses: lane reads row lr of a 32-row block, k chunk 2 kk + lk, stored at
-  // chunk (2 kk + lk) ^ swizzle(lr) (the block's first row is a multiple of 16)
-  const int lr = lane & 31, lk = lane >> 5;
+  // fragment addresses: lane reads row lr of a 16-row block, k chunk 4 kk + lk, stored at
+  // chunk (4 kk + lk) ^ swizzle(lr) (the block's first row is a multiple of 16)
+  const int lr = lane & 15, lk = lane >> 4;
   const int sw = (lr / (16 / CPR)) % CPR;
   const int x_lane = (tok0 + lr) * ROW_BYTES;
   const int w_lane = W_BASE + (wm * (TN / WGM) + lr) * ROW_BYTES;
   int c_part[KK];
 #pragma unroll
-  for (int kk = 0; kk < KK; ++kk) c_part[kk] = 16 * ((2 * kk + lk) ^ sw);
-  const int nk = K / TK;
+  for (int kk = 0; kk < KK; ++kk) c_part[kk] = 16 * ((4 * kk + lk) ^ sw);
 
-  auto run = [&](auto nj_tag) {
-    constexpr int NJ = decltype(nj_tag)::value;
-    constexpr int NX = NJ > 0 ? NJ : 1;
-    bf16x8 wf[2][FI], xf[2][NX];
-    // fragments of k part kk of the tile in A's buffer t % NBX and W's buffer at w_off
-    auto read_part = [&](int set, int t, int w_off, int kk) {
-      if constexpr (NJ == 0) return;
-      const unsigned char* xb = smem + (t % NBX) * X_BYTES + c_part[kk];
-      const unsigned char* wb = smem + w_off + c_part[kk];
+  // NJ: 16-row token blocks of the wave; ONCE: the panel of W has this block as its only reader
+  auto run = [&](auto nj_tag, auto once_tag) {
+    constexpr int NJ = decltype(nj_tag)::value, H0 = (NJ + 1) / 2, H1 = NJ - H0;
+    // loads i0 .. i1 - 1 of A's tile t into its buffer, and of W's tile t into the one at w_off.
+    // A panel of W that one block alone reads is loaded non-temporal (the last argument: 2), so that
+    // it does not push the rows of A, which the expert's other feature tiles read again, out of L2 (6 to
+    // 9% at 137 rows per expert; with two tiles per expert the second finds the panel in L2 and the
+    // mark costs 4%).
+    auto issue_x = [&](int t) {
+      unsigned char* buf = smem + (t % NBX) * X_BYTES + wave * 1024;
+      const int k = k_bytes(t);
 #pragma unroll
-      for (int i = 0; i < FI; ++i) wf[set][i] = *(const bf16x8*)(wb + w_lane + i * 32 * ROW_BYTES);
-#pragma unroll
-      for (int jj = 0; jj < NJ; ++jj) xf[set][jj] = *(const bf16x8*)(xb + x_lane + jj * 32 * ROW_BYTES);
+      for (int i = 0; i < NL; ++i)
+        if (x_live & (1u << i))
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(x_res, (lptr)(buf + i * (WAVES * 1024)), 16, xoff[i], k, 0, 0);
     };
-    auto multiply = [&](int set) {
+    auto issue_w = [&](int t, int w_off, auto from, auto to) {
+      unsigned char* buf = smem + W_BASE + w_off + wave * 1024;
+      const int k = k_bytes(t);
 #pragma unroll
-      for (int jj = 0; jj < NJ; ++jj)
+      for (int i = decltype(from)::value; i < decltype(to)::value; ++i)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(w_res, (lptr)(buf + i * (WAVES * 1024)), 16, woff[i], k, 0,
+                                                 decltype(once_tag)::value ? 2 : 0);
+    };
+    std::integral_constant<int, 0> i0;
+    std::integral_constant<int, NL / 2> i2;
+    std::integral_constant<int, NL * 3 / 4> i3;
+    std::integral_constant<int, NL> i4;
+    bf16x8 wf[KK][FI], x0[H0 > 0 ? H0 : 1], x1[H1 > 0 ? H1 : 1];
+    // fragments of depth kk: W's, the first and the second half of the token blocks'
+    auto read_w = [&](int kk, int w_off) {
+      if constexpr (NJ == 0) return;
+      const unsigned char* p = smem + w_off + c_part[kk] + w_lane;
+#pragma unroll
+      for (int i = 0; i < FI; ++i) wf[kk][i] = *(const bf16x8*)(p + i * 16 * ROW_BYTES);
+    };
+    auto read_x0 = [&](int kk, int t) {
+      const unsigned char* p = smem + (t % NBX) * X_BYTES + c_part[kk] + x_lane;
+#pragma unroll
+      for (int jj = 0; jj < H0; ++jj) x0[jj] = *(const bf16x8*)(p + jj * 16 * ROW_BYTES);
+    };
+    auto read_x1 = [&](int kk, int t) {
+      const unsigned char* p = smem + (t % NBX) * X_BYTES + c_part[kk] + x_lane;
+#pragma unroll
+      for (int jj = 0; jj < H1; ++jj) x1[jj] = *(const bf16x8*)(p + (H0 + jj) * 16 * ROW_BYTES);
+    };
+    auto multiply0 = [&](int kk) {
+#pragma unroll
+      for (int jj = 0; jj < H0; ++jj)
 #pragma unroll
         for (int i = 0; i < FI; ++i)
-          acc[i][jj] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[set][i], xf[set][jj], acc[i][jj], 0, 0, 0);
+          acc[i][jj] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[kk][i], x0[jj], acc[i][jj], 0, 0, 0);
     };
-    // The order of a quarter: every fragment read of the next quarter goes between two
-    // products of this one, so that it has returned when its products begin.
-    auto interleave = [&]() {
+    auto multiply1 = [&](int kk) {
 #pragma unroll
-      for (int i = 0; i < FI + NJ; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // one MFMA
-        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // one LDS read
-      }
-      __builtin_amdgcn_sched_group_barrier(0x008, FI * NJ > FI + NJ ? FI * NJ - FI - NJ : 0, 0);
+      for (int jj = 0; jj < H1; ++jj)
+#pragma unroll
+        for (int i = 0; i < FI; ++i)
+          acc[i][H0 + jj] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[kk][i], x1[jj], acc[i][H0 + jj], 0, 0, 0);
     };
-    // A wave's loads return in the order of their issue: A 0, W 0, A 1, W 1, W 2, then per
-    // tile t A t + 2, W t + 3. When tile t + 1 is needed, the only younger loads are W's
-    // tile t + 2 (NL loads), which stay on their way.
+    // A wave's loads return in the order of their issue: A 0, W 0, A 1, W 1, then per tile t W t + 2,
+    // A t + 2. When tile t + 1 is needed, the only younger loads are W's tile t + 2 (NL loads), which
+    // stay on their way. (Loads of A that are left out only make a wait longer than it has to be.)
     issue_x(0);
-    issue_w(0, 0);
+    issue_w(0, 0, i0, i4);
     if (nk > 1) {
       issue_x(1);
-      issue_w(1, W_BYTES);
+      issue_w(1, W_BYTES, i0, i4);
+      wait_loads<NL>();
+    } else {
+      wait_loads<0>();
     }
-    if (nk > 2) issue_w(2, 2 * W_BYTES);
-    if (nk > 2) wait_loads<3 * NL>();
-    else if (nk > 1) wait_loads<2 * NL>();
-    else wait_loads<0>();
     __builtin_amdgcn_s_barrier();
-    read_part(0, 0, 0, 0);
+    read_w(0, 0);
+    read_x0(0, 0);
     int t = 0, w_cur = 0;   // w_cur: where W's tile t lies
-    // steady state, free of conditions: W's tile t + 3 exists
-    for (; t + NBW < nk; ++t) {
-#pragma unroll
-      for (int kk = 0; kk + 1 < KK; ++kk) {
-        read_part((kk + 1) & 1, t, w_cur, kk + 1);
-        multiply(kk & 1);
-        interleave();
-      }
+    // steady state, free of conditions on t: the tile t + 2 exists
+    for (; t + 2 < nk; ++t) {
+      const int w_nxt = next_w(w_cur), w_far = next_w(w_nxt);
+      read_x1(0, t);
+      issue_w(t + 2, w_far, i0, i2);
+      multiply0(0);
+      spread_over_products<0, FI * H0, H1, NL / 2>();
+      read_w(1, w_cur);
+      read_x0(1, t);
+      issue_w(t + 2, w_far, i2, i3);
+      multiply1(0);
+      spread_over_products<0, FI * H1, FI + H0, NL * 3 / 4 - NL / 2>();
+      read_x1(1, t);
+      issue_w(t + 2, w_far, i3, i4);
+      multiply0(1);
+      spread_over_products<0, FI * H0, H1, NL - NL * 3 / 4>();
       // this wave's loads of tile t + 1 have landed and its last fragments of tile t are in
       // registers; after the barrier that holds for every wave, and tile t's buffers are free
       wait_loads_and_lds<NL>();
       __builtin_amdgcn_s_barrier();
-      issue_x(t + NBX);
-      issue_w(t + NBW, w_cur);
-      w_cur = next_w(w_cur);
-      read_part(KK & 1, t + 1, w_cur, 0);
-      multiply((KK - 1) & 1);
-      interleave();
+      w_cur = w_nxt;
+      issue_x(t + 2);
+      read_w(0, w_cur);
+      read_x0(0, t + 1);
+      multiply1(1);
+      spread_over_products<0, FI * H1, FI + H0, NL>();
     }
-    // the last NBW tiles: A's tile t + 2 still to issue while it exists
+    // the last two tiles: nothing left to issue
     for (; t < nk; ++t) {
-#pragma unroll
-      for (int kk = 0; kk + 1 < KK; ++kk) {
-        read_part((kk + 1) & 1, t, w_cur, kk + 1);
-        multiply(kk & 1);
-      }
-      if (t + NBW == nk) wait_loads_and_lds<NL>();   // W's last tile may stay on its way
-      else wait_loads_and_lds<0>();
+      read_x1(0, t);
+      multiply0(0);
+      read_w(1, w_cur);
+      read_x0(1, t);
+      multiply1(0);
+      read_x1(1, t);
+      multiply0(1);
+      wait_loads_and_lds<0>();
       __builtin_amdgcn_s_barrier();
-      if (t + NBX < nk) issue_x(t + NBX);
       w_cur = next_w(w_cur);
-      if (t + 1 < nk) read_part(KK & 1, t + 1, w_cur, 0);
-      multiply((KK - 1) & 1);
+      if (t + 1 < nk) {
+        read_w(0, w_cur);
+        read_x0(0, t + 1);
+      }
+      multiply1(1);
     }
   };
-  // one straight-line instance per count of live token blocks
-  switch (n_jj) {
-    case 0: run(std::integral_constant<int, 0>{}); break;
-    case 1: run(std::integral_constant<int, 1>{}); break;
-    case 2: run(std::integral_constant<int, 2>{}); break;
-    case 3: run(std::integral_constant<int, 3>{}); break;
-    default: run(std::integral_constant<int, 4>{}); break;
+  // one straight-line instance per count of live 32-row token blocks
+  auto run_rows = [&](auto once) {
+    switch (n_jj) {
+      case 0: run(std::integral_constant<int, 0>{}, once); break;
+      case 1: run(std::integral_constant<int, 2>{}, once); break;
+      case 2: run(std::integral_constant<int, 4>{}, once); break;
+      case 3: run(std::integral_constant<int, 6>{}, once); break;
+      default: run(std::integral_constant<int, 8>{}, once); break;
+    }
+  };
+  if constexpr (GROUPED) {   // an expert whose rows fit one tile
+    if (row_end - a.offsets[group] <= TM) run_rows(std::true_type{});
+    else run_rows(std::false_type{});
+  } else {
+    run_rows(std::false_type{});
   }
-  static_assert(WAVES * FJ * 32 * FI * 64 <= NBX * X_BYTES + NBW * W_BYTES, "the epilogue's stage exceeds the buffers");
+  static_assert(WAVES * FJ * 16 * FI * 32 <= NBX * X_BYTES + NBW * W_BYTES, "the epilogue's stage exceeds the buffers");
   __syncthreads();   // every wave has read its last fragments: the buffers become the epilogue's stage
-  write_tile<FI, FJ, SWIGLU, TC>(a, acc, smem + wave * (FJ * 32 * FI * 64), tok0, row0, rows_here,
+  write_tile<FI, FJ, SWIGLU, TC>(a, acc, smem + wave * (FJ * 16 * FI * 32), tok0, row0, rows_here,
                                  out0 + OUT_PER_WAVE * wm, row_of);
+#endif
 }
 
 bool gemm_tile_direct_takes(const GemmArgs& a) {
+  // (its loads take offsets of 32 bits: rows of A and the W of one group below 4 GB)
+  const int64_t four_gb = 1ll << 32, w_rows = epilogue_gated(a.epilogue) ? 2ll * a.N : a.N;
   return a.in_dtype == kBF16 && a.K % 64 == 0 && a.lda % 8 == 0 &&
-         ((uintptr_t)a.A % 16 == 0) && ((uintptr_t)a.W % 16 == 0) && a.w_group_stride % 8 == 0;
+         ((uintptr_t)a.A % 16 == 0) && ((uintptr_t)a.W % 16 == 0) && a.w_group_stride % 8 == 0 &&
+         2ll * a.M * a.lda < four_gb && 2 * w_rows * a.K < four_gb;
 }
 
 template <int TK>
@@ -347,9 +394,9 @@ static int launch_direct(const GemmArgs& a, hipStream_t stream) {
     g.whole = g.parts > 1 ? tiles - last : tiles;
     if (g.parts > 1) grid = dim3(g.whole + (tiles - g.whole) * g.parts);
   }
-#define NINFER_DIRECT_KERNEL(SW, TYPE, CUT)                                                     \
+#define NINFER_DIRECT_KERNEL(SW, TYPE, MODE)                                                    \
   do {                                                                                          \
-    auto kern = gemm_tile_direct_kernel<TK, SW, TYPE, CUT>;                                     \
+    auto kern = gemm_tile_direct_kernel<TK, SW, TYPE, MODE>;                                    \
     hipError_t e = hipFuncSetAttribute((const void*)kern,                                       \
                                        hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);  \
     if (e != hipSuccess) return set_error(-2, "gemm: cannot get %d bytes of LDS", LDS_BYTES);   \
@@ -357,8 +404,9 @@ static int launch_direct(const GemmArgs& a, hipStream_t stream) {
   } while (0)
 #define NINFER_DIRECT_LAUNCH(SW, TYPE)                                                          \
   do {                                                                                          \
-    if (g.parts > 1) NINFER_DIRECT_KERNEL(SW, TYPE, true);                                      \
-    else NINFER_DIRECT_KERNEL(SW, TYPE, false);                                                 \
+    if (a.offsets) NINFER_DIRECT_KERNEL(SW, TYPE, kGrouped);                                    \
+    else if (g.parts > 1) NINFER_DIRECT_KERNEL(SW, TYPE, kDenseCut);                            \
+    else NINFER_DIRECT_KERNEL(SW, TYPE, kDense);                                                \
   } while (0)
   if (a.out_dtype == kF32) {
     if (swiglu) NINFER_DIRECT_LAUNCH(true, float); else NINFER_DIRECT_LAUNCH(false, float);
