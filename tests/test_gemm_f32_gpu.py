@@ -40,6 +40,20 @@ def test_linear(ops, gen, m, n, k):
     assert torch.equal(one[0], more[m - 1])
 
 
+# One shape for each tile that a launch may choose (eight waves of 1 x 1, 1 x 2 and 2 x 2 tiles, four of 1 x 2,
+# 2 x 2 and 3 x 2); K whose segments are an odd number of chunks, so that a stage holds the end of one segment
+# and the start of the next, and K that ends inside a chunk.
+@pytest.mark.parametrize("m,n,k", [(17, 2048, 1412), (16, 6144, 1408), (17, 6130, 1408), (70, 6160, 1412),
+                                   (150, 6144, 1424), (40, 6130, 1412)])
+def test_every_tile(ops, gen, m, n, k):
+    x, w = (torch.randn(r, k, generator=gen, device="cuda") for r in (m, n))
+    out, one = torch.empty(m, n, device="cuda"), torch.empty(1, n, device="cuda")
+    ops.linear(x, w, out)
+    within(out, x, w, x.double() @ w.double().T)
+    ops.linear(x[m - 1:], w, one)
+    assert torch.equal(one[0], out[m - 1])
+
+
 @pytest.mark.parametrize("m,n,k", [(1, 17, 64), (40, 100, 200), (70, 1408, 256)])
 def test_gated_rows_alone_and_together(ops, gen, m, n, k):
     x, w = torch.randn(m, k, generator=gen, device="cuda"), torch.randn(2 * n, k, generator=gen, device="cuda")
