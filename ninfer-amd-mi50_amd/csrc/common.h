@@ -33,7 +33,7 @@ constexpr int kWave = 64;
 // workgroups to them in turn (block id mod 8). Kernels that share operands through L2 map
 // block ids to work with this number.
 constexpr int kXcds = 8;
-// Rows of a tall tile of the grouped products (the height of gemm_tile_direct's tiles):
+// Rows of a tall tile of the grouped products (the height of gemm_tile_direct.hip's tall tiles):
 // what routing's list of tall tiles is made for.
 constexpr int kGroupedTileRows = 256;
 

@@ -56,7 +56,7 @@ struct GemmArgs {
   const int* a_index;    // sorted row -> a_index[r] / a_div is the row of A, or null
   const int* c_index;    // sorted row -> row of C, or null
   const int* tiles16;    // grouped: {expert, first row, end row, 0} per 16-row tile, or null
-  const int* tiles_big;  // the same for the tall tiles (256 rows: gemm_tile_direct's)
+  const int* tiles_big;  // the same for the tall tiles (256 rows)
   const int* tile_counts;  // {number of 16-row tiles, number of big tiles}
   int64_t w_group_stride;  // elements between the weights of two groups
   int M;                 // rows (dense) or number of sorted rows (grouped)

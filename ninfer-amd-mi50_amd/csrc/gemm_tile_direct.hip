@@ -1,24 +1,30 @@
-// C = A W^T for very many rows per weight matrix (bf16): 256 x 256 tiles, loaded
-// from global memory straight into LDS (buffer_load_dwordx4 ... lds), so that no
-// registers stage the tiles, in k tiles of 64 (whole 128-byte lines of every
+// C = A W^T for many rows per weight matrix (bf16) on the matrix cores, dense or grouped by expert with one
+// launch for all experts, with a bias or a SwiGLU epilogue: tiles of 256 x 256, 128 x 128 or 64 x 128
+// (activation rows x rows of W), loaded from global memory straight into LDS (buffer_load_dwordx4 ... lds),
+// so that no registers stage them, in k tiles of 64 (whole 128-byte lines of every
 // row): two buffers for the rows of A, which neighbours share through L2, and
-// three for the rows of W (all 160 KB of a CU's LDS). Dense or grouped by expert, bias or
-// SwiGLU epilogue, as the staged kernel beside it; the reference sends these products to rocBLAS
+// three for the rows of W. The tall tile takes all 160 KB of a CU's LDS, of the others two blocks share a
+// CU. The reference sends these products to rocBLAS
 // (src/ops/linear.hip:21-35, src/models/model.hip:406-425).
 //
-// A block has 8 waves, two per SIMD, as a 4 x 2 grid; each wave owns 64 W rows
-// x 128 tokens = 4 x 8 tiles of v_mfma_f32_16x16x32_bf16 (128 accumulator
-// registers).
-// What bounds it on full tiles is power: the matrix cores alone reach 2.06 PFLOP/s with
+// The waves of a block form a grid, 4 x 2 (two per SIMD) for the tall tile and 2 x 2 for the others; each owns
+// 64 W rows x TM / 2 tokens in tiles of v_mfma_f32_16x16x32_bf16 (up to 128 accumulator registers). W rows
+// are the A operand (lane l: row l % 16, k = 8 (l / 16) .. + 7), activation rows the B operand, so a
+// lane's accumulator holds, for token l % 16, four consecutive output features.
+// With the SwiGLU epilogue the first half of a wave's W rows are gate rows and the second half their up rows,
+// so silu(g) * u is formed in registers and the block writes TN / 2 output features.
+// What bounds the tall tile when full is power: the matrix cores alone reach 2.06 PFLOP/s with
 // this instruction and 1.75 with 32x32x16 on random operands (2.4 both on zeros): its
 // accumulators travel half as often per product. Products and fragment reads without the loads
 // from global memory run at 1.75 PFLOP/s (8,192 x 8,192, K 8,192), the whole at 1.47; with
 // 32x32x16, loads in one burst per k tile and k walks of their own per block it was 1.17.
 // Four waves of 128 x 128 read a third less from LDS and were slower (0.98).
+// The lower tiles staged their operands through registers before: 512 rows of 2 x 5,632, K 2,048, 43 -> 36 us
+// in tiles of 128, 512 rows of 2 x 2,816 29 -> 20 in tiles of 64.
 // A wave column multiplies only its 32-row blocks that hold rows (the tile's rows
 // fill the columns' blocks one after the other, the first column's first), and
 // a wave loads only the pieces of A that hold rows, so a tile with few rows costs little
-// more than its share: one tile height serves every count of rows per expert.
+// more than its share.
 //
 // LDS rows are 128 bytes (64 bf16) and unpadded, because a wave's load writes
 // 1 KB contiguously (lane l at 16 l); the eight 16-byte chunks of row r are
@@ -40,14 +46,6 @@
 #include <type_traits>
 
 namespace ninfer {
-
-namespace direct {
-constexpr int TM = 256, TN = 256;
-constexpr int WGM = 4, WGN = 2;
-constexpr int WAVES = WGM * WGN;
-constexpr int COL = TM / WGN;             // staged token rows per wave column
-constexpr int FI = TN / WGM / 16, FJ = TM / WGN / 16;
-}  // namespace direct
 
 // Wait until at most N of this wave's loads are under way (and, with LDS, until its LDS
 // reads have returned).
@@ -84,11 +82,14 @@ template <int I, int M, int R, int L> __device__ __forceinline__ void spread_ove
 
 enum DirectMode : int { kDense, kDenseCut, kGrouped };   // (kDenseCut: the launch cuts its last round)
 
-template <int TK, bool SWIGLU, typename TC, DirectMode MODE>
-__global__ __launch_bounds__(direct::WAVES * 64, 1) void gemm_tile_direct_kernel(GemmArgs a, DirectGrid grid) {
+template <int TM, int TN, int WGM, int WGN, bool SWIGLU, typename TC, DirectMode MODE>
+__global__ __launch_bounds__(WGM * WGN * 64, TM == 256 ? 1 : 2) void gemm_tile_kernel(GemmArgs a, DirectGrid grid) {
 #if defined(__HIP_DEVICE_COMPILE__)   // (the host pass does not know buffer resources)
-  using namespace direct;
   constexpr bool CUT = MODE == kDenseCut, GROUPED = MODE == kGrouped;
+  constexpr int TK = 64;
+  constexpr int WAVES = WGM * WGN;
+  constexpr int COL = TM / WGN;                            // staged token rows per wave column
+  constexpr int FI = TN / WGM / 16, FJ = COL / 16;         // 16-row blocks of W and of tokens per wave
   constexpr int KK = TK / 32;                // parts of a k tile: one MFMA depth each
   static_assert(KK == 2, "the phases of a k tile are written for two depths");
   constexpr int ROW_BYTES = TK * 2;
@@ -127,10 +128,11 @@ __global__ __launch_bounds__(direct::WAVES * 64, 1) void gemm_tile_direct_kernel
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // the same in every lane: a scalar
   const int wm = wave % WGM, wn = wave / WGM;
   const int K = a.K, N = a.N;
-  const bf16* W = (const bf16*)a.W + (int64_t)group * a.w_group_stride;
   constexpr int OUT_PER_BLOCK = SWIGLU ? TN / 2 : TN;
   constexpr int OUT_PER_WAVE = OUT_PER_BLOCK / WGM;
   const int out0 = by * OUT_PER_BLOCK;
+  const int w_first = min(out0, N - 1);
+  const bf16* W = (const bf16*)a.W + (int64_t)group * a.w_group_stride + (int64_t)w_first * K;
   const int rows_here = min(TM, row_end - row0);
   // The tile's rows go to the two wave columns in whole blocks of 32, the first column
   // taking the odd one: a SIMD holds a wave of each column, so its matrix instructions are
@@ -146,47 +148,60 @@ __global__ __launch_bounds__(direct::WAVES * 64, 1) void gemm_tile_direct_kernel
     return rows0 + i < rows_here ? rows0 + i : TM;
   };
 
-  // Loads: instruction i of wave w fills the 1 KB piece i * 8 + w of the X (and
+  // Loads: instruction i of wave w fills the 1 KB piece i * WAVES + w of the X (and
   // of the W) part of a buffer: RPP rows, lane l at row l / CPR, stored chunk
   // l % CPR, which holds the row's chunk (l % CPR) ^ swizzle(row), where
   // swizzle(row) = (row / (16 / CPR)) % CPR.
-  constexpr int NL = TM * ROW_BYTES / 1024 / WAVES;   // load instructions per wave, k tile and operand
-  // the row's part of the swizzle that the piece's number leaves: pieces i * 8 + w differ
-  // in multiples of 8 RPP rows between the loads of a wave, which the swizzle does not see
+  constexpr int NLX = X_BYTES / 1024 / WAVES, NLW = W_BYTES / 1024 / WAVES;   // load instructions per wave and k tile
+  // the row's part of the swizzle that the piece's number leaves: pieces i * WAVES + w differ
+  // in multiples of WAVES * RPP rows between the loads of a wave, which the swizzle does not see
   const int chunk = (lane % CPR) ^ (((wave * RPP + lane / CPR) / (16 / CPR)) % CPR);
   static_assert((WAVES * RPP / (16 / CPR)) % CPR == 0, "the loads of a wave must share their swizzle");
-  // byte offsets from A and from the group's W (gemm_tile_direct_takes: below 4 GB)
-  unsigned xoff[NL], woff[NL];
-  int x_row[NL];
+  // byte offsets: of A's rows from its first one (from the tile's first, where no index gathers them), of W's
+  // from the block's first (gemm_tile_takes: below 4 GB)
+  unsigned xoff[NLX], woff[NLW];
+  int x_row[NLX];
   unsigned x_live = 0;   // bit i: piece i of this wave's loads of A holds rows of the tile
 #pragma unroll
-  for (int i = 0; i < NL; ++i) {
-    const int l = (i * WAVES + wave) * RPP + lane / CPR;
-    const int r = row_of(l);
+  for (int i = 0; i < NLX; ++i) {
+    const int r = row_of((i * WAVES + wave) * RPP + lane / CPR);
     // rows beyond the tile's last read its first row (one line, from L1): their results are
     // never stored
-    x_row[i] = r < rows_here ? row0 + r : row0;
+    x_row[i] = r < rows_here ? r : 0;
     // a piece none of whose rows the tile has is not loaded (what the fragments read there goes
     // into sums that are never stored); staged rows of a piece are neighbours in one column, so
     // its first row decides
     if (row_of((i * WAVES + wave) * RPP) < rows_here) x_live |= 1u << i;
-    woff[i] = (unsigned)staged_w_row<TN, WGM, SWIGLU>(l, out0, N) * (unsigned)(2 * K) + 16 * chunk;
+  }
+#pragma unroll
+  for (int i = 0; i < NLW; ++i) {
+    const int n = staged_w_row<TN, WGM, SWIGLU>((i * WAVES + wave) * RPP + lane / CPR, out0, N);
+    woff[i] = (unsigned)(n - w_first) * (unsigned)(2 * K) + 16 * chunk;
   }
   if (a.a_index) {   // the index loads in flight together
-    int idx[NL];
+    int idx[NLX];
 #pragma unroll
-    for (int i = 0; i < NL; ++i) idx[i] = a.a_index[x_row[i]];
+    for (int i = 0; i < NLX; ++i) idx[i] = a.a_index[row0 + x_row[i]];
 #pragma unroll
-    for (int i = 0; i < NL; ++i) x_row[i] = idx[i] / a.a_div;
+    for (int i = 0; i < NLX; ++i) x_row[i] = idx[i] / a.a_div;
   }
 #pragma unroll
-  for (int i = 0; i < NL; ++i) xoff[i] = (unsigned)x_row[i] * (unsigned)(2 * a.lda) + 16 * chunk;
-  const auto x_res = __builtin_amdgcn_make_buffer_rsrc((void*)a.A, 0, 0xffffffffu, 0x00020000);
+  for (int i = 0; i < NLX; ++i) xoff[i] = (unsigned)x_row[i] * (unsigned)(2 * a.lda) + 16 * chunk;
+  const bf16* A = (const bf16*)a.A + (a.a_index ? 0 : (int64_t)row0 * a.lda);
+  const auto x_res = __builtin_amdgcn_make_buffer_rsrc((void*)A, 0, 0xffffffffu, 0x00020000);
   const auto w_res = __builtin_amdgcn_make_buffer_rsrc((void*)W, 0, 0xffffffffu, 0x00020000);
   typedef __attribute__((address_space(3))) void* lptr;
   // Every lane of every load takes part: with some lanes switched off, a load into LDS did
   // not leave the other lanes' bytes where this layout expects them (products came out wrong).
-  const int nk = K / TK;
+  // a product cut along K: this block's k tiles are kt_first .. kt_first + nk - 1, and its
+  // sums go to part blockIdx.z of C
+  int nk = K / TK, kt_first = 0;
+  if (!GROUPED && a.k_parts > 1) {
+    const int per = (nk + a.k_parts - 1) / a.k_parts;
+    kt_first = blockIdx.z * per;
+    nk = min(per, nk - kt_first);
+    a.C = (TC*)a.C + (int64_t)blockIdx.z * a.M * a.ldc;
+  }
   // Where the walk over the k tiles starts. Dense: at the first for every block: the 32 blocks of an
   // XCD share their rows of A and W through its L2 only while they walk in step (with starts of their own
   // 8,192 x 8,192, K 8,192 took 0.94 instead of 0.85 ms, 2,048 rows of 2 x 5,632, K 2,048, 119 instead of
@@ -198,7 +213,7 @@ __global__ __launch_bounds__(direct::WAVES * 64, 1) void gemm_tile_direct_kernel
   const int phase = GROUPED ? (int)((group * 5u + by * 3u) % (unsigned)nk) : 0;
   auto k_bytes = [&](int t) {   // of the t-th k tile of this block's walk
     const int kt = t + phase;
-    return (GROUPED && kt >= nk ? kt - nk : kt) * (2 * TK);
+    return (kt_first + (GROUPED && kt >= nk ? kt - nk : kt)) * (2 * TK);
   };
   auto next_w = [](int w_off) { return w_off == (NBW - 1) * W_BYTES ? 0 : w_off + W_BYTES; };
 
@@ -237,7 +252,7 @@ __global__ __launch_bounds__(direct::WAVES * 64, 1) void gemm_tile_direct_kernel
       unsigned char* buf = smem + (t % NBX) * X_BYTES + wave * 1024;
       const int k = k_bytes(t);
 #pragma unroll
-      for (int i = 0; i < NL; ++i)
+      for (int i = 0; i < NLX; ++i)
         if (x_live & (1u << i))
           __builtin_amdgcn_raw_ptr_buffer_load_lds(x_res, (lptr)(buf + i * (WAVES * 1024)), 16, xoff[i], k, 0, 0);
     };
@@ -250,9 +265,9 @@ __global__ __launch_bounds__(direct::WAVES * 64, 1) void gemm_tile_direct_kernel
                                                  decltype(once_tag)::value ? 2 : 0);
     };
     std::integral_constant<int, 0> i0;
-    std::integral_constant<int, NL / 2> i2;
-    std::integral_constant<int, NL * 3 / 4> i3;
-    std::integral_constant<int, NL> i4;
+    std::integral_constant<int, NLW / 2> i2;
+    std::integral_constant<int, NLW * 3 / 4> i3;
+    std::integral_constant<int, NLW> i4;
     bf16x8 wf[KK][FI], x0[H0 > 0 ? H0 : 1], x1[H1 > 0 ? H1 : 1];
     // fragments of depth kk: W's, the first and the second half of the token blocks'
     auto read_w = [&](int kk, int w_off) {
@@ -286,14 +301,14 @@ __global__ __launch_bounds__(direct::WAVES * 64, 1) void gemm_tile_direct_kernel
           acc[i][H0 + jj] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[kk][i], x1[jj], acc[i][H0 + jj], 0, 0, 0);
     };
     // A wave's loads return in the order of their issue: A 0, W 0, A 1, W 1, then per tile t W t + 2,
-    // A t + 2. When tile t + 1 is needed, the only younger loads are W's tile t + 2 (NL loads), which
+    // A t + 2. When tile t + 1 is needed, the only younger loads are W's tile t + 2 (NLW loads), which
     // stay on their way. (Loads of A that are left out only make a wait longer than it has to be.)
     issue_x(0);
     issue_w(0, 0, i0, i4);
     if (nk > 1) {
       issue_x(1);
       issue_w(1, W_BYTES, i0, i4);
-      wait_loads<NL>();
+      wait_loads<NLW>();
     } else {
       wait_loads<0>();
     }
@@ -307,26 +322,26 @@ __global__ __launch_bounds__(direct::WAVES * 64, 1) void gemm_tile_direct_kernel
       read_x1(0, t);
       issue_w(t + 2, w_far, i0, i2);
       multiply0(0);
-      spread_over_products<0, FI * H0, H1, NL / 2>();
+      spread_over_products<0, FI * H0, H1, NLW / 2>();
       read_w(1, w_cur);
       read_x0(1, t);
       issue_w(t + 2, w_far, i2, i3);
       multiply1(0);
-      spread_over_products<0, FI * H1, FI + H0, NL * 3 / 4 - NL / 2>();
+      spread_over_products<0, FI * H1, FI + H0, NLW * 3 / 4 - NLW / 2>();
       read_x1(1, t);
       issue_w(t + 2, w_far, i3, i4);
       multiply0(1);
-      spread_over_products<0, FI * H0, H1, NL - NL * 3 / 4>();
+      spread_over_products<0, FI * H0, H1, NLW - NLW * 3 / 4>();
       // this wave's loads of tile t + 1 have landed and its last fragments of tile t are in
       // registers; after the barrier that holds for every wave, and tile t's buffers are free
-      wait_loads_and_lds<NL>();
+      wait_loads_and_lds<NLW>();
       __builtin_amdgcn_s_barrier();
       w_cur = w_nxt;
       issue_x(t + 2);
       read_w(0, w_cur);
       read_x0(0, t + 1);
       multiply1(1);
-      spread_over_products<0, FI * H1, FI + H0, NL>();
+      spread_over_products<0, FI * H1, FI + H0, NLX>();
     }
     // the last two tiles: nothing left to issue
     for (; t < nk; ++t) {
@@ -349,13 +364,11 @@ __global__ __launch_bounds__(direct::WAVES * 64, 1) void gemm_tile_direct_kernel
   };
   // one straight-line instance per count of live 32-row token blocks
   auto run_rows = [&](auto once) {
-    switch (n_jj) {
-      case 0: run(std::integral_constant<int, 0>{}, once); break;
-      case 1: run(std::integral_constant<int, 2>{}, once); break;
-      case 2: run(std::integral_constant<int, 4>{}, once); break;
-      case 3: run(std::integral_constant<int, 6>{}, once); break;
-      default: run(std::integral_constant<int, 8>{}, once); break;
-    }
+    if (n_jj == 0) run(std::integral_constant<int, 0>{}, once);
+    else if (FJ > 2 && n_jj == 1) run(std::integral_constant<int, 2>{}, once);
+    else if (FJ > 4 && n_jj == 2) run(std::integral_constant<int, (FJ > 4 ? 4 : FJ)>{}, once);
+    else if (FJ > 6 && n_jj == 3) run(std::integral_constant<int, (FJ > 6 ? 6 : FJ)>{}, once);
+    else run(std::integral_constant<int, FJ>{}, once);
   };
   if constexpr (GROUPED) {   // an expert whose rows fit one tile
     if (row_end - a.offsets[group] <= TM) run_rows(std::true_type{});
@@ -370,60 +383,63 @@ __global__ __launch_bounds__(direct::WAVES * 64, 1) void gemm_tile_direct_kernel
 #endif
 }
 
-bool gemm_tile_direct_takes(const GemmArgs& a) {
-  // (its loads take offsets of 32 bits: rows of A and the W of one group below 4 GB)
-  const int64_t four_gb = 1ll << 32, w_rows = epilogue_gated(a.epilogue) ? 2ll * a.N : a.N;
-  return a.in_dtype == kBF16 && a.K % 64 == 0 && a.lda % 8 == 0 &&
-         ((uintptr_t)a.A % 16 == 0) && ((uintptr_t)a.W % 16 == 0) && a.w_group_stride % 8 == 0 &&
-         2ll * a.M * a.lda < four_gb && 2 * w_rows * a.K < four_gb;
+// K a whole number of k tiles of 64; byte offsets of 32 bits: the rows of A that an index gathers, and from a
+// gate row to its up row.
+bool gemm_tile_takes(const GemmArgs& a) {
+  const int64_t four_gb = 1ll << 32;
+  return a.in_dtype == kBF16 && a.K % 64 == 0 && a.lda % 8 == 0 && ((uintptr_t)a.A % 16 == 0) &&
+         ((uintptr_t)a.W % 16 == 0) && a.w_group_stride % 8 == 0 &&
+         2 * (a.a_index ? (int64_t)a.M : 256) * a.lda < four_gb &&
+         2 * ((epilogue_gated(a.epilogue) ? a.N : 0) + 256ll) * a.K < four_gb;
 }
 
-template <int TK>
-static int launch_direct(const GemmArgs& a, hipStream_t stream) {
-  using namespace direct;
-  constexpr int LDS_BYTES = (2 * TM + 3 * TN) * TK * 2;
+template <int TM, int TN, int WGM, int WGN>
+static int launch_tiles(const GemmArgs& a, hipStream_t stream) {
+  constexpr int LDS_BYTES = (2 * TM + 3 * TN) * 64 * 2;
   const bool swiglu = epilogue_gated(a.epilogue);
   int m_tiles = (a.M + TM - 1) / TM + (a.offsets ? a.groups : 0);
   if (a.offsets) m_tiles = (m_tiles + kXcds - 1) / kXcds * kXcds;   // block_to_tile's bijection
   const int per_block = swiglu ? TN / 2 : TN;
   DirectGrid g = {m_tiles, (a.N + per_block - 1) / per_block, 0, 1};
-  dim3 grid(g.m_tiles, g.n_tiles);
-  if (!a.offsets) {
+  dim3 grid(g.m_tiles, g.n_tiles, a.k_parts > 1 ? a.k_parts : 1);
+  if (TM == 256 && !a.offsets && a.k_parts <= 1) {
     const int tiles = g.m_tiles * g.n_tiles, cus = device_cu_count(), last = tiles % cus;
     g.parts = a.beside || last == 0 || tiles < cus ? 1 : 4 * last <= cus ? 4 : 2 * last <= cus ? 2 : 1;
     g.whole = g.parts > 1 ? tiles - last : tiles;
     if (g.parts > 1) grid = dim3(g.whole + (tiles - g.whole) * g.parts);
   }
-#define NINFER_DIRECT_KERNEL(SW, TYPE, MODE)                                                    \
+#define NINFER_TILE_KERNEL(SW, TYPE, MODE)                                                      \
   do {                                                                                          \
-    auto kern = gemm_tile_direct_kernel<TK, SW, TYPE, MODE>;                                    \
+    auto kern = gemm_tile_kernel<TM, TN, WGM, WGN, SW, TYPE, MODE>;                             \
     hipError_t e = hipFuncSetAttribute((const void*)kern,                                       \
                                        hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);  \
     if (e != hipSuccess) return set_error(-2, "gemm: cannot get %d bytes of LDS", LDS_BYTES);   \
-    kern<<<grid, direct::WAVES * 64, LDS_BYTES, stream>>>(a, g);                                \
+    kern<<<grid, WGM * WGN * 64, LDS_BYTES, stream>>>(a, g);                                    \
   } while (0)
-#define NINFER_DIRECT_LAUNCH(SW, TYPE)                                                          \
+#define NINFER_TILE_LAUNCH(SW, TYPE)                                                            \
   do {                                                                                          \
-    if (a.offsets) NINFER_DIRECT_KERNEL(SW, TYPE, kGrouped);                                    \
-    else if (g.parts > 1) NINFER_DIRECT_KERNEL(SW, TYPE, kDenseCut);                            \
-    else NINFER_DIRECT_KERNEL(SW, TYPE, kDense);                                                \
+    if (a.offsets) NINFER_TILE_KERNEL(SW, TYPE, kGrouped);                                      \
+    else if (TM == 256 && g.parts > 1) NINFER_TILE_KERNEL(SW, TYPE, (TM == 256 ? kDenseCut : kDense)); \
+    else NINFER_TILE_KERNEL(SW, TYPE, kDense);                                                  \
   } while (0)
   if (a.out_dtype == kF32) {
-    if (swiglu) NINFER_DIRECT_LAUNCH(true, float); else NINFER_DIRECT_LAUNCH(false, float);
+    if (swiglu) NINFER_TILE_LAUNCH(true, float); else NINFER_TILE_LAUNCH(false, float);
   } else {
-    if (swiglu) NINFER_DIRECT_LAUNCH(true, bf16); else NINFER_DIRECT_LAUNCH(false, bf16);
+    if (swiglu) NINFER_TILE_LAUNCH(true, bf16); else NINFER_TILE_LAUNCH(false, bf16);
   }
-#undef NINFER_DIRECT_KERNEL
-#undef NINFER_DIRECT_LAUNCH
+#undef NINFER_TILE_KERNEL
+#undef NINFER_TILE_LAUNCH
   NINFER_LAUNCH_CHECK();
   return 0;
 }
 
-int gemm_tile_direct(const GemmArgs& a, hipStream_t stream) {
-  static_assert(direct::TM == kGroupedTileRows, "the grouped tile lists are made for this height");
-  // k tiles of 64: measured faster than tiles of 32 in twice the buffers (whole 128-byte
-  // lines per row beat the deeper queue of loads)
-  return launch_direct<64>(a, stream);
+// k tiles of 64 at every height: measured faster than tiles of 32 in twice the buffers (whole
+// 128-byte lines per row beat the deeper queue of loads).
+int gemm_tile_rows(const GemmArgs& a, int rows, hipStream_t stream) {
+  static_assert(kGroupedTileRows == 256, "the grouped tile lists are made for the tall tiles");
+  if (rows == 256) return launch_tiles<256, 256, 4, 2>(a, stream);
+  if (rows == 128) return launch_tiles<128, 128, 2, 2>(a, stream);
+  return launch_tiles<64, 128, 2, 2>(a, stream);
 }
 
 }  // namespace ninfer
