@@ -2,7 +2,7 @@
 // launch for all experts, with a bias or a SwiGLU epilogue: tiles of 256 x 256, 128 x 128 or 64 x 128
 // (activation rows x rows of W), loaded from global memory straight into LDS (buffer_load_dwordx4 ... lds),
 // so that no registers stage them, in k tiles of 64 (whole 128-byte lines of every
-// row): two buffers for the rows of A, which neighbours share through L2, and
+// row): two buffers for the rows of A, which neighbours share through L2 (three in the lowest tile), and
 // three for the rows of W. The tall tile takes all 160 KB of a CU's LDS, of the others two blocks share a
 // CU. The reference sends these products to rocBLAS
 // (src/ops/linear.hip:21-35, src/models/model.hip:406-425).
@@ -41,7 +41,11 @@
 // t + 2 go one by one between the products of the first three phases (into the third buffer).
 // All loads in one burst behind the barrier keep the waves from issuing products while the CU
 // takes them in: 0.79 against 0.75 ms at 8,192 x 8,192, K 8,192, and 90 against 85 us at 2,048 rows of
-// 2 x 5,632, K 2,048.
+// 2 x 5,632, K 2,048. With a third buffer for the rows of A as well (the lowest tile, whose two blocks still
+// fit a CU) all loads of tile t + 2 go into the first three phases and have two k tiles' time to land: 512 rows
+// of 2 x 5,632 50 -> 42 us, 32 groups of 16 rows of 2 x 1,408 69 -> 60. More buffers and one block a CU gain
+// nothing (64 rows of 2 x 5,632 20.7 us with three, 20.7 with six): few blocks wait for their chains of
+// fragment reads and barriers.
 #include "gemm_tile.h"
 #include <type_traits>
 
@@ -82,8 +86,8 @@ template <int I, int M, int R, int L> __device__ __forceinline__ void spread_ove
 
 enum DirectMode : int { kDense, kDenseCut, kGrouped };   // (kDenseCut: the launch cuts its last round)
 
-template <int TM, int TN, int WGM, int WGN, bool SWIGLU, typename TC, DirectMode MODE>
-__global__ __launch_bounds__(WGM * WGN * 64, TM == 256 ? 1 : 2) void gemm_tile_kernel(GemmArgs a, DirectGrid grid) {
+template <int TM, int TN, int WGM, int WGN, int NBX, int NBW, bool SWIGLU, typename TC, DirectMode MODE>
+__global__ __launch_bounds__(WGM * WGN * 64, (NBX * TM + NBW * TN) * 128 > 80 * 1024 ? 1 : 2) void gemm_tile_kernel(GemmArgs a, DirectGrid grid) {
 #if defined(__HIP_DEVICE_COMPILE__)   // (the host pass does not know buffer resources)
   constexpr bool CUT = MODE == kDenseCut, GROUPED = MODE == kGrouped;
   constexpr int TK = 64;
@@ -96,7 +100,9 @@ __global__ __launch_bounds__(WGM * WGN * 64, TM == 256 ? 1 : 2) void gemm_tile_k
   constexpr int CPR = ROW_BYTES / 16;        // 16-byte chunks of a staged row
   constexpr int RPP = 64 / CPR;              // rows of a 1 KB piece
   constexpr int X_BYTES = TM * ROW_BYTES, W_BYTES = TN * ROW_BYTES;
-  constexpr int NBX = 2, NBW = 3;            // buffers of A rows, of W rows
+  // buffers of A rows and of W rows: two and three, or three of both
+  constexpr bool EVEN = NBX == NBW;
+  static_assert((EVEN || NBX == 2) && NBW == 3, "buffers");
   constexpr int W_BASE = NBX * X_BYTES;
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
 
@@ -216,6 +222,7 @@ __global__ __launch_bounds__(WGM * WGN * 64, TM == 256 ? 1 : 2) void gemm_tile_k
     return (kt_first + (GROUPED && kt >= nk ? kt - nk : kt)) * (2 * TK);
   };
   auto next_w = [](int w_off) { return w_off == (NBW - 1) * W_BYTES ? 0 : w_off + W_BYTES; };
+  auto next_x = [](int x_off) { return x_off == (NBX - 1) * X_BYTES ? 0 : x_off + X_BYTES; };
 
   f32x4 acc[FI][FJ];
 #pragma unroll
@@ -248,12 +255,12 @@ __global__ __launch_bounds__(WGM * WGN * 64, TM == 256 ? 1 : 2) void gemm_tile_k
     // it does not push the rows of A, which the expert's other feature tiles read again, out of L2 (6 to
     // 9% at 137 rows per expert; with two tiles per expert the second finds the panel in L2 and the
     // mark costs 4%).
-    auto issue_x = [&](int t) {
-      unsigned char* buf = smem + (t % NBX) * X_BYTES + wave * 1024;
+    auto issue_x = [&](int t, int x_off, auto from, auto to) {
+      unsigned char* buf = smem + x_off + wave * 1024;
       const int k = k_bytes(t);
 #pragma unroll
-      for (int i = 0; i < NLX; ++i)
-        if (x_live & (1u << i))
+      for (int i = decltype(from)::value; i < decltype(to)::value; ++i)
+        if (EVEN || (x_live & (1u << i)))   // (EVEN: all, so that a wait is a constant count)
           __builtin_amdgcn_raw_ptr_buffer_load_lds(x_res, (lptr)(buf + i * (WAVES * 1024)), 16, xoff[i], k, 0, 0);
     };
     auto issue_w = [&](int t, int w_off, auto from, auto to) {
@@ -268,6 +275,7 @@ __global__ __launch_bounds__(WGM * WGN * 64, TM == 256 ? 1 : 2) void gemm_tile_k
     std::integral_constant<int, NLW / 2> i2;
     std::integral_constant<int, NLW * 3 / 4> i3;
     std::integral_constant<int, NLW> i4;
+    std::integral_constant<int, NLX> x4;
     bf16x8 wf[KK][FI], x0[H0 > 0 ? H0 : 1], x1[H1 > 0 ? H1 : 1];
     // fragments of depth kk: W's, the first and the second half of the token blocks'
     auto read_w = [&](int kk, int w_off) {
@@ -276,13 +284,13 @@ __global__ __launch_bounds__(WGM * WGN * 64, TM == 256 ? 1 : 2) void gemm_tile_k
 #pragma unroll
       for (int i = 0; i < FI; ++i) wf[kk][i] = *(const bf16x8*)(p + i * 16 * ROW_BYTES);
     };
-    auto read_x0 = [&](int kk, int t) {
-      const unsigned char* p = smem + (t % NBX) * X_BYTES + c_part[kk] + x_lane;
+    auto read_x0 = [&](int kk, int x_off) {
+      const unsigned char* p = smem + x_off + c_part[kk] + x_lane;
 #pragma unroll
       for (int jj = 0; jj < H0; ++jj) x0[jj] = *(const bf16x8*)(p + jj * 16 * ROW_BYTES);
     };
-    auto read_x1 = [&](int kk, int t) {
-      const unsigned char* p = smem + (t % NBX) * X_BYTES + c_part[kk] + x_lane;
+    auto read_x1 = [&](int kk, int x_off) {
+      const unsigned char* p = smem + x_off + c_part[kk] + x_lane;
 #pragma unroll
       for (int jj = 0; jj < H1; ++jj) x1[jj] = *(const bf16x8*)(p + (H0 + jj) * 16 * ROW_BYTES);
     };
@@ -300,64 +308,107 @@ __global__ __launch_bounds__(WGM * WGN * 64, TM == 256 ? 1 : 2) void gemm_tile_k
         for (int i = 0; i < FI; ++i)
           acc[i][H0 + jj] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[kk][i], x1[jj], acc[i][H0 + jj], 0, 0, 0);
     };
-    // A wave's loads return in the order of their issue: A 0, W 0, A 1, W 1, then per tile t W t + 2,
-    // A t + 2. When tile t + 1 is needed, the only younger loads are W's tile t + 2 (NLW loads), which
-    // stay on their way. (Loads of A that are left out only make a wait longer than it has to be.)
-    issue_x(0);
-    issue_w(0, 0, i0, i4);
-    if (nk > 1) {
-      issue_x(1);
-      issue_w(1, W_BYTES, i0, i4);
-      wait_loads<NLW>();
-    } else {
-      wait_loads<0>();
-    }
-    __builtin_amdgcn_s_barrier();
-    read_w(0, 0);
-    read_x0(0, 0);
-    int t = 0, w_cur = 0;   // w_cur: where W's tile t lies
-    // steady state, free of conditions on t: the tile t + 2 exists
-    for (; t + 2 < nk; ++t) {
-      const int w_nxt = next_w(w_cur), w_far = next_w(w_nxt);
-      read_x1(0, t);
-      issue_w(t + 2, w_far, i0, i2);
-      multiply0(0);
-      spread_over_products<0, FI * H0, H1, NLW / 2>();
-      read_w(1, w_cur);
-      read_x0(1, t);
-      issue_w(t + 2, w_far, i2, i3);
-      multiply1(0);
-      spread_over_products<0, FI * H1, FI + H0, NLW * 3 / 4 - NLW / 2>();
-      read_x1(1, t);
-      issue_w(t + 2, w_far, i3, i4);
-      multiply0(1);
-      spread_over_products<0, FI * H0, H1, NLW - NLW * 3 / 4>();
-      // this wave's loads of tile t + 1 have landed and its last fragments of tile t are in
-      // registers; after the barrier that holds for every wave, and tile t's buffers are free
-      wait_loads_and_lds<NLW>();
+    int t = 0, x_cur = 0, w_cur = 0;   // w_cur, x_cur: where W's and A's tile t lie
+    if constexpr (EVEN) {
+      // Tile t + 2 is loaded during tile t's first three phases into the buffers that tile t - 1 has
+      // left. When tile t + 1 is needed, its loads stay on their way.
+      constexpr int PER = NLX + NLW;
+      issue_x(0, 0, i0, x4);
+      issue_w(0, 0, i0, i4);
+      if (nk > 1) {
+        issue_x(1, X_BYTES, i0, x4);
+        issue_w(1, W_BYTES, i0, i4);
+        wait_loads<PER>();
+      } else {
+        wait_loads<0>();
+      }
       __builtin_amdgcn_s_barrier();
-      w_cur = w_nxt;
-      issue_x(t + 2);
-      read_w(0, w_cur);
-      read_x0(0, t + 1);
-      multiply1(1);
-      spread_over_products<0, FI * H1, FI + H0, NLX>();
+      read_w(0, 0);
+      read_x0(0, 0);
+      int x_far = 2 * X_BYTES, w_far = 2 * W_BYTES;
+      for (; t + 2 < nk; ++t) {
+        read_x1(0, x_cur);
+        issue_w(t + 2, w_far, i0, i2);
+        multiply0(0);
+        spread_over_products<0, FI * H0, H1, NLW / 2>();
+        read_w(1, w_cur);
+        read_x0(1, x_cur);
+        issue_w(t + 2, w_far, i2, i4);
+        multiply1(0);
+        spread_over_products<0, FI * H1, FI + H0, NLW - NLW / 2>();
+        read_x1(1, x_cur);
+        issue_x(t + 2, x_far, i0, x4);
+        multiply0(1);
+        spread_over_products<0, FI * H0, H1, NLX>();
+        wait_loads_and_lds<PER>();
+        __builtin_amdgcn_s_barrier();
+        x_far = x_cur, w_far = w_cur;
+        x_cur = next_x(x_cur), w_cur = next_w(w_cur);
+        read_w(0, w_cur);
+        read_x0(0, x_cur);
+        multiply1(1);
+        spread_over_products<0, FI * H1, FI + H0, 0>();
+      }
+    } else {
+      // A wave's loads return in the order of their issue: A 0, W 0, A 1, W 1, then per tile t W t + 2,
+      // A t + 2. When tile t + 1 is needed, the only younger loads are W's tile t + 2 (NLW loads), which
+      // stay on their way. (Loads of A that are left out only make a wait longer than it has to be.)
+      issue_x(0, 0, i0, x4);
+      issue_w(0, 0, i0, i4);
+      if (nk > 1) {
+        issue_x(1, X_BYTES, i0, x4);
+        issue_w(1, W_BYTES, i0, i4);
+        wait_loads<NLW>();
+      } else {
+        wait_loads<0>();
+      }
+      __builtin_amdgcn_s_barrier();
+      read_w(0, 0);
+      read_x0(0, 0);
+      // steady state, free of conditions on t: the tile t + 2 exists
+      for (; t + 2 < nk; ++t) {
+        const int w_nxt = next_w(w_cur), w_far = next_w(w_nxt);
+        read_x1(0, x_cur);
+        issue_w(t + 2, w_far, i0, i2);
+        multiply0(0);
+        spread_over_products<0, FI * H0, H1, NLW / 2>();
+        read_w(1, w_cur);
+        read_x0(1, x_cur);
+        issue_w(t + 2, w_far, i2, i3);
+        multiply1(0);
+        spread_over_products<0, FI * H1, FI + H0, NLW * 3 / 4 - NLW / 2>();
+        read_x1(1, x_cur);
+        issue_w(t + 2, w_far, i3, i4);
+        multiply0(1);
+        spread_over_products<0, FI * H0, H1, NLW - NLW * 3 / 4>();
+        // this wave's loads of tile t + 1 have landed and its last fragments of tile t are in
+        // registers; after the barrier that holds for every wave, and tile t's buffers are free
+        wait_loads_and_lds<NLW>();
+        __builtin_amdgcn_s_barrier();
+        issue_x(t + 2, x_cur, i0, x4);
+        w_cur = w_nxt;
+        x_cur = next_x(x_cur);
+        read_w(0, w_cur);
+        read_x0(0, x_cur);
+        multiply1(1);
+        spread_over_products<0, FI * H1, FI + H0, NLX>();
+      }
     }
     // the last two tiles: nothing left to issue
     for (; t < nk; ++t) {
-      read_x1(0, t);
+      read_x1(0, x_cur);
       multiply0(0);
       read_w(1, w_cur);
-      read_x0(1, t);
+      read_x0(1, x_cur);
       multiply1(0);
-      read_x1(1, t);
+      read_x1(1, x_cur);
       multiply0(1);
       wait_loads_and_lds<0>();
       __builtin_amdgcn_s_barrier();
-      w_cur = next_w(w_cur);
+      x_cur = next_x(x_cur), w_cur = next_w(w_cur);
       if (t + 1 < nk) {
         read_w(0, w_cur);
-        read_x0(0, t + 1);
+        read_x0(0, x_cur);
       }
       multiply1(1);
     }
@@ -393,9 +444,9 @@ bool gemm_tile_takes(const GemmArgs& a) {
          2 * ((epilogue_gated(a.epilogue) ? a.N : 0) + 256ll) * a.K < four_gb;
 }
 
-template <int TM, int TN, int WGM, int WGN>
+template <int TM, int TN, int WGM, int WGN, int NBX, int NBW>
 static int launch_tiles(const GemmArgs& a, hipStream_t stream) {
-  constexpr int LDS_BYTES = (2 * TM + 3 * TN) * 64 * 2;
+  constexpr int LDS_BYTES = (NBX * TM + NBW * TN) * 64 * 2;
   const bool swiglu = epilogue_gated(a.epilogue);
   int m_tiles = (a.M + TM - 1) / TM + (a.offsets ? a.groups : 0);
   if (a.offsets) m_tiles = (m_tiles + kXcds - 1) / kXcds * kXcds;   // block_to_tile's bijection
@@ -410,7 +461,7 @@ static int launch_tiles(const GemmArgs& a, hipStream_t stream) {
   }
 #define NINFER_TILE_KERNEL(SW, TYPE, MODE)                                                      \
   do {                                                                                          \
-    auto kern = gemm_tile_kernel<TM, TN, WGM, WGN, SW, TYPE, MODE>;                             \
+    auto kern = gemm_tile_kernel<TM, TN, WGM, WGN, NBX, NBW, SW, TYPE, MODE>;                             \
     hipError_t e = hipFuncSetAttribute((const void*)kern,                                       \
                                        hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);  \
     if (e != hipSuccess) return set_error(-2, "gemm: cannot get %d bytes of LDS", LDS_BYTES);   \
@@ -437,9 +488,9 @@ static int launch_tiles(const GemmArgs& a, hipStream_t stream) {
 // 128-byte lines per row beat the deeper queue of loads).
 int gemm_tile_rows(const GemmArgs& a, int rows, hipStream_t stream) {
   static_assert(kGroupedTileRows == 256, "the grouped tile lists are made for the tall tiles");
-  if (rows == 256) return launch_tiles<256, 256, 4, 2>(a, stream);
-  if (rows == 128) return launch_tiles<128, 128, 2, 2>(a, stream);
-  return launch_tiles<64, 128, 2, 2>(a, stream);
+  if (rows == 256) return launch_tiles<256, 256, 4, 2, 2, 3>(a, stream);
+  if (rows == 128) return launch_tiles<128, 128, 2, 2, 2, 3>(a, stream);
+  return launch_tiles<64, 128, 2, 2, 3, 3>(a, stream);
 }
 
 }  // namespace ninfer
