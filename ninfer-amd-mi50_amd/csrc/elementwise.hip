@@ -81,7 +81,8 @@ __device__ __forceinline__ void store_vec(bf16* p, const float* f) {
 template <typename T, int VEC>
 __global__ void rmsnorm_kernel(float* __restrict__ x, const T* __restrict__ delta, MoeSum ms,
                                const float* __restrict__ gain, T* __restrict__ out,
-                               const int* __restrict__ rows, int H, float eps, int center) {
+                               const int* __restrict__ rows, int H, float eps, int center,
+                               const float* __restrict__ gain2, T* __restrict__ out2) {
   constexpr int G = kNormPerThread / VEC;   // groups per thread
   __shared__ float red[16];
   int64_t r_out = blockIdx.x;
@@ -182,6 +183,12 @@ __global__ void rmsnorm_kernel(float* __restrict__ x, const T* __restrict__ delt
 #pragma unroll
       for (int e = 0; e < VEC; ++e) o[e] = (vals[c][e] - mean) * inv * gv[e];
       store_vec<VEC>(orow + i, o);
+      if (gain2) {   // the same rows under a second norm's gain
+        load_vec<VEC>(gain2 + i, gv);
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) o[e] = (vals[c][e] - mean) * inv * gv[e];
+        store_vec<VEC>(out2 + r_out * H + i, o);
+      }
     }
   }
 }
@@ -447,12 +454,13 @@ extern "C" int ninfer_embed(const int* tokens, const void* table, float* out, in
 
 // moe_* describe an optional weighted sum of rows added before the norm (all
 // null / 0: none): y [rows * k, H], w [rows, k], shared [rows, H], gate logits
-// with stride gate_stride.
+// with stride gate_stride. gain2, out2: a second norm of the same rows, with another gain (null: none).
 extern "C" int ninfer_rmsnorm(float* x, const void* delta, const float* gain, void* out,
                               const int* rows, int n_rows, int H, float eps, int dtype,
                               const void* moe_y, const float* moe_w, const void* moe_shared,
                               const float* moe_gate, int moe_gate_stride, int moe_k,
-                              int center, hipStream_t stream) {
+                              int center, const float* gain2, void* out2, hipStream_t stream) {
+  NINFER_REQUIRE((!gain2) == (!out2), "rmsnorm: a second gain and its output come together or not at all");
   NINFER_REQUIRE(n_rows > 0 && H > 0, "rmsnorm: rows=%d H=%d must be positive", n_rows, H);
   NINFER_REQUIRE(dtype == kF32 || dtype == kBF16, "rmsnorm: unknown dtype %d", dtype);
   NINFER_REQUIRE(H <= 1024 * kNormPerThread, "rmsnorm: width %d exceeds %d", H,
@@ -462,7 +470,7 @@ extern "C" int ninfer_rmsnorm(float* x, const void* delta, const float* gain, vo
   // groups of 4 consecutive elements when every row pointer stays 16-byte aligned
   auto aligned = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
   const bool vec = H % 4 == 0 && aligned(x) && aligned(delta) && aligned(out) && aligned(gain) &&
-                   aligned(moe_y) && aligned(moe_shared);
+                   aligned(moe_y) && aligned(moe_shared) && aligned(gain2) && aligned(out2);
   // few elements per thread (short chains of loads), at most 1024 threads
   int per_thread = vec ? 4 : 2;
   int block = ((H + per_thread - 1) / per_thread + 63) / 64 * 64;
@@ -471,17 +479,17 @@ extern "C" int ninfer_rmsnorm(float* x, const void* delta, const float* gain, vo
   if (dtype == kF32) {
     if (vec)
       rmsnorm_kernel<float, 4><<<n_rows, block, 0, stream>>>(x, (const float*)delta, ms, gain,
-                                                            (float*)out, rows, H, eps, center);
+                                                            (float*)out, rows, H, eps, center, gain2, (float*)out2);
     else
       rmsnorm_kernel<float, 1><<<n_rows, block, 0, stream>>>(x, (const float*)delta, ms, gain,
-                                                            (float*)out, rows, H, eps, center);
+                                                            (float*)out, rows, H, eps, center, gain2, (float*)out2);
   } else {
     if (vec)
       rmsnorm_kernel<bf16, 4><<<n_rows, block, 0, stream>>>(x, (const bf16*)delta, ms, gain,
-                                                           (bf16*)out, rows, H, eps, center);
+                                                           (bf16*)out, rows, H, eps, center, gain2, (bf16*)out2);
     else
       rmsnorm_kernel<bf16, 1><<<n_rows, block, 0, stream>>>(x, (const bf16*)delta, ms, gain,
-                                                           (bf16*)out, rows, H, eps, center);
+                                                           (bf16*)out, rows, H, eps, center, gain2, (bf16*)out2);
   }
   NINFER_LAUNCH_CHECK();
   return 0;

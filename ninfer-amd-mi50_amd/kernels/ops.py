@@ -502,11 +502,13 @@ class HipOps:
             ctypes.c_void_p(_ptr(pos_table)), 0 if pos_table is None else pos_table.shape[0],
             self._stream()))
 
-    def rmsnorm(self, x, gain, eps, out, delta=None, rows=None, rows_sum=None, center=False):
+    def rmsnorm(self, x, gain, eps, out, delta=None, rows=None, rows_sum=None, center=False,
+                second=None):
         """out = norm(x [+ delta] [+ rows_sum]); `rows_sum` is a weighted sum of
         rows (an object with y, weights, shared, gate) added on the fly. norm(v) =
         v rsqrt(mean(v^2) + eps) gain, or with `center` the layer norm without a bias,
-        (v - mean(v)) rsqrt(mean((v - mean(v))^2) + eps) gain."""
+        (v - mean(v)) rsqrt(mean((v - mean(v))^2) + eps) gain. `second` = (gain, out): the same
+        rows under another gain, by the same kernel."""
         _dev(x, "x", torch.float32, 2)
         _dev(gain, "gain", torch.float32, 1)
         _dev(out, "out", dims=2)
@@ -520,6 +522,12 @@ class HipOps:
             _need(out.shape[0] == rows.shape[0], "rmsnorm: out has the wrong number of rows")
         else:
             _need(out.shape[0] == x.shape[0], "rmsnorm: out has the wrong number of rows")
+        gain2 = out2 = None
+        if second is not None:
+            _dev(second[0], "second gain", torch.float32, 1)
+            _dev(second[1], "second out", out.dtype, 2)
+            _need(second[0].shape[0] == h and second[1].shape == out.shape, "rmsnorm: the second norm's sizes")
+            gain2, out2 = second[0].data_ptr(), second[1].data_ptr()
         my, mw, msh, mg, mgs, mk = None, None, None, None, 0, 0
         if rows_sum is not None:
             mk, mgs = self._check_rows_sum(rows_sum, x.shape[0], h, out.dtype)
@@ -530,7 +538,11 @@ class HipOps:
             ctypes.c_void_p(gain.data_ptr()), ctypes.c_void_p(out.data_ptr()),
             ctypes.c_void_p(_ptr(rows)), out.shape[0], h, ctypes.c_float(eps), _DT[out.dtype],
             ctypes.c_void_p(my), ctypes.c_void_p(mw), ctypes.c_void_p(msh), ctypes.c_void_p(mg),
-            mgs, mk, 1 if center else 0, self._stream()))
+            mgs, mk, 1 if center else 0, ctypes.c_void_p(gain2), ctypes.c_void_p(out2), self._stream()))
+
+    def rmsnorm_two(self, x, gain, eps, out, gain2, out2, delta=None, rows_sum=None, center=False):
+        """Two norms of the same rows that differ in their gains alone, by one kernel."""
+        self.rmsnorm(x, gain, eps, out, delta, None, rows_sum, center, second=(gain2, out2))
 
     @staticmethod
     def _check_rows_sum(rs, t, h, dtype):

@@ -16,6 +16,7 @@ import torch
 from ..weights.source import TensorSpec
 from .base import (Block, CallInfo, FeedForward, Mixer, Norm, Part, PendingRows, ReadyRows,
                    StepContext, WeightBinder, plain_rows, settle)
+from .norm import RMSNorm
 
 
 class PreNormBlock(Block):
@@ -266,9 +267,12 @@ class ParallelBlock(Block):
         return g
 
     def forward(self, ctx: StepContext, residual, pending, call: CallInfo):
-        h = self.norm.forward(ctx, residual, pending)
-        h2 = h
-        if self.ff_norm is not None:
+        if self.ff_norm is None:
+            h2 = h = self.norm.forward(ctx, residual, pending)
+        elif isinstance(self.norm, RMSNorm):
+            h, h2 = self.norm.forward_two(ctx, residual, pending, self.ff_norm)
+        else:
+            h = self.norm.forward(ctx, residual, pending)
             h2 = self.ff_norm.forward(ctx, residual, None)
         a = plain_rows(ctx, self.mixer.forward(ctx, h, residual, call))
         f = self.feed_forward.forward(ctx, h2, residual) if self.feed_forward is not None else None
@@ -277,8 +281,9 @@ class ParallelBlock(Block):
             return None
         if self.mixer_scale is not None or self.ff_scale is not None:
             raise ValueError("learned column factors beside gates or a multiplier are not built")
-        ctx.ops.gated_sum_add(residual, a, self._gate(ctx, h, self.mixer_gate), self.mixer_gate_bias,
-                              f, self._gate(ctx, h2, self.ff_gate), self.ff_gate_bias, self.mult)
+        with ctx.ops.together():   # few rows: both gates in one launch
+            g1, g2 = self._gate(ctx, h, self.mixer_gate), self._gate(ctx, h2, self.ff_gate)
+        ctx.ops.gated_sum_add(residual, a, g1, self.mixer_gate_bias, f, g2, self.ff_gate_bias, self.mult)
         return None
 
 

@@ -82,9 +82,10 @@ class GatedLinearAttention(Mixer):
         ops = ctx.ops
         qk, _, v, _ = self._widths()
         proj = ctx.empty((ctx.T, 2 * qk + 2 * v))
-        ops.linear(x, self.w_in, proj)
         low = ctx.empty((ctx.T, self.w_a1.shape[0]))
-        ops.linear(x, self.w_a1, low)
+        with ops.together():   # few rows: one launch
+            ops.linear(x, self.w_in, proj)
+            ops.linear(x, self.w_a1, low)
         z = ctx.empty((ctx.T, qk), torch.float32)     # the decay's logits, 32-bit from here on
         ops.linear(low, self.w_a2, z, bias=self.b_a2)
         o = ctx.empty((ctx.T, v), torch.float32)

@@ -121,16 +121,20 @@ class LatentAttention(Mixer):
         cache = call.cache
         T, H, R, rd = ctx.T, self.heads, self.kv_rank, self.rot_dim
         q = ctx.empty((T, H * (self.dim + rd)))
+        dkv_g = ctx.empty((T, self.w_dkv_g.shape[0]))
+        # (few rows: the two products of x in one launch)
         if self.q_rank is None:
-            ops.linear(x, self.w_q, q)
+            with ops.together():
+                ops.linear(x, self.w_q, q)
+                ops.linear(x, self.w_dkv_g, dkv_g)
         else:   # the queries' latent: projected into 32-bit, normed there, then up
             cq32 = ctx.empty((T, self.q_rank), torch.float32)
-            ops.linear(x, self.w_dq, cq32)
+            with ops.together():
+                ops.linear(x, self.w_dq, cq32)
+                ops.linear(x, self.w_dkv_g, dkv_g)
             cq = ctx.empty((T, self.q_rank))
             ops.rmsnorm(cq32, self.q_norm_w, self.eps, cq)
             ops.linear(cq, self.w_q, q)
-        dkv_g = ctx.empty((T, self.w_dkv_g.shape[0]))
-        ops.linear(x, self.w_dkv_g, dkv_g)
         q_abs = ctx.empty((T, H, R + rd), torch.float32)
         ops.latent_kv_write(dkv_g, q, q_abs, cache["latent"], cache.block_table, ctx, H, self.dim,
                             R, rd, self.norm_w, self.eps, self.position.table(),

@@ -65,3 +65,21 @@ def test_sums(ops, dtype, width, k, t):
         got.append((res, gated))
     for u, v in zip(*got):
         assert torch.equal(u, v) and not torch.equal(u, x)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("width", [2048, 1022, 7])
+@pytest.mark.parametrize("center", [False, True])
+def test_two_norms_of_the_same_rows(ops, dtype, width, center):
+    """Bit for bit what the two norms give one after the other, with a sum before the first."""
+    gen = torch.Generator(device="cuda").manual_seed(width)
+    x = torch.randn(5, width, generator=gen, device="cuda")
+    gains = torch.randn(2, width, generator=gen, device="cuda")
+    delta = torch.randn(5, width, generator=gen, device="cuda").to(dtype)
+    once, twice = x.clone(), x.clone()
+    want, got = ([torch.empty(5, width, dtype=dtype, device="cuda") for _ in range(2)] for _ in range(2))
+    ops.rmsnorm(once, gains[0].contiguous(), 1e-6, want[0], delta=delta, center=center)
+    ops.rmsnorm(once, gains[1].contiguous(), 1e-6, want[1], center=center)
+    ops.rmsnorm_two(twice, gains[0].contiguous(), 1e-6, got[0], gains[1].contiguous(), got[1], delta=delta,
+                    center=center)
+    assert torch.equal(once, twice) and torch.equal(want[0], got[0]) and torch.equal(want[1], got[1])
