@@ -28,6 +28,9 @@
 //                    (steps of few rows would otherwise leave most of the GPU idle); a request's
 //                    tiles are shared out evenly over its chunks.
 //
+//   latent_attention_rows  the blocks of 64 rows for latents of 256 or 512 numbers with 32 or 64 turned
+//                    ones: four waves that keep 16 rows each, nothing between them but the keys.
+//
 // Latent 512 + 64, 16 heads, against blocks of four waves and 32 rows with the queries in LDS and the
 // values gathered by two-byte reads: a 2,048-token prompt 688 -> 192 us (73 GFLOP, 380 TFLOP/s; the
 // LDS traffic alone, 3,000 cycles a tile of 64 keys, is 42 us), 64 requests at 1,950 to 2,600 keys
@@ -320,6 +323,12 @@ static void latent_tile_split(const LatentArgs& a, int rows, int* tiles, int* n_
   *n_chunks = want < 1 ? 1 : want;
 }
 
+// Has the row a form of its own in the kernel whose waves keep whole rows? Latents of 256 or 512 numbers with 32
+// or 64 turned ones behind them; the output's rows in pieces of 8 bytes.
+static bool latent_rows_takes(const LatentArgs& a) {
+  return (a.R == 256 || a.R == 512) && (a.rd == 32 || a.rd == 64) && ((uintptr_t)a.out % 8 == 0);
+}
+
 // What a step takes in blocks of 16 or 64 rows, in us on this part: rounds of blocks, each a start and
 // a walk over its keys, and the merge of chunks. Low blocks start sooner (queries, first tile, output:
 // 10 against 24 us at 576 numbers a row) and meet a tile of 64 keys in 0.9 us while few of them run and
@@ -332,8 +341,9 @@ static float latent_tile_us(const LatentArgs& a, int rows, int half) {
   latent_tile_split(a, rows, &tiles, &n_chunks);
   const int key_tiles = (a.max_kv_len + kLatKeys - 1) / kLatKeys, steps = (key_tiles + n_chunks - 1) / n_chunks;
   const float filled = (float)tiles * n_chunks / device_cu_count(), numbers = half / 18.f;
-  const float start = rows == 16 ? 10.f : 24.f;
-  const float step = rows == 16 ? 0.9f + 1.2f * (filled < 1.f ? filled : 1.f) : 3.6f;
+  const float high = latent_rows_takes(a) ? 0.7f : 1.f;   // (the kernel whose waves keep whole rows)
+  const float start = rows == 16 ? 10.f : 24.f * high;
+  const float step = rows == 16 ? 0.9f + 1.2f * (filled < 1.f ? filled : 1.f) : 3.6f * high;
   const float round = start * (0.4f + 0.6f * numbers) + steps * step * numbers;
   return round * (filled > 1.f ? filled : 1.f) + (n_chunks > 1 ? 6.f : 0.f);
 }
@@ -649,6 +659,286 @@ __global__ __launch_bounds__(kLatThreads, 2) void latent_attention_tile_kernel(L
   }
 }
 
+// The same in blocks of 64 rows for cached rows of 32 QF numbers whose first 16 NC are the latent: four
+// waves of 16 (token, head) rows each, which keep their queries, their running maxima and sums and all
+// columns of their outputs in registers, so that nothing passes between waves but the keys. Tiles
+// of 32 keys come straight into LDS (global_load_lds), the next one while this one is multiplied: one barrier a
+// tile, two blocks a CU. S^T = K Q^T leaves the lane (c, g) with row c and keys 4 g .. + 3 of each 16; the
+// products with the values take the keys in that order (the transposing reads follow it), so the
+// probabilities go from the scores to the operand without leaving the lane. A row's exponent reference
+// follows its maximum only in jumps of 2^8, so that the 4 NC output registers are rescaled rarely.
+// What bounds it is the LDS (68 KB of operands a wave and tile at 512 + 64 numbers, twice the matrix cores' time)
+// and, with 251 registers, reads only two or three products ahead. Against the kernel above: prompts of 2,048
+// tokens, 16 heads, 512 + 64 numbers 202 -> 140 us; 8 heads, 256 + 32 numbers 111 -> 74; 512 tokens behind 2,000 cached
+// ones 190 -> 146; 64 requests of one row and 40 heads at 2,500 keys 83 -> 67.
+// In LDS rows are unpadded (a load writes 1 KB side by side): the 16-byte piece p of key k lies at
+// p ^ x(k) (lat_swizzle), chosen on the global side, so that the 16 keys of a fragment read fall into
+// different columns of the banks.
+constexpr int kLatRowsKeys = 32;
+template <int PIECES_A_ROW> __device__ __forceinline__ int lat_swizzle(int key) {
+  if constexpr (PIECES_A_ROW % 8 == 0) return (key >> 1) & 7;
+  else return (key >> 2) & 3;   // (a multiple of 4: QF steps of 32 numbers)
+}
+
+template <int QF, int NC>
+__global__ __launch_bounds__(256, 2) void latent_attention_rows_kernel(LatentArgs a, LatentTilePlan pl) {
+#if defined(__HIP_DEVICE_COMPILE__)   // (the host pass does not know buffer resources)
+  constexpr int ROWS = 64, KT = kLatRowsKeys, CPR = 4 * QF, DK = 32 * QF;
+  constexpr int LOADS = (8 * CPR + 63) / 64;          // of a wave and tile: 8 keys, 1 KB a load
+  constexpr int TILE = 4 * LOADS * 1024;
+  static_assert(KT == 32 && 16 * DK < 65536, "a wave's keys");
+  extern __shared__ float smem[];
+  unsigned char* Ks = (unsigned char*)smem;           // [2][TILE]
+  int (*page_s)[KT] = (int (*)[KT])(Ks + 2 * TILE);   // [2][KT]
+  const int R = a.R, H = a.Hq;
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = lane & 15, g = lane >> 4;
+
+  // Which request and which of its row tiles: as in the kernel above, the longest first.
+  int s = -1, lt = 0, total = 0;
+  for (int i = 0; i < a.S; ++i)
+    total += ((a.seq_row_start[i + 1] - a.seq_row_start[i]) * H + ROWS - 1) / ROWS;
+  int left = total - 1 - (int)blockIdx.x;
+  for (int i = 0; i < a.S && left >= 0; ++i) {
+    const int nt = ((a.seq_row_start[i + 1] - a.seq_row_start[i]) * H + ROWS - 1) / ROWS;
+    if (left < nt) {
+      s = i;
+      lt = left;
+      break;
+    }
+    left -= nt;
+  }
+  if (s < 0) return;
+  const int chunk_id = blockIdx.y;
+  const int row0 = a.seq_row_start[s];
+  const int n_flat = (a.seq_row_start[s + 1] - row0) * H;
+  const int pos0 = a.seq_pos0[s];
+  const int f0 = lt * ROWS;
+  const int rows_here = min(ROWS, n_flat - f0);
+  const int tok_first = f0 / H, tok_last = (f0 + rows_here - 1) / H;
+  const int pos_last = pos0 + tok_last;
+  const int lo_first = a.window > 0 ? max(0, pos0 + tok_first - a.window + 1) : 0;
+  const int first_tile = lo_first / kLatKeys, n_tiles = pos_last / kLatKeys + 1 - first_tile;
+  const int per_chunk = (n_tiles + pl.n_chunks - 1) / pl.n_chunks;
+  const int k_begin = (first_tile + min(chunk_id * per_chunk, n_tiles)) * kLatKeys;
+  const int k_end = min((first_tile + min((chunk_id + 1) * per_chunk, n_tiles)) * kLatKeys, pos_last + 1);
+  const int* bt = a.block_table + (int64_t)s * a.bt_stride;
+  const __bf16* pool = (const __bf16*)a.pool;
+
+  typedef const __attribute__((address_space(1))) void* gptr;
+  typedef __attribute__((address_space(3))) void* lptr;
+  // Wave w fetches keys 8 w .. + 7 of a tile, CPR loads of 8 lanes' worth a key: LOADS of 64 lanes, of which the
+  // last may reach into padding. Where all keys of the tile are seen by some row and pages hold 8 keys or more, the
+  // wave's keys lie side by side in one page: a scalar base and the lanes' offsets, which no tile changes.
+  // Elsewhere (the first and last tile, small pages, pages that the table does not hold) key by key: keys
+  // outside what the rows see from the nearest that they do (their probabilities are 0).
+  auto place = [&](int ln, int j, int& key, int& piece) {
+    const int f = 8 * CPR % 64 ? min(64 * j + ln, 8 * CPR - 1) : 64 * j + ln;
+    key = f / CPR;
+    piece = (f % CPR) ^ lat_swizzle<CPR>(8 * w + key);
+  };
+  // Byte offsets of two loads each, where they fit the registers; with 32 tiles of output columns they are
+  // formed again in every tile (kept they spill: 2,048 tokens of 16 heads, 512 + 64 numbers, 254 against 140 us; formed
+  // again at 8 heads of 256 + 32 84 against 74).
+  constexpr bool KEPT = NC <= 16;
+  unsigned off2[KEPT ? (LOADS + 1) / 2 : 1] = {};
+  if constexpr (KEPT) {
+#pragma unroll
+    for (int j = 0; j < LOADS; ++j) {
+      int key, piece;
+      place(lane, j, key, piece);
+      off2[j / 2] |= (unsigned)(key * (2 * DK) + 16 * piece) << (j % 2 ? 16 : 0);
+    }
+  }
+  auto fetch = [&](int kt, int buf) {
+    unsigned char* to = Ks + buf * TILE + w * (LOADS * 1024);
+    int ln = lane;
+    asm volatile("" : "+v"(ln));   // (so that nothing formed from it is kept)
+    const int page = __builtin_amdgcn_readfirstlane(page_s[buf][8 * w]);
+    if (kt >= lo_first && kt + KT - 1 <= pos_last && a.page_size >= 8 && page >= 0) {
+      const __bf16* base = pool + ((int64_t)page * a.page_size + ((kt + 8 * w) & (a.page_size - 1))) * DK;
+      const auto res = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, 16 * DK, 0x00020000);   // (8 keys)
+#pragma unroll
+      for (int j = 0; j < LOADS; ++j) {
+        unsigned at;
+        if constexpr (KEPT) {
+          at = j % 2 ? off2[j / 2] >> 16 : off2[j / 2] & 0xffff;
+        } else {
+          int key, piece;
+          place(ln, j, key, piece);
+          at = key * (2 * DK) + 16 * piece;
+        }
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(res, (lptr)(to + j * 1024), 16, at, 0, 0, 0);
+      }
+      return;
+    }
+#pragma unroll 1
+    for (int j = 0; j < LOADS; ++j) {
+      int key, piece;
+      place(ln, j, key, piece);
+      const int kp = min(max(kt + 8 * w + key, lo_first), pos_last), pg = page_s[buf][8 * w + key];
+      const __bf16* at = pool + ((int64_t)pg * a.page_size + (kp & (a.page_size - 1))) * DK + 8 * piece;
+      __builtin_amdgcn_global_load_lds((gptr)(pg >= 0 ? (const void*)at : (const void*)&kLatNoKey), (lptr)(to + j * 1024),
+                                       16, 0, 0);
+    }
+  };
+  // pages of a tile's keys, looked up by lanes of wave 0 two tiles ahead
+  auto page_of = [&](int kt) { return bt[min(max(kt + (lane & (KT - 1)), lo_first), pos_last) >> pl.page_shift]; };
+  int page_next = 0;
+  if (w == 0 && k_begin < k_end) {
+    if (lane < KT) {
+      page_s[0][lane] = page_of(k_begin);
+      page_s[1][lane] = page_of(k_begin + KT);
+    }
+    page_next = page_of(k_begin + 2 * KT);
+  }
+  __syncthreads();
+  if (k_begin < k_end) fetch(k_begin, 0);
+
+  // Q' as the products' operand, rounded to bfloat16 once: lane (c, g) has row 16 w + c, numbers 8 g .. of a step
+  const int my = 16 * w + c, f_row = f0 + min(my, rows_here - 1);
+  lat_bf16x8 qf[QF];
+  {
+    const float* src = a.q_abs + ((int64_t)(row0 + f_row / H) * H + f_row % H) * DK + 8 * g;
+#pragma unroll
+    for (int st = 0; st < QF; ++st) {
+      const lat_f32x4 lo = *(const lat_f32x4*)(src + 32 * st), up = *(const lat_f32x4*)(src + 32 * st + 4);
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        qf[st][x] = (__bf16)lo[x];
+        qf[st][4 + x] = (__bf16)up[x];
+      }
+    }
+  }
+  const int my_pos = pos0 + f_row / H, my_lo = a.window > 0 ? max(0, my_pos - a.window + 1) : 0;
+  const float scale2 = a.scale * kLatLog2e;
+  float m_ref = -INFINITY, l_run = 0.f;   // (of the scores times log2 e); l: this lane's keys alone
+  lat_f32x4 acc[NC];
+#pragma unroll
+  for (int ct = 0; ct < NC; ++ct) acc[ct] = lat_f32x4{0.f, 0.f, 0.f, 0.f};
+
+  // Fragment addresses in a tile. Keys 16 i + c: piece 4 st + g, at (4 st + g) ^ x; x's third bit swaps the
+  // steps 2 n and 2 n + 1. (x is the same for keys 16 apart.)
+  const int xk = lat_swizzle<CPR>(c), k_low = (c >> 3) * (LOADS * 1024) + (c & 7) * (16 * CPR) + 16 * (g ^ (xk & 3)), k_swap = 64 * (xk >> 2);
+  // Values: transposing reads, lane at key 4 g + c / 4 (and 16 further), columns 4 (c % 4) of a tile of 16
+  // (pieces 2 ct and 2 ct + 1; x moves them within a group of eight, so four tiles have addresses of their own)
+  const int v_key = 4 * g + (c >> 2), xv = lat_swizzle<CPR>(v_key);
+  int v_at[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    v_at[j] = (v_key >> 3) * (LOADS * 1024) + (v_key & 7) * (16 * CPR) + 8 * (c & 1) + 16 * ((2 * j + ((c >> 1) & 1)) ^ xv);
+  typedef __attribute__((address_space(3))) lat_short4* trptr;
+
+  int turn = 0;
+  for (int kt = k_begin; kt < k_end; kt += KT, turn ^= 1) {
+    // this wave's part of the tile has landed, and after the barrier everybody's has; everybody has also
+    // read the tile before, whose place the next one takes
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (kt + KT < k_end) fetch(kt + KT, turn ^ 1);
+    if (w == 0) {   // (the places of this tile's pages were read one tile ago)
+      if (lane < KT) page_s[turn][lane] = page_next;
+      page_next = page_of(kt + 3 * KT);
+    }
+    const unsigned char* tile = Ks + turn * TILE;
+    // (fragments are read two steps, and values three tiles of columns, ahead of their products; the fences
+    // keep the compiler from moving the reads back to them)
+    lat_f32x4 sc[2] = {};
+    lat_bf16x8 kf[3][2];
+    auto read_keys = [&](int st) {
+      const unsigned char* at = tile + k_low + 64 * st + (st % 2 ? -k_swap : k_swap);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) kf[st % 3][i] = *(const lat_bf16x8*)(at + i * (2 * LOADS * 1024));
+    };
+    read_keys(0);
+    read_keys(1);
+#pragma unroll
+    for (int st = 0; st < QF; ++st) {
+      if (st + 2 < QF) read_keys(st + 2);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        sc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[st % 3][i], qf[st], sc[i], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    float sv[8], mx = -INFINITY;
+#pragma unroll
+    for (int x = 0; x < 8; ++x) {
+      const int kp = kt + 16 * (x / 4) + 4 * g + x % 4;
+      const float v = sc[x / 4][x % 4] * scale2;
+      sv[x] = kp <= my_pos && kp >= my_lo ? v : -INFINITY;
+      mx = fmaxf(mx, sv[x]);
+    }
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    if (__any(mx > m_ref + 8.f)) {   // (also a row's first visible key: its reference is minus infinity)
+      const float m_new = fmaxf(m_ref, mx);
+      const float al = m_new == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m_ref - m_new);
+      l_run *= al;
+#pragma unroll
+      for (int ct = 0; ct < NC; ++ct) acc[ct] *= al;
+      m_ref = m_new;
+    }
+    const float ref = m_ref == -INFINITY ? 0.f : m_ref;   // nothing seen so far: all terms are 0
+    lat_bf16x8 pf;
+#pragma unroll
+    for (int x = 0; x < 8; ++x) {
+      const float p = __builtin_amdgcn_exp2f(sv[x] - ref);
+      pf[x] = (__bf16)p;
+      l_run += p;
+    }
+    lat_short4 vf[4][2];
+    auto read_values = [&](int ct) {
+      const unsigned char* v = tile + v_at[ct % 4] + 128 * (ct / 4);
+      vf[ct % 4][0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((trptr)v);
+      vf[ct % 4][1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((trptr)(v + 2 * LOADS * 1024));
+    };
+#pragma unroll
+    for (int ct = 0; ct < 3; ++ct) read_values(ct);
+#pragma unroll
+    for (int ct = 0; ct < NC; ++ct) {
+      if (ct + 3 < NC) read_values(ct + 3);
+      __builtin_amdgcn_sched_barrier(0);
+      const lat_short4 lo = vf[ct % 4][0], up = vf[ct % 4][1];
+      const lat_short8 both = {lo.x, lo.y, lo.z, lo.w, up.x, up.y, up.z, up.w};
+      acc[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(lat_bf16x8, both), pf, acc[ct], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+
+  l_run += __shfl_xor(l_run, 16, 64);
+  l_run += __shfl_xor(l_run, 32, 64);
+  if (my >= rows_here) return;
+  // The lane holds its row's columns 16 ct + 4 g ..
+  const int t = row0 + f_row / H, h = f_row % H;
+  if (pl.n_chunks > 1) {
+    float* part = a.workspace + (((int64_t)t * H + h) * pl.n_chunks + chunk_id) * (R + 2);
+    if (g == 0) {
+      part[R] = m_ref * (1.f / kLatLog2e);   // (of the scores themselves: what the merge expects)
+      part[R + 1] = l_run;
+    }
+#pragma unroll
+    for (int ct = 0; ct < NC; ++ct)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) part[16 * ct + 4 * g + r] = acc[ct][r];
+    return;
+  }
+  float factor = l_run > 0.f ? 1.f / l_run : 0.f;
+  if (a.gate) {
+    const float z = __bfloat162float(((const bf16*)a.gate)[(int64_t)t * a.gate_stride + h]);
+    factor *= 1.f / (1.f + expf(-z));
+  }
+  typedef __bf16 lat_bf16x4 __attribute__((ext_vector_type(4)));
+  __bf16* orow = (__bf16*)a.out + ((int64_t)t * H + h) * R;
+#pragma unroll
+  for (int ct = 0; ct < NC; ++ct) {
+    lat_bf16x4 o;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) o[r] = (__bf16)(acc[ct][r] * factor);
+    *(lat_bf16x4*)(orow + 16 * ct + 4 * g) = o;
+  }
+#endif
+}
+
 // out[t, h] = sum_c e^(m_c - M) O_c / sum_c e^(m_c - M) l_c over the chunks that saw keys.
 __global__ void latent_attention_merge_kernel(LatentArgs a, int n_chunks) {
   extern __shared__ float smem[];   // [n_chunks] weight of each chunk: e^(m_c - M) / L (0: saw no key)
@@ -707,13 +997,28 @@ static int launch_latent_rows(const LatentArgs& a, const LatentTilePlan& p, hipS
   return few ? launch_latent_tile<ROWS, 20, 2>(a, p, stream) : launch_latent_tile<ROWS, 20, 4>(a, p, stream);
 }
 
+template <int QF, int NC>
+static int launch_latent_waves(const LatentArgs& a, const LatentTilePlan& p, hipStream_t stream) {
+  constexpr size_t lds = 2 * 4 * ((8 * 4 * QF + 63) / 64 * 1024) + 2 * kLatRowsKeys * sizeof(int);
+  auto kern = latent_attention_rows_kernel<QF, NC>;
+  hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  if (e != hipSuccess) return set_error(-2, "latent_attention: cannot get %zu bytes of LDS", lds);
+  kern<<<dim3(p.tiles, p.n_chunks), 256, lds, stream>>>(a, p);
+  NINFER_LAUNCH_CHECK();
+  return 0;
+}
+
 static int latent_attention_tile(const LatentArgs& a, hipStream_t stream) {
   const LatentTilePlan p = latent_tile_plan(a);
   const int64_t need = latent_tile_workspace_floats(a, p);
   NINFER_REQUIRE(need == 0 || (a.workspace && a.workspace_floats >= need),
                  "latent_attention: the workspace holds %lld floats, %lld are needed",
                  (long long)a.workspace_floats, (long long)need);
-  int rc = p.rows == 16 ? launch_latent_rows<16>(a, p, stream) : launch_latent_rows<64>(a, p, stream);
+  int rc;
+  if (p.rows == 16) rc = launch_latent_rows<16>(a, p, stream);
+  else if (!latent_rows_takes(a)) rc = launch_latent_rows<64>(a, p, stream);
+  else if (a.R == 512) rc = a.rd == 64 ? launch_latent_waves<18, 32>(a, p, stream) : launch_latent_waves<17, 32>(a, p, stream);
+  else rc = a.rd == 64 ? launch_latent_waves<10, 16>(a, p, stream) : launch_latent_waves<9, 16>(a, p, stream);
   if (rc) return rc;
   if (p.n_chunks > 1) {
     const int block = a.R >= 256 ? 256 : (a.R + 63) / 64 * 64;

@@ -462,6 +462,26 @@ def test_latent_forms(ops, rank, rd, heads, new_rows):
     assert worst < 8e-3
 
 
+@pytest.mark.parametrize("rank,rd", [(256, 32), (256, 64), (512, 32), (512, 64)])
+@pytest.mark.parametrize("heads,ps,window", [(16, 16, 0), (5, 4, 100), (24, 64, 0)])
+def test_latent_prompts_whose_waves_keep_whole_rows(ops, rank, rd, heads, ps, window):
+    """Portions that end a row before, at and behind tiles of 32 keys and blocks of 64 rows, behind cached
+    tokens and without, tokens that two blocks share (5 heads), pages smaller than the 8 keys that a wave
+    fetches, and a gate."""
+    lengths, new_rows = [31, 32, 65, 700, 330, 97], [31, 32, 65, 420, 161, 1]
+    if heads == 5:
+        lengths, new_rows = [1200, 33, 129], [1100, 33, 129]
+    ctx, pool, table, q, cached = _latent_case(ops, torch.bfloat16, heads, rank, rd, ps, lengths, new_rows, seed=rank + ps)
+    gate = torch.randn(ctx.T, heads).bfloat16()
+    out = torch.full((ctx.T + 1, heads * rank), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops.latent_attention(q.to(DEV), pool.bfloat16().to(DEV), table.to(DEV), ctx, heads, rank, rd, ps, 0.1, out[:-1],
+                         gate=gate.to(DEV), window=window)
+    want = _plain_latent_rows(q, cached, lengths, new_rows, rank, 0.1, window, gate.float())
+    got = out[:-1].float().cpu().reshape(ctx.T, heads, rank)
+    assert (out[-1] == 7.0).all()
+    assert max(rel_err(g, w) for g, w in zip(got, want)) < 8e-3   # (the bound of the forms above)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("where", [0, 1, 15, 16, 63, 64, 300, 498])
 def test_latent_attention_finds_one_key(ops, dtype, where):
