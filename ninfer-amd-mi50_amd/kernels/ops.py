@@ -387,6 +387,7 @@ class HipOps:
         # activation at every row count (70 against 98 us at 64 rows of 40960 x 3584; whole
         # prompt portions of 256 to 8,192 tokens 2 to 4% faster at 2048 -> 2 x 5632, the same
         # within 1% at 3584 -> 2 x 20480)
+        self._cus = None
         self.split_max_rows = 512   # most rows of a product that may be cut along K (gemm_split)
         # a plain product of at most this many rows runs on the tile kernel here when it is on
         # the second stream: the library's product there took the 512-token portion 7.25 ms in
@@ -731,6 +732,16 @@ class HipOps:
                                             or weight_bytes < self.beside_heavy_bytes):
             return False
         return not torch.cuda.is_current_stream_capturing()
+
+    def leaves_room(self, rows: int, features: int) -> bool:
+        """Does a product of this size leave CUs, or places on them, to short kernels on another stream?
+        While its tall tiles (256 x 256, one to a CU) would be fewer than the CUs. Measured on the shared
+        expert's products started before the routing against after it: steps of 512 rows of the headline
+        model (88 tiles of 2 x 5,632 features) 9.07 -> 8.68 ms, 1,531 rows of 2 x 2,816 (132) 4.03 -> 4.01;
+        2,048 rows of 2 x 5,632 (352) 13.31 -> 13.67."""
+        if self._cus is None:
+            self._cus = torch.cuda.get_device_properties(torch.cuda.current_device()).multi_processor_count
+        return -(-rows // 256) * -(-features // 256) < self._cus
 
     def beside(self):
         """Context manager for work that nothing on the current stream waits for until

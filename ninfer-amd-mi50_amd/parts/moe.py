@@ -266,12 +266,19 @@ class SparseMoE(FeedForward):
         # of the device empty in their last round of blocks.
         logits = ctx.empty((x.shape[0], self.router.experts + 1), torch.float32)
         if ctx.ops.wants_beside(x.shape[0], self.shared.weight_bytes()):
-            # routing first: its short kernels would crawl beside the shared expert's long ones
+            # While its blocks leave the GPU room, the second stream starts before the routing's short
+            # kernels and fills the device beside them; else after them: they would crawl.
+            room = getattr(ctx.ops, "leaves_room", None)
+            early = room is not None and room(x.shape[0], 2 * self.shared.inner)
+            if early:
+                with ctx.ops.beside():
+                    shared = self.shared.down(ctx, self.shared.gate_up(ctx, x))
             ctx.ops.linear(x, self.router_and_gate, logits)
             routing = self.router.route(ctx, logits)
             self.last_ids = routing.ids
-            with ctx.ops.beside():
-                shared = self.shared.down(ctx, self.shared.gate_up(ctx, x))
+            if not early:
+                with ctx.ops.beside():
+                    shared = self.shared.down(ctx, self.shared.gate_up(ctx, x))
             y = self.experts.run(ctx, x, routing)
             ctx.ops.join()
             return PendingRows(y, routing.weights, shared, logits[:, self.router.experts])
