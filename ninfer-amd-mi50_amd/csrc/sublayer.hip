@@ -54,31 +54,27 @@ __global__ void short_conv_kernel(const float* __restrict__ x, const float* __re
 }
 
 // The same for 2 to 4 taps and rows of whole 16-byte pieces: a thread has four channels of ROWS
-// neighbouring rows, their weights in registers, every load of a row on its way at once. The same
-// sums in the same order. 2,048 rows of 2,048 channels with four taps (16 MB in, 8 MB out): 8.6
-// us, 2.8 TB/s, where a thread per number with its weights fetched one by one takes 23.
-template <typename T, int TAPS, int ROWS>
+// neighbouring rows, their weights in registers, and loads the ROWS + TAPS - 1 input rows that they see
+// at once. The same sums in the same order.
+// SINGLE: every request brings one row, and the thread shifts its state. Else the state is the business of the
+// thread whose rows hold the request's first one. It also has those of the TAPS - 2 rows behind
+// that see the old state (nobody else reads it, wherever the rows fall), and writes the new state when
+// they are done.
+// Memory-bound. 2,048 rows of 2,048 channels with four taps (16 MB in, 8 MB out): 8.6 us from launch to launch,
+// where loading each row's four inputs by themselves and the state in a launch of its own took 10.9, and a
+// thread per number with its weights fetched one by one 23.
+template <typename T, int TAPS, int ROWS, bool SINGLE>
 __global__ __launch_bounds__(256) void short_conv_rows_kernel(
     const float* __restrict__ x, const float* __restrict__ w, float* __restrict__ state, int64_t state_stride,
     T* __restrict__ out, const int* __restrict__ row_seq, const int* __restrict__ seq_row_start,
-    const int* __restrict__ seq_slots, int rows, int H, int update) {
+    const int* __restrict__ seq_slots, int rows, int H) {
   const int c = 4 * (blockIdx.y * blockDim.x + threadIdx.x);
   if (c >= H) return;
+  const int base = blockIdx.x * ROWS;
   float wc[4 * TAPS];   // [channel][tap]
 #pragma unroll
   for (int e = 0; e < TAPS; ++e) load_row<4>(w + (int64_t)c * TAPS + 4 * e, wc + 4 * e);
-#pragma unroll
-  for (int n = 0; n < ROWS; ++n) {
-    const int t = blockIdx.x * ROWS + n;
-    if (t >= rows) return;
-    const int s = row_seq[t], r0 = seq_row_start[s], i = t - r0;
-    float* st = state + (int64_t)seq_slots[s] * state_stride + c;
-    float v[TAPS][4];
-#pragma unroll
-    for (int j = 0; j < TAPS; ++j) {
-      const int src = i - (TAPS - 1 - j);
-      load_row<4>(src >= 0 ? x + (int64_t)(r0 + src) * H + c : st + (int64_t)(TAPS - 1 + src) * H, v[j]);
-    }
+  auto finish = [&](int t, const float(*v)[4]) {   // v: the inputs of the row's taps
     float o[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -88,9 +84,73 @@ __global__ __launch_bounds__(256) void short_conv_rows_kernel(
       o[e] = v[TAPS - 1][e] + acc;
     }
     store_row<4>(out + (int64_t)t * H + c, o);
-    if (update) {   // this row is the request's only one: the state moves on by one input
+  };
+  if constexpr (SINGLE) {
+#pragma unroll
+    for (int n = 0; n < ROWS; ++n) {
+      const int t = base + n;
+      if (t >= rows) return;
+      float* st = state + (int64_t)seq_slots[row_seq[t]] * state_stride + c;
+      float v[TAPS][4];
+#pragma unroll
+      for (int j = 0; j < TAPS; ++j)
+        load_row<4>(j == TAPS - 1 ? x + (int64_t)t * H + c : st + (int64_t)j * H, v[j]);
+      finish(t, v);
 #pragma unroll
       for (int k = 0; k + 1 < TAPS; ++k) store_row<4>(st + (int64_t)k * H, v[k + 1]);
+    }
+  } else {
+    float xs[ROWS + TAPS - 1][4];   // (rows that are not there: the nearest one, not used)
+#pragma unroll
+    for (int m = 0; m < ROWS + TAPS - 1; ++m) {
+      const int t = min(max(base - (TAPS - 1) + m, 0), rows - 1);
+      load_row<4>(x + (int64_t)t * H + c, xs[m]);
+    }
+    bool starts = false;   // a request starts in these rows
+#pragma unroll
+    for (int n = 0; n < ROWS; ++n) {
+      const int t = base + n;
+      if (t >= rows) break;
+      const int s = row_seq[t], r0 = seq_row_start[s], i = t - r0;
+      if (i >= TAPS - 1) {
+        finish(t, xs + n);
+      } else if (r0 >= base) {   // (else it is with the rows before)
+        starts = true;
+        const float* st = state + (int64_t)seq_slots[s] * state_stride + c;
+        float v[TAPS][4];
+#pragma unroll
+        for (int j = 0; j < TAPS; ++j) {
+          const int src = i - (TAPS - 1 - j);
+          load_row<4>(src >= 0 ? x + (int64_t)(r0 + src) * H + c : st + (int64_t)(TAPS - 1 + src) * H, v[j]);
+        }
+        finish(t, v);
+      }
+    }
+    if (!starts) return;
+    for (int t = base + ROWS; t < min(base + ROWS + TAPS - 2, rows); ++t) {   // rows behind that see the old state
+      const int s = row_seq[t], r0 = seq_row_start[s], i = t - r0;
+      if (i >= TAPS - 1 || r0 >= base + ROWS) break;
+      const float* st = state + (int64_t)seq_slots[s] * state_stride + c;
+      float v[TAPS][4];
+#pragma unroll
+      for (int j = 0; j < TAPS; ++j) {
+        const int src = i - (TAPS - 1 - j);
+        load_row<4>(src >= 0 ? x + (int64_t)(r0 + src) * H + c : st + (int64_t)(TAPS - 1 + src) * H, v[j]);
+      }
+      finish(t, v);
+    }
+    for (int t = base; t < min(base + ROWS, rows); ++t) {   // (as in short_conv_state_kernel)
+      const int s = row_seq[t], r0 = seq_row_start[s];
+      if (t != r0) continue;
+      const int n = seq_row_start[s + 1] - r0;
+      float* st = state + (int64_t)seq_slots[s] * state_stride + c;
+#pragma unroll
+      for (int k = 0; k < TAPS - 1; ++k) {
+        const int p = n - (TAPS - 1) + k;
+        float v[4];
+        load_row<4>(p >= 0 ? x + (int64_t)(r0 + p) * H + c : st + (int64_t)(k + n) * H, v);
+        store_row<4>(st + (int64_t)k * H, v);
+      }
     }
   }
 }
@@ -449,17 +509,18 @@ static int row_block(int H) {
 
 using namespace ninfer;
 
+// Whether the launch also moves the state on.
 template <typename T>
-static void launch_short_conv(const float* x, const float* w, float* state, long long state_stride, T* out,
+static bool launch_short_conv(const float* x, const float* w, float* state, long long state_stride, T* out,
                               const int* row_seq, const int* seq_row_start, const int* seq_slots, int rows, int H,
-                              int taps, int update, hipStream_t stream) {
+                              int taps, bool single, hipStream_t stream) {
   const bool wide = taps >= 2 && taps <= 4 && H % 4 == 0 && state_stride % 4 == 0 && row_aligned(x) &&
                     row_aligned(w) && row_aligned(state) && row_aligned(out);
   if (!wide) {
     const int block = row_block(H);
     short_conv_kernel<T><<<dim3(rows, (H + block - 1) / block), block, 0, stream>>>(
-        x, w, state, state_stride, out, row_seq, seq_row_start, seq_slots, H, taps, update);
-    return;
+        x, w, state, state_stride, out, row_seq, seq_row_start, seq_slots, H, taps, single ? 1 : 0);
+    return single;
   }
   // four rows to a thread share its weights where that leaves the CUs enough waves, from 1.5 Mi numbers on:
   // 2,048 rows of 2,048 channels 10.1 us and 15.2 with one row to a thread, of 1,024 6.3 and 9.3; but 516 rows
@@ -467,19 +528,23 @@ static void launch_short_conv(const float* x, const float* w, float* state, long
   const int per = (int64_t)rows * H >= (3 << 19) ? 4 : 1;
   const int block = row_block(H / 4);
   const dim3 grid((rows + per - 1) / per, (H / 4 + block - 1) / block);
-#define NINFER_CONV(TAPS)                                                                                     \
-  do {                                                                                                        \
-    if (per == 4)                                                                                             \
-      short_conv_rows_kernel<T, TAPS, 4><<<grid, block, 0, stream>>>(x, w, state, state_stride, out, row_seq,   \
-                                                                   seq_row_start, seq_slots, rows, H, update); \
-    else                                                                                                      \
-      short_conv_rows_kernel<T, TAPS, 1><<<grid, block, 0, stream>>>(x, w, state, state_stride, out, row_seq,   \
-                                                                   seq_row_start, seq_slots, rows, H, update); \
+  auto launch = [&](auto kern) {
+    kern<<<grid, block, 0, stream>>>(x, w, state, state_stride, out, row_seq, seq_row_start, seq_slots, rows, H);
+  };
+#define NINFER_CONV(TAPS)                                                                       \
+  do {                                                                                          \
+    if (per == 4)                                                                               \
+      single ? launch(short_conv_rows_kernel<T, TAPS, 4, true>)                                 \
+             : launch(short_conv_rows_kernel<T, TAPS, 4, false>);                               \
+    else                                                                                        \
+      single ? launch(short_conv_rows_kernel<T, TAPS, 1, true>)                                 \
+             : launch(short_conv_rows_kernel<T, TAPS, 1, false>);                               \
   } while (0)
   if (taps == 2) NINFER_CONV(2);
   else if (taps == 3) NINFER_CONV(3);
   else NINFER_CONV(4);
 #undef NINFER_CONV
+  return true;
 }
 
 extern "C" int ninfer_short_conv(const float* x, const float* w, float* state,
@@ -493,14 +558,13 @@ extern "C" int ninfer_short_conv(const float* x, const float* w, float* state,
                  state_stride, taps - 1, H);
   NINFER_REQUIRE(dtype == kF32 || dtype == kBF16, "short_conv: unknown dtype %d", dtype);
   const int block = row_block(H);
-  if (dtype == kF32)
-    launch_short_conv(x, w, state, state_stride, (float*)out, row_seq, seq_row_start, seq_slots, T, H, taps,
-                      all_single, stream);
-  else
-    launch_short_conv(x, w, state, state_stride, (bf16*)out, row_seq, seq_row_start, seq_slots, T, H, taps,
-                      all_single, stream);
+  const bool moved =
+      dtype == kF32 ? launch_short_conv(x, w, state, state_stride, (float*)out, row_seq, seq_row_start, seq_slots, T,
+                                        H, taps, all_single != 0, stream)
+                    : launch_short_conv(x, w, state, state_stride, (bf16*)out, row_seq, seq_row_start, seq_slots, T,
+                                        H, taps, all_single != 0, stream);
   NINFER_LAUNCH_CHECK();
-  if (!all_single && taps > 1) {
+  if (!moved && taps > 1) {
     short_conv_state_kernel<<<dim3(S, (H + block - 1) / block), block, 0, stream>>>(
         x, state, state_stride, seq_row_start, seq_slots, H, taps);
     NINFER_LAUNCH_CHECK();

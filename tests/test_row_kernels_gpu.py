@@ -44,6 +44,14 @@ def test_short_conv(ops, dtype, taps, width, seqs):
     assert torch.equal(states[0], states[1]) and torch.equal(states[0][-1], first[-1])
 
 
+@pytest.mark.parametrize("taps", [2, 3, 4])
+@pytest.mark.parametrize("seqs", [[(i, 1 + i % 5) for i in range(10)], [(i, 1 + i % 5) for i in range(540)]])
+def test_short_conv_of_requests_that_start_anywhere(ops, taps, seqs):
+    """The thread that holds a request's first row moves its state on: requests of one to five rows
+    that start at every place of a thread's rows (one row; four rows from 540 requests on)."""
+    test_short_conv(ops, torch.float32, taps, 1028, seqs)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("width", [4, 1028])
 @pytest.mark.parametrize("k", [0, 1, 5])
