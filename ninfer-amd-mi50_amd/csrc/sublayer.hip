@@ -522,9 +522,10 @@ static bool launch_short_conv(const float* x, const float* w, float* state, long
         x, w, state, state_stride, out, row_seq, seq_row_start, seq_slots, H, taps, single ? 1 : 0);
     return single;
   }
-  // four rows to a thread share its weights where that leaves the CUs enough waves, from 1.5 Mi numbers on:
-  // 2,048 rows of 2,048 channels 10.1 us and 15.2 with one row to a thread, of 1,024 6.3 and 9.3; but 516 rows
-  // of 2,048 6.5 and 5.9, 300 of 1,024 5.3 and 4.7, 300 of 64 4.7 and 4.1 (four taps)
+  // four rows to a thread share its loads where that leaves the CUs enough waves, from 1.5 Mi numbers on:
+  // 2,048 rows of 2,048 channels 8.7 us and 12.6 with one row to a thread, of 1,024 6.2 and 7.8. Below, a
+  // prompt of 516 rows of 2,048 alone would gain (5.2 and 6.5) and lose behind seven requests of one row (8.2
+  // and 6.4); 64 such requests 3.1 and 2.3, 300 rows of 64 3.4 and 3.1 (four taps)
   const int per = (int64_t)rows * H >= (3 << 19) ? 4 : 1;
   const int block = row_block(H / 4);
   const dim3 grid((rows + per - 1) / per, (H / 4 + block - 1) / block);
