@@ -128,13 +128,21 @@ __device__ inline bool find_tile(const int* __restrict__ offsets, int groups, in
   return info[2] >= 0;
 }
 
+// The entry of a tile list that block row `ti` reads before it knows how many there are: a launch may have more
+// block rows than the list has entries (M / tile_rows + groups, which no grouping exceeds; of 16-row tiles no
+// more than M either, nor has a launch). Those behind read its last entry and leave by the count.
+__host__ __device__ inline int list_entry(const GemmArgs& a, int tile_rows, int ti) {
+  const int last = a.M / tile_rows + a.groups - 1;
+  return ti < last ? ti : last;
+}
+
 // The rows of tile `ti`: from the tile list routing wrote (one 16-byte load),
 // or by scanning the offsets when there is no list. `info` is 3 ints of LDS.
 __device__ inline bool grouped_tile(const GemmArgs& a, const int* __restrict__ tiles, int which,
                                     int tile_rows, int ti, int* info) {
   if (!tiles) return find_tile(a.offsets, a.groups, tile_rows, ti, info);
   int count = a.tile_counts[which];
-  int4 t = ((const int4*)tiles)[ti];
+  int4 t = ((const int4*)tiles)[list_entry(a, tile_rows, ti)];
   if (ti >= count) return false;
   info[0] = t.y;
   info[1] = t.z;
@@ -144,6 +152,7 @@ __device__ inline bool grouped_tile(const GemmArgs& a, const int* __restrict__ t
 
 int gemm_check(const GemmArgs& a);
 bool gemm_skinny_takes(const GemmArgs& a);
+int gemm_skinny_row_tiles(const GemmArgs& a);   // block rows of a launch in tiles of 16 rows
 int gemm_skinny(const GemmArgs& a, hipStream_t stream);
 bool gemm_skinny_rows_takes(const GemmArgs& a);
 int gemm_skinny_rows(const GemmArgs& a, hipStream_t stream);
@@ -156,6 +165,7 @@ bool gemm_skinny_route_pair_takes(const GemmArgs& a, const GemmArgs& b, const Ro
 int gemm_skinny_route_pair(const GemmArgs& a, const GemmArgs& b, const RouteArgs& rt,
                            hipStream_t stream);
 bool gemm_tile_takes(const GemmArgs& a);
+int gemm_tile_row_tiles(const GemmArgs& a, int rows);   // block rows of a launch in tiles of 64, 128 or 256 rows
 int gemm_tile(const GemmArgs& a, hipStream_t stream);
 int gemm_generic(const GemmArgs& a, hipStream_t stream);
 bool gemm_f32_takes(const GemmArgs& a);

@@ -46,6 +46,12 @@ extern "C" int ninfer_gemm_split_parts(const GemmArgs* args) {
   return gemm_split_parts(*args);
 }
 
+// The last entry of the list of 16-row tiles (tall = 0) or of tall ones that a grouped launch reads.
+extern "C" int ninfer_gemm_last_list_entry(const GemmArgs* a, int tall) {
+  const int rows = tall ? kGroupedTileRows : 16;
+  return list_entry(*a, rows, (tall ? gemm_tile_row_tiles(*a, rows) : gemm_skinny_row_tiles(*a)) - 1);
+}
+
 // Two products that do not depend on each other. Pairs of few-row products that have a
 // kernel of their own run as one launch; all others one after the other.
 extern "C" int ninfer_gemm_pair(const GemmArgs* a, const GemmArgs* b, int force_generic,

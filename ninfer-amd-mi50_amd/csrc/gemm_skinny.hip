@@ -147,7 +147,7 @@ __device__ __forceinline__ void skinny_block(const GemmArgs& a, int rows_arg, in
   if (a.offsets && a.tiles16) {
     // every thread reads the tile's entry itself: no barrier before the first loads
     int count = a.tile_counts[0];
-    int4 t = ((const int4*)a.tiles16)[by];
+    int4 t = ((const int4*)a.tiles16)[list_entry(a, SM, by)];
     if (by >= count) return;
     group = t.x;
     row0 = t.y;
@@ -408,9 +408,14 @@ __global__ __launch_bounds__(1024) void gemm_skinny_route_kernel(GemmArgs a, Rou
   else skinny_route_block<4>(a, rt, red, stage);
 }
 
+// (grouped: at most one tile per sorted row, and one partial tile per group)
+int gemm_skinny_row_tiles(const GemmArgs& a) {
+  return a.offsets ? min((a.M + SM - 1) / SM + a.groups, a.M) : (a.M + SM - 1) / SM;
+}
+
 template <int WAVES>
 static void launch_skinny(const GemmArgs& a, int rows, bool two, hipStream_t stream) {
-  int m_tiles = a.offsets ? min((a.M + SM - 1) / SM + a.groups, a.M) : (a.M + SM - 1) / SM;
+  int m_tiles = gemm_skinny_row_tiles(a);
   dim3 grid((a.N + rows - 1) / rows, m_tiles);   // as plan_skinny counts them
   if (!a.offsets && m_tiles > 1)   // one line of blocks, the row tiles of a feature tile side by side
     grid = dim3(line_ids(grid.x, m_tiles), 1);
@@ -451,9 +456,8 @@ constexpr long kSkinnyTwoMinBlocks = 4096;   // GemmArgs::skinny_two overrides t
 
 static SkinnyPlan plan_skinny(const GemmArgs& a) {
   SkinnyPlan p;
-  // more waves per block when the grid alone would leave CUs idle (grouped: at most one tile
-  // per sorted row, and one partial tile per group)
-  p.grid_y = a.offsets ? min((a.M + SM - 1) / SM + a.groups, a.M) : (a.M + SM - 1) / SM;
+  // more waves per block when the grid alone would leave CUs idle
+  p.grid_y = gemm_skinny_row_tiles(a);
   int m_tiles = p.grid_y;
   long blocks = (long)((a.N + 15) / 16) * m_tiles;
   int chunks = a.K / 128;

@@ -444,14 +444,18 @@ bool gemm_tile_takes(const GemmArgs& a) {
          2 * ((epilogue_gated(a.epilogue) ? a.N : 0) + 256ll) * a.K < four_gb;
 }
 
+int gemm_tile_row_tiles(const GemmArgs& a, int rows) {
+  const int tiles = (a.M + rows - 1) / rows;
+  if (!a.offsets) return tiles;
+  return (tiles + a.groups + kXcds - 1) / kXcds * kXcds;   // block_to_tile's bijection
+}
+
 template <int TM, int TN, int WGM, int WGN, int NBX, int NBW>
 static int launch_tiles(const GemmArgs& a, hipStream_t stream) {
   constexpr int LDS_BYTES = (NBX * TM + NBW * TN) * 64 * 2;
   const bool swiglu = epilogue_gated(a.epilogue);
-  int m_tiles = (a.M + TM - 1) / TM + (a.offsets ? a.groups : 0);
-  if (a.offsets) m_tiles = (m_tiles + kXcds - 1) / kXcds * kXcds;   // block_to_tile's bijection
   const int per_block = swiglu ? TN / 2 : TN;
-  DirectGrid g = {m_tiles, (a.N + per_block - 1) / per_block, 0, 1};
+  DirectGrid g = {gemm_tile_row_tiles(a, TM), (a.N + per_block - 1) / per_block, 0, 1};
   dim3 grid(g.m_tiles, g.n_tiles, a.k_parts > 1 ? a.k_parts : 1);
   if (TM == 256 && !a.offsets && a.k_parts <= 1) {
     const int tiles = g.m_tiles * g.n_tiles, cus = device_cu_count(), last = tiles % cus;

@@ -62,6 +62,17 @@ def test_height_of_dense_tiles(lib, m, n, k, gated, beside, rows):
     assert lib.ninfer_gemm_tile_rows(ctypes.byref(args)) == rows
 
 
+def test_no_block_reads_behind_a_tile_list(lib):
+    """The lists hold min(n, n // 16 + experts) and n // 256 + experts tiles of n sorted rows; a launch rounds its
+    block rows up and may have more."""
+    from ninfer_amd.kernels.ops import _GemmArgs
+    for groups in (1, 2, 7, 60, 64, 130):
+        for n in list(range(1, 70)) + [100, 255, 256, 257, 1025, 1279, 1280, 4095, 8192]:
+            args = _GemmArgs(M=n, N=64, K=64, groups=groups, offsets=16)
+            assert lib.ninfer_gemm_last_list_entry(ctypes.byref(args), 0) < min(n, n // 16 + groups), (groups, n)
+            assert lib.ninfer_gemm_last_list_entry(ctypes.byref(args), 1) < n // 256 + groups, (groups, n)
+
+
 def test_a_products_arguments_have_one_size(lib, monkeypatch):
     """The bindings' layout against the library's, compared when the library is loaded."""
     from ninfer_amd.kernels import ops
