@@ -24,20 +24,33 @@ static bool many_rows(const GemmArgs& a) {
 // Bytes of GemmArgs: a caller that lays it out for itself compares its own.
 extern "C" int ninfer_gemm_args_bytes() { return (int)sizeof(GemmArgs); }
 
+// The kernels, in the order in which they are asked.
+enum GemmKernel : int { kGemmGeneric = 0, kGemmF32 = 1, kGemmSplit = 2, kGemmSkinnyRows = 3, kGemmTile = 4, kGemmSkinny = 5 };
+static GemmKernel gemm_kernel(const GemmArgs& a) {
+  if (gemm_f32_takes(a)) return kGemmF32;
+  if (gemm_split_parts(a) >= 2) return kGemmSplit;
+  if (gemm_skinny_rows_takes(a)) return kGemmSkinnyRows;
+  if (many_rows(a) && gemm_tile_takes(a)) return kGemmTile;
+  return gemm_skinny_takes(a) ? kGemmSkinny : kGemmGeneric;
+}
+
+// Which of them ninfer_gemm would run.
+extern "C" int ninfer_gemm_kernel(const GemmArgs* args) { return gemm_kernel(*args); }
+
 // force_generic != 0 runs the plain tiled kernel whatever the shape (tests
 // compare the fast kernels with it).
 extern "C" int ninfer_gemm(const GemmArgs* args, int force_generic, hipStream_t stream) {
   int rc = gemm_check(*args);
   if (rc) return rc;
   const GemmArgs& a = *args;
-  if (!force_generic) {
-    if (gemm_f32_takes(a)) return gemm_f32(a, stream);
-    if (gemm_split_parts(a) >= 2) return gemm_split(a, stream);
-    if (gemm_skinny_rows_takes(a)) return gemm_skinny_rows(a, stream);
-    if (many_rows(a) && gemm_tile_takes(a)) return gemm_tile(a, stream);
-    if (gemm_skinny_takes(a)) return gemm_skinny(a, stream);
+  switch (force_generic ? kGemmGeneric : gemm_kernel(a)) {
+    case kGemmF32: return gemm_f32(a, stream);
+    case kGemmSplit: return gemm_split(a, stream);
+    case kGemmSkinnyRows: return gemm_skinny_rows(a, stream);
+    case kGemmTile: return gemm_tile(a, stream);
+    case kGemmSkinny: return gemm_skinny(a, stream);
+    default: return gemm_generic(a, stream);
   }
-  return gemm_generic(a, stream);
 }
 
 // Into how many parts along K ninfer_gemm would cut this product (< 2: it would not).

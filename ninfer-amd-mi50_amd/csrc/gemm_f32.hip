@@ -33,7 +33,9 @@ template <int N> __device__ __forceinline__ void f32_wait_loads() {   // until a
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-template <int WAVES, int RT, int CT, bool GATED>
+// FAR: an index gathers rows of A, and some may lie 4 GB and more behind its first: every lane keeps whole addresses of
+// its rows (other operands' rows have 32-bit offsets from the block's own first ones).
+template <int WAVES, int RT, int CT, bool GATED, bool FAR>
 __global__ __launch_bounds__(64 * WAVES) void gemm_f32_kernel(GemmArgs a, int n_tiles, int m_tiles) {
 #if defined(__HIP_DEVICE_COMPILE__)   // (the host pass does not know buffer resources)
   constexpr int SEGS = kF32Segments / WAVES;        // segments of a wave
@@ -71,25 +73,34 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_f32_kernel(GemmArgs a, int n_
   // Load i of a stage: staged rows 8 i .. 8 i + 7, the lane at row lane / 8. Of a staged row (128 bytes)
   // the 16-byte chunk c lies at c ^ ((row / 2) % 8), chosen on the global side, so that the 16 rows of a
   // fragment read fall into different columns of the banks. Rows that are not there read the last one
-  // that is; nothing of them is stored. (Offsets of 32 bits: gemm_f32_takes.)
+  // that is; nothing of them is stored. Byte offsets: of A's rows from the block's first one (gathered: from
+  // A's), of W's from the block's first gate row and its up row.
   unsigned off[NL];
+  const char* far_row[FAR ? BM / 8 : 1];
+  const int w_first = min(n0, a.N - 1);
 #pragma unroll
   for (int i = 0; i < NL; ++i) {
     const int r = 8 * i + (lane >> 3);
     if (r < BM) {
       const int row = min(row0 + r, row_end - 1);
-      off[i] = (unsigned)(a.a_index ? a.a_index[row] / a.a_div : row) * (unsigned)(4 * a.lda);
+      if constexpr (FAR) {
+        far_row[i] = (const char*)((const float*)a.A + (int64_t)(a.a_index[row] / a.a_div) * a.lda);
+        off[i] = 0;
+      } else {
+        off[i] = (unsigned)(a.a_index ? a.a_index[row] / a.a_div : row - row0) * (unsigned)(4 * a.lda);
+      }
     } else {
-      const int j = (r - BM) / 16;
-      const bool up = GATED && j >= CT / 2;
-      const int n = min(n0 + (up ? j - CT / 2 : j) * 16 + r % 16, a.N - 1) + (up ? a.N : 0);
-      off[i] = (unsigned)n * (unsigned)(4 * K);
+      const int j = (r - BM) / 16, f = n0 + (GATED && j >= CT / 2 ? j - CT / 2 : j) * 16 + r % 16;
+      off[i] = (unsigned)(min(f, a.N - 1) - w_first) * (unsigned)(4 * K);
     }
   }
   const int lane_chunk = (lane & 7) ^ (lane >> 4);   // (load i's rows add 4 i to the row / 2)
-  const float* W = (const float*)a.W + (int64_t)group * a.w_group_stride;
-  const auto a_res = __builtin_amdgcn_make_buffer_rsrc((void*)a.A, 0, 0xffffffffu, 0x00020000);
+  const float* A = (const float*)a.A + (a.a_index ? 0 : (int64_t)row0 * a.lda);
+  const float* W = (const float*)a.W + (int64_t)group * a.w_group_stride + (int64_t)w_first * K;
+  const auto a_res = __builtin_amdgcn_make_buffer_rsrc((void*)A, 0, 0xffffffffu, 0x00020000);
   const auto w_res = __builtin_amdgcn_make_buffer_rsrc((void*)W, 0, 0xffffffffu, 0x00020000);
+  const auto up_res = __builtin_amdgcn_make_buffer_rsrc((void*)(W + (GATED ? (int64_t)a.N * K : 0)), 0, 0xffffffffu, 0x00020000);
+  typedef const __attribute__((address_space(1))) void* gptr;
   typedef __attribute__((address_space(3))) void* lptr;
   unsigned char* ring = smem + wave * 2 * STAGE;
 
@@ -106,12 +117,16 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_f32_kernel(GemmArgs a, int n_
     for (int i = 0; i < NL; ++i) {
       // (what lies behind the row's end is never read: its last 16 bytes again)
       const unsigned o = off[i] + 16 * min(lane_chunk ^ ((4 * i) & 7), (K - k0) / 4 - 1);
-      if (8 * i < BM)
+      const auto rows_of_w = GATED && (8 * i - BM) / 16 >= CT / 2 ? up_res : w_res;
+      if (FAR && 8 * i < BM)
+        __builtin_amdgcn_global_load_lds((gptr)(far_row[FAR && 8 * i < BM ? i : 0] + o + (int64_t)k0 * 4),
+                                         (lptr)(buf + i * 1024), 16, 0, 0);
+      else if (8 * i < BM)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(a_res, (lptr)(buf + i * 1024), 16, o, k0 * 4, 0, 0);
       else if (once)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(w_res, (lptr)(buf + i * 1024), 16, o, k0 * 4, 0, 2);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rows_of_w, (lptr)(buf + i * 1024), 16, o, k0 * 4, 0, 2);
       else
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(w_res, (lptr)(buf + i * 1024), 16, o, k0 * 4, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rows_of_w, (lptr)(buf + i * 1024), 16, o, k0 * 4, 0, 0);
     }
   };
   // Fragments of chunk c of stage g: the lane holds four neighbouring k of one row, so a chunk is
@@ -211,17 +226,17 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_f32_kernel(GemmArgs a, int n_
 #endif
 }
 
-// 32-bit operands whose rows are whole 16-byte pieces, A and a group's W below 4 GB each. That
-// depends on the operands' layout alone and not on the number of rows (short of 4 GB of them): a
-// model's product takes the same kernel in every step.
+// 32-bit operands whose rows are whole 16-byte pieces, a block's rows (at most 48 of A and 32 of W) below 4 GB. That
+// depends on the operands' layout alone and not on the number of rows: a model's product takes the same
+// kernel in every step.
 bool gemm_f32_takes(const GemmArgs& a) {
-  const int64_t four_gb = 1ll << 32, w_rows = epilogue_gated(a.epilogue) ? 2ll * a.N : a.N;
+  const int64_t four_gb = 1ll << 32;
   return a.in_dtype == kF32 && a.out_dtype == kF32 && a.K % 4 == 0 && a.lda % 4 == 0 &&
          a.w_group_stride % 4 == 0 && ((uintptr_t)a.A | (uintptr_t)a.W) % 16 == 0 &&
-         4ll * a.M * a.lda < four_gb && 4 * w_rows * a.K < four_gb;
+         4ll * 48 * a.lda < four_gb && 4ll * 32 * a.K < four_gb;
 }
 
-template <int WAVES, int RT, int CT>
+template <int WAVES, int RT, int CT, bool FAR = false>
 static void launch(const GemmArgs& a, hipStream_t stream) {
   const bool gated = epilogue_gated(a.epilogue);
   const int bn = 16 * (gated ? CT / 2 : CT);
@@ -230,11 +245,11 @@ static void launch(const GemmArgs& a, hipStream_t stream) {
   const int grid = (n_tiles + kXcds - 1) / kXcds * kXcds * m_tiles;
   if constexpr (CT > 1) {
     if (gated) {
-      gemm_f32_kernel<WAVES, RT, CT, true><<<grid, 64 * WAVES, 0, stream>>>(a, n_tiles, m_tiles);
+      gemm_f32_kernel<WAVES, RT, CT, true, FAR><<<grid, 64 * WAVES, 0, stream>>>(a, n_tiles, m_tiles);
       return;
     }
   }
-  gemm_f32_kernel<WAVES, RT, CT, false><<<grid, 64 * WAVES, 0, stream>>>(a, n_tiles, m_tiles);
+  gemm_f32_kernel<WAVES, RT, CT, false, FAR><<<grid, 64 * WAVES, 0, stream>>>(a, n_tiles, m_tiles);
 }
 
 int gemm_f32(const GemmArgs& a, hipStream_t stream) {
@@ -261,13 +276,16 @@ int gemm_f32(const GemmArgs& a, hipStream_t stream) {
     const float us = t.alone + t.further * ((t.shared ? 0.5f * (per_cu + whole) : whole) - 1.f);
     if (best < 0 || us < least) best = i, least = us;
   }
+  // 4 GB of rows that an index gathers are many: the tallest tile. (Every tile gives the same bits.)
+  if (a.a_index && 4ll * a.M * a.lda >= 1ll << 32) best = 6;
   switch (best) {
     case 0: launch<8, 1, 1>(a, stream); break;
     case 1: launch<8, 1, 2>(a, stream); break;
     case 2: launch<8, 2, 2>(a, stream); break;
     case 3: launch<4, 1, 2>(a, stream); break;
     case 4: launch<4, 2, 2>(a, stream); break;
-    default: launch<4, 3, 2>(a, stream); break;
+    case 5: launch<4, 3, 2>(a, stream); break;
+    default: launch<4, 3, 2, true>(a, stream); break;
   }
   NINFER_LAUNCH_CHECK();
   return 0;

@@ -54,6 +54,47 @@ def test_every_tile(ops, gen, m, n, k):
     assert torch.equal(one[0], out[m - 1])
 
 
+# Operands that end beyond 4 GB, in rows of 32 KB: weights (gate rows and, as far behind again, their up rows), rows
+# of A and rows of A that an index gathers.
+K_FAR, N_FAR = 8192, 131120
+
+
+def test_weights_beyond_4_gb(ops, gen):
+    x, w = (torch.randn(r, K_FAR, generator=gen, device="cuda") for r in (3, 2 * N_FAR))
+    w *= K_FAR ** -0.5
+    out, gated = torch.empty(3, 2 * N_FAR, device="cuda"), torch.empty(3, N_FAR, device="cuda")
+    ops.linear(x, w, out)
+    ops.swiglu_linear(x, w, gated)
+    ends = torch.tensor([0, 1, N_FAR - 33, N_FAR - 1, N_FAR, 2 * N_FAR - 2, 2 * N_FAR - 1], device="cuda")
+    within(out[:, ends], x, w[ends], x.double() @ w[ends].double().T)
+    # a feature's bits are those of a product of its rows alone
+    part = torch.empty(3, 64, device="cuda")
+    ops.linear(x, w[-64:].contiguous(), part)
+    assert torch.equal(out[:, -64:], part)
+    ops.swiglu_linear(x, torch.cat([w[N_FAR - 64:N_FAR], w[-64:]]), part)
+    assert torch.equal(gated[:, -64:], part)
+
+
+def test_rows_beyond_4_gb(ops, gen):
+    x, w = (torch.randn(r, K_FAR, generator=gen, device="cuda") for r in (N_FAR, 34))
+    out, gated, one = torch.empty(N_FAR, 34, device="cuda"), torch.empty(N_FAR, 17, device="cuda"), torch.empty(5, 34, device="cuda")
+    ends = torch.tensor([0, 7, N_FAR // 2, N_FAR - 2, N_FAR - 1], device="cuda")
+    ops.linear(x, w, out)
+    within(out[ends], x[ends], w, x[ends].double() @ w.double().T)
+    ops.linear(x[ends], w, one)
+    assert torch.equal(out[ends], one)
+    # rows dealt to two groups in an order of their own: each row's product is that of the row alone
+    w2 = torch.randn(2, 34, K_FAR, generator=gen, device="cuda")
+    order = torch.randperm(N_FAR, generator=gen, device="cuda").int()
+    cut = N_FAR // 3
+    offsets = torch.tensor([0, cut, N_FAR], device="cuda", dtype=torch.int32)
+    ops.grouped_swiglu(x, w2, offsets, order, 1, gated)
+    for place in (0, cut - 1, cut, N_FAR - 1, int((order == N_FAR - 1).nonzero()), int((order == 0).nonzero())):
+        want = torch.empty(1, 17, device="cuda")
+        ops.swiglu_linear(x[order[place].long()][None], w2[int(place >= cut)], want)
+        assert torch.equal(gated[place], want[0])
+
+
 @pytest.mark.parametrize("m,n,k", [(1, 17, 64), (40, 100, 200), (70, 1408, 256)])
 def test_gated_rows_alone_and_together(ops, gen, m, n, k):
     x, w = torch.randn(m, k, generator=gen, device="cuda"), torch.randn(2 * n, k, generator=gen, device="cuda")

@@ -62,6 +62,19 @@ def test_height_of_dense_tiles(lib, m, n, k, gated, beside, rows):
     assert lib.ninfer_gemm_tile_rows(ctypes.byref(args)) == rows
 
 
+# (32-bit operands on both sides of 4 GB: an output head, a gated product's weights, a prompt's rows, rows that an
+# index gathers)
+@pytest.mark.parametrize("m,n,k,gated,indexed", [
+    (1, 131056, 8192, 0, 0), (1, 152064, 8192, 0, 0), (200, 152064, 8192, 0, 0), (1, 90000, 8192, 1, 0),
+    (150000, 61, 8192, 0, 0), (150000, 1408, 8192, 1, 1)])
+def test_large_operands_keep_the_32_bit_kernel(lib, m, n, k, gated, indexed):
+    from ninfer_amd.kernels.ops import _GemmArgs
+    args = _GemmArgs(A=16, W=16, C=16, M=m, N=n, K=k, lda=k, ldc=n, groups=1, a_div=1, epilogue=gated)
+    if indexed:
+        args.offsets, args.a_index, args.w_group_stride = 16, 16, 2 * n * k
+    assert lib.ninfer_gemm_kernel(ctypes.byref(args)) == 1
+
+
 def test_no_block_reads_behind_a_tile_list(lib):
     """The lists hold min(n, n // 16 + experts) and n // 256 + experts tiles of n sorted rows; a launch rounds its
     block rows up and may have more."""
