@@ -265,6 +265,7 @@ __device__ inline void write_tile(const GemmArgs& a, const f32x4 (&acc)[FI][FJ],
   write_accumulators<FI, FJ, SWIGLU, TC>(a, acc, tok0, row0, rows_here, feat0, row_of);
 }
 
+bool gemm_tile_far(const GemmArgs& a);   // rows of A with whole addresses: tiles of 128 rows only
 int gemm_tile_rows(const GemmArgs& a, int rows, hipStream_t stream);   // in tiles of 64, 128 or 256 rows
 
 }  // namespace ninfer

@@ -40,6 +40,7 @@ static float dense_us_256(int tiles, int cus, int K, bool beside) {
 // 1,024: 1,531 x 12,800 56 us in tiles of 256 and 68 in those of 128, 3,000 x 6,144 53 and 66). force_kernel
 // (tests) forces 64, 128 or 256 rows.
 static int tile_rows_of(const GemmArgs& a) {
+  if (gemm_tile_far(a)) return 128;
   if (a.force_kernel >= 1 && a.force_kernel <= 3) return 32 << a.force_kernel;
   const bool gated = epilogue_gated(a.epilogue);
   const int n_units = gated ? 2 * a.N : a.N;   // W rows

@@ -84,12 +84,14 @@ template <int I, int M, int R, int L> __device__ __forceinline__ void spread_ove
   }
 }
 
-enum DirectMode : int { kDense, kDenseCut, kGrouped };   // (kDenseCut: the launch cuts its last round)
+// kDenseCut: the launch cuts its last round. kGroupedFar: an index gathers rows of A of which some may lie 4 GB and
+// more behind its first: every lane keeps whole addresses of its rows.
+enum DirectMode : int { kDense, kDenseCut, kGrouped, kGroupedFar };
 
 template <int TM, int TN, int WGM, int WGN, int NBX, int NBW, bool SWIGLU, typename TC, DirectMode MODE>
 __global__ __launch_bounds__(WGM * WGN * 64, (NBX * TM + NBW * TN) * 128 > 80 * 1024 ? 1 : 2) void gemm_tile_kernel(GemmArgs a, DirectGrid grid) {
 #if defined(__HIP_DEVICE_COMPILE__)   // (the host pass does not know buffer resources)
-  constexpr bool CUT = MODE == kDenseCut, GROUPED = MODE == kGrouped;
+  constexpr bool CUT = MODE == kDenseCut, FAR = MODE == kGroupedFar, GROUPED = FAR || MODE == kGrouped;
   constexpr int TK = 64;
   constexpr int WAVES = WGM * WGN;
   constexpr int COL = TM / WGN;                            // staged token rows per wave column
@@ -164,8 +166,9 @@ __global__ __launch_bounds__(WGM * WGN * 64, (NBX * TM + NBW * TN) * 128 > 80 * 
   const int chunk = (lane % CPR) ^ (((wave * RPP + lane / CPR) / (16 / CPR)) % CPR);
   static_assert((WAVES * RPP / (16 / CPR)) % CPR == 0, "the loads of a wave must share their swizzle");
   // byte offsets: of A's rows from its first one (from the tile's first, where no index gathers them), of W's
-  // from the block's first (gemm_tile_takes: below 4 GB)
+  // from the block's first gate row and its up row (gemm_tile_takes: below 4 GB)
   unsigned xoff[NLX], woff[NLW];
+  const unsigned char* x_far[FAR ? NLX : 1];
   int x_row[NLX];
   unsigned x_live = 0;   // bit i: piece i of this wave's loads of A holds rows of the tile
 #pragma unroll
@@ -182,7 +185,7 @@ __global__ __launch_bounds__(WGM * WGN * 64, (NBX * TM + NBW * TN) * 128 > 80 * 
 #pragma unroll
   for (int i = 0; i < NLW; ++i) {
     const int n = staged_w_row<TN, WGM, SWIGLU>((i * WAVES + wave) * RPP + lane / CPR, out0, N);
-    woff[i] = (unsigned)(n - w_first) * (unsigned)(2 * K) + 16 * chunk;
+    woff[i] = (unsigned)((n < N ? n : n - N) - w_first) * (unsigned)(2 * K) + 16 * chunk;
   }
   if (a.a_index) {   // the index loads in flight together
     int idx[NLX];
@@ -192,10 +195,22 @@ __global__ __launch_bounds__(WGM * WGN * 64, (NBX * TM + NBW * TN) * 128 > 80 * 
     for (int i = 0; i < NLX; ++i) x_row[i] = idx[i] / a.a_div;
   }
 #pragma unroll
-  for (int i = 0; i < NLX; ++i) xoff[i] = (unsigned)x_row[i] * (unsigned)(2 * a.lda) + 16 * chunk;
+  for (int i = 0; i < NLX; ++i) {
+    xoff[i] = (unsigned)x_row[i] * (unsigned)(2 * a.lda) + 16 * chunk;
+    if constexpr (FAR) x_far[i] = (const unsigned char*)((const bf16*)a.A + (int64_t)x_row[i] * a.lda) + 16 * chunk;
+  }
   const bf16* A = (const bf16*)a.A + (a.a_index ? 0 : (int64_t)row0 * a.lda);
   const auto x_res = __builtin_amdgcn_make_buffer_rsrc((void*)A, 0, 0xffffffffu, 0x00020000);
-  const auto w_res = __builtin_amdgcn_make_buffer_rsrc((void*)W, 0, 0xffffffffu, 0x00020000);
+  // (a load's rows of W are all gate rows or all up rows; with eight waves that is the same for all of a wave's
+  // loads, with four for every second one)
+  constexpr int HALF = TN / WGM / 2 / RPP;   // loads of half a wave row's rows of W
+  static_assert(!SWIGLU || WAVES % HALF == 0, "a wave's loads i and i + 2 must be alike");
+  auto w_rows = [&](int i) {
+    const bool up = SWIGLU && (i * WAVES + wave) / HALF % 2;
+    return __builtin_amdgcn_make_buffer_rsrc((void*)(W + (up ? (int64_t)N * K : 0)), 0, 0xffffffffu, 0x00020000);
+  };
+  const auto w_res0 = w_rows(0), w_res1 = w_rows(1);
+  typedef const __attribute__((address_space(1))) void* gptr;
   typedef __attribute__((address_space(3))) void* lptr;
   // Every lane of every load takes part: with some lanes switched off, a load into LDS did
   // not leave the other lanes' bytes where this layout expects them (products came out wrong).
@@ -259,17 +274,21 @@ __global__ __launch_bounds__(WGM * WGN * 64, (NBX * TM + NBW * TN) * 128 > 80 * 
       unsigned char* buf = smem + x_off + wave * 1024;
       const int k = k_bytes(t);
 #pragma unroll
-      for (int i = decltype(from)::value; i < decltype(to)::value; ++i)
-        if (EVEN || (x_live & (1u << i)))   // (EVEN: all, so that a wait is a constant count)
+      for (int i = decltype(from)::value; i < decltype(to)::value; ++i) {
+        if (!EVEN && !(x_live & (1u << i))) continue;   // (EVEN: all, so that a wait is a constant count)
+        if constexpr (FAR)
+          __builtin_amdgcn_global_load_lds((gptr)(x_far[i] + k), (lptr)(buf + i * (WAVES * 1024)), 16, 0, 0);
+        else
           __builtin_amdgcn_raw_ptr_buffer_load_lds(x_res, (lptr)(buf + i * (WAVES * 1024)), 16, xoff[i], k, 0, 0);
+      }
     };
     auto issue_w = [&](int t, int w_off, auto from, auto to) {
       unsigned char* buf = smem + W_BASE + w_off + wave * 1024;
       const int k = k_bytes(t);
 #pragma unroll
       for (int i = decltype(from)::value; i < decltype(to)::value; ++i)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(w_res, (lptr)(buf + i * (WAVES * 1024)), 16, woff[i], k, 0,
-                                                 decltype(once_tag)::value ? 2 : 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(i % 2 ? w_res1 : w_res0, (lptr)(buf + i * (WAVES * 1024)), 16, woff[i], k,
+                                                 0, decltype(once_tag)::value ? 2 : 0);
     };
     std::integral_constant<int, 0> i0;
     std::integral_constant<int, NLW / 2> i2;
@@ -434,14 +453,15 @@ __global__ __launch_bounds__(WGM * WGN * 64, (NBX * TM + NBW * TN) * 128 > 80 * 
 #endif
 }
 
-// K a whole number of k tiles of 64; byte offsets of 32 bits: the rows of A that an index gathers, and from a
-// gate row to its up row.
+// Do rows of A that an index gathers need whole addresses?
+bool gemm_tile_far(const GemmArgs& a) { return a.a_index && 2ll * a.M * a.lda >= 1ll << 32; }
+
+// K a whole number of k tiles of 64; a tile's rows below 4 GB.
 bool gemm_tile_takes(const GemmArgs& a) {
   const int64_t four_gb = 1ll << 32;
   return a.in_dtype == kBF16 && a.K % 64 == 0 && a.lda % 8 == 0 && ((uintptr_t)a.A % 16 == 0) &&
          ((uintptr_t)a.W % 16 == 0) && a.w_group_stride % 8 == 0 &&
-         2 * (a.a_index ? (int64_t)a.M : 256) * a.lda < four_gb &&
-         2 * ((epilogue_gated(a.epilogue) ? a.N : 0) + 256ll) * a.K < four_gb;
+         2 * 256ll * a.lda < four_gb && 2 * 256ll * a.K < four_gb && (a.offsets || !gemm_tile_far(a));
 }
 
 int gemm_tile_row_tiles(const GemmArgs& a, int rows) {
@@ -473,7 +493,9 @@ static int launch_tiles(const GemmArgs& a, hipStream_t stream) {
   } while (0)
 #define NINFER_TILE_LAUNCH(SW, TYPE)                                                            \
   do {                                                                                          \
-    if (a.offsets) NINFER_TILE_KERNEL(SW, TYPE, kGrouped);                                      \
+    if (TM == 128 && a.offsets && gemm_tile_far(a))                                             \
+      NINFER_TILE_KERNEL(SW, TYPE, (TM == 128 ? kGroupedFar : kGrouped));                       \
+    else if (a.offsets) NINFER_TILE_KERNEL(SW, TYPE, kGrouped);                                 \
     else if (TM == 256 && g.parts > 1) NINFER_TILE_KERNEL(SW, TYPE, (TM == 256 ? kDenseCut : kDense)); \
     else NINFER_TILE_KERNEL(SW, TYPE, kDense);                                                  \
   } while (0)

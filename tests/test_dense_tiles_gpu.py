@@ -64,3 +64,43 @@ def test_gated_last_round(ops):
     with ops.tuned(force_kernel=1):
         ops.swiglu_linear(x, w, whole)
     torch.testing.assert_close(out.float(), whole.float(), atol=1e-3, rtol=2.0 ** -7)
+
+
+@pytest.mark.parametrize("force", [1, 2, 3])
+def test_gated_weights_beyond_4_gb(ops, force):
+    """Up rows 4 GB behind their gate rows: the bits are those of a product of the same rows alone."""
+    m, n, k = 40, 262200, 8192
+    g = torch.Generator("cuda").manual_seed(9)
+    x, w = (torch.randn(r, k, generator=g, device="cuda", dtype=torch.bfloat16) for r in (m, 2 * n))
+    w *= k ** -0.5
+    out, part = (torch.empty(m, f, device="cuda", dtype=torch.bfloat16) for f in (n, 160))   # (129 features and more run here)
+    with ops.tuned(force_kernel=force):
+        ops.swiglu_linear(x, w, out)
+        for first in (0, n // 2, n - 160):
+            ops.swiglu_linear(x, torch.cat([w[first:first + 160], w[n + first:n + first + 160]]), part)
+            assert torch.equal(out[:, first:first + 160], part)
+    last = torch.cat([w[n - 40:n], w[2 * n - 40:]]).double()
+    gate, up = (x.double() @ last.T).split(40, 1)
+    torch.testing.assert_close(out[:, -40:].double(), gate * torch.sigmoid(gate) * up, atol=1e-2, rtol=2.0 ** -7)
+
+
+def test_gathered_rows_beyond_4_gb(ops):
+    """Rows that an index gathers from more than 4 GB: the bits of the same rows gathered from a few."""
+    t, e, h, inner = 524400, 2, 4096, 72
+    g = torch.Generator("cuda").manual_seed(11)
+    x = torch.randn(t, h, generator=g, device="cuda", dtype=torch.bfloat16)
+    w = torch.randn(e, 2 * inner, h, generator=g, device="cuda", dtype=torch.bfloat16) * h ** -0.5
+    order, cut = torch.randperm(t, generator=g, device="cuda").int(), t // 3
+    i32 = lambda *v: torch.tensor(v, device="cuda", dtype=torch.int32)
+    out, few = (torch.empty(r, inner, device="cuda", dtype=torch.bfloat16) for r in (t, 60))
+    ops.grouped_swiglu(x, w, i32(0, cut, t), order, 1, out)
+    last = (order == t - 1).nonzero().flatten()   # the place of A's last row, at one end of its group's choice
+    places = torch.cat([torch.arange(0, 20, device="cuda"), torch.arange(cut - 10, cut + 10, device="cuda"),
+                        torch.arange(t - 19, t, device="cuda"), last]).sort().values
+    with ops.tuned(force_kernel=2):
+        ops.grouped_swiglu(x[order[places].long()], w, i32(0, int((places < cut).sum()), 60),
+                           torch.arange(60, device="cuda", dtype=torch.int32), 1, few)
+    assert torch.equal(out[places], few)
+    rows = x[order[places[-8:]].long()].double()
+    gate, up = (rows @ w[1].double().T).split(inner, 1)
+    torch.testing.assert_close(out[places[-8:]].double(), gate * torch.sigmoid(gate) * up, atol=1e-2, rtol=2.0 ** -7)

@@ -75,6 +75,19 @@ def test_large_operands_keep_the_32_bit_kernel(lib, m, n, k, gated, indexed):
     assert lib.ninfer_gemm_kernel(ctypes.byref(args)) == 1
 
 
+@pytest.mark.parametrize("m,n,k,gated,indexed,rows", [
+    (40, 262143, 8192, 1, 0, 0), (40, 262200, 8192, 1, 0, 0), (40, 600000, 8192, 0, 0, 0), (600000, 512, 4096, 0, 0, 0),
+    (524287, 1408, 4096, 1, 1, 256), (524288, 1408, 4096, 1, 1, 128)])
+def test_large_operands_keep_the_many_row_kernel(lib, m, n, k, gated, indexed, rows):
+    from ninfer_amd.kernels.ops import _GemmArgs
+    args = _GemmArgs(A=16, W=16, C=16, M=m, N=n, K=k, lda=k, ldc=n, groups=1, a_div=1, epilogue=gated, in_dtype=BF16,
+                     out_dtype=BF16)
+    if indexed:
+        args.offsets, args.a_index, args.w_group_stride = 16, 16, 2 * n * k
+        assert lib.ninfer_gemm_tile_rows(ctypes.byref(args)) == rows
+    assert lib.ninfer_gemm_kernel(ctypes.byref(args)) == 4
+
+
 def test_no_block_reads_behind_a_tile_list(lib):
     """The lists hold min(n, n // 16 + experts) and n // 256 + experts tiles of n sorted rows; a launch rounds its
     block rows up and may have more."""
