@@ -871,7 +871,8 @@ __global__ __launch_bounds__(256, 2) void latent_attention_rows_kernel(LatentArg
     mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
     if (__any(mx > m_ref + 8.f)) {   // (also a row's first visible key: its reference is minus infinity)
-      const float m_new = fmaxf(m_ref, mx);
+      // (each row by its own maximum: rows that do not jump keep their reference, whatever their neighbours do)
+      const float m_new = mx > m_ref + 8.f ? mx : m_ref;
       const float al = m_new == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m_ref - m_new);
       l_run *= al;
 #pragma unroll
@@ -1034,4 +1035,9 @@ static int latent_attention_tile(const LatentArgs& a, hipStream_t stream) {
 extern "C" long long ninfer_latent_attention_workspace_floats(const ninfer::LatentArgs* a) {
   if (!ninfer::latent_tile_takes(*a)) return 0;
   return ninfer::latent_tile_workspace_floats(*a, ninfer::latent_tile_plan(*a));
+}
+
+// (token, head) rows of a block of the matrix-core kernels for a step of this shape, 16 or 64 (0: the plain kernel).
+extern "C" int ninfer_latent_attention_block_rows(const ninfer::LatentArgs* a) {
+  return ninfer::latent_tile_takes(*a) ? ninfer::latent_tile_plan(*a).rows : 0;
 }

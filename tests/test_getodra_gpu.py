@@ -4,6 +4,7 @@ decoded token by token, in portions down to two tokens, in mixed batches with pa
 state slots that are given back and used again, and generated greedily through the
 scheduler. bfloat16 is compared with the plain implementation on the bfloat16-rounded
 weights; the 32-bit bound is that of rounding."""
+import ctypes
 import json
 import math
 import os
@@ -480,6 +481,30 @@ def test_latent_prompts_whose_waves_keep_whole_rows(ops, rank, rd, heads, ps, wi
     got = out[:-1].float().cpu().reshape(ctx.T, heads, rank)
     assert (out[-1] == 7.0).all()
     assert max(rel_err(g, w) for g, w in zip(got, want)) < 8e-3   # (the bound of the forms above)
+
+
+def _latent_block_rows(ops, ctx, pool, table, q, rank, rd, ps):
+    """Rows of a block of the kernel that this step runs."""
+    a = ops._latent_args(ctx, pool, table, q.shape[1], 0, rank, rd, 0, ps, pool.dtype)
+    a.q_abs = q.data_ptr()
+    return ops.lib.ninfer_latent_attention_block_rows(ctypes.byref(a))
+
+
+@pytest.mark.parametrize("rank,rd", [(256, 32), (512, 64)])
+def test_latent_rows_do_not_depend_on_their_neighbours(ops, rank, rd):
+    """A row's bits stay what they are when the maxima of the other heads of its token, which share its wave, jump."""
+    heads, n, ps = 16, 2000, 16
+    ctx, pool, table, q, _ = _latent_case(ops, torch.bfloat16, heads, rank, rd, ps, [n], [n], seed=rank)
+    pool, table, outs = pool.bfloat16().to(DEV), table.to(DEV), []
+    for loud in (1.0, 30.0):
+        q2 = q.clone()
+        q2[:, 1:] *= loud
+        q2 = q2.to(DEV)
+        assert _latent_block_rows(ops, ctx, pool, table, q2, rank, rd, ps) == 64
+        out = torch.empty(n, heads * rank, dtype=torch.bfloat16, device=DEV)
+        ops.latent_attention(q2, pool, table, ctx, heads, rank, rd, ps, 0.1, out)
+        outs.append(out.reshape(n, heads, rank))
+    assert torch.equal(outs[0][:, 0], outs[1][:, 0]) and not torch.equal(outs[0][:, 1], outs[1][:, 1])
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
