@@ -366,6 +366,33 @@ static int64_t latent_tile_workspace_floats(const LatentArgs& a, const LatentTil
   return p.n_chunks > 1 ? (int64_t)a.T * a.Hq * p.n_chunks * (a.R + 2) : 0;
 }
 
+// Which request (s) and which of its row tiles (lt) is this block's? The tiles are dealt out from
+// the last one backwards: within a request the later tiles see more keys and run longer,
+// and the long ones should start first. False: there is none.
+template <int ROWS>
+__device__ __forceinline__ bool latent_block_tile(const LatentArgs& a, int& s, int& lt) {
+  if (a.max_qlen == 1) {   // every request has one row's tiles: no walk over the requests
+    const int nt = (a.Hq + ROWS - 1) / ROWS, from_last = (int)blockIdx.x;
+    s = a.S - 1 - from_last / nt;
+    lt = nt - 1 - from_last % nt;
+    return s >= 0;
+  }
+  int total = 0;
+  for (int i = 0; i < a.S; ++i)
+    total += ((a.seq_row_start[i + 1] - a.seq_row_start[i]) * a.Hq + ROWS - 1) / ROWS;
+  int left = total - 1 - (int)blockIdx.x;
+  if (left < 0) return false;
+  for (s = 0; s < a.S; ++s) {
+    const int nt = ((a.seq_row_start[s + 1] - a.seq_row_start[s]) * a.Hq + ROWS - 1) / ROWS;
+    if (left < nt) {
+      lt = left;
+      return true;
+    }
+    left -= nt;
+  }
+  return false;
+}
+
 // Eight waves. HALF: steps of 16 numbers of half a cached row. CT: tiles of 16 output columns of a
 // wave, whose columns are 16 CT w ... In LDS lie one tile of 64 keys, the scores (two halves of
 // the sum) and the probabilities; the queries stay in registers.
@@ -388,33 +415,8 @@ __global__ __launch_bounds__(kLatThreads, 2) void latent_attention_tile_kernel(L
   __shared__ int page_s[2][kLatKeys];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
 
-  // Which request and which of its row tiles is this block's? The tiles are dealt out from
-  // the last one backwards: within a request the later tiles see more keys and run longer,
-  // and the long ones should start first.
-  int s = -1, lt = 0;
-  if (a.max_qlen == 1) {   // every request has one row's tiles: no walk over the requests
-    const int nt = (H + ROWS - 1) / ROWS, from_last = (int)blockIdx.x;
-    if (from_last < a.S * nt) {
-      s = a.S - 1 - from_last / nt;
-      lt = nt - 1 - from_last % nt;
-    }
-  } else {
-    int total = 0;
-    for (int i = 0; i < a.S; ++i)
-      total += ((a.seq_row_start[i + 1] - a.seq_row_start[i]) * H + ROWS - 1) / ROWS;
-    int left = total - 1 - (int)blockIdx.x;
-    for (int i = 0; i < a.S && left >= 0; ++i) {
-      const int n = (a.seq_row_start[i + 1] - a.seq_row_start[i]) * H;
-      const int nt = (n + ROWS - 1) / ROWS;
-      if (left < nt) {
-        s = i;
-        lt = left;
-        break;
-      }
-      left -= nt;
-    }
-  }
-  if (s < 0) return;
+  int s, lt;
+  if (!latent_block_tile<ROWS>(a, s, lt)) return;
   const int chunk_id = blockIdx.y;
   const int row0 = a.seq_row_start[s];
   const int n_flat = (a.seq_row_start[s + 1] - row0) * H;
@@ -670,7 +672,7 @@ __global__ __launch_bounds__(kLatThreads, 2) void latent_attention_tile_kernel(L
 // What bounds it is the LDS (68 KB of operands a wave and tile at 512 + 64 numbers, twice the matrix cores' time)
 // and, with 251 registers, reads only two or three products ahead. Against the kernel above: prompts of 2,048
 // tokens, 16 heads, 512 + 64 numbers 202 -> 140 us; 8 heads, 256 + 32 numbers 111 -> 74; 512 tokens behind 2,000 cached
-// ones 190 -> 146; 64 requests of one row and 40 heads at 2,500 keys 83 -> 67.
+// ones 190 -> 146; 64 requests of one row and 40 heads at 2,500 keys 83 -> 60.
 // In LDS rows are unpadded (a load writes 1 KB side by side): the 16-byte piece p of key k lies at
 // p ^ x(k) (lat_swizzle), chosen on the global side, so that the 16 keys of a fragment read fall into
 // different columns of the banks.
@@ -694,27 +696,15 @@ __global__ __launch_bounds__(256, 2) void latent_attention_rows_kernel(LatentArg
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 15, g = lane >> 4;
 
-  // Which request and which of its row tiles: as in the kernel above, the longest first.
-  int s = -1, lt = 0, total = 0;
-  for (int i = 0; i < a.S; ++i)
-    total += ((a.seq_row_start[i + 1] - a.seq_row_start[i]) * H + ROWS - 1) / ROWS;
-  int left = total - 1 - (int)blockIdx.x;
-  for (int i = 0; i < a.S && left >= 0; ++i) {
-    const int nt = ((a.seq_row_start[i + 1] - a.seq_row_start[i]) * H + ROWS - 1) / ROWS;
-    if (left < nt) {
-      s = i;
-      lt = left;
-      break;
-    }
-    left -= nt;
-  }
-  if (s < 0) return;
+  int s, lt;
+  if (!latent_block_tile<ROWS>(a, s, lt)) return;
   const int chunk_id = blockIdx.y;
   const int row0 = a.seq_row_start[s];
   const int n_flat = (a.seq_row_start[s + 1] - row0) * H;
   const int pos0 = a.seq_pos0[s];
   const int f0 = lt * ROWS;
   const int rows_here = min(ROWS, n_flat - f0);
+  if (rows_here <= 0) return;   // (a request without rows in a decode-only step)
   const int tok_first = f0 / H, tok_last = (f0 + rows_here - 1) / H;
   const int pos_last = pos0 + tok_last;
   const int lo_first = a.window > 0 ? max(0, pos0 + tok_first - a.window + 1) : 0;

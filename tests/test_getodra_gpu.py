@@ -491,6 +491,24 @@ def _latent_block_rows(ops, ctx, pool, table, q, rank, rd, ps):
 
 
 @pytest.mark.parametrize("rank,rd", [(256, 32), (512, 64)])
+@pytest.mark.parametrize("heads,without", [(128, []), (130, [0, 7, 8, 255]), (64, list(range(0, 250)))])
+def test_latent_decode_in_blocks_of_64_rows(ops, rank, rd, heads, without):
+    """Decode-only steps of many heads: whole blocks, a last block of two rows, requests that bring no row."""
+    ps, lengths = 16, [1 + (37 * i) % 260 for i in range(256)]
+    new_rows = [0 if i in without else 1 for i in range(256)]
+    ctx, pool, table, q, cached = _latent_case(ops, torch.bfloat16, heads, rank, rd, ps, lengths, new_rows, seed=heads)
+    ctx.max_kv_len = 2600   # (a bound, as of a captured step: the walk over the keys is cut by it)
+    pool, table = pool.bfloat16().to(DEV), table.to(DEV)
+    assert ctx.max_qlen == 1 and _latent_block_rows(ops, ctx, pool, table, q.to(DEV), rank, rd, ps) == 64
+    out = torch.full((ctx.T + 1, heads * rank), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops.latent_attention(q.to(DEV), pool, table, ctx, heads, rank, rd, ps, 0.1, out[:-1])
+    want = _plain_latent_rows(q, cached, lengths, new_rows, rank, 0.1, 0)
+    got = out[:-1].float().cpu().reshape(ctx.T, heads, rank)
+    assert max(rel_err(a, b) for a, b in zip(got, want)) < 8e-3   # (the bound of the forms above)
+    assert (out[-1] == 7.0).all()
+
+
+@pytest.mark.parametrize("rank,rd", [(256, 32), (512, 64)])
 def test_latent_rows_do_not_depend_on_their_neighbours(ops, rank, rd):
     """A row's bits stay what they are when the maxima of the other heads of its token, which share its wave, jump."""
     heads, n, ps = 16, 2000, 16
