@@ -324,9 +324,10 @@ static void latent_tile_split(const LatentArgs& a, int rows, int* tiles, int* n_
 }
 
 // Has the row a form of its own in the kernel whose waves keep whole rows? Latents of 256 or 512 numbers with 32
-// or 64 turned ones behind them; the output's rows in pieces of 8 bytes.
-static bool latent_rows_takes(const LatentArgs& a) {
-  return (a.R == 256 || a.R == 512) && (a.rd == 32 || a.rd == 64) && ((uintptr_t)a.out % 8 == 0);
+// or 64 turned ones behind them. (By the sizes alone, as the plan is, so that the workspace does not depend on
+// where the output lies; an output that does not take pieces of 8 bytes runs the other kernel.)
+static bool latent_rows_form(const LatentArgs& a) {
+  return (a.R == 256 || a.R == 512) && (a.rd == 32 || a.rd == 64);
 }
 
 // What a step takes in blocks of 16 or 64 rows, in us on this part: rounds of blocks, each a start and
@@ -341,7 +342,7 @@ static float latent_tile_us(const LatentArgs& a, int rows, int half) {
   latent_tile_split(a, rows, &tiles, &n_chunks);
   const int key_tiles = (a.max_kv_len + kLatKeys - 1) / kLatKeys, steps = (key_tiles + n_chunks - 1) / n_chunks;
   const float filled = (float)tiles * n_chunks / device_cu_count(), numbers = half / 18.f;
-  const float high = latent_rows_takes(a) ? 0.7f : 1.f;   // (the kernel whose waves keep whole rows)
+  const float high = latent_rows_form(a) ? 0.7f : 1.f;   // (the kernel whose waves keep whole rows)
   const float start = rows == 16 ? 10.f : 24.f * high;
   const float step = rows == 16 ? 0.9f + 1.2f * (filled < 1.f ? filled : 1.f) : 3.6f * high;
   const float round = start * (0.4f + 0.6f * numbers) + steps * step * numbers;
@@ -1007,7 +1008,7 @@ static int latent_attention_tile(const LatentArgs& a, hipStream_t stream) {
                  (long long)a.workspace_floats, (long long)need);
   int rc;
   if (p.rows == 16) rc = launch_latent_rows<16>(a, p, stream);
-  else if (!latent_rows_takes(a)) rc = launch_latent_rows<64>(a, p, stream);
+  else if (!latent_rows_form(a) || (uintptr_t)a.out % 8 != 0) rc = launch_latent_rows<64>(a, p, stream);
   else if (a.R == 512) rc = a.rd == 64 ? launch_latent_waves<18, 32>(a, p, stream) : launch_latent_waves<17, 32>(a, p, stream);
   else rc = a.rd == 64 ? launch_latent_waves<10, 16>(a, p, stream) : launch_latent_waves<9, 16>(a, p, stream);
   if (rc) return rc;

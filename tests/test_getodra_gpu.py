@@ -490,6 +490,20 @@ def _latent_block_rows(ops, ctx, pool, table, q, rank, rd, ps):
     return ops.lib.ninfer_latent_attention_block_rows(ctypes.byref(a))
 
 
+@pytest.mark.parametrize("rank,rd,lengths,new_rows", [(256, 32, [700], [700]), (512, 64, [2040, 131], [40, 131])])
+def test_latent_output_at_an_odd_place(ops, rank, rd, lengths, new_rows):
+    """Blocks of 64 rows whose output takes no pieces of 8 bytes, whole walks and walks cut into chunks."""
+    heads, ps = 16, 16
+    ctx, pool, table, q, cached = _latent_case(ops, torch.bfloat16, heads, rank, rd, ps, lengths, new_rows, seed=rank)
+    pool, table, q2 = pool.bfloat16().to(DEV), table.to(DEV), q.to(DEV)
+    assert _latent_block_rows(ops, ctx, pool, table, q2, rank, rd, ps) == 64
+    out = torch.full((ctx.T * heads * rank + 2,), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops.latent_attention(q2, pool, table, ctx, heads, rank, rd, ps, 0.1, out[1:-1].view(ctx.T, heads * rank))
+    want = _plain_latent_rows(q, cached, lengths, new_rows, rank, 0.1, 0)
+    assert rel_err(out[1:-1].float().cpu().reshape(ctx.T, heads, rank), want) < 8e-3   # (the bound of the forms above)
+    assert out[0] == 7.0 and out[-1] == 7.0
+
+
 @pytest.mark.parametrize("rank,rd", [(256, 32), (512, 64)])
 @pytest.mark.parametrize("heads,without", [(128, []), (130, [0, 7, 8, 255]), (64, list(range(0, 250)))])
 def test_latent_decode_in_blocks_of_64_rows(ops, rank, rd, heads, without):

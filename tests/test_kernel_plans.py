@@ -88,6 +88,20 @@ def test_large_operands_keep_the_many_row_kernel(lib, m, n, k, gated, indexed, r
     assert lib.ninfer_gemm_kernel(ctypes.byref(args)) == 4
 
 
+@pytest.mark.parametrize("rows,keys,heads", [(1, 2600, 40), (40, 2040, 16), (300, 800, 16), (300, 300, 24), (1100, 2100, 16)])
+def test_latent_workspace_by_the_sizes_alone(lib, rows, keys, heads):
+    """What a step of latent attention asks for does not depend on where its output lies."""
+    from ninfer_amd.kernels.ops import _LatentArgs
+    lib.ninfer_latent_attention_workspace_floats.restype = ctypes.c_longlong
+    plans = set()
+    for out in (0, 16, 18):
+        a = _LatentArgs(pool=16, q_abs=16, out=out, seq_row_start=16, seq_pos0=16, S=1, T=rows, Hq=heads, R=512, rd=64,
+                        max_kv_len=keys, max_qlen=rows, page_size=16, dtype=BF16)
+        plans.add((lib.ninfer_latent_attention_workspace_floats(ctypes.byref(a)),
+                   lib.ninfer_latent_attention_block_rows(ctypes.byref(a))))
+    assert len(plans) == 1
+
+
 def test_no_block_reads_behind_a_tile_list(lib):
     """The lists hold min(n, n // 16 + experts) and n // 256 + experts tiles of n sorted rows; a launch rounds its
     block rows up and may have more."""
