@@ -268,8 +268,7 @@ class SparseMoE(FeedForward):
         if ctx.ops.wants_beside(x.shape[0], self.shared.weight_bytes()):
             # While its blocks leave the GPU room, the second stream starts before the routing's short
             # kernels and fills the device beside them; else after them: they would crawl.
-            room = getattr(ctx.ops, "leaves_room", None)
-            early = room is not None and room(x.shape[0], 2 * self.shared.inner)
+            early = ctx.ops.leaves_room(x.shape[0], 2 * self.shared.inner)
             if early:
                 with ctx.ops.beside():
                     shared = self.shared.down(ctx, self.shared.gate_up(ctx, x))

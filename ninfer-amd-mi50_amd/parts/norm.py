@@ -58,11 +58,10 @@ class RMSNorm(Norm):
 
     def forward_two(self, ctx: StepContext, residual, pending, other: Norm):
         """This norm's rows and `other`'s, of the residual with `pending` added: by one kernel where
-        the two differ in nothing but their gains (a launch of 4.8 us for a few rows less) and the
-        operations in use have that kernel."""
+        the two differ in nothing but their gains (a launch of 4.8 us for a few rows less)."""
         alike = isinstance(other, RMSNorm) and other.size == self.size and other.eps == self.eps \
             and other.center == self.center
-        if not alike or isinstance(pending, (SumRows, NormedRows)) or not hasattr(ctx.ops, "rmsnorm_two"):
+        if not alike or isinstance(pending, (SumRows, NormedRows)):
             return self.forward(ctx, residual, pending), other.forward(ctx, residual, None)
         out, out2 = (ctx.empty((residual.shape[0], self.size)) for _ in range(2))
         pending = plain_rows(ctx, pending)

@@ -31,6 +31,9 @@ class PlainOps:
     def wants_beside(self, rows, weight_bytes=0):
         return rows >= self.beside_min_rows
 
+    def leaves_room(self, rows, features):
+        return rows < 2 * self.beside_min_rows   # (so that they walk both orders)
+
     def beside(self):
         """Work for a second stream: here it simply runs where it is called."""
         return contextlib.nullcontext()
@@ -67,6 +70,10 @@ class PlainOps:
             v = v - v.mean(-1, keepdim=True)
         ms = (v * v).sum(-1, keepdim=True) / v.shape[-1]
         out.copy_((v * torch.rsqrt(ms + eps) * gain).to(out.dtype))
+
+    def rmsnorm_two(self, x, gain, eps, out, gain2, out2, delta=None, rows_sum=None, center=False):
+        self.rmsnorm(x, gain, eps, out, delta, None, rows_sum, center)
+        self.rmsnorm(x, gain2, eps, out2, center=center)
 
     def norm_add(self, residual, y, gain, eps, center=False, weights=None):
         v = _f(y)
