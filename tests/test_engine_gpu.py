@@ -308,7 +308,8 @@ def test_graph_replay_with_many_requests(model_dirs):
 
 # Wide enough, with a prompt long enough, that the engine's steps run the kernels for many rows:
 # prompt attention on the matrix cores over hundreds of keys with a window that ends inside
-# them, grouped products in tiles of 256, 128 and 64 rows, dense products by the library.
+# them, grouped products in tiles of 128 and, of short portions, 64 rows (of 256 at the benchmark's shapes
+# below), dense products by the library.
 CONFIG_WIDE = {
     "architectures": ["Qwen2MoeForCausalLM"], "model_type": "qwen2_moe",
     "num_hidden_layers": 2, "hidden_size": 256, "num_attention_heads": 4,
@@ -354,6 +355,11 @@ def test_long_prompt_on_the_many_row_kernels(wide_case, dtype):
         whole = util.run_schedule(runner, util.schedule_whole("a", toks))["a"]
         assert ops._side is not None and not ops._side_open
         again = util.run_schedule(runner, util.schedule_whole("a2", toks))["a2"]
+        # (at this width the second stream starts before the routing; behind it where it would leave no room)
+        ops.leaves_room = lambda rows, features: False
+        behind = util.run_schedule(runner, util.schedule_whole("a5", toks))["a5"]
+        del ops.leaves_room
+        assert ops.leaves_room(640, 2 * 256)
         ops.beside_min_rows = 1 << 30
         one_stream = util.run_schedule(runner, util.schedule_whole("a1", toks))["a1"]
         ops.beside_min_rows, ops.side_own_max_rows = 512, 1 << 30
@@ -361,6 +367,7 @@ def test_long_prompt_on_the_many_row_kernels(wide_case, dtype):
         other_again = util.run_schedule(runner, util.schedule_whole("a4", toks))["a4"]
     finally:
         ops.beside_min_rows, ops.side_own_max_rows = saved
+        ops.__dict__.pop("leaves_room", None)
     torch.testing.assert_close(other_kernel, ref, **bound(dtype), msg=lambda m: f"other: {m}")
     assert torch.equal(other_again, other_kernel)
     # the second stream from 65 rows on, as for a shared expert with very large weights
@@ -376,7 +383,7 @@ def test_long_prompt_on_the_many_row_kernels(wide_case, dtype):
     assert not ops._side_open and torch.equal(few_two, few_one)
     torch.testing.assert_close(few_two, ref[:90], **bound(dtype), msg=lambda m: f"few rows: {m}")
     torch.testing.assert_close(whole, ref, **bound(dtype), msg=lambda m: f"whole: {m}")
-    assert torch.equal(one_stream, whole) and torch.equal(again, whole)
+    assert torch.equal(one_stream, whole) and torch.equal(again, whole) and torch.equal(behind, whole)
     cut = [("b", toks[:200], list(range(200))), ("b", toks[200:260], list(range(60))),
            ("b", toks[260:], list(range(380)))]
     steps = [([entry], ["b"] if i == len(cut) - 1 else []) for i, entry in enumerate(cut)]

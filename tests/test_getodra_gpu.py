@@ -444,6 +444,26 @@ def test_latent_pages_that_the_table_does_not_hold(ops, rank, rd, heads, new_row
     assert rel_err(out.float().cpu().reshape(ctx.T, heads, rank), want) < 8e-3
 
 
+@pytest.mark.parametrize("rank,rd", [(256, 32), (512, 64), (512, 128)])
+@pytest.mark.parametrize("ps,lengths,new_rows", [(16, [720, 333], [720, 300]), (4, [700], [600]), (64, [2040, 200], [60, 131])])
+def test_latent_pages_that_the_table_does_not_hold_in_blocks_of_64_rows(ops, rank, rd, ps, lengths, new_rows):
+    """The same in long portions: pages that hold all of a wave's keys of a tile, a part of them, several tiles."""
+    heads = 16
+    ctx, pool, table, q, cached = _latent_case(ops, torch.bfloat16, heads, rank, rd, ps, lengths, new_rows, seed=rank)
+    for i, p in ((0, 0), (0, 5), (0, lengths[0] // ps - 1), (len(lengths) - 1, 2)):
+        table[i, p] = -1
+        cached[i][p * ps:(p + 1) * ps] = 0
+    pool, table, q2 = pool.bfloat16().to(DEV), table.to(DEV), q.to(DEV)
+    assert _latent_block_rows(ops, ctx, pool, table, q2, rank, rd, ps) == 64
+    out = torch.empty(ctx.T, heads * rank, dtype=torch.bfloat16, device=DEV)
+    ops.latent_attention(q2, pool, table, ctx, heads, rank, rd, ps, 0.1, out)
+    want = _plain_latent_rows(q, cached, lengths, new_rows, rank, 0.1, 0)
+    # (rows of zeros alone have an output of zero)
+    got, size = out.float().cpu().reshape(ctx.T, heads, rank), want.abs().amax().item()
+    assert max(rel_err(a, b) for a, b in zip(got, want) if b.abs().amax() > 1e-3 * size) < 8e-3
+    assert all(a.abs().amax() == 0 for a, b in zip(got, want) if b.abs().amax() == 0)
+
+
 @pytest.mark.parametrize("rank,rd", LATENT_FORMS)
 @pytest.mark.parametrize("heads,new_rows", [(16, [260, 130, 64]), (40, [1, 1, 1]), (70, [1, 1, 1]), (3, [1, 90, 40]),
                                             (40, [260, 1, 200])])

@@ -62,6 +62,19 @@ def test_height_of_dense_tiles(lib, m, n, k, gated, beside, rows):
     assert lib.ninfer_gemm_tile_rows(ctypes.byref(args)) == rows
 
 
+# (both sides of 40 rows a group, and of as many tall tiles as CUs: 16 groups of 2 x 704 features are 16 x 6)
+@pytest.mark.parametrize("m,groups,n,gated,rows", [
+    (60 * 40, 60, 1408, 1, 64), (60 * 41 - 1, 60, 1408, 1, 64), (60 * 41, 60, 1408, 1, 256), (60 * 17, 60, 2048, 0, 64),
+    (60 * 137, 60, 1408, 1, 256), (60 * 137, 60, 2048, 0, 256), (16 * 255, 16, 704, 1, 128), (16 * 256, 16, 704, 1, 128),
+    (16 * 512, 16, 704, 1, 256), (31 * 60, 31, 1024, 1, 128), (32 * 60, 32, 1024, 1, 256), (16 * 2048, 16, 512, 0, 256),
+    (1280, 4, 192, 1, 128)])
+def test_height_of_grouped_tiles(lib, m, groups, n, gated, rows):
+    from ninfer_amd.kernels.ops import _GemmArgs
+    args = _GemmArgs(M=m, N=n, K=1024, lda=1024, ldc=n, in_dtype=BF16, out_dtype=BF16, epilogue=gated, groups=groups,
+                     offsets=16)
+    assert lib.ninfer_gemm_tile_rows(ctypes.byref(args)) == rows
+
+
 # (32-bit operands on both sides of 4 GB: an output head, a gated product's weights, a prompt's rows, rows that an
 # index gathers)
 @pytest.mark.parametrize("m,n,k,gated,indexed", [

@@ -378,7 +378,7 @@ def test_routing_in_one_call_with_tile_lists(ops, gen, t, e, k):
     assert sorted(r1.order.tolist()) == list(range(n))
 
 
-@pytest.mark.parametrize("force,big", [(1, 64), (2, 128), (0, 256)])
+@pytest.mark.parametrize("force,big", [(1, 64), (2, 128), (3, 256), (0, 256)])   # (0: the height the library takes)
 def test_grouped_products_do_not_depend_on_the_order_within_an_expert(ops, gen, force, big):
     """The grouping leaves the rows of an expert in the order its atomic counters gave
     them, which differs from run to run. A routed row's result must not depend on its

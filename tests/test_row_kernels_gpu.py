@@ -91,3 +91,23 @@ def test_two_norms_of_the_same_rows(ops, dtype, width, center):
     ops.rmsnorm_two(twice, gains[0].contiguous(), 1e-6, got[0], gains[1].contiguous(), got[1], delta=delta,
                     center=center)
     assert torch.equal(once, twice) and torch.equal(want[0], got[0]) and torch.equal(want[1], got[1])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("width", [2048, 1022])
+@pytest.mark.parametrize("shared", [False, True])
+def test_two_norms_of_the_same_rows_behind_a_weighted_sum(ops, dtype, width, shared):
+    """The same where the sum before the first is that of a sparse feed-forward's rows."""
+    from ninfer_amd.parts import PendingRows
+    gen = torch.Generator(device="cuda").manual_seed(width)
+    draw = lambda *size: torch.randn(*size, generator=gen, device="cuda")
+    x, gains, logits = draw(5, width), draw(2, width), draw(5, 7)
+    rows = PendingRows(draw(15, width).to(dtype), draw(5, 3).abs(), draw(5, width).to(dtype) if shared else None,
+                       logits[:, 6] if shared else None)
+    once, twice = x.clone(), x.clone()
+    want, got = ([torch.empty(5, width, dtype=dtype, device="cuda") for _ in range(2)] for _ in range(2))
+    ops.rmsnorm(once, gains[0].contiguous(), 1e-6, want[0], rows_sum=rows)
+    ops.rmsnorm(once, gains[1].contiguous(), 1e-6, want[1])
+    ops.rmsnorm_two(twice, gains[0].contiguous(), 1e-6, got[0], gains[1].contiguous(), got[1], rows_sum=rows)
+    assert not torch.equal(once, x) and torch.equal(once, twice)
+    assert torch.equal(want[0], got[0]) and torch.equal(want[1], got[1])
