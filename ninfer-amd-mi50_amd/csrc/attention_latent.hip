@@ -334,18 +334,23 @@ static bool latent_rows_form(const LatentArgs& a) {
 // a walk over its keys, and the merge of chunks. Low blocks start sooner (queries, first tile, output:
 // 10 against 24 us at 576 numbers a row) and meet a tile of 64 keys in 0.9 us while few of them run and
 // in 2.1 when they fill the GPU (every block brings the same bytes from L2), high ones in 3.6 and for
-// four times the rows. 512 + 64 numbers, 16 heads, us in low and in high blocks: a prompt of 64 tokens 14
-// and 32 (blocks of 32 rows of four waves, the kernel before: 23), of 300 30 and 54, of 2,048 389 and
-// 188; 40 heads, 64 requests at 2,500 keys 118 and 84, at 300 26 and 44.
+// four times the rows; in the kernel whose waves keep whole rows 0.7 of that. 512 + 64 numbers, 16 heads, us in low
+// and in high blocks, of which the last in that kernel: a prompt of 64 tokens 14, 32 and 15, of 300 29, 54 and 36, of
+// 2,048 389, 188 and 140; 40 heads, 64 requests at 2,500 keys 118, 84 and 60.
+// A prompt of its own sees half of its keys on average, which counts once its blocks run in rounds; without that, prompts
+// of 200 to 300 tokens whose few high blocks need chunks and a merge went to them (40 heads, 256 + 32 numbers, 200
+// tokens: 18 us in low blocks, 29 in high ones). Taken into account for the forms of that kernel, where both were measured.
 static float latent_tile_us(const LatentArgs& a, int rows, int half) {
   int tiles, n_chunks;
   latent_tile_split(a, rows, &tiles, &n_chunks);
   const int key_tiles = (a.max_kv_len + kLatKeys - 1) / kLatKeys, steps = (key_tiles + n_chunks - 1) / n_chunks;
   const float filled = (float)tiles * n_chunks / device_cu_count(), numbers = half / 18.f;
-  const float high = latent_rows_form(a) ? 0.7f : 1.f;   // (the kernel whose waves keep whole rows)
+  const bool waves = latent_rows_form(a);   // (the kernel whose waves keep whole rows)
+  const float high = waves ? 0.7f : 1.f;
   const float start = rows == 16 ? 10.f : 24.f * high;
   const float step = rows == 16 ? 0.9f + 1.2f * (filled < 1.f ? filled : 1.f) : 3.6f * high;
-  const float round = start * (0.4f + 0.6f * numbers) + steps * step * numbers;
+  const float seen = waves && filled > 1.f && a.max_qlen == a.max_kv_len ? 0.55f : 1.f;
+  const float round = start * (0.4f + 0.6f * numbers) + steps * step * numbers * seen;
   return round * (filled > 1.f ? filled : 1.f) + (n_chunks > 1 ? 6.f : 0.f);
 }
 

@@ -101,6 +101,21 @@ def test_large_operands_keep_the_many_row_kernel(lib, m, n, k, gated, indexed, r
     assert lib.ninfer_gemm_kernel(ctypes.byref(args)) == 4
 
 
+# (prompts of their own, portions behind cached keys and decode steps; both heights of blocks measured)
+@pytest.mark.parametrize("rank,rd,heads,requests,new,keys,rows", [
+    (256, 32, 40, 1, 200, 200, 16), (512, 64, 16, 1, 300, 300, 16), (256, 32, 24, 1, 300, 300, 16),
+    (512, 64, 16, 1, 400, 400, 16), (512, 64, 8, 1, 700, 700, 16), (512, 64, 16, 1, 512, 512, 64),
+    (512, 64, 24, 1, 400, 400, 64), (256, 32, 40, 1, 300, 300, 64), (512, 64, 16, 1, 2048, 2048, 64),
+    (512, 64, 16, 1, 512, 2512, 64), (512, 64, 8, 8, 505, 701, 64), (512, 64, 40, 64, 1, 2500, 64),
+    (512, 64, 40, 64, 1, 300, 16), (512, 64, 16, 1, 1, 4000, 16)])
+def test_height_of_latent_blocks(lib, rank, rd, heads, requests, new, keys, rows):
+    from ninfer_amd.kernels.ops import _LatentArgs
+    t = requests if new == 1 else new + requests - 1   # (one portion, the others single rows)
+    a = _LatentArgs(pool=16, q_abs=16, out=16, seq_row_start=16, seq_pos0=16, S=requests, T=t, Hq=heads, R=rank, rd=rd,
+                    max_kv_len=keys, max_qlen=new, page_size=16, dtype=BF16)
+    assert lib.ninfer_latent_attention_block_rows(ctypes.byref(a)) == rows
+
+
 @pytest.mark.parametrize("rows,keys,heads", [(1, 2600, 40), (40, 2040, 16), (300, 800, 16), (300, 300, 24), (1100, 2100, 16)])
 def test_latent_workspace_by_the_sizes_alone(lib, rows, keys, heads):
     """What a step of latent attention asks for does not depend on where its output lies."""
