@@ -29,12 +29,29 @@ static float dense_us_256(int tiles, int cus, int K, bool beside) {
   return round * (1.22f * whole + (last == 0 ? 0.f : 4 * last <= cus ? 0.52f : 2 * last <= cus ? 0.62f : 1.22f));
 }
 
-// Tile height of a product. Grouped: the tall tile, which loads and multiplies only the 32-row blocks that
-// hold rows, except for few rows per group, where tiles of 64 rows, two blocks a CU, stream the weights
-// better (60 groups of 2 x 1,408 x 2,048 and 2,048 x 1,408: 34 rows on average 122 + 63 us against 129 + 66, 17 rows
-// 116 + 59 against 123 + 63; 60 rows 152 + 81 against 136 + 71), and where the tall tiles would leave CUs
-// without a block (16 groups of 2 x 704 x 1,024 and 1,024 x 704, 256 rows on average: tiles of 128 rows 26 + 18 us
-// against 31 + 23). Dense: 64 rows while taller tiles would leave CUs without a block, else 128 or 256 by
+// Tile height of a grouped product, by the number of tiles that a CU gets. A row tile's blocks run on one
+// XCD (block_to_tile), so that is the number of feature tiles times that of the row tiles an XCD gets: of evenly
+// filled groups, each of which has one up to three quarters of a tile's rows and a half filled one more beyond.
+// - Up to 40 rows a group on average 64 rows, two blocks a CU, which stream the weights better: 60 groups of
+//   2 x 1,408 x 2,048 and 2,048 x 1,408, 34 rows 122 + 63 us against 129 + 66 in tall tiles (60 rows 152 + 81 against
+//   136 + 71). With choices that fall off as 1 / rank they are 2 to 10% slower instead, and up to 29% with few groups of many
+//   features, where one row tile more is an XCD's second (8 groups of 2 x 14,336 x 4,096, 25 rows: 290 us against 324, so
+//   432 against 336): there tall tiles.
+// - 128 rows while a CU gets less than the two such tiles that it holds side by side: 16 groups of 2 x 704 x 1,024 and
+//   1,024 x 704, 191 rows 23 + 14 us against 28 + 20 in tall tiles; 4 groups of 2,048 x 4,096, 256 rows 42 against 78.
+//   From two on tall tiles: 10 groups of 2 x 4,096 x 4,096, 140 rows 138 us against 83; 8 of 4,096 x 14,336, 128 rows 352
+//   against 229; 32 of 2 x 256 x 768, 512 rows 37 against 26.
+// - The tall tile loads and multiplies only the 32-row blocks that hold rows.
+static int grouped_rows_of(const GemmArgs& a, int w_rows, int cus) {
+  auto per_cu = [&](int tm, int tn) {
+    const float filled = (float)a.M / a.groups / tm, row_tiles = a.groups * (filled <= 0.75f ? 1.f : filled + 0.5f);
+    return ceilf(row_tiles / kXcds) * ((w_rows + tn - 1) / tn) * kXcds / cus;
+  };
+  if (a.M / a.groups <= 40) return a.groups <= 16 && per_cu(256, 256) >= 3.f ? kGroupedTileRows : 64;
+  return per_cu(128, 128) < 2.f ? 128 : kGroupedTileRows;
+}
+
+// Tile height of a dense product: 64 rows while taller tiles would leave CUs without a block, else 128 or 256 by
 // an estimate of both times (dense_us_128, dense_us_256); where one output a feature is stored instead of
 // one of two, as many tall tiles as CUs decide for them too, whose stores cost less (32-bit outputs, K
 // 1,024: 1,531 x 12,800 56 us in tiles of 256 and 68 in those of 128, 3,000 x 6,144 53 and 66). force_kernel
@@ -46,11 +63,7 @@ static int tile_rows_of(const GemmArgs& a) {
   const int n_units = gated ? 2 * a.N : a.N;   // W rows
   auto blocks = [&](int tm, int tn) { return ((a.M + tm - 1) / tm) * ((n_units + tn - 1) / tn); };
   const int cus = device_cu_count(), low = blocks(128, 128), tall = blocks(256, 256);
-  if (a.offsets) {
-    const int mean = a.M / a.groups;
-    if (mean <= 40) return 64;
-    return a.groups * (mean / 256 + 1) * ((n_units + 255) / 256) < cus ? 128 : kGroupedTileRows;
-  }
+  if (a.offsets) return grouped_rows_of(a, n_units, cus);
   if (a.M <= 64 || low < cus) return 64;   // (no taller than the rows there are)
   if (a.M <= 128) return 128;
   return (!gated && tall >= cus) || dense_us_256(tall, cus, a.K, a.beside) < dense_us_128(low, cus, a.K) ? 256 : 128;

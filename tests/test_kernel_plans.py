@@ -62,12 +62,15 @@ def test_height_of_dense_tiles(lib, m, n, k, gated, beside, rows):
     assert lib.ninfer_gemm_tile_rows(ctypes.byref(args)) == rows
 
 
-# (both sides of 40 rows a group, and of as many tall tiles as CUs: 16 groups of 2 x 704 features are 16 x 6)
+# (both sides of 40 rows a group and of two tiles of 128 rows a CU; few groups of many features)
 @pytest.mark.parametrize("m,groups,n,gated,rows", [
     (60 * 40, 60, 1408, 1, 64), (60 * 41 - 1, 60, 1408, 1, 64), (60 * 41, 60, 1408, 1, 256), (60 * 17, 60, 2048, 0, 64),
     (60 * 137, 60, 1408, 1, 256), (60 * 137, 60, 2048, 0, 256), (16 * 255, 16, 704, 1, 128), (16 * 256, 16, 704, 1, 128),
-    (16 * 512, 16, 704, 1, 256), (31 * 60, 31, 1024, 1, 128), (32 * 60, 32, 1024, 1, 256), (16 * 2048, 16, 512, 0, 256),
-    (1280, 4, 192, 1, 128)])
+    (16 * 512, 16, 704, 1, 256), (16 * 512, 16, 1024, 0, 256), (1280, 4, 192, 1, 128), (4 * 256, 4, 2048, 0, 128),
+    (4 * 87, 4, 4096, 1, 256), (8 * 87, 8, 2048, 1, 128), (8 * 128, 8, 2048, 1, 256), (8 * 512, 8, 1024, 0, 128),
+    (1400, 10, 4096, 1, 256), (8 * 128, 8, 4096, 0, 256), (32 * 512, 32, 256, 1, 256), (64 * 143, 64, 320, 1, 256),
+    (40 * 512, 40, 512, 0, 256), (8 * 25, 8, 14336, 1, 256), (16 * 32, 16, 8192, 1, 256), (12 * 25, 12, 2816, 1, 64),
+    (17 * 25, 17, 14336, 1, 64)])
 def test_height_of_grouped_tiles(lib, m, groups, n, gated, rows):
     from ninfer_amd.kernels.ops import _GemmArgs
     args = _GemmArgs(M=m, N=n, K=1024, lda=1024, ldc=n, in_dtype=BF16, out_dtype=BF16, epilogue=gated, groups=groups,
