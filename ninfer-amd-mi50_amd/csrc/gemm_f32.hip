@@ -21,6 +21,7 @@
 // 175 -> 127; 2 x 5,632 features 158 -> 95, 84 of the 155 TFLOP/s that a large matrix product reaches; 6,144
 // features 85 -> 55; 2,048 features 31 -> 20. One row: 92 MB of gate/up 22 -> 18, 2,048 features 9.3 -> 7.7.
 #include "gemm.h"
+#include <type_traits>
 
 namespace ninfer {
 
@@ -113,21 +114,23 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_f32_kernel(GemmArgs a, int n_
   auto issue = [&](int g) {
     unsigned char* buf = ring + (g & 1) * STAGE;
     const int k0 = (b0 + 2 * g) * kF32Chunk;
+    // (what lies behind the row's end is never read: its last 16 bytes again)
+    auto at = [&](int i) { return off[i] + 16 * min(lane_chunk ^ ((4 * i) & 7), (K - k0) / 4 - 1); };
 #pragma unroll
-    for (int i = 0; i < NL; ++i) {
-      // (what lies behind the row's end is never read: its last 16 bytes again)
-      const unsigned o = off[i] + 16 * min(lane_chunk ^ ((4 * i) & 7), (K - k0) / 4 - 1);
-      const auto rows_of_w = GATED && (8 * i - BM) / 16 >= CT / 2 ? up_res : w_res;
-      if (FAR && 8 * i < BM)
-        __builtin_amdgcn_global_load_lds((gptr)(far_row[FAR && 8 * i < BM ? i : 0] + o + (int64_t)k0 * 4),
-                                         (lptr)(buf + i * 1024), 16, 0, 0);
-      else if (8 * i < BM)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(a_res, (lptr)(buf + i * 1024), 16, o, k0 * 4, 0, 0);
-      else if (once)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rows_of_w, (lptr)(buf + i * 1024), 16, o, k0 * 4, 0, 2);
+    for (int i = 0; i < BM / 8; ++i) {
+      if constexpr (FAR)
+        __builtin_amdgcn_global_load_lds((gptr)(far_row[i] + at(i) + (int64_t)k0 * 4), (lptr)(buf + i * 1024), 16, 0, 0);
       else
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rows_of_w, (lptr)(buf + i * 1024), 16, o, k0 * 4, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(a_res, (lptr)(buf + i * 1024), 16, at(i), k0 * 4, 0, 0);
     }
+    auto weights = [&](auto mark) {
+#pragma unroll
+      for (int i = BM / 8; i < NL; ++i)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(GATED && (8 * i - BM) / 16 >= CT / 2 ? up_res : w_res,
+                                                 (lptr)(buf + i * 1024), 16, at(i), k0 * 4, 0, decltype(mark)::value);
+    };
+    if (once) weights(std::integral_constant<int, 2>{});
+    else weights(std::integral_constant<int, 0>{});
   };
   // Fragments of chunk c of stage g: the lane holds four neighbouring k of one row, so a chunk is
   // four instructions with k dealt alike to both operands.
