@@ -255,30 +255,40 @@ static void launch(const GemmArgs& a, hipStream_t stream) {
   gemm_f32_kernel<WAVES, RT, CT, false, FAR><<<grid, 64 * WAVES, 0, stream>>>(a, n_tiles, m_tiles);
 }
 
-int gemm_f32(const GemmArgs& a, hipStream_t stream) {
-  // The tile whose blocks take the least time. Of each: a block alone on its CU, and what every further
-  // block on that CU adds, in us at K 2,048 (measured over 1 to 1,024 rows of 61 to 151,936 features, K 1,024
-  // to 5,632; both go with K). Where one block fills a CU its blocks come in whole rounds; where several
-  // share one, a part of a round costs less. (173 rows, measured: 6,144 features 55 with four waves and 3 x 2
-  // tiles, 55 with 1 x 2, 60 with eight waves and 1 x 1; 2,048 features 20, 20 and 23; one row, 2,048 features: 20,
-  // 11 and 7.7; gated 2 x 5,632, 64 rows: 53, 43, and 41 with eight waves and 2 x 2.)
-  struct Tile { int waves, rt, ct; float alone, further; bool shared; };
-  static const Tile tiles[] = {{8, 1, 1, 3.5f, 3.4f, true}, {8, 1, 2, 5.f, 8.f, false}, {8, 2, 2, 8.5f, 12.4f, false},
-                               {4, 1, 2, 7.f, 6.2f, true},  {4, 2, 2, 11.f, 11.9f, true}, {4, 3, 2, 15.5f, 16.9f, true}};
+// The tile whose blocks take the least time. Of each: a block alone on its CU, and what every further
+// block on that CU adds, in us at K 2,048 (measured over 1 to 1,024 rows of 61 to 151,936 features, K 1,024
+// to 5,632; both go with K), and of both what is left as K goes from 1,024 to nothing (starts, the 8 sums added up: 32 groups
+// of 512 x 384, 4 rows each, 12.5 us with eight waves and 1 x 1 tiles, 7.3 with four and 1 x 2; 2,048 rows of 384 x 512 20.6 with
+// eight and 2 x 2, 17.6 with four). Where one block fills a CU its blocks come in whole rounds; where several
+// share one, a part of a round costs less. (173 rows, measured: 6,144 features 55 with four waves and 3 x 2
+// tiles, 55 with 1 x 2, 60 with eight waves and 1 x 1; 2,048 features 20, 20 and 23; one row, 2,048 features: 20,
+// 11 and 7.7; gated 2 x 5,632, 64 rows: 53, 43, and 41 with eight waves and 2 x 2.)
+struct F32Tile { int waves, rt, ct; float alone, further, alone_short, further_short; bool shared; };
+static const F32Tile kF32Tiles[] = {{8, 1, 1, 3.5f, 3.4f, 0.f, 1.5f, true},     {8, 1, 2, 5.f, 8.f, 0.f, 3.f, false},
+                                    {8, 2, 2, 8.5f, 12.4f, 1.f, 6.f, false},    {4, 1, 2, 7.f, 6.2f, 0.f, 1.f, true},
+                                    {4, 2, 2, 11.f, 11.9f, 1.f, 2.f, true},     {4, 3, 2, 15.5f, 16.9f, 4.5f, 6.f, true}};
+static int f32_tile(const GemmArgs& a) {
   const bool gated = epilogue_gated(a.epilogue);
-  const float columns = (float)a.N * (gated ? 2 : 1), cus = device_cu_count();
+  const float columns = (float)a.N * (gated ? 2 : 1), cus = device_cu_count(), k = fminf(1.f, a.K / 1024.f);
   int best = -1;
   float least = 0.f;
   for (int i = 0; i < 6; ++i) {
-    const Tile& t = tiles[i];
+    const F32Tile& t = kF32Tiles[i];
     if (gated && t.ct == 1) continue;
     const float rows = 16.f * t.rt;
     // (a group's last tile is half full on average)
     const float m_tiles = a.offsets ? a.M / rows + 0.5f * a.groups : ceilf(a.M / rows);
     const float per_cu = fmaxf(1.f, ceilf(columns / (16 * t.ct)) * m_tiles / cus), whole = ceilf(per_cu);
-    const float us = t.alone + t.further * ((t.shared ? 0.5f * (per_cu + whole) : whole) - 1.f);
+    const float alone = t.alone_short + (t.alone - t.alone_short) * k;
+    const float further = t.further_short + (t.further - t.further_short) * k;
+    const float us = alone + further * ((t.shared ? 0.5f * (per_cu + whole) : whole) - 1.f);
     if (best < 0 || us < least) best = i, least = us;
   }
+  return best;
+}
+
+int gemm_f32(const GemmArgs& a, hipStream_t stream) {
+  int best = f32_tile(a);
   // 4 GB of rows that an index gathers are many: the tallest tile. (Every tile gives the same bits.)
   if (a.a_index && 4ll * a.M * a.lda >= 1ll << 32) best = 6;
   switch (best) {
@@ -295,3 +305,9 @@ int gemm_f32(const GemmArgs& a, hipStream_t stream) {
 }
 
 }  // namespace ninfer
+
+// The tile of a 32-bit product: 100 x waves + 10 x tiles of 16 rows + tiles of 16 rows of W.
+extern "C" int ninfer_gemm_f32_tile(const ninfer::GemmArgs* args) {
+  const ninfer::F32Tile& t = ninfer::kF32Tiles[ninfer::f32_tile(*args)];
+  return 100 * t.waves + 10 * t.rt + t.ct;
+}

@@ -62,6 +62,17 @@ def test_height_of_dense_tiles(lib, m, n, k, gated, beside, rows):
     assert lib.ninfer_gemm_tile_rows(ctypes.byref(args)) == rows
 
 
+# (a short K, where starts and sums outweigh the products, and a model's)
+@pytest.mark.parametrize("m,groups,n,k,gated,tile", [
+    (128, 32, 512, 384, 0, 412), (264, 32, 768, 256, 0, 412), (2048, 0, 384, 512, 0, 422), (2048, 0, 192, 512, 1, 422),
+    (1, 0, 2048, 2048, 0, 811), (173, 0, 2048, 2048, 0, 432), (173, 0, 6144, 2048, 0, 432), (64, 0, 5632, 2048, 1, 822),
+    (692, 60, 1408, 2048, 1, 412), (300, 0, 2048, 5632, 0, 432)])
+def test_tile_of_32_bit_products(lib, m, groups, n, k, gated, tile):
+    from ninfer_amd.kernels.ops import _GemmArgs
+    args = _GemmArgs(M=m, N=n, K=k, lda=k, ldc=n, epilogue=gated, groups=groups or 1, offsets=16 if groups else 0)
+    assert lib.ninfer_gemm_f32_tile(ctypes.byref(args)) == tile
+
+
 # (both sides of 40 rows a group and of two tiles of 128 rows a CU; few groups of many features)
 @pytest.mark.parametrize("m,groups,n,gated,rows", [
     (60 * 40, 60, 1408, 1, 64), (60 * 41 - 1, 60, 1408, 1, 64), (60 * 41, 60, 1408, 1, 256), (60 * 17, 60, 2048, 0, 64),
