@@ -77,8 +77,7 @@ struct GemmArgs {
   // What tests and measurements ask of one call (all 0: the library chooses). Per call, not
   // state of the library: a caller that forgets to reset it changes nothing for the next.
   int64_t split_min_bytes;  // least bytes of weights for a cut along K (0: 48 MB)
-  int force_kernel;      // many-row kernel: 1, 2, 3 = tiles of 64, 128, 256 rows (grouped
-                         // products run 256-row tiles unless told otherwise here)
+  int force_kernel;      // many-row kernel: 1, 2, 3 = tiles of 64, 128, 256 rows
   int skinny_two;        // few-row grouped products with two feature sets per block: 1 = whenever
                          // the shape allows, -1 = never
   float act_limit;       // kEpilogueClampedSwish: the range both halves are cut to (> 0)

@@ -22,9 +22,9 @@
 // The lower tiles staged their operands through registers before: 512 rows of 2 x 5,632, K 2,048, 43 -> 36 us
 // in tiles of 128, 512 rows of 2 x 2,816 29 -> 20 in tiles of 64.
 // A wave column multiplies only its 32-row blocks that hold rows (the tile's rows
-// fill the columns' blocks one after the other, the first column's first), and
+// fill the columns' blocks one after the other, the first column's first), and in the two taller tiles
 // a wave loads only the pieces of A that hold rows, so a tile with few rows costs little
-// more than its share.
+// more than its share (the lowest tile loads all its pieces, so that a wait is a constant count).
 //
 // LDS rows are 128 bytes (64 bf16) and unpadded, because a wave's load writes
 // 1 KB contiguously (lane l at 16 l); the eight 16-byte chunks of row r are
@@ -63,9 +63,9 @@ template <int N> __device__ __forceinline__ void wait_loads_and_lds() {
 // A dense product's tiles run in rounds of one to a CU. The tiles of the last round, when they
 // leave half of the CUs idle or more, are cut into 2 or 4 blocks of 128 or 64 rows, which take a
 // half to two thirds of a whole tile's time (2 x 5,632 features, K 2,048: 2,048 rows, 352 tiles on
-// 256 CUs, 134 -> 120 us; 1,531 rows, 264 tiles, 125 -> 104). Not beside other products, whose
+// 256 CUs, 96 -> 84 us; 1,531 rows, 264 tiles, 94 -> 75). Not beside other products, whose
 // blocks take those CUs: a 2,048-token prompt of the headline model, whose shared expert runs beside
-// the routed ones, 14.31 -> 14.74 ms with the cut.
+// the routed ones, 13.38 -> 13.56 ms with the cut.
 struct DirectGrid {
   int m_tiles, n_tiles;
   int whole;   // tiles that are one block each: those before the last round
