@@ -733,15 +733,17 @@ class HipOps:
             return False
         return not torch.cuda.is_current_stream_capturing()
 
-    def leaves_room(self, rows: int, features: int) -> bool:
+    def leaves_room(self, rows: int, features: int, to_fill: bool = False) -> bool:
         """Does a product of this size leave CUs, or places on them, to short kernels on another stream?
-        While its tall tiles (256 x 256, one to a CU) would be fewer than the CUs. Measured on the shared
+        While its tall tiles (256 x 256, one to a CU) would be fewer than the CUs, or than half of them where
+        the work behind the short kernels has a last round that it had better fill (`to_fill`). Measured on the shared
         expert's products started before the routing against after it: steps of 512 rows of the headline
-        model (88 tiles of 2 x 5,632 features) 9.07 -> 8.68 ms, 1,531 rows of 2 x 2,816 (132) 4.03 -> 4.01;
-        2,048 rows of 2 x 5,632 (352) 13.31 -> 13.67."""
+        model (88 tiles of 2 x 5,632 features) 8.37 -> 7.99 ms, 600 (132) 9.00 -> 8.64; 2,048 (352) 13.14 -> 13.55; with
+        `to_fill` 850 (176) 9.17 -> 9.46, 1,024 (176) 9.55 -> 9.86, 700 (132) 8.97 -> 9.02; 2,048 rows of
+        2 x 2,816 (176) without it 5.18 -> 5.08; Qwen2-57B-A14B's layers, 200 rows (160) 5.20 -> 4.95 for six of them."""
         if self._cus is None:
             self._cus = torch.cuda.get_device_properties(torch.cuda.current_device()).multi_processor_count
-        return -(-rows // 256) * -(-features // 256) < self._cus
+        return -(-rows // 256) * -(-features // 256) < (self._cus // 2 if to_fill else self._cus)
 
     def beside(self):
         """Context manager for work that nothing on the current stream waits for until

@@ -251,6 +251,12 @@ class SparseMoE(FeedForward):
             w.hold(self.router.prefix + self.router.leaf, self.router.weight)
             w.hold(self.prefix + self.names["shared_gate"], self.shared_gate)
 
+    def _shared_fills(self, rows: int) -> bool:
+        """Had the shared expert better fill the last round of the routed products' tiles than run before
+        them? Where those are tall (more than 40 rows an expert) and it is more than half of a token's routed work."""
+        k = self.router.top_k
+        return rows * k > 40 * self.router.experts and 2 * self.shared.inner > k * self.experts.inner
+
     def forward(self, ctx: StepContext, x, residual):
         if self.shared is None:
             with ctx.ops.together():   # for few rows the logits' block routes the rows itself
@@ -268,7 +274,7 @@ class SparseMoE(FeedForward):
         if ctx.ops.wants_beside(x.shape[0], self.shared.weight_bytes()):
             # While its blocks leave the GPU room, the second stream starts before the routing's short
             # kernels and fills the device beside them; else after them: they would crawl.
-            early = ctx.ops.leaves_room(x.shape[0], 2 * self.shared.inner)
+            early = ctx.ops.leaves_room(x.shape[0], 2 * self.shared.inner, self._shared_fills(x.shape[0]))
             if early:
                 with ctx.ops.beside():
                     shared = self.shared.down(ctx, self.shared.gate_up(ctx, x))

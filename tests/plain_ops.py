@@ -31,7 +31,7 @@ class PlainOps:
     def wants_beside(self, rows, weight_bytes=0):
         return rows >= self.beside_min_rows
 
-    def leaves_room(self, rows, features):
+    def leaves_room(self, rows, features, to_fill=False):
         return rows < 2 * self.beside_min_rows   # (so that they walk both orders)
 
     def beside(self):

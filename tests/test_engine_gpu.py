@@ -356,7 +356,7 @@ def test_long_prompt_on_the_many_row_kernels(wide_case, dtype):
         assert ops._side is not None and not ops._side_open
         again = util.run_schedule(runner, util.schedule_whole("a2", toks))["a2"]
         # (at this width the second stream starts before the routing; behind it where it would leave no room)
-        ops.leaves_room = lambda rows, features: False
+        ops.leaves_room = lambda rows, features, to_fill=False: False
         behind = util.run_schedule(runner, util.schedule_whole("a5", toks))["a5"]
         del ops.leaves_room
         assert ops.leaves_room(640, 2 * 256)

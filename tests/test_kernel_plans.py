@@ -62,6 +62,21 @@ def test_height_of_dense_tiles(lib, m, n, k, gated, beside, rows):
     assert lib.ninfer_gemm_tile_rows(ctypes.byref(args)) == rows
 
 
+# (experts, chosen, inner, shared inner; rows: does the shared expert start before the routing?)
+@pytest.mark.parametrize("sizes,rows,early", [
+    ((60, 4, 1408, 5632), 512, True), ((60, 4, 1408, 5632), 600, True), ((60, 4, 1408, 5632), 700, False),
+    ((60, 4, 1408, 5632), 1024, False), ((60, 4, 1408, 5632), 2048, False), ((32, 4, 1408, 2816), 1531, True),
+    ((32, 4, 1408, 2816), 2048, True), ((16, 2, 704, 1408), 2048, True), ((64, 8, 2560, 20480), 200, True),
+    ((64, 8, 2560, 20480), 300, False)])
+def test_which_starts_first(sizes, rows, early):
+    from types import SimpleNamespace
+    from ninfer_amd.kernels.ops import HipOps
+    from ninfer_amd.parts.moe import SparseMoE
+    experts, top, inner, shared = sizes
+    moe = SparseMoE("m.", 2048, experts, top, inner, False, shared_inner=shared)
+    assert HipOps.leaves_room(SimpleNamespace(_cus=256), rows, 2 * shared, moe._shared_fills(rows)) == early
+
+
 # (a short K, where starts and sums outweigh the products, and a model's)
 @pytest.mark.parametrize("m,groups,n,k,gated,tile", [
     (128, 32, 512, 384, 0, 412), (264, 32, 768, 256, 0, 412), (2048, 0, 384, 512, 0, 422), (2048, 0, 192, 512, 1, 422),
