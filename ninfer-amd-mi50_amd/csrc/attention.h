@@ -53,6 +53,14 @@ struct AttnArgs {
   const void* gate;         // of the activation dtype, or null
   int gate_stride;
   const float* sinks;       // [Hq] or null (0): the score of head h's sink, not scaled
+  // Keys and values in rows of their own instead of pages (prompts in bfloat16, every head with keys of its
+  // own, no window): a request's key of position p is row key_start[request] + p of kpool and vpool (rows of
+  // kv_stride numbers, kdim and Dv to a head) and of krot, the D - kdim numbers that all heads share behind
+  // them. The gate then is one number a head: [T, gate_stride], out of head h times sigmoid(gate[t, h]).
+  const void* krot;         // [keys, D - kdim], or null: keys and values in pages
+  const int* key_start;     // [S]
+  int kv_stride;
+  int kdim;
 };
 
 // The score of head h's sink.

@@ -69,7 +69,9 @@ __device__ __forceinline__ void tr_read2(unsigned addr, short4v& r0, short4v& r1
 }
 
 // HEADS: rows are the query heads of one token (decode)
-template <int D, int NQ, bool HEADS, bool BLOCKS>
+// FLAT_DV > 0: prompts over keys and values that lie in rows of their own, one row per key
+// (AttnArgs::krot), with values of FLAT_DV numbers
+template <int D, int NQ, bool HEADS, bool BLOCKS, int FLAT_DV>
 __global__ __launch_bounds__(NQ * 128, 2) void attn_prefill_kernel(AttnArgs a, int CHUNK,
                                                                    int paired) {
   constexpr int KH = 2;             // waves per group of 32 rows: each meets one half of a tile's keys
@@ -77,8 +79,11 @@ __global__ __launch_bounds__(NQ * 128, 2) void attn_prefill_kernel(AttnArgs a, i
   constexpr int NT = NW * 64;
   constexpr int NKB = 2 / KH;       // 32-key blocks of a tile that one wave meets
   constexpr int PQ = NQ * 32;       // query rows per block
+  constexpr bool FLAT = FLAT_DV > 0;
+  static_assert(!FLAT || (!HEADS && !BLOCKS), "keys in rows of their own: prompts without blocks");
+  constexpr int DV = FLAT ? FLAT_DV : D;   // numbers of a value
   constexpr int KS = D / 16;        // k-steps of Q K^T
-  constexpr int DB = D / 32;        // 32-row blocks of O^T
+  constexpr int DB = DV / 32;       // 32-row blocks of O^T
   // Keys and values lie in LDS as they lie in the cache, [key][d], rows of 2 D bytes without
   // padding: they are loaded from global memory straight into LDS (global_load_lds_dwordx4:
   // no staging registers, no LDS stores), and such a load fills 1 KB of LDS contiguously,
@@ -89,9 +94,11 @@ __global__ __launch_bounds__(NQ * 128, 2) void attn_prefill_kernel(AttnArgs a, i
   constexpr int ROW_BYTES = 2 * D;
   constexpr int CPR = ROW_BYTES / 16;        // 16-byte chunks of a row
   constexpr int RPP = 64 / CPR;              // rows that one load of a wave fills (1 KB)
-  constexpr int TILE_BYTES = PK * ROW_BYTES; // of the keys, and of the values, of a tile
-  constexpr int KPT = PK / RPP / NW;         // loads per wave for a tile's keys (as many for its values)
-  static_assert(PK % (RPP * NW) == 0, "tile does not divide over the block's waves");
+  constexpr int TILE_BYTES = PK * ROW_BYTES; // of the keys of a tile
+  constexpr int KPT = PK / RPP / NW;         // loads per wave for a tile's keys
+  constexpr int VROW_BYTES = 2 * DV;         // the same of the values
+  constexpr int VCPR = VROW_BYTES / 16, VRPP = 64 / VCPR, VPT = PK / VRPP / NW;
+  static_assert(PK % (RPP * NW) == 0 && PK % (VRPP * NW) == 0, "tile does not divide over the block's waves");
   // Tiles in LDS: the one being multiplied and NST - 1 on their way. Three where one block
   // fills a CU anyway; two for the blocks of four waves, so that two of them fit a CU.
   constexpr int NST = NQ == 4 ? 3 : 2;
@@ -99,7 +106,7 @@ __global__ __launch_bounds__(NQ * 128, 2) void attn_prefill_kernel(AttnArgs a, i
   constexpr bool EARLY = true;
   // All stages lie in one array of dynamic LDS, a tile's keys, then its values, stage after
   // stage; tile_info's three ints and the merge's (max, sum) pairs behind them.
-  constexpr int STAGE_BYTES = 2 * TILE_BYTES;
+  constexpr int STAGE_BYTES = TILE_BYTES + PK * VROW_BYTES;
   extern __shared__ __attribute__((aligned(1024))) unsigned char stages[];   // NST x STAGE_BYTES + kPrefillExtra
   // At the end the stages merge the two key halves: the output registers of a group of 32
   // rows' second wave, 16 DB floats per lane stored [register][lane], two groups to a stage.
@@ -161,14 +168,14 @@ __global__ __launch_bounds__(NQ * 128, 2) void attn_prefill_kernel(AttnArgs a, i
     pos_last = pos_first + n_rows - 1;
     lo_first = a.window > 0 ? max(0, pos_first - a.window + 1) : 0;
   }
-  const int* bt = a.block_table + (int64_t)seq * a.bt_stride;
+  const int* bt = FLAT ? nullptr : a.block_table + (int64_t)seq * a.bt_stride;
   // the blocks' tiles: n_bt of them, at "keys" t_start .. t_first - 1
   const int t_first = (lo_first / PK) * PK;
   const int* bt_b = BLOCKS ? a.blk_table + (int64_t)seq * a.blk_bt_stride : nullptr;
   const int blocks_last = BLOCKS ? attention_blocks_seen(pos_last, a.window, a.block) : 0;
   const int t_start = BLOCKS ? t_first - (blocks_last + PK - 1) / PK * PK : t_first;
   // the page size divides the tile of 64 keys: a power of two
-  const int ps_shift = __builtin_ctz(a.page_size), ps_mask = a.page_size - 1, Hkv = a.Hkv;
+  const int ps_shift = FLAT ? 0 : __builtin_ctz(a.page_size), ps_mask = a.page_size - 1, Hkv = a.Hkv;
 
   // this lane's query (B operand): row q = qg * 32 + c, dims 16 ks + 8 j .. +7; the wave
   // meets the 32 NKB keys from 32 NKB kh of every tile
@@ -229,7 +236,7 @@ __global__ __launch_bounds__(NQ * 128, 2) void attn_prefill_kernel(AttnArgs a, i
   const int wave_u = __builtin_amdgcn_readfirstlane(wave);
   const int l_row = lane / CPR, l_pos = lane % CPR;
   auto k_swizzle = [](int row) { return (row / (16 / CPR)) % CPR; };
-  auto v_swizzle = [](int row) { return 4 * ((row / (16 / CPR)) % (CPR / 4)); };
+  auto v_swizzle = [](int row) { return 4 * ((row / (16 / VCPR)) % (VCPR / 4)); };
   // A tile starts at a multiple of the page size, so the place of a lane's row inside its
   // page is the same in every tile: address = pool + page * page_stride + in_page + chunk.
   const int64_t page_stride = ((int64_t)Hkv << ps_shift) * D;
@@ -241,8 +248,32 @@ __global__ __launch_bounds__(NQ * 128, 2) void attn_prefill_kernel(AttnArgs a, i
     k_chunk[i] = 8 * (l_pos ^ k_swizzle(row));
     v_chunk[i] = 8 * (l_pos ^ v_swizzle(row));
   }
+  // Keys in rows of their own: row key_start + position of the keys' own numbers (kdim per head), of the numbers
+  // that all heads share behind them (krot), and of the values. A lane's 16 bytes of a tile's row lie in the
+  // same place of every row: its address is a base of its own plus the key's row times a stride of its own.
+  const bf16* k_from[FLAT ? KPT : 1];
+  const bf16* v_from[FLAT ? VPT : 1];
+  int k_row[FLAT ? KPT : 1], k_step[FLAT ? KPT : 1], v_row[FLAT ? VPT : 1];
+  if constexpr (FLAT) {
+    const int64_t first = a.key_start[seq];
+    const int own = a.kdim, shared = D - a.kdim;
+#pragma unroll
+    for (int i = 0; i < KPT; ++i) {
+      k_row[i] = (i * NW + wave_u) * RPP + l_row;
+      const bool is_own = k_chunk[i] < own;
+      k_step[i] = is_own ? a.kv_stride : shared;
+      k_from[i] = is_own ? (const bf16*)a.kpool + first * a.kv_stride + (int64_t)h * own + k_chunk[i]
+                         : (const bf16*)a.krot + first * shared + (k_chunk[i] - own);
+    }
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) {
+      v_row[i] = (i * NW + wave_u) * VRPP + lane / VCPR;
+      v_from[i] = (const bf16*)a.vpool + first * a.kv_stride + (int64_t)h * DV +
+                  8 * ((lane % VCPR) ^ v_swizzle(v_row[i]));
+    }
+  }
   const int pos_last_u = __builtin_amdgcn_readfirstlane(pos_last);
-  const int64_t last_at =
+  const int64_t last_at = FLAT ? 0 :
       (int64_t)bt[pos_last >> ps_shift] * page_stride + (((int64_t)g << ps_shift) + (pos_last & ps_mask)) * D;
   const int64_t last_at_b = !BLOCKS || blocks_last == 0 ? 0
       : (int64_t)bt_b[(blocks_last - 1) >> ps_shift] * page_stride +
@@ -269,6 +300,7 @@ __global__ __launch_bounds__(NQ * 128, 2) void attn_prefill_kernel(AttnArgs a, i
   const int t_first_u = __builtin_amdgcn_readfirstlane(t_first), t_start_u = __builtin_amdgcn_readfirstlane(t_start);
   int kpage[NST][KPT];
   auto load_pages = [&](int slot, int t0) {
+    if constexpr (FLAT) return;
 #pragma unroll
     for (int i = 0; i < KPT; ++i) {
       const int kp = t0 + (i * NW + wave_u) * RPP;   // the load's first row
@@ -286,6 +318,17 @@ __global__ __launch_bounds__(NQ * 128, 2) void attn_prefill_kernel(AttnArgs a, i
   auto issue_tile = [&](int buf, int slot, int t0) {
     unsigned char* kb = stages + buf * STAGE_BYTES + wave_u * 1024;
     unsigned char* vb = kb + TILE_BYTES;
+    if constexpr (FLAT) {   // (a key behind the last row's: the last row's own)
+#pragma unroll
+      for (int i = 0; i < KPT; ++i)
+        __builtin_amdgcn_global_load_lds((gptr)(k_from[i] + (int64_t)min(t0 + k_row[i], pos_last) * k_step[i]),
+                                         (lptr)(kb + i * (NW * 1024)), 16, 0, 0);
+#pragma unroll
+      for (int i = 0; i < VPT; ++i)
+        __builtin_amdgcn_global_load_lds((gptr)(v_from[i] + (int64_t)min(t0 + v_row[i], pos_last) * a.kv_stride),
+                                         (lptr)(vb + i * (NW * 1024)), 16, 0, 0);
+      return;
+    }
     const bool is_b = BLOCKS && t0 < t_first_u;
     const bf16* kpool = is_b ? (const bf16*)a.kblk : (const bf16*)a.kpool;
     const bf16* vpool = is_b ? (const bf16*)a.vblk : (const bf16*)a.vpool;
@@ -313,7 +356,7 @@ __global__ __launch_bounds__(NQ * 128, 2) void attn_prefill_kernel(AttnArgs a, i
     const int row = 32 * NKB * kh + tr_key;
 #pragma unroll
     for (int db = 0; db < DB; ++db)
-      v_at[db] = TILE_BYTES + row * ROW_BYTES + 16 * ((4 * db + tr_dim / 8) ^ v_swizzle(row)) + 2 * (tr_dim % 8);
+      v_at[db] = TILE_BYTES + row * VROW_BYTES + 16 * ((4 * db + tr_dim / 8) ^ v_swizzle(row)) + 2 * (tr_dim % 8);
   }
   // the products of this wave's part of the tile at keys t0.. in LDS buffer buf
   auto multiply = [&](int buf, int t0) {
@@ -366,8 +409,8 @@ __global__ __launch_bounds__(NQ * 128, 2) void attn_prefill_kernel(AttnArgs a, i
       const unsigned base = (unsigned)(uintptr_t)(lds_short4*)k_s;
 #pragma unroll
       for (int db = 0; db < DB; ++db) {
-        tr_read2<0, 8 * ROW_BYTES>(base + v_at[db], vlo[db][0], vhi[db][0]);
-        tr_read2<16 * ROW_BYTES, 24 * ROW_BYTES>(base + v_at[db], vlo[db][1], vhi[db][1]);
+        tr_read2<0, 8 * VROW_BYTES>(base + v_at[db], vlo[db][0], vhi[db][0]);
+        tr_read2<16 * VROW_BYTES, 24 * VROW_BYTES>(base + v_at[db], vlo[db][1], vhi[db][1]);
       }
     }
     // lane holds, for query c, keys k0 + 32 kb + 8 (v / 4) + 4 j + v % 4
@@ -452,10 +495,10 @@ __global__ __launch_bounds__(NQ * 128, 2) void attn_prefill_kernel(AttnArgs a, i
     }
   };
 
-  // A wave's loads return in the order of their issue. Per tile it issues 2 KPT loads into
+  // A wave's loads return in the order of their issue. Per tile it issues KPT + VPT loads into
   // LDS (and nothing else that the vector memory counter counts); when tile i is needed, the
   // loads issued after its own are those of the NST - 2 tiles after it.
-  constexpr int YOUNGER = (NST - 2) * 2 * KPT;
+  constexpr int YOUNGER = (NST - 2) * (KPT + VPT);
 #pragma unroll
   for (int st = 0; st < NST; ++st) load_pages(st, t_start + st * PK);
 #pragma unroll
@@ -530,9 +573,13 @@ __global__ __launch_bounds__(NQ * 128, 2) void attn_prefill_kernel(AttnArgs a, i
   }
   if (q_valid) {
     // lane holds, of its query's output, dims 32 db + 8 (v / 4) + 4 j + v % 4
-    const float inv = 1.f / l;
-    bf16* orow = (bf16*)a.out + ((int64_t)(row0 + q_local) * a.Hq + h) * D;
-    if (a.gate) {
+    float inv = 1.f / l;
+    bf16* orow = (bf16*)a.out + ((int64_t)(row0 + q_local) * a.Hq + h) * DV;
+    if constexpr (FLAT) {   // the gate: one number a head
+      if (a.gate)
+        inv /= 1.f + __builtin_amdgcn_exp2f(-1.44269504088896f *
+                                            to_f32(((const bf16*)a.gate)[(int64_t)(row0 + q_local) * a.gate_stride + h]));
+    } else if (a.gate) {
       const bf16* grow = (const bf16*)a.gate + (int64_t)(row0 + q_local) * a.gate_stride + h * D;
 #pragma unroll
       for (int db = 0; db < DB; ++db)
@@ -558,10 +605,10 @@ __global__ __launch_bounds__(NQ * 128, 2) void attn_prefill_kernel(AttnArgs a, i
 // LDS of a block beside its stages: tile_info, then the merge's (max, sum) pairs.
 constexpr int kPrefillExtra = 16 + 4 * 64 * 2 * 4;
 
-// Bytes of dynamic LDS of attn_prefill_kernel<D, NQ, .> (as the kernel lays them out).
-static size_t prefill_lds(int D, int nq) {
+// Bytes of dynamic LDS of attn_prefill_kernel<D, NQ, .> with values of DV numbers (as the kernel lays them out).
+static size_t prefill_lds(int D, int DV, int nq) {
   const int stages = nq == 4 ? 3 : 2;
-  return (size_t)stages * 2 * PK * 2 * D + kPrefillExtra;
+  return (size_t)stages * PK * 2 * (D + DV) + kPrefillExtra;
 }
 
 // Pages the matrix-core kernels take: a power of two that divides the tile of 64 keys and
@@ -571,10 +618,10 @@ static bool prefill_page_ok(const AttnArgs& a) {
   return PK % a.page_size == 0 && a.page_size * 2 * a.D >= 1024;
 }
 
-template <int D, int NQ, bool HEADS, bool BLOCKS = false>
+template <int D, int NQ, bool HEADS, bool BLOCKS = false, int FLAT_DV = 0>
 static int launch_attn(const AttnArgs& a, dim3 grid, int chunk, int paired, hipStream_t stream) {
-  auto kern = attn_prefill_kernel<D, NQ, HEADS, BLOCKS>;
-  const size_t lds = prefill_lds(D, NQ);
+  auto kern = attn_prefill_kernel<D, NQ, HEADS, BLOCKS, FLAT_DV>;
+  const size_t lds = prefill_lds(D, FLAT_DV > 0 ? FLAT_DV : D, NQ);
   if (lds > 48 * 1024) {
     hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return set_error(-2, "paged_attention: cannot get %zu bytes of LDS", lds);
@@ -604,7 +651,7 @@ int attention_decode_heads(const AttnArgs& a, int chunk, int n_chunks, hipStream
 }
 
 bool attention_prefill_takes(const AttnArgs& a) {
-  return a.dtype == kBF16 && (a.D == 64 || a.D == 128) && a.q_stride % 8 == 0 &&
+  return a.dtype == kBF16 && (a.D == 64 || a.D == 128) && a.q_stride % 8 == 0 && !a.krot &&
          prefill_page_ok(a) && a.seq_row_start != nullptr && (a.Dv == 0 || a.Dv == a.D) &&
          (!a.kblk || (a.blk_page_size == a.page_size && !a.slopes)) &&
          (!a.gate || (a.gate_stride % 4 == 0 && (uintptr_t)a.gate % 8 == 0));
@@ -618,6 +665,10 @@ template <int NQ>
 static int launch_prefill(const AttnArgs& a, int paired, hipStream_t stream) {
   constexpr int PQ = NQ * 32;
   dim3 grid(prefill_tiles(a, PQ), a.Hq);
+  if (a.krot) {
+    if (a.Dv == 128) return launch_attn<128, NQ, false, false, 128>(a, grid, 0, paired, stream);
+    return launch_attn<128, NQ, false, false, 64>(a, grid, 0, paired, stream);
+  }
   if (a.kblk) {
     if (a.D == 128) return launch_attn<128, NQ, false, true>(a, grid, 0, paired, stream);
     return launch_attn<64, NQ, false, true>(a, grid, 0, paired, stream);

@@ -196,7 +196,8 @@ class ModelRunner:
         host = torch.from_numpy(np.concatenate(parts))
         shape = dict(T=T, S=S, sizes=sizes, widths=[t.shape[1] for t in tables],
                      max_qlen=int(qlen.max()), max_kv_len=max_kv_len, wants=bool(want_rows),
-                     single_rows=single_rows)
+                     single_rows=single_rows,
+                     portion_keys=sum(p + len(c.tokens) for c, p in zip(chunks[single_rows:], pos0[single_rows:])))
         if graph:
             logits = self._step_graph(host, shape)
         else:
@@ -280,7 +281,8 @@ class ModelRunner:
             tokens=views[0], positions=views[1], row_seq=views[2], seq_slots=views[3],
             seq_row_start=views[4], seq_qlen=views[5], seq_pos0=views[6],
             max_qlen=shape["max_qlen"], max_kv_len=shape["max_kv_len"],
-            all_decode=shape["max_qlen"] == 1, single_rows=shape["single_rows"])
+            all_decode=shape["max_qlen"] == 1, single_rows=shape["single_rows"],
+            portion_keys=shape["portion_keys"])
         es = self.cache.state[:, self._embedding_state] if self._embedding_state is not None else None
         return self.spec.forward(ctx, self._call_infos(d_tables),
                                  views[7] if shape["wants"] else None, es, self.tap)

@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import ctypes
 import weakref
+from dataclasses import replace
 from typing import Optional
 
 import torch
@@ -54,6 +55,15 @@ class _RouteArgs(ctypes.Structure):
                 ("renorm_eps", ctypes.c_float), ("weightless", ctypes.c_int)]
 
 
+# Prompts over a cached latent form keys and values per head where the cached rows to form them from are no more
+# than LATENT_HEADS_FEW, or than LATENT_HEADS_RATIO times the rows that read them, and LATENT_HEADS_KEYS at most (7 KB
+# a row at 16 heads of 64 + 128 numbers; the other form keeps 52 KB per row of the step). us in the latent's space
+# and so, 16 heads of 512 + 64 numbers: 2,048 tokens 178 and 61, 512 61 and 26, 16 25 and 12; 512 after 4,096 cached 277
+# and 90; 64 after 512 44 and 27, after 2,000 53 and 59; 16 after 1,000 40 and 35. 8 heads of 256 + 32: 2,048 115 and 42,
+# 512 after 7,500 126 and 112, 128 after 2,000 39 and 41, 16 after 1,000 23 and 26.
+LATENT_HEADS_KEYS = 16384
+LATENT_HEADS_FEW = 512
+LATENT_HEADS_RATIO = 16
 BIG_TILE_ROWS = 256   # rows of a tall tile of the grouped products (the library's kGroupedTileRows)
 ROUTE_ROWS_PER_BLOCK = 1024  # the library's kAlignRowsPerBlock
 # rows (tokens) from which the grouping runs as several blocks side by side: 12.5 against 13 us
@@ -85,7 +95,8 @@ class _AttnArgs(ctypes.Structure):
                 ("kblk", ctypes.c_void_p), ("vblk", ctypes.c_void_p), ("blk_table", ctypes.c_void_p),
                 ("blk_bt_stride", ctypes.c_int), ("blk_page_size", ctypes.c_int),
                 ("block", ctypes.c_int), ("gate", ctypes.c_void_p), ("gate_stride", ctypes.c_int),
-                ("sinks", ctypes.c_void_p)]
+                ("sinks", ctypes.c_void_p), ("krot", ctypes.c_void_p), ("key_start", ctypes.c_void_p),
+                ("kv_stride", ctypes.c_int), ("kdim", ctypes.c_int)]
 
 
 class _QkvWideArgs(ctypes.Structure):
@@ -197,7 +208,13 @@ class _LatentArgs(ctypes.Structure):
                 ("rd", ctypes.c_int), ("rot_n", ctypes.c_int), ("page_size", ctypes.c_int),
                 ("window", ctypes.c_int), ("write_kv", ctypes.c_int), ("dtype", ctypes.c_int),
                 ("eps", ctypes.c_float), ("magnitude", ctypes.c_float), ("scale", ctypes.c_float),
-                ("interleaved", ctypes.c_int)]
+                ("interleaved", ctypes.c_int), ("abs_rows", ctypes.c_int)]
+
+
+class _LatentHeadsArgs(ctypes.Structure):
+    _fields_ = [("latent", ctypes.c_void_p), ("krot", ctypes.c_void_p), ("key_start", ctypes.c_void_p),
+                ("kv", ctypes.c_void_p), ("q", ctypes.c_void_p), ("out", ctypes.c_void_p),
+                ("seq_qlen", ctypes.c_void_p), ("keys", ctypes.c_int), ("vdim", ctypes.c_int)]
 
 
 class _DiffAttnArgs(ctypes.Structure):
@@ -1577,14 +1594,15 @@ class HipOps:
 
     def latent_kv_write(self, dkv, q, q_abs, pool, block_table, ctx, heads, dim, rank, rot_dim,
                         norm_w, eps, freq, rot_n, magnitude, page_size, write_kv=True,
-                        interleaved=False):
+                        interleaved=False, abs_rows=None):
         """Per row: the first `rank` columns of `dkv` normed (x rsqrt(mean(x^2) + eps) norm_w)
         and the next `rot_dim`, turned by the row's position, go to the request's page of
         `pool` [pages, page_size, rank + rot_dim]; the rotated part of every head of `q`
         ([T, heads * (dim + rot_dim)]) is turned and written behind the first `rank` numbers of
         the head's row of `q_abs` [T, heads, rank + rot_dim] (32-bit). Pair (i, i + rot_n / 2)
         (with `interleaved`: pair (2i, 2i + 1)) of the first rot_n rotated numbers turns by
-        pos * freq[i]; cos and sin times `magnitude`."""
+        pos * freq[i]; cos and sin times `magnitude`. With `abs_rows` q_abs holds only the first
+        so many rows, and the rotated parts of the rows behind them are turned in `q` itself."""
         _need(dkv.is_cuda and dkv.dim() == 2 and dkv.stride(1) == 1 and dkv.shape[1] >= rank + rot_dim,
               "latent_kv_write: dkv must be rows of at least rank + rot_dim columns")
         _dev(q, "q", dkv.dtype, 2)
@@ -1592,8 +1610,8 @@ class HipOps:
         _dev(norm_w, "norm_w", torch.float32, 1)
         t = ctx.T
         _need(dkv.shape[0] == t and q.shape == (t, heads * (dim + rot_dim))
-              and q_abs.shape == (t, heads, rank + rot_dim) and norm_w.shape[0] == rank,
-              "latent_kv_write: shapes")
+              and q_abs.shape == (t if abs_rows is None else abs_rows, heads, rank + rot_dim)
+              and q_abs.shape[0] <= t and norm_w.shape[0] == rank, "latent_kv_write: shapes")
         a = self._latent_args(ctx, pool, block_table, heads, dim, rank, rot_dim, rot_n, page_size,
                               dkv.dtype)
         if rot_n:
@@ -1603,7 +1621,7 @@ class HipOps:
         a.dkv, a.q, a.q_abs, a.norm_w = dkv.data_ptr(), q.data_ptr(), q_abs.data_ptr(), norm_w.data_ptr()
         a.dkv_stride = dkv.stride(0) if t > 1 else max(dkv.shape[1], dkv.stride(0))
         a.eps, a.magnitude, a.scale, a.write_kv = eps, magnitude, 1.0, 1 if write_kv else 0
-        a.interleaved = 1 if interleaved else 0
+        a.interleaved, a.abs_rows = 1 if interleaved else 0, q_abs.shape[0]
         self._ok(self.lib.ninfer_latent_kv_write(ctypes.byref(a), self._stream()))
 
     def latent_attention(self, q_abs, pool, block_table, ctx, heads, rank, rot_dim, page_size,
@@ -1631,6 +1649,74 @@ class HipOps:
             ws = self._workspace(need, q_abs.device)
             a.workspace, a.workspace_floats = ws.data_ptr(), ws.numel()
         self._ok(self.lib.ninfer_latent_attention(ctypes.byref(a), self._stream()))
+
+    def latent_heads_rows(self, ctx, heads, dim, rank, rot_dim, vdim, window) -> int:
+        """The first of the step's rows whose prompts had better attend with keys and values formed
+        per head (`latent_heads_attention`); ctx.T: none. These are the rows behind the single ones, where
+        the sizes have such a kernel and the cached rows to form keys and values from are few beside
+        the rows that read them."""
+        portion = ctx.T - ctx.single_rows
+        if (portion <= 0 or not 0 < ctx.portion_keys <= min(LATENT_HEADS_KEYS, max(LATENT_HEADS_FEW, LATENT_HEADS_RATIO * portion))
+                or ctx.act_dtype != torch.bfloat16 or window or self.force_generic or self.conv_pieces_always):
+            return ctx.T
+        a = _LatentArgs()
+        a.seq_row_start = a.seq_pos0 = 1   # (asked for the sizes alone; they are there)
+        a.S, a.dim, a.rd, a.R, a.dtype = 1, dim, rot_dim, rank, _DT[ctx.act_dtype]
+        return ctx.single_rows if self.lib.ninfer_latent_heads_takes(ctypes.byref(a), vdim) else ctx.T
+
+    def latent_heads_attention(self, q, pool, block_table, ctx, heads, dim, rank, rot_dim, vdim, page_size, scale,
+                               w_kv, out, gate=None):
+        """Softmax attention of the prompts behind a step's single rows, rows q [T, heads * (dim + rot_dim)]
+        (turned), over the cached rows [c | r] of `pool`: keys [w_k c | r] and values w_v c of every head are
+        formed first, with w_kv [heads * dim + heads * vdim, rank] (w_k of all heads, then w_v). Writes
+        the rows' heads of `out` [T, heads * vdim], times sigmoid(gate[t, h]) when `gate` [T, heads] is given."""
+        n, dt = ctx.single_rows, pool.dtype
+        keys = ctx.portion_keys
+        _dev(q, "q", dt, 2)
+        _dev(out, "out", dt, 2)
+        _dev(w_kv, "w_kv", dt, 2)
+        _need(0 <= n < ctx.S and keys >= ctx.T - n and q.shape == (ctx.T, heads * (dim + rot_dim))
+              and out.shape == (ctx.T, heads * vdim) and w_kv.shape == (heads * (dim + vdim), rank),
+              "latent_heads_attention: shapes")
+        p = self._portion(ctx)
+        a = self._latent_args(p, pool, block_table[n:], heads, dim, rank, rot_dim, 0, page_size, dt)
+        a.scale = scale
+        if gate is not None:
+            _need(gate.is_cuda and gate.dtype == dt and gate.shape == (ctx.T, heads)
+                  and gate.stride(1) == 1, "latent_heads_attention: the gate must be [T, heads] columns")
+            a.gate, a.gate_stride = gate.data_ptr(), gate.stride(0) if ctx.T > 1 else max(heads, gate.stride(0))
+        b = _LatentHeadsArgs()
+        latent = torch.empty((keys, rank), dtype=dt, device=q.device)
+        krot = torch.empty((keys, rot_dim), dtype=dt, device=q.device)
+        start = torch.empty(p.S, dtype=torch.int32, device=q.device)
+        kv = torch.empty((keys, heads * (dim + vdim)), dtype=dt, device=q.device)
+        b.latent, b.krot, b.key_start, b.kv = latent.data_ptr(), krot.data_ptr(), start.data_ptr(), kv.data_ptr()
+        b.q, b.out, b.seq_qlen, b.keys, b.vdim = q.data_ptr(), out.data_ptr(), p.seq_qlen.data_ptr(), keys, vdim
+        self._ok(self.lib.ninfer_latent_rows(ctypes.byref(a), ctypes.byref(b), self._stream()))
+        self.linear(latent, w_kv, kv)
+        self._ok(self.lib.ninfer_latent_heads_attention(ctypes.byref(a), ctypes.byref(b), self._stream()))
+
+    def _portion(self, ctx):
+        """The step without its single rows, which come first: its requests (rows and positions stay
+        where they are). Made once per step and kept in its scratch."""
+        n = ctx.single_rows
+        if n == 0:
+            return ctx
+        if "portion" not in ctx.scratch:
+            ctx.scratch["portion"] = replace(
+                ctx, T=ctx.T - n, S=ctx.S - n, seq_slots=ctx.seq_slots[n:], seq_row_start=ctx.seq_row_start[n:],
+                seq_qlen=ctx.seq_qlen[n:], seq_pos0=ctx.seq_pos0[n:], single_rows=0, scratch={})
+        return ctx.scratch["portion"]
+
+    def singles(self, ctx):
+        """The step of its single rows alone, made once per step like `_portion`."""
+        n = ctx.single_rows
+        if "singles" not in ctx.scratch:
+            ctx.scratch["singles"] = replace(
+                ctx, T=n, S=n, tokens=ctx.tokens[:n], positions=ctx.positions[:n], row_seq=ctx.row_seq[:n],
+                seq_slots=ctx.seq_slots[:n], seq_row_start=ctx.seq_row_start[:n + 1], seq_qlen=ctx.seq_qlen[:n],
+                seq_pos0=ctx.seq_pos0[:n], max_qlen=1, all_decode=True, portion_keys=0, scratch={})
+        return ctx.scratch["singles"]
 
     def _workspace(self, floats: int, device) -> torch.Tensor:
         """The attention kernels' 32-bit scratch, grown when a step needs more. A captured graph

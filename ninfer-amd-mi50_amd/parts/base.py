@@ -134,6 +134,7 @@ class StepContext:
     max_kv_len: int = 1
     all_decode: bool = False
     single_rows: int = 0          # the first single_rows requests bring one row each (rows 0 ..)
+    portion_keys: int = 0         # cached positions of the requests behind them, this step's included (0: not said)
     scratch: Dict[str, Any] = field(default_factory=dict)
 
     def empty(self, shape, dtype=None) -> torch.Tensor:

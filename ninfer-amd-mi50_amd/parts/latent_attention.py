@@ -7,11 +7,13 @@
     y = W_o concat_h( sigmoid(W_g h)_h * sum_j p_j v_h,j )
 
 Only c and turn(r) are cached, one row of kv_rank + rot_dim numbers per token for all heads
-(pool 'latent'). The heads' keys and values are never formed: the query goes into the
+(pool 'latent'). In decode steps the heads' keys and values are never formed: the query goes into the
 latent's space, q'_h = W_uk,h^T q_unrot (a product per head), the attention kernel scores
 q' and the rotated part against the cached rows and sums the latents, and the head's value
 is W_uv,h applied to that sum (another product per head). The gate, one number per head and
-row, scales the head's output in the attention kernel. `position` turns the first
+row, scales the head's output in the attention kernel. Prompts whose rows are many beside their cached
+ones have the keys and values formed (one product over the cached rows) and attend with those:
+dim + rot_dim and vdim numbers a head and key instead of kv_rank + rot_dim and kv_rank. `position` turns the first
 `position.rot_dim` of the rot_dim rotated numbers (half-split pairs or neighbours, as its
 `pairing` says) with its table and magnitude. Norm, angles, scores and softmax are 32-bit;
 q' is kept in 32-bit. With `q_rank` the queries pass a latent of their own first:
@@ -63,6 +65,7 @@ class LatentAttention(Mixer):
         self.w_q: Optional[torch.Tensor] = None
         self.w_dkv_g: Optional[torch.Tensor] = None   # W_dkv, then W_g
         self.norm_w: Optional[torch.Tensor] = None
+        self.w_kv: Optional[torch.Tensor] = None      # W_uk, then W_uv
         self.w_absorb: Optional[torch.Tensor] = None  # [heads, kv_rank, dim]: W_uk,h transposed
         self.w_uv: Optional[torch.Tensor] = None      # [heads, vdim, kv_rank]
         self.w_o: Optional[torch.Tensor] = None
@@ -110,10 +113,14 @@ class LatentAttention(Mixer):
         if self.output_gate:
             w.matrix_into(p + n[5], self.w_dkv_g[lat:])
         self.norm_w = w.float32(p + n[2])
-        uk = w.matrix(p + n[3])
+        self.w_kv = torch.empty((self.heads * (self.dim + self.vdim), self.kv_rank), dtype=w.act_dtype,
+                                device=w.device)
+        uk, uv = self.w_kv[:self.heads * self.dim], self.w_kv[self.heads * self.dim:]
+        w.matrix_into(p + n[3], uk)
+        w.matrix_into(p + n[4], uv)
         # q'_h = W_uk,h^T q: as a product x w^T, w is W_uk,h transposed, [kv_rank, dim]
         self.w_absorb = uk.view(self.heads, self.dim, self.kv_rank).transpose(1, 2).contiguous()
-        self.w_uv = w.matrix(p + n[4]).view(self.heads, self.vdim, self.kv_rank)
+        self.w_uv = uv.view(self.heads, self.vdim, self.kv_rank)
         self.w_o = w.matrix(p + n[6])
 
     def forward(self, ctx: StepContext, x, residual, call: CallInfo):
@@ -135,20 +142,32 @@ class LatentAttention(Mixer):
             cq = ctx.empty((T, self.q_rank))
             ops.rmsnorm(cq32, self.q_norm_w, self.eps, cq)
             ops.linear(cq, self.w_q, q)
-        q_abs = ctx.empty((T, H, R + rd), torch.float32)
+        # the rows before `first` attend in the latent's space, those from there on with keys and
+        # values per head
+        first = T
+        if ctx.portion_keys and x.is_cuda:
+            first = ops.latent_heads_rows(ctx, H, self.dim, R, rd, self.vdim, self.window)
+        q_abs = ctx.empty((first, H, R + rd), torch.float32)
+        extra = {} if first == T else {"abs_rows": first}
         ops.latent_kv_write(dkv_g, q, q_abs, cache["latent"], cache.block_table, ctx, H, self.dim,
                             R, rd, self.norm_w, self.eps, self.position.table(),
                             self.position.rot_dim, getattr(self.position, "magnitude", 1.0),
                             cache.page_size, write_kv=call.writes_cache,
-                            interleaved=self.position.pairing == "interleaved")
-        ops.per_head_linear(q.view(T, H, self.dim + rd), self.w_absorb, q_abs, ctx, self.dim, R)
-        mixed = ctx.empty((T, H * R))
-        ops.latent_attention(q_abs, cache["latent"], cache.block_table, ctx, H, R, rd,
-                             cache.page_size, self.scale, mixed,
-                             gate=dkv_g[:, R + rd:] if self.output_gate else None,
-                             window=self.window)
+                            interleaved=self.position.pairing == "interleaved", **extra)
+        gate = dkv_g[:, R + rd:] if self.output_gate else None
         heads_out = ctx.empty((T, H, self.vdim))
-        ops.per_head_linear(mixed.view(T, H, R), self.w_uv, heads_out, ctx, R, self.vdim)
+        if first < T:
+            ops.latent_heads_attention(q, cache["latent"], cache.block_table, ctx, H, self.dim, R, rd, self.vdim,
+                                       cache.page_size, self.scale, self.w_kv, heads_out.view(T, H * self.vdim),
+                                       gate=gate)
+        if first:
+            sub = ctx if first == T else ops.singles(ctx)
+            ops.per_head_linear(q[:first].view(first, H, self.dim + rd), self.w_absorb, q_abs, sub, self.dim, R)
+            mixed = ctx.empty((first, H * R))
+            ops.latent_attention(q_abs, cache["latent"], cache.block_table[:sub.S], sub, H, R, rd,
+                                 cache.page_size, self.scale, mixed,
+                                 gate=gate[:first] if gate is not None else None, window=self.window)
+            ops.per_head_linear(mixed.view(first, H, R), self.w_uv, heads_out[:first], sub, R, self.vdim)
         out = ctx.empty((T, self.hidden))
         ops.linear(heads_out.view(T, H * self.vdim), self.w_o, out)
         return out

@@ -444,6 +444,46 @@ def test_latent_pages_that_the_table_does_not_hold(ops, rank, rd, heads, new_row
     assert rel_err(out.float().cpu().reshape(ctx.T, heads, rank), want) < 8e-3
 
 
+@pytest.mark.parametrize("heads,rank,rd,vdim", [(16, 512, 64, 128), (8, 256, 32, 64), (3, 72, 64, 128), (1, 128, 120, 64)])
+@pytest.mark.parametrize("ps,lengths,new_rows", [
+    (16, [700], [700]),                                   # one prompt
+    (16, [40, 17, 2], [40, 17, 2]),                       # parts of a tile
+    (8, [65, 300, 129, 64], [1, 300, 2, 63]),             # a single row first, keys of earlier steps
+    (4, [33, 1, 1025], [1, 1, 900]),                      # two single rows
+    (3, [80, 192], [70, 191]),                            # pages of any size
+    (16, [31] * 70, [1] * 3 + [31] * 67)])                # more requests than lanes
+def test_latent_attention_with_keys_and_values_per_head(ops, heads, rank, rd, vdim, ps, lengths, new_rows):
+    """The prompts behind a step's single rows against the softmax over W_uk c, r and W_uv c written out: keys, values,
+    probabilities and outputs are rounded to bfloat16 once each (2^-9 of their size: 8e-3 for the four)."""
+    g = torch.Generator().manual_seed(heads)
+    dim = 128 - rd
+    ctx, pool, table, q, cached = _latent_case(ops, torch.bfloat16, heads, rank, rd, ps, lengths, new_rows, seed=rank)
+    n = sum(1 for m in new_rows if m == 1)
+    ctx.single_rows, ctx.portion_keys = n, sum(lengths[n:])
+    assert ops.latent_heads_rows(ctx, heads, dim, rank, rd, vdim, None) in (n, ctx.T)
+    if lengths == [700]:
+        table[0, 3], cached[0][3 * ps:4 * ps] = -1, 0     # a page that the table does not hold: zeros
+    q = torch.randn(ctx.T, heads * 128, generator=g).bfloat16()
+    w = (torch.randn(heads * (dim + vdim), rank, generator=g) * rank ** -0.5).bfloat16()
+    gate = torch.randn(ctx.T, heads + 5, generator=g).bfloat16()
+    out = torch.full((ctx.T, heads * vdim), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops.latent_heads_attention(q.to(DEV), pool.bfloat16().to(DEV), table.to(DEV), ctx, heads, dim, rank, rd, vdim, ps,
+                               0.1, w.to(DEV), out, gate=gate.to(DEV)[:, 5:])
+    got = out.double().cpu().view(ctx.T, heads, vdim)
+    assert (got[:n] == 7.0).all()                         # the single rows are the other form's
+    wk, wv = w[:heads * dim].double().view(heads, dim, rank), w[heads * dim:].double().view(heads, vdim, rank)
+    r = n
+    for rows, total, m in list(zip(cached, lengths, new_rows))[n:]:
+        c = rows[:, :rank].double()
+        k = torch.cat([torch.einsum("hdr,jr->hjd", wk, c), rows[:, rank:].double().expand(heads, -1, -1)], -1)
+        s = torch.einsum("thd,hjd->htj", q[r:r + m].double().view(m, heads, 128), k) * 0.1
+        s.masked_fill_(torch.arange(total)[None, :] > torch.arange(total - m, total)[:, None], float("-inf"))
+        want = torch.einsum("htj,hjv->thv", torch.softmax(s, -1), torch.einsum("hvr,jr->hjv", wv, c))
+        want *= torch.sigmoid(gate[r:r + m, 5:].double())[..., None]
+        assert rel_err(got[r:r + m], want) < 8e-3
+        r += m
+
+
 @pytest.mark.parametrize("rank,rd", [(256, 32), (512, 64), (512, 128)])
 @pytest.mark.parametrize("ps,lengths,new_rows", [(16, [720, 333], [720, 300]), (4, [700], [600]), (64, [2040, 200], [60, 131])])
 def test_latent_pages_that_the_table_does_not_hold_in_blocks_of_64_rows(ops, rank, rd, ps, lengths, new_rows):
