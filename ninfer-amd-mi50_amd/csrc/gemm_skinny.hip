@@ -578,7 +578,7 @@ bool gemm_skinny_route_pair_takes(const GemmArgs& a, const GemmArgs& b, const Ro
 
 int gemm_skinny_route_pair(const GemmArgs& a, const GemmArgs& b, const RouteArgs& rt,
                            hipStream_t stream) {
-  const SkinnyPlan pb = plan_skinny(b);
+  SkinnyPlan pb = plan_skinny(b);
   // The router's block has work for 16 waves and is the launch's longest beside a short
   // dense product. But a block of 16 waves is alone on its CU, and the dense product's blocks
   // then follow each other with nothing overlapping their starts and ends (they stream at 5.5
@@ -591,6 +591,14 @@ int gemm_skinny_route_pair(const GemmArgs& a, const GemmArgs& b, const RouteArgs
   static_assert(16 * kRouteMaxFeatures * 4 + (kRouteMaxFeatures + 1) * 4 + 16 * 64 * 4 <= 8 * 2048,
                 "the routing block's LDS (8 waves' stage at least)");
   static_assert((kRouteMaxFeatures + 15) / 16 <= 8, "a wave's two feature groups x 8 waves hold them");
+  // Blocks of 16 waves stand two to a CU. Where the dense product's alone take every place, the router's would
+  // make the launch's last block start when the first ones end, 4 us behind them (one row of 2,048, 2 x 5,632
+  // features: 13.8 us to the last block's end, of which 9.6 to its start): a feature more to a block makes room.
+  const long places = 2L * device_cu_count();
+  if (threads == 1024 && pb.grid_y == 1 && pb.grid_x % places == 0 && pb.rows < 16) {
+    pb.rows = (int)((b.N + pb.grid_x - 2) / (pb.grid_x - 1));
+    pb.grid_x = (b.N + pb.rows - 1) / pb.rows;
+  }
   const long blocks = 1 + (long)pb.grid_x * pb.grid_y;
   NINFER_REQUIRE(blocks < (1L << 31), "gemm pair: %ld blocks are too many", blocks);
   gemm_skinny_route_pair_kernel<false, true, bf16>
