@@ -398,7 +398,7 @@ class HipOps:
         self.lightning_chunk_min_rows = 8   # a step's longest portion from which lightning attention runs in chunks
         self.library_min_rows = 32  # dense bf16 products with more rows go to the library
         self.rows_kernel_max = 64   # ... unless the kernel for 33 to 64 rows takes them
-        self.rows_kernel_features = (4096, 32768)   # (gemm_skinny_rows.hip: where it beats the library)
+        self.rows_kernel_features = (4096, 32768)   # (there no call of the library's, whatever the rows)
         # ... but never a SwiGLU's gate/up product: the tile kernels here have the activation in
         # their epilogue, which beats the library's product followed by a kernel for the
         # activation at every row count (70 against 98 us at 64 rows of 40960 x 3584; whole
@@ -824,10 +824,14 @@ class HipOps:
         if act is None and self._use_library(x, out, w) and bias is None and not (
                 x.shape[0] <= self.side_own_max_rows
                 and w.numel() * w.element_size() <= self.side_own_max_bytes and self._on_side()):
-            if x.shape[0] > self.split_max_rows or not self._gemm(
-                    x, w, out, m=x.shape[0], n=w.shape[0], k=x.shape[1], only_if_split=True):
-                torch.matmul(x, w.t(), out=out)
-            return
+            own = self._rows_kernel_takes(x, w)
+            if not own or self._tune["split_min_bytes"]:
+                if x.shape[0] <= self.split_max_rows and self._gemm(
+                        x, w, out, m=x.shape[0], n=w.shape[0], k=x.shape[1], only_if_split=True):
+                    return
+                if not own:
+                    torch.matmul(x, w.t(), out=out)
+                    return
         self._gemm(x, w, out, m=x.shape[0], n=w.shape[0], k=x.shape[1], bias=bias,
                    epilogue=UNGATED_ACTS[act])
 
@@ -844,6 +848,16 @@ class HipOps:
                 and self.rows_kernel_features[0] <= w.shape[0] <= self.rows_kernel_features[1]:
             return False
         return rows > self.library_min_rows
+
+    @staticmethod
+    def _rows_kernel_takes(x, w) -> bool:
+        """Plain dense products of 33 to 512 rows that the kernel for them runs faster than the library
+        (gemm_skinny_rows.hip), and for the host: a launch costs it 3 us and the library's call 18. Not
+        weights of 48 MB and more, which gain by a cut along K, or by the library's taller tiles."""
+        rows, (n, k) = x.shape[0], w.shape
+        return (rows <= 512 and n > 128 and k % 128 == 0
+                and n * -(-rows // 32) <= (16384 if rows <= 128 else 8192) and n * k < (24 << 20)
+                and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
     @staticmethod
     def _gate_epilogue(act: str) -> int:

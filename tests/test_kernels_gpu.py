@@ -224,6 +224,53 @@ def test_linear_of_33_to_64_rows(ops, gen, m, n, k):
         ops.force_generic = saved
 
 
+@pytest.mark.parametrize("m,n,k,gated", [
+    (17, 2561, 128, False), (32, 6144, 2048, False), (31, 2049, 384, True),      # one row part
+    (33, 129, 2048, False), (64, 2048, 5632, False), (63, 8191, 256, False), (64, 6144, 2048, True),
+    (65, 5461, 128, False), (80, 2048, 2048, False), (96, 1000, 1152, True),     # three row parts on an XCD's places
+    (128, 4096, 1024, False), (128, 3072, 128, True), (129, 1638, 768, False), (300, 300, 2048, False),
+    (512, 512, 128, False), (512, 768, 256, True)])
+def test_products_in_blocks_of_32_rows(ops, gen, m, n, k, gated):
+    """Dense bf16 products whose blocks own 32 rows and up to 32 rows of the weights: sizes at the edges of its range,
+    the last block's features and rows partly there, K of fewer chunks than waves; every epilogue and both
+    outputs against the plain product, nothing written beyond the rows and columns."""
+    x, w = rnd((m, k), torch.bfloat16, gen), rnd((n * (2 if gated else 1), k), torch.bfloat16, gen)
+    bias = torch.randn(w.shape[0], generator=gen, device="cuda")
+    args = _gemm_args(m, n, k, 1 if gated else 0)
+    assert ops.lib.ninfer_gemm_kernel(ctypes.byref(args)) == 3
+    saved, ops.force_generic = ops.force_generic, False
+    try:
+        for out_dtype in (torch.bfloat16, torch.float32):
+            for b in (None, bias):
+                whole = torch.full((m + 1, n), 7.0, device="cuda", dtype=out_dtype)
+                want = torch.empty(m, n, device="cuda", dtype=out_dtype)
+                if not gated:
+                    for act in (None, "relu2"):
+                        ops._gemm(x, w, whole, m=m, n=n, k=k, bias=b, epilogue=3 if act else 0)
+                        PlainOps().linear(x, w, want, bias=b, act=act)
+                        close(whole[:m], want, out_dtype, scale=math.sqrt(k) * (k ** 0.5 if act else 1))
+                        if act is None and b is None and out_dtype == torch.bfloat16:
+                            other = torch.empty_like(want)
+                            ops.linear(x, w, other)   # the same kernel or the library's
+                            close(other, want, out_dtype, scale=math.sqrt(k))
+                elif out_dtype == torch.bfloat16:
+                    for act in ("silu", "gelu_pytorch_tanh"):
+                        ops.swiglu_linear(x, w, whole[:m], act=act, bias=b)
+                        PlainOps().swiglu_linear(x, w, want, act=act, bias=b)
+                        close(whole[:m], want, out_dtype, scale=k * 0.2)
+                assert bool((whole[m] == 7.0).all())
+    finally:
+        ops.force_generic = saved
+
+
+def _gemm_args(m, n, k, epilogue):
+    from ninfer_amd.kernels.ops import _GemmArgs
+    a = _GemmArgs(4096, 4096, 4096)
+    a.M, a.N, a.K, a.lda, a.ldc, a.groups, a.a_div, a.in_dtype, a.out_dtype, a.epilogue = \
+        m, n, k, k, n, 1, 1, 1, 1, epilogue
+    return a
+
+
 @pytest.mark.parametrize("m", [17, 32])
 def test_linear_with_very_large_weights_at_17_to_32_rows(ops, gen, m):
     """A plain product of 17 to 32 rows against weights that no cache holds (an output head of
