@@ -14,7 +14,9 @@
 // heads that share the kv head, so keys and values are read once for all of
 // them. Lane groups, then waves, are merged by the usual log-sum-exp rule and
 // the chunk's (m, l, acc) goes to the workspace.
-// Pass 2, grid (rows, query heads): merges the chunks of a row in a fixed order.
+// Pass 2, grid (rows, query heads): merges the chunks of a row in a fixed order; a sink of the softmax is one more
+// chunk there, and a gate on the output its last factor (16 query heads on 4 of 128 numbers, us in the kernels of
+// attention_tiles.hip and here: 64 rows in a window of 1,024 keys 48 and 35, 8 rows 19 and 13, 1 row 16 and 10).
 // With three or more query heads per kv head (and heads of 64 or 128), pass 1 is the
 // matrix-core kernel of attention_prefill.hip with the heads of a kv head as its rows;
 // it writes the same (m, l, acc) per chunk, and pass 2 is the same.
@@ -238,7 +240,9 @@ __global__ __launch_bounds__(kMergeThreads) void attn_decode_merge_kernel(AttnAr
   mx = wave_max(mx);
   if ((tid & 63) == 0) red[tid >> 6] = mx;
   __syncthreads();
-  float M = red[0];
+  // (a sink is one more chunk, of sum 1 and no output)
+  const float sink = a.sink ? attention_sink(a, h) : -INFINITY;
+  float M = fmaxf(red[0], sink);
 #pragma unroll
   for (int w = 1; w < kMergeThreads / 64; ++w) M = fmaxf(M, red[w]);
   float lsum = 0.f;
@@ -250,7 +254,7 @@ __global__ __launch_bounds__(kMergeThreads) void attn_decode_merge_kernel(AttnAr
   lsum = wave_sum(lsum);
   if ((tid & 63) == 0) red[kMergeThreads / 64 + (tid >> 6)] = lsum;
   __syncthreads();
-  float total = 0.f;
+  float total = a.sink ? __expf(sink - M) : 0.f;
 #pragma unroll
   for (int w = 0; w < kMergeThreads / 64; ++w) total += red[kMergeThreads / 64 + w];
   const int parts = kMergeThreads / D;          // D <= 256: at least 2
@@ -265,7 +269,9 @@ __global__ __launch_bounds__(kMergeThreads) void attn_decode_merge_kernel(AttnAr
   if (tid < D) {
     float sum = 0.f;
     for (int p = 0; p < parts; ++p) sum += part_s[p * D + tid];
-    ((bf16*)a.out)[((int64_t)t * a.Hq + h) * D + tid] = __float2bfloat16(sum / total);
+    sum /= total;
+    if (a.gate) sum *= sigmoid_for<bf16>(to_f32(((const bf16*)a.gate)[(int64_t)t * a.gate_stride + h * D + tid]));
+    ((bf16*)a.out)[((int64_t)t * a.Hq + h) * D + tid] = __float2bfloat16(sum);
   }
 }
 
@@ -279,7 +285,12 @@ bool attention_decode_takes(const AttnArgs& a) {
   bool d_ok = d == 16 || d == 32 || d == 64 || d == 128 || d == 256;
   bool ps_ok = (a.page_size & (a.page_size - 1)) == 0;
   return a.dtype == kBF16 && d_ok && ps_ok && a.q_stride % 8 == 0 && a.workspace != nullptr &&
-         (a.Dv == 0 || a.Dv == a.D) && !a.sink && !a.kblk && !a.gate;
+         (a.Dv == 0 || a.Dv == a.D) && !a.kblk &&
+         // (a sink and a gate on the output: the merge's. What does not fit its workspace goes to the kernels of
+         // attention_tiles.hip, which cut the keys into as many chunks as fit)
+         ((!a.sink && !a.gate) ||
+          (a.workspace_floats >= attention_decode_workspace_floats(a.T, a.Hq, a.D, a.max_kv_len) &&
+           a.max_kv_len < (1 << 19)));
 }
 
 template <int LPK, int CHUNK>
@@ -311,10 +322,11 @@ void attention_decode_plan(const AttnArgs& a, bool* heads, int* chunk, int* n_ch
   *chunk = decode_chunk(a.T, a.Hkv, a.max_kv_len);
   if (*heads) {
     // the matrix-core kernel has a start-up of several tiles: the largest chunk that still
-    // gives every CU two blocks
+    // gives the CUs one and a half blocks (of two places each; 4 kv heads of 128, 16 rows at 1,500 keys:
+    // 384 blocks of 256 keys 16.0 us, 768 of 128 19.7; 32 rows at 1,200: 384 of 512 21.5, 640 of 256 23.7)
     *chunk = 128;
     for (int c = 1024; c > 128; c /= 2)
-      if ((long)a.T * a.Hkv * ((a.max_kv_len + c - 1) / c) >= 2L * device_cu_count()) {
+      if (2L * a.T * a.Hkv * ((a.max_kv_len + c - 1) / c) >= 3L * device_cu_count()) {
         *chunk = c;
         break;
       }

@@ -636,7 +636,7 @@ bool attention_decode_heads_takes(const AttnArgs& a) {
   const int group = a.Hq / a.Hkv;
   return a.dtype == kBF16 && (a.D == 64 || a.D == 128) && a.q_stride % 8 == 0 &&
          prefill_page_ok(a) && group >= 3 && group <= 32 && a.workspace != nullptr &&
-         a.row_seq != nullptr && (a.Dv == 0 || a.Dv == a.D) && !a.sink && !a.kblk && !a.gate;
+         a.row_seq != nullptr && (a.Dv == 0 || a.Dv == a.D) && !a.kblk;
 }
 
 // Pass 1 of split-context decoding for grouped heads; the caller merges the chunks.

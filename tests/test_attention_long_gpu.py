@@ -164,6 +164,38 @@ def test_decode_rows_at_long_contexts(ops, name):
     assert float(o2.float().abs().mean()) > 0.1
 
 
+@pytest.mark.parametrize("n_q,n_kv,d", [(16, 4, 128), (8, 2, 64), (12, 1, 128), (4, 4, 32), (6, 3, 256), (2, 2, 16)])
+@pytest.mark.parametrize("window", [0, 200])
+@pytest.mark.parametrize("sink,learned,gated", [(True, False, False), (True, True, True), (False, False, True)])
+def test_decode_rows_with_a_sink_and_a_gate(ops, n_q, n_kv, d, window, sink, learned, gated):
+    """Single rows of layers with a sink, its learned scores (one above every key's, one of minus infinity) and a gate in
+    columns of wider rows: the split-context kernels, a sink and gate in their merge, alone and before a
+    prompt's portion; and the kernels that cut by what a small workspace holds."""
+    g = torch.Generator(device="cuda").manual_seed(d)
+    for seqs in ([(p, 1) for p in (700, 127, 128, 0, 511, 1300)], [(300, 1), (64, 1), (0, 70)]):
+        case = shared_stream_case(seqs, n_q, n_kv, d, 16, torch.bfloat16, window)
+        ctx, qkv, k_pool, v_pool, bt, perm = case
+        ctx.single_rows = sum(1 for _, m in seqs if m == 1)
+        wide = torch.randn(ctx.T, n_q * d + 4, generator=g, device="cuda").bfloat16()
+        gate = wide[:, 4:] if gated else None
+        sinks = torch.randn(n_q, generator=g, device="cuda") if learned else None
+        if learned:
+            sinks[0], sinks[1] = 40.0, float("-inf")
+        outs = []
+        for plain in (False, True):
+            ops.force_generic = plain
+            try:
+                out = torch.full((ctx.T, n_q * d), float("nan"), device="cuda", dtype=torch.bfloat16)
+                ops.paged_attention(qkv, k_pool, v_pool, bt, ctx, n_q, n_kv, d, 16, window, 1 / math.sqrt(d), out,
+                                    sink=sink, sinks=sinks, gate=gate)
+                outs.append(out.double())
+            finally:
+                ops.force_generic = False
+        assert torch.isfinite(outs[0]).all()
+        # probabilities and outputs are rounded to bfloat16 once each (2^-9 of their size), in either kernel
+        assert ((outs[0] - outs[1]).norm() / outs[1].norm()).item() < 8e-3
+
+
 @pytest.mark.parametrize("name", ["scalar128-b8-8k", "scalar256-b32-8k", "scalar256-b8-32k",
                                   "heads1024-b8-32k", "heads512-b8-8k", "heads256-b8-4k",
                                   "scalar128-b8-8k-window", "scalar256-b32-8k-window",
