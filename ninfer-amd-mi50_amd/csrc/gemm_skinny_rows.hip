@@ -1,8 +1,8 @@
-// C = A W^T (+ bias, an activation, or gated) for a dense product of 17 to 512 rows: too many for a block that owns
+// C = A W^T (+ bias, an activation, or gated) for a dense product of 17 to 512 rows (any number for a router's few features): too many for a block that owns
 // all of them, too few to pay for the tiles of the many-row kernel.
 //
 // A block owns 32 rows of A and up to 32 rows of W: two sets of up to 16 (of a gated product a set of the gate's and
-// the same of the other half's), or one set. Its 8 waves split K, each a contiguous part walked in chunks of 128;
+// the same of the other half's), or one set. Its 8 waves (a router's 8 or 16) split K, each a contiguous part walked in chunks of 128;
 // partial tiles meet in LDS and are summed in wave order, so a row's result depends neither on timing nor on the other
 // rows. Both operands are loaded as whole 128-byte lines (8 rows an instruction) and reach the matrix instruction's
 // layout through 2 KB of LDS per wave. The row parts of a feature tile lie side by side on one XCD
@@ -23,30 +23,34 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kRowsMax = 512;
-constexpr int kRowsWaves = 8, kRowsTiles = 2, kRowsOfBlock = 16 * kRowsTiles;
+constexpr int kRowsTiles = 2, kRowsOfBlock = 16 * kRowsTiles;
 
 static int rows_parts(const GemmArgs& a) { return (a.M + kRowsOfBlock - 1) / kRowsOfBlock; }
 
 struct RowsPlan {
   int sets;     // sets of W rows in a block: 1 or 2
   int rows;     // W rows of a set, up to 16
+  int waves;    // 8 or 16
   int grid_x;   // feature tiles
   int grid_y;   // row parts
 };
 
 // AGAIN: another block reads the same weights (they are to stay in L2)
-template <int SETS, bool GATED, bool AGAIN, typename TC>
-__global__ __launch_bounds__(kRowsWaves * 64) void gemm_skinny_rows_kernel(GemmArgs a, RowsPlan p) {
+template <int WAVES, int SETS, bool GATED, bool AGAIN, typename TC>
+__global__ __launch_bounds__(WAVES * 64) void gemm_skinny_rows_kernel(GemmArgs a, RowsPlan p) {
   static_assert(!GATED || SETS == 2, "a gated product's two sets");
   constexpr int RT = kRowsTiles, GROUPS = GATED ? 1 : SETS;   // groups of features
   // partial tiles: [wave][set][row tile][token 16][feature 16]; the first bytes are the waves' 2 KB
   // each while the K range is walked
-  __shared__ __attribute__((aligned(16))) float red[kRowsWaves * SETS * RT * 256];
+  __shared__ __attribute__((aligned(16))) float red[WAVES * SETS * RT * 256];
   unsigned char* stage = (unsigned char*)red;
-  static_assert(SETS * RT * 1024 >= 2048, "the lines fit in the partial tiles' memory");
+  static_assert(WAVES * SETS * RT * 1024 >= WAVES * 2048, "the lines fit in the partial tiles' memory");
   const int slot = blockIdx.x / kXcds;   // line_tile: the row parts of a feature tile on one XCD
-  const int by = slot % p.grid_y, bx = (slot / p.grid_y) * kXcds + blockIdx.x % kXcds;
-  if (bx >= p.grid_x) return;
+  // (few features: the feature tiles of a row part, so that the rows come from HBM once)
+  const bool few = a.N <= 128;
+  const int by = few ? slot / p.grid_x * kXcds + blockIdx.x % kXcds : slot % p.grid_y;
+  const int bx = few ? slot % p.grid_x : slot / p.grid_y * kXcds + blockIdx.x % kXcds;
+  if (bx >= p.grid_x || by >= p.grid_y) return;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int r = lane & 15, j = lane >> 4;
   const int n0 = bx * p.rows * GROUPS, row0 = by * kRowsOfBlock, K = a.K;
@@ -81,7 +85,7 @@ __global__ __launch_bounds__(kRowsWaves * 64) void gemm_skinny_rows_kernel(GemmA
   const int st_write = ((lane >> 3) * 128) + 16 * ((lane & 7) ^ ((lane >> 3) & 7));   // + 1024 q
   const int st_read = r * 128;
   const bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
-  const int chunks = K / 128, per_wave = (chunks + kRowsWaves - 1) / kRowsWaves;
+  const int chunks = K / 128, per_wave = (chunks + WAVES - 1) / WAVES;
   const int c_end = min((wave + 1) * per_wave, chunks);
   for (int c = wave * per_wave; c < c_end; ++c) {
     bf16x8 wl[SETS][2][2], x[RT][2][2];   // [set or row tile][half of the chunk][q]
@@ -135,13 +139,13 @@ __global__ __launch_bounds__(kRowsWaves * 64) void gemm_skinny_rows_kernel(GemmA
       for (int v = 0; v < 4; ++v)
         red[((wave * SETS + s) * RT + t) * 256 + r * 16 + 4 * j + v] = acc[s][t][v];
   __syncthreads();
-  for (int idx = threadIdx.x; idx < GROUPS * RT * 256; idx += kRowsWaves * 64) {
+  for (int idx = threadIdx.x; idx < GROUPS * RT * 256; idx += WAVES * 64) {
     const int gt = idx >> 8, g = gt / RT, t = gt % RT, m = (idx >> 4) & 15, f = idx & 15;
     const int row = row0 + 16 * t + m, col = n0 + g * p.rows + f;
     if (row >= a.M || f >= p.rows || col >= a.N) continue;
     float v = 0.f, u = 0.f;
 #pragma unroll
-    for (int w = 0; w < kRowsWaves; ++w) {
+    for (int w = 0; w < WAVES; ++w) {
       v += red[((w * SETS + g) * RT + t) * 256 + (idx & 255)];
       if (GATED) u += red[((w * SETS + 1) * RT + t) * 256 + (idx & 255)];
     }
@@ -166,18 +170,19 @@ __global__ __launch_bounds__(kRowsWaves * 64) void gemm_skinny_rows_kernel(GemmA
 // - 33 rows and more, against the library's product: 2,048 features, 64 rows 6.0 and 8.9, 128 rows 7.0 and 8.3 (K 5,632
 //   12.1 and 17.9, 14.7 and 15.9); 6,144 64 rows 12.1 and 12.7, 128 15.7 and 14.9; 8,192 (K 8,192) 64 rows 42 and 33.
 //   Against tiles of 64 rows: gated 2 x 5,632 64 rows 17.7 and 20.8, 80 22.0 and 19.0; 2 x 2,816 128 rows 9.8 and
-//   11.6; 2 x 1,408 256 rows 14.5 and 18; 2 x 20,480 64 rows 87 and 72; a few hundred features 5.2 and 13. (Up to 128
-//   features: the few-row kernel.)
+//   11.6; 2 x 1,408 256 rows 14.5 and 18; 2 x 20,480 64 rows 87 and 72; a few hundred features 5.2 and 13.
 // - beyond 128 rows, against the library's product: 2,048 features 160 rows 9.9 and 9.1; 1,024 (K 2,816) 256 rows 7.7 and
 //   8.5; 768 256 rows 6.4 and 8.4, 384 9.5 and 9.1.
+// - up to 128 features (a router's), against the few-row kernel, whose rows came 64 bytes at a time: 61 features, K 2,048,
+//   512 rows 5.5 and 6.1, 2,048 rows 6.3 and 13.2, 4,096 8.7 and 22.7 (the same bits).
 bool gemm_skinny_rows_takes(const GemmArgs& a) {
-  if (a.offsets || a.a_index || a.c_index || a.groups > 1 || a.force_kernel || a.in_dtype != kBF16 || a.M <= 16 ||
-      a.M > kRowsMax || a.K % 128 || a.lda % 8 || (uintptr_t)a.A % 16 || (uintptr_t)a.W % 16)
+  if (a.offsets || a.a_index || a.c_index || a.groups > 1 || a.force_kernel || a.in_dtype != kBF16 || a.M <= 16 || a.K % 128 || a.lda % 8 || (uintptr_t)a.A % 16 || (uintptr_t)a.W % 16)
     return false;
   const bool gated = epilogue_gated(a.epilogue);
   const int64_t w_rows = (int64_t)a.N * (gated ? 2 : 1);
   if (a.M <= 32) return w_rows > (gated ? 4096 : 2560);
-  return a.N > 128 && w_rows * rows_parts(a) <= (gated ? 24576 : a.M <= 128 ? 16384 : 8192);
+  if (a.N <= 128) return !gated && a.M > 64;
+  return a.M <= kRowsMax && w_rows * rows_parts(a) <= (gated ? 24576 : a.M <= 128 ? 16384 : 8192);
 }
 
 // Features a block, so that the blocks on an XCD (the row parts of its feature tiles) fill rounds of one a CU: 6,144
@@ -189,7 +194,8 @@ static RowsPlan plan_rows(const GemmArgs& a) {
   const int most = gated ? 16 : 32, slots = max(1, device_cu_count() / kXcds);
   p.grid_y = rows_parts(a);
   int f = most;
-  for (int rounds = 1; rounds <= 8; ++rounds) {
+  if (a.N <= 128) f = a.N <= 16 || (int64_t)p.grid_y * ((a.N + 15) / 16) <= 2 * device_cu_count() ? 16 : 32;
+  else for (int rounds = 1; rounds <= 8; ++rounds) {
     const int tiles = slots * rounds / p.grid_y * kXcds;   // feature tiles on all XCDs
     if (tiles > 0 && (a.N + tiles - 1) / tiles <= most) {
       f = gated ? max(8, (a.N + tiles - 1) / tiles) : max(16, (a.N + tiles - 1) / tiles);
@@ -198,6 +204,9 @@ static RowsPlan plan_rows(const GemmArgs& a) {
   }
   p.sets = gated || f > 16 ? 2 : 1;
   p.rows = gated || p.sets == 1 ? f : (f + 1) / 2;
+  // (up to 128 features: as many waves as the few-row kernel, so that a router's sums are the same in either)
+  const int row_tiles = (a.M + 15) / 16;
+  p.waves = a.N <= 128 && (a.N + 15) / 16 * row_tiles < device_cu_count() && a.K >= 2048 ? 16 : 8;
   const int of_block = gated ? p.rows : p.sets * p.rows;
   p.grid_x = (a.N + of_block - 1) / of_block;
   return p;
@@ -206,15 +215,18 @@ static RowsPlan plan_rows(const GemmArgs& a) {
 int gemm_skinny_rows(const GemmArgs& a, hipStream_t stream) {
   NINFER_REQUIRE(gemm_skinny_rows_takes(a), "gemm: not a product for blocks of 32 rows");
   const RowsPlan p = plan_rows(a);
-  const int64_t blocks = (int64_t)((p.grid_x + kXcds - 1) / kXcds) * kXcds * p.grid_y;
+  const int on_xcds = a.N <= 128 ? p.grid_y : p.grid_x, beside = a.N <= 128 ? p.grid_x : p.grid_y;
+  const int64_t blocks = (int64_t)((on_xcds + kXcds - 1) / kXcds) * kXcds * beside;
   NINFER_REQUIRE(blocks < (1LL << 31), "gemm: %lld blocks are too many", (long long)blocks);
-  const dim3 grid((unsigned)blocks), block(kRowsWaves * 64);
+  const dim3 grid((unsigned)blocks), block(p.waves * 64);
   auto launch = [&](auto again, auto tc) {
     constexpr bool AGAIN = decltype(again)::value;
     typedef decltype(tc) TC;
-    if (epilogue_gated(a.epilogue)) gemm_skinny_rows_kernel<2, true, AGAIN, TC><<<grid, block, 0, stream>>>(a, p);
-    else if (p.sets == 2) gemm_skinny_rows_kernel<2, false, AGAIN, TC><<<grid, block, 0, stream>>>(a, p);
-    else gemm_skinny_rows_kernel<1, false, AGAIN, TC><<<grid, block, 0, stream>>>(a, p);
+    if (epilogue_gated(a.epilogue)) gemm_skinny_rows_kernel<8, 2, true, AGAIN, TC><<<grid, block, 0, stream>>>(a, p);
+    else if (p.waves == 16 && p.sets == 2) gemm_skinny_rows_kernel<16, 2, false, AGAIN, TC><<<grid, block, 0, stream>>>(a, p);
+    else if (p.waves == 16) gemm_skinny_rows_kernel<16, 1, false, AGAIN, TC><<<grid, block, 0, stream>>>(a, p);
+    else if (p.sets == 2) gemm_skinny_rows_kernel<8, 2, false, AGAIN, TC><<<grid, block, 0, stream>>>(a, p);
+    else gemm_skinny_rows_kernel<8, 1, false, AGAIN, TC><<<grid, block, 0, stream>>>(a, p);
   };
   auto typed = [&](auto again) {
     if (a.out_dtype == kF32) launch(again, float{});
