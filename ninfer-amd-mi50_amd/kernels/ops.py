@@ -1270,11 +1270,12 @@ class HipOps:
             ctypes.c_void_p(ctx.seq_row_start.data_ptr()), ctypes.c_void_p(ctx.seq_slots.data_ptr()),
             t, ctx.S, h, taps, 1 if ctx.max_qlen == 1 else 0, _DT[out.dtype], self._stream()))
 
-    def norm_add(self, residual, y, gain, eps, center=False, weights=None):
+    def norm_add(self, residual, y, gain, eps, center=False, weights=None, then=None):
         """residual += y rsqrt(mean(y^2) + eps) gain; gain holds one number or one per column.
         `center`: the layer norm instead, (y - mean(y)) rsqrt(mean((y - mean(y))^2) + eps) gain.
         `weights` [T, k] (32-bit): y holds T * k rows and stands for the rows
-        sum_j weights[t, j] y[t * k + j], formed in 32-bit (a sparse feed-forward's output)."""
+        sum_j weights[t, j] y[t * k + j], formed in 32-bit (a sparse feed-forward's output).
+        `then` = (gain [H], eps, center, out [T, H] of y's dtype): a norm of the new residual, by the same kernel."""
         _dev(residual, "residual", torch.float32, 2)
         _dev(y, "y", dims=2)
         _dev(gain, "gain", torch.float32, 1)
@@ -1288,11 +1289,17 @@ class HipOps:
             _need(y.shape == residual.shape, "norm_add: y does not fit the residual")
         _need(y.dtype in _DT, "norm_add: y's dtype")
         _need(gain.shape[0] in (1, y.shape[1]), "norm_add: one gain, or one per column")
+        gain2, eps2, center2, out2 = then if then is not None else (None, 0.0, False, None)
+        if then is not None:
+            _dev(gain2, "second gain", torch.float32, 1)
+            _dev(out2, "out", y.dtype, 2)
+            _need(gain2.shape[0] == y.shape[1] and out2.shape == residual.shape, "norm_add: the second norm's sizes")
         self._ok(self.lib.ninfer_norm_add(
             ctypes.c_void_p(residual.data_ptr()), ctypes.c_void_p(y.data_ptr()),
             ctypes.c_void_p(gain.data_ptr()), gain.shape[0], residual.shape[0], y.shape[1],
             ctypes.c_float(eps), _DT[y.dtype], 1 if center else 0,
-            ctypes.c_void_p(_ptr(weights)), k, self._stream()))
+            ctypes.c_void_p(_ptr(weights)), k, ctypes.c_void_p(_ptr(gain2)), ctypes.c_void_p(_ptr(out2)),
+            ctypes.c_float(eps2), 1 if center2 else 0, self._stream()))
 
     def post_norm(self, residual, y, gain, eps, alpha, out=None, weights=None):
         """residual <- norm(alpha residual + y) in 32-bit, norm(z) = z rsqrt(mean(z^2) + eps)

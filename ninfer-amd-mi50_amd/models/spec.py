@@ -15,7 +15,7 @@ from typing import Dict, List, Optional
 
 import torch
 
-from ..parts.base import Block, CallInfo, Norm, Part, StepContext, WeightBinder
+from ..parts.base import Block, CallInfo, Norm, NormedOutput, Part, StepContext, WeightBinder
 from ..parts.embedding import LMHead, TokenEmbedding
 from ..weights.source import TensorSpec
 
@@ -112,6 +112,12 @@ class ModelSpec:
                 residual = self.joins[call.before].forward(ctx, residual, pending, first)
                 pending = None
             pending = self.blocks[call.layer].forward(ctx, residual, pending, info)
+            if isinstance(pending, NormedOutput):
+                after = self.plan[i + 1] if i + 1 < len(self.plan) else None
+                if tap is not None or after is None or after.before is not None \
+                        or not self.blocks[after.layer].takes_normed_output:
+                    pending.norm.add(ctx, residual, pending.y)
+                    pending = None
             if tap is not None:
                 tap(i, residual, pending)
         if logit_rows is None or logit_rows.numel() == 0:

@@ -227,6 +227,14 @@ def _formed(ctx: "StepContext", pending, like: torch.Tensor) -> torch.Tensor:
     return total.to(ctx.act_dtype)
 
 
+@dataclass
+class NormedOutput:
+    """What a block leaves to be normed and added to the residual: norm.add(ctx, residual, y). Handed on only to
+    a block that takes it (`Block.takes_normed_output`), whose first norm then runs in the same kernel."""
+    norm: Any
+    y: Any
+
+
 def plain_rows(ctx: "StepContext", y):
     """What a part handed on as something that any part takes: a NormedSum, a SumRows or a
     NormedRows becomes rows, a ReadyRows nothing; everything else is handed back unchanged."""
@@ -419,6 +427,7 @@ class Block(Part):
     """Arrangement of norms, mixer and feed-forward around the residual."""
 
     mixer: Mixer
+    takes_normed_output = False   # `forward` takes a NormedOutput of the block before as `pending`
 
     def state_floats(self) -> int:
         """32-bit numbers of per-request state of one run of this block: the mixer's, and

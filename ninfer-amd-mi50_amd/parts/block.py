@@ -14,7 +14,7 @@ from ..registry import register_part
 import torch
 
 from ..weights.source import TensorSpec
-from .base import (Block, CallInfo, FeedForward, Mixer, Norm, Part, PendingRows, ReadyRows,
+from .base import (Block, CallInfo, FeedForward, Mixer, Norm, NormedOutput, Part, PendingRows, ReadyRows,
                    StepContext, WeightBinder, plain_rows, settle)
 from .norm import RMSNorm
 
@@ -119,7 +119,10 @@ class SandwichBlock(Block):
     x += post2(feed_forward(pre2(x))). The norms before are `Norm`s of the residual, those after
     parts with `add(ctx, residual, y)` (they norm y and add it into the 32-bit residual; a
     sparse feed-forward's weighted rows are summed by the same kernel). `feed_forward` may be
-    None (a layer with a mixer only)."""
+    None (a layer with a mixer only). The norm behind a sublayer and the one in front of the next run as one
+    kernel; the block's last one is handed on for the next block's first."""
+
+    takes_normed_output = True
 
     def __init__(self, mixer_norm: Norm, mixer: Mixer, mixer_out_norm: Part,
                  ff_norm: Optional[Norm] = None, feed_forward: Optional[FeedForward] = None,
@@ -134,15 +137,18 @@ class SandwichBlock(Block):
                             self.feed_forward, self.ff_out_norm) if p is not None]
 
     def forward(self, ctx: StepContext, residual, pending, call: CallInfo):
-        h = self.mixer_norm.forward(ctx, residual, pending)
-        self.mixer_out_norm.add(ctx, residual, self.mixer.forward(ctx, h, residual, call))
-        if self.feed_forward is not None:
-            h = self.ff_norm.forward(ctx, residual, None)
-            y = self.feed_forward.forward(ctx, h, residual)
-            if y is None:
-                raise ValueError("a feed-forward between two norms hands its rows back")
-            self.ff_out_norm.add(ctx, residual, y)
-        return None
+        if isinstance(pending, NormedOutput):
+            h = pending.norm.add_then(ctx, residual, pending.y, self.mixer_norm)
+        else:
+            h = self.mixer_norm.forward(ctx, residual, pending)
+        y = self.mixer.forward(ctx, h, residual, call)
+        if self.feed_forward is None:
+            return NormedOutput(self.mixer_out_norm, y)
+        h = self.mixer_out_norm.add_then(ctx, residual, y, self.ff_norm)
+        y = self.feed_forward.forward(ctx, h, residual)
+        if y is None:
+            raise ValueError("a feed-forward between two norms hands its rows back")
+        return NormedOutput(self.ff_out_norm, y)
 
 
 register_part("block", "sandwich", SandwichBlock)

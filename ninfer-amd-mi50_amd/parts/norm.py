@@ -116,6 +116,20 @@ class OutputRMSNorm(Part):
         else:
             ctx.ops.norm_add(residual, y, self.gain, self.eps, center=self.center)
 
+    def add_then(self, ctx: StepContext, residual: torch.Tensor, y, norm: Norm) -> torch.Tensor:
+        """`add`, and the rows that `norm` makes of the new residual: one kernel on the GPU."""
+        y = plain_rows(ctx, y)
+        rows, weights = (y.y, y.weights) if isinstance(y, PendingRows) else (y, None)
+        if not (residual.is_cuda and isinstance(norm, RMSNorm) and norm.size == residual.shape[1]
+                and rows.dtype == ctx.act_dtype) or getattr(y, "shared", None) is not None \
+                or getattr(y, "ids", None) is not None:
+            self.add(ctx, residual, y)
+            return norm.forward(ctx, residual, None)
+        out = ctx.empty(residual.shape)
+        ctx.ops.norm_add(residual, rows, self.gain, self.eps, center=self.center, weights=weights,
+                         then=(norm.gain, norm.eps, norm.center, out))
+        return out
+
 
 class ResidualRMSNorm(Part):
     """The norm of a block that norms the residual stream itself, behind the sum:

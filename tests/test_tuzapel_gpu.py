@@ -237,6 +237,35 @@ SHAPES = [  # heads, kv, dim, vdim, window, page
     (40, 1, 16, 16, 9, 4)]
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,width", [(1, 2048), (64, 1024), (3, 30), (5, 8192), (7, 258)])
+@pytest.mark.parametrize("k,center,single", [(0, False, False), (0, True, True), (4, True, False)])
+def test_norm_behind_a_sublayer_and_the_next_in_front(ops, dtype, rows, width, k, center, single):
+    """A norm added to the residual, and another norm of the sum by the same kernel: against both written out
+    (32-bit sums of `width` terms; the rows rounded once to their type), and the residual bit for bit the one
+    that the first norm alone leaves."""
+    g = torch.Generator().manual_seed(rows + width + k)
+    x = torch.randn(rows, width, generator=g) * 3 + 1
+    y = (torch.randn(rows * max(k, 1), width, generator=g) - 0.5).to(dtype)
+    w = torch.rand(rows, k, generator=g) if k else None
+    g1, g2 = torch.randn(1 if single else width, generator=g), torch.randn(width, generator=g)
+
+    def norm(v, gain, eps, c):
+        v = v - v.mean(-1, keepdim=True) if c else v
+        return v / torch.sqrt((v * v).mean(-1, keepdim=True) + eps) * gain.double()
+
+    plain = y.double() if not k else (w.double()[..., None] * y.double().view(rows, k, width)).sum(1)
+    new = x.double() + norm(plain, g1, 1e-6, center)
+    alone, both = x.to(DEV), x.to(DEV)
+    out = torch.full((rows + 1, width), 7.0, dtype=dtype, device=DEV)
+    wd = w.to(DEV) if k else None
+    ops.norm_add(alone, y.to(DEV), g1.to(DEV), 1e-6, center=center, weights=wd)
+    ops.norm_add(both, y.to(DEV), g1.to(DEV), 1e-6, center=center, weights=wd, then=(g2.to(DEV), 1e-3, not center, out[:rows]))
+    assert torch.equal(alone, both) and (out[rows] == 7.0).all()
+    assert rel_err(both, new) < 1e-6
+    assert rel_err(out[:rows], norm(new, g2, 1e-3, not center)) < (2e-6 if dtype == torch.float32 else 3e-3)
+
+
 @pytest.mark.parametrize("dtype,plain_kernel", [(torch.float32, False), (torch.bfloat16, False), (torch.bfloat16, True)])
 @pytest.mark.parametrize("sink", [True, False])
 @pytest.mark.parametrize("heads,kv,dim,vdim,window,ps", SHAPES)
