@@ -73,6 +73,8 @@ __host__ __device__ inline int attention_blocks_seen(int pos, int window, int bl
 
 int attention_check(const AttnArgs& a);
 int attention_generic(const AttnArgs& a, hipStream_t stream);
+bool attention_rows_f32_takes(const AttnArgs& a);   // prompt portions in 32-bit, with the plain kernel's bits
+int attention_rows_f32(const AttnArgs& a, hipStream_t stream);
 
 int64_t attention_decode_workspace_floats(int T, int Hq, int D, int max_kv_len);
 bool attention_decode_takes(const AttnArgs& a);

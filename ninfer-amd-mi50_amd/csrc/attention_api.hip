@@ -89,6 +89,21 @@ extern "C" int ninfer_paged_attention(const AttnArgs* a, int force_generic, hipS
   }
   // ... and prompt portions of any such shape on the matrix cores
   if (tiles) return attention_tiles(*a, apart ? n : 0, stream);
+  if (!force_generic && n < a->S && attention_rows_f32_takes(*a)) {
+    if (n > 0) {
+      AttnArgs d = *a;
+      d.T = n;
+      d.S = n;
+      d.max_qlen = 1;
+      if (int rc = attention_generic(d, stream)) return rc;
+    }
+    AttnArgs p = *a;
+    p.seq_row_start += n;
+    p.block_table += (int64_t)n * a->bt_stride;
+    p.S = a->S - n;
+    p.T = a->T - n;
+    return attention_rows_f32(p, stream);
+  }
   return attention_generic(*a, stream);
 }
 

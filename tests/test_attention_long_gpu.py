@@ -196,6 +196,41 @@ def test_decode_rows_with_a_sink_and_a_gate(ops, n_q, n_kv, d, window, sink, lea
         assert ((outs[0] - outs[1]).norm() / outs[1].norm()).item() < 8e-3
 
 
+@pytest.mark.parametrize("n_q,n_kv,d,vdim", [(16, 16, 128, 128), (8, 2, 64, 128), (4, 1, 100, 36), (3, 3, 4, 8)])
+@pytest.mark.parametrize("window,ps", [(0, 16), (70, 8), (1, 4)])
+@pytest.mark.parametrize("extras", ["", "slopes", "sink", "sinks gate"])
+def test_prompt_rows_in_32_bit_bit_for_bit_as_the_plain_kernel(ops, n_q, n_kv, d, vdim, window, ps, extras):
+    """Portions of 1 to 173 rows (parts of a block's 8 rows, of a tile of 64 keys, behind cached keys, single rows in
+    front), with a window, a position bias, sinks and a gate: the same bits as one wave per row and head."""
+    seqs = [(127, 1), (64, 1), (0, 173), (60, 9), (199, 2), (63, 1), (300, 64)]
+    case = shared_stream_case(seqs, n_q, n_kv, d, ps, torch.float32, window)
+    ctx, qkv, k_pool, v_pool, bt, perm = case
+    g = torch.Generator(device="cuda").manual_seed(d)
+    rnd = lambda *shape: torch.randn(*shape, generator=g, device="cuda")
+    v_pool = rnd(*k_pool.shape[:3], vdim)
+    kw = {"vdim": vdim}
+    if "slopes" in extras:
+        kw["slopes"] = rnd(n_q)
+    if "sink" in extras:
+        kw["sink"] = True
+    if "sinks" in extras:
+        kw["sinks"] = rnd(n_q)
+    if "gate" in extras:
+        kw["gate"] = rnd(ctx.T, n_q * vdim + 4)[:, 4:]
+    for single in (0, 2):
+        ctx.single_rows = single
+        outs = []
+        for plain in (True, False):
+            ops.force_generic = plain
+            try:
+                out = torch.full((ctx.T, n_q * vdim), float("nan"), device="cuda")
+                ops.paged_attention(qkv, k_pool, v_pool, bt, ctx, n_q, n_kv, d, ps, window, 1 / math.sqrt(d), out, **kw)
+                outs.append(out)
+            finally:
+                ops.force_generic = False
+        assert torch.isfinite(outs[0]).all() and torch.equal(outs[0], outs[1])
+
+
 @pytest.mark.parametrize("name", ["scalar128-b8-8k", "scalar256-b32-8k", "scalar256-b8-32k",
                                   "heads1024-b8-32k", "heads512-b8-8k", "heads256-b8-4k",
                                   "scalar128-b8-8k-window", "scalar256-b32-8k-window",
