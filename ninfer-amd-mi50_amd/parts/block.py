@@ -16,7 +16,7 @@ import torch
 from ..weights.source import TensorSpec
 from .base import (Block, CallInfo, FeedForward, Mixer, Norm, NormedOutput, Part, PendingRows, ReadyRows,
                    StepContext, WeightBinder, plain_rows, settle)
-from .norm import RMSNorm
+from .norm import OutputRMSNorm, RMSNorm
 
 
 class PreNormBlock(Block):
@@ -114,6 +114,14 @@ class OutputNormBlock(Block):
 register_part("block", "output_norm", OutputNormBlock)
 
 
+def add_then(ctx: StepContext, residual, out_norm: Part, y, norm: Norm):
+    """The norm behind a sublayer that gave y, and the rows that `norm` makes of the new residual."""
+    if isinstance(out_norm, OutputRMSNorm):
+        return out_norm.add_then(ctx, residual, y, norm)
+    out_norm.add(ctx, residual, y)
+    return norm.forward(ctx, residual, None)
+
+
 class SandwichBlock(Block):
     """A block with a norm before and after each sublayer: x += post1(mixer(pre1(x))), then
     x += post2(feed_forward(pre2(x))). The norms before are `Norm`s of the residual, those after
@@ -138,13 +146,13 @@ class SandwichBlock(Block):
 
     def forward(self, ctx: StepContext, residual, pending, call: CallInfo):
         if isinstance(pending, NormedOutput):
-            h = pending.norm.add_then(ctx, residual, pending.y, self.mixer_norm)
+            h = add_then(ctx, residual, pending.norm, pending.y, self.mixer_norm)
         else:
             h = self.mixer_norm.forward(ctx, residual, pending)
         y = self.mixer.forward(ctx, h, residual, call)
         if self.feed_forward is None:
             return NormedOutput(self.mixer_out_norm, y)
-        h = self.mixer_out_norm.add_then(ctx, residual, y, self.ff_norm)
+        h = add_then(ctx, residual, self.mixer_out_norm, y, self.ff_norm)
         y = self.feed_forward.forward(ctx, h, residual)
         if y is None:
             raise ValueError("a feed-forward between two norms hands its rows back")

@@ -117,12 +117,14 @@ class OutputRMSNorm(Part):
             ctx.ops.norm_add(residual, y, self.gain, self.eps, center=self.center)
 
     def add_then(self, ctx: StepContext, residual: torch.Tensor, y, norm: Norm) -> torch.Tensor:
-        """`add`, and the rows that `norm` makes of the new residual: one kernel on the GPU."""
+        """`add`, and the rows that `norm` makes of the new residual: one kernel on the GPU where both norms are the
+        ones of this module, none with an `add` or a `forward` of its own."""
         y = plain_rows(ctx, y)
         rows, weights = (y.y, y.weights) if isinstance(y, PendingRows) else (y, None)
-        if not (residual.is_cuda and isinstance(norm, RMSNorm) and norm.size == residual.shape[1]
-                and rows.dtype == ctx.act_dtype) or getattr(y, "shared", None) is not None \
-                or getattr(y, "ids", None) is not None:
+        alike = type(self).add is OutputRMSNorm.add and isinstance(norm, RMSNorm) \
+            and type(norm).forward is RMSNorm.forward
+        if not (alike and residual.is_cuda and norm.size == residual.shape[1] and rows.dtype == ctx.act_dtype) \
+                or getattr(y, "shared", None) is not None or getattr(y, "ids", None) is not None:
             self.add(ctx, residual, y)
             return norm.forward(ctx, residual, None)
         out = ctx.empty(residual.shape)

@@ -389,3 +389,33 @@ def test_host_new_parts_inside_other_blocks():
     got = torch.cat([runner.step([Chunk(slot, toks[:11], list(range(11)))]),
                      runner.step([Chunk(slot, toks[11:], list(range(8)))])])
     torch.testing.assert_close(got.double(), want, atol=2e-4, rtol=2e-4)
+
+
+def test_host_sandwich_block_with_a_part_that_only_adds():
+    """The part behind a sublayer needs `add` alone."""
+    from ninfer_amd.parts import RMSNorm, SandwichBlock
+    from ninfer_amd.parts.base import Mixer, NormedOutput, Part
+
+    class Adds(Part):
+        def add(self, ctx, residual, y):
+            residual += 2 * y
+
+    class Doubles(Mixer):
+        def forward(self, ctx, x, residual, call=None):
+            return 2 * x
+
+    class Takes(RMSNorm):
+        def forward(self, ctx, residual, pending):
+            assert pending is None
+            return residual + 1
+    blocks = [SandwichBlock(Takes("a", 4, 1e-5), Doubles(), Adds(), Takes("b", 4, 1e-5), Doubles(), Adds()) for _ in range(2)]
+    x = torch.arange(4.)
+    want = x.clone()
+    for _ in range(4):
+        want = want + 4 * (want + 1)
+    pending = None
+    for b in blocks:
+        pending = b.forward(None, x, pending, None)
+    assert isinstance(pending, NormedOutput)
+    pending.norm.add(None, x, pending.y)
+    assert torch.equal(x, want)
