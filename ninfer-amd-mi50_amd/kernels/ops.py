@@ -2085,6 +2085,16 @@ class HipOps:
         self._ok(self.lib.ninfer_sigmoid_attention(ctypes.byref(a), self._stream()))
 
     # ---- sampling -------------------------------------------------------------------
+    def uniforms(self, seeds, keys, draws, out):
+        """out (32-bit floats in host memory) <- the uniform number of every row's (seed, key, draw), given
+        as arrays of 64-bit numbers: a counter hash, on the host."""
+        at = [v.buffer_info() for v in (seeds, keys, draws)]
+        n = at[0][1]
+        _need(at[1][1] == n == at[2][1] and out.shape == (n,) and out.dtype.char == "f" and out.flags.c_contiguous
+              and out.flags.writeable and all(v.itemsize == 8 for v in (seeds, keys, draws)), "uniforms: the arrays' sizes")
+        self.lib.ninfer_uniforms(ctypes.c_void_p(at[0][0]), ctypes.c_void_p(at[1][0]), ctypes.c_void_p(at[2][0]),
+                                 n, ctypes.c_void_p(out.ctypes.data))
+
     FEW_TOKENS = 64   # most tokens a row may keep (top_k) for the two-launch sampling path
 
     def sample(self, logits, temperature, uniform, out, top_k=None, top_p=None, rep_penalty=None,

@@ -11,6 +11,8 @@ the request gets a seed from the operating system when it is added.
 from __future__ import annotations
 
 import os
+from array import array
+from operator import attrgetter
 from typing import Dict, Iterable, List, Optional, Sequence, Tuple
 
 import numpy as np
@@ -19,6 +21,8 @@ import torch
 from .params import SamplingParams
 
 _MASK = (1 << 64) - 1
+_OPTIONS = attrgetter("temperature", "top_p", "repetition_penalty", "top_k")
+_STREAM = attrgetter("seed", "key", "draw")
 
 
 def _splitmix64(x: int) -> int:
@@ -34,6 +38,16 @@ def uniform(seed: int, key: int, draw: int) -> float:
     return (h >> 40) / float(1 << 24)
 
 
+def _streams(rows: Sequence["SampleRow"]) -> List[array]:
+    """The rows' seeds, keys and draws as arrays of 64-bit numbers."""
+    def u64s(vs):
+        try:
+            return array("Q", vs)
+        except (OverflowError, TypeError):   # (of other sizes or signs: their last 64 bits)
+            return array("Q", [v & _MASK for v in vs])
+    return [u64s(vs) for vs in zip(*map(_STREAM, rows))]
+
+
 def uniforms(rows: Sequence["SampleRow"]) -> np.ndarray:
     """`uniform` of every row's (seed, key, draw) at once, in 32-bit floats (24 bits each: exact)."""
     u64 = np.uint64
@@ -44,8 +58,7 @@ def uniforms(rows: Sequence["SampleRow"]) -> np.ndarray:
         x = (x ^ (x >> u64(27))) * u64(0x94D049BB133111EB)
         return x ^ (x >> u64(31))
 
-    seed, key, draw = (np.array([v & _MASK for v in vs], dtype=u64)
-                       for vs in zip(*((row.seed, row.key, row.draw) for row in rows)))
+    seed, key, draw = (np.frombuffer(v, dtype=u64) for v in _streams(rows))
     return (mix(mix(mix(seed) ^ key) ^ draw) >> u64(40)).astype(np.float32) / np.float32(1 << 24)
 
 
@@ -62,32 +75,33 @@ class History:
     def __init__(self, tokens: Iterable[int] = ()):
         toks, counts = np.unique(np.asarray(list(tokens), dtype=np.int64), return_counts=True)
         n = int(toks.shape[0])
-        cap = max(64, 2 * n)
-        self._tok = np.zeros(cap, np.int32)
-        self._cnt = np.zeros(cap, np.int32)
-        self._tok[:n] = toks
-        self._cnt[:n] = counts
+        self._both = np.zeros((2, max(64, 2 * n)), np.int32)   # tokens, then counts
+        self._both[0, :n] = toks
+        self._both[1, :n] = counts
         self._n = n
         self._where: Optional[Dict[int, int]] = None   # token -> index, made at the first add
 
     def add(self, token: int) -> None:
         if self._where is None:
-            self._where = {int(t): i for i, t in enumerate(self._tok[:self._n])}
+            self._where = {int(t): i for i, t in enumerate(self._both[0, :self._n])}
         i = self._where.get(token)
         if i is not None:
-            self._cnt[i] += 1
+            self._both[1, i] += 1
             return
-        if self._n == self._tok.shape[0]:
-            self._tok = np.concatenate([self._tok, np.zeros_like(self._tok)])
-            self._cnt = np.concatenate([self._cnt, np.zeros_like(self._cnt)])
-        self._tok[self._n] = token
-        self._cnt[self._n] = 1
+        if self._n == self._both.shape[1]:
+            self._both = np.concatenate([self._both, np.zeros_like(self._both)], axis=1)
+        self._both[0, self._n] = token
+        self._both[1, self._n] = 1
         self._where[token] = self._n
         self._n += 1
 
     def arrays(self) -> Tuple[np.ndarray, np.ndarray]:
         """(distinct tokens, their counts), int32 views of equal length."""
-        return self._tok[:self._n], self._cnt[:self._n]
+        return self._both[0, :self._n], self._both[1, :self._n]
+
+    def both(self) -> np.ndarray:
+        """`arrays` as the two rows of one view."""
+        return self._both[:, :self._n]
 
     def count(self, token: int) -> int:
         toks, cnts = self.arrays()
@@ -144,15 +158,16 @@ class Sampler:
         # 32-bit floats and one int per row, the offsets of the penalties, then their tokens
         # and counts. (Copies queue behind the step that makes the logits, one after the other:
         # every further one would add its latency to the step.)
+        temps, tops, penalties, top_ks = zip(*map(_OPTIONS, (row.params for row in rows))) if r else ((),) * 4
         pens = []
-        offsets = [0]
-        for row in rows:
-            n = offsets[-1]
-            if row.params.repetition_penalty != 1.0:
-                pens.append(row.history.arrays())
-                n += pens[-1][0].shape[0]
-            offsets.append(n)
-        n_pen = offsets[-1]
+        offsets = [0] * (r + 1)
+        n_pen = 0
+        for i, (row, penalty) in enumerate(zip(rows, penalties), 1):
+            if penalty != 1.0:
+                both = row.history.both()
+                pens.append(both)
+                n_pen += both.shape[1]
+            offsets[i] = n_pen
         o = 5 * r
         n = o + (r + 1 + 2 * n_pen if n_pen > 0 else 0)
         cuda = self.device.type == "cuda"
@@ -161,22 +176,25 @@ class Sampler:
         else:
             packed = np.empty(n, np.int32)
         floats = packed[:4 * r].view(np.float32).reshape(4, r)
-        floats[0] = [row.params.temperature for row in rows]
-        floats[1] = [row.params.top_p for row in rows]
-        floats[2] = [row.params.repetition_penalty for row in rows]
-        drawn = [i for i, row in enumerate(rows) if row.params.temperature > 0]   # (greedy rows draw nothing)
-        floats[3] = 0.0
-        if len(drawn) > 24:   # (whole arrays 32 us for 16 rows, 34 for 24, 47 for 64; one by one 21, 31 and 83)
-            floats[3, drawn] = uniforms([rows[i] for i in drawn])
-        else:
-            for i in drawn:
-                floats[3, i] = uniform(rows[i].seed, rows[i].key, rows[i].draw)
-        packed[4 * r:o] = [row.params.top_k for row in rows]
+        floats[0] = temps
+        floats[1] = tops
+        floats[2] = penalties
+        drawn = [row for row, t in zip(rows, temps) if t > 0]   # (greedy rows draw nothing)
+        if len(drawn) < r:
+            floats[3] = 0.0
+        if drawn:
+            to = floats[3] if len(drawn) == r else np.empty(len(drawn), np.float32)
+            if cuda:
+                self.ops.uniforms(*_streams(drawn), to)
+            else:
+                to[:] = uniforms(drawn)
+            if len(drawn) < r:
+                floats[3, [i for i, t in enumerate(temps) if t > 0]] = to
+        packed[4 * r:o] = top_ks
         if n_pen > 0:
             packed[o:o + r + 1] = offsets
             o += r + 1
-            np.concatenate([p[0] for p in pens], out=packed[o:o + n_pen])
-            np.concatenate([p[1] for p in pens], out=packed[o + n_pen:n])
+            np.concatenate(pens, axis=1, out=packed[o:n].reshape(2, n_pen))
         if cuda:
             dev = torch.empty(n, dtype=torch.int32, device=self.device)
             dev.copy_(pinned[:n], non_blocking=True)
@@ -193,8 +211,7 @@ class Sampler:
         # top_k = 50) take the path that reads the logits with the whole GPU
         most = getattr(self.ops, "FEW_TOKENS", 0)
         # (rows that are all greedy stay with the one launch: it is short as it is)
-        if most and any(row.params.temperature > 0 for row in rows) and all(
-                row.params.temperature <= 0 or 1 <= row.params.top_k <= most for row in rows):
+        if most and drawn and all(t <= 0 or 1 <= k <= most for t, k in zip(temps, top_ks)):
             pen["few"] = True
         self.ops.sample(logits, f[:r], f[3 * r:4 * r], out, top_k=dev[4 * r:5 * r], top_p=f[r:2 * r],
                         rep_penalty=f[2 * r:3 * r], **pen)
