@@ -174,14 +174,15 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_rows_kernel(GemmArgs a
 // - beyond 128 rows, against the library's product: 2,048 features 160 rows 9.9 and 9.1; 1,024 (K 2,816) 256 rows 7.7 and
 //   8.5; 768 256 rows 6.4 and 8.4, 384 9.5 and 9.1.
 // - up to 128 features (a router's), against the few-row kernel, whose rows came 64 bytes at a time: 61 features, K 2,048,
-//   512 rows 5.5 and 6.1, 2,048 rows 6.3 and 13.2, 4,096 8.7 and 22.7 (the same bits).
+//   512 rows 5.5 and 6.1 alone, but 8.6 in either beside the shared expert's products; 2,048 rows 6.3 and 13.2, 4,096 8.7
+//   and 22.7 (the same bits).
 bool gemm_skinny_rows_takes(const GemmArgs& a) {
   if (a.offsets || a.a_index || a.c_index || a.groups > 1 || a.force_kernel || a.in_dtype != kBF16 || a.M <= 16 || a.K % 128 || a.lda % 8 || (uintptr_t)a.A % 16 || (uintptr_t)a.W % 16)
     return false;
   const bool gated = epilogue_gated(a.epilogue);
   const int64_t w_rows = (int64_t)a.N * (gated ? 2 : 1);
   if (a.M <= 32) return w_rows > (gated ? 4096 : 2560);
-  if (a.N <= 128) return !gated && a.M > 64;
+  if (a.N <= 128) return !gated && a.M > kRowsMax;
   return a.M <= kRowsMax && w_rows * rows_parts(a) <= (gated ? 24576 : a.M <= 128 ? 16384 : 8192);
 }
 
