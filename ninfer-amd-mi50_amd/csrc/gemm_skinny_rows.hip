@@ -1,4 +1,4 @@
-// C = A W^T (+ bias, an activation, or gated) for a dense product of 17 to 512 rows (any number for a router's few features): too many for a block that owns
+// C = A W^T (+ bias, an activation, or gated) for a dense product of 17 to 512 rows (more than that for a router's few features): too many for a block that owns
 // all of them, too few to pay for the tiles of the many-row kernel.
 //
 // A block owns 32 rows of A and up to 32 rows of W: two sets of up to 16 (of a gated product a set of the gate's and

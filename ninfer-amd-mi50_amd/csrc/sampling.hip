@@ -688,7 +688,7 @@ __global__ __launch_bounds__(kCandThreads) void sample_few_kernel(
 using namespace ninfer;
 
 // out[i] <- a number in [0, 1) of 24 random bits from (seeds[i], keys[i], draws[i]), on the host: sampling/sampler.py's
-// `uniform`. Whole arrays in numpy took 44 us for 64 rows, 27 passes over each; here 1.
+// `uniform`. 64 rows as whole arrays in numpy took 44 us, 27 passes; here 5 and 14 for the arrays.
 extern "C" void ninfer_uniforms(const unsigned long long* seeds, const unsigned long long* keys,
                                 const unsigned long long* draws, int n, float* out) {
   auto mix = [](unsigned long long x) {   // splitmix64's step and finalizer
