@@ -196,6 +196,25 @@ def test_decode_rows_with_a_sink_and_a_gate(ops, n_q, n_kv, d, window, sink, lea
         assert ((outs[0] - outs[1]).norm() / outs[1].norm()).item() < 8e-3
 
 
+@pytest.mark.parametrize("n_q,n_kv,d", [(16, 4, 128), (8, 2, 64), (12, 1, 128)])
+@pytest.mark.parametrize("keys", [65, 500, 1300])
+@pytest.mark.parametrize("sink", [False, True])
+def test_decode_rows_of_one_key_give_its_value(ops, n_q, n_kv, d, keys, sink):
+    """Single rows of grouped heads, one key far above the others (by 40 and more: all else is lost in 32 bits): its
+    value, bit for bit, as its probability is not rounded apart from the sum that divides it."""
+    seqs = [(keys - 1 - i, 1) for i in range(5)]
+    ctx, qkv, k_pool, v_pool, bt, perm = shared_stream_case(seqs, n_q, n_kv, d, 16, torch.bfloat16)
+    ctx.single_rows = 5
+    key = keys // 2
+    for row in range(5):
+        place_dominant_key(qkv, k_pool, perm, row, key, n_q, n_kv, d, 16, torch.bfloat16)
+    qkv.copy_((qkv.float() * 0.9).bfloat16())
+    out = torch.full((5, n_q * d), float("nan"), device="cuda", dtype=torch.bfloat16)
+    ops.paged_attention(qkv, k_pool, v_pool, bt, ctx, n_q, n_kv, d, 16, 0, 1 / math.sqrt(d), out, sink=sink)
+    want = v_pool[int(perm[key // 16]), :, key % 16].repeat_interleave(n_q // n_kv, 0).reshape(1, -1)
+    assert torch.equal(out, want.expand(5, -1))
+
+
 @pytest.mark.parametrize("n_q,n_kv,d,vdim", [(16, 16, 128, 128), (8, 2, 64, 128), (4, 1, 100, 36), (3, 3, 4, 8)])
 @pytest.mark.parametrize("window,ps", [(0, 16), (70, 8), (1, 4)])
 @pytest.mark.parametrize("extras", ["", "slopes", "sink", "sinks gate"])
