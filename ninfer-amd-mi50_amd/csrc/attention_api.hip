@@ -35,23 +35,31 @@ int attention_check(const AttnArgs& args) {
 }
 }  // namespace ninfer
 
+// The step's single rows (which come first; all rows of a step without prompt portions) as a step of their own.
+static AttnArgs single_rows_of(const AttnArgs& a) {
+  AttnArgs d = a;
+  if (a.max_qlen > 1) d.T = d.S = a.single_rows;
+  d.max_qlen = 1;
+  return d;
+}
+
+// Do the single rows `d` of step `a` walk their contexts split over many blocks? By their own number, never the
+// step's: its portions have no part in that, nor in the workspace.
+static bool single_rows_split(const AttnArgs& a, const AttnArgs& d) {
+  return d.S > 0 && (a.max_qlen == 1 || (d.S < a.S && attention_prefill_takes(a))) && attention_decode_takes(d);
+}
+
 // force_generic != 0 runs the plain one-wave-per-(row, head) kernel whatever
 // the shape (tests compare the fast kernels with it).
 extern "C" int ninfer_paged_attention(const AttnArgs* a, int force_generic, hipStream_t stream) {
   if (int rc = attention_check(*a)) return rc;
-  if (!force_generic && a->max_qlen == 1 && attention_decode_takes(*a))
-    return attention_decode(*a, stream);
-  if (!force_generic && a->single_rows > 0 && a->single_rows < a->S &&
-      attention_decode_takes(*a) && attention_prefill_takes(*a)) {
-    // A step that mixes decoded tokens with prompt portions: the single rows, which come
-    // first, walk their contexts split over many blocks; in the prompt kernel each would be
-    // one block that walks its whole context alone.
-    const int n = a->single_rows;
-    AttnArgs d = *a;
-    d.T = n;
-    d.S = n;
-    d.max_qlen = 1;
+  const AttnArgs d = single_rows_of(*a);
+  const int n = d.S;
+  if (!force_generic && single_rows_split(*a, d)) {
     if (int rc = attention_decode(d, stream)) return rc;
+    if (a->max_qlen == 1) return 0;
+    // A step that mixes decoded tokens with prompt portions: in the prompt kernel each single
+    // row would be one block that walks its whole context alone.
     AttnArgs p = *a;   // rows and their positions stay where they are: only the requests move
     p.seq_row_start += n;
     p.seq_qlen += n;
@@ -61,17 +69,12 @@ extern "C" int ninfer_paged_attention(const AttnArgs* a, int force_generic, hipS
     p.T = a->T - n;
     return attention_prefill(p, stream);
   }
-  // single rows (which come first) of layers with values of another size, a sink, blocks or a
-  // gate: the heads of a kv head as a tile's rows
-  const int n = a->max_qlen == 1 ? a->S : a->single_rows;
+  // single rows of layers with values of another size or blocks, or with a sink or a gate where
+  // they are not split: the heads of a kv head as a tile's rows
   const bool tiles = !force_generic && attention_tiles_takes(*a);
   const bool apart = tiles && n > 0 && attention_tiles_heads_takes(*a) &&
                      (!attention_prefill_takes(*a) || a->kblk || a->gate || a->sink);
   if (apart) {
-    AttnArgs d = *a;
-    d.T = n;
-    d.S = n;
-    d.max_qlen = 1;
     if (int rc = attention_tiles_heads(d, stream)) return rc;
     if (n == a->S) return 0;
   }
@@ -90,13 +93,8 @@ extern "C" int ninfer_paged_attention(const AttnArgs* a, int force_generic, hipS
   // ... and prompt portions of any such shape on the matrix cores
   if (tiles) return attention_tiles(*a, apart ? n : 0, stream);
   if (!force_generic && n < a->S && attention_rows_f32_takes(*a)) {
-    if (n > 0) {
-      AttnArgs d = *a;
-      d.T = n;
-      d.S = n;
-      d.max_qlen = 1;
+    if (n > 0)
       if (int rc = attention_generic(d, stream)) return rc;
-    }
     AttnArgs p = *a;
     p.seq_row_start += n;
     p.block_table += (int64_t)n * a->bt_stride;
@@ -112,17 +110,18 @@ extern "C" long long ninfer_attention_workspace_floats(int T, int Hq, int D, int
   return attention_decode_workspace_floats(T, Hq, D, max_kv_len);
 }
 
-// How a step of single-token rows would run (nothing is launched): kernel 0 = the plain
-// kernel, 1 = split contexts on scalar FMAs, 2 = split contexts on the matrix cores (grouped
+// How a step's single rows would run (nothing is launched): kernel 0 = another (the plain one, the prompts', or the
+// tiles of attention_tiles.hip), 1 = split contexts on scalar FMAs, 2 = split contexts on the matrix cores (grouped
 // heads); the keys per chunk and the number of chunks the merge kernel adds up. Tests name
 // the kernel variant they mean to reach with it.
 extern "C" int ninfer_attention_decode_plan(const AttnArgs* a, int* kernel, int* chunk, int* n_chunks) {
   *kernel = 0;
   *chunk = *n_chunks = 0;
   if (int rc = attention_check(*a)) return rc;
-  if (!attention_decode_takes(*a)) return 0;
+  const AttnArgs d = single_rows_of(*a);
+  if (!single_rows_split(*a, d)) return 0;
   bool heads;
-  attention_decode_plan(*a, &heads, chunk, n_chunks);
+  attention_decode_plan(d, &heads, chunk, n_chunks);
   *kernel = heads ? 2 : 1;
   return 0;
 }

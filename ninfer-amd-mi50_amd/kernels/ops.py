@@ -1066,19 +1066,12 @@ class HipOps:
         single = int(getattr(ctx, "single_rows", 0))
         if (ctx.max_qlen == 1 or single > 0) and qkv.dtype == torch.bfloat16 \
                 and not self.force_generic:
+            # (two chunks more than the split-context kernels need, for a window that starts inside a tile and
+            # blocks before it. The call is told what its own sizes ask for, never how much is there:
+            # its kernel and its chunks are to depend on nothing that ran before)
             ws_floats = int(self.lib.ninfer_attention_workspace_floats(
-                t if ctx.max_qlen == 1 else single, n_q, max(head_dim, vdim), ctx.max_kv_len))
-            if self._attn_ws is None or self._attn_ws.numel() < ws_floats:
-                # A captured graph may hold the address of the workspace it was recorded
-                # with: an outgrown one is kept, never given back (a replay would write
-                # into whatever took its place), and growth at least doubles, which bounds
-                # what is kept to the size of the largest.
-                if self._attn_ws is not None:
-                    self._outgrown.append(self._attn_ws)
-                    ws_floats = max(ws_floats, 2 * self._attn_ws.numel())
-                self._attn_ws = torch.empty(ws_floats, dtype=torch.float32, device=qkv.device)
-            ws_floats = self._attn_ws.numel()
-            ws = self._attn_ws.data_ptr()
+                t if ctx.max_qlen == 1 else single, n_q, max(head_dim, vdim), ctx.max_kv_len + 256))
+            ws = self._workspace(ws_floats, qkv.device).data_ptr()
         args = _AttnArgs(
             qkv.data_ptr(), k_pool.data_ptr(), v_pool.data_ptr(), out.data_ptr(),
             block_table.data_ptr(), ctx.positions.data_ptr(), ctx.row_seq.data_ptr(),

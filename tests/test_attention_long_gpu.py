@@ -196,6 +196,29 @@ def test_decode_rows_with_a_sink_and_a_gate(ops, n_q, n_kv, d, window, sink, lea
         assert ((outs[0] - outs[1]).norm() / outs[1].norm()).item() < 8e-3
 
 
+@pytest.mark.parametrize("d,vdim", [(128, 128), (128, 64)])
+@pytest.mark.parametrize("prompt", [0, 90])
+def test_rows_with_a_sink_have_the_same_bits_whatever_ran_before(ops, d, vdim, prompt):
+    """Kernel and chunks of a step's single rows go by the step's own sizes, not by how large a workspace earlier
+    steps have left."""
+    n_q, n_kv, ps = 16, 4, 16
+    seqs = [(1400 - 3 * i, 1) for i in range(5)] + [(0, prompt)] * (prompt > 0)
+    ctx, qkv, k_pool, v_pool, bt, perm = shared_stream_case(seqs, n_q, n_kv, d, ps, torch.bfloat16)
+    ctx.single_rows, v_pool = 5, v_pool[..., :vdim].contiguous()
+    outs = []
+    for before in (0, 1 << 24):
+        new = type(ops)(ops.lib_path)
+        if before:
+            new._workspace(before, qkv.device)
+        out = torch.full((ctx.T, n_q * vdim), float("nan"), device="cuda", dtype=torch.bfloat16)
+        kw = dict(sink=True, vdim=vdim)
+        plan = new.paged_attention(qkv, k_pool, v_pool, bt, ctx, n_q, n_kv, d, ps, 0, 0.1, out, plan_only=True, **kw)
+        assert plan["kernel"] == ("heads" if vdim == d else "plain")
+        new.paged_attention(qkv, k_pool, v_pool, bt, ctx, n_q, n_kv, d, ps, 0, 0.1, out, **kw)
+        outs.append(out)
+    assert torch.isfinite(outs[0]).all() and torch.equal(outs[0], outs[1])
+
+
 @pytest.mark.parametrize("n_q,n_kv,d", [(16, 4, 128), (8, 2, 64), (12, 1, 128)])
 @pytest.mark.parametrize("keys", [65, 500, 1300])
 @pytest.mark.parametrize("sink", [False, True])

@@ -130,6 +130,29 @@ def test_large_operands_keep_the_many_row_kernel(lib, m, n, k, gated, indexed, r
     assert lib.ninfer_gemm_kernel(ctypes.byref(args)) == 4
 
 
+def _attention(rows, keys, n_q, n_kv, d, prompt=0, window=0, page=16, **more):
+    """The arguments of `rows` single rows (and a prompt's), with the workspace that the single rows ask for."""
+    from ninfer_amd.kernels.ops import _AttnArgs
+    floats = rows * n_q * (-(-keys // 128)) * (d + 2)
+    return _AttnArgs(q=16, kpool=16, vpool=16, out=16, block_table=16, positions=16, row_seq=16, seq_row_start=16, seq_qlen=16,
+                     seq_pos0=16, workspace=16, workspace_floats=floats, q_stride=(n_q + 2 * n_kv) * d, bt_stride=999,
+                     T=rows + prompt, S=rows + (prompt > 0), Hq=n_q, Hkv=n_kv, D=d, page_size=page, window=window, scale=1.0,
+                     dtype=BF16, max_qlen=max(1, prompt), max_kv_len=max(keys, prompt), single_rows=rows, **more)
+
+
+def _single_rows_plan(lib, a):
+    got = [ctypes.c_int() for _ in range(3)]
+    assert lib.ninfer_attention_decode_plan(ctypes.byref(a), *map(ctypes.byref, got)) == 0
+    return [v.value for v in got]   # kernel (1 scalar, 2 grouped heads, 0 another), keys a chunk, chunks
+
+
+@pytest.mark.parametrize("more", [{}, {"sink": 1}, {"gate": 16, "gate_stride": 2048}])
+@pytest.mark.parametrize("prompt", [2, 1100])
+def test_single_rows_beside_a_prompt_run_as_they_would_alone(lib, prompt, more):
+    alone = _single_rows_plan(lib, _attention(16, 1500, 16, 4, 128, **more))
+    assert alone[0] == 2 and _single_rows_plan(lib, _attention(16, 1500, 16, 4, 128, prompt, **more)) == alone
+
+
 # (prompts of their own, portions behind cached keys and decode steps; both heights of blocks measured)
 @pytest.mark.parametrize("rank,rd,heads,requests,new,keys,rows", [
     (256, 32, 40, 1, 200, 200, 16), (512, 64, 16, 1, 300, 300, 16), (256, 32, 24, 1, 300, 300, 16),
