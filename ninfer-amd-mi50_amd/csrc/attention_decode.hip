@@ -315,6 +315,9 @@ static void launch_decode_chunk(const AttnArgs& a, int chunk, int n_chunks, hipS
     launch_decode<LPK, 256>(a, n_chunks, stream);
 }
 
+// Two chunks of which the second is short: the blocks of the first decide, with half the device idle behind them.
+static bool uneven(const AttnArgs& a, int chunk) { return a.max_kv_len > chunk && 2 * a.max_kv_len < 3 * chunk; }
+
 // Which pass-1 kernel a decode step runs and how it cuts the contexts: the matrix-core
 // kernel for grouped heads (`heads`) or the scalar one, chunks of `chunk` keys.
 void attention_decode_plan(const AttnArgs& a, bool* heads, int* chunk, int* n_chunks) {
@@ -322,14 +325,22 @@ void attention_decode_plan(const AttnArgs& a, bool* heads, int* chunk, int* n_ch
   *chunk = decode_chunk(a.T, a.Hkv, a.max_kv_len);
   if (*heads) {
     // the matrix-core kernel has a start-up of several tiles: the largest chunk that still
-    // gives the CUs one and a half blocks (of two places each; 4 kv heads of 128, 16 rows at 1,500 keys:
-    // 384 blocks of 256 keys 16.0 us, 768 of 128 19.7; 32 rows at 1,200: 384 of 512 21.5, 640 of 256 23.7)
+    // gives every CU two blocks, or, where all chunks of a context are seen, one and a half: with heads of 128 (4 kv
+    // heads, us: 16 rows at 1,500 keys 384 blocks of 256 keys 14.3, 768 of 128 17.0; 32 rows at 2,600 384 of 1,024 31,
+    // 768 of 512 36) unless they are two chunks of 512 and more, the second a short one (48 rows at 1,200 keys 33
+    // against 27); with heads of 64, whose chunks take half as long beside the same start, only of long contexts'
+    // smallest (8 kv heads, 3 rows at 5,000 keys 11.5 against 12.3; but 16 rows at 1,200 keys in chunks of 512 13.7
+    // against 12.0). Not in a window, which leaves most of them without work (16 rows at 6,000 keys, a window of
+    // 1,024, 29 against 24)
+    const bool windowed = a.window > 0 && a.window < a.max_kv_len;
     *chunk = 128;
-    for (int c = 1024; c > 128; c /= 2)
-      if (2L * a.T * a.Hkv * ((a.max_kv_len + c - 1) / c) >= 3L * device_cu_count()) {
+    for (int c = 1024; c > 128; c /= 2) {
+      const bool full = !windowed && (a.D == 128 ? c < 512 || !uneven(a, c) : c == 256 && a.max_kv_len >= 3000);
+      if (2L * a.T * a.Hkv * ((a.max_kv_len + c - 1) / c) >= (full ? 3L : 4L) * device_cu_count()) {
         *chunk = c;
         break;
       }
+    }
   }
   *n_chunks = (a.max_kv_len + *chunk - 1) / *chunk;
 }

@@ -153,6 +153,18 @@ def test_single_rows_beside_a_prompt_run_as_they_would_alone(lib, prompt, more):
     assert alone[0] == 2 and _single_rows_plan(lib, _attention(16, 1500, 16, 4, 128, prompt, **more)) == alone
 
 
+# (heads of 128 from one and a half blocks a CU on, but not in two uneven chunks nor in a window; heads of 64 from two on
+# but for long contexts' smallest)
+@pytest.mark.parametrize("rows,keys,n_q,n_kv,d,window,chunk", [
+    (16, 1500, 16, 4, 128, 0, 256), (16, 1500, 16, 4, 128, 1500, 256), (16, 1500, 16, 4, 128, 1499, 128),
+    (16, 6000, 16, 4, 128, 1024, 512), (16, 6000, 16, 4, 128, 0, 1024), (48, 1200, 16, 4, 128, 0, 512),
+    (48, 1535, 16, 4, 128, 0, 512), (48, 1536, 16, 4, 128, 0, 1024), (48, 600, 28, 4, 128, 0, 256),
+    (48, 300, 16, 4, 128, 0, 256), (16, 1200, 32, 8, 64, 0, 256), (48, 1200, 12, 4, 64, 0, 512),
+    (64, 2600, 16, 4, 128, 1024, 1024), (3, 5000, 64, 8, 64, 0, 256), (3, 5000, 64, 8, 64, 4000, 128), (8, 2999, 32, 4, 64, 0, 128), (8, 3000, 32, 4, 64, 0, 256)])
+def test_chunks_of_grouped_heads(lib, rows, keys, n_q, n_kv, d, window, chunk):
+    assert _single_rows_plan(lib, _attention(rows, keys, n_q, n_kv, d, window=window)) == [2, chunk, -(-keys // chunk)]
+
+
 # (prompts of their own, portions behind cached keys and decode steps; both heights of blocks measured)
 @pytest.mark.parametrize("rank,rd,heads,requests,new,keys,rows", [
     (256, 32, 40, 1, 200, 200, 16), (512, 64, 16, 1, 300, 300, 16), (256, 32, 24, 1, 300, 300, 16),
