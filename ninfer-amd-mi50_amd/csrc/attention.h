@@ -78,6 +78,7 @@ int attention_rows_f32(const AttnArgs& a, hipStream_t stream);
 
 int64_t attention_decode_workspace_floats(int T, int Hq, int D, int max_kv_len);
 bool attention_decode_takes(const AttnArgs& a);
+bool attention_decode_pays(const AttnArgs& a);      // ... and are they the faster ones (rows with a sink or a gate)
 int attention_decode(const AttnArgs& a, hipStream_t stream);
 void attention_decode_plan(const AttnArgs& a, bool* heads, int* chunk, int* n_chunks);
 bool attention_decode_heads_takes(const AttnArgs& a);

@@ -46,7 +46,8 @@ static AttnArgs single_rows_of(const AttnArgs& a) {
 // Do the single rows `d` of step `a` walk their contexts split over many blocks? By their own number, never the
 // step's: its portions have no part in that, nor in the workspace.
 static bool single_rows_split(const AttnArgs& a, const AttnArgs& d) {
-  return d.S > 0 && (a.max_qlen == 1 || (d.S < a.S && attention_prefill_takes(a))) && attention_decode_takes(d);
+  return d.S > 0 && (a.max_qlen == 1 || (d.S < a.S && attention_prefill_takes(a))) &&
+         attention_decode_takes(d) && attention_decode_pays(d);
 }
 
 // force_generic != 0 runs the plain one-wave-per-(row, head) kernel whatever

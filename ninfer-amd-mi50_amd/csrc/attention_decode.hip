@@ -345,6 +345,58 @@ void attention_decode_plan(const AttnArgs& a, bool* heads, int* chunk, int* n_ch
   *n_chunks = (a.max_kv_len + *chunk - 1) / *chunk;
 }
 
+// Rows with a sink or a gate: these kernels, or those of attention_tiles.hip? The latter cut what a row sees
+// evenly, read its keys once for all heads of a kv head whatever the sizes, and need no merge while a row's keys are one
+// chunk; these cut at absolute positions and launch a block for every chunk of a context, also for those that a window
+// has passed. us there and here, r = kv heads of all rows:
+// - grouped heads of 128: 200 to 12,000 keys, r 4 to 512, 15 to 211 and 9.6 to 167; 64 keys, r 1,024, 15 and 35. In windows
+//   while a chunk is less than one (1,024 keys at 5,000, r 16 17 and 11) or the context not much more than one (at 2,560,
+//   r 256, 39 and 35; at 3,584 39 and 53; at 1,331, a full chunk and a short one, 39 and 42).
+// - grouped heads of 64: 600 keys r 128 14 and 13, r 256 15 and 17; 2,600 r 512 60 and 59. In windows in chunks of a quarter of
+//   them (1,024 keys at 3,072, r 64, 12 and 10.5; r 128, chunks of 512, 15 and 15.5).
+// - one query head to a kv head: 600 keys r 512 22 and 18, r 1,024 29 and 30 (heads of 128 65 and 51). In windows of 1,024 at
+//   2,048, r 256, 21 and 18, but at 16,384, r 128, 14 and 15.5. Heads of 32: at 2,048, r 64, 9.4 and 8.8, r 128 11 and 11.7.
+// - two query heads: heads of 128, r 256, at 600 keys 27 and 25; heads of 64 only the fewest of rows (12,000 keys, r 8, 16
+//   and 12; r 64 as long). More, where the matrix cores don't take them (small heads or pages): 2 kv heads of 12 at 4,000
+//   keys, 64 rows, 22 and 113; never.
+// - heads of 256 have only the plain kernel there: 1,000 keys 210 and 29, 64 keys 16 and 25.
+bool attention_decode_pays(const AttnArgs& a) {
+  if (!a.sink && !a.gate) return true;
+  const int group = a.Hq / a.Hkv;
+  const int64_t keys = a.max_kv_len, r = (int64_t)a.T * a.Hkv, cus = device_cu_count();
+  const bool windowed = a.window > 0 && a.window < keys;
+  if (!attention_tiles_heads_takes(a)) {   // (the plain kernel, or the prompts')
+    if (attention_tiles_takes(a) || attention_prefill_takes(a)) return false;
+    return keys > 64 && !(windowed && keys > (group > 2 ? 5LL : 8LL) * a.window && a.T > 64);
+  }
+  bool heads;
+  int chunk, n_chunks;
+  attention_decode_plan(a, &heads, &chunk, &n_chunks);
+  if (heads && windowed) {
+    if (a.D == 128)
+      return chunk <= 512 || (n_chunks == 1 && r <= 2 * cus) ||
+             (keys <= 3LL * a.window && !uneven(a, chunk) && 1024 * r <= cus * a.window);
+    if (chunk == 128) return r <= cus / 2;
+    return chunk == 256 ? 4 * chunk <= a.window : 8 * chunk <= a.window && keys <= 5LL * a.window;
+  }
+  if (heads) {
+    if (a.D == 128) return r < 4 * cus || keys >= 1024;
+    return (r <= cus / 2 && keys >= 100) || (r <= cus && keys >= 900 && !uneven(a, chunk)) || keys >= 2600;
+  }
+  if (a.D == 128) {
+    if (group > 2) return false;
+    if (group == 1) return !windowed || r <= 2 * cus || keys <= 5LL * a.window || a.window >= 1024;
+    return windowed ? r <= cus / 8 || (r <= cus && keys <= 5LL * a.window) : r <= 2 * cus || keys >= 1024;
+  }
+  if (group > 1) return group == 2 && a.D == 64 && r <= cus / 16 && keys >= 1300;
+  if (!windowed) return (r <= 2 * cus && keys >= 100) || keys >= 1300;
+  // (where a row's blocks are whole rounds of the CUs, those that have keys meet on the same ones in every row: 4,000
+  // keys, r 64, 9.1 and 11.2; at 3,584 8.9 and 8.3)
+  if (r <= cus / 16) return true;
+  return keys <= 5LL * a.window &&
+         (a.window >= 4096 || (r <= (a.D == 64 ? cus : cus / 4) && (int64_t)a.Hkv * n_chunks % cus != 0));
+}
+
 int attention_decode(const AttnArgs& a, hipStream_t stream) {
   bool heads;
   int chunk, n_chunks;

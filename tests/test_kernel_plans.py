@@ -165,6 +165,28 @@ def test_chunks_of_grouped_heads(lib, rows, keys, n_q, n_kv, d, window, chunk):
     assert _single_rows_plan(lib, _attention(rows, keys, n_q, n_kv, d, window=window)) == [2, chunk, -(-keys // chunk)]
 
 
+# (kernel 0: the tiles of heads. Sizes on both sides of the rule's lines, and some far from them)
+@pytest.mark.parametrize("rows,keys,n_q,n_kv,d,window,page,kernel", [
+    (16, 1500, 16, 4, 128, 0, 16, 2), (128, 64, 64, 8, 128, 0, 16, 0), (128, 1024, 64, 8, 128, 0, 16, 2),
+    (64, 2560, 16, 4, 128, 1024, 16, 2), (64, 3584, 16, 4, 128, 1024, 16, 0), (64, 1331, 16, 4, 128, 1024, 16, 0),
+    (65, 2560, 16, 4, 128, 1024, 16, 0), (4, 5000, 16, 4, 128, 1024, 16, 2), (128, 512, 16, 4, 128, 256, 16, 2),
+    (16, 600, 32, 8, 64, 0, 16, 2), (32, 600, 32, 8, 64, 0, 16, 0), (32, 900, 32, 8, 64, 0, 16, 2), (64, 2600, 32, 8, 64, 0, 16, 2),
+    (8, 3072, 32, 8, 64, 1024, 16, 2), (16, 3072, 32, 8, 64, 1024, 16, 0), (16, 600, 32, 8, 64, 256, 16, 2),
+    (4, 1000, 32, 8, 64, 0, 4, 0), (64, 600, 8, 8, 64, 0, 16, 1), (128, 600, 8, 8, 64, 0, 16, 0),
+    (128, 600, 8, 8, 128, 0, 16, 1), (32, 600, 16, 8, 128, 0, 16, 1), (128, 600, 16, 8, 128, 0, 16, 0),
+    (1, 12000, 16, 8, 64, 0, 16, 1), (8, 12000, 16, 8, 64, 0, 16, 0), (32, 2048, 8, 8, 64, 1024, 16, 1),
+    (32, 16384, 8, 8, 64, 1024, 16, 0), (4, 1900, 16, 16, 32, 1024, 16, 1), (8, 1900, 16, 16, 32, 1024, 16, 0),
+    (8, 4000, 8, 8, 16, 1024, 16, 0), (64, 8192, 8, 8, 16, 4096, 16, 1), (16, 100, 32, 8, 64, 0, 16, 2), (16, 99, 32, 8, 64, 0, 16, 0), (8, 3584, 8, 8, 16, 1024, 16, 1), (4, 4000, 24, 2, 32, 0, 16, 0),
+    (4, 4000, 8, 4, 32, 0, 16, 0), (4, 64, 8, 1, 256, 0, 16, 0), (4, 65, 8, 1, 256, 0, 16, 1), (1, 300, 64, 1, 128, 0, 16, 0)])
+@pytest.mark.parametrize("more", [{"sink": 1}, {"gate": 16}])
+def test_which_rows_with_a_sink_or_a_gate_are_split(lib, rows, keys, n_q, n_kv, d, window, page, kernel, more):
+    more = dict(more, gate_stride=n_q * d) if "gate" in more else more
+    a = _attention(rows, keys, n_q, n_kv, d, window=window, page=page, **more)
+    assert _single_rows_plan(lib, a)[0] == kernel
+    plain = _attention(rows, keys, n_q, n_kv, d, window=window, page=page)
+    assert _single_rows_plan(lib, plain)[0] != 0   # (plain layers' always are)
+
+
 # (prompts of their own, portions behind cached keys and decode steps; both heights of blocks measured)
 @pytest.mark.parametrize("rank,rd,heads,requests,new,keys,rows", [
     (256, 32, 40, 1, 200, 200, 16), (512, 64, 16, 1, 300, 300, 16), (256, 32, 24, 1, 300, 300, 16),
