@@ -48,6 +48,7 @@ extern "C" int ninfer_decode_attention_static(const AttnArgs* args, hipStream_t 
   NINFER_REQUIRE(a.max_qlen == 1 && a.T == a.S, "decode_attention_static: single-token rows only "
                  "(%d rows of %d requests, longest %d)", a.T, a.S, a.max_qlen);
   NINFER_REQUIRE(a.dtype == kBF16, "decode_attention_static: bf16 only");
+  NINFER_REQUIRE(!a.sink && !a.gate, "decode_attention_static: a sink or a gate on the output is not built");
   const long long need = attention_decode_workspace_floats(a.T, a.Hq, a.D, a.max_kv_len);
   NINFER_REQUIRE(need <= kScratchFloats, "decode_attention_static: %d rows of %d heads over %d keys "
                  "need %lld floats of workspace; the fixed one holds %lld", a.T, a.Hq, a.max_kv_len,

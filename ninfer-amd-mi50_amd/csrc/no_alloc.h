@@ -11,7 +11,8 @@
 // Limits and rules:
 //  - single-token rows only (max_qlen == 1), bf16, the shapes the split-context
 //    kernels take (head sizes 16, 32, 64, 128, 256, a page size that is a power
-//    of two); anything else is refused with an error, never run another way;
+//    of two), without a sink or a gate on the output; anything else is refused with an
+//    error, never run another way;
 //  - T * Hq * ceil(max_kv_len / 128) * (D + 2) floats must fit in
 //    ninfer_decode_attention_static_max_floats() (4 Mi floats = 16 MiB, which
 //    every GPU the library runs on holds until the process ends): 8 rows of 16

@@ -165,6 +165,13 @@ def test_chunks_of_grouped_heads(lib, rows, keys, n_q, n_kv, d, window, chunk):
     assert _single_rows_plan(lib, _attention(rows, keys, n_q, n_kv, d, window=window)) == [2, chunk, -(-keys // chunk)]
 
 
+def test_attention_without_allocation_refuses_sinks_and_gates(lib):
+    lib.ninfer_last_error.restype = ctypes.c_char_p
+    for more in ({"sink": 1}, {"gate": 16, "gate_stride": 2048}):
+        assert lib.ninfer_decode_attention_static(ctypes.byref(_attention(2, 300, 16, 4, 128, **more)), None) != 0
+        assert b"sink" in lib.ninfer_last_error()
+
+
 # (kernel 0: the tiles of heads. Sizes on both sides of the rule's lines, and some far from them)
 @pytest.mark.parametrize("rows,keys,n_q,n_kv,d,window,page,kernel", [
     (16, 1500, 16, 4, 128, 0, 16, 2), (128, 64, 64, 8, 128, 0, 16, 0), (128, 1024, 64, 8, 128, 0, 16, 2),
