@@ -93,18 +93,12 @@ extern "C" int ninfer_paged_attention(const AttnArgs* a, int force_generic, hipS
   }
   // ... and prompt portions of any such shape on the matrix cores
   if (tiles) return attention_tiles(*a, apart ? n : 0, stream);
-  if (!force_generic && n < a->S && attention_rows_f32_takes(*a)) {
-    if (n > 0)
-      if (int rc = attention_generic(d, stream)) return rc;
-    AttnArgs p = *a;
-    p.seq_row_start += n;
-    p.block_table += (int64_t)n * a->bt_stride;
-    p.S = a->S - n;
-    p.T = a->T - n;
-    return attention_rows_f32(p, stream);
-  }
+  if (!force_generic && attention_rows_f32_takes(*a)) return attention_rows_f32(*a, stream);
   return attention_generic(*a, stream);
 }
+
+// Does a 32-bit step of this shape run eight rows of a request to a block?
+extern "C" int ninfer_attention_rows_f32_takes(const AttnArgs* a) { return attention_rows_f32_takes(*a); }
 
 // 32-bit floats of workspace the split-KV decode kernel needs for this shape.
 extern "C" long long ninfer_attention_workspace_floats(int T, int Hq, int D, int max_kv_len) {

@@ -9,7 +9,7 @@
 // What bounds the plain kernel is that its lanes each walk a key's row of their own through L1, once per row; here a
 // tile's chain of some 1,100 instructions a wave, 4.3 us for two rows. us there and here, 16 heads of 128: a prompt of
 // 173 tokens 39 and 24, of 600 250 and 110, of 2,048 2,420 and 850; 64 rows behind 2,000 keys 360 and 148, 2 rows of four
-// requests 321 and 140. Within one tile of keys the plain kernel (16 tokens 8.1 and 9.4); single rows too.
+// requests 321 and 140. Within one tile of keys the plain kernel (16 tokens 8.1 and 9.4).
 #include "attention.h"
 #include "gemm.h"
 #include <type_traits>
@@ -223,11 +223,25 @@ __global__ __launch_bounds__(256) void attention_rows_f32_kernel(AttnArgs a) {
   }
 }
 
-// Keys and values of up to 128 numbers in whole pieces of 16 bytes, no blocks before the window.
+// Keys and values of up to 128 numbers in whole pieces of 16 bytes, no blocks before the window; and steps whose
+// requests bring blocks enough rows, so that these pay for their start (some 5 us, one block to a CU) beside the plain
+// kernel's waves, one a row. Single rows of such a step share the launch. us there and here:
+// - heads of more than 64: 16 heads, 7 rows at 2,500 keys beside 505 new ones 425 and 190; 16 requests of 2 rows at 66 keys 18
+//   and 14; 63 rows at 200 keys beside 17 of a prompt 50 and 59 (45 and 59 on 4 kv heads), beside 2,048 2,430 and 880. Sizes
+//   that fill no whole pieces of 128 bytes: 32 heads of 100, 16 requests of 2 rows 19 and 24, of 5 rows 38 and 33.
+// - of 33 to 64: 8 heads, 505 rows 77 and 46 (39 and 27 in a window of 200), 64 requests of 8 rows at 300 keys 91 and 38,
+//   but of 40 of 100 rows 83 and 90, 600 rows in a window of 70 22 and 27; 64 rows at 2,000 keys 193 and 133, 9 at 500 35
+//   and 39, 17 beside a single row at 2,000 127 and 142. Smaller ones: 600 rows of 16 heads 80 and 86.
 bool attention_rows_f32_takes(const AttnArgs& a) {
-  const int dv = a.Dv > 0 ? a.Dv : a.D;
-  return a.dtype == kF32 && a.max_qlen > 1 && a.max_kv_len > kRowsKeys && !a.kblk && !a.krot && a.seq_row_start && a.D % 4 == 0 && dv % 4 == 0 &&
-         a.D <= 128 && dv <= 128 && ((uintptr_t)a.kpool | (uintptr_t)a.vpool) % 16 == 0;
+  const int dv = a.Dv > 0 ? a.Dv : a.D, most = max(a.D, dv);
+  if (a.dtype != kF32 || a.max_qlen <= 1 || a.max_kv_len <= kRowsKeys || a.kblk || a.krot || !a.seq_row_start || a.D % 4 || dv % 4 ||
+      most > 128 || most <= 32 || ((uintptr_t)a.kpool | (uintptr_t)a.vpool) % 16)
+    return false;
+  const long blocks = (long)a.S * a.Hq, cus = device_cu_count();   // (one a request and head at the least)
+  if (most > 64) return a.D % 32 || dv % 32 ? blocks <= cus || a.T >= 8L * a.S : blocks <= 2 * cus || a.T >= 4L * a.S;
+  const bool windowed = a.window > 0 && a.window < a.max_kv_len;
+  if (a.T >= 256 && a.T >= (a.single_rows > 0 ? 16L : 8L) * a.S && a.max_kv_len >= 200) return !windowed || a.window >= 128;
+  return !windowed && a.single_rows == 0 && a.max_kv_len >= 1000 && a.T >= 32L * a.S && blocks <= cus;
 }
 
 static size_t rows_lds(int D, int Dv) {

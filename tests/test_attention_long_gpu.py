@@ -273,6 +273,26 @@ def test_prompt_rows_in_32_bit_bit_for_bit_as_the_plain_kernel(ops, n_q, n_kv, d
         assert torch.isfinite(outs[0]).all() and torch.equal(outs[0], outs[1])
 
 
+@pytest.mark.parametrize("n_q,n_kv,d,vdim", [(8, 8, 64, 64), (4, 2, 40, 64), (2, 1, 60, 36), (16, 4, 128, 128)])
+@pytest.mark.parametrize("window", [0, 70])
+def test_single_rows_beside_prompts_in_32_bit_bit_for_bit_as_the_plain_kernel(ops, n_q, n_kv, d, vdim, window):
+    """Single rows in the launch of the portions, heads of up to 64 among them: the same bits as one wave per row and
+    head; a row's are the same whether its request is announced as a single row or not."""
+    seqs = [(127, 1), (640, 1), (0, 1), (0, 173), (60, 9), (300, 200)]
+    ctx, qkv, k_pool, v_pool, bt, perm = shared_stream_case(seqs, n_q, n_kv, d, 8, torch.float32, window)
+    v_pool = torch.randn(*k_pool.shape[:3], vdim, generator=torch.Generator(device="cuda").manual_seed(d), device="cuda")
+    outs = []
+    for plain, single in ((True, 3), (False, 3), (False, 0)):
+        ops.force_generic, ctx.single_rows = plain, single
+        try:
+            out = torch.full((ctx.T, n_q * vdim), float("nan"), device="cuda")
+            ops.paged_attention(qkv, k_pool, v_pool, bt, ctx, n_q, n_kv, d, 8, window, 0.1, out, vdim=vdim)
+            outs.append(out)
+        finally:
+            ops.force_generic = False
+    assert torch.isfinite(outs[0]).all() and torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+
+
 @pytest.mark.parametrize("name", ["scalar128-b8-8k", "scalar256-b32-8k", "scalar256-b8-32k",
                                   "heads1024-b8-32k", "heads512-b8-8k", "heads256-b8-4k",
                                   "scalar128-b8-8k-window", "scalar256-b32-8k-window",

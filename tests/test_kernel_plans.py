@@ -165,6 +165,22 @@ def test_chunks_of_grouped_heads(lib, rows, keys, n_q, n_kv, d, window, chunk):
     assert _single_rows_plan(lib, _attention(rows, keys, n_q, n_kv, d, window=window)) == [2, chunk, -(-keys // chunk)]
 
 
+# (prompt rows of one request after single rows of others; requests 0: that many rows of each of several)
+@pytest.mark.parametrize("singles,rows,requests,keys,heads,d,vdim,window,taken", [
+    (0, 173, 1, 173, 16, 128, 128, 0, 1), (0, 64, 1, 64, 16, 128, 128, 0, 0), (7, 505, 1, 2500, 16, 128, 128, 0, 1),
+    (31, 2, 1, 200, 16, 128, 128, 0, 1), (63, 17, 1, 200, 16, 128, 128, 0, 0), (63, 193, 1, 200, 16, 128, 128, 0, 1),
+    (63, 192, 1, 200, 16, 128, 128, 0, 0), (0, 2, 16, 66, 16, 128, 128, 0, 1), (0, 2, 16, 66, 32, 100, 100, 0, 0),
+    (0, 8, 16, 110, 32, 100, 100, 0, 1), (0, 2, 8, 66, 32, 100, 100, 0, 1), (0, 2, 4, 66, 16, 64, 128, 0, 1),
+    (0, 505, 1, 505, 8, 64, 64, 200, 1), (0, 255, 1, 505, 8, 64, 64, 0, 0), (0, 64, 1, 2064, 8, 64, 64, 0, 1),
+    (0, 64, 1, 2064, 8, 64, 64, 200, 0), (0, 64, 1, 999, 8, 64, 64, 0, 0), (0, 8, 64, 308, 8, 64, 64, 0, 1),
+    (0, 600, 1, 600, 8, 64, 64, 127, 0), (0, 100, 40, 100, 8, 64, 64, 0, 0), (1, 64, 1, 2064, 8, 64, 64, 0, 0),
+    (0, 31, 1, 2064, 8, 64, 64, 0, 0), (24, 375, 1, 308, 8, 64, 64, 0, 0), (24, 376, 1, 308, 8, 64, 64, 0, 1), (0, 600, 1, 600, 16, 16, 16, 0, 0)])
+def test_which_32_bit_steps_run_eight_rows_to_a_block(lib, singles, rows, requests, keys, heads, d, vdim, window, taken):
+    a = _attention(singles, keys, heads, heads, d, window=window, Dv=vdim)
+    a.dtype, a.T, a.S, a.max_qlen = 0, singles + rows * requests, singles + requests, rows
+    assert lib.ninfer_attention_rows_f32_takes(ctypes.byref(a)) == taken
+
+
 def test_attention_without_allocation_refuses_sinks_and_gates(lib):
     lib.ninfer_last_error.restype = ctypes.c_char_p
     for more in ({"sink": 1}, {"gate": 16, "gate_stride": 2048}):
