@@ -168,22 +168,26 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_rows_kernel(GemmArgs a
 // - 17 to 32 rows, against the few-row kernel: 2,048 features 5.8 and 5.7, 3,072 6.0 and 8.0, 6,144 8.7 and 11.4, 32,000
 //   27 and 42; gated 2 x 1,408 7.3 and 6.8, 2 x 2,816 (K 1,024) 5.8 and 6.6, 2 x 20,480 (K 3,584) 52 and 73.
 // - 33 rows and more, against the library's product: 2,048 features, 64 rows 6.0 and 8.9, 128 rows 7.0 and 8.3 (K 5,632
-//   12.1 and 17.9, 14.7 and 15.9); 6,144 64 rows 12.1 and 12.7, 128 15.7 and 14.9; 8,192 (K 8,192) 64 rows 42 and 33.
+//   12.1 and 17.9, 14.7 and 15.9); 6,144 64 rows 12.1 and 12.7, 128 15.7 and 14.9.
 //   Against tiles of 64 rows: gated 2 x 5,632 64 rows 17.7 and 20.8, 80 22.0 and 19.0; 2 x 2,816 128 rows 9.8 and
-//   11.6; 2 x 1,408 256 rows 14.5 and 18; 2 x 20,480 64 rows 87 and 72; a few hundred features 5.2 and 13.
+//   11.6; 2 x 1,408 256 rows 14.5 and 18; 2 x 20,480 64 rows 87 and 72; a few hundred features 5.2 and 13. Of K 512 to 896,
+//   where a second round of blocks costs more than it multiplies, gated 2 x 4,096 64 rows 5.7 and 6.7, 96 7.4 and 6.5; 2 x 3,072
+//   of K 768, 96 rows 8.5 and 7.6; K 1,024 9.9 and 10.8. (Below 512 a launch is a few us in either: K 384 7.3 and 5.9.)
 // - beyond 128 rows, against the library's product: 2,048 features 160 rows 9.9 and 9.1; 1,024 (K 2,816) 256 rows 7.7 and
 //   8.5; 768 256 rows 6.4 and 8.4, 384 9.5 and 9.1.
 // - up to 128 features (a router's), against the few-row kernel, whose rows came 64 bytes at a time: 61 features, K 2,048,
 //   512 rows 5.5 and 6.1 alone, but 8.6 in either beside the shared expert's products; 2,048 rows 6.3 and 13.2, 4,096 8.7
-//   and 22.7 (the same bits).
+//   and 22.7.
 bool gemm_skinny_rows_takes(const GemmArgs& a) {
-  if (a.offsets || a.a_index || a.c_index || a.groups > 1 || a.force_kernel || a.in_dtype != kBF16 || a.M <= 16 || a.K % 128 || a.lda % 8 || (uintptr_t)a.A % 16 || (uintptr_t)a.W % 16)
+  if (a.offsets || a.a_index || a.c_index || a.groups > 1 || a.force_kernel || a.in_dtype != kBF16 || a.M <= 16 ||
+      a.K % 128 || a.lda % 8 || (uintptr_t)a.A % 16 || (uintptr_t)a.W % 16)
     return false;
   const bool gated = epilogue_gated(a.epilogue);
   const int64_t w_rows = (int64_t)a.N * (gated ? 2 : 1);
   if (a.M <= 32) return w_rows > (gated ? 4096 : 2560);
   if (a.N <= 128) return !gated && a.M > kRowsMax;
-  return a.M <= kRowsMax && w_rows * rows_parts(a) <= (gated ? 24576 : a.M <= 128 ? 16384 : 8192);
+  const int most = !gated ? a.M <= 128 ? 16384 : 8192 : a.K >= 512 && a.K < 1024 ? 16384 : 24576;
+  return a.M <= kRowsMax && w_rows * rows_parts(a) <= most;
 }
 
 // Features a block, so that the blocks on an XCD (the row parts of its feature tiles) fill rounds of one a CU: 6,144

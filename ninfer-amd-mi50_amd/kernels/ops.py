@@ -853,10 +853,19 @@ class HipOps:
     def _rows_kernel_takes(x, w) -> bool:
         """Plain dense products of 33 to 512 rows that the kernel for them runs faster than the library
         (gemm_skinny_rows.hip), and for the host: a launch costs it 3 us and the library's call 18. Not
-        weights of 48 MB and more, which gain by a cut along K, or by the library's taller tiles."""
+        weights of 48 MB and more, which gain by a cut along K, or by the library's taller tiles; nor where
+        blocks of 32 rows are few for a long K (us there and here: 129 features of K 8,192, 33 to 512 rows,
+        8.6 to 11.6 and 9.7 to 13.3; 512 of K 5,632, 64 rows, 7.8 and 8.1, 128 10.3 and 8.2), or many of rows
+        that do not fill the last one (K 5,632, 4,096 features: 80 rows 19.5 and 23.1, 96 27.2 and 24.3, 112 21.3
+        and 24.2; 3,072: 80 rows 26.5 and 22.0, 112 20.7 and 22.2)."""
         rows, (n, k) = x.shape[0], w.shape
+        parts = -(-rows // 32)
+        if k > 4096 and (n <= 256 and n * rows <= 70000 or n <= 512 and rows <= 64):
+            return False
+        if k >= 4096 and rows > 64 and rows % 32 and n * parts > 9216:
+            return False
         return (rows <= 512 and n > 128 and k % 128 == 0
-                and n * -(-rows // 32) <= (16384 if rows <= 128 else 8192) and n * k < (24 << 20)
+                and n * parts <= (16384 if rows <= 128 else 8192) and n * k < (24 << 20)
                 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
     @staticmethod

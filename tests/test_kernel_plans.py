@@ -62,6 +62,28 @@ def test_height_of_dense_tiles(lib, m, n, k, gated, beside, rows):
     assert lib.ninfer_gemm_tile_rows(ctypes.byref(args)) == rows
 
 
+@pytest.mark.parametrize("m,n,k,gated,kernel", [
+    (96, 3072, 768, 1, 4), (64, 4096, 768, 1, 3), (64, 4097, 768, 1, 4), (96, 4096, 1024, 1, 3), (96, 4097, 1024, 1, 4),
+    (64, 8192, 768, 0, 3), (128, 4096, 512, 0, 3), (128, 4097, 512, 0, 4)])
+def test_which_products_run_in_blocks_of_32_rows(lib, m, n, k, gated, kernel):
+    from ninfer_amd.kernels.ops import _GemmArgs
+    args = _GemmArgs(A=4096, W=4096, C=4096, M=m, N=n, K=k, lda=k, ldc=n, groups=1, a_div=1, in_dtype=BF16, out_dtype=BF16,
+                     epilogue=gated)
+    assert lib.ninfer_gemm_kernel(ctypes.byref(args)) == kernel
+
+
+@pytest.mark.parametrize("rows,n,k,own", [
+    (64, 2048, 5632, True), (33, 129, 8192, False), (512, 129, 8192, False), (33, 129, 4096, True), (64, 512, 5632, False),
+    (65, 512, 5632, True), (384, 256, 5632, True), (80, 4096, 5632, False), (96, 4096, 5632, True), (112, 3072, 4096, False),
+    (80, 3072, 4096, True), (80, 4096, 3584, True), (128, 4096, 4096, True), (160, 1638, 2048, True), (160, 1639, 2048, False),
+    (64, 8192, 3072, False), (64, 2048, 2000, False)])
+def test_which_plain_products_stay_out_of_the_library(rows, n, k, own):
+    from types import SimpleNamespace
+    from ninfer_amd.kernels.ops import HipOps
+    at = lambda *shape: SimpleNamespace(shape=shape, data_ptr=lambda: 4096)
+    assert HipOps._rows_kernel_takes(at(rows, k), at(n, k)) == own
+
+
 # (experts, chosen, inner, shared inner; rows: does the shared expert start before the routing?)
 @pytest.mark.parametrize("sizes,rows,early", [
     ((60, 4, 1408, 5632), 512, True), ((60, 4, 1408, 5632), 600, True), ((60, 4, 1408, 5632), 700, False),
