@@ -397,8 +397,11 @@ class HipOps:
         self.scan_chunk_min_rows = 8        # ... and for the scans with one decay per head and token
         self.lightning_chunk_min_rows = 8   # a step's longest portion from which lightning attention runs in chunks
         self.library_min_rows = 32  # dense bf16 products with more rows go to the library
-        self.rows_kernel_max = 64   # ... unless the kernel for 33 to 64 rows takes them
-        self.rows_kernel_features = (4096, 32768)   # (there no call of the library's, whatever the rows)
+        # ... but up to 64 rows of 4,096 to 32,768 features never, whatever the sizes within: a launch here costs the host 3 us,
+        # the library's call 18, and steps of so few rows are bound by the host when they run eagerly. Up to 8,192 features
+        # blocks of 32 rows (gemm_skinny_rows.hip), beyond them tiles of 64; both cut along K where `_rows_cut` says
+        self.rows_kernel_max = 64
+        self.rows_kernel_features = (4096, 32768)
         # ... but never a SwiGLU's gate/up product: the tile kernels here have the activation in
         # their epilogue, which beats the library's product followed by a kernel for the
         # activation at every row count (70 against 98 us at 64 rows of 40960 x 3584; whole
@@ -832,15 +835,18 @@ class HipOps:
                 if not own:
                     torch.matmul(x, w.t(), out=out)
                     return
+        elif act is None and bias is None and self._rows_cut(x, out, w) and self._gemm(
+                x, w, out, m=x.shape[0], n=w.shape[0], k=x.shape[1], only_if_split=True):
+            return
         self._gemm(x, w, out, m=x.shape[0], n=w.shape[0], k=x.shape[1], bias=bias,
                    epilogue=UNGATED_ACTS[act])
 
     def _use_library(self, x, out, w) -> bool:
         """Plain dense products of many bf16 rows go to the vendor library, as
         the reference sends every multi-row product to rocBLAS
-        (src/ops/linear.hip:21-35); few rows, 32-bit, grouped and fused products
-        run on the hand-written kernels, and so do products of up to `rows_kernel_max` rows
-        whose sizes the kernel for them takes (gemm_skinny_rows.hip)."""
+        (src/ops/linear.hip:21-35), unless `_rows_kernel_takes` them; few rows, 32-bit, grouped and
+        fused products run on the hand-written kernels, and so do products of up to
+        `rows_kernel_max` rows and `rows_kernel_features` features."""
         if self.force_generic or x.dtype != torch.bfloat16 or out.dtype != x.dtype:
             return False
         rows = x.shape[0]
@@ -848,6 +854,18 @@ class HipOps:
                 and self.rows_kernel_features[0] <= w.shape[0] <= self.rows_kernel_features[1]:
             return False
         return rows > self.library_min_rows
+
+    def _rows_cut(self, x, out, w) -> bool:
+        """33 to 64 rows that `_use_library` keeps from the library, weights of 48 MB and more (`kSplitMinBytes`): is the
+        product the faster one cut along K? us in blocks of 32 rows or tiles of 64 (in the library) and so, 64 rows:
+        5,120 features of K 5,632 24.5 (22) and 22, 8,192 of K 8,192 40 (32) and 34; 12,288 of K 4,096 39 (25) and
+        28.5, 20,480 of K 3,584 36.7 (34.4) and 36.5. But 4,096 of K 8,192 22 and 25, 8,192 of K 3,584 20.0 and 20.4,
+        16,384 of K 2,048 21.1 and 23.5, 24,576 of K 3,584 38.5 and 44.5."""
+        rows, (n, k) = x.shape[0], w.shape
+        return (not self.force_generic and x.dtype == torch.bfloat16 and out.dtype == x.dtype
+                and self.library_min_rows < rows <= self.rows_kernel_max
+                and self.rows_kernel_features[0] <= n <= 20480 and n % 32 == 0 and k % 128 == 0
+                and (k >= 5120 and n >= 5120 or k >= 3584 and n > 8192) and n * k >= 24 << 20)
 
     @staticmethod
     def _rows_kernel_takes(x, w) -> bool:

@@ -84,6 +84,21 @@ def test_which_plain_products_stay_out_of_the_library(rows, n, k, own):
     assert HipOps._rows_kernel_takes(at(rows, k), at(n, k)) == own
 
 
+@pytest.mark.parametrize("rows,n,k,cut", [
+    (64, 8192, 8192, True), (33, 10240, 3584, True), (32, 10240, 3584, False), (65, 10240, 3584, False), (64, 8192, 3584, False),
+    (64, 5120, 5632, True), (64, 4096, 8192, False), (64, 5120, 4864, False), (64, 20480, 3584, True), (64, 20512, 3584, False),
+    (64, 16384, 2048, False), (64, 5100, 8192, False), (64, 5120, 5200, False)])
+def test_which_products_of_33_to_64_rows_are_cut(rows, n, k, cut):
+    import torch
+    from types import SimpleNamespace
+    from ninfer_amd.kernels.ops import HipOps
+    ops = SimpleNamespace(force_generic=False, library_min_rows=32, rows_kernel_max=64, rows_kernel_features=(4096, 32768))
+    at = lambda *shape: SimpleNamespace(shape=shape, dtype=torch.bfloat16)
+    assert HipOps._rows_cut(ops, at(rows, k), at(rows, n), at(n, k)) == cut
+    # (what is asked is what the library keeps from the library)
+    assert not cut or not HipOps._use_library(ops, at(rows, k), at(rows, n), at(n, k))
+
+
 # (experts, chosen, inner, shared inner; rows: does the shared expert start before the routing?)
 @pytest.mark.parametrize("sizes,rows,early", [
     ((60, 4, 1408, 5632), 512, True), ((60, 4, 1408, 5632), 600, True), ((60, 4, 1408, 5632), 700, False),

@@ -224,6 +224,24 @@ def test_linear_of_33_to_64_rows(ops, gen, m, n, k):
         ops.force_generic = saved
 
 
+@pytest.mark.parametrize("n,k", [(8192, 8192), (10240, 3584), (20480, 3584)])
+def test_linear_of_33_to_64_rows_cut_along_k(ops, gen, n, k):
+    """Weights of 48 MB and more: by default cut along K, and a row's bits the same among 33 rows as among 64."""
+    x, w = rnd((64, k), torch.bfloat16, gen), rnd((n, k), torch.bfloat16, gen)
+    saved, ops.force_generic = ops.force_generic, False
+    try:
+        o1, o2, cut = (torch.empty(64, n, device="cuda", dtype=torch.bfloat16) for _ in range(3))
+        ops.linear(x, w, o1)
+        assert ops._gemm(x, w, cut, m=64, n=n, k=k, only_if_split=True) and torch.equal(o1, cut)
+        PlainOps().linear(x, w, o2)
+        close(o1, o2, torch.bfloat16, scale=math.sqrt(k))
+        part = torch.empty(33, n, device="cuda", dtype=torch.bfloat16)
+        ops.linear(x[:33].contiguous(), w, part)
+        assert torch.equal(part, o1[:33])
+    finally:
+        ops.force_generic = saved
+
+
 @pytest.mark.parametrize("m,n,k,gated", [
     (17, 2561, 128, False), (32, 6144, 2048, False), (31, 2049, 384, True),      # one row part
     (33, 129, 2048, False), (64, 2048, 5632, False), (63, 8191, 256, False), (64, 6144, 2048, True),
