@@ -15,7 +15,7 @@ from typing import Dict, List, Optional
 
 import torch
 
-from ..parts.base import Block, CallInfo, Norm, NormedOutput, Part, StepContext, WeightBinder
+from ..parts.base import Block, CallInfo, Norm, NormedOutput, Part, StepContext, WeightBinder, settle
 from ..parts.embedding import LMHead, TokenEmbedding
 from ..weights.source import TensorSpec
 
@@ -25,6 +25,11 @@ class LayerCall:
     layer: int                       # index into ModelSpec.blocks
     cache_from: Optional[int] = None  # index of an earlier plan entry whose cache is read
     before: Optional[int] = None     # index into ModelSpec.joins: what the stream passes first
+
+
+def _knows_normed_output(block: Block) -> bool:
+    # (not where its `forward` was replaced)
+    return block.takes_normed_output and "forward" not in vars(block)
 
 
 class ModelSpec:
@@ -111,13 +116,15 @@ class ModelSpec:
             if call.before is not None:
                 residual = self.joins[call.before].forward(ctx, residual, pending, first)
                 pending = None
-            pending = self.blocks[call.layer].forward(ctx, residual, pending, info)
-            if isinstance(pending, NormedOutput):
-                after = self.plan[i + 1] if i + 1 < len(self.plan) else None
-                if tap is not None or after is None or after.before is not None \
-                        or not self.blocks[after.layer].takes_normed_output:
-                    pending.norm.add(ctx, residual, pending.y)
-                    pending = None
+            block = self.blocks[call.layer]
+            after = self.plan[i + 1] if i + 1 < len(self.plan) else None
+            taken = tap is None and after is not None and after.before is None \
+                and _knows_normed_output(block) and _knows_normed_output(self.blocks[after.layer])
+            if info is not None:
+                info.hands_on = taken
+            pending = block.forward(ctx, residual, pending, info)
+            if isinstance(pending, NormedOutput) and not taken:
+                pending = settle(ctx, residual, pending)
             if tap is not None:
                 tap(i, residual, pending)
         if logit_rows is None or logit_rows.numel() == 0:

@@ -104,10 +104,11 @@ class CallInfo:
     """How one entry of the layer plan runs: which cache it uses, whether it
     writes it (false when it reads another call's cache), and the slice of the
     per-request state that belongs to it ([slots, floats], or None): a block's for the block,
-    the mixer's for the mixer."""
+    the mixer's for the mixer. `hands_on`: whoever runs the block takes a `NormedOutput` from it."""
     cache: Optional[CacheView] = None
     writes_cache: bool = True
     state: Optional[torch.Tensor] = None
+    hands_on: bool = False
 
 
 @dataclass
@@ -229,25 +230,32 @@ def _formed(ctx: "StepContext", pending, like: torch.Tensor) -> torch.Tensor:
 
 @dataclass
 class NormedOutput:
-    """What a block leaves to be normed and added to the residual: norm.add(ctx, residual, y). Handed on only to
-    a block that takes it (`Block.takes_normed_output`), whose first norm then runs in the same kernel."""
+    """What a block leaves to be normed and added to the residual: norm.add(ctx, residual, y). Handed on only where
+    the call says so (`CallInfo.hands_on`), to a block that takes it (`Block.takes_normed_output`), whose first norm
+    then runs in the same kernel."""
     norm: Any
     y: Any
 
 
 def plain_rows(ctx: "StepContext", y):
     """What a part handed on as something that any part takes: a NormedSum, a SumRows or a
-    NormedRows becomes rows, a ReadyRows nothing; everything else is handed back unchanged."""
+    NormedRows becomes rows, a ReadyRows nothing; everything else is handed back unchanged. (A NormedOutput is no
+    part's to take here: it needs the residual.)"""
+    if isinstance(y, NormedOutput):
+        raise ValueError("a block's last norm was handed on to a part that does not take it")
     if isinstance(y, (NormedSum, SumRows, NormedRows)):
         return y.rows(ctx)
     return None if isinstance(y, ReadyRows) else y
 
 
 def settle(ctx: "StepContext", residual: torch.Tensor, pending) -> Optional[torch.Tensor]:
-    """For parts that take only plain rows: a PendingRows is added into the
+    """For parts that take only plain rows: a PendingRows or a NormedOutput is added into the
     residual now; a tensor (or None) is handed back unchanged."""
     if isinstance(pending, PendingRows):
         pending.add_to(ctx, residual)
+        return None
+    if isinstance(pending, NormedOutput):
+        pending.norm.add(ctx, residual, pending.y)
         return None
     return plain_rows(ctx, pending)
 
@@ -427,7 +435,12 @@ class Block(Part):
     """Arrangement of norms, mixer and feed-forward around the residual."""
 
     mixer: Mixer
-    takes_normed_output = False   # `forward` takes a NormedOutput of the block before as `pending`
+    takes_normed_output = False   # `forward` takes a NormedOutput of the block before as `pending`, and may hand one on
+
+    def __init_subclass__(cls, **kw):
+        super().__init_subclass__(**kw)
+        if "forward" in vars(cls) and "takes_normed_output" not in vars(cls):
+            cls.takes_normed_output = False   # (a `forward` of its own, which need not know of it)
 
     def state_floats(self) -> int:
         """32-bit numbers of per-request state of one run of this block: the mixer's, and

@@ -128,7 +128,7 @@ class SandwichBlock(Block):
     parts with `add(ctx, residual, y)` (they norm y and add it into the 32-bit residual; a
     sparse feed-forward's weighted rows are summed by the same kernel). `feed_forward` may be
     None (a layer with a mixer only). The norm behind a sublayer and the one in front of the next run as one
-    kernel; the block's last one is handed on for the next block's first."""
+    kernel; the block's last one is handed on for the next block's first where the call says that it is taken."""
 
     takes_normed_output = True
 
@@ -150,13 +150,17 @@ class SandwichBlock(Block):
         else:
             h = self.mixer_norm.forward(ctx, residual, pending)
         y = self.mixer.forward(ctx, h, residual, call)
-        if self.feed_forward is None:
-            return NormedOutput(self.mixer_out_norm, y)
-        h = add_then(ctx, residual, self.mixer_out_norm, y, self.ff_norm)
-        y = self.feed_forward.forward(ctx, h, residual)
-        if y is None:
-            raise ValueError("a feed-forward between two norms hands its rows back")
-        return NormedOutput(self.ff_out_norm, y)
+        last = self.mixer_out_norm
+        if self.feed_forward is not None:
+            h = add_then(ctx, residual, last, y, self.ff_norm)
+            y = self.feed_forward.forward(ctx, h, residual)
+            if y is None:
+                raise ValueError("a feed-forward between two norms hands its rows back")
+            last = self.ff_out_norm
+        if call is None or call.hands_on:
+            return NormedOutput(last, y)
+        last.add(ctx, residual, y)
+        return None
 
 
 register_part("block", "sandwich", SandwichBlock)

@@ -419,3 +419,91 @@ def test_host_sandwich_block_with_a_part_that_only_adds():
     assert isinstance(pending, NormedOutput)
     pending.norm.add(None, x, pending.y)
     assert torch.equal(x, want)
+
+
+@pytest.mark.parametrize("kind", ["plain", "subclass", "reads on", "inside another", "replaced", "takes nothing"])
+def test_host_sandwich_blocks_beside_blocks_that_know_nothing_of_handed_on_norms(kind):
+    """A block's last norm is handed on only to a block that takes it: a subclass with a `forward` of its own, a block
+    around one, a block whose `forward` was replaced and any other block find a whole residual and no such
+    pending, and leave one."""
+    from ninfer_amd.models.spec import ModelSpec
+    from ninfer_amd.parts import RMSNorm, SandwichBlock
+    from ninfer_amd.parts.base import Block, CallInfo, Mixer, NormedOutput, Part
+
+    class Adds(Part):
+        def add(self, ctx, residual, y):
+            residual += 2 * y
+
+    class Doubles(Mixer):
+        def forward(self, ctx, x, residual, call=None):
+            return 2 * x
+
+    class Takes(RMSNorm):
+        def forward(self, ctx, residual, pending):
+            assert pending is None
+            return residual + 1
+
+    class Same(Part):
+        def forward(self, ctx, *a):
+            return torch.arange(4.).repeat(2, 1)
+
+        def forward_rows(self, ctx, residual, rows, pending=None):
+            assert pending is None
+            return residual[rows]
+
+    class Head(Part):
+        def forward(self, ctx, x):
+            return x
+
+    made = lambda cls: cls(Takes("a", 4, 1e-5), Doubles(), Adds(), Takes("b", 4, 1e-5), Doubles(), Adds())
+    seen = []
+
+    class Own(SandwichBlock):
+        def forward(self, ctx, residual, pending, call):
+            h = self.mixer_norm.forward(ctx, residual, pending)
+            self.mixer_out_norm.add(ctx, residual, self.mixer.forward(ctx, h, residual, call))
+            h = self.ff_norm.forward(ctx, residual, None)
+            self.ff_out_norm.add(ctx, residual, self.feed_forward.forward(ctx, h, residual))
+
+    class ReadsOn(SandwichBlock):
+        def forward(self, ctx, residual, pending, call):
+            assert not isinstance(pending, NormedOutput)
+            out = super().forward(ctx, residual, pending, call)
+            seen.append(residual.clone())
+            return out
+
+    class Around(Block):
+        def __init__(self):
+            self.inner = made(SandwichBlock)
+
+        def forward(self, ctx, residual, pending, call):
+            assert not isinstance(pending, NormedOutput)
+            out = self.inner.forward(ctx, residual, pending, call)
+            seen.append(residual.clone())
+            return out
+
+    other = {"plain": SandwichBlock, "subclass": Own, "reads on": ReadsOn}.get(kind)
+    other = made(other) if other else Around() if kind == "inside another" else made(SandwichBlock)
+    if kind == "replaced":
+        whole = other.forward
+        other.forward = lambda ctx, residual, pending, call: (seen.append(residual.clone()), whole(ctx, residual, pending, call))[1]
+    if kind == "takes nothing":
+        class Whole(Block):
+            def forward(self, ctx, residual, pending, call):
+                assert pending is None
+                seen.append(residual.clone())
+        other = Whole()
+    spec = ModelSpec(embedding=Same(), blocks=[made(SandwichBlock), other, made(SandwichBlock)], final_norm=Same(), head=Head(),
+                     vocab_size=4)
+    step = lambda x: x + 4 * (x + 1)
+    x = torch.arange(4.)
+    states = [x]
+    for b in range(3):
+        states.append(states[-1] if b == 1 and kind == "takes nothing" else step(step(states[-1])))
+    for calls in ([CallInfo() for _ in range(3)], [None] * 3):
+        seen.clear()
+        got = spec.forward(None, calls, torch.tensor([0, 1]))
+        assert torch.equal(got, states[3].repeat(2, 1))
+        if calls[0] is not None:
+            at = 1 if kind in ("replaced", "takes nothing") else 2
+            assert all(torch.equal(s, states[at].repeat(2, 1)) for s in seen) and (seen or kind in ("plain", "subclass"))
