@@ -56,14 +56,21 @@ class _RouteArgs(ctypes.Structure):
 
 
 # Prompts over a cached latent form keys and values per head where the cached rows to form them from are no more
-# than LATENT_HEADS_FEW, or than LATENT_HEADS_RATIO times the rows that read them, and LATENT_HEADS_KEYS at most (7 KB
-# a row at 16 heads of 64 + 128 numbers; the other form keeps 52 KB per row of the step). us in the latent's space
-# and so, 16 heads of 512 + 64 numbers: 2,048 tokens 178 and 61, 512 61 and 26, 16 25 and 12; 512 after 4,096 cached 277
-# and 90; 64 after 512 44 and 27, after 2,000 53 and 59; 16 after 1,000 40 and 35. 8 heads of 256 + 32: 2,048 115 and 42,
-# 512 after 7,500 126 and 112, 128 after 2,000 39 and 41, 16 after 1,000 23 and 26.
+# than LATENT_HEADS_FEW, or than LATENT_HEADS_RATIO times the rows that read them, and LATENT_HEADS_KEYS at most (scratch: 7 KB
+# a row at 16 heads of 64 + 128 numbers, and as much more with more heads, where the other form keeps 52 KB per row of the
+# step). us of a layer in the latent's space and so, 16 heads of 512 + 64 numbers: 2,048 tokens 254 and 122, 512 111 and 64,
+# 16 53 and 30; 512 after 4,096 cached 328 and 125; 64 after 1,000 85 and 57; 30 requests of 2 rows at 500 keys beside
+# a prompt of 1,000 172 and 158. 8 heads of 256 + 32: 2,048 161 and 79, 512 after 7,500 163 and 137, 16 after 1,000 46 and 39.
+# Cached rows of many requests with few rows each cost a block per head, and are left where they outnumber the rows
+# LATENT_HEADS_MANY times (32 heads: the 30 requests beside the prompt 229 and 313, 100 of 4 rows at 44 keys 120 and 159).
+# Single rows of the step then run apart, some 25 us: only beside LATENT_HEADS_APART rows and heads, and 16 rows to each (16
+# heads, 8 rows at 1,500 keys beside 512 new ones 161 and 112, beside 16 75 and 74; 32 at 300 beside 64 82 and 85; 8
+# heads, 8 at 1,500 beside 300 after 1,000 83 and 88; 3 at 2,500 beside 20 46 and 55).
 LATENT_HEADS_KEYS = 16384
 LATENT_HEADS_FEW = 512
 LATENT_HEADS_RATIO = 16
+LATENT_HEADS_MANY = 8
+LATENT_HEADS_APART = 4096
 BIG_TILE_ROWS = 256   # rows of a tall tile of the grouped products (the library's kGroupedTileRows)
 ROUTE_ROWS_PER_BLOCK = 1024  # the library's kAlignRowsPerBlock
 # rows (tokens) from which the grouping runs as several blocks side by side: 12.5 against 13 us
@@ -1694,11 +1701,15 @@ class HipOps:
     def latent_heads_rows(self, ctx, heads, dim, rank, rot_dim, vdim, window) -> int:
         """The first of the step's rows whose prompts had better attend with keys and values formed
         per head (`latent_heads_attention`); ctx.T: none. These are the rows behind the single ones, where
-        the sizes have such a kernel and the cached rows to form keys and values from are few beside
-        the rows that read them."""
+        the sizes have such a kernel, the cached rows to form keys and values from are few beside
+        the rows that read them, and the single rows few beside these."""
         portion = ctx.T - ctx.single_rows
         if (portion <= 0 or not 0 < ctx.portion_keys <= min(LATENT_HEADS_KEYS, max(LATENT_HEADS_FEW, LATENT_HEADS_RATIO * portion))
                 or ctx.act_dtype != torch.bfloat16 or window or self.force_generic or self.conv_pieces_always):
+            return ctx.T
+        if ctx.portion_keys > LATENT_HEADS_MANY * portion and (ctx.S - ctx.single_rows) * heads > 512:
+            return ctx.T
+        if ctx.single_rows and (portion * heads < LATENT_HEADS_APART or portion < 16 * ctx.single_rows):
             return ctx.T
         a = _LatentArgs()
         a.seq_row_start = a.seq_pos0 = 1   # (asked for the sizes alone; they are there)

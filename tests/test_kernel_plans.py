@@ -297,3 +297,30 @@ def test_a_products_arguments_have_one_size(lib, monkeypatch):
     monkeypatch.setattr(ops, "_GemmArgs", Longer)
     with pytest.raises(ops.KernelError, match="lay a product's arguments out differently"):
         ops.HipOps()
+
+
+# (rows and cached keys, these included, of each portion behind the single rows; does the step form keys and values?)
+@pytest.mark.parametrize("heads,rank,rd,vdim,singles,portions,taken", [
+    (16, 512, 64, 128, 0, [(2048, 2048)], True), (8, 256, 32, 64, 0, [(2, 2)], True), (16, 512, 64, 128, 0, [(2, 512)], True),
+    (16, 512, 64, 128, 0, [(2, 513)], False), (16, 512, 64, 128, 0, [(64, 1024)], True), (16, 512, 64, 128, 0, [(64, 1025)], False),
+    (16, 512, 64, 128, 0, [(2048, 16384)], True), (16, 512, 64, 128, 0, [(2048, 16385)], False),
+    (16, 512, 64, 128, 0, [(1000, 1000)] + [(2, 502)] * 30, True), (32, 512, 64, 128, 0, [(1000, 1000)] + [(2, 502)] * 30, False),
+    (32, 512, 64, 128, 0, [(4, 44)] * 100, False), (32, 512, 64, 128, 0, [(8, 48)] * 60, True), (32, 512, 64, 128, 0, [(2, 32)] * 16, True),
+    (16, 512, 64, 128, 1, [(256, 256)], True), (16, 512, 64, 128, 1, [(255, 255)], False), (8, 256, 32, 64, 1, [(511, 511)], False),
+    (8, 256, 32, 64, 1, [(512, 512)], True), (16, 512, 64, 128, 32, [(512, 512)], True), (16, 512, 64, 128, 33, [(512, 512)], False),
+    (16, 512, 64, 128, 5, [], False), (16, 512, 64, 96, 0, [(64, 64)], False), (16, 512, 32, 128, 0, [(64, 64)], True),
+    (16, 512, 0, 128, 0, [(64, 64)], False), (3, 72, 64, 128, 0, [(64, 64)], True), (3, 68, 64, 128, 0, [(64, 64)], False)])
+def test_which_prompts_form_keys_and_values_per_head(lib, heads, rank, rd, vdim, singles, portions, taken):
+    import torch
+    from types import SimpleNamespace
+    from ninfer_amd.kernels.ops import HipOps
+    rows, keys = sum(r for r, _ in portions), sum(k for _, k in portions)
+    ctx = SimpleNamespace(T=singles + rows, S=singles + len(portions), single_rows=singles, portion_keys=keys,
+                          act_dtype=torch.bfloat16)
+    ops = SimpleNamespace(lib=lib, force_generic=False, conv_pieces_always=False)
+    first = lambda **kw: HipOps.latent_heads_rows(SimpleNamespace(**{**vars(ops), **kw}), ctx, heads, 128 - rd, rank, rd, vdim, None)
+    assert first() == (singles if taken else ctx.T)
+    assert first(force_generic=True) == ctx.T
+    assert HipOps.latent_heads_rows(ops, ctx, heads, 128 - rd, rank, rd, vdim, 4096) == ctx.T
+    ctx.act_dtype = torch.float32
+    assert first() == ctx.T
