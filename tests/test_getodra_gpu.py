@@ -684,6 +684,33 @@ def test_latent_kv_write(ops, dtype, heads, dim, rank, rd, turning):
         assert (q_abs[t, :, :rank] == 5.0).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("pairing", ["half", "interleaved"])
+@pytest.mark.parametrize("heads,dim,rank,rd,turning", [(3, 24, 40, 8, 8), (16, 64, 72, 64, 64), (2, 96, 32, 32, 16), (1, 8, 16, 4, 0)])
+@pytest.mark.parametrize("rows", [0, 1, 4, 10])
+def test_latent_kv_write_turns_queries_in_place(ops, dtype, pairing, heads, dim, rank, rd, turning, rows):
+    """Of the rows behind the first `abs_rows` the rotated parts stay in q, turned: what the other rows' go to q_abs as,
+    rounded once; all else of q, the cached rows and the first rows' q_abs are the same bits."""
+    torch.manual_seed(rank)
+    ps = 4
+    ctx = util.make_context(ops, dtype, [(17, 1), (5, 6), (0, 3)])
+    table = torch.tensor([[2, 4, 5, 6, 8], [3, 1, 7, -1, -1], [0, -1, -1, -1, -1]], dtype=torch.int32, device=DEV)
+    down = torch.randn(ctx.T, rank + rd).to(dtype).to(DEV)
+    q = torch.randn(ctx.T, heads * (dim + rd)).to(dtype).to(DEV)
+    norm_w, freq = torch.randn(rank, device=DEV), torch.rand(max(turning, 2) // 2, device=DEV) if turning else None
+    got = []
+    for n in (None, rows):
+        qn, pool = q.clone(), torch.zeros(9, ps, rank + rd, dtype=dtype, device=DEV)
+        q_abs = torch.full((ctx.T if n is None else n, heads, rank + rd), 5.0, device=DEV)
+        ops.latent_kv_write(down, qn, q_abs, pool, table, ctx, heads, dim, rank, rd, norm_w, 1e-5, freq, turning, 1.25, ps,
+                            interleaved=pairing == "interleaved", abs_rows=n)
+        got.append((qn.view(ctx.T, heads, dim + rd), q_abs, pool))
+    (qa, abs_a, pool_a), (qb, abs_b, pool_b) = got
+    assert torch.equal(qa.view_as(q), q) and torch.equal(pool_a, pool_b) and torch.equal(abs_a[:rows], abs_b)
+    assert torch.equal(qb[:rows], qa[:rows]) and torch.equal(qb[..., :dim], qa[..., :dim])
+    assert torch.equal(qb[rows:, :, dim:], abs_a[rows:, :, rank:].to(dtype))
+
+
 # ---- whole models ----------------------------------------------------------------------------
 
 PROMPT_LENGTHS = [70, 1, 23, 97, 40, 64]
@@ -902,6 +929,50 @@ def test_models_of_one_kind_of_layer(kind, dtype, tmp_path):
     for sched in (util.schedule_whole("x", toks), util.schedule_tail("x", toks, 20),
                   util.schedule_portions("x", toks, seed=1)):
         check_logits(case, dtype, util.run_schedule(runner, sched), "one kind of layer")
+
+
+@pytest.mark.parametrize("sizes", [(64, 64, 64, 128, 72), (96, 32, 16, 64, 40), (96, 32, 32, 128, 256)])
+def test_prompts_that_form_keys_and_values_per_head(sizes, tmp_path, monkeypatch):
+    """Layers whose heads of 128 numbers have a prompt kernel, in bfloat16: prompts, portions behind cached rows and
+    portions beside single rows through the layer itself, a layer with the weights of another among them, against the
+    plain implementation; and the form was taken, for all rows or for those behind the single ones."""
+    import ninfer_amd
+    from ninfer_amd import EngineOptions, load_model
+    from ninfer_amd.kernels import ops as kernels
+    monkeypatch.setattr(kernels, "LATENT_HEADS_APART", 0)   # (few heads, few rows)
+    dim, rd, turning, vdim, rank = sizes
+    la = getodra_cases._latent(3, dim, rd, vdim, rank, dims=turning)
+    raw = {"architecture": "Getodra", "vocab": 150, "width": 96, "max_positions": 200, "norm": {"eps": 1e-5},
+           "canon": {"taps": 3}, "layers": [getodra_cases._layer("latent_attention", la, 64),
+                                            getodra_cases._layer("lightning", getodra_cases._lightning(2, 16, 24, [0.8, 0.97]), 64),
+                                            getodra_cases._layer("latent_attention", la, 64, weights_of=0)]}
+    d = str(tmp_path)
+    ninfer_amd.write_random_model(d, raw, 5, dtype="bfloat16", std=STD)
+    cfg, w = util.read_folder(d)
+    reqs = {f"r{i}": util.random_tokens(n, raw["vocab"], 70 + i) for i, n in enumerate([90, 40, 131, 65])}
+    ref = {k: plain_getodra.forward(w, cfg, v) for k, v in reqs.items()}
+    case = {"name": str(sizes), "ref": {"bfloat16": ref}, "noise": {"bfloat16": {k: noise_of(cfg, w, v, ref[k]) for k, v in reqs.items()}}}
+    runner = load_model(d, EngineOptions(dtype="bfloat16", max_context=200, num_sequences=4, page_size=8, num_pages=80,
+                                         check_pages=True, poison_freed_pages=True))
+    seen, inner = [], type(runner.ops).latent_heads_attention
+    monkeypatch.setattr(type(runner.ops), "latent_heads_attention",
+                        lambda self, q, pool, table, ctx, *a, **k: (seen.append((ctx.single_rows, ctx.T)), inner(self, q, pool, table, ctx, *a, **k))[1])
+    for k, v in reqs.items():
+        for what, sched in (("whole", util.schedule_whole(k, v)), ("tail", util.schedule_tail(k, v, 12)),
+                            ("portions", util.schedule_portions(k, v, seed=len(v)))):
+            seen.clear()
+            check_logits(case, "bfloat16", util.run_schedule(runner, sched), what)
+            assert seen and (what != "whole" or seen == [(0, len(v))] * 2)
+    # single rows of two requests beside a portion of a third, again and again
+    a, b, c = reqs["r0"], reqs["r1"], reqs["r2"]
+    steps = [([("r0", a[:80], list(range(80))), ("r1", b[:30], list(range(30)))], [])]
+    for i in range(3):
+        steps.append(([("r0", [a[80 + i]], [0]), ("r1", [b[30 + i]], [0]), ("r2", c[40 * i:40 * i + 40], list(range(40)))], []))
+    steps.append(([("r0", a[83:], list(range(7))), ("r1", b[33:], list(range(7))), ("r2", c[120:], list(range(11)))], ["r0", "r1", "r2"]))
+    seen.clear()
+    check_logits(case, "bfloat16", util.run_schedule(runner, steps), "beside single rows")
+    assert seen.count((2, 42)) == 6
+    runner.release()
 
 
 def test_greedy_generation_through_the_scheduler(case):

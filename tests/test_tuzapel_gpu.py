@@ -679,6 +679,46 @@ def test_random_configurations(seed, tmp_path):
         runner.release()
 
 
+@pytest.mark.parametrize("q_rank", [None, 24])
+def test_prompts_that_form_keys_and_values_per_head(q_rank, tmp_path, monkeypatch):
+    """Latent layers of this design (neighbours turn, no gate, queries of a latent of their own or none) whose heads
+    of 128 numbers have a prompt kernel, in bfloat16: prompts, portions behind cached rows and beside single rows."""
+    import ninfer_amd
+    from ninfer_amd import EngineOptions, load_model
+    from ninfer_amd.kernels import ops as kernels
+    monkeypatch.setattr(kernels, "LATENT_HEADS_APART", 0)   # (few heads, few rows)
+    L = tuzapel_cases
+    raw = {"architecture": "Tuzapel", "vocab": 150, "width": 96, "norm": {"eps": 1e-5}, "logit_softcap": 15.0,
+           "layers": [L.layer(L.latent(4, 64, 64, 128, 72, q_rank=q_rank), L.dense(64)),
+                      L.layer(L.attention(4, 2, 32, 32, window=40, taps=2), L.dense(64)),
+                      L.layer(L.latent(2, 96, 32, 64, 40, q_rank=q_rank, base=500.0), L.dense(64))]}
+    d = str(tmp_path)
+    ninfer_amd.write_random_model(d, raw, 9, dtype="bfloat16", std=STD)
+    cfg, w = util.read_folder(d)
+    reqs = {f"q{i}": util.random_tokens(n, raw["vocab"], 30 + i) for i, n in enumerate([70, 100, 33])}
+    ref = {k: plain.forward(cfg, w, v)[0] for k, v in reqs.items()}
+    sub = {"name": f"per head {q_rank}", "ref": {"bfloat16": ref},
+           "noise": {"bfloat16": {k: noise_of(cfg, w, v, ref[k]) for k, v in reqs.items()}}}
+    runner = load_model(d, EngineOptions(dtype="bfloat16", max_context=128, num_sequences=3, page_size=8, num_pages=48,
+                                         check_pages=True, poison_freed_pages=True))
+    seen, inner = [], type(runner.ops).latent_heads_attention
+    monkeypatch.setattr(type(runner.ops), "latent_heads_attention",
+                        lambda self, q, pool, table, ctx, *a, **k: (seen.append((ctx.single_rows, ctx.T)), inner(self, q, pool, table, ctx, *a, **k))[1])
+    for k, v in reqs.items():
+        check_logits(sub, "bfloat16", util.run_schedule(runner, util.schedule_whole(k, v)), "whole")
+        assert seen[-2:] == [(0, len(v))] * 2
+        check_logits(sub, "bfloat16", util.run_schedule(runner, util.schedule_portions(k, v, seed=2)), "portions")
+    a, b = reqs["q0"], reqs["q1"]
+    steps = [([("q0", a[:67], list(range(67)))], [])]
+    for i in range(2):
+        steps.append(([("q0", [a[67 + i]], [0]), ("q1", b[40 * i:40 * i + 40], list(range(40)))], []))
+    steps.append(([("q0", [a[69]], [0]), ("q1", b[80:], list(range(20)))], ["q0", "q1"]))
+    seen.clear()
+    check_logits(sub, "bfloat16", util.run_schedule(runner, steps), "beside single rows")
+    assert seen.count((1, 41)) == 4 and seen.count((1, 21)) == 2
+    runner.release()
+
+
 def test_greedy_generation_through_the_scheduler(case):
     """The framework's own entry point: prompts of unequal length generated greedily by the
     scheduler (admission, portions under a token budget, batched decoding, sampling kernel),
