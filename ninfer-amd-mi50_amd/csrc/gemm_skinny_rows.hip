@@ -1,8 +1,9 @@
-// C = A W^T (+ bias, an activation, or gated) for a dense product of 17 to 512 rows (more than that for a router's few features): too many for a block that owns
-// all of them, too few to pay for the tiles of the many-row kernel.
+// C = A W^T (+ bias, an activation, or gated) for a dense product of 17 to 512 rows (more than that for a router's few
+// features): too many for a block that owns all of them, too few to pay for the tiles of the many-row kernel.
 //
 // A block owns 32 rows of A and up to 32 rows of W: two sets of up to 16 (of a gated product a set of the gate's and
-// the same of the other half's), or one set. Its 8 waves (a router's 8 or 16) split K, each a contiguous part walked in chunks of 128;
+// the same of the other half's), or one set. Its 8 waves (a router's 8 or 16) split K, each a contiguous part walked in
+// chunks of 128;
 // partial tiles meet in LDS and are summed in wave order, so a row's result depends neither on timing nor on the other
 // rows. Both operands are loaded as whole 128-byte lines (8 rows an instruction) and reach the matrix instruction's
 // layout through 2 KB of LDS per wave. The row parts of a feature tile lie side by side on one XCD
@@ -209,7 +210,9 @@ static RowsPlan plan_rows(const GemmArgs& a) {
   }
   p.sets = gated || f > 16 ? 2 : 1;
   p.rows = gated || p.sets == 1 ? f : (f + 1) / 2;
-  // (up to 128 features: as many waves as the few-row kernel, so that a router's sums are the same in either)
+  // (up to 128 features: as many waves as the few-row kernel has of a K of 1,024 and more while its blocks are fewer than
+  // eight a CU, so that a router's sums are the same in either; it has four of a shorter K or with more blocks. 16 go with one
+  // set: two sets are for blocks beyond two a CU)
   const int row_tiles = (a.M + 15) / 16;
   p.waves = a.N <= 128 && (a.N + 15) / 16 * row_tiles < device_cu_count() && a.K >= 2048 ? 16 : 8;
   const int of_block = gated ? p.rows : p.sets * p.rows;
@@ -228,7 +231,6 @@ int gemm_skinny_rows(const GemmArgs& a, hipStream_t stream) {
     constexpr bool AGAIN = decltype(again)::value;
     typedef decltype(tc) TC;
     if (epilogue_gated(a.epilogue)) gemm_skinny_rows_kernel<8, 2, true, AGAIN, TC><<<grid, block, 0, stream>>>(a, p);
-    else if (p.waves == 16 && p.sets == 2) gemm_skinny_rows_kernel<16, 2, false, AGAIN, TC><<<grid, block, 0, stream>>>(a, p);
     else if (p.waves == 16) gemm_skinny_rows_kernel<16, 1, false, AGAIN, TC><<<grid, block, 0, stream>>>(a, p);
     else if (p.sets == 2) gemm_skinny_rows_kernel<8, 2, false, AGAIN, TC><<<grid, block, 0, stream>>>(a, p);
     else gemm_skinny_rows_kernel<8, 1, false, AGAIN, TC><<<grid, block, 0, stream>>>(a, p);

@@ -282,6 +282,23 @@ def test_products_in_blocks_of_32_rows(ops, gen, m, n, k, gated):
         ops.force_generic = saved
 
 
+@pytest.mark.parametrize("n,k", [(61, 2048), (128, 1024), (17, 4096), (64, 1152), (8, 1024), (128, 2048)])
+def test_router_products_have_the_same_bits_in_either_kernel(ops, gen, n, k):
+    """512 rows in the few-row kernel, 513 in blocks of 32 rows, where both cut K alike: a row's logits are the same."""
+    x, w = rnd((513, k), torch.bfloat16, gen), rnd((n, k), torch.bfloat16, gen)
+    few, many = torch.empty(512, n, device="cuda"), torch.empty(513, n, device="cuda")
+    saved, ops.force_generic = ops.force_generic, False
+    try:
+        for m, out, kernel in ((512, few, 5), (513, many, 3)):
+            args = _gemm_args(m, n, k, 0)
+            args.out_dtype = 0
+            assert ops.lib.ninfer_gemm_kernel(ctypes.byref(args)) == kernel
+            ops.linear(x[:m].contiguous(), w, out)
+    finally:
+        ops.force_generic = saved
+    assert torch.equal(few, many[:512])
+
+
 def _gemm_args(m, n, k, epilogue):
     from ninfer_amd.kernels.ops import _GemmArgs
     a = _GemmArgs(4096, 4096, 4096)
