@@ -184,7 +184,10 @@ class Sampler:
             floats[3] = 0.0
         if drawn:
             to = floats[3] if len(drawn) == r else np.empty(len(drawn), np.float32)
-            if cuda:
+            # (us one by one 1.5 a row; in the library 5.5 to 6.6 for 1 to 8; as whole arrays 31 for 16 rows, 34 for 24)
+            if len(drawn) <= (3 if cuda else 20):
+                to[:] = [uniform(row.seed, row.key, row.draw) for row in drawn]
+            elif cuda:
                 self.ops.uniforms(*_streams(drawn), to)
             else:
                 to[:] = uniforms(drawn)

@@ -72,3 +72,22 @@ def test_what_the_kernel_is_given(rows, temperatures, penalties):
         assert got["pen_tokens"][at:at + len(toks)].tolist() == toks
         assert got["pen_counts"][at:at + len(toks)].tolist() == counts
         at += len(toks)
+
+
+@pytest.mark.parametrize("rows,arrays", [(1, False), (20, False), (21, True)])
+def test_few_rows_draw_one_by_one(monkeypatch, rows, arrays):
+    """The numbers of few rows do not pay for the arrays that those of many are laid out in."""
+    import ninfer_amd.sampling.sampler as sampler
+    asked = []
+    monkeypatch.setattr(sampler, "uniforms", lambda drawn: (asked.append(len(drawn)), uniforms(drawn))[1])
+
+    class Asked:
+        def sample(self, logits, temperature, uniform, out, **rest):
+            self.got = uniform.tolist()
+            out.zero_()
+
+    made = [SampleRow(SamplingParams(temperature=0.7 if i != 3 else 0.0), History([1]), key=i, draw=2, seed=9) for i in range(rows + (rows > 3))]
+    ops = Asked()
+    Sampler(ops, torch.device("cpu")).sample(torch.zeros(len(made), 10), made)
+    assert asked == [rows] * arrays
+    assert ops.got == [uniform(r.seed, r.key, r.draw) if r.params.temperature > 0 else 0 for r in made]
