@@ -169,8 +169,8 @@ def test_decode_rows_at_long_contexts(ops, name):
 @pytest.mark.parametrize("sink,learned,gated", [(True, False, False), (True, True, True), (False, False, True)])
 def test_decode_rows_with_a_sink_and_a_gate(ops, n_q, n_kv, d, window, sink, learned, gated):
     """Single rows of layers with a sink, its learned scores (one above every key's, one of minus infinity) and a gate in
-    columns of wider rows: the split-context kernels, a sink and gate in their merge, alone and before a
-    prompt's portion; and the kernels that cut by what a small workspace holds."""
+    columns of wider rows, alone and before a prompt's portion: the split-context kernels, a sink and gate in their
+    merge, and at the sizes where those do not pay the tiles of heads or the plain kernel."""
     g = torch.Generator(device="cuda").manual_seed(d)
     for seqs in ([(p, 1) for p in (700, 127, 128, 0, 511, 1300)], [(300, 1), (64, 1), (0, 70)]):
         case = shared_stream_case(seqs, n_q, n_kv, d, 16, torch.bfloat16, window)

@@ -460,7 +460,8 @@ def test_latent_attention_with_keys_and_values_per_head(ops, heads, rank, rd, vd
     ctx, pool, table, q, cached = _latent_case(ops, torch.bfloat16, heads, rank, rd, ps, lengths, new_rows, seed=rank)
     n = sum(1 for m in new_rows if m == 1)
     ctx.single_rows, ctx.portion_keys = n, sum(lengths[n:])
-    assert ops.latent_heads_rows(ctx, heads, dim, rank, rd, vdim, None) in (n, ctx.T)
+    # (few rows beside single ones may stay in the latent's space: tests/test_kernel_plans.py has the rule)
+    assert ops.latent_heads_rows(ctx, heads, dim, rank, rd, vdim, None) in ((n, ctx.T) if n else (0,))
     if lengths == [700]:
         table[0, 3], cached[0][3 * ps:4 * ps] = -1, 0     # a page that the table does not hold: zeros
     q = torch.randn(ctx.T, heads * 128, generator=g).bfloat16()
