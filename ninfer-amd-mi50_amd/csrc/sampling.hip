@@ -112,25 +112,59 @@ __device__ uint32_t radix_select(int V, unsigned long long target, RadixHist<COP
   return prefix;
 }
 
-__global__ __launch_bounds__(kSampleThreads) void sample_kernel(
-    const float* __restrict__ logits, int ld, int V, float* __restrict__ work,
-    const float* __restrict__ temperature, const int* __restrict__ top_k,
-    const float* __restrict__ top_p, const float* __restrict__ rep_penalty,
-    const int* __restrict__ pen_tokens, const int* __restrict__ pen_counts,
-    const int* __restrict__ pen_offsets, const float* __restrict__ uniform, int* __restrict__ out) {
-  __shared__ RadixHist<8> hist;
-  __shared__ unsigned long long sums[2 * kSampleThreads / 64];
-  __shared__ float fred[kSampleThreads / 64];
-  __shared__ int ired[kSampleThreads / 64];
+// What a call asks of its rows.
+struct SampleArgs {
+  const float* logits;   // [R, ld]
+  const float* temperature;
+  const int* top_k;      // or null, as the next two
+  const float* top_p;
+  const float* rep_penalty;
+  const int* pen_tokens;
+  const int* pen_counts;
+  const int* pen_offsets;
+  const float* uniform;
+  int* out;
+  float* work;           // [R, V]
+  int ld, V;
+};
 
-  const int r = blockIdx.x, tid = threadIdx.x;
-  const float* row = logits + (int64_t)r * ld;
-  float* w = work + (int64_t)r * V;
-  const float temp = temperature[r];
+struct RowLds {
+  RadixHist<8> hist;
+  unsigned long long sums[2 * kSampleThreads / 64];
+  float fred[kSampleThreads / 64];
+  int ired[kSampleThreads / 64];
+};
+
+__device__ __forceinline__ bool row_penalised(const SampleArgs& a, int r, float& rp) {
+  rp = a.rep_penalty ? a.rep_penalty[r] : 1.f;
+  return rp != 1.f && a.pen_offsets && a.pen_offsets[r + 1] > a.pen_offsets[r];
+}
+__device__ __forceinline__ float penalise(float v, float rp, int count) {
+  for (int c = 0; c < count; ++c) v = v > 0.f ? v / rp : v * rp;
+  return v;
+}
+
+// Row r by one block of kSampleThreads, every option and size.
+__device__ __forceinline__ void sample_whole_row(const SampleArgs& a, int r, RowLds& lds) {
+  RadixHist<8>& hist = lds.hist;
+  unsigned long long (&sums)[2 * kSampleThreads / 64] = lds.sums;
+  float (&fred)[kSampleThreads / 64] = lds.fred;
+  int (&ired)[kSampleThreads / 64] = lds.ired;
+  const int* pen_tokens = a.pen_tokens;
+  const int* pen_counts = a.pen_counts;
+  const int* pen_offsets = a.pen_offsets;
+  const int* top_k = a.top_k;
+  const float* top_p = a.top_p;
+  const float* uniform = a.uniform;
+  int* out = a.out;
+  const int V = a.V, tid = threadIdx.x;
+  const float* row = a.logits + (int64_t)r * a.ld;
+  float* w = a.work + (int64_t)r * V;
+  const float temp = a.temperature[r];
 
   // repetition penalty on a copy of the row (greedy rows without a penalty read the row itself)
-  float rp = rep_penalty ? rep_penalty[r] : 1.f;
-  const bool penalised = rp != 1.f && pen_offsets && pen_offsets[r + 1] > pen_offsets[r];
+  float rp;
+  const bool penalised = row_penalised(a, r, rp);
   if (!(temp > 0.f) && !penalised) {
     w = const_cast<float*>(row);
   } else {
@@ -148,9 +182,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
     for (int e = pen_offsets[r] + tid; e < pen_offsets[r + 1]; e += blockDim.x) {
       int tok = pen_tokens[e];
       if (tok < 0 || tok >= V) continue;
-      float v = w[tok];
-      for (int c = 0; c < pen_counts[e]; ++c) v = v > 0.f ? v / rp : v * rp;
-      w[tok] = v;
+      w[tok] = penalise(w[tok], rp, pen_counts[e]);
     }
   }
   __syncthreads();
@@ -376,311 +408,642 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
   if (mine > 0 && goal >= before && goal < before + mine) out[r] = (int)walk(before, true);
 }
 
-// Rows that keep few tokens (greedy, or top-k up to kCandPerSlice) in two launches that use the
-// whole GPU. First the row is cut into slices of kSlice tokens, one block each, which holds its
-// slice in LDS, applies the repetition penalty to it, and writes out, in index order, its own k best
-// tokens under the order (scaled logit descending, index ascending). Every token of the row's k
-// best is among its slice's k best, so the k best of all candidates are the row's, and the second
-// launch, a block per row, finds them and draws: the same kept set, masses and token as
-// sample_kernel's on the whole row.
-//
-// The k-th largest of n keys without a histogram: of the threads' largest keys, the k-th largest
-// is a bound that at least k keys reach, and hardly more do; those are listed and ranked among
-// themselves, each by a thread that compares it with all others. Lists that do not fit (many equal
-// logits) go through radix_select. 64 rows of 151,936 tokens with top-k 50: candidates 126 -> 36 us
-// and the draw 83 -> 21 us, against four and eight passes of a histogram (the keys share few upper
-// bytes, so its atomics follow each other, and one thread added the bins up).
-constexpr int kSlice = 4096;
-constexpr int kCandPerSlice = 64;
-constexpr int kCandThreads = 256;
-constexpr int kFewList = 256;
+__global__ __launch_bounds__(kSampleThreads) void sample_kernel(SampleArgs a) {
+  __shared__ RowLds lds;
+  sample_whole_row(a, blockIdx.x, lds);
+}
 
-struct FewLds {
-  uint4 best[kCandThreads / 4];   // the threads' largest keys, four by four
-  uint32_t key[kFewList];
-  int idx[kFewList];
-  int kept[kFewList];             // index of a kept one
-  uint32_t bound;
-  int count;
-  int wave_tot[kCandThreads / 64];
-  RadixHist<1> hist;
+// The same by the whole GPU, for rows that are greedy, keep at most kFewTokens tokens (top-k) or
+// cut nothing by top-k: the same kept set, masses and token. A row is cut into slices of kSlice
+// tokens, one block each.
+//
+// Few tokens kept, two launches. The slices' blocks apply the penalty and leave the largest key of
+// every thread's 16 tokens (sample_maxima_kernel). A block per row then finds a bound that at least
+// k tokens reach, from the largest keys of its own threads: the k-th largest of them. Hardly more than k
+// threads' keys of the first launch reach it; their tokens alone are read again, and those that reach the bound are ranked
+// among themselves, each by a thread that compares it with all others (sample_draw_kernel).
+// Bound by the one read of the logits and two chains of loads: 64 rows of 151,936 tokens with top-k 50 13 + 18 us (with
+// the k best of every slice found by its block, and the row's among those, 36 + 21); with top-k 200 35 in all, by
+// sample_whole_row 341; one row 15 and 23.
+//
+// Nothing cut by top-k, four launches: between the two, the slices' blocks add their tokens' masses into a
+// histogram of the row over the distance to its largest logit (sample_masses_kernel), then every
+// block finds in it the bin in which top-p cuts, sums its slice's mass above and lists its tokens of that bin
+// (sample_cut_kernel). The row's block finds the cut among the listed ones, the slice that holds the draw, and
+// the token in it. 64 rows of 151,936 tokens at top-p 0.95 73 to 84 us, by sample_whole_row 320; one row 30 and
+// 267; 32,000 tokens, one row, 30 and 74, with top-p 1 23 and 33; 6,000 tokens the same in both.
+//
+// Rows that fit neither, lists that do not fit (many equal logits) and rows with NaN or +infinity go through sample_whole_row.
+constexpr int kSlice = 4096;
+constexpr int kSliceThreads = 256;
+constexpr int kPerThread = kSlice / kSliceThreads;   // tokens of a subgroup: tid + kSliceThreads * u
+constexpr int kFewTokens = 256;
+constexpr int kSubs = 512;          // subgroups that a row's block reads again
+constexpr int kSubTable = 2048;     // places to look one of them up
+constexpr int kFewList = 1024;      // tokens that reach the bound
+constexpr int kBins = 512;          // of 1/16 in scaled logits: beyond 23 tokens have no mass
+constexpr float kBinsPerUnit = 16.f;
+constexpr int kCutList = 4096;      // tokens of the bin that top-p cuts
+constexpr int kMaxSlices = 1024;    // of a row whose draw may keep all
+
+struct SampleScratch {
+  uint32_t* maxima;             // [R, slices * kSliceThreads]
+  uint32_t* slice_max;          // [R, slices]
+  int* listed;                  // [R]: tokens in the row's list
+  uint2* list;                  // [R, kCutList]: key, token
+  unsigned long long* bins;     // [R, kBins]: masses
+  unsigned long long* slice_mass;   // [R, slices]: of the tokens above the cut's bin
+  int slices;
+  bool wide;                    // the launches between ran
 };
 
-// The k best of keys 0 .. n - 1 (1 <= k <= kCandPerSlice, k <= n): put(place, i) is called once for
-// each, places counted in index order. Every thread of the block must call.
-template <typename KeyFn, typename PutFn>
-__device__ void few_best(int n, int k, FewLds& l, KeyFn key, PutFn put) {
-  const int tid = threadIdx.x;
-  uint32_t mine = 0;
-  for (int i = tid; i < n; i += kCandThreads) mine = max(mine, key(i));
-  ((uint32_t*)l.best)[tid] = mine;
-  if (tid == 0) l.count = 0;
+enum RowKind : int { kRowFew, kRowWide, kRowOther };
+__device__ __forceinline__ RowKind row_kind(const SampleArgs& a, const SampleScratch& s, int r) {
+  const int k = a.top_k ? a.top_k[r] : 0;
+  if (!(a.temperature[r] > 0.f) || (k >= 1 && k <= kFewTokens)) return kRowFew;
+  return s.wide && (k <= 0 || k >= a.V) ? kRowWide : kRowOther;
+}
+__device__ __forceinline__ float row_inverse_temperature(const SampleArgs& a, int r) {
+  const float t = a.temperature[r];
+  return t > 0.f ? 1.f / t : 1.f;
+}
+__device__ __forceinline__ float key_value(uint32_t key) {   // ordered_key's inverse
+  return __uint_as_float((key & 0x80000000u) ? (key & 0x7fffffffu) : ~key);
+}
+// Above this key, that of the largest finite number, lie +infinity and NaN.
+constexpr uint32_t kFiniteKey = 0xff7fffffu;
+
+__device__ __forceinline__ int mass_bin(float scaled, float m) {   // the same or more for every smaller logit
+  return min(kBins - 1, (int)((m - scaled) * kBinsPerUnit));
+}
+
+// Wave-wide inclusive sums.
+__device__ __forceinline__ unsigned long long wave_sums(unsigned long long v) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const unsigned long long o = __shfl_up(v, d, 64);
+    if (lane >= d) v += o;
+  }
+  return v;
+}
+
+__global__ __launch_bounds__(kSliceThreads) void sample_maxima_kernel(SampleArgs a, SampleScratch s) {
+  __shared__ float vals[kSlice];
+  __shared__ uint32_t wave_max[kSliceThreads / 64];
+  const int r = blockIdx.y, b = blockIdx.x, tid = threadIdx.x;
+  const int s0 = b * kSlice, n = min(kSlice, a.V - s0);
+  const float* row = a.logits + (int64_t)r * a.ld + s0;
+  float x[kPerThread];   // every load on its way at once
+#pragma unroll
+  for (int u = 0; u < kPerThread; ++u) x[u] = row[min(tid + u * kSliceThreads, n - 1)];
+  const RowKind kind = row_kind(a, s, r);
+  if (kind == kRowOther) return;
+  float rp;
+  if (row_penalised(a, r, rp)) {
+    const int first = a.pen_offsets[r], end = a.pen_offsets[r + 1];
+    int pen[8];   // penalised tokens, eight at a time, the first beside the slice
+    auto load_pens = [&](int e0) {
+#pragma unroll
+      for (int u = 0; u < 8; ++u) pen[u] = a.pen_tokens[min(e0 + u * kSliceThreads, end - 1)];
+    };
+    load_pens(first + tid);
+#pragma unroll
+    for (int u = 0; u < kPerThread; ++u) vals[tid + u * kSliceThreads] = x[u];
+    __syncthreads();
+    for (int e0 = first + tid; e0 < end; e0 += 8 * kSliceThreads) {
+      if (e0 != first + tid) load_pens(e0);
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int e = e0 + u * kSliceThreads, t = pen[u] - s0;
+        if (e < end && t >= 0 && t < n) vals[t] = penalise(vals[t], rp, a.pen_counts[e]);
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kPerThread; ++u) x[u] = vals[tid + u * kSliceThreads];
+    if (kind == kRowWide) {
+      float* w = a.work + (int64_t)r * a.V + s0;
+#pragma unroll
+      for (int u = 0; u < kPerThread; ++u)
+        if (tid + u * kSliceThreads < n) w[tid + u * kSliceThreads] = x[u];
+    }
+  }
+  const float inv_t = row_inverse_temperature(a, r);
+  uint32_t best = 0;   // (below every number's key)
+#pragma unroll
+  for (int u = 0; u < kPerThread; ++u)
+    if (tid + u * kSliceThreads < n) best = max(best, ordered_key(x[u] * inv_t));
+  s.maxima[((int64_t)r * s.slices + b) * kSliceThreads + tid] = best;
+  if (kind != kRowWide) return;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) best = max(best, (uint32_t)__shfl_xor((int)best, off, 64));
+  if ((tid & 63) == 0) wave_max[tid >> 6] = best;
+  // the row's bins and list start empty
+  for (int i = b * kSliceThreads + tid; i < kBins; i += s.slices * kSliceThreads) s.bins[(int64_t)r * kBins + i] = 0;
+  if (b == 0 && tid == 0) s.listed[r] = 0;
   __syncthreads();
-  if (tid < 64) {   // the k-th largest of the 256, bit by bit: the largest bound that k of them reach
+  if (tid == 0) {
+#pragma unroll
+    for (int w = 1; w < kSliceThreads / 64; ++w) best = max(best, wave_max[w]);
+    s.slice_max[(int64_t)r * s.slices + b] = best;
+  }
+}
+
+// The largest key of a row, by every wave for itself.
+__device__ __forceinline__ uint32_t row_max(const SampleScratch& s, int r) {
+  uint32_t best = 0;
+  for (int i = threadIdx.x & 63; i < s.slices; i += 64) best = max(best, s.slice_max[(int64_t)r * s.slices + i]);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) best = max(best, (uint32_t)__shfl_xor((int)best, off, 64));
+  return best;
+}
+
+__device__ __forceinline__ const float* wide_row(const SampleArgs& a, int r) {
+  float rp;
+  return row_penalised(a, r, rp) ? a.work + (int64_t)r * a.V : a.logits + (int64_t)r * a.ld;
+}
+
+__global__ __launch_bounds__(kSliceThreads) void sample_masses_kernel(SampleArgs a, SampleScratch s) {
+  __shared__ unsigned long long bins[kBins];
+  const int r = blockIdx.y, b = blockIdx.x, tid = threadIdx.x;
+  if (row_kind(a, s, r) != kRowWide) return;
+  const int s0 = b * kSlice, n = min(kSlice, a.V - s0);
+  const float* row = wide_row(a, r) + s0;
+  float x[kPerThread];
+#pragma unroll
+  for (int u = 0; u < kPerThread; ++u) x[u] = row[min(tid + u * kSliceThreads, n - 1)];
+  for (int i = tid; i < kBins; i += kSliceThreads) bins[i] = 0;
+  const uint32_t most = row_max(s, r);
+  if (most > kFiniteKey) return;
+  const float m = key_value(most), inv_t = row_inverse_temperature(a, r);
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < kPerThread; ++u) {
+    const float scaled = x[u] * inv_t;
+    const unsigned long long mass = token_mass(scaled, m);
+    if (tid + u * kSliceThreads < n && mass) atomicAdd(&bins[mass_bin(scaled, m)], mass);
+  }
+  __syncthreads();
+  for (int i = tid; i < kBins; i += kSliceThreads)
+    if (bins[i]) atomicAdd(&s.bins[(int64_t)r * kBins + i], bins[i]);
+}
+
+// Where top-p cuts a row, by the first wave from its bins: the bin (kBins: nothing is cut), the mass of the bins
+// above it, the mass that is to be kept, and of all.
+struct Cut {
+  int bin;
+  unsigned long long above, target, total;
+};
+__device__ __forceinline__ void find_cut(const SampleArgs& a, const SampleScratch& s, int r, Cut& cut) {
+  typedef unsigned long long u64;
+  constexpr int EACH = kBins / 64;
+  const int lane = threadIdx.x & 63;
+  const u64* bins = s.bins + (int64_t)r * kBins + EACH * lane;
+  u64 bin[EACH], mine = 0;
+#pragma unroll
+  for (int i = 0; i < EACH; ++i) bin[i] = bins[i];
+#pragma unroll
+  for (int i = 0; i < EACH; ++i) mine += bin[i];
+  const u64 incl = wave_sums(mine), total = __shfl(incl, 63, 64);
+  const float pp = a.top_p ? a.top_p[r] : 1.f;
+  u64 target = (u64)((double)pp * (double)total);
+  if (target < 1) target = 1;
+  const u64 hit = __ballot(incl >= target);
+  const bool cuts = pp < 1.f && hit;
+  if (lane == (cuts ? __ffsll(hit) - 1 : 63)) {
+    u64 run = incl - mine;
+    int x = 0;
+#pragma unroll
+    for (int i = 0; i < EACH - 1; ++i)
+      if (x == i && run + bin[i] < target) run += bin[i], ++x;
+    cut.bin = cuts ? EACH * lane + x : kBins;
+    cut.above = cuts ? run : total;
+    cut.target = target;
+    cut.total = total;
+  }
+}
+
+__global__ __launch_bounds__(kSliceThreads) void sample_cut_kernel(SampleArgs a, SampleScratch s) {
+  __shared__ Cut cut;
+  __shared__ unsigned long long sums[kSliceThreads / 64];
+  __shared__ uint2 list[kSlice];   // (its own first: one place in the row's list is asked for a block)
+  __shared__ int listed, place;
+  const int r = blockIdx.y, b = blockIdx.x, tid = threadIdx.x;
+  if (row_kind(a, s, r) != kRowWide) return;
+  if (tid == 0) listed = 0;
+  const int s0 = b * kSlice, n = min(kSlice, a.V - s0);
+  const float* row = wide_row(a, r) + s0;
+  float x[kPerThread];
+#pragma unroll
+  for (int u = 0; u < kPerThread; ++u) x[u] = row[min(tid + u * kSliceThreads, n - 1)];
+  const uint32_t most = row_max(s, r);
+  if (most > kFiniteKey) return;
+  const float m = key_value(most), inv_t = row_inverse_temperature(a, r);
+  if (tid < 64) find_cut(a, s, r, cut);
+  __syncthreads();
+  const int cut_bin = cut.bin;
+  unsigned long long above = 0;
+#pragma unroll
+  for (int u = 0; u < kPerThread; ++u) {
+    const float scaled = x[u] * inv_t;
+    const unsigned long long mass = token_mass(scaled, m);
+    if (tid + u * kSliceThreads >= n || !mass) continue;
+    const int bin = mass_bin(scaled, m);
+    if (bin < cut_bin) above += mass;
+    else if (bin == cut_bin) list[atomicAdd(&listed, 1)] = make_uint2(ordered_key(scaled), s0 + tid + u * kSliceThreads);
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) above += __shfl_xor(above, off, 64);
+  if ((tid & 63) == 0) sums[tid >> 6] = above;
+  __syncthreads();
+  if (tid == 0) {
+#pragma unroll
+    for (int w = 1; w < kSliceThreads / 64; ++w) above += sums[w];
+    s.slice_mass[(int64_t)r * s.slices + b] = above;
+    place = listed ? atomicAdd(&s.listed[r], listed) : 0;
+  }
+  __syncthreads();
+  for (int i = tid; i < listed && place + i < kCutList; i += kSliceThreads) s.list[(int64_t)r * kCutList + place + i] = list[i];
+}
+
+union DrawLds {
+  RowLds row;
+  struct {
+    float vals[kSubs * kPerThread];
+    unsigned long long tokens[kFewList + 8];   // key, then the token's complement: in the order by which tokens are kept
+    unsigned kept[kFewList + 16];              // token of a kept one, else the largest number
+    unsigned long long by_rank[kFewTokens], by_place[kFewTokens];   // masses
+    int place_of[kFewTokens], token_at[kFewTokens];                 // of a rank; at a place
+    int sub[kSubs];
+    uint32_t place_of_sub[kSubTable];       // (subgroup + 1) * kSubs + its place in `sub`, hashed, or 0
+    uint4 best[kSampleThreads / 4];
+    int subs, listed;
+    uint32_t bound, nan;
+  } few;
+  struct {
+    uint2 list[kCutList];
+    unsigned long long slice[kMaxSlices];
+    RadixHist<1> hist;
+    unsigned long long sums[kSampleThreads / 64];
+    int ranks[kSampleThreads / 64];
+    unsigned ties[kCutList];   // tokens with the threshold's key
+    Cut cut;
+    unsigned long long mass_gt, before;
+    int cnt_eq, cnt_before, at;
+  } wide;
+};
+
+// The largest bound of 20 bits that k of the block's threads' keys reach (0 if fewer are numbers); of 17 bits, which a few tokens
+// more reach, beyond 64. Of up to 64 the keys of four threads count as one, their largest.
+__device__ __forceinline__ void few_bound(uint32_t mine, int k, DrawLds& lds) {
+  const int tid = threadIdx.x;
+  auto& l = lds.few;
+  if (k <= 64) {
+    mine = max(mine, (uint32_t)__shfl_xor((int)mine, 1, 64));
+    mine = max(mine, (uint32_t)__shfl_xor((int)mine, 2, 64));
+    if (tid % 4 == 0) ((uint32_t*)l.best)[tid / 4] = mine;
+  } else {
+    ((uint32_t*)l.best)[tid] = mine;
+  }
+  __syncthreads();
+  if (tid >= 64) return;
+  uint32_t bound = 0;
+  if (k <= 64) {
     const uint4 m = l.best[tid];
-    uint32_t bound = 0;
-    for (int bit = 31; bit >= 0; --bit) {
+    for (int bit = 31; bit >= 12; --bit) {
       const uint32_t at = bound | (1u << bit);
       const int reach = __popcll(__ballot(m.x >= at)) + __popcll(__ballot(m.y >= at)) +
                         __popcll(__ballot(m.z >= at)) + __popcll(__ballot(m.w >= at));
       if (reach >= k) bound = at;
     }
-    if (tid == 0) l.bound = bound;
+  } else {
+    uint4 m[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) m[i] = l.best[tid + 64 * i];
+    for (int bit = 31; bit >= 15; --bit) {
+      const uint32_t at = bound | (1u << bit);
+      int reach = 0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        reach += __popcll(__ballot(m[i].x >= at)) + __popcll(__ballot(m[i].y >= at)) +
+                 __popcll(__ballot(m[i].z >= at)) + __popcll(__ballot(m[i].w >= at));
+      if (reach >= k) bound = at;
+    }
   }
+  if (tid == 0) l.bound = bound;
+}
+
+// A row that keeps few tokens; got: the first of the row's keys that are this thread's. False: through sample_whole_row.
+constexpr int kLookKeys = 12;
+__device__ __forceinline__ bool draw_few(const SampleArgs& a, const SampleScratch& s, int r, DrawLds& lds,
+                                         const uint32_t (&got)[kLookKeys]) {
+  constexpr int LOOK = kLookKeys;
+  typedef unsigned long long u64;
+  auto& l = lds.few;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int groups = s.slices * kSliceThreads;
+  if (groups >= 1 << 22) return false;   // (their numbers share 32 bits with a place)
+  const uint32_t* maxima = s.maxima + (int64_t)r * groups;
+  const float temp = a.temperature[r], inv_t = row_inverse_temperature(a, r);
+  const int k = min(temp > 0.f ? a.top_k[r] : 1, a.V);
+  float rp;
+  const bool penalised = row_penalised(a, r, rp);
+  const int first = penalised ? a.pen_offsets[r] : 0, end = penalised ? a.pen_offsets[r + 1] : 0;
+  constexpr int PENS = 2;   // of a thread, on their way beside the keys
+  int pen[PENS];
+#pragma unroll
+  for (int u = 0; u < PENS; ++u) pen[u] = end > first ? a.pen_tokens[min(first + tid + u * kSampleThreads, end - 1)] : 0;
+
+  uint32_t mine = 0;
+#pragma unroll
+  for (int u = 0; u < LOOK; ++u) mine = max(mine, got[u]);
+  for (int g = tid + LOOK * kSampleThreads; g < groups; g += kSampleThreads) mine = max(mine, maxima[g]);
+  for (int i = tid; i < kSubTable; i += kSampleThreads) l.place_of_sub[i] = 0;
+  if (tid == 0) l.subs = l.listed = 0, l.nan = 0;
+  few_bound(mine, k, lds);
   __syncthreads();
   const uint32_t bound = l.bound;
-  for (int i = tid; i < n; i += kCandThreads) {
-    const uint32_t kk = key(i);
-    if (kk >= bound) {
-      const int at = atomicAdd(&l.count, 1);
-      if (at < kFewList) {
-        l.key[at] = kk;
-        l.idx[at] = i;
-      }
-    }
+  auto slot_of = [](int g) { return (unsigned)g * 2654435761u >> 21; };
+  static_assert(kSubTable == 1 << 11, "slot_of has 11 bits");
+  auto take = [&](int g, uint32_t key) {   // (key 0: no token)
+    if (key < bound || key == 0) return;
+    const int at = atomicAdd(&l.subs, 1);
+    if (at >= kSubs) return;
+    l.sub[at] = g;
+    // (a quarter of the places at most is taken: the search ends)
+    for (unsigned h = slot_of(g); penalised && atomicCAS(&l.place_of_sub[h], 0u, (g + 1u) * kSubs + at); h = (h + 1) % kSubTable) {}
+  };
+  if (mine >= bound) {
+#pragma unroll
+    for (int u = 0; u < LOOK; ++u) take(tid + u * kSampleThreads, got[u]);
+    for (int g = tid + LOOK * kSampleThreads; g < groups; g += kSampleThreads) take(g, maxima[g]);
   }
   __syncthreads();
-  const int count = l.count;
-  if (count <= kFewList) {
-    const int padded = (count + 15) / 16 * 16;
-    if (tid >= count && tid < padded) {   // places that nothing follows and nothing counts
-      l.key[tid] = 0;
-      l.idx[tid] = 0x7fffffff;
-      l.kept[tid] = 0x7fffffff;
-    }
-    __syncthreads();
-    uint32_t kk = 0;
-    int i = 0, better = 0;
-    if (tid < count) {
-      kk = l.key[tid];
-      i = l.idx[tid];
-#pragma unroll 16
-      for (int j = 0; j < padded; ++j) better += l.key[j] > kk || (l.key[j] == kk && l.idx[j] < i);
-      l.kept[tid] = better < k ? i : 0x7fffffff;
-    }
-    __syncthreads();
-    if (tid < count && better < k) {
-      int place = 0;
-#pragma unroll 16
-      for (int j = 0; j < padded; ++j) place += l.kept[j] < i;
-      put(place, i);
-    }
-    __syncthreads();
-    return;
-  }
-  const uint32_t thr = k < n ? radix_select(n, (unsigned long long)k, l.hist, key, [](int, uint32_t) { return 1ull; }) : 0;
-  auto block_count = [&](int v) -> int {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    if ((tid & 63) == 0) l.wave_tot[tid >> 6] = v;
-    __syncthreads();
-    v = 0;
-    for (int i = 0; i < kCandThreads / 64; ++i) v += l.wave_tot[i];
-    __syncthreads();
-    return v;
+  const int subs = l.subs;
+  if (subs > kSubs) return false;
+  const float* row = a.logits + (int64_t)r * a.ld;
+  auto token_of = [&](int i) {   // of place i of `vals`
+    const int g = l.sub[i / kPerThread];
+    return g / kSliceThreads * kSlice + g % kSliceThreads + i % kPerThread * kSliceThreads;
   };
-  int above = 0;
-  for (int i = tid; i < n; i += kCandThreads) above += key(i) > thr;
-  const int quota = k - block_count(above);   // of the keys tied at thr, the first so many
-  auto scan = [&](int v) -> int {   // sum over the threads before this one
-    const int lane = tid & 63, wv = tid >> 6;
-    int incl = v;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const int o = __shfl_up(incl, d, 64);
-      if (lane >= d) incl += o;
-    }
-    if (lane == 63) l.wave_tot[wv] = incl;
-    __syncthreads();
-    int base = 0;
-    for (int i = 0; i < wv; ++i) base += l.wave_tot[i];
-    __syncthreads();
-    return base + incl - v;
-  };
-  const int run = (n + kCandThreads - 1) / kCandThreads, i0 = min(n, tid * run), i1 = min(n, i0 + run);
-  int eq = 0;
-  for (int i = i0; i < i1; ++i) eq += key(i) == thr;
-  const int rank0 = scan(eq);
-  int kept = 0, tie = rank0;
-  for (int i = i0; i < i1; ++i) {
-    const uint32_t kk = key(i);
-    kept += kk > thr || (kk == thr && tie++ < quota);
-  }
-  int place = scan(kept);
-  tie = rank0;
-  for (int i = i0; i < i1; ++i) {
-    const uint32_t kk = key(i);
-    if (kk > thr || (kk == thr && tie++ < quota)) put(place++, i);
-  }
-  __syncthreads();
-}
-
-__global__ __launch_bounds__(kCandThreads) void sample_candidates_kernel(
-    const float* __restrict__ logits, int ld, int V, const float* __restrict__ temperature,
-    const int* __restrict__ top_k, const float* __restrict__ rep_penalty,
-    const int* __restrict__ pen_tokens, const int* __restrict__ pen_counts,
-    const int* __restrict__ pen_offsets, float* __restrict__ cand_val, int* __restrict__ cand_idx) {
-  __shared__ float vals[kSlice];
-  __shared__ FewLds l;
-  const int r = blockIdx.y, b = blockIdx.x, tid = threadIdx.x;
-  const int s0 = b * kSlice, n = min(kSlice, V - s0);
-  const int C = gridDim.x * kCandPerSlice;
-  const float* row = logits + (int64_t)r * ld;
-  float x[kSlice / kCandThreads];   // every load on its way at once
-#pragma unroll
-  for (int u = 0; u < kSlice / kCandThreads; ++u) x[u] = row[s0 + min(tid + u * kCandThreads, n - 1)];
-  const float rp = rep_penalty ? rep_penalty[r] : 1.f;
-  const bool penalised = rp != 1.f && pen_offsets && pen_offsets[r + 1] > pen_offsets[r];
-  const int first_pen = penalised ? pen_offsets[r] : 0, end_pen = penalised ? pen_offsets[r + 1] : 0;
-  int pen[8];   // penalised tokens, eight at a time, the first beside the slice
-  auto load_pens = [&](int e0) {
-#pragma unroll
-    for (int u = 0; u < 8; ++u) pen[u] = pen_tokens[min(e0 + u * kCandThreads, end_pen - 1)];
-  };
-  if (penalised) load_pens(first_pen + tid);
-#pragma unroll
-  for (int u = 0; u < kSlice / kCandThreads; ++u) vals[tid + u * kCandThreads] = x[u];
+  for (int i = tid; i < subs * kPerThread; i += kSampleThreads) l.vals[i] = row[min(token_of(i), a.V - 1)];
   __syncthreads();
   if (penalised) {
-    for (int e0 = first_pen + tid; e0 < end_pen; e0 += 8 * kCandThreads) {
-      if (e0 != first_pen + tid) load_pens(e0);
+    auto apply = [&](int e, int t) {
+      if (e >= end || t < 0 || t >= a.V) return;
+      const int g = t / kSlice * kSliceThreads + t % kSliceThreads;
+      uint32_t found = 0;
+      for (unsigned h = slot_of(g); (found = l.place_of_sub[h]) != 0 && found / kSubs != g + 1u; h = (h + 1) % kSubTable) {}
+      if (!found) return;
+      float& v = l.vals[found % kSubs * kPerThread + t % kSlice / kSliceThreads];
+      v = penalise(v, rp, a.pen_counts[e]);
+    };
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int e = e0 + u * kCandThreads, t = pen[u] - s0;
-        if (e >= end_pen || t < 0 || t >= n) continue;
-        float v = vals[t];
-        for (int c = 0; c < pen_counts[e]; ++c) v = v > 0.f ? v / rp : v * rp;
-        vals[t] = v;
-      }
-    }
+    for (int u = 0; u < PENS; ++u) apply(first + tid + u * kSampleThreads, pen[u]);
+    for (int e = first + tid + PENS * kSampleThreads; e < end; e += kSampleThreads) apply(e, a.pen_tokens[e]);
     __syncthreads();
   }
-  const float temp = temperature[r];
-  const float inv_t = temp > 0.f ? 1.f / temp : 1.f;
-  int k = temp > 0.f ? top_k[r] : 1;            // greedy is the best one
-  if (k < 1 || k > kCandPerSlice) k = kCandPerSlice;   // (not this entry's rows: kept in bounds)
-  k = min(k, n);
-  float* cv = cand_val + (int64_t)r * C + b * kCandPerSlice;
-  int* ci = cand_idx + (int64_t)r * C + b * kCandPerSlice;
-  few_best(n, k, l, [&](int i) { return ordered_key(vals[i] * inv_t); },
-           [&](int place, int i) {
-             cv[place] = vals[i];
-             ci[place] = s0 + i;
-           });
-  // the places left over hold nothing: never the largest, no mass
-  for (int i = k + tid; i < kCandPerSlice; i += kCandThreads) {
-    cv[i] = -INFINITY;
-    ci[i] = 0;
-  }
-}
-
-// The draw among a row's C candidates (in index order); sample_kernel says what it is. STAGED: they
-// fit LDS (vocabularies of up to 262,144 tokens).
-template <bool STAGED>
-__global__ __launch_bounds__(kCandThreads) void sample_few_kernel(
-    const float* __restrict__ cand_val, const int* __restrict__ cand_idx, int C,
-    const float* __restrict__ temperature, const int* __restrict__ top_k, const float* __restrict__ top_p,
-    const float* __restrict__ uniform, int* __restrict__ out) {
-  typedef unsigned long long u64;
-  __shared__ FewLds l;
-  __shared__ float fred[kCandThreads / 64];
-  __shared__ int ired[kCandThreads / 64];
-  __shared__ float val_s[kCandPerSlice];
-  __shared__ int idx_s[kCandPerSlice];
-  __shared__ u64 mass_s[kCandPerSlice];
-  __shared__ uint32_t key_s[kCandPerSlice];
-  const int r = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
-  __shared__ float staged[STAGED ? kSlice : 1];
-  const float* row = cand_val + (int64_t)r * C;
-  const int* idx = cand_idx + (int64_t)r * C;
-  if (STAGED) {
-    float x[kSlice / kCandThreads];
-#pragma unroll
-    for (int u = 0; u < kSlice / kCandThreads; ++u) x[u] = row[min(tid + u * kCandThreads, C - 1)];
-#pragma unroll
-    for (int u = 0; u < kSlice / kCandThreads; ++u) staged[tid + u * kCandThreads] = x[u];
-    __syncthreads();
-  }
-  auto value = [&](int i) { return STAGED ? staged[i] : row[i]; };
-  float best = -INFINITY;
-  int best_i = 0x7fffffff;
-  for (int i = tid; i < C; i += kCandThreads) {
-    const float v = value(i);
-    if (v > best) {
-      best = v;
-      best_i = i;
-    }
-  }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    const float ob = __shfl_xor(best, off, 64);
-    const int oi = __shfl_xor(best_i, off, 64);
-    if (ob > best || (ob == best && oi < best_i)) {
-      best = ob;
-      best_i = oi;
-    }
-  }
-  if (lane == 0) {
-    fred[tid >> 6] = best;
-    ired[tid >> 6] = best_i;
+  for (int i = tid; i < subs * kPerThread; i += kSampleThreads) {
+    const int t = token_of(i);
+    const uint32_t key = ordered_key(l.vals[i] * inv_t);
+    if (t >= a.V || key < bound) continue;
+    if (key > kFiniteKey) l.nan = 1;
+    const int at = atomicAdd(&l.listed, 1);
+    if (at < kFewList) l.tokens[at] = (u64)key << 32 | (0xffffffffu - (unsigned)t);
   }
   __syncthreads();
-  best = fred[0];
-  best_i = ired[0];
-  for (int i = 1; i < kCandThreads / 64; ++i)
-    if (fred[i] > best || (fred[i] == best && ired[i] < best_i)) {
-      best = fred[i];
-      best_i = ired[i];
-    }
-  const float temp = temperature[r];
-  if (!(temp > 0.f)) {
-    // (a row without a number above minus infinity: the first place)
-    if (tid == 0) out[r] = idx[best_i < C ? best_i : 0];
-    return;
+  const int count = l.listed;
+  if (count > kFewList || l.nan || count < k) return false;
+  if (tid < 16) {   // places that nothing follows and nothing counts
+    if (tid < 8) l.tokens[count + tid] = 0;
+    l.kept[count + tid] = 0xffffffffu;
   }
-  const float inv_t = 1.f / temp, m = best * inv_t;
-  int k = top_k[r];
-  if (k < 1 || k > kCandPerSlice) k = kCandPerSlice;
-  few_best(C, k, l, [&](int i) { return ordered_key(value(i) * inv_t); },
-           [&](int place, int i) {
-             val_s[place] = value(i);
-             idx_s[place] = idx[i];
-           });
-  if (tid >= 64) return;
-  // One wave: lane j has the j-th kept token in index order. Its mass, and that of the tokens before
-  // it in the order (logit descending, index ascending): top-p keeps those before the target.
-  const bool have = lane < k;
-  const uint32_t kk = have ? ordered_key(val_s[lane] * inv_t) : 0;
-  const u64 mass = have ? token_mass(val_s[lane] * inv_t, m) : 0;
-  mass_s[lane] = mass;
-  key_s[lane] = kk;
-  // (one wave: its LDS accesses run in order, and the fence keeps the compiler from changing that)
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  u64 total = 0, ahead = 0;
-#pragma unroll 8
-  for (int j = 0; j < kCandPerSlice; ++j) {   // (places from k on have no mass)
-    const u64 o = mass_s[j];
-    total += o;
-    if (key_s[j] > kk || (key_s[j] == kk && j < lane)) ahead += o;
+  __syncthreads();
+  // Four threads a token: how many come before it, of every fourth pair of them each.
+  const int part = tid & 3;
+  auto before = [&](int mine) {
+    mine += __shfl_xor(mine, 1, 64);
+    return mine + __shfl_xor(mine, 2, 64);
+  };
+  const int rounds = (count + kSampleThreads / 4 - 1) / (kSampleThreads / 4);
+  int rank[kFewList / (kSampleThreads / 4)];
+#pragma unroll
+  for (int i = 0; i < kFewList / (kSampleThreads / 4); ++i) {
+    rank[i] = k;
+    const int e = tid / 4 + i * (kSampleThreads / 4);
+    if (i >= rounds || e >= count) continue;
+    const u64 mine = l.tokens[e];
+    int n = 0;
+#pragma unroll 4
+    for (int j = 2 * part; j < count; j += 8) n += (l.tokens[j] > mine) + (l.tokens[j + 1] > mine);
+    rank[i] = before(n);
+    if (part) continue;
+    const unsigned token = 0xffffffffu - (unsigned)mine;
+    if (rank[i] == 0 && !(temp > 0.f)) a.out[r] = (int)token;
+    l.kept[e] = rank[i] < k ? token : 0xffffffffu;
+    if (rank[i] < k) l.by_rank[rank[i]] = mine >> 32;   // (its key)
   }
-  const float pp = top_p ? top_p[r] : 1.f;
+  if (!(temp > 0.f)) return true;
+  __syncthreads();
+  const float m = key_value((uint32_t)l.by_rank[0]);   // the largest scaled logit
+#pragma unroll
+  for (int i = 0; i < kFewList / (kSampleThreads / 4); ++i) {
+    const int e = tid / 4 + i * (kSampleThreads / 4);
+    if (i >= rounds || rank[i] >= k) continue;
+    const unsigned mine = l.kept[e];
+    int n = 0;
+#pragma unroll 4
+    for (int j = 4 * part; j < count; j += 16)
+      n += (l.kept[j] < mine) + (l.kept[j + 1] < mine) + (l.kept[j + 2] < mine) + (l.kept[j + 3] < mine);
+    const int place = before(n);
+    if (part) continue;
+    l.place_of[rank[i]] = place;
+    l.token_at[place] = (int)mine;
+  }
+  __syncthreads();
+  if (tid >= 64) return true;
+  // One wave: masses by rank, of which those before the target are kept, then by place, where the draw is.
+  constexpr int EACH = kFewTokens / 64;
+  u64 here[EACH], sum = 0;
+#pragma unroll
+  for (int i = 0; i < EACH; ++i) {
+    const int at = EACH * lane + i;
+    here[i] = at < k ? token_mass(key_value((uint32_t)l.by_rank[at]), m) : 0;
+    sum += here[i];
+  }
+  u64 incl = wave_sums(sum);
+  u64 total = __shfl(incl, 63, 64);
+  const float pp = a.top_p ? a.top_p[r] : 1.f;
   u64 target = total;
   if (pp < 1.f) {
     target = (u64)((double)pp * (double)total);
     if (target < 1) target = 1;
   }
-  const u64 kept = have && ahead < target ? mass : 0;
-  u64 incl = kept;
+  u64 run = incl - sum;
 #pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const u64 o = __shfl_up(incl, d, 64);
-    if (lane >= d) incl += o;
+  for (int i = 0; i < EACH; ++i) {
+    if (EACH * lane + i < k) l.by_place[l.place_of[EACH * lane + i]] = run < target ? here[i] : 0;
+    run += here[i];
   }
+  // (one wave: its LDS accesses run in order, and the fence keeps the compiler from changing that)
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  sum = 0;
+#pragma unroll
+  for (int i = 0; i < EACH; ++i) {
+    here[i] = EACH * lane + i < k ? l.by_place[EACH * lane + i] : 0;
+    sum += here[i];
+  }
+  incl = wave_sums(sum);
   total = __shfl(incl, 63, 64);
-  u64 goal = (u64)((double)uniform[r] * (double)total);
+  u64 goal = (u64)((double)a.uniform[r] * (double)total);
   if (goal >= total) goal = total - 1;
-  if (kept > 0 && goal >= incl - kept && goal < incl) out[r] = idx_s[lane];
+  run = incl - sum;
+#pragma unroll
+  for (int i = 0; i < EACH; ++i) {
+    if (here[i] > 0 && goal >= run && goal < run + here[i]) a.out[r] = l.token_at[EACH * lane + i];
+    run += here[i];
+  }
+  return true;
+}
+
+// A row of which top-k cuts nothing. False: through sample_whole_row.
+__device__ __forceinline__ bool draw_wide(const SampleArgs& a, const SampleScratch& s, int r, DrawLds& lds) {
+  typedef unsigned long long u64;
+  auto& l = lds.wide;
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const uint32_t most = row_max(s, r);
+  if (most > kFiniteKey) return false;
+  const float m = key_value(most), inv_t = row_inverse_temperature(a, r);
+  const int n = s.listed[r];
+  if (n > kCutList) return false;
+  if (wv == 0) find_cut(a, s, r, l.cut);
+  for (int i = tid; i < n; i += kSampleThreads) l.list[i] = s.list[(int64_t)r * kCutList + i];
+  for (int i = tid; i < s.slices; i += kSampleThreads) l.slice[i] = s.slice_mass[(int64_t)r * s.slices + i];
+  if (tid == 0) l.mass_gt = 0, l.cnt_eq = 0;
+  __syncthreads();
+  // Kept are the tokens above key `thr` and of those with it the first `quota` in index order.
+  uint32_t thr = 0;
+  u64 total = l.cut.total, quota = ~0ull, mass_thr = 0;
+  auto mass_of = [&](uint32_t key) { return token_mass(key_value(key), m); };
+  if (l.cut.bin < kBins) {
+    thr = radix_select(n, l.cut.target - l.cut.above, l.hist, [&](int i) { return l.list[i].x; },
+                       [&](int, uint32_t key) { return mass_of(key); });
+    u64 gt = 0;
+    for (int i = tid; i < n; i += kSampleThreads) {
+      const uint2 e = l.list[i];
+      if (e.x > thr) gt += mass_of(e.x);
+      else if (e.x == thr) l.ties[atomicAdd(&l.cnt_eq, 1)] = e.y;
+    }
+    if (gt) atomicAdd(&l.mass_gt, gt);
+    __syncthreads();
+    mass_thr = mass_of(thr);
+    quota = (u64)l.cnt_eq;
+    const u64 mass_gt = l.cut.above + l.mass_gt;
+    if (mass_thr > 0) {
+      const u64 need = (l.cut.target - mass_gt + mass_thr - 1) / mass_thr;
+      if (need < quota) quota = need;
+    }
+    total = mass_gt + quota * mass_thr;
+    // the listed tokens that are kept count in their slices
+    for (int i = tid; i < n; i += kSampleThreads) {
+      const uint2 e = l.list[i];
+      bool kept = e.x > thr;
+      if (e.x == thr) {
+        u64 rank = 0;
+        if (quota < (u64)l.cnt_eq)
+          for (int j = 0; j < l.cnt_eq; ++j) rank += l.ties[j] < e.y;
+        kept = rank < quota;
+      }
+      if (kept) atomicAdd(&l.slice[e.y / kSlice], mass_of(e.x));
+    }
+    __syncthreads();
+  }
+  u64 goal = (u64)((double)a.uniform[r] * (double)total);
+  if (goal >= total) goal = total - 1;
+  if (wv == 0) {   // the slice that holds the goal
+    u64 run = 0;
+    int at = s.slices - 1;
+    for (int b0 = 0; b0 < s.slices; b0 += 64) {
+      const u64 mine = b0 + lane < s.slices ? l.slice[b0 + lane] : 0;
+      const u64 incl = run + wave_sums(mine);
+      const u64 hit = __ballot(goal < incl);
+      if (hit) {
+        const int first = __ffsll(hit) - 1;
+        at = b0 + first;
+        run = __shfl(incl - mine, first, 64);
+        break;
+      }
+      run = __shfl(incl, 63, 64);
+    }
+    if (lane == 0) l.at = at, l.before = run, l.cnt_before = 0;
+  }
+  __syncthreads();
+  const int s0 = l.at * kSlice, end = min(a.V, s0 + kSlice);
+  constexpr int EACH = kSlice / kSampleThreads;   // neighbours of a thread
+  const float* row = wide_row(a, r);
+  uint32_t key[EACH];
+#pragma unroll
+  for (int i = 0; i < EACH; ++i) {
+    const int t = s0 + EACH * tid + i;
+    key[i] = t < end ? ordered_key(row[t] * inv_t) : 0;
+  }
+  u64 rank = 0;   // tokens at the threshold before this thread's
+  const bool ties = quota < (u64)l.cnt_eq;
+  if (ties) {
+    int before = 0, mine = 0;
+    for (int i = tid; i < l.cnt_eq; i += kSampleThreads) before += (int)l.ties[i] < s0;
+    if (before) atomicAdd(&l.cnt_before, before);
+#pragma unroll
+    for (int i = 0; i < EACH; ++i) mine += key[i] == thr && s0 + EACH * tid + i < end;
+    int incl = mine;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int o = __shfl_up(incl, d, 64);
+      if (lane >= d) incl += o;
+    }
+    if (lane == 63) l.ranks[wv] = incl;
+    __syncthreads();
+    rank = l.cnt_before + incl - mine;
+    for (int i = 0; i < wv; ++i) rank += l.ranks[i];
+  }
+  u64 mass[EACH], mine = 0;
+#pragma unroll
+  for (int i = 0; i < EACH; ++i) {
+    mass[i] = 0;
+    if (s0 + EACH * tid + i >= end) continue;
+    if (key[i] > thr) mass[i] = mass_of(key[i]);
+    else if (key[i] == thr && (!ties || rank++ < quota)) mass[i] = mass_thr;
+    mine += mass[i];
+  }
+  const u64 incl = wave_sums(mine);
+  if (lane == 63) l.sums[wv] = incl;
+  __syncthreads();
+  u64 run = l.before + incl - mine;
+  for (int i = 0; i < wv; ++i) run += l.sums[i];
+#pragma unroll
+  for (int i = 0; i < EACH; ++i) {
+    if (mass[i] && goal >= run && goal < run + mass[i]) a.out[r] = s0 + EACH * tid + i;
+    run += mass[i];
+  }
+  return true;
+}
+
+__global__ __launch_bounds__(kSampleThreads) void sample_draw_kernel(SampleArgs a, SampleScratch s) {
+  __shared__ DrawLds lds;
+  const int r = blockIdx.x, groups = s.slices * kSliceThreads;
+  uint32_t got[kLookKeys];   // (asked for before the row's kind is known; a row of another kind has left some undefined)
+#pragma unroll
+  for (int u = 0; u < kLookKeys; ++u) {
+    const int g = threadIdx.x + u * kSampleThreads;
+    got[u] = g < groups ? s.maxima[(int64_t)r * groups + g] : 0;
+  }
+  const RowKind kind = row_kind(a, s, r);
+  if (kind == kRowFew && draw_few(a, s, r, lds, got)) return;
+  if (kind == kRowWide && draw_wide(a, s, r, lds)) return;
+  __syncthreads();
+  sample_whole_row(a, r, lds.row);
 }
 
 }  // namespace ninfer
@@ -700,6 +1063,13 @@ extern "C" void ninfer_uniforms(const unsigned long long* seeds, const unsigned 
   for (int i = 0; i < n; ++i) out[i] = (float)(mix(mix(mix(seeds[i]) ^ keys[i]) ^ draws[i]) >> 40) * 0x1p-24f;
 }
 
+static int sample_check(const SampleArgs& a, int R) {
+  NINFER_REQUIRE(R > 0 && a.V > 0, "sample: R=%d V=%d must be positive", R, a.V);
+  NINFER_REQUIRE(a.ld >= a.V, "sample: row stride %d < vocabulary %d", a.ld, a.V);
+  NINFER_REQUIRE(a.temperature && a.uniform && a.out, "sample: a required array is null");
+  return 0;
+}
+
 // logits [R, ld] (V used); work [R, V] scratch; per-row temperature, top_k,
 // top_p, rep_penalty, uniform; penalties as (token, count) pairs in
 // pen_tokens/pen_counts[pen_offsets[r] .. pen_offsets[r+1]) (null: none);
@@ -709,47 +1079,75 @@ extern "C" int ninfer_sample(const float* logits, int ld, int V, int R, float* w
                              const float* rep_penalty, const int* pen_tokens,
                              const int* pen_counts, const int* pen_offsets, const float* uniform,
                              int* out, hipStream_t stream) {
-  NINFER_REQUIRE(R > 0 && V > 0, "sample: R=%d V=%d must be positive", R, V);
-  NINFER_REQUIRE(ld >= V, "sample: row stride %d < vocabulary %d", ld, V);
-  NINFER_REQUIRE(temperature && uniform && work && out, "sample: a required array is null");
-  sample_kernel<<<R, kSampleThreads, 0, stream>>>(logits, ld, V, work, temperature, top_k, top_p,
-                                                  rep_penalty, pen_tokens, pen_counts, pen_offsets,
-                                                  uniform, out);
+  const SampleArgs a = {logits, temperature, top_k, top_p, rep_penalty, pen_tokens, pen_counts, pen_offsets,
+                        uniform, out, work, ld, V};
+  int rc = sample_check(a, R);
+  if (rc) return rc;
+  NINFER_REQUIRE(work, "sample: a required array is null");
+  sample_kernel<<<R, kSampleThreads, 0, stream>>>(a);
   NINFER_LAUNCH_CHECK();
   return 0;
 }
 
-// Places per row that ninfer_sample_few needs in each of cand_val and cand_idx.
-extern "C" long long ninfer_sample_few_places(int V) {
-  return (long long)((V + kSlice - 1) / kSlice) * kCandPerSlice;
+// The scratch of ninfer_sample_spread, behind work [R, V]: offsets in bytes, and the whole.
+struct SpreadLayout {
+  long long maxima, slice_max, listed, list, bins, slice_mass, bytes;
+  int slices;
+};
+static SpreadLayout spread_layout(int V, int R, bool wide) {
+  SpreadLayout p;
+  p.slices = (V + kSlice - 1) / kSlice;
+  long long at = 0;
+  auto take = [&](long long bytes) {
+    const long long here = at;
+    at += (bytes + 255) / 256 * 256;
+    return here;
+  };
+  take((long long)R * V * 4);   // work
+  p.maxima = take((long long)R * p.slices * kSliceThreads * 4);
+  p.slice_max = take(wide ? (long long)R * p.slices * 4 : 0);
+  p.listed = take(wide ? (long long)R * 4 : 0);
+  p.list = take(wide ? (long long)R * kCutList * 8 : 0);
+  p.bins = take(wide ? (long long)R * kBins * 8 : 0);
+  p.slice_mass = take(wide ? (long long)R * p.slices * 8 : 0);
+  p.bytes = at;
+  return p;
 }
 
-// The same for rows that all keep few tokens: every row greedy (temperature <= 0) or with
-// 1 <= top_k <= 64, which the caller asserts (a row with another top_k would be cut to its 64
-// best per slice). Same result as ninfer_sample, from two launches that use the whole GPU.
-// cand_val, cand_idx: [R, ninfer_sample_few_places(V)].
-extern "C" int ninfer_sample_few(const float* logits, int ld, int V, int R, float* cand_val,
-                                 int* cand_idx, const float* temperature,
-                                 const int* top_k, const float* top_p, const float* rep_penalty,
-                                 const int* pen_tokens, const int* pen_counts,
-                                 const int* pen_offsets, const float* uniform, int* out,
-                                 hipStream_t stream) {
-  NINFER_REQUIRE(R > 0 && V > 0, "sample: R=%d V=%d must be positive", R, V);
-  NINFER_REQUIRE(ld >= V, "sample: row stride %d < vocabulary %d", ld, V);
-  NINFER_REQUIRE(temperature && top_k && uniform && cand_val && cand_idx && out,
-                 "sample: a required array is null");
-  const int slices = (V + kSlice - 1) / kSlice, C = slices * kCandPerSlice;
+extern "C" int ninfer_sample_few_tokens() { return kFewTokens; }
+extern "C" long long ninfer_sample_spread_bytes(int V, int R, int wide) { return spread_layout(V, R, wide).bytes; }
+
+// The same token for every row, by the whole GPU where a row is greedy or keeps at most kFewTokens
+// tokens (top_k) and, with `wide`, where top_k cuts nothing; other rows are as with ninfer_sample.
+// scratch: ninfer_sample_spread_bytes(V, R, wide) bytes, aligned to 256.
+extern "C" int ninfer_sample_spread(const float* logits, int ld, int V, int R, int wide, void* scratch,
+                                    const float* temperature, const int* top_k, const float* top_p,
+                                    const float* rep_penalty, const int* pen_tokens,
+                                    const int* pen_counts, const int* pen_offsets, const float* uniform,
+                                    int* out, hipStream_t stream) {
+  const SampleArgs a = {logits, temperature, top_k, top_p, rep_penalty, pen_tokens, pen_counts, pen_offsets,
+                        uniform, out, (float*)scratch, ld, V};
+  int rc = sample_check(a, R);
+  if (rc) return rc;
+  NINFER_REQUIRE(scratch && (uintptr_t)scratch % 256 == 0, "sample: scratch is null or not aligned");
   NINFER_REQUIRE(R <= 65535, "sample: %d rows are too many", R);
-  sample_candidates_kernel<<<dim3(slices, R), kCandThreads, 0, stream>>>(
-      logits, ld, V, temperature, top_k, rep_penalty, pen_tokens, pen_counts, pen_offsets, cand_val,
-      cand_idx);
+  if ((V + kSlice - 1) / kSlice > kMaxSlices) wide = 0;
+  const SpreadLayout p = spread_layout(V, R, wide);
+  char* base = (char*)scratch;
+  typedef unsigned long long u64;
+  const SampleScratch s = {(uint32_t*)(base + p.maxima), (uint32_t*)(base + p.slice_max), (int*)(base + p.listed),
+                           (uint2*)(base + p.list),      (u64*)(base + p.bins),           (u64*)(base + p.slice_mass),
+                           p.slices,                     wide != 0};
+  const dim3 grid(p.slices, R);
+  sample_maxima_kernel<<<grid, kSliceThreads, 0, stream>>>(a, s);
   NINFER_LAUNCH_CHECK();
-  if (C <= kSlice)
-    sample_few_kernel<true><<<R, kCandThreads, 0, stream>>>(cand_val, cand_idx, C, temperature, top_k, top_p,
-                                                            uniform, out);
-  else
-    sample_few_kernel<false><<<R, kCandThreads, 0, stream>>>(cand_val, cand_idx, C, temperature, top_k, top_p,
-                                                             uniform, out);
+  if (wide) {
+    sample_masses_kernel<<<grid, kSliceThreads, 0, stream>>>(a, s);
+    NINFER_LAUNCH_CHECK();
+    sample_cut_kernel<<<grid, kSliceThreads, 0, stream>>>(a, s);
+    NINFER_LAUNCH_CHECK();
+  }
+  sample_draw_kernel<<<R, kSampleThreads, 0, stream>>>(a, s);
   NINFER_LAUNCH_CHECK();
   return 0;
 }

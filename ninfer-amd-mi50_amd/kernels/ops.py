@@ -369,7 +369,7 @@ class HipOps:
         self.lib.ninfer_attention_workspace_floats.restype = ctypes.c_longlong
         self.lib.ninfer_event_create.restype = ctypes.c_void_p
         self.lib.ninfer_stream_after.argtypes = [ctypes.c_void_p] * 3
-        self.lib.ninfer_sample_few_places.restype = ctypes.c_longlong
+        self.lib.ninfer_sample_spread_bytes.restype = ctypes.c_longlong
         self.lib.ninfer_latent_attention_workspace_floats.restype = ctypes.c_longlong
         self.lib.ninfer_gla_segment_floats.restype = ctypes.c_longlong
         self.lib.ninfer_lightning_chunk_floats.restype = ctypes.c_longlong
@@ -2126,12 +2126,14 @@ class HipOps:
         self.lib.ninfer_uniforms(ctypes.c_void_p(at[0][0]), ctypes.c_void_p(at[1][0]), ctypes.c_void_p(at[2][0]),
                                  n, ctypes.c_void_p(out.ctypes.data))
 
-    FEW_TOKENS = 64   # most tokens a row may keep (top_k) for the two-launch sampling path
+    FEW_TOKENS = 256   # most tokens a row may keep (top_k) for the two-launch sampling path
 
     def sample(self, logits, temperature, uniform, out, top_k=None, top_p=None, rep_penalty=None,
-               pen_tokens=None, pen_counts=None, pen_offsets=None, few=False):
-        """One token per row. `few`: the caller asserts that every row is greedy
-        (temperature <= 0) or has 1 <= top_k <= FEW_TOKENS; same result, much faster."""
+               pen_tokens=None, pen_counts=None, pen_offsets=None, few=False, spread=False):
+        """One token per row. `few`, `spread`: the same tokens from kernels that use the whole GPU for a
+        row, in two launches for rows that are greedy (temperature <= 0) or have 1 <= top_k <= FEW_TOKENS,
+        with `spread` in four for those and rows of which top_k cuts nothing; other rows are
+        as slow as without."""
         _dev(logits, "logits", torch.float32, 2)
         r, v = logits.shape
         _dev(temperature, "temperature", torch.float32, 1)
@@ -2149,18 +2151,13 @@ class HipOps:
             _dev(pen_tokens, "pen_tokens", torch.int32, 1)
             _dev(pen_counts, "pen_counts", torch.int32, 1)
             _need(pen_offsets.shape[0] == r + 1, "sample: pen_offsets has the wrong size")
-        if few:
-            # every row keeps few tokens (the caller knows its rows' options): candidates from
-            # the whole GPU first, then the same selection and draw on those
-            _need(top_k is not None, "sample: rows that keep few tokens need top_k")
-            places = int(self.lib.ninfer_sample_few_places(v))
-            cand_val = torch.empty((r, places), dtype=torch.float32, device=logits.device)
-            cand_idx = torch.empty((r, places), dtype=torch.int32, device=logits.device)
-            self._ok(self.lib.ninfer_sample_few(
-                ctypes.c_void_p(logits.data_ptr()), logits.stride(0), v, r,
-                ctypes.c_void_p(cand_val.data_ptr()), ctypes.c_void_p(cand_idx.data_ptr()),
-                ctypes.c_void_p(temperature.data_ptr()),
-                ctypes.c_void_p(top_k.data_ptr()), ctypes.c_void_p(_ptr(top_p)),
+        if few or spread:
+            scratch = torch.empty(int(self.lib.ninfer_sample_spread_bytes(v, r, int(spread))), dtype=torch.uint8,
+                                  device=logits.device)
+            self._ok(self.lib.ninfer_sample_spread(
+                ctypes.c_void_p(logits.data_ptr()), logits.stride(0), v, r, int(spread),
+                ctypes.c_void_p(scratch.data_ptr()), ctypes.c_void_p(temperature.data_ptr()),
+                ctypes.c_void_p(_ptr(top_k)), ctypes.c_void_p(_ptr(top_p)),
                 ctypes.c_void_p(_ptr(rep_penalty)), ctypes.c_void_p(_ptr(pen_tokens)),
                 ctypes.c_void_p(_ptr(pen_counts)), ctypes.c_void_p(_ptr(pen_offsets)),
                 ctypes.c_void_p(uniform.data_ptr()), ctypes.c_void_p(out.data_ptr()),

@@ -21,6 +21,11 @@ import torch
 from .params import SamplingParams
 
 _MASK = (1 << 64) - 1
+# Tokens of a vocabulary beyond which rows that top-k does not cut go through four launches by the whole GPU (one row of
+# 9,000, us so and by one block: 29 and 36, with top-p 1 23 and 19; 32,000 30 and 74, 23 and 33), and greedy ones with
+# a penalty through two (32,000 tokens 11 and 10, 64 rows 12 and 13; 151,936 11 and 25, 21 and 33)
+SPREAD_TOKENS = 12288
+FEW_GREEDY_TOKENS = 32768
 _OPTIONS = attrgetter("temperature", "top_p", "repetition_penalty", "top_k")
 _STREAM = attrgetter("seed", "key", "draw")
 
@@ -210,12 +215,15 @@ class Sampler:
             pen = dict(pen_offsets=dev[o - r - 1:o], pen_tokens=dev[o:o + n_pen],
                        pen_counts=dev[o + n_pen:n])
         out = torch.empty(r, dtype=torch.int32, device=self.device)
-        # rows that are greedy or keep at most a few dozen tokens (the reference's default is
-        # top_k = 50) take the path that reads the logits with the whole GPU
-        most = getattr(self.ops, "FEW_TOKENS", 0)
-        # (rows that are all greedy stay with the one launch: it is short as it is)
-        if most and drawn and all(t <= 0 or 1 <= k <= most for t, k in zip(temps, top_ks)):
-            pen["few"] = True
+        # rows that are greedy, keep few tokens (the reference's default is top_k = 50) or cut nothing by top-k take
+        # the paths that read the logits with the whole GPU
+        most, vocab = getattr(self.ops, "FEW_TOKENS", 0), logits.shape[1]
+        # (greedy rows without a penalty stay with the one launch: it is short as it is)
+        if most and (drawn or n_pen > 0 and vocab > FEW_GREEDY_TOKENS):
+            if all(t <= 0 or 1 <= k <= most for t, k in zip(temps, top_ks)):
+                pen["few"] = True
+            elif vocab > SPREAD_TOKENS and all(t <= 0 or k <= most or k >= vocab for t, k in zip(temps, top_ks)):
+                pen["spread"] = True
         self.ops.sample(logits, f[:r], f[3 * r:4 * r], out, top_k=dev[4 * r:5 * r], top_p=f[r:2 * r],
                         rep_penalty=f[2 * r:3 * r], **pen)
         return out.tolist()

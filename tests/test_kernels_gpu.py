@@ -1257,6 +1257,41 @@ def test_sample_rows_that_keep_few_tokens(ops, gen, v):
     assert int(a[2]) == v - 1 or float(temp[2]) > 0
 
 
+@pytest.mark.parametrize("v", [3, 300, 4096, 4097, 8191, 32000, 151936])
+def test_sample_rows_by_the_whole_gpu(ops, gen, v):
+    """Rows of every kind in one call of the four launches: top-k cuts nothing (0, or the vocabulary and more), keeps
+    up to 256 tokens, or more; top-p that cuts in the first tokens, among many and not at all; flat logits, ties at the cut,
+    logits of which most are -inf, all equal, one +inf, and NaN among them: the one-block path's tokens."""
+    wide = [(0.3, 0, 0.8), (0.7, 0, 0.95), (1.2, 0, 0.8), (1.2, v, 0.95), (1.0, 0, 1.0), (2.0, v + 3, 0.999), (5.0, 0, 0.5)]
+    rows = wide * 2 + [(0.7, 200, 0.95), (1.0, 256, 1.0), (1.0, 257, 0.9), (0.0, 0, 1.0), (0.9, 65, 0.8)] + [(0.7, 0, 0.9)] * 6
+    r = len(rows)
+    logits = torch.randn(r, v, generator=gen, device="cuda") * 3
+    logits[len(wide):2 * len(wide)] = logits[len(wide):2 * len(wide)].round()   # ties
+    special = logits[-6:]
+    special[0] = 1.0
+    special[1, 1:] = -float("inf")
+    special[2, v // 2] = float("inf")
+    special[3, v // 3] = float("nan")
+    special[4] = -2.0 - torch.arange(v, device="cuda") % 2
+    special[5, : v // 2] = -3e38
+    temp, top_k, top_p = (torch.tensor(x, device="cuda", dtype=d) for x, d in zip(zip(*rows), (torch.float32, torch.int32, torch.float32)))
+    pens = [list(range(i % 3, v, 5 + i)) if i % 2 else [] for i in range(r)]
+    offs = [0]
+    for p in pens:
+        offs.append(offs[-1] + len(p))
+    i32 = lambda x: torch.tensor(x, device="cuda", dtype=torch.int32)
+    args = dict(top_k=top_k, top_p=top_p, rep_penalty=torch.full((r,), 1.2, device="cuda"), pen_tokens=i32(sum(pens, [])),
+                pen_counts=i32([1 + i % 2 for i in range(offs[-1])]), pen_offsets=i32(offs))
+    for u in torch.linspace(0.0, 0.999999, 24).tolist():
+        uniform = torch.full((r,), u, device="cuda")
+        got = []
+        for spread in (False, True):
+            out = torch.full((r,), -7, device="cuda", dtype=torch.int32)
+            ops.sample(logits, temp, uniform, out, spread=spread, **args)
+            got.append(out)
+        assert torch.equal(*got), f"u={u}: {got[0].tolist()} vs {got[1].tolist()}"
+
+
 @pytest.mark.parametrize("top_p", [1.0, 0.999])
 def test_few_tokens_path_has_the_masses_of_the_whole_row(ops, gen, top_p):
     """Numbers drawn right at the border between two kept tokens, one of them at the threshold: both paths
