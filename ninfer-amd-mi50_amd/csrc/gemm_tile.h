@@ -235,9 +235,10 @@ __device__ inline void write_accumulators_staged(const GemmArgs& a, const f32x4 
   bf16* C = (bf16*)a.C;
   const int c = lane % U;
 #pragma unroll
-  for (int it = 0; it < ROWS / RPI; ++it) {
+  for (int it = 0; it < (ROWS + RPI - 1) / RPI; ++it) {   // (rows beyond the stage's have no row of C)
     const int tok = it * RPI + lane / U;
     const int dst = __shfl(c_row[(it * RPI) / 64], tok & 63, 64);
+    if (ROWS % RPI && tok >= ROWS) continue;
     const bf16x8 val = *(const bf16x8*)(stage + tok * RB + ((c ^ (tok & (U - 1))) << 4));
     const int f = feat0 + 8 * c;
     if (dst >= 0 && f < N) *(bf16x8*)(C + (int64_t)dst * a.ldc + f) = val;

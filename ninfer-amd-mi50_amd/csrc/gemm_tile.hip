@@ -69,7 +69,9 @@ static int tile_rows_of(const GemmArgs& a) {
   return (!gated && tall >= cus) || dense_us_256(tall, cus, a.K, a.beside) < dense_us_128(low, cus, a.K) ? 256 : 128;
 }
 
-int gemm_tile(const GemmArgs& a, hipStream_t stream) { return gemm_tile_rows(a, tile_rows_of(a), stream); }
+int gemm_tile(const GemmArgs& a, hipStream_t stream) {
+  return gemm_mid_takes(a) ? gemm_mid(a, stream) : gemm_tile_rows(a, tile_rows_of(a), stream);
+}
 
 // out[m][n] = sum over the parts, in their order, of ws[z][m][n] (+ bias[n]); four features a thread.
 template <typename TC>
@@ -139,5 +141,5 @@ int gemm_split(const GemmArgs& a, hipStream_t stream) {
 
 }  // namespace ninfer
 
-// Rows of the tiles that ninfer_gemm would run a product of many rows in.
+// Rows of the tiles that ninfer_gemm would run a product of many rows in that is not one round of gemm_mid's.
 extern "C" int ninfer_gemm_tile_rows(const ninfer::GemmArgs* args) { return ninfer::tile_rows_of(*args); }

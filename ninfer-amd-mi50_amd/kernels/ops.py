@@ -700,7 +700,7 @@ class HipOps:
     # ---- products ---------------------------------------------------------------
     def _gemm(self, a, w, c, *, n, k, m, bias=None, offsets=None, a_index=None, c_index=None,
               a_div=1, groups=1, epilogue=0, w_group_stride=0, tiles=None, only_if_split=False,
-              act_limit=0.0, act_alpha=1.0):
+              only_if_mid=False, act_limit=0.0, act_alpha=1.0):
         t16 = t64 = tc = None
         if tiles is not None and tiles.tiles16 is not None:
             t16, t64, tc = tiles.tiles16.data_ptr(), tiles.tiles_big.data_ptr(), \
@@ -729,11 +729,14 @@ class HipOps:
                 return False
             self._ok(self.lib.ninfer_gemm(ctypes.byref(args), 0, self._stream()))
             return True
+        if only_if_mid and not self.lib.ninfer_gemm_mid_tile(ctypes.byref(args)):
+            return False
         if self._held is not None:
             self._held.append((args, (a, w, c, bias, offsets, a_index, c_index, tiles)))
-            return
+            return True
         self._ok(self.lib.ninfer_gemm(ctypes.byref(args), 1 if self.force_generic else 0,
                                       self._stream()))
+        return True
 
     def _on_side(self) -> bool:
         return self._side is not None and (self._stream().value or 0) == self._side.cuda_stream
@@ -840,7 +843,10 @@ class HipOps:
                         x, w, out, m=x.shape[0], n=w.shape[0], k=x.shape[1], only_if_split=True):
                     return
                 if not own:
-                    torch.matmul(x, w.t(), out=out)
+                    # one round of tiles: as fast here as in the library, or faster, and 16 us less of the host's
+                    # time a call, which bounds short steps that run eagerly (gemm_mid.hip)
+                    if not self._gemm(x, w, out, m=x.shape[0], n=w.shape[0], k=x.shape[1], only_if_mid=True):
+                        torch.matmul(x, w.t(), out=out)
                     return
         elif act is None and bias is None and self._rows_cut(x, out, w) and self._gemm(
                 x, w, out, m=x.shape[0], n=w.shape[0], k=x.shape[1], only_if_split=True):

@@ -1,0 +1,92 @@
+"""Dense products that are one round of tiles, at the edges of every tile: rows and features that end inside a
+block, K of one k tile, of fewer than a stage's and of a last stage that K does not fill, every epilogue."""
+import ctypes
+
+import pytest
+import torch
+
+BF16 = 1
+
+
+def _args(m, n, k, **more):
+    from ninfer_amd.kernels.ops import _GemmArgs
+    return _GemmArgs(A=4096, W=4096, C=4096, M=m, N=n, K=k, lda=k, ldc=n, groups=1, a_div=1, in_dtype=BF16, out_dtype=BF16, **more)
+
+
+# (256 CUs, as the library assumes without a GPU: both sides of a round of each tile; what no round holds, too few
+# rows or features, an index or a K that is not whole k tiles)
+@pytest.mark.parametrize("m,n,k,gated,tile", [
+    (64, 8192, 2048, 0, 32064), (65, 8193, 2048, 0, 96064), (64, 16384, 2048, 0, 64064), (96, 16384, 2048, 0, 96064),
+    (64, 16385, 2048, 0, 64096), (129, 16384, 2048, 0, 192064), (129, 16385, 2048, 0, 192128), (128, 16384, 64, 0, 128064), (256, 8192, 64, 1, 128128),
+    (512, 2048, 2048, 0, 64064), (513, 2048, 2048, 0, 96064), (1024, 6144, 2048, 0, 128192), (1025, 6144, 2048, 0, 0),
+    (1536, 4096, 2048, 0, 192128), (1537, 4096, 2048, 0, 0), (1536, 2048, 2048, 1, 192128), (1024, 3072, 2048, 1, 0),
+    (32, 2048, 2048, 0, 0), (33, 2048, 2048, 0, 32064), (512, 63, 2048, 0, 0), (512, 2048, 2080, 0, 0)])
+def test_which_tile(m, n, k, gated, tile):
+    from ninfer_amd.kernels.build import ensure_built
+    lib = ctypes.CDLL(ensure_built())
+    assert lib.ninfer_gemm_mid_tile(ctypes.byref(_args(m, n, k, epilogue=gated))) == tile
+    assert lib.ninfer_gemm_mid_tile(ctypes.byref(_args(m, n, k, epilogue=gated, a_index=16, offsets=16))) == 0
+
+
+SHAPES = [(33, 8192, 64), (64, 2056, 192), (64, 16384, 320), (130, 2050, 64), (512, 2048, 2048), (700, 2047, 192), (760, 2048, 320),
+          (250, 6100, 128), (129, 8190, 448), (900, 2304, 192), (1500, 2040, 64), (1140, 2900, 576), (1500, 4090, 128),
+          (1020, 6100, 256), (2048, 64, 704)]
+EPILOGUES = ["none", "f32", "relu2", "bias", "gated", "gated bias"]
+CASES = [(*s, e) for s in SHAPES for e in EPILOGUES if not (e.startswith("gated") and s in SHAPES[-2:])]   # (not a round of gated tiles)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k,epilogue", CASES)
+def test_products(m, n, k, epilogue):
+    from ninfer_amd.kernels import load_ops
+    ops = load_ops()
+    gated = epilogue.startswith("gated")
+    g = torch.Generator("cuda").manual_seed(m + n)
+    rows = 2 * (n // 2) if gated else n
+    x, w = (torch.randn(r, k, generator=g, device="cuda").bfloat16() for r in (m, rows))
+    inner = rows // 2 if gated else n
+    bias = torch.randn(rows, generator=g, device="cuda") if "bias" in epilogue else None
+    dtype = torch.float32 if epilogue == "f32" else torch.bfloat16
+    whole = torch.full((m + 1, inner), 7.0, device="cuda", dtype=dtype)
+    out = whole[:m]
+    assert ops.lib.ninfer_gemm_mid_tile(ctypes.byref(_args(m, inner, k, epilogue=int(gated))))
+    with ops.tuned(split_min_bytes=1 << 40):   # (nothing is cut along K)
+        if gated:
+            w = w * 0.1
+            ops.swiglu_linear(x, w, out, bias=bias)
+        else:
+            ops._gemm(x, w, out, m=m, n=n, k=k, bias=bias, epilogue=3 if epilogue == "relu2" else 0)
+    sums = x.double() @ w.double().T
+    # exact products, k of them added in 32-bit in any order
+    bound = 2 * k * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T) + 1e-6
+    if bias is not None:
+        sums = sums + bias.double()
+        bound = bound + 2.0 ** -23 * sums.abs()
+    if gated:
+        a, u = sums[:, :inner], sums[:, inner:]
+        want = a * torch.sigmoid(a) * u
+        # |d silu| <= 1.1 |d a|; the hardware's exponential and reciprocal, 1 ulp each, and two products
+        bound = 1.1 * bound[:, :inner] * u.abs() + a.abs() * bound[:, inner:] + 2.0 ** -20 * want.abs() + 1e-6
+    elif epilogue == "relu2":
+        want = sums.clamp(min=0) ** 2
+        bound = 2 * sums.abs() * bound + bound * bound + 2.0 ** -23 * want
+    else:
+        want = sums
+    if dtype == torch.bfloat16:
+        bound = bound + 2.0 ** -8 * (want.abs() + bound)
+    assert ((out.double() - want).abs() <= bound).all()
+    assert (whole[m:] == 7.0).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [(65, 4096, 2048), (512, 2048, 5632), (700, 1024, 1024), (1024, 6144, 2048)])
+def test_plain_products_of_one_round_stay_out_of_the_library(monkeypatch, m, n, k):
+    from ninfer_amd.kernels import load_ops
+    ops = load_ops()
+    g = torch.Generator("cuda").manual_seed(m)
+    x, w = (torch.randn(r, k, generator=g, device="cuda").bfloat16() for r in (m, n))
+    want = torch.matmul(x.double(), w.double().T)
+    out = torch.empty(m, n, device="cuda", dtype=torch.bfloat16)
+    monkeypatch.setattr(torch, "matmul", None)
+    ops.linear(x, w, out)
+    assert float((out.double() - want).norm() / want.norm()) < 2.0 ** -8
