@@ -1074,19 +1074,21 @@ static int sample_check(const SampleArgs& a, int R) {
 // top_p, rep_penalty, uniform; penalties as (token, count) pairs in
 // pen_tokens/pen_counts[pen_offsets[r] .. pen_offsets[r+1]) (null: none);
 // out [R] token ids.
+static int sample_by_rows(const SampleArgs& a, int R, hipStream_t stream) {
+  int rc = sample_check(a, R);
+  if (rc) return rc;
+  NINFER_REQUIRE(a.work, "sample: a required array is null");
+  sample_kernel<<<R, kSampleThreads, 0, stream>>>(a);
+  NINFER_LAUNCH_CHECK();
+  return 0;
+}
 extern "C" int ninfer_sample(const float* logits, int ld, int V, int R, float* work,
                              const float* temperature, const int* top_k, const float* top_p,
                              const float* rep_penalty, const int* pen_tokens,
                              const int* pen_counts, const int* pen_offsets, const float* uniform,
                              int* out, hipStream_t stream) {
-  const SampleArgs a = {logits, temperature, top_k, top_p, rep_penalty, pen_tokens, pen_counts, pen_offsets,
-                        uniform, out, work, ld, V};
-  int rc = sample_check(a, R);
-  if (rc) return rc;
-  NINFER_REQUIRE(work, "sample: a required array is null");
-  sample_kernel<<<R, kSampleThreads, 0, stream>>>(a);
-  NINFER_LAUNCH_CHECK();
-  return 0;
+  return sample_by_rows({logits, temperature, top_k, top_p, rep_penalty, pen_tokens, pen_counts, pen_offsets,
+                         uniform, out, work, ld, V}, R, stream);
 }
 
 // The scratch of ninfer_sample_spread, behind work [R, V]: offsets in bytes, and the whole.
@@ -1120,13 +1122,9 @@ extern "C" long long ninfer_sample_spread_bytes(int V, int R, int wide) { return
 // The same token for every row, by the whole GPU where a row is greedy or keeps at most kFewTokens
 // tokens (top_k) and, with `wide`, where top_k cuts nothing; other rows are as with ninfer_sample.
 // scratch: ninfer_sample_spread_bytes(V, R, wide) bytes, aligned to 256.
-extern "C" int ninfer_sample_spread(const float* logits, int ld, int V, int R, int wide, void* scratch,
-                                    const float* temperature, const int* top_k, const float* top_p,
-                                    const float* rep_penalty, const int* pen_tokens,
-                                    const int* pen_counts, const int* pen_offsets, const float* uniform,
-                                    int* out, hipStream_t stream) {
-  const SampleArgs a = {logits, temperature, top_k, top_p, rep_penalty, pen_tokens, pen_counts, pen_offsets,
-                        uniform, out, (float*)scratch, ld, V};
+static int sample_by_slices(const SampleArgs& a, int R, int wide, hipStream_t stream) {
+  const int V = a.V;
+  void* const scratch = a.work;
   int rc = sample_check(a, R);
   if (rc) return rc;
   NINFER_REQUIRE(scratch && (uintptr_t)scratch % 256 == 0, "sample: scratch is null or not aligned");
@@ -1149,5 +1147,47 @@ extern "C" int ninfer_sample_spread(const float* logits, int ld, int V, int R, i
   }
   sample_draw_kernel<<<R, kSampleThreads, 0, stream>>>(a, s);
   NINFER_LAUNCH_CHECK();
+  return 0;
+}
+extern "C" int ninfer_sample_spread(const float* logits, int ld, int V, int R, int wide, void* scratch,
+                                    const float* temperature, const int* top_k, const float* top_p,
+                                    const float* rep_penalty, const int* pen_tokens,
+                                    const int* pen_counts, const int* pen_offsets, const float* uniform,
+                                    int* out, hipStream_t stream) {
+  return sample_by_slices({logits, temperature, top_k, top_p, rep_penalty, pen_tokens, pen_counts, pen_offsets,
+                           uniform, out, (float*)scratch, ld, V}, R, wide, stream);
+}
+
+// Pinned host memory to the device, 16 bytes a thread and turn. (As a kernel: a copy by the runtime costs the host 5 us
+// more, and the same on the device.)
+__global__ __launch_bounds__(256) void sample_fetch_kernel(const int4* __restrict__ from, int4* __restrict__ to, long long n) {
+  for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long long)gridDim.x * 256) to[i] = from[i];
+}
+
+// A sampler's whole call: the rows' parameters, laid out in pinned host memory (aligned to 16 bytes), go to the device, the
+// kernels run (mode 0: ninfer_sample, 1 and 2: ninfer_sample_spread without and with `wide`), write the tokens back into
+// pinned memory, and the host waits for them. What bounds such a call is the host: as a copy, launches and a copy back through
+// tensors and events it took 62 us for one row of 151,936 tokens, 78 for 8 and 139 for 64 with 1,500 tokens of history, 40, 50 and 123 so.
+// host: temperature[R], top_p[R], rep_penalty[R], uniform[R] (floats), top_k[R], and with n_pen > 0 pen_offsets[R + 1],
+// pen_tokens[n_pen], pen_counts[n_pen]; `ints` numbers in all, a multiple of 4 of them reserved here and in `params` (device
+// memory); tokens [R] in pinned memory. scratch: as the two ask for.
+extern "C" int ninfer_sample_rows(const float* logits, int ld, int V, int R, int mode, const int* host, int* params,
+                                  long long ints, int n_pen, void* scratch, int* tokens, hipStream_t stream) {
+  const long long need = 5ll * R + (n_pen > 0 ? R + 1 + 2ll * n_pen : 0);
+  NINFER_REQUIRE(R > 0 && host && params && tokens && n_pen >= 0 && ints == need && (uintptr_t)host % 16 == 0 &&
+                 (uintptr_t)params % 16 == 0, "sample: %lld numbers of %d rows with %d penalties", ints, R, n_pen);
+  const long long quads = (ints + 3) / 4;
+  sample_fetch_kernel<<<(unsigned)min(256ll, (quads + 255) / 256), 256, 0, stream>>>((const int4*)host, (int4*)params, quads);
+  NINFER_LAUNCH_CHECK();
+  const float* f = (const float*)params;
+  const int* pen = n_pen > 0 ? params + 5 * R : nullptr;
+  const SampleArgs a = {logits, f, params + 4 * R, f + R, f + 2 * R, pen ? pen + R + 1 : nullptr, pen ? pen + R + 1 + n_pen : nullptr,
+                        pen, f + 3 * R, tokens, (float*)scratch, ld, V};
+  // (not through the two entry points above: the engine's C interface has a function by the name of one, and in a program
+  // that is linked to it a call by that name would end there)
+  const int rc = mode == 0 ? sample_by_rows(a, R, stream) : sample_by_slices(a, R, mode == 2, stream);
+  const hipError_t e = hipStreamSynchronize(stream);   // (also after an error: the caller's buffers are its own again)
+  if (rc) return rc;
+  if (e != hipSuccess) return set_error(-2, "sample: %s", hipGetErrorString(e));
   return 0;
 }

@@ -370,6 +370,8 @@ class HipOps:
         self.lib.ninfer_event_create.restype = ctypes.c_void_p
         self.lib.ninfer_stream_after.argtypes = [ctypes.c_void_p] * 3
         self.lib.ninfer_sample_spread_bytes.restype = ctypes.c_longlong
+        p, i = ctypes.c_void_p, ctypes.c_int
+        self.lib.ninfer_sample_rows.argtypes = [p, i, i, i, i, p, p, ctypes.c_longlong, i, p, p, p]
         self.lib.ninfer_latent_attention_workspace_floats.restype = ctypes.c_longlong
         self.lib.ninfer_gla_segment_floats.restype = ctypes.c_longlong
         self.lib.ninfer_lightning_chunk_floats.restype = ctypes.c_longlong
@@ -2133,6 +2135,22 @@ class HipOps:
                                  n, ctypes.c_void_p(out.ctypes.data))
 
     FEW_TOKENS = 256   # most tokens a row may keep (top_k) for the two-launch sampling path
+
+    def sample_rows(self, logits, rows, pinned, ints, n_pen, few=False, spread=False):
+        """One token per row, and the host waits for them. `pinned`: 32-bit numbers in pinned host memory, `ints` of them
+        the rows' temperature, top_p, rep_penalty, uniform (floats), top_k and, with n_pen > 0, pen_offsets, pen_tokens and
+        pen_counts side by side; the tokens come into the `rows` behind them, from the next multiple of 4 on. `few`,
+        `spread`: as in `sample`."""
+        _dev(logits, "logits", torch.float32, 2)
+        (r, v), at, room = logits.shape, (ints + 3) // 4 * 4, pinned.numel()
+        _need(r == rows and pinned.dtype == torch.int32 and pinned.is_pinned() and room >= at + r, "sample: the rows' numbers")
+        mode = 2 if spread else 1 if few else 0
+        size = int(self.lib.ninfer_sample_spread_bytes(v, r, mode - 1)) if mode else 4 * r * v
+        size = (size + 255) // 256 * 256
+        scratch = torch.empty(size + 4 * at, dtype=torch.uint8, device=logits.device)
+        host, dev = pinned.data_ptr(), scratch.data_ptr()
+        self._ok(self.lib.ninfer_sample_rows(logits.data_ptr(), logits.stride(0), v, r, mode, host, dev + size, ints, n_pen,
+                                             dev, host + 4 * at, self._stream()))
 
     def sample(self, logits, temperature, uniform, out, top_k=None, top_p=None, rep_penalty=None,
                pen_tokens=None, pen_counts=None, pen_offsets=None, few=False, spread=False):

@@ -12,6 +12,7 @@ from __future__ import annotations
 
 import os
 from array import array
+from itertools import accumulate
 from operator import attrgetter
 from typing import Dict, Iterable, List, Optional, Sequence, Tuple
 
@@ -133,26 +134,20 @@ class Sampler:
     def __init__(self, ops, device):
         self.ops = ops
         self.device = device
-        self._staging: List[list] = []   # pinned buffers (and the event after each one's copy)
-        self._staging_next = 0
+        self._free: List[tuple] = []   # pinned buffers that no call uses
 
-    def _staged(self, n: int) -> list:
-        """[a buffer of at least n ints, the event after its last copy, the same memory as an array]:
-        one of a few pinned buffers used in turn, its last copy done. The rows' parameters are
-        written into it and copied from it, so that the copy is queued behind the step that makes
-        the logits and the host goes on (a copy out of pageable memory makes the host wait until
-        the device has reached it, and the sampling kernel would then be launched only after the
-        step has ended)."""
-        if len(self._staging) < 4:
-            slot = [None, torch.cuda.Event(), None]
-            self._staging.append(slot)
-        else:
-            slot = self._staging[self._staging_next]
-            self._staging_next = (self._staging_next + 1) % len(self._staging)
-            slot[1].synchronize()
-        if slot[0] is None or slot[0].numel() < n:
-            slot[0] = torch.empty(max(n if slot[0] is None else 2 * n, 1024), dtype=torch.int32).pin_memory()
-            slot[2] = slot[0].numpy()
+    def _staged(self, n: int) -> tuple:
+        """(a buffer of at least n ints in pinned memory, the same memory as an array), which no other call uses until
+        it is given back. The rows' parameters are written into it and fetched from it behind the step that makes
+        the logits, while the host goes on (a copy out of pageable memory makes the host wait until the device has
+        reached it, and the sampling kernel would then be launched only after the step has ended)."""
+        try:
+            slot = self._free.pop()
+        except IndexError:
+            slot = None
+        if slot is None or slot[0].numel() < n:
+            buffer = torch.empty(max(n if slot is None else 2 * n, 1024), dtype=torch.int32).pin_memory()
+            slot = (buffer, buffer.numpy())
         return slot
 
     def sample(self, logits: torch.Tensor, rows: Sequence[SampleRow]) -> List[int]:
@@ -164,20 +159,14 @@ class Sampler:
         # and counts. (Copies queue behind the step that makes the logits, one after the other:
         # every further one would add its latency to the step.)
         temps, tops, penalties, top_ks = zip(*map(_OPTIONS, (row.params for row in rows))) if r else ((),) * 4
-        pens = []
-        offsets = [0] * (r + 1)
-        n_pen = 0
-        for i, (row, penalty) in enumerate(zip(rows, penalties), 1):
-            if penalty != 1.0:
-                both = row.history.both()
-                pens.append(both)
-                n_pen += both.shape[1]
-            offsets[i] = n_pen
+        listed = [len(row.history) if penalty != 1.0 else 0 for row, penalty in zip(rows, penalties)]
+        n_pen = sum(listed)
         o = 5 * r
         n = o + (r + 1 + 2 * n_pen if n_pen > 0 else 0)
         cuda = self.device.type == "cuda"
         if cuda:
-            pinned, copied, packed = self._staged(n)
+            at = (n + 3) // 4 * 4   # (the tokens come behind the parameters)
+            slot = pinned, packed = self._staged(at + r)
         else:
             packed = np.empty(n, np.int32)
         floats = packed[:4 * r].view(np.float32).reshape(4, r)
@@ -200,30 +189,32 @@ class Sampler:
                 floats[3, [i for i, t in enumerate(temps) if t > 0]] = to
         packed[4 * r:o] = top_ks
         if n_pen > 0:
-            packed[o:o + r + 1] = offsets
+            packed[o:o + r + 1] = list(accumulate(listed, initial=0))
             o += r + 1
-            np.concatenate(pens, axis=1, out=packed[o:n].reshape(2, n_pen))
+            np.concatenate([row.history.both() for row, n_row in zip(rows, listed) if n_row], axis=1,
+                           out=packed[o:n].reshape(2, n_pen))
+        # rows that are greedy, keep few tokens (the reference's default is top_k = 50) or cut nothing by top-k take
+        # the paths that read the logits with the whole GPU
+        path = {}
+        most, vocab = getattr(self.ops, "FEW_TOKENS", 0), logits.shape[1]
+        # (greedy rows without a penalty stay with the one launch: it is short as it is)
+        if most and (drawn or n_pen > 0 and vocab > FEW_GREEDY_TOKENS):
+            if all(t <= 0 or 1 <= k <= most for t, k in zip(temps, top_ks)):
+                path["few"] = True
+            elif vocab > SPREAD_TOKENS and all(t <= 0 or k <= most or k >= vocab for t, k in zip(temps, top_ks)):
+                path["spread"] = True
         if cuda:
-            dev = torch.empty(n, dtype=torch.int32, device=self.device)
-            dev.copy_(pinned[:n], non_blocking=True)
-            copied.record()
-        else:
-            dev = torch.from_numpy(packed)
+            self.ops.sample_rows(logits, r, pinned, n, n_pen, **path)
+            tokens = packed[at:at + r].tolist()
+            self._free.append(slot)   # (a call that failed keeps its buffer)
+            return tokens
+        dev = torch.from_numpy(packed)
         f = dev[:4 * r].view(torch.float32)
         pen = {}
         if n_pen > 0:
             pen = dict(pen_offsets=dev[o - r - 1:o], pen_tokens=dev[o:o + n_pen],
                        pen_counts=dev[o + n_pen:n])
         out = torch.empty(r, dtype=torch.int32, device=self.device)
-        # rows that are greedy, keep few tokens (the reference's default is top_k = 50) or cut nothing by top-k take
-        # the paths that read the logits with the whole GPU
-        most, vocab = getattr(self.ops, "FEW_TOKENS", 0), logits.shape[1]
-        # (greedy rows without a penalty stay with the one launch: it is short as it is)
-        if most and (drawn or n_pen > 0 and vocab > FEW_GREEDY_TOKENS):
-            if all(t <= 0 or 1 <= k <= most for t, k in zip(temps, top_ks)):
-                pen["few"] = True
-            elif vocab > SPREAD_TOKENS and all(t <= 0 or k <= most or k >= vocab for t, k in zip(temps, top_ks)):
-                pen["spread"] = True
         self.ops.sample(logits, f[:r], f[3 * r:4 * r], out, top_k=dev[4 * r:5 * r], top_p=f[r:2 * r],
-                        rep_penalty=f[2 * r:3 * r], **pen)
+                        rep_penalty=f[2 * r:3 * r], **pen, **path)
         return out.tolist()
