@@ -765,6 +765,18 @@ class HipOps:
             return False
         return not torch.cuda.is_current_stream_capturing()
 
+    def pays_beside(self, rows: int, weight_bytes: int, dtype) -> bool:
+        """Are a routed path and the independent work beside it (whose weights are so many bytes together) long enough on the
+        device for two streams where `wants_beside` says no? The host needs some 205 us a layer with them and 170 without, and
+        the device's time is near 165 us a GB of weights and 0.33 us a row: from 230 us on, for a step that finds the device
+        idle waits for the host first. ms a step on one stream and on two: 60 experts of 17 MB and a shared one of 69, 80 rows 5.77 and 5.92, 96
+        5.76 and 5.59, 128 6.11 and 6.10, 160 6.57 and 6.17, 420 7.75 and 7.08, in 32-bit 17 rows 6.44 and 6.23, 33
+        8.17 and 7.78, 100 11.71 and 11.35, but 150 13.8 and 14.6; 32 experts and one of 35 MB, 256 rows 2.08 and 2.12, 450 2.41 and
+        2.30; 16 experts of 4 MB 1.28 and 1.66. (In bfloat16 up to 64 rows,
+        in 32-bit up to 16, one stream: a decode step takes the same kernels run eagerly and captured.)"""
+        few, many = (65, 1 << 30) if dtype == torch.bfloat16 else (17, 100)
+        return few <= rows <= many and weight_bytes + rows * 2_000_000 >= 1_400_000_000
+
     def leaves_room(self, rows: int, features: int, to_fill: bool = False) -> bool:
         """Does a product of this size leave CUs, or places on them, to short kernels on another stream?
         While its tall tiles (256 x 256, one to a CU) would be fewer than the CUs, or than half of them where

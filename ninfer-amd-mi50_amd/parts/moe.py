@@ -171,6 +171,10 @@ class RoutedExperts(Part):
             w.matrix_into(p + self.names[1], self.w_gate_up[e, i:])
             w.matrix_into(p + self.names[2], self.w_down[e])
 
+    def weight_bytes(self) -> int:
+        """What a pass that chooses every expert reads of weights."""
+        return 3 * self.experts * self.inner * self.hidden * self.w_down.element_size()
+
     def gate_up(self, ctx: StepContext, x: torch.Tensor, routing: "Routing") -> torch.Tensor:
         """Activations [T*k, inner] in sorted order (row r belongs to the expert that
         owns sorted position r)."""
@@ -271,7 +275,10 @@ class SparseMoE(FeedForward):
         # they run on a stream of their own beside the routed path, whose kernels leave part
         # of the device empty in their last round of blocks.
         logits = ctx.empty((x.shape[0], self.router.experts + 1), torch.float32)
-        if ctx.ops.wants_beside(x.shape[0], self.shared.weight_bytes()):
+        own = self.shared.weight_bytes()
+        if ctx.ops.wants_beside(x.shape[0], own) or (
+                x.is_cuda and ctx.ops.pays_beside(x.shape[0], self.experts.weight_bytes() + own, x.dtype)
+                and not torch.cuda.is_current_stream_capturing()):
             # While its blocks leave the GPU room, the second stream starts before the routing's short
             # kernels and fills the device beside them; else after them: they would crawl.
             early = ctx.ops.leaves_room(x.shape[0], 2 * self.shared.inner, self._shared_fills(x.shape[0]))

@@ -324,3 +324,17 @@ def test_which_prompts_form_keys_and_values_per_head(lib, heads, rank, rd, vdim,
     assert HipOps.latent_heads_rows(ops, ctx, heads, 128 - rd, rank, rd, vdim, 4096) == ctx.T
     ctx.act_dtype = torch.float32
     assert first() == ctx.T
+
+
+# (experts, inner, shared inner of width 2,048; bytes a number)
+@pytest.mark.parametrize("sizes,size,rows,two", [
+    ((60, 1408, 5632), 2, 128, False), ((60, 1408, 5632), 2, 160, True), ((60, 1408, 5632), 4, 16, False), ((60, 1408, 5632), 4, 17, True),
+    ((32, 1408, 2816), 2, 384, False), ((32, 1408, 2816), 2, 420, True), ((60, 1408, 5632), 4, 100, True), ((60, 1408, 5632), 4, 101, False), ((32, 1408, 2816), 4, 30, False),
+    ((16, 704, 1408), 4, 500, False), ((60, 7040, 28160), 2, 64, False), ((60, 7040, 28160), 2, 65, True)])
+def test_which_short_steps_take_two_streams(sizes, size, rows, two):
+    import torch
+    from types import SimpleNamespace
+    from ninfer_amd.kernels.ops import HipOps
+    experts, inner, shared = sizes
+    weights = 3 * 2048 * (experts * inner + shared) * size
+    assert HipOps.pays_beside(SimpleNamespace(), rows, weights, torch.bfloat16 if size == 2 else torch.float32) == two
