@@ -325,7 +325,9 @@ class ModelRunner:
         if entry["graph"] is None:
             torch.cuda.synchronize()
             g = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(g):
+            capture = torch.cuda.graph(g)
+            self.ops.library_workspace(capture.capture_stream)
+            with capture:
                 entry["logits"] = self._forward(entry["meta"], shape)
             entry["graph"] = g
             if not self._holds_graphs:

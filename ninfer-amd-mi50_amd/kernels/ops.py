@@ -325,6 +325,7 @@ class _Beside:
         ops = self.ops
         if ops._side is None:
             ops._side = torch.cuda.Stream()   # default priority
+            ops.library_workspace(ops._side)
             ops._side_events = (ops._new_event(), ops._new_event())
         raw = ops._stream().value or 0
         if ops._main is None or ops._main.cuda_stream != raw:
@@ -739,6 +740,15 @@ class HipOps:
         self._ok(self.lib.ninfer_gemm(ctypes.byref(args), 1 if self.force_generic else 0,
                                       self._stream()))
         return True
+
+    @staticmethod
+    def library_workspace(stream) -> None:
+        """The library's products keep a workspace per stream (76 MB) from their first call on it until the process ends. Made
+        here, before anything else of the stream, it has memory of its own; made later it may lie in a larger block
+        that a step has left, which then cannot go back to the device."""
+        with torch.cuda.stream(stream):
+            t = torch.zeros(64, 64, dtype=torch.bfloat16, device="cuda")
+            torch.matmul(t, t.t())
 
     def _on_side(self) -> bool:
         return self._side is not None and (self._stream().value or 0) == self._side.cuda_stream

@@ -334,28 +334,6 @@ def wide_case(tmp_path_factory):
     return dirs, util.safe_prompt(w16, rcfg, 640, 5)
 
 
-@pytest.mark.parametrize("dtype,rows", [("float32", 17), ("float32", 200), ("bfloat16", 65), ("bfloat16", 200)])
-def test_short_steps_on_two_streams(wide_case, dtype, rows):
-    """Steps whose weights are many take the second stream from far fewer rows on: the same products (in 32-bit the same
-    bits; the first stream's logits are the plain model's within the usual bound)."""
-    from ninfer_amd import EngineOptions, load_model
-    dirs, toks = wide_case
-    rcfg, w = util.read_folder(dirs[dtype])
-    runner = load_model(dirs[dtype], EngineOptions(dtype=dtype, max_context=704, prefill_chunk=640, num_sequences=2,
-                                                   page_size=16))
-    ops, got = runner.ops, {}
-    try:
-        for two in (False, True):
-            ops.pays_beside = lambda rows, weight_bytes, dtype: two
-            got[two] = util.run_schedule(runner, util.schedule_whole(f"s{two}", toks[:rows]))[f"s{two}"]
-    finally:
-        del ops.pays_beside
-    assert ops._side is not None and not ops._side_open
-    if dtype == "float32":
-        assert torch.equal(got[True], got[False])
-    torch.testing.assert_close(got[True], plain_model.forward(w, rcfg, toks[:rows]), **bound(dtype))
-
-
 @pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
 def test_long_prompt_on_the_many_row_kernels(wide_case, dtype):
     from ninfer_amd import EngineOptions, load_model

@@ -1,0 +1,33 @@
+"""A shared expert on the second stream beside the routed experts, in steps of fewer rows than always take it."""
+import pytest
+import torch
+
+import plain_model
+import util
+from test_engine_gpu import CONFIG_WIDE, bound
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype,rows", [("float32", 17), ("float32", 200), ("bfloat16", 65), ("bfloat16", 200)])
+def test_short_steps_on_two_streams(tmp_path, dtype, rows):
+    """Steps whose weights are many take the second stream from far fewer rows on: the same products (in 32-bit the same
+    bits; the first stream's logits are the plain model's within the usual bound)."""
+    import ninfer_amd
+    from ninfer_amd import EngineOptions, load_model
+    ninfer_amd.write_random_model(str(tmp_path), CONFIG_WIDE, 77, dtype=dtype, std=0.06)
+    rcfg, w = util.read_folder(str(tmp_path))
+    toks = util.safe_prompt(w, rcfg, rows, 5)
+    runner = load_model(str(tmp_path), EngineOptions(dtype=dtype, max_context=704, prefill_chunk=640, num_sequences=2,
+                                                   page_size=16))
+    ops, got = runner.ops, {}
+    try:
+        for two in (False, True):
+            ops.pays_beside = lambda rows, weight_bytes, dtype: two
+            got[two] = util.run_schedule(runner, util.schedule_whole(f"s{two}", toks))[f"s{two}"]
+    finally:
+        del ops.pays_beside
+    assert ops._side is not None and not ops._side_open
+    if dtype == "float32":
+        assert torch.equal(got[True], got[False])
+    torch.testing.assert_close(got[True], plain_model.forward(w, rcfg, toks), **bound(dtype))
