@@ -59,6 +59,22 @@ extern "C" int ninfer_gemm_split_parts(const GemmArgs* args) {
   return gemm_split_parts(*args);
 }
 
+// A plain dense product, if the kernels here cut it along K (with a workspace) or run it in one round of tiles: 1, or 0: the
+// caller's library has it.
+extern "C" int ninfer_gemm_cut_or_mid(const GemmArgs* args, hipStream_t stream) {
+  const GemmArgs& a = *args;
+  int rc = gemm_check(a);
+  if (rc) return rc < 0 ? rc : -rc;
+  if (gemm_split_parts(a) >= 2) {
+    rc = gemm_split(a, stream);
+  } else {
+    if (!gemm_mid_takes(a)) return 0;
+    const GemmKernel kernel = gemm_kernel(a);   // (which need not be that of the tiles)
+    rc = kernel == kGemmTile ? gemm_mid(a, stream) : ninfer_gemm(args, 0, stream);
+  }
+  return rc == 0 ? 1 : rc < 0 ? rc : -rc;
+}
+
 // The last entry of the list of 16-row tiles (tall = 0) or of tall ones that a grouped launch reads.
 extern "C" int ninfer_gemm_last_list_entry(const GemmArgs* a, int tall) {
   const int rows = tall ? kGroupedTileRows : 16;

@@ -365,13 +365,14 @@ class HipOps:
         self.lib_path = lib_path or ensure_built()
         self.lib = ctypes.CDLL(self.lib_path)
         self.lib.ninfer_last_error.restype = ctypes.c_char_p
-        _need(self.lib.ninfer_gemm_args_bytes() == ctypes.sizeof(_GemmArgs),
-              f"{self.lib_path} and these bindings lay a product's arguments out differently")
+        if not (self.lib.ninfer_gemm_args_bytes() == ctypes.sizeof(_GemmArgs)):
+            raise KernelError(f"{self.lib_path} and these bindings lay a product's arguments out differently")
         self.lib.ninfer_attention_workspace_floats.restype = ctypes.c_longlong
         self.lib.ninfer_event_create.restype = ctypes.c_void_p
         self.lib.ninfer_stream_after.argtypes = [ctypes.c_void_p] * 3
         self.lib.ninfer_sample_spread_bytes.restype = ctypes.c_longlong
         p, i = ctypes.c_void_p, ctypes.c_int
+        self.lib.ninfer_gemm.argtypes = [p, i, p]
         self.lib.ninfer_sample_rows.argtypes = [p, i, i, i, i, p, p, ctypes.c_longlong, i, p, p, p]
         self.lib.ninfer_latent_attention_workspace_floats.restype = ctypes.c_longlong
         self.lib.ninfer_gla_segment_floats.restype = ctypes.c_longlong
@@ -487,7 +488,8 @@ class HipOps:
         pages that were given back)."""
         _dev(pool, "pool")
         _dev(pages, "pages", torch.int32, 1)
-        _need(pool.dtype in _DT, f"fill_nan_pages: pool of {pool.dtype}")
+        if not (pool.dtype in _DT):
+            raise KernelError(f"fill_nan_pages: pool of {pool.dtype}")
         per_page = pool.numel() // pool.shape[0]
         self._ok(self.lib.ninfer_fill_nan_pages(
             ctypes.c_void_p(pool.data_ptr()), ctypes.c_void_p(pages.data_ptr()), pages.shape[0],
@@ -498,7 +500,8 @@ class HipOps:
         function of the 64-bit key and the flat index (see weights/counter_random.py, which
         computes the same bits on the host)."""
         _dev(out, "out")
-        _need(out.dtype in _DT, f"fill_random: tensor of {out.dtype}")
+        if not (out.dtype in _DT):
+            raise KernelError(f"fill_random: tensor of {out.dtype}")
         self._ok(self.lib.ninfer_fill_random(
             ctypes.c_void_p(out.data_ptr()), ctypes.c_longlong(out.numel()),
             ctypes.c_ulonglong(key & ((1 << 64) - 1)), ctypes.c_float(std), ctypes.c_float(mean),
@@ -605,7 +608,8 @@ class HipOps:
         _dev(qkv, "qkv", dims=2)
         t = qkv.shape[0]
         width = (n_q + 2 * n_kv) * head_dim
-        _need(qkv.shape[1] == width, f"rope_kv_write: qkv width {qkv.shape[1]} != {width}")
+        if not (qkv.shape[1] == width):
+            raise KernelError(f"rope_kv_write: qkv width {qkv.shape[1]} != {width}")
         if bias is not None:
             _dev(bias, "bias", torch.float32, 1)
             _need(bias.shape[0] == width, "rope_kv_write: bias has the wrong size")
@@ -617,9 +621,9 @@ class HipOps:
             _need(inv_freq.shape[0] == rot_dim // 2, "rope_kv_write: table size != rot_dim / 2")
         _dev(k_pool, "k_pool", qkv.dtype, 4)
         _dev(v_pool, "v_pool", qkv.dtype, 4)
-        _need(k_pool.shape == v_pool.shape and k_pool.shape[1:] == (n_kv, page_size, head_dim),
-              f"rope_kv_write: pools {tuple(k_pool.shape)} do not fit (kv heads {n_kv}, page "
-              f"{page_size}, head {head_dim})")
+        if not (k_pool.shape == v_pool.shape and k_pool.shape[1:] == (n_kv, page_size, head_dim)):
+            raise KernelError(f"rope_kv_write: pools {tuple(k_pool.shape)} do not fit (kv heads {n_kv}, page "
+                              f"{page_size}, head {head_dim})")
         _dev(block_table, "block_table", torch.int32, 2)
         _need((q_norm is None) == (k_norm is None), "rope_kv_write: both heads' norms or neither")
         if q_norm is not None:
@@ -701,45 +705,58 @@ class HipOps:
             ctypes.c_void_p(_ptr(gate)), stride, t, h, k, _DT[y.dtype], self._stream()))
 
     # ---- products ---------------------------------------------------------------
-    def _gemm(self, a, w, c, *, n, k, m, bias=None, offsets=None, a_index=None, c_index=None,
-              a_div=1, groups=1, epilogue=0, w_group_stride=0, tiles=None, only_if_split=False,
-              only_if_mid=False, act_limit=0.0, act_alpha=1.0):
+    def _gemm_args(self, a, w, c, n, k, m, bias=None, offsets=None, a_index=None, c_index=None, a_div=1, groups=1,
+                   epilogue=0, w_group_stride=0, tiles=None, act_limit=0.0, act_alpha=1.0, workspace=None):
         t16 = t64 = tc = None
         if tiles is not None and tiles.tiles16 is not None:
             t16, t64, tc = tiles.tiles16.data_ptr(), tiles.tiles_big.data_ptr(), \
                 tiles.tile_counts.data_ptr()
-        args = _GemmArgs(a.data_ptr(), w.data_ptr(), c.data_ptr(), _ptr(bias), _ptr(offsets),
-                         _ptr(a_index), _ptr(c_index), t16, t64, tc, w_group_stride, m, n, k,
-                         a.shape[1],
-                         c.shape[1], groups, a_div, _DT[a.dtype], _DT[c.dtype], epilogue)
-        args.force_kernel = self._tune["force_kernel"]
-        args.split_min_bytes = self._tune["split_min_bytes"]
-        args.skinny_two = self._tune["skinny_two"]
-        args.act_limit, args.act_alpha = float(act_limit), float(act_alpha)
-        args.beside = 1 if self._side_inside or self._side_open else 0
+        tune = self._tune
+        # (by position: setting fields one by one costs the host twice the time)
+        return _GemmArgs(a.data_ptr(), w.data_ptr(), c.data_ptr(), None if bias is None else bias.data_ptr(),
+                         None if offsets is None else offsets.data_ptr(), None if a_index is None else a_index.data_ptr(),
+                         None if c_index is None else c_index.data_ptr(), t16, t64, tc, w_group_stride, m, n, k,
+                         a.shape[1], c.shape[1], groups, a_div, _DT[a.dtype], _DT[c.dtype], epilogue, 0,
+                         None if workspace is None else workspace.data_ptr(), 0 if workspace is None else workspace.numel(),
+                         tune["split_min_bytes"], tune["force_kernel"], tune["skinny_two"], float(act_limit),
+                         float(act_alpha), 1 if self._side_inside or self._side_open else 0)
+
+    def _split_workspace(self, device):
+        """The one workspace of products cut along K. It belongs to the main stream: on the second nothing is cut."""
+        if self._split_ws is None:
+            self._split_ws = torch.empty(1 << 23, dtype=torch.float32, device=device)
+        return self._split_ws
+
+    def _gemm(self, a, w, c, *, n, k, m, only_if_split=False, only_if_mid=False, **more):
         if only_if_split:
             # a dense product of few dozen rows: the library's unless the kernels here cut it
-            # along K (its output tiles alone would not fill the GPU). The one workspace of
-            # the cut belongs to the main stream: on the second stream nothing is cut (the
-            # library's product runs instead).
+            # along K (its output tiles alone would not fill the GPU)
             if self._on_side():
                 return False
-            if self._split_ws is None:
-                self._split_ws = torch.empty(1 << 23, dtype=torch.float32, device=a.device)
-            args.workspace = self._split_ws.data_ptr()
-            args.workspace_floats = self._split_ws.numel()
+            args = self._gemm_args(a, w, c, n, k, m, workspace=self._split_workspace(a.device), **more)
             if self.lib.ninfer_gemm_split_parts(ctypes.byref(args)) < 2:
                 return False
             self._ok(self.lib.ninfer_gemm(ctypes.byref(args), 0, self._stream()))
             return True
+        args = self._gemm_args(a, w, c, n, k, m, **more)
         if only_if_mid and not self.lib.ninfer_gemm_mid_tile(ctypes.byref(args)):
             return False
         if self._held is not None:
-            self._held.append((args, (a, w, c, bias, offsets, a_index, c_index, tiles)))
+            self._held.append((args, (a, w, c, more)))
             return True
         self._ok(self.lib.ninfer_gemm(ctypes.byref(args), 1 if self.force_generic else 0,
                                       self._stream()))
         return True
+
+    def _gemm_cut_or_mid(self, a, w, c, *, n, k, m, cut):
+        """A plain dense product, if the kernels here cut it along K (`cut`: they may) or it is one round of tiles; False: it
+        is the library's. One set of arguments and one call, where asking for each and then launching took three:
+        6 us of the host's time a product, of some 14, which bounds steps of up to a few hundred rows."""
+        args = self._gemm_args(a, w, c, n, k, m, workspace=self._split_workspace(a.device) if cut else None)
+        rc = self.lib.ninfer_gemm_cut_or_mid(ctypes.byref(args), self._stream())
+        if rc < 0:
+            self._ok(rc)
+        return rc > 0
 
     @staticmethod
     def library_workspace(stream) -> None:
@@ -848,35 +865,41 @@ class HipOps:
         """out = x w^T (+ bias); out may be 32-bit whatever the inputs are. `act` 'relu2': the
         square of relu on every element of out."""
         # (an activation runs in the product's epilogue, on the kernels here at every row count)
-        _need(act in UNGATED_ACTS, f"linear: activation {act!r} is not one of {sorted(map(str, UNGATED_ACTS))}")
+        if not (act in UNGATED_ACTS):
+            raise KernelError(f"linear: activation {act!r} is not one of {sorted(map(str, UNGATED_ACTS))}")
         _dev(x, "x", dims=2)
         _dev(w, "w", x.dtype, 2)
         _dev(out, "out", dims=2)
-        _need(x.shape[1] == w.shape[1], f"linear: x has {x.shape[1]} columns, w has {w.shape[1]}")
-        _need(out.shape == (x.shape[0], w.shape[0]), "linear: out has the wrong shape")
+        (rows, k), (n, wk) = x.shape, w.shape
+        if k != wk:
+            raise KernelError(f"linear: x has {k} columns, w has {wk}")
+        _need(out.shape == (rows, n), "linear: out has the wrong shape")
         _need(out.dtype in (x.dtype, torch.float32), "linear: bad out dtype")
         if bias is not None:
             _dev(bias, "bias", torch.float32, 1)
-            _need(bias.shape[0] == w.shape[0], "linear: bias has the wrong size")
-        if act is None and self._use_library(x, out, w) and bias is None and not (
-                x.shape[0] <= self.side_own_max_rows
-                and w.numel() * w.element_size() <= self.side_own_max_bytes and self._on_side()):
+            _need(bias.shape[0] == n, "linear: bias has the wrong size")
+        if act is None and bias is None and self._use_library(x, out, w) and not (
+                rows <= self.side_own_max_rows
+                and n * k * w.element_size() <= self.side_own_max_bytes and self._on_side()):
             own = self._rows_kernel_takes(x, w)
             if not own or self._tune["split_min_bytes"]:
-                if x.shape[0] <= self.split_max_rows and self._gemm(
-                        x, w, out, m=x.shape[0], n=w.shape[0], k=x.shape[1], only_if_split=True):
-                    return
-                if not own:
+                cut = rows <= self.split_max_rows
+                if not own and self._held is None:
                     # one round of tiles: as fast here as in the library, or faster, and 16 us less of the host's
                     # time a call, which bounds short steps that run eagerly (gemm_mid.hip)
-                    if not self._gemm(x, w, out, m=x.shape[0], n=w.shape[0], k=x.shape[1], only_if_mid=True):
+                    if not self._gemm_cut_or_mid(x, w, out, m=rows, n=n, k=k, cut=cut and not self._on_side()):
+                        torch.matmul(x, w.t(), out=out)
+                    return
+                if cut and self._gemm(x, w, out, m=rows, n=n, k=k, only_if_split=True):
+                    return
+                if not own:
+                    if not self._gemm(x, w, out, m=rows, n=n, k=k, only_if_mid=True):
                         torch.matmul(x, w.t(), out=out)
                     return
         elif act is None and bias is None and self._rows_cut(x, out, w) and self._gemm(
-                x, w, out, m=x.shape[0], n=w.shape[0], k=x.shape[1], only_if_split=True):
+                x, w, out, m=rows, n=n, k=k, only_if_split=True):
             return
-        self._gemm(x, w, out, m=x.shape[0], n=w.shape[0], k=x.shape[1], bias=bias,
-                   epilogue=UNGATED_ACTS[act])
+        self._gemm(x, w, out, m=rows, n=n, k=k, bias=bias, epilogue=UNGATED_ACTS[act])
 
     def _use_library(self, x, out, w) -> bool:
         """Plain dense products of many bf16 rows go to the vendor library, as
@@ -925,7 +948,8 @@ class HipOps:
 
     @staticmethod
     def _gate_epilogue(act: str) -> int:
-        _need(act in GATE_ACTS, f"gated product: activation {act!r} is not one of {sorted(GATE_ACTS)}")
+        if not (act in GATE_ACTS):
+            raise KernelError(f"gated product: activation {act!r} is not one of {sorted(GATE_ACTS)}")
         return GATE_ACTS[act]
 
     def swiglu_linear(self, x, w_gate_up, out, act="silu", bias=None, limit=0.0, alpha=1.0):
@@ -990,8 +1014,10 @@ class HipOps:
         neighbours each) with the largest best score (+ bias) are candidates (`group_top` > 1:
         with the largest sum of their group_top best); `renorm_eps` is added to the sum the
         chosen scores are divided by."""
-        _need(score in _SCORES, f"routing: score {score!r} is not one of {sorted(_SCORES)}")
-        _need(1 <= top_k <= experts, f"routing: top_k {top_k} not in [1, {experts}]")
+        if not (score in _SCORES):
+            raise KernelError(f"routing: score {score!r} is not one of {sorted(_SCORES)}")
+        if not (1 <= top_k <= experts):
+            raise KernelError(f"routing: top_k {top_k} not in [1, {experts}]")
         if choice_bias is not None:
             _dev(choice_bias, "choice_bias", torch.float32, 1)
             _need(choice_bias.shape[0] == experts, "routing: one bias per expert")
@@ -1171,12 +1197,12 @@ class HipOps:
     def _blocks_fit(blocks, dtype, n_kv, dim, vdim, ctx, who):
         for name, n in (("k_block", dim), ("v_block", vdim)):
             _dev(blocks[name], name, dtype, 4)
-            _need(blocks[name].shape[1:] == (n_kv, blocks.page_size, n)
-                  and blocks[name].shape[0] == blocks["k_block"].shape[0],
-                  f"{who}: the pools of blocks do not fit the head layout")
+            if not (blocks[name].shape[1:] == (n_kv, blocks.page_size, n)
+                    and blocks[name].shape[0] == blocks["k_block"].shape[0]):
+                raise KernelError(f"{who}: the pools of blocks do not fit the head layout")
         _dev(blocks.block_table, "blocks.block_table", torch.int32, 2)
-        _need(blocks.block_table.shape[0] == ctx.S and blocks.stride >= 1,
-              f"{who}: block table rows of blocks != requests")
+        if not (blocks.block_table.shape[0] == ctx.S and blocks.stride >= 1):
+            raise KernelError(f"{who}: block table rows of blocks != requests")
 
     def qkv_wide(self, u, ctx, q_out, heads, kv_heads, dim, vdim, k_pool, v_pool, block_table,
                  page_size, v_col=None, q_norm=None, k_norm=None, norm_eps=0.0, inv_freq=None,
@@ -1200,8 +1226,8 @@ class HipOps:
         _dev(block_table, "block_table", torch.int32, 2)
         t, nq, nk, nv = ctx.T, heads * dim, kv_heads * dim, kv_heads * vdim
         v_col = nq + nk if v_col is None else int(v_col)
-        _need(u.shape[0] == t and u.shape[1] >= max(nq + nk, v_col + nv) and v_col >= 0
-              and q_out.shape == (t, nq), f"qkv_wide: rows of {tuple(u.shape)} do not hold the heads")
+        if not (u.shape[0] == t and u.shape[1] >= max(nq + nk, v_col + nv) and v_col >= 0 and q_out.shape == (t, nq)):
+            raise KernelError(f"qkv_wide: rows of {tuple(u.shape)} do not hold the heads")
         _need(k_pool.shape[0] == v_pool.shape[0] and k_pool.shape[1:] == (kv_heads, page_size, dim)
               and v_pool.shape[1:] == (kv_heads, page_size, vdim) and block_table.shape[0] == ctx.S,
               "qkv_wide: pools or block table do not fit the head layout")
@@ -1209,7 +1235,8 @@ class HipOps:
                            (inv_freq if rot_dim else None, rot_dim // 2, "inv_freq")):
             if g is not None:
                 _dev(g, name, torch.float32, 1)
-                _need(g.shape[0] == n, f"qkv_wide: {name} has {g.shape[0]} numbers, not {n}")
+                if not (g.shape[0] == n):
+                    raise KernelError(f"qkv_wide: {name} has {g.shape[0]} numbers, not {n}")
         _need(rot_dim == 0 or (inv_freq is not None and rot_dim <= dim), "qkv_wide: rotation without a table")
         a = _QkvWideArgs()
         a.u, a.q_out, a.kpool, a.vpool = u.data_ptr(), q_out.data_ptr(), k_pool.data_ptr(), v_pool.data_ptr()
@@ -1249,8 +1276,8 @@ class HipOps:
         _dev(q_out, "q_out", u.dtype, 2)
         t = ctx.T
         channels = heads * dim + kv_heads * (dim + vdim)
-        _need(u.dtype in _DT and u.shape == (t, channels) and q_out.shape == (t, heads * dim),
-              f"qkv_conv: rows of {tuple(u.shape)} for {channels} channels")
+        if not (u.dtype in _DT and u.shape == (t, channels) and q_out.shape == (t, heads * dim)):
+            raise KernelError(f"qkv_conv: rows of {tuple(u.shape)} for {channels} channels")
         a = _QkvConvArgs()
         a.u, a.q_out = u.data_ptr(), q_out.data_ptr()
         taps = 0
@@ -1282,7 +1309,8 @@ class HipOps:
         for g, name in ((q_norm, "q_norm"), (k_norm, "k_norm")):
             if g is not None:
                 _dev(g, name, torch.float32, 1)
-                _need(g.shape[0] == dim, f"qkv_conv: {name} has one gain per number of a head")
+                if not (g.shape[0] == dim):
+                    raise KernelError(f"qkv_conv: {name} has one gain per number of a head")
         _need(kv_heads == 0 or (q_norm is None) == (k_norm is None), "qkv_conv: both heads' norms or neither")
         a.q_gain, a.k_gain = _ptr(q_norm), _ptr(k_norm)
         if rot_dim:
@@ -1310,7 +1338,8 @@ class HipOps:
         t, h = x.shape
         taps = w.shape[1]
         _need(w.shape[0] == h and out.shape == (t, h), "short_conv: shapes")
-        _need(out.dtype in _DT, f"short_conv: out of {out.dtype}")
+        if not (out.dtype in _DT):
+            raise KernelError(f"short_conv: out of {out.dtype}")
         if taps == 1 and state is None:   # one tap keeps nothing
             state_ptr, state_stride = None, 0
         else:
@@ -1409,7 +1438,8 @@ class HipOps:
         _dev(weight, "weight", torch.float32, 1)
         _dev(out, "out", dims=2)
         t, n = o.shape
-        _need(gate_act in ("sigmoid", "silu"), f"gated_rmsnorm: gate activation {gate_act!r}")
+        if not (gate_act in ("sigmoid", "silu")):
+            raise KernelError(f"gated_rmsnorm: gate activation {gate_act!r}")
         _need(group >= 0 and (group == 0 or n % group == 0), "gated_rmsnorm: groups do not fill the rows")
         _need(out.shape == (t, n) and weight.shape[0] in (group or n, n) and out.dtype in _DT,
               "gated_rmsnorm: shapes")
@@ -1492,15 +1522,15 @@ class HipOps:
     @staticmethod
     def _columns(x, width, who):
         """The row stride of [T, >= width] columns of a row-major tensor."""
-        _need(x.is_cuda and x.dim() == 2 and x.stride(1) == 1 and x.dtype in _DT and x.shape[1] >= width,
-              f"{who} must be columns of rows")
+        if not (x.is_cuda and x.dim() == 2 and x.stride(1) == 1 and x.dtype in _DT and x.shape[1] >= width):
+            raise KernelError(f"{who} must be columns of rows")
         return x.stride(0) if x.shape[0] > 1 else max(x.shape[1], x.stride(0))
 
     @staticmethod
     def _state_rows(state, floats, who):
-        _need(state is not None and state.is_cuda and state.dtype == torch.float32 and state.dim() == 2
-              and state.stride(1) == 1 and state.shape[1] >= floats,
-              f"{who}: the state must be 32-bit rows of at least {floats} numbers")
+        if not (state is not None and state.is_cuda and state.dtype == torch.float32 and state.dim() == 2
+                and state.stride(1) == 1 and state.shape[1] >= floats):
+            raise KernelError(f"{who}: the state must be 32-bit rows of at least {floats} numbers")
 
     def conv_silu(self, u, w, bias, state, ctx, out):
         """out = silu(bias + sum_j w[j] u_(t - taps + 1 + j)) per channel over the rows of each
@@ -1581,7 +1611,8 @@ class HipOps:
         a = self._scan_args(xbc, inner + groups * dim, inner, 0, dt, dt_bias, heads, groups, dim, vdim, state, ctx, 0)
         for g, name in ((rate, "rate"), (skip, "skip")):
             _dev(g, name, torch.float32, 1)
-            _need(g.shape[0] == heads, f"state_space: one {name} per head")
+            if not (g.shape[0] == heads):
+                raise KernelError(f"state_space: one {name} per head")
         _dev(out, "out", torch.float32, 2)
         _need(out.shape == (ctx.T, inner), "state_space: out has the wrong shape")
         a.rate, a.skip, a.out = rate.data_ptr(), skip.data_ptr(), out.data_ptr()
@@ -1623,7 +1654,8 @@ class HipOps:
         _dev(decay, "decay", torch.float32, 1)
         _dev(out, "out", torch.float32, 2)
         t = qkv.shape[0]
-        _need(qkv.dtype in _DT, f"lightning_attention: rows of {qkv.dtype}")
+        if not (qkv.dtype in _DT):
+            raise KernelError(f"lightning_attention: rows of {qkv.dtype}")
         _need(decay.shape[0] == heads and out.shape == (t, heads * vdim) and ctx.T == t,
               "lightning_attention: shapes")
         for off, n in ((q_off, heads * dim), (k_off, heads * dim), (v_off, heads * vdim)):
@@ -1654,9 +1686,9 @@ class HipOps:
     def _latent_args(self, ctx, pool, block_table, heads, dim, rank, rot_dim, rot_n, page_size,
                      dtype):
         _dev(pool, "pool", dtype, 3)
-        _need(pool.shape[1:] == (page_size, rank + rot_dim),
-              f"latent attention: pool {tuple(pool.shape)} does not fit pages of {page_size} rows "
-              f"of {rank + rot_dim}")
+        if not (pool.shape[1:] == (page_size, rank + rot_dim)):
+            raise KernelError(f"latent attention: pool {tuple(pool.shape)} does not fit pages of {page_size} rows "
+                              f"of {rank + rot_dim}")
         _dev(block_table, "block_table", torch.int32, 2)
         _need(block_table.shape[0] == ctx.S, "latent attention: block table rows != requests")
         a = _LatentArgs()
@@ -1894,7 +1926,8 @@ class HipOps:
         for name, sc in (("s1", s1), ("s2", s2)):
             if sc is not None:
                 _dev(sc, name, torch.float32, 1)
-                _need(sc.shape[0] == h, f"scaled_sum_add: {name} has the wrong size")
+                if not (sc.shape[0] == h):
+                    raise KernelError(f"scaled_sum_add: {name} has the wrong size")
         dense = y = w = shared = gate = None
         k = gs = 0
         if f is not None and hasattr(f, "weights"):
@@ -1924,7 +1957,8 @@ class HipOps:
     def relu_square(self, x):
         """x <- max(x, 0)^2 in place."""
         _dev(x, "x")
-        _need(x.dtype in _DT, f"relu_square: tensor of {x.dtype}")
+        if not (x.dtype in _DT):
+            raise KernelError(f"relu_square: tensor of {x.dtype}")
         self._ok(self.lib.ninfer_relu_square(ctypes.c_void_p(x.data_ptr()),
                                              ctypes.c_longlong(x.numel()), _DT[x.dtype],
                                              self._stream()))
@@ -1940,7 +1974,8 @@ class HipOps:
         by out_scale. Scores: (q . k) scale (1 + temp_coef ln(floor((p + 1) / temp_every) + 1))
         at the row's position p, then cap tanh(. / cap) when cap > 0. out: [T, heads x vdim]."""
         _dev(qkv, "qkv", dims=2)
-        _need(qkv.dtype in _DT, f"diff_attention: rows of {qkv.dtype}")
+        if not (qkv.dtype in _DT):
+            raise KernelError(f"diff_attention: rows of {qkv.dtype}")
         _dev(k_pool, "k_pool", qkv.dtype, 4)
         _dev(v_pool, "v_pool", qkv.dtype, 4)
         _dev(out, "out", qkv.dtype, 2)
@@ -2013,11 +2048,13 @@ class HipOps:
             if g is None:
                 continue
             _dev(g, "g" + name, dtype, 2)
-            _need(g.shape == (t, h), f"gated_sum_add: gate {name} does not fit")
+            if not (g.shape == (t, h)):
+                raise KernelError(f"gated_sum_add: gate {name} does not fit")
             setattr(p, "g" + name, g.data_ptr())
             if b is not None:
                 _dev(b, "b" + name, torch.float32, 1)
-                _need(b.shape[0] == h, f"gated_sum_add: bias {name} has the wrong size")
+                if not (b.shape[0] == h):
+                    raise KernelError(f"gated_sum_add: bias {name} has the wrong size")
                 setattr(p, "b" + name, b.data_ptr())
         p.dtype = _DT[dtype]
         self._ok(self.lib.ninfer_gated_sum_add(ctypes.byref(p), self._stream()))
@@ -2051,7 +2088,8 @@ class HipOps:
         _dev(out, "out", torch.float32, 2)
         t = qkv.shape[0]
         row = qkv.stride(0) if t > 1 else max(qkv.shape[1], qkv.stride(0))
-        _need(qkv.dtype in _DT, f"gated_linear_attention: rows of {qkv.dtype}")
+        if not (qkv.dtype in _DT):
+            raise KernelError(f"gated_linear_attention: rows of {qkv.dtype}")
         _need(out.shape == (t, heads * vdim) and ctx.T == t, "gated_linear_attention: shapes")
         f_off, f_bias, lower = forget if forget is not None else (0, None, None)
         if forget is None:
@@ -2060,7 +2098,8 @@ class HipOps:
         else:
             for g, name in ((f_bias, "bias"), (lower, "lower")):
                 _dev(g, name, torch.float32, 1)
-                _need(g.shape[0] == heads * dim, f"gated_linear_attention: {name} has one number per channel")
+                if not (g.shape[0] == heads * dim):
+                    raise KernelError(f"gated_linear_attention: {name} has one number per channel")
         gate_args = (int(f_off), ctypes.c_void_p(_ptr(f_bias)), ctypes.c_void_p(_ptr(lower)))
         for off, n in ((q_off, heads * dim), (k_off if forget is None else f_off, heads * dim),
                        (v_off, heads * vdim)):
@@ -2105,7 +2144,8 @@ class HipOps:
         weights are mixed (w'_a = sum_b mix[a, b] w_b); head a applies its weights to the
         values of kv head a // (heads / kv_heads). out: [T, heads x vdim]."""
         _dev(qkv, "qkv", dims=2)
-        _need(qkv.dtype in _DT, f"sigmoid_attention: rows of {qkv.dtype}")
+        if not (qkv.dtype in _DT):
+            raise KernelError(f"sigmoid_attention: rows of {qkv.dtype}")
         _dev(k_pool, "k_pool", qkv.dtype, 4)
         _dev(v_pool, "v_pool", qkv.dtype, 4)
         _dev(out, "out", qkv.dtype, 2)
@@ -2191,7 +2231,8 @@ class HipOps:
                             ("rep_penalty", rep_penalty, torch.float32)):
             if t is not None:
                 _dev(t, name, dt, 1)
-                _need(t.shape[0] == r, f"sample: {name} has the wrong size")
+                if not (t.shape[0] == r):
+                    raise KernelError(f"sample: {name} has the wrong size")
         if pen_offsets is not None:
             _dev(pen_offsets, "pen_offsets", torch.int32, 1)
             _dev(pen_tokens, "pen_tokens", torch.int32, 1)

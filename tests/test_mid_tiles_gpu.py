@@ -90,3 +90,23 @@ def test_plain_products_of_one_round_stay_out_of_the_library(monkeypatch, m, n, 
     monkeypatch.setattr(torch, "matmul", None)
     ops.linear(x, w, out)
     assert float((out.double() - want).norm() / want.norm()) < 2.0 ** -8
+
+
+# (rows, features, K: cut along K, one round of tiles, more rows than are cut, more than a round)
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k,taken", [(100, 3584, 20480, True), (256, 2048, 2048, True), (513, 2048, 1024, True),
+                                         (4096, 8192, 512, False)])
+def test_one_call_runs_what_the_questions_one_by_one_would(m, n, k, taken):
+    from ninfer_amd.kernels import load_ops
+    ops = load_ops()
+    gen = torch.Generator("cuda").manual_seed(m)
+    x, w = (torch.randn(*s, generator=gen, device="cuda").to(torch.bfloat16) for s in ((m, k), (n, k)))
+    one, each = (torch.zeros(m, n, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    assert ops._gemm_cut_or_mid(x, w, one, m=m, n=n, k=k, cut=m <= ops.split_max_rows) == taken
+    asked = m <= ops.split_max_rows and ops._gemm(x, w, each, m=m, n=n, k=k, only_if_split=True) or \
+        ops._gemm(x, w, each, m=m, n=n, k=k, only_if_mid=True)
+    assert asked == taken and torch.equal(one, each)
+    ops.linear(x, w, each)
+    assert not taken or torch.equal(one, each)
+    with pytest.raises(Exception, match="lda"):
+        ops._gemm_cut_or_mid(x[:, :64].contiguous(), w, one, m=m, n=n, k=k, cut=True)
