@@ -2,20 +2,23 @@
 // to some 2,000 rows of hundreds to thousands of features. Tiles of nine sizes, 32 x 64 to 192 x 128 and 128 x 192 (rows of A x
 // rows of W), one block of eight waves to a CU; the smallest of which a round holds all is taken.
 //
+// Every output is one chain of sums along K, 32 numbers an instruction, as in the taller tiles and in the library's products
+// that are not cut along K: the same bits, whichever of them a product's size sends it to. (Groups of waves that took k tiles
+// in turn and added their sums at the end were no faster, and moved a model's logits by as much as bfloat16's rounding does.)
+//
 // What bounds a lone block is its way from L2 into LDS: some 80 GB/s a CU for loads straight into LDS (37 bytes a
 // clock), so a tile's time goes with its rows of A and W together, whatever it multiplies, and four waves that wait for each
-// other at a barrier per k tile leave even that unused (64 x 128 in four waves 18 us at K 2,048, so 16). The lower
-// tiles' waves therefore form two or four groups that take k tiles in turn, with one barrier for two or four of
-// them; the groups' sums meet in LDS. Where a CU's rows are more, all eight waves share a k tile. Stages lie in a ring, all of it
-// asked for ahead: when a wave passes the barrier of stage s, stage s + 1 has landed for every wave and every wave
-// holds the last fragments of stage s in registers, so its place takes stage s + NB. The first half's fragments of the next
-// stage are read while the second half of this one is multiplied.
-// Against the library's product, us, K 2,048 (host time 9 us a call against 24): 2,048 features, 256 rows 10.5 and 12.1, 512
-// 12.0 and 13.1, 1,280 18.5 and 22.0, 2,048 21.1 and 23.5; 4,096, 160 rows 10.6 and 15.4, 768 20.4 and 23.2, 1,531 26.6 and
-// 28.2; 6,144, 256 rows 15.5 and 23.5, 512 21.1 and 23.6, 1,024 28.8 and 28.9; 1,024 features of K 1,024, 512 rows 6.5 and
-// 8.5; of K 2,816 10.1 and 12.0; 2,048 of K 5,632, 256 rows 21.8 and 20.8, 384 28.3 and 25.3, 768 32.6 and 33.6.
-// Against tiles of 64 and 128 rows in four waves, gated: 2 x 2,816 features, 192 rows 15.7 and 19.2, 512 22.0 and 25.3; 2 x 5,632,
-// 256 rows 23.1 and 26.0, 384 28.5 and 31.6; 2 x 1,408, 1,024 rows 20.8 and 24.5.
+// other at a barrier per k tile leave even that unused (64 x 128 in four waves 18 us at K 2,048, so 12.5). A stage is
+// therefore one, two or four k tiles, the more the lower the tile, with one barrier for all of them, and all eight waves share
+// each. Stages lie in a ring, all of it asked for ahead: when a wave passes the barrier of stage s, stage s + 1 has landed for
+// every wave and every wave holds the last fragments of stage s in registers, so its place takes stage s + NB. The fragments
+// of a half k tile are read while those of the half before are multiplied.
+// Against the library's product, us, with weights that come from HBM (host time 9 us a call against 24), K 2,048: 2,048
+// features, 256 rows 8.4 and 9.9, 512 10.1 and 11.5, 1,280 17.4 and 18.8, 2,048 19.9 and 22.5; 4,096, 160 rows 11.7 and 16.6, 768 20.5 and
+// 23.2, 1,531 27.9 and 30.7; 6,144, 256 rows 15.9 and 23.9, 512 22.0 and 24.6, 1,024 30.4 and 32.3; 1,024 features of K 1,024,
+// 512 rows 6.2 and 8.6; of K 2,816 10.0 and 12.0. (With groups in turn 512 rows of 2,048 features 12.0, 256 of 6,144 15.5.)
+// Against tiles of 64 and 128 rows in four waves, gated: 2 x 2,816 features, 192 rows 15.3 and 19.5, 512 21.9 and 25.1; 2 x 5,632,
+// 256 rows 23.5 and 26.2, 384 27.9 and 31.3; 2 x 1,408, 1,024 rows 20.8 and 23.9.
 // The reference sends these products to rocBLAS (src/ops/linear.hip:21-35).
 #include "gemm_tile.h"
 
@@ -32,16 +35,15 @@ template <int NL, int NB> __device__ __forceinline__ void mid_wait_stages(int n)
   else mid_wait<0>();
 }
 
-// TM x TN: the tile. WM x WN waves (over rows of W and of A) multiply a k tile of 64, G groups of them take k tiles in turn; a
-// stage is G k tiles, NB of them in LDS.
-template <int TM, int TN, int WM, int WN, int G, int NB, bool GATED, typename TC>
+// TM x TN: the tile, by WM x WN waves (over rows of W and of A). A stage is KT k tiles of 64, NB of them in LDS.
+template <int TM, int TN, int WM, int WN, int KT, int NB, bool GATED, typename TC>
 __global__ __launch_bounds__(512, 2) void gemm_mid_kernel(GemmArgs a, int m_tiles, int n_tiles) {
 #if defined(__HIP_DEVICE_COMPILE__)   // (the host pass does not know buffer resources)
-  static_assert(WM * WN * G == 8 && NB >= 2 && NB <= 4, "eight waves");
+  static_assert(WM * WN == 8 && NB >= 2 && NB <= 4, "eight waves");
   constexpr int FI = TN / WM / 16, FJ = TM / WN / 16;     // 16-row blocks of W and of A of a wave
   static_assert(!GATED || FI % 2 == 0, "a wave's blocks of W are gate rows, then their up rows");
   constexpr int ROW = 128;                                // bytes of a staged row: a k tile of 64
-  constexpr int X_BYTES = TM * ROW, SUB = (TM + TN) * ROW, STAGE = G * SUB;
+  constexpr int X_BYTES = TM * ROW, SUB = (TM + TN) * ROW, STAGE = KT * SUB;
   constexpr int PER_SUB = SUB / 1024, X_PIECES = X_BYTES / 1024;   // pieces of 1 KB, 8 rows: a wave's load
   constexpr int NL = STAGE / 1024 / 8;                    // loads of a wave and stage
   static_assert(STAGE / 1024 % 8 == 0, "whole loads");
@@ -49,7 +51,7 @@ __global__ __launch_bounds__(512, 2) void gemm_mid_kernel(GemmArgs a, int m_tile
   int bx, by;
   dense_tile(spread_over_xcds(blockIdx.x, m_tiles * n_tiles), m_tiles, n_tiles, bx, by);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int g = wave / (WM * WN), wi = wave % (WM * WN), wm = wi % WM, wn = wi / WM;
+  const int wm = wave % WM, wn = wave / WM;
   const int K = a.K, N = a.N;
   constexpr int OUT = GATED ? TN / 2 : TN;
   const int row0 = bx * TM, out0 = by * OUT, rows_here = min(TM, a.M - row0);
@@ -76,13 +78,13 @@ __global__ __launch_bounds__(512, 2) void gemm_mid_kernel(GemmArgs a, int m_tile
   const auto w_res = __builtin_amdgcn_make_buffer_rsrc((void*)W, 0, 0xffffffffu, 0x00020000);
   const auto up_res = __builtin_amdgcn_make_buffer_rsrc((void*)(W + (GATED ? (int64_t)N * K : 0)), 0, 0xffffffffu, 0x00020000);
   typedef __attribute__((address_space(3))) void* lptr;
-  const int nk = K / 64, stages = (nk + G - 1) / G;
+  const int nk = K / 64, stages = (nk + KT - 1) / KT;
   auto issue = [&](int s, int at) {
     unsigned char* buf = smem + at + wave * 1024;
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
       const int piece = 8 * i + wave, p = piece % PER_SUB;
-      const int k = min(s * G + piece / PER_SUB, nk - 1) * ROW;   // (a last stage that K does not fill: the last k tile again)
+      const int k = min(s * KT + piece / PER_SUB, nk - 1) * ROW;   // (a last stage that K does not fill: the last k tile again)
       if (p < X_PIECES)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(x_res, (lptr)(buf + i * 8192), 16, off[i], k, 0, 0);
       else if (GATED && (p - X_PIECES) * 8 % (TN / WM) >= TN / WM / 2)
@@ -98,10 +100,10 @@ __global__ __launch_bounds__(512, 2) void gemm_mid_kernel(GemmArgs a, int m_tile
 #pragma unroll
     for (int j = 0; j < FJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int lr = lane & 15, lk = lane >> 4, sw = (lr >> 1) & 7;
-  const int x_lane = g * SUB + (wn * (TM / WN) + lr) * ROW, w_lane = g * SUB + X_BYTES + (wm * (TN / WM) + lr) * ROW;
+  const int x_lane = (wn * (TM / WN) + lr) * ROW, w_lane = X_BYTES + (wm * (TN / WM) + lr) * ROW;
   const int chunk[2] = {16 * (lk ^ sw), 16 * ((4 + lk) ^ sw)};
   bf16x8 wf[2][FI], xf[2][FJ];
-  auto read = [&](int h, int at) {
+  auto read = [&](int h, int at) {   // half h of the k tile at `at`
     const unsigned char* p = smem + at + chunk[h];
 #pragma unroll
     for (int i = 0; i < FI; ++i) wf[h][i] = *(const bf16x8*)(p + w_lane + i * 16 * ROW);
@@ -121,9 +123,18 @@ __global__ __launch_bounds__(512, 2) void gemm_mid_kernel(GemmArgs a, int m_tile
   __builtin_amdgcn_s_barrier();
   read(0, 0);
   int at = 0, s = 0;
+  auto most_of_stage = [&]() {   // all but the last half k tile, whose fragments are in registers
+#pragma unroll
+    for (int u = 0; u < KT; ++u) {
+      read(1, at + u * SUB);
+      multiply(0);
+      if (u + 1 == KT) break;
+      read(0, at + (u + 1) * SUB);
+      multiply(1);
+    }
+  };
   for (; s + NB < stages; ++s) {
-    read(1, at);
-    multiply(0);
+    most_of_stage();
     mid_wait<(NB - 2) * NL>();
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
@@ -133,8 +144,7 @@ __global__ __launch_bounds__(512, 2) void gemm_mid_kernel(GemmArgs a, int m_tile
     at = next(at);
   }
   for (; s + 1 < stages; ++s) {   // nothing left to ask for
-    read(1, at);
-    multiply(0);
+    most_of_stage();
     mid_wait_stages<NL, NB>(stages - s - 2);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
@@ -142,53 +152,31 @@ __global__ __launch_bounds__(512, 2) void gemm_mid_kernel(GemmArgs a, int m_tile
     multiply(1);
     at = next(at);
   }
-  if (s * G + g < nk) {   // (a group may have no k tile in the last stage)
-    read(1, at);
+#pragma unroll
+  for (int u = 0; u < KT; ++u) {
+    if (s * KT + u >= nk) break;   // (a last stage that K does not fill)
+    if (u) read(0, at + u * SUB);
+    read(1, at + u * SUB);
     multiply(0);
     multiply(1);
   }
-  __syncthreads();   // every wave has read its last fragments: the ring becomes the sums' and the epilogue's place
-  if constexpr (G > 1) {   // the first group adds the others' sums in their order
-    constexpr int SUMS = FI * FJ * 1024;   // bytes of a wave
-    static_assert((G - 1) * WM * WN * SUMS <= NB * STAGE, "the sums fit the ring");
-    if (g > 0) {
-      f32x4* d = (f32x4*)(smem + ((g - 1) * WM * WN + wi) * SUMS) + lane;
-#pragma unroll
-      for (int i = 0; i < FI; ++i)
-#pragma unroll
-        for (int j = 0; j < FJ; ++j) d[(i * FJ + j) * 64] = acc[i][j];
-    }
-    __syncthreads();
-    if (g == 0) {
-#pragma unroll
-      for (int o = 0; o < G - 1; ++o) {
-        const f32x4* d = (const f32x4*)(smem + (o * WM * WN + wi) * SUMS) + lane;
-#pragma unroll
-        for (int i = 0; i < FI; ++i)
-#pragma unroll
-          for (int j = 0; j < FJ; ++j) acc[i][j] += d[(i * FJ + j) * 64];
-      }
-    }
-    __syncthreads();   // the sums are read: the epilogue stages its rows in their place
-    if (g > 0) return;
-  }
+  __syncthreads();   // every wave has read its last fragments: the ring becomes the epilogue's place
   static_assert(WM * WN * FJ * 16 * FI * 32 <= NB * STAGE, "the epilogue's stage fits the ring");
   auto row_of = [&](int l) { return l; };
   const int tok0 = wn * (TM / WN), feat0 = out0 + wm * (OUT / WM);
   if constexpr (FI % 3 == 0)   // (rows of the epilogue's stage are powers of two)
     write_accumulators<FI, FJ, GATED, TC>(a, acc, tok0, row0, rows_here, feat0, row_of);
   else
-    write_tile<FI, FJ, GATED, TC>(a, acc, smem + wi * (FJ * 16 * FI * 32), tok0, row0, rows_here, feat0, row_of);
+    write_tile<FI, FJ, GATED, TC>(a, acc, smem + wave * (FJ * 16 * FI * 32), tok0, row0, rows_here, feat0, row_of);
 #endif
 }
 
-// The tiles, and what one round of each takes: us = start + K * per_k, measured over 96 to 2,048 rows of 1,024 to 8,192 features and K
-// 1,024 to 5,632. A second round costs 0.8 of the first and more, with which no tile beats the taller ones or the
-// library's: products of more than a round of the largest tile are not taken.
-struct MidTile { int rows, w_rows; bool gated; float start, per_k; };
-static const MidTile kMidTiles[] = {{32, 64, true, 2.5f, 0.0034f},   {64, 64, true, 2.5f, 0.0045f},   {96, 64, true, 3.f, 0.0049f},
-                                    {64, 96, false, 3.f, 0.0054f},   {128, 64, true, 3.f, 0.0063f},   {192, 64, true, 3.f, 0.0078f},
-                                    {128, 128, true, 3.f, 0.0091f},  {192, 128, true, 4.5f, 0.0100f}, {128, 192, false, 4.f, 0.0110f}};
+// The tiles in the order of what a round of each takes (K 1,024 and 4,096, us: 6.2 and 15.4, 7.0 and 19.8, 8.5 and 23.0, 8.0 and
+// 23.6, 9.2 and 28, 10.7 and 34, 11.9 and 36, 14.2 and 45, 15.2 and 46). A second round costs 0.8 of the first and more, with which no tile
+// beats the taller ones or the library's: products of more than a round of the largest tile are not taken.
+struct MidTile { int rows, w_rows; bool gated; };
+static const MidTile kMidTiles[] = {{32, 64, false}, {64, 64, true},   {96, 64, false},  {64, 96, false}, {128, 64, true},
+                                    {192, 64, true}, {128, 128, true}, {192, 128, true}, {128, 192, false}};
 constexpr int kMidTileCount = sizeof(kMidTiles) / sizeof(kMidTiles[0]);
 
 static int mid_tiles(const GemmArgs& a, const MidTile& t) {
@@ -196,15 +184,9 @@ static int mid_tiles(const GemmArgs& a, const MidTile& t) {
   return (int)min((int64_t)(1 << 30), (int64_t)((a.M + t.rows - 1) / t.rows) * ((w_rows + t.w_rows - 1) / t.w_rows));
 }
 static int mid_tile(const GemmArgs& a) {
-  int best = -1;
-  float least = 0.f;
-  for (int i = 0; i < kMidTileCount; ++i) {
-    const MidTile& t = kMidTiles[i];
-    if ((epilogue_gated(a.epilogue) && !t.gated) || mid_tiles(a, t) > device_cu_count()) continue;
-    const float us = t.start + a.K * t.per_k;
-    if (best < 0 || us < least) best = i, least = us;
-  }
-  return best;
+  for (int i = 0; i < kMidTileCount; ++i)
+    if ((!epilogue_gated(a.epilogue) || kMidTiles[i].gated) && mid_tiles(a, kMidTiles[i]) <= device_cu_count()) return i;
+  return -1;
 }
 
 // Dense products of more than 32 rows that are one round of tiles. (Fewer rows go to the few-row kernel.)
@@ -215,9 +197,9 @@ bool gemm_mid_takes(const GemmArgs& a) {
   return mid_tile(a) >= 0;
 }
 
-template <int TM, int TN, int WM, int WN, int G, int NB>
+template <int TM, int TN, int WM, int WN, int KT, int NB>
 static int launch_mid(const GemmArgs& a, hipStream_t stream) {
-  constexpr int LDS = G * (TM + TN) * 128 * NB;
+  constexpr int LDS = KT * (TM + TN) * 128 * NB;
   const bool gated = epilogue_gated(a.epilogue);
   const int w_rows = gated ? 2 * a.N : a.N, m_tiles = (a.M + TM - 1) / TM, n_tiles = (w_rows + TN - 1) / TN;
   auto launch = [&](auto kernel) {
@@ -230,13 +212,13 @@ static int launch_mid(const GemmArgs& a, hipStream_t stream) {
   const bool f32 = a.out_dtype == kF32;
   if constexpr (TN / WM / 16 % 2 == 0) {
     if (gated) {
-      rc = f32 ? launch(gemm_mid_kernel<TM, TN, WM, WN, G, NB, true, float>) : launch(gemm_mid_kernel<TM, TN, WM, WN, G, NB, true, bf16>);
+      rc = f32 ? launch(gemm_mid_kernel<TM, TN, WM, WN, KT, NB, true, float>) : launch(gemm_mid_kernel<TM, TN, WM, WN, KT, NB, true, bf16>);
       if (rc) return rc;
       NINFER_LAUNCH_CHECK();
       return 0;
     }
   }
-  rc = f32 ? launch(gemm_mid_kernel<TM, TN, WM, WN, G, NB, false, float>) : launch(gemm_mid_kernel<TM, TN, WM, WN, G, NB, false, bf16>);
+  rc = f32 ? launch(gemm_mid_kernel<TM, TN, WM, WN, KT, NB, false, float>) : launch(gemm_mid_kernel<TM, TN, WM, WN, KT, NB, false, bf16>);
   if (rc) return rc;
   NINFER_LAUNCH_CHECK();
   return 0;
@@ -245,11 +227,11 @@ static int launch_mid(const GemmArgs& a, hipStream_t stream) {
 int gemm_mid(const GemmArgs& a, hipStream_t stream) {
   NINFER_REQUIRE(gemm_mid_takes(a), "gemm: not a product of one round of tiles");
   switch (mid_tile(a)) {
-    case 0: return launch_mid<32, 64, 2, 1, 4, 3>(a, stream);
-    case 1: return launch_mid<64, 64, 2, 2, 2, 4>(a, stream);
-    case 2: return launch_mid<96, 64, 2, 2, 2, 3>(a, stream);
-    case 3: return launch_mid<64, 96, 2, 2, 2, 3>(a, stream);
-    case 4: return launch_mid<128, 64, 2, 2, 2, 3>(a, stream);
+    case 0: return launch_mid<32, 64, 4, 2, 4, 3>(a, stream);
+    case 1: return launch_mid<64, 64, 2, 4, 2, 4>(a, stream);
+    case 2: return launch_mid<96, 64, 4, 2, 2, 3>(a, stream);
+    case 3: return launch_mid<64, 96, 2, 4, 2, 3>(a, stream);
+    case 4: return launch_mid<128, 64, 2, 4, 2, 3>(a, stream);
     case 5: return launch_mid<192, 64, 2, 4, 1, 4>(a, stream);
     case 6: return launch_mid<128, 128, 2, 4, 1, 4>(a, stream);
     case 7: return launch_mid<192, 128, 2, 4, 1, 3>(a, stream);

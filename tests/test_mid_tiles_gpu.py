@@ -110,3 +110,33 @@ def test_one_call_runs_what_the_questions_one_by_one_would(m, n, k, taken):
     assert not taken or torch.equal(one, each)
     with pytest.raises(Exception, match="lda"):
         ops._gemm_cut_or_mid(x[:, :64].contiguous(), w, one, m=m, n=n, k=k, cut=True)
+
+
+# Each tile at a K whose stages go round its ring and whose last stage K does not fill.
+LONG = [(70, 2040, 1600, 32064), (700, 1400, 832, 64064), (760, 2040, 832, 96064), (640, 2400, 832, 64096), (1000, 2040, 832, 128064),
+        (1500, 2040, 576, 192064), (1100, 3500, 576, 128128), (1500, 4000, 448, 192128), (1020, 6100, 448, 128192)]
+LONG_GATED = [(70, 2040, 1600, 64064), (1000, 2040, 832, 128064), (1500, 2040, 576, 192064), (1100, 3500, 576, 128128), (1500, 4000, 448, 192128)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k,tile,gated", [(*c, False) for c in LONG] + [(*c, True) for c in LONG_GATED])
+def test_sums_are_one_chain_along_k(m, n, k, tile, gated):
+    """The bits of the taller tiles' sums (and of the library's, where it does not cut K): which kernel a size goes to does not show
+    in a model's logits."""
+    from ninfer_amd.kernels import load_ops
+    ops = load_ops()
+    inner = n // 2 if gated else n
+    args = _args(m, inner, k, epilogue=int(gated))
+    assert ops.lib.ninfer_gemm_mid_tile(ctypes.byref(args)) == tile and ops.lib.ninfer_gemm_kernel(ctypes.byref(args)) == 4
+    g = torch.Generator("cuda").manual_seed(m)
+    x, w = (torch.randn(r, k, generator=g, device="cuda").bfloat16() for r in (m, n))
+    got, tall, low = (torch.empty(m, inner, device="cuda", dtype=torch.bfloat16) for _ in range(3))
+    for out, force in ((got, 0), (low, 2), (tall, 3)):
+        with ops.tuned(force_kernel=force, split_min_bytes=1 << 40):
+            ops._gemm(x, w, out, m=m, n=inner, k=k, epilogue=int(gated))
+    assert torch.equal(got, low) and torch.equal(got, tall)
+    if not gated:
+        want = x.double() @ w.double().T
+        # products exact, k of them added in 32 bits, rounded to bfloat16
+        bound = k * 2.0 ** -23 * (x.double().abs() @ w.double().abs().T)
+        assert ((got.double() - want).abs() <= bound + 2.0 ** -8 * (want.abs() + bound)).all()
