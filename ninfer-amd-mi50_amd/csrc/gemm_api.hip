@@ -59,19 +59,22 @@ extern "C" int ninfer_gemm_split_parts(const GemmArgs* args) {
   return gemm_split_parts(*args);
 }
 
+// Is a plain dense product, which the caller's library would have otherwise, one round of gemm_mid's tiles? Not where ninfer_gemm
+// runs another kernel: products that blocks of 32 rows take by their size, but more slowly than the library, are not asked of them by
+// the caller (us here and there: 80 rows of 4,096 features, K 5,632, 23.1 and 19.5, 112 rows 24.2 and 21.3; 129 features of K
+// 8,192, 512 rows 13.3 and 11.6), and up to 128 features go to the few-row kernels.
+static bool plain_mid(const GemmArgs& a) { return gemm_mid_takes(a) && gemm_kernel(a) == kGemmTile; }
+extern "C" int ninfer_gemm_plain_mid(const GemmArgs* args) { return !gemm_check(*args) && plain_mid(*args); }
+
 // A plain dense product, if the kernels here cut it along K (with a workspace) or run it in one round of tiles: 1, or 0: the
 // caller's library has it.
 extern "C" int ninfer_gemm_cut_or_mid(const GemmArgs* args, hipStream_t stream) {
   const GemmArgs& a = *args;
   int rc = gemm_check(a);
   if (rc) return rc < 0 ? rc : -rc;
-  if (gemm_split_parts(a) >= 2) {
-    rc = gemm_split(a, stream);
-  } else {
-    if (!gemm_mid_takes(a)) return 0;
-    const GemmKernel kernel = gemm_kernel(a);   // (which need not be that of the tiles)
-    rc = kernel == kGemmTile ? gemm_mid(a, stream) : ninfer_gemm(args, 0, stream);
-  }
+  if (gemm_split_parts(a) >= 2) rc = gemm_split(a, stream);
+  else if (plain_mid(a)) rc = gemm_mid(a, stream);
+  else return 0;
   return rc == 0 ? 1 : rc < 0 ? rc : -rc;
 }
 

@@ -241,7 +241,8 @@ int gemm_mid(const GemmArgs& a, hipStream_t stream) {
 
 }  // namespace ninfer
 
-// The tile of a product that ninfer_gemm runs in one round: 1,000 x its rows of A + its rows of W (0: it does not).
+// The tile in which gemm_mid runs a product: 1,000 x its rows of A + its rows of W (0: it does not take it). Whether ninfer_gemm asks
+// gemm_mid for it is ninfer_gemm_kernel's to say.
 extern "C" int ninfer_gemm_mid_tile(const ninfer::GemmArgs* args) {
   if (!ninfer::gemm_mid_takes(*args)) return 0;
   const ninfer::MidTile& t = ninfer::kMidTiles[ninfer::mid_tile(*args)];

@@ -739,7 +739,7 @@ class HipOps:
             self._ok(self.lib.ninfer_gemm(ctypes.byref(args), 0, self._stream()))
             return True
         args = self._gemm_args(a, w, c, n, k, m, **more)
-        if only_if_mid and not self.lib.ninfer_gemm_mid_tile(ctypes.byref(args)):
+        if only_if_mid and not self.lib.ninfer_gemm_plain_mid(ctypes.byref(args)):
             return False
         if self._held is not None:
             self._held.append((args, (a, w, c, more)))

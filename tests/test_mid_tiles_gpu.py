@@ -112,6 +112,32 @@ def test_one_call_runs_what_the_questions_one_by_one_would(m, n, k, taken):
         ops._gemm_cut_or_mid(x[:, :64].contiguous(), w, one, m=m, n=n, k=k, cut=True)
 
 
+# Plain products that blocks of 32 rows or the few-row kernels would take, more slowly than the library (the last two: they are not
+# taken by size either way).
+NOT_OURS = [(80, 4096, 5632), (112, 4096, 5632), (112, 3072, 5632), (100, 4096, 4096), (64, 512, 5632), (512, 129, 8192),
+            (2048, 64, 2048), (700, 128, 704), (4096, 8192, 512), (512, 2048, 2080)]
+
+
+@pytest.mark.parametrize("m,n,k,ours", [(*s, 0) for s in NOT_OURS] + [(96, 8192, 2048, 1), (513, 2048, 1024, 1), (700, 129, 704, 1)])
+def test_which_plain_products_leave_the_library(m, n, k, ours):
+    from ninfer_amd.kernels.build import ensure_built
+    lib = ctypes.CDLL(ensure_built())
+    assert lib.ninfer_gemm_plain_mid(ctypes.byref(_args(m, n, k))) == ours
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", NOT_OURS)
+def test_what_the_library_runs_faster_stays_with_it(monkeypatch, m, n, k):
+    from ninfer_amd.kernels import load_ops
+    ops = load_ops()
+    g = torch.Generator("cuda").manual_seed(m)
+    x, w = (torch.randn(r, k, generator=g, device="cuda").bfloat16() for r in (m, n))
+    out, calls, matmul = torch.empty(m, n, device="cuda", dtype=torch.bfloat16), [], torch.matmul
+    monkeypatch.setattr(torch, "matmul", lambda *a, **b: (calls.append(1), matmul(*a, **b)))
+    ops.linear(x, w, out)
+    assert calls and torch.equal(out, matmul(x, w.t()))
+
+
 # Each tile at a K whose stages go round its ring and whose last stage K does not fill.
 LONG = [(70, 2040, 1600, 32064), (700, 1400, 832, 64064), (760, 2040, 832, 96064), (640, 2400, 832, 64096), (1000, 2040, 832, 128064),
         (1500, 2040, 576, 192064), (1100, 3500, 576, 128128), (1500, 4000, 448, 192128), (1020, 6100, 448, 128192)]
