@@ -167,6 +167,7 @@ bool gemm_tile_takes(const GemmArgs& a);
 int gemm_tile_row_tiles(const GemmArgs& a, int rows);   // block rows of a launch in tiles of 64, 128 or 256 rows
 int gemm_tile(const GemmArgs& a, hipStream_t stream);
 bool gemm_mid_takes(const GemmArgs& a);   // (asked by gemm_tile)
+bool gemm_mid_beats_library(const GemmArgs& a);
 int gemm_mid(const GemmArgs& a, hipStream_t stream);
 int gemm_generic(const GemmArgs& a, hipStream_t stream);
 bool gemm_f32_takes(const GemmArgs& a);

@@ -62,8 +62,10 @@ extern "C" int ninfer_gemm_split_parts(const GemmArgs* args) {
 // Is a plain dense product, which the caller's library would have otherwise, one round of gemm_mid's tiles? Not where ninfer_gemm
 // runs another kernel: products that blocks of 32 rows take by their size, but more slowly than the library, are not asked of them by
 // the caller (us here and there: 80 rows of 4,096 features, K 5,632, 23.1 and 19.5, 112 rows 24.2 and 21.3; 129 features of K
-// 8,192, 512 rows 13.3 and 11.6), and up to 128 features go to the few-row kernels.
-static bool plain_mid(const GemmArgs& a) { return gemm_mid_takes(a) && gemm_kernel(a) == kGemmTile; }
+// 8,192, 512 rows 13.3 and 11.6), and up to 128 features go to the few-row kernels. Nor where the library is the faster one.
+static bool plain_mid(const GemmArgs& a) {
+  return gemm_mid_takes(a) && gemm_kernel(a) == kGemmTile && gemm_mid_beats_library(a);
+}
 extern "C" int ninfer_gemm_plain_mid(const GemmArgs* args) { return !gemm_check(*args) && plain_mid(*args); }
 
 // A plain dense product, if the kernels here cut it along K (with a workspace) or run it in one round of tiles: 1, or 0: the
