@@ -69,9 +69,10 @@ static bool plain_mid(const GemmArgs& a) {
 extern "C" int ninfer_gemm_plain_mid(const GemmArgs* args) { return !gemm_check(*args) && plain_mid(*args); }
 
 // A plain dense product, if the kernels here cut it along K (with a workspace) or run it in one round of tiles: 1, or 0: the
-// caller's library has it.
+// caller's library has it (a product without features or over nothing too, which the kernels here refuse).
 extern "C" int ninfer_gemm_cut_or_mid(const GemmArgs* args, hipStream_t stream) {
   const GemmArgs& a = *args;
+  if (a.N == 0 || a.K == 0) return 0;
   int rc = gemm_check(a);
   if (rc) return rc < 0 ? rc : -rc;
   if (gemm_split_parts(a) >= 2) rc = gemm_split(a, stream);

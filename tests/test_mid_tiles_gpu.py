@@ -141,6 +141,23 @@ def test_what_the_library_runs_faster_stays_with_it(monkeypatch, m, n, k):
     assert calls and torch.equal(out, matmul(x, w.t()))
 
 
+@pytest.mark.parametrize("n,k", [(0, 256), (256, 0), (0, 0)])
+def test_products_of_nothing_are_the_librarys(n, k):
+    from ninfer_amd.kernels.build import ensure_built
+    lib = ctypes.CDLL(ensure_built())
+    assert lib.ninfer_gemm_cut_or_mid(ctypes.byref(_args(600, n, k)), None) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,k", [(0, 256), (256, 0), (0, 0)])
+def test_linear_over_nothing(n, k):
+    from ninfer_amd.kernels import load_ops
+    x, w = (torch.ones(r, k, device="cuda", dtype=torch.bfloat16) for r in (600, n))
+    out = torch.full((600, n), 7.0, device="cuda", dtype=torch.bfloat16)
+    load_ops().linear(x, w, out)
+    assert (out == 0).all()
+
+
 # Each tile at a K whose stages go round its ring and whose last stage K does not fill.
 LONG = [(70, 2040, 1600, 32064), (700, 1400, 832, 64064), (760, 2040, 832, 96064), (640, 2400, 832, 64096), (1000, 2040, 832, 128064),
         (1500, 2040, 576, 192064), (1100, 3500, 576, 128128), (1500, 4000, 448, 192128), (1020, 6100, 448, 128192)]
