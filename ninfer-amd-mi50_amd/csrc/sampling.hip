@@ -235,6 +235,7 @@ __device__ __forceinline__ void sample_whole_row(const SampleArgs& a, int r, Row
       best_i = ired[i];
     }
   }
+  if (best_i == 0x7fffffff) best_i = 0;   // (nothing above -infinity: the first token, as where few tokens are kept)
   if (!(temp > 0.f)) {
     if (tid == 0) out[r] = best_i;
     return;
@@ -327,6 +328,11 @@ __device__ __forceinline__ void sample_whole_row(const SampleArgs& a, int r, Row
       if (need < quota) quota = need;
     }
     total = mass_gt + quota * mass_thr;
+  }
+
+  if (total == 0) {   // no token has mass (+infinity is the largest logit, or -infinity, or all are NaN): the largest
+    if (tid == 0) out[r] = best_i;
+    return;
   }
 
   // Inverse CDF over the kept tokens in index order, in two steps. First every wave sums a run of
@@ -897,6 +903,7 @@ __device__ __forceinline__ bool draw_few(const SampleArgs& a, const SampleScratc
   }
   incl = wave_sums(sum);
   total = __shfl(incl, 63, 64);
+  if (total == 0 && lane == 0) a.out[r] = l.token_at[l.place_of[0]];   // (all that is kept is -infinity)
   u64 goal = (u64)((double)a.uniform[r] * (double)total);
   if (goal >= total) goal = total - 1;
   run = incl - sum;
@@ -926,6 +933,7 @@ __device__ __forceinline__ bool draw_wide(const SampleArgs& a, const SampleScrat
   // Kept are the tokens above key `thr` and of those with it the first `quota` in index order.
   uint32_t thr = 0;
   u64 total = l.cut.total, quota = ~0ull, mass_thr = 0;
+  if (total == 0) return false;
   auto mass_of = [&](uint32_t key) { return token_mass(key_value(key), m); };
   if (l.cut.bin < kBins) {
     thr = radix_select(n, l.cut.target - l.cut.above, l.hist, [&](int i) { return l.list[i].x; },

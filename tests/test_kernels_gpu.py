@@ -1292,6 +1292,23 @@ def test_sample_rows_by_the_whole_gpu(ops, gen, v):
         assert torch.equal(*got), f"u={u}: {got[0].tolist()} vs {got[1].tolist()}"
 
 
+@pytest.mark.parametrize("v", [3, 300, 5000, 40000])
+@pytest.mark.parametrize("path", [{}, {"few": True}, {"spread": True}])
+def test_sample_rows_without_mass(ops, v, path):
+    """Rows of -inf, of NaN of either sign, and with +inf among numbers: a token of the row, the same by every path (the first one, or
+    that of +inf), greedy and drawn, whatever `out` held."""
+    logits = torch.full((12, v), -float("inf"), device="cuda")
+    logits[1::4] = float("nan")
+    logits[2::4] = torch.tensor(-0x400000, dtype=torch.int32, device="cuda").view(torch.float32)
+    logits[3::4] = torch.linspace(-4, 4, v, device="cuda")
+    logits[3::4, v // 2] = float("inf")
+    i32, f32 = (lambda x, d=d: torch.tensor(x, device="cuda", dtype=d) for d in (torch.int32, torch.float32))
+    temp, top_k, top_p = f32([0.0] * 4 + [0.8] * 8), i32([0] * 4 + [40] * 4 + [0 if "few" not in path else 7] * 4), f32([0.9] * 12)
+    out = torch.full((12,), -7, device="cuda", dtype=torch.int32)
+    ops.sample(logits, temp, torch.full((12,), 0.4, device="cuda"), out, top_k=top_k, top_p=top_p, **path)
+    assert out.tolist() == [0, 0, 0, v // 2] * 3
+
+
 @pytest.mark.parametrize("top_p", [1.0, 0.999])
 def test_few_tokens_path_has_the_masses_of_the_whole_row(ops, gen, top_p):
     """Numbers drawn right at the border between two kept tokens, one of them at the threshold: both paths
