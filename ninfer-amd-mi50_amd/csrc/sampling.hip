@@ -479,7 +479,10 @@ __device__ __forceinline__ float key_value(uint32_t key) {   // ordered_key's in
 // Above this key, that of the largest finite number, lie +infinity and NaN.
 constexpr uint32_t kFiniteKey = 0xff7fffffu;
 
-__device__ __forceinline__ int mass_bin(float scaled, float m) {   // the same or more for every smaller logit
+// The same or more for every smaller scaled logit, and the same for equal ones: `scaled` is a product, which must not go
+// unrounded into the difference (token_mass).
+__device__ __forceinline__ int mass_bin(float scaled, float m) {
+#pragma clang fp contract(off)
   return min(kBins - 1, (int)((m - scaled) * kBinsPerUnit));
 }
 

@@ -1292,6 +1292,56 @@ def test_sample_rows_by_the_whole_gpu(ops, gen, v):
         assert torch.equal(*got), f"u={u}: {got[0].tolist()} vs {got[1].tolist()}"
 
 
+def _pairs_at_a_bin_edge(inv_t, count):
+    """(largest logit, a, b) in float32: a and b differ, are the same once scaled, and the distance of that from the largest
+    scaled logit is a whole number of sixteenths to the last bit, while the unrounded products lie on its two sides."""
+    import numpy as np
+    rng, found = np.random.RandomState(4), []
+    inv_t = np.float32(inv_t)
+    while len(found) < count:
+        top = np.float32(rng.uniform(9, 10))
+        m = top * inv_t
+        for n in range(16, 64):
+            s = np.float32(m - np.float32(n / 16))
+            if np.float32(m - s) != np.float32(n / 16):
+                continue
+            x = np.float32(s / inv_t)
+            near = [x]
+            for to in (-np.inf, np.inf):
+                y = x
+                for _ in range(3):
+                    y = np.nextafter(y, np.float32(to))
+                    near.append(y)
+            same = sorted(float(y) for y in near if y * inv_t == s)
+            exact = [y * float(inv_t) for y in same]
+            if len(same) > 1 and exact[0] < float(s) < exact[-1]:
+                found.append((float(top), same[0], same[-1]))
+    return found[:count]
+
+
+def test_ties_after_scaling_stay_together(ops, gen):
+    """Logits that differ but are the same once scaled, at a whole number of sixteenths from the largest: they have one mass and one rank by
+    index, whichever way the distance is computed."""
+    v, temp = 20000, 0.7
+    inv_t = float(torch.tensor(1.0) / torch.tensor(temp))
+    pairs = _pairs_at_a_bin_edge(inv_t, 24)
+    logits = torch.full((len(pairs), v), -40.0, device="cuda")
+    for i, (top, a, b) in enumerate(pairs):
+        logits[i, 5 + 7 * i] = top
+        logits[i, 1000:3000:2] = a
+        logits[i, 1001:3001:2] = b
+    r = len(pairs)
+    same = lambda x, d=torch.float32: torch.full((r,), x, device="cuda", dtype=d)
+    for p in (0.3, 0.5, 0.8, 0.99):
+        for u in (0.0, 0.02, 0.3, 0.5, 0.9, 0.9999):
+            got = []
+            for spread in (False, True):
+                out = same(-7, torch.int32)
+                ops.sample(logits, same(temp), same(u), out, top_k=same(0, torch.int32), top_p=same(p), spread=spread)
+                got.append(out)
+            assert torch.equal(*got), f"p={p} u={u}: {got[0].tolist()} vs {got[1].tolist()}"
+
+
 @pytest.mark.parametrize("v", [3, 300, 5000, 40000])
 @pytest.mark.parametrize("path", [{}, {"few": True}, {"spread": True}])
 def test_sample_rows_without_mass(ops, v, path):
