@@ -439,7 +439,8 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(SampleArgs a) {
 // the token in it. 64 rows of 151,936 tokens at top-p 0.95 73 to 84 us, by sample_whole_row 320; one row 30 and
 // 267; 32,000 tokens, one row, 30 and 74, with top-p 1 23 and 33; 6,000 tokens the same in both.
 //
-// Rows that fit neither, lists that do not fit (many equal logits) and rows with NaN or +infinity go through sample_whole_row.
+// Rows that fit neither, lists that do not fit (many equal logits; 151,936 normal ones of a deviation below some 0.2 once scaled)
+// and rows with NaN or +infinity go through sample_whole_row: 64 that are too flat 420 us, 389 without the launches in front.
 constexpr int kSlice = 4096;
 constexpr int kSliceThreads = 256;
 constexpr int kPerThread = kSlice / kSliceThreads;   // tokens of a subgroup: tid + kSliceThreads * u
@@ -447,8 +448,7 @@ constexpr int kFewTokens = 256;
 constexpr int kSubs = 512;          // subgroups that a row's block reads again
 constexpr int kSubTable = 2048;     // places to look one of them up
 constexpr int kFewList = 1024;      // tokens that reach the bound
-constexpr int kBins = 512;          // of 1/16 in scaled logits: beyond 23 tokens have no mass
-constexpr float kBinsPerUnit = 16.f;
+constexpr int kBins = 512;          // (450 that tokens fall into: beyond a distance of 22.2 they have no mass)
 constexpr int kCutList = 4096;      // tokens of the bin that top-p cuts
 constexpr int kMaxSlices = 1024;    // of a row whose draw may keep all
 
@@ -480,10 +480,13 @@ __device__ __forceinline__ float key_value(uint32_t key) {   // ordered_key's in
 constexpr uint32_t kFiniteKey = 0xff7fffffu;
 
 // The same or more for every smaller scaled logit, and the same for equal ones: `scaled` is a product, which must not go
-// unrounded into the difference (token_mass).
+// unrounded into the difference (token_mass). 128 bins for each doubling of the distance + 2 (its float's upper bits): 64 to a
+// unit up to 2, 32 up to 6, 16 up to 14, 8 beyond, as the flatter a row, the nearer to its largest logit, and the more crowded, is
+// where top-p cuts it. With 16 to a unit everywhere the cut's bin of 151,936 normal logits of deviation 0.6 (top-p 0.8) held 4,400
+// tokens, more than the list: 64 such rows 420 us, 124 so.
 __device__ __forceinline__ int mass_bin(float scaled, float m) {
 #pragma clang fp contract(off)
-  return min(kBins - 1, (int)((m - scaled) * kBinsPerUnit));
+  return min(kBins - 1, (int)((__float_as_uint(m - scaled + 2.f) - __float_as_uint(2.f)) >> 16));
 }
 
 // Wave-wide inclusive sums.

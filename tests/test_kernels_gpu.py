@@ -1292,6 +1292,22 @@ def test_sample_rows_by_the_whole_gpu(ops, gen, v):
         assert torch.equal(*got), f"u={u}: {got[0].tolist()} vs {got[1].tolist()}"
 
 
+@pytest.mark.parametrize("temp", [0.05, 3.0, 5.0, 10.0, 40.0])
+def test_sample_flat_and_peaked_rows(ops, gen, temp):
+    """Rows that top-p cuts far from or near the largest logit, where many tokens lie close together or one has all the mass."""
+    r, v = 4, 151936
+    logits = torch.randn(r, v, generator=gen, device="cuda") * 3
+    same = lambda x, d=torch.float32: torch.full((r,), x, device="cuda", dtype=d)
+    for p in (0.05, 0.5, 0.8, 0.95, 0.9999):
+        for u in (0.0, 0.3, 0.77, 0.99999):
+            got = []
+            for spread in (False, True):
+                out = same(-7, torch.int32)
+                ops.sample(logits, same(temp), same(u), out, top_k=same(0, torch.int32), top_p=same(p), spread=spread)
+                got.append(out)
+            assert torch.equal(*got), f"p={p} u={u}: {got[0].tolist()} vs {got[1].tolist()}"
+
+
 def _pairs_at_a_bin_edge(inv_t, count):
     """(largest logit, a, b) in float32: a and b differ, are the same once scaled, and the distance of that from the largest
     scaled logit is a whole number of sixteenths to the last bit, while the unrounded products lie on its two sides."""
