@@ -367,6 +367,9 @@ class HipOps:
         self.lib.ninfer_last_error.restype = ctypes.c_char_p
         if not (self.lib.ninfer_gemm_args_bytes() == ctypes.sizeof(_GemmArgs)):
             raise KernelError(f"{self.lib_path} and these bindings lay a product's arguments out differently")
+        if self.lib.ninfer_sample_few_tokens() != self.FEW_TOKENS:
+            raise KernelError(f"{self.lib_path} samples rows of up to {self.lib.ninfer_sample_few_tokens()} tokens by "
+                              f"the whole GPU, these bindings say {self.FEW_TOKENS}")
         self.lib.ninfer_attention_workspace_floats.restype = ctypes.c_longlong
         self.lib.ninfer_event_create.restype = ctypes.c_void_p
         self.lib.ninfer_stream_after.argtypes = [ctypes.c_void_p] * 3

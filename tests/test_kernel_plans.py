@@ -338,3 +338,11 @@ def test_which_short_steps_take_two_streams(sizes, size, rows, two):
     experts, inner, shared = sizes
     weights = 3 * 2048 * (experts * inner + shared) * size
     assert HipOps.pays_beside(SimpleNamespace(), rows, weights, torch.bfloat16 if size == 2 else torch.float32) == two
+
+
+def test_the_bindings_say_how_many_tokens_a_sampled_row_may_keep(lib, monkeypatch):
+    from ninfer_amd.kernels.ops import HipOps, KernelError
+    assert lib.ninfer_sample_few_tokens() == HipOps.FEW_TOKENS
+    monkeypatch.setattr(HipOps, "FEW_TOKENS", 64)
+    with pytest.raises(KernelError, match="whole GPU"):
+        HipOps()
