@@ -795,6 +795,12 @@ class HipOps:
             return False
         return not torch.cuda.is_current_stream_capturing()
 
+    def wants_beside_short(self, rows: int, weight_bytes: int, dtype) -> bool:
+        """`pays_beside`, as a step that `wants_beside` says no to asks it: not while a graph is being captured, and not where
+        `beside_min_rows` has been put out of reach, to have one stream (32 times the step's rows and more)."""
+        return (32 * rows >= self.beside_min_rows and self.pays_beside(rows, weight_bytes, dtype)
+                and not torch.cuda.is_current_stream_capturing())
+
     def pays_beside(self, rows: int, weight_bytes: int, dtype) -> bool:
         """Are a routed path and the independent work beside it (whose weights are so many bytes together) long enough on the
         device for two streams where `wants_beside` says no? The host needs some 205 us a layer with them and 170 without, and

@@ -340,6 +340,19 @@ def test_which_short_steps_take_two_streams(sizes, size, rows, two):
     assert HipOps.pays_beside(SimpleNamespace(), rows, weights, torch.bfloat16 if size == 2 else torch.float32) == two
 
 
+@pytest.mark.parametrize("min_rows,rows,capturing,two", [(512, 17, False, True), (512, 2048, False, True), (1 << 30, 2048, False, False),
+                                                         (1 << 30, 65, False, False), (512, 160, True, False), (1, 1, False, True)])
+def test_one_stream_when_it_is_asked_for(monkeypatch, min_rows, rows, capturing, two):
+    import torch
+    from types import SimpleNamespace
+    from ninfer_amd.kernels.ops import HipOps
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing)
+    ops = SimpleNamespace(beside_min_rows=min_rows, pays_beside=lambda *a: True)
+    assert HipOps.wants_beside_short(ops, rows, 1 << 40, torch.float32) == two
+    ops.pays_beside = lambda *a: False
+    assert not HipOps.wants_beside_short(ops, rows, 1 << 40, torch.float32)
+
+
 def test_the_bindings_say_how_many_tokens_a_sampled_row_may_keep(lib, monkeypatch):
     from ninfer_amd.kernels.ops import HipOps, KernelError
     assert lib.ninfer_sample_few_tokens() == HipOps.FEW_TOKENS

@@ -31,3 +31,20 @@ def test_short_steps_on_two_streams(tmp_path, dtype, rows):
     if dtype == "float32":
         assert torch.equal(got[True], got[False])
     torch.testing.assert_close(got[True], plain_model.forward(w, rcfg, toks), **bound(dtype))
+
+
+def test_one_stream_when_it_is_asked_for(tmp_path, monkeypatch):
+    """`beside_min_rows` out of reach is one stream, also where a step's weights are many."""
+    import ninfer_amd
+    from ninfer_amd import EngineOptions, load_model
+    ninfer_amd.write_random_model(str(tmp_path), CONFIG_WIDE, 77, dtype="bfloat16", std=0.06)
+    runner = load_model(str(tmp_path), EngineOptions(dtype="bfloat16", max_context=704, prefill_chunk=640, num_sequences=2, page_size=16))
+    ops, blocks = runner.ops, []
+    inner = ops.beside
+    monkeypatch.setattr(ops, "pays_beside", lambda rows, weight_bytes, dtype: True)
+    monkeypatch.setattr(ops, "beside", lambda: (blocks.append(1), inner())[1])
+    for min_rows, some in ((512, True), (1 << 30, False)):
+        monkeypatch.setattr(ops, "beside_min_rows", min_rows)
+        blocks.clear()
+        util.run_schedule(runner, util.schedule_whole(f"r{min_rows}", list(range(5, 205))))
+        assert bool(blocks) == some
