@@ -326,7 +326,8 @@ class ModelRunner:
             torch.cuda.synchronize()
             g = torch.cuda.CUDAGraph()
             capture = torch.cuda.graph(g)
-            self.ops.library_workspace(capture.capture_stream)
+            if self.ops.captures_library(shape["T"], self.act_dtype):
+                self.ops.library_workspace(capture.capture_stream)
             with capture:
                 entry["logits"] = self._forward(entry["meta"], shape)
             entry["graph"] = g

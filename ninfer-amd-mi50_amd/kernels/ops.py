@@ -325,7 +325,6 @@ class _Beside:
         ops = self.ops
         if ops._side is None:
             ops._side = torch.cuda.Stream()   # default priority
-            ops.library_workspace(ops._side)
             ops._side_events = (ops._new_event(), ops._new_event())
         raw = ops._stream().value or 0
         if ops._main is None or ops._main.cuda_stream != raw:
@@ -389,6 +388,7 @@ class HipOps:
         self._held_route = None     # ... and a routing by the logits one of them writes
         self._side = None           # the second stream of `beside()`, made at first use
         self._side_events = None    # (start, end) of the `beside()` block
+        self._side_library = False  # the library's workspace of the second stream is made
         self._side_inside = False   # inside a `beside()` block
         self._side_open = False     # a `beside()` block that `join()` has not waited for
         self._main = None           # the stream that the last `beside()` block left and returns to
@@ -761,11 +761,16 @@ class HipOps:
             self._ok(rc)
         return rc > 0
 
+    def captures_library(self, rows: int, dtype) -> bool:
+        """May a captured step of this many rows hold a product of the library's?"""
+        return dtype == torch.bfloat16 and rows > self.library_min_rows and not self.force_generic
+
     @staticmethod
     def library_workspace(stream) -> None:
         """The library's products keep a workspace per stream (76 MB) from their first call on it until the process ends. Made
-        here, before anything else of the stream, it has memory of its own; made later it may lie in a larger block
-        that a step has left, which then cannot go back to the device."""
+        here, before the first product that may be the library's (on the second stream) and before a capture that may hold one
+        (`captures_library`), it has memory of its own; made later it may lie in a larger block that a step has left,
+        which then cannot go back to the device. Streams that no such product runs on keep none."""
         with torch.cuda.stream(stream):
             t = torch.zeros(64, 64, dtype=torch.bfloat16, device="cuda")
             torch.matmul(t, t.t())
@@ -890,6 +895,9 @@ class HipOps:
         if act is None and bias is None and self._use_library(x, out, w) and not (
                 rows <= self.side_own_max_rows
                 and n * k * w.element_size() <= self.side_own_max_bytes and self._on_side()):
+            if self._side_inside and not self._side_library:
+                self.library_workspace(self._side)
+                self._side_library = True
             own = self._rows_kernel_takes(x, w)
             if not own or self._tune["split_min_bytes"]:
                 cut = rows <= self.split_max_rows

@@ -48,3 +48,26 @@ def test_one_stream_when_it_is_asked_for(tmp_path, monkeypatch):
         blocks.clear()
         util.run_schedule(runner, util.schedule_whole(f"r{min_rows}", list(range(5, 205))))
         assert bool(blocks) == some
+
+
+@pytest.mark.parametrize("dtype,batch,kept", [("float32", 40, False), ("bfloat16", 4, False), ("bfloat16", 40, True)])
+def test_streams_without_the_librarys_products_keep_no_workspace(tmp_path, monkeypatch, dtype, batch, kept):
+    """A graph of few rows or in 32-bit, and the second stream of a 32-bit engine, hold no product of the library's."""
+    import ninfer_amd
+    from ninfer_amd import Chunk, EngineOptions, load_model
+    ninfer_amd.write_random_model(str(tmp_path), CONFIG_WIDE, 78, dtype=dtype, std=0.06)
+    runner = load_model(str(tmp_path), EngineOptions(dtype=dtype, max_context=704, prefill_chunk=640, num_sequences=48, page_size=16,
+                                                   use_graph=True))
+    ops, streams = runner.ops, []
+    inner = ops.library_workspace
+    monkeypatch.setattr(ops, "library_workspace", lambda stream: (streams.append(stream), inner(stream)))
+    monkeypatch.setattr(ops, "_side_library", False)
+    monkeypatch.setattr(ops, "side_own_max_rows", 0)   # (the second stream's short products would stay out of the library)
+    monkeypatch.setattr(ops, "pays_beside", lambda rows, weight_bytes, dtype: True)
+    slots = [runner.open() for _ in range(batch)]
+    runner.step([Chunk(s, list(range(5)), []) for s in slots])   # rows on two streams
+    beside = len(streams)
+    for i in range(4):   # eager, captured, replayed
+        runner.step([Chunk(s, [7 + i], [0]) for s in slots])
+    assert runner._graphs and ops._side is not None
+    assert (beside > 0) == (dtype == "bfloat16" and 5 * batch > 32) and (len(streams) > beside) == kept
