@@ -1,5 +1,6 @@
 """Dense products that are one round of tiles, at the edges of every tile: rows and features that end inside a
-block, K of one k tile, of fewer than a stage's and of a last stage that K does not fill, every epilogue."""
+block, K of one k tile, of fewer than a stage's, of a last stage that K does not fill and of more stages than the ring holds, every
+epilogue; and which products come to them."""
 import ctypes
 
 import pytest
@@ -30,7 +31,7 @@ def test_which_tile(m, n, k, gated, tile):
 
 SHAPES = [(33, 8192, 64), (64, 2056, 192), (64, 16384, 320), (130, 2050, 64), (512, 2048, 2048), (700, 2047, 192), (760, 2048, 320),
           (250, 6100, 128), (129, 8190, 448), (900, 2304, 192), (1500, 2040, 64), (1140, 2900, 576), (1500, 4090, 128),
-          (1020, 6100, 256), (2048, 64, 704)]
+          (1020, 6100, 256), (2048, 136, 704)]
 EPILOGUES = ["none", "f32", "relu2", "bias", "gated", "gated bias"]
 CASES = [(*s, e) for s in SHAPES for e in EPILOGUES if not (e.startswith("gated") and s in SHAPES[-2:])]   # (not a round of gated tiles)
 
@@ -49,7 +50,8 @@ def test_products(m, n, k, epilogue):
     dtype = torch.float32 if epilogue == "f32" else torch.bfloat16
     whole = torch.full((m + 1, inner), 7.0, device="cuda", dtype=dtype)
     out = whole[:m]
-    assert ops.lib.ninfer_gemm_mid_tile(ctypes.byref(_args(m, inner, k, epilogue=int(gated))))
+    args = _args(m, inner, k, epilogue=int(gated))
+    assert ops.lib.ninfer_gemm_mid_tile(ctypes.byref(args)) and ops.lib.ninfer_gemm_kernel(ctypes.byref(args)) == 4
     with ops.tuned(split_min_bytes=1 << 40):   # (nothing is cut along K)
         if gated:
             w = w * 0.1
@@ -106,6 +108,10 @@ def test_one_call_runs_what_the_questions_one_by_one_would(m, n, k, taken):
     asked = m <= ops.split_max_rows and ops._gemm(x, w, each, m=m, n=n, k=k, only_if_split=True) or \
         ops._gemm(x, w, each, m=m, n=n, k=k, only_if_mid=True)
     assert asked == taken and torch.equal(one, each)
+    # products exact, k of them added in 32 bits in any order, rounded to bfloat16
+    want = x.double() @ w.double().T
+    bound = k * 2.0 ** -23 * (x.double().abs() @ w.double().abs().T)
+    assert not taken or ((one.double() - want).abs() <= bound + 2.0 ** -8 * (want.abs() + bound)).all()
     ops.linear(x, w, each)
     assert not taken or torch.equal(one, each)
     with pytest.raises(Exception, match="lda"):
