@@ -451,6 +451,7 @@ constexpr int kFewList = 1024;      // tokens that reach the bound
 constexpr int kBins = 512;          // (450 that tokens fall into: beyond a distance of 22.2 they have no mass)
 constexpr int kCutList = 4096;      // tokens of the bin that top-p cuts
 constexpr int kMaxSlices = 1024;    // of a row whose draw may keep all
+constexpr int kSpreadRows = 65535;  // a grid's second dimension
 
 struct SampleScratch {
   uint32_t* maxima;             // [R, slices * kSliceThreads]
@@ -1142,7 +1143,7 @@ static int sample_by_slices(const SampleArgs& a, int R, int wide, hipStream_t st
   int rc = sample_check(a, R);
   if (rc) return rc;
   NINFER_REQUIRE(scratch && (uintptr_t)scratch % 256 == 0, "sample: scratch is null or not aligned");
-  NINFER_REQUIRE(R <= 65535, "sample: %d rows are too many", R);
+  NINFER_REQUIRE(R <= kSpreadRows, "sample: %d rows are too many", R);
   if ((V + kSlice - 1) / kSlice > kMaxSlices) wide = 0;
   const SpreadLayout p = spread_layout(V, R, wide);
   char* base = (char*)scratch;
@@ -1199,7 +1200,8 @@ extern "C" int ninfer_sample_rows(const float* logits, int ld, int V, int R, int
                         pen, f + 3 * R, tokens, (float*)scratch, ld, V};
   // (not through the two entry points above: the engine's C interface has a function by the name of one, and in a program
   // that is linked to it a call by that name would end there)
-  const int rc = mode == 0 ? sample_by_rows(a, R, stream) : sample_by_slices(a, R, mode == 2, stream);
+  const bool by_rows = mode == 0 || R > kSpreadRows;   // (the same tokens; the others' scratch begins with this one's)
+  const int rc = by_rows ? sample_by_rows(a, R, stream) : sample_by_slices(a, R, mode == 2, stream);
   const hipError_t e = hipStreamSynchronize(stream);   // (also after an error: the caller's buffers are its own again)
   if (rc) return rc;
   if (e != hipSuccess) return set_error(-2, "sample: %s", hipGetErrorString(e));

@@ -43,6 +43,18 @@ def test_tokens_are_those_of_the_kernels(ops, rows, penalty, top_k, temperature)
         assert len(sampler._free) == 1
 
 
+def test_more_rows_than_a_grid_is_high(ops):
+    rows, vocab = 65537, 12800
+    logits = torch.randn(rows, vocab, device="cuda")
+    params, nothing = SamplingParams(temperature=0.8, top_k=0, top_p=0.9, repetition_penalty=1.0), History([])
+    got = Sampler(ops, torch.device("cuda:0")).sample(logits, [SampleRow(params, nothing, key=i, draw=0, seed=7) for i in range(rows)])
+    every = list(range(0, rows, 997)) + [rows - 1]
+    f32 = lambda v: torch.tensor(v, dtype=torch.float32, device="cuda")
+    out = torch.empty(len(every), dtype=torch.int32, device="cuda")
+    ops.sample(logits[every].contiguous(), f32([0.8] * len(every)), f32([uniform(7, i, 0) for i in every]), out, top_p=f32([0.9] * len(every)))
+    assert [got[i] for i in every] == out.tolist()
+
+
 def test_what_it_refuses(ops):
     from ninfer_amd.kernels.ops import KernelError
     logits, numbers = torch.zeros(2, 50, device="cuda"), torch.zeros(64, dtype=torch.int32)
