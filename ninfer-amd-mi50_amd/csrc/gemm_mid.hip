@@ -189,12 +189,30 @@ static int mid_tile(const GemmArgs& a) {
   return -1;
 }
 
-// Dense products of more than 32 rows that are one round of tiles. (Fewer rows go to the few-row kernel.)
+// Does a product take less in the four-wave tiles of 64 x 128, of which a CU holds two, or as long? Measured on products that are gated
+// or have a bias or 32-bit outputs, some 2,000 sizes (us here and there; elsewhere none of more than 2% takes longer here, but for single
+// sizes whose rows of W lie badly in memory):
+// - 192 x 64 leaves CUs without a block, and rows of A without a number, where those tiles are one a CU as well: 2 x 4,296 features
+//   of K 1,280, 144 rows 15.3 and 13.1; 10,432 of K 1,792, 160 rows 20.0 and 17.8 (100 sizes of up to 192 rows 0.85 to 0.96 of their
+//   speed). From three quarters of their number and a K beyond 2,048 on its blocks are the faster ones: 2 x 2,904 of K 4,800, 305 rows
+//   36.2 and 39.0.
+// - 128 x 128 for up to 64 rows: 32,000 features of K 1,024, 64 rows 20.4 and 16.0, 33 rows 16.5 and 15.4; K 2,048 34.4 and 34.8.
+// - 128 x 128 and 128 x 192 of few rows more, which fill the GPU: 31,264 of K 1,024, 65 rows 20.1 and 17.3; 47,352 of K 896, 33 rows 23.8
+//   and 20.0; but 28,456 of K 1,216, 66 rows 17.5 and 20.5, 36,112, 64 rows 22.0 and 26.9.
+static bool low_tiles_beat(const GemmArgs& a, const MidTile& t) {
+  const int cus = device_cu_count(), here = mid_tiles(a, t), low = mid_tiles(a, {64, 128, true});
+  if (t.rows == 192 && t.w_rows == 64) return low <= cus && (4 * here < 3 * low || a.K <= 2048);
+  if (t.rows != 128 || t.w_rows == 64) return false;
+  return (a.M <= 64 && t.w_rows == 128) || (a.M <= 72 && a.K <= 1536 && 16 * here >= 15 * cus);
+}
+
+// Dense products of more than 32 rows that are one round of tiles, and no faster in lower ones. (Fewer rows go to the few-row kernel.)
 bool gemm_mid_takes(const GemmArgs& a) {
   if (a.offsets || a.a_index || a.c_index || a.groups > 1 || a.k_parts > 1 || a.force_kernel || a.M <= 32 || a.N < 64 ||
       !gemm_tile_takes(a))
     return false;
-  return mid_tile(a) >= 0;
+  const int tile = mid_tile(a);
+  return tile >= 0 && !low_tiles_beat(a, kMidTiles[tile]);
 }
 
 // Of a plain product, which the library has otherwise: is it no slower here? Up to K 4,032 it is (95 sizes of 65 to 2,000 rows:

@@ -29,6 +29,21 @@ def test_which_tile(m, n, k, gated, tile):
     assert lib.ninfer_gemm_mid_tile(ctypes.byref(_args(m, n, k, epilogue=gated, a_index=16, offsets=16))) == 0
 
 
+# Both sides of where tiles of 64 x 128, two a CU, are the faster ones (256 CUs): 192 x 64 that leaves CUs without a block, 128 rows for up to
+# 64, tiles of 128 rows that fill the GPU for few more.
+@pytest.mark.parametrize("m,n,k,gated,tile", [
+    (144, 4296, 1280, 1, 0), (144, 4296, 7168, 1, 0), (160, 10432, 1792, 0, 0), (315, 3152, 2048, 1, 0), (305, 2904, 4800, 1, 192064), (257, 6000, 2112, 0, 192064), (257, 6000, 2048, 0, 0),
+    (130, 10944, 1792, 0, 192064), (144, 11008, 1280, 0, 192064), (33, 32000, 1024, 0, 0), (64, 32000, 4096, 0, 0), (64, 16000, 2048, 1, 0),
+    (65, 32000, 1536, 0, 0), (72, 30721, 1024, 0, 0), (72, 30592, 1024, 0, 128128), (73, 32000, 1024, 0, 128128), (65, 32000, 1600, 0, 128128),
+    (64, 46144, 1024, 0, 0), (64, 45888, 1024, 0, 128192), (48, 46144, 1600, 0, 128192), (100, 14000, 1024, 0, 128064)])
+def test_what_lower_tiles_run_faster_stays_with_them(m, n, k, gated, tile):
+    from ninfer_amd.kernels.build import ensure_built
+    lib = ctypes.CDLL(ensure_built())
+    assert lib.ninfer_gemm_mid_tile(ctypes.byref(_args(m, n, k, epilogue=gated))) == tile
+    if tile == 0:
+        assert lib.ninfer_gemm_kernel(ctypes.byref(_args(m, n, k, epilogue=gated))) == 4 and lib.ninfer_gemm_tile_rows(ctypes.byref(_args(m, n, k, epilogue=gated))) == 64
+
+
 SHAPES = [(33, 8192, 64), (64, 2056, 192), (64, 16384, 320), (130, 2050, 64), (512, 2048, 2048), (700, 2047, 192), (760, 2048, 320),
           (250, 6100, 128), (129, 8190, 448), (900, 2304, 192), (1500, 2040, 64), (1140, 2900, 576), (1500, 4090, 128),
           (1020, 6100, 256), (2048, 136, 704)]
