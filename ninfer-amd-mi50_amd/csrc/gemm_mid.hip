@@ -215,23 +215,27 @@ bool gemm_mid_takes(const GemmArgs& a) {
   return tile >= 0 && !low_tiles_beat(a, kMidTiles[tile]);
 }
 
-// Of a plain product, which the library has otherwise: is it no slower here? Up to K 4,032 it is (95 sizes of 65 to 2,000 rows:
-// 0.97 to 1.5 of the library's speed). A longer K costs a lone block most where its rows of W are few for the weights there are; us in the
-// library and here, K 4,096 to 8,192:
+// Of a plain product that gemm_mid takes, which the library has otherwise: is it no slower here? Up to K 4,032 it is (2,400 sizes of
+// 33 to 2,000 rows: 1.2 of the library's speed on average, 0.96 and more but for one in twenty, half of them of a few hundred features, us
+// in the library and here: 192 of K 832, 768 rows 5.0 and 5.8, 256 of K 2,624, 33 rows 7.4 and 8.7, 7,296 of K 3,712, 380 rows, where the
+// library's time jumps, 31.4 and 35.3; against 15 us of the host's time). A longer K costs a lone block most
+// where its rows of W are few for the weights there are, and the library cuts products of few blocks along K; K 4,096 to 8,192:
 // - 32 x 64: 1,216 features of K 5,632, 338 rows 17.2 and 15.9; but 1,600 of K 5,120, 276 rows 19.7 and 21.1, 2,688 of K 7,168, 140
-//   rows 22.3 and 25.2.
+//   rows 22.3 and 25.2. From K 5,120 on it takes longer only where its tiles are at most half of the CUs: 320 of K 5,376, 768 rows
+//   12.3 and 14.6, 1,344 of K 7,616, 45 rows 19.0 and 25.7; 1,024 of K 6,336, 507 rows 28.0 and 17.5.
 // - 64 x 64: 2,048 of K 5,632, 335 rows 25.3 and 23.1, 512 27.8 and 27.8; but 2,176 of K 6,144, 384 rows 28.0 and 30.2.
 // - 192 x 64: 1,600 of K 5,120, 1,294 rows 36.9 and 43.0, 1,920 of K 5,632, 1,482 rows 43.6 and 46.9 (and 2,560 of K 5,632, 806
 //   rows, 47.7 and 40.8: the library's times jump).
 // - 128 x 128: 2,048 of K 5,632, 2,048 rows 58.7 and 55.2; but 6,400 of K 4,608, 473 rows 38.8 and 44.8.
-// - the others 0.95 to 1.7 of its speed.
-// Beyond K 8,192 the library cuts products along K: 1,408 features of K 14,336, 173 rows 38.9 and 43.0.
+// - the others 0.93 to 1.7 of its speed.
+// Beyond K 8,192 the library cuts more products along K: 1,408 features of K 14,336, 173 rows 38.9 and 43.0.
 bool gemm_mid_beats_library(const GemmArgs& a) {
   if (a.K < 4096) return true;
   const int tile = mid_tile(a);
   if (a.K > 8192 || tile < 0) return false;
   const MidTile& t = kMidTiles[tile];
-  if (t.w_rows == 64 && t.rows == 32) return a.K == 4096 || a.N < 1536;
+  if (t.w_rows == 64 && t.rows == 32)
+    return a.K == 4096 || (a.N < 1536 && (a.K < 5120 || 2 * mid_tiles(a, t) > device_cu_count()));
   if (t.w_rows == 64 && t.rows == 64) return a.K < 6144;
   if (t.w_rows == 64 && t.rows == 192) return false;
   return t.w_rows != 128 || t.rows != 128 || a.M > 512;

@@ -137,11 +137,13 @@ def test_one_call_runs_what_the_questions_one_by_one_would(m, n, k, taken):
 # tiles; and those of a long K that are slower in one round of tiles than in the library.
 NOT_OURS = [(80, 4096, 5632), (112, 4096, 5632), (112, 3072, 5632), (100, 4096, 4096), (64, 512, 5632), (512, 129, 8192),
             (2048, 64, 2048), (700, 128, 704), (4096, 8192, 512), (512, 2048, 2080),
+            (768, 320, 5376), (45, 1344, 7616), (110, 192, 7616), (180, 8448, 1792),
             (276, 1600, 5120), (140, 2688, 7168), (384, 2176, 6144), (1294, 1600, 5120), (1482, 1920, 5632), (512, 6400, 4608), (1043, 576, 8256)]
 
 
 @pytest.mark.parametrize("m,n,k,ours", [(*s, 0) for s in NOT_OURS] + [
     (96, 8192, 2048, 1), (513, 2048, 1024, 1), (700, 129, 704, 1), (1294, 1600, 4032, 1), (142, 2688, 4096, 1), (338, 1472, 5632, 1),
+    (720, 320, 5056, 1), (1010, 576, 5568, 1), (380, 7296, 3072, 1),
     (512, 2048, 5632, 1), (513, 6400, 4608, 1), (900, 2048, 5632, 1), (2048, 2048, 8192, 1)])
 def test_which_plain_products_leave_the_library(m, n, k, ours):
     from ninfer_amd.kernels.build import ensure_built
