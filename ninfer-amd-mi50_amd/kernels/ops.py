@@ -2255,6 +2255,7 @@ class HipOps:
             _dev(pen_tokens, "pen_tokens", torch.int32, 1)
             _dev(pen_counts, "pen_counts", torch.int32, 1)
             _need(pen_offsets.shape[0] == r + 1, "sample: pen_offsets has the wrong size")
+        _need(not few or top_k is not None, "sample: rows that keep few tokens need top_k")
         if few or spread:
             scratch = torch.empty(int(self.lib.ninfer_sample_spread_bytes(v, r, int(spread))), dtype=torch.uint8,
                                   device=logits.device)

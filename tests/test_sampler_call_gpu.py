@@ -64,3 +64,12 @@ def test_what_it_refuses(ops):
             ops.sample_rows(logits, rows, buffer, ints, n_pen)
     with pytest.raises(KernelError):
         Sampler(ops, torch.device("cuda:0")).sample(logits[:0], [])
+
+
+def test_rows_that_keep_few_tokens_say_how_many(ops):
+    from ninfer_amd.kernels.ops import KernelError
+    logits, f32 = torch.zeros(2, 50, device="cuda"), torch.ones(2, device="cuda")
+    out = torch.full((2,), -7, dtype=torch.int32, device="cuda")
+    with pytest.raises(KernelError, match="top_k"):
+        ops.sample(logits, f32, f32 * 0.5, out, few=True)
+    assert out.tolist() == [-7, -7]
