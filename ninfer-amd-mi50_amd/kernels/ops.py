@@ -800,11 +800,14 @@ class HipOps:
             return False
         return not torch.cuda.is_current_stream_capturing()
 
-    def wants_beside_short(self, rows: int, weight_bytes: int, dtype) -> bool:
+    def wants_beside_short(self, rows: int, weight_bytes: int, dtype, own_bytes: Optional[int] = None) -> bool:
         """`pays_beside`, as a step that `wants_beside` says no to asks it: not while a graph is being captured, and not where
-        `beside_min_rows` has been put out of reach, to have one stream (32 times the step's rows and more)."""
-        return (32 * rows >= self.beside_min_rows and self.pays_beside(rows, weight_bytes, dtype)
-                and not torch.cuda.is_current_stream_capturing())
+        `beside_min_rows` has been put out of reach, to have one stream (32 times the step's rows and more); nor where the work
+        beside (`own_bytes` of the weights) is less than a 32nd of all, which two streams then cost more than they hide (one
+        stream's time by two's: 128 experts and a shared one of 1,024, 65 to 480 rows 0.98 to 1.00, in 32-bit 17 to 100 rows 0.98 to
+        0.995; 64 of 2,048 0.98 to 1.02; 16 of 7,168 1.01 to 1.05, in 32-bit 1.00 to 1.03)."""
+        return (32 * rows >= self.beside_min_rows and (own_bytes is None or 32 * own_bytes >= weight_bytes)
+                and self.pays_beside(rows, weight_bytes, dtype) and not torch.cuda.is_current_stream_capturing())
 
     def pays_beside(self, rows: int, weight_bytes: int, dtype) -> bool:
         """Are a routed path and the independent work beside it (whose weights are so many bytes together) long enough on the

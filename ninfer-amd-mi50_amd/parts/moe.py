@@ -277,7 +277,7 @@ class SparseMoE(FeedForward):
         logits = ctx.empty((x.shape[0], self.router.experts + 1), torch.float32)
         own = self.shared.weight_bytes()
         if ctx.ops.wants_beside(x.shape[0], own) or (
-                x.is_cuda and ctx.ops.wants_beside_short(x.shape[0], self.experts.weight_bytes() + own, x.dtype)):
+                x.is_cuda and ctx.ops.wants_beside_short(x.shape[0], self.experts.weight_bytes() + own, x.dtype, own)):
             # While its blocks leave the GPU room, the second stream starts before the routing's short
             # kernels and fills the device beside them; else after them: they would crawl.
             early = ctx.ops.leaves_room(x.shape[0], 2 * self.shared.inner, self._shared_fills(x.shape[0]))

@@ -353,6 +353,19 @@ def test_one_stream_when_it_is_asked_for(monkeypatch, min_rows, rows, capturing,
     assert not HipOps.wants_beside_short(ops, rows, 1 << 40, torch.float32)
 
 
+# (experts and their inner size, the shared expert's, width 2,048)
+@pytest.mark.parametrize("experts,inner,shared,two", [(60, 1408, 5632, True), (16, 7168, 7168, True), (31, 2048, 2048, True),
+                                                      (32, 2048, 2048, False), (64, 2048, 2048, False), (128, 1024, 1024, False)])
+def test_a_shared_expert_of_little_work_stays_on_the_stream(monkeypatch, experts, inner, shared, two):
+    import torch
+    from types import SimpleNamespace
+    from ninfer_amd.kernels.ops import HipOps
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    ops = SimpleNamespace(beside_min_rows=512, pays_beside=lambda *a: True)
+    own = 3 * 2048 * shared * 2
+    assert HipOps.wants_beside_short(ops, 128, 3 * 2048 * experts * inner * 2 + own, torch.bfloat16, own) == two
+
+
 def test_the_bindings_say_how_many_tokens_a_sampled_row_may_keep(lib, monkeypatch):
     from ninfer_amd.kernels.ops import HipOps, KernelError
     assert lib.ninfer_sample_few_tokens() == HipOps.FEW_TOKENS
