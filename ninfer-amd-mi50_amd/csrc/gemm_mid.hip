@@ -216,7 +216,7 @@ bool gemm_mid_takes(const GemmArgs& a) {
 }
 
 // Of a plain product that gemm_mid takes, which the library has otherwise: is it no slower here? Up to K 4,032 it is (2,400 sizes of
-// 33 to 2,000 rows: 1.2 of the library's speed on average, 0.96 and more but for one in twenty, half of them of a few hundred features, us
+// 33 to 2,000 rows: 1.2 of the library's speed on average, 0.96 and more but for one in forty, half of them of a few hundred features, us
 // in the library and here: 192 of K 832, 768 rows 5.0 and 5.8, 256 of K 2,624, 33 rows 7.4 and 8.7, 7,296 of K 3,712, 380 rows, where the
 // library's time jumps, 31.4 and 35.3; against 15 us of the host's time). A longer K costs a lone block most
 // where its rows of W are few for the weights there are, and the library cuts products of few blocks along K; K 4,096 to 8,192:
